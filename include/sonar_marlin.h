@@ -112,6 +112,29 @@ int sonar_awq_marlin_repack(const uint32_t* b_q_weight, uint32_t* out,
                             int64_t size_k, int64_t size_n, int num_bits,
                             void* stream);
 
+/* A stack of matrices in one launch (gptq_marlin_moe_repack / awq_marlin_moe_repack,
+ * aphrodite/_custom_ops.py:1424-1461, which loop over the experts): 4-bit codes, matrix e at
+ * b_q_weight + e * K * N / 8 words, its perm (may be NULL for all) at perm + e * K. */
+int sonar_gptq_marlin_moe_repack(const uint32_t* b_q_weight, const int32_t* perm, uint32_t* out,
+                                 int64_t experts, int64_t size_k, int64_t size_n, void* stream);
+int sonar_awq_marlin_moe_repack(const uint32_t* b_q_weight, uint32_t* out, int64_t experts,
+                                int64_t size_k, int64_t size_n, void* stream);
+
+/* The checkpoint tensors around the codes.
+ * marlin_permute_scales (grouped != 0: 64-column pattern; 0: the 32-column pattern of one group and
+ * of marlin_permute_bias) on 16-bit elements, aphrodite quantization/utils/marlin_utils.py:404-434. */
+int sonar_marlin_permute_scales(const void* in, void* out, int64_t numel, int grouped, void* stream);
+/* Zero points packed along N, eight to a word, in plain or AWQ nibble order -> (rows, N/8) words in the
+ * order the GEMM reads (marlin_utils.py:457-559: marlin_zero_points, awq_to_marlin_zero_points);
+ * in[row * row_stride + word * word_stride]. */
+int sonar_marlin_pack_zero_points(const uint32_t* in, uint32_t* out, int64_t rows, int64_t size_n,
+                                  int64_t row_stride, int64_t word_stride, int awq_order, int is_a_8bit,
+                                  void* stream);
+/* AutoAWQ codes (K, N/8) -> GPTQ codes (K/8, N); AutoAWQ zero points (G, N/8) -> plain column order,
+ * transposed to (N/8, G) (_convert_awq_to_standard_format, layers/quantization/auto_awq.py:93-153). */
+int sonar_awq_to_gptq(const uint32_t* in, uint32_t* out, int64_t size_k, int64_t size_n, void* stream);
+int sonar_awq_zeros_to_plain(const uint32_t* in, uint32_t* out, int64_t groups, int64_t size_n, void* stream);
+
 /* Marlin (K/16, 2N) int32 <-> gfx950 streaming order, same number of words.
  * K % 32 == 0, N % 64 == 0.  in and out must not overlap. */
 int sonar_marlin_to_gfx950(const uint32_t* marlin, uint32_t* out,

@@ -36,6 +36,13 @@ PROTOTYPES = {
     "sonar_debug_moe_tile_schedule": (c_int64, [c_int64, c_int64, c_int64, c_int64, c_int, c_int, c_void_p, c_int64]),
     "sonar_gptq_marlin_repack": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int, c_void_p]),
     "sonar_awq_marlin_repack": (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_int, c_void_p]),
+    "sonar_gptq_marlin_moe_repack": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_void_p]),
+    "sonar_awq_marlin_moe_repack": (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_int64, c_void_p]),
+    "sonar_marlin_permute_scales": (c_int, [c_void_p, c_void_p, c_int64, c_int, c_void_p]),
+    "sonar_marlin_pack_zero_points": (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_int, c_int,
+                                              c_void_p]),
+    "sonar_awq_to_gptq": (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_void_p]),
+    "sonar_awq_zeros_to_plain": (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_void_p]),
     "sonar_marlin_to_gfx950": (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_void_p]),
     "sonar_gfx950_to_marlin": (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_void_p]),
     "sonar_marlin8_to_gfx950": (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_void_p]),

@@ -1,7 +1,6 @@
 // Weight re-ordering kernels: checkpoint packings -> Marlin tile order, and
-// Marlin tile order <-> the gfx950 streaming order.  Pure integer work; each
-// thread assembles one 32-bit output word from eight source nibbles, so the
-// stores of a wavefront are one contiguous 256-byte run.
+// Marlin tile order <-> the gfx950 streaming order.  Pure integer work; the
+// stores of a wavefront are one contiguous run.
 #include "common.hpp"
 
 namespace sonar {
@@ -24,57 +23,108 @@ __device__ __forceinline__ void marlin_word_sources(int word, int slot, int& row
   col = 16 * j + c + 8 * ((slot >> 1) & 1);
 }
 
+// GPTQ / AWQ words -> Marlin words, for one matrix or a stack of them (`tiles_each` tiles of one
+// matrix, `in_each` its source words; the matrices follow each other in memory).  Bound by HBM:
+// every source word is read once and every output word written once.  Half a wavefront owns a
+// 16 x 64 tile: each lane fetches 16 bytes of it (32 lanes: two 256-byte rows of GPTQ words or
+// sixteen 32-byte rows of AWQ words), the tile meets in LDS and each lane assembles the 16 bytes of
+// Marlin lane `l`.  One thread per output word gathering its eight nibbles from global memory, as
+// this kernel was first written, issued eight 4-byte loads per word stored and ran at 2.2 TB/s
+// (117 MB moved for a 4096 x 28672 matrix in 53 us; 23 us = 5.1 TB/s this way).
+// kRepackTiles tiles a workgroup.
+constexpr int kRepackTiles = 8;
+constexpr int kRepackLdsStride = 136;   // words between the tiles of a wavefront: neighbours on other banks
+
+// Marlin word of the low and high nibbles of four source bytes: nibble slots 0..3 are the low nibbles
+// of b0, b1, b2, b3, slots 4..7 the high ones.
+__device__ __forceinline__ uint32_t interleave_nibbles(uint32_t b0, uint32_t b1, uint32_t b2, uint32_t b3) {
+  const uint32_t x = b0 | (b2 << 8);   // slots 0 and 2
+  const uint32_t y = b1 | (b3 << 8);   // slots 1 and 3
+  const uint32_t lo = (x & 0x0F0Fu) | ((y & 0x0F0Fu) << 4);
+  const uint32_t hi = ((x >> 4) & 0x0F0Fu) | (y & 0xF0F0u);
+  return lo | (hi << 16);
+}
+
+// With HAS_PERM (act-order) the sixteen rows of a tile come from sixteen words of different rows: a
+// half wavefront reads each as 256 bytes and leaves the selected nibbles in LDS in the source's own packing.
 template <bool HAS_PERM>
 __global__ __launch_bounds__(256) void gptq_to_marlin_kernel(
-    const uint32_t* __restrict__ in, const int32_t* __restrict__ perm,
-    uint32_t* __restrict__ out, int size_k, int size_n, long total_words) {
-  const int n_tiles = size_n / kMarlinTileN;
-  for (long idx = (long)blockIdx.x * blockDim.x + threadIdx.x; idx < total_words;
-       idx += (long)gridDim.x * blockDim.x) {
-    const long tile = idx / kMarlinTileWords;
-    const int word = (int)(idx % kMarlinTileWords);
-    const int kt = (int)(tile / n_tiles);
-    const int nt = (int)(tile % n_tiles);
-    uint32_t packed = 0;
+    const uint32_t* __restrict__ in, const int32_t* __restrict__ perm, uint32_t* __restrict__ out, int size_k,
+    int size_n, uint32_t tiles_each, long in_each, uint32_t total_tiles) {
+  __shared__ alignas(16) uint32_t lds[kRepackTiles * kRepackLdsStride];
+  const uint32_t n_tiles = size_n / kMarlinTileN;
+  const int sub = threadIdx.x >> 5, l = threadIdx.x & 31;
+  const uint32_t tile = blockIdx.x * kRepackTiles + sub;
+  const bool live = tile < total_tiles;
+  uint32_t* mine = lds + sub * kRepackLdsStride;
+  if (live) {
+    const uint32_t matrix = tile / tiles_each, t = tile - matrix * tiles_each;
+    const int kt = (int)(t / n_tiles), nt = (int)(t - kt * n_tiles);
+    const uint32_t* src = in + matrix * in_each + nt * kMarlinTileN;
+    const int half = l >> 4, col = 4 * (l & 15);   // which eight rows of the tile, first of four columns
+    u32x4_t v;
+    if constexpr (HAS_PERM) {
+      const int32_t* rows = perm + (long)matrix * size_k + kt * kMarlinTileK + 8 * half;
+      v = u32x4_t{0, 0, 0, 0};
 #pragma unroll
-    for (int slot = 0; slot < 8; ++slot) {
-      int row, col;
-      marlin_word_sources(word, slot, row, col);
-      int k = kt * kMarlinTileK + row;
-      if (HAS_PERM) k = perm[k];
-      const int n = nt * kMarlinTileN + col;
-      const uint32_t src = in[(long)(k >> 3) * size_n + n];
-      packed |= ((src >> (4 * (k & 7))) & 0xFu) << (4 * slot);
+      for (int r = 0; r < 8; ++r) {
+        const int k = rows[r];
+        const u32x4_t w = *reinterpret_cast<const u32x4_t*>(src + (long)(k >> 3) * size_n + col);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] |= ((w[i] >> (4 * (k & 7))) & 0xFu) << (4 * r);
+      }
+    } else {
+      v = *reinterpret_cast<const u32x4_t*>(src + (long)(2 * kt + half) * size_n + col);
     }
-    out[idx] = packed;
+    *reinterpret_cast<u32x4_t*>(mine + half * kMarlinTileN + col) = v;
   }
+  __syncthreads();
+  if (!live) return;
+  const int c = l >> 2, h = l & 3;
+  u32x4_t o;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    // byte h of a source word: rows 2h (low nibble) and 2h + 1 of its column
+    const uint32_t* w = mine + 16 * j + c;
+    o[j] = interleave_nibbles((w[0] >> (8 * h)) & 0xFFu, (w[kMarlinTileN] >> (8 * h)) & 0xFFu,
+                              (w[8] >> (8 * h)) & 0xFFu, (w[kMarlinTileN + 8] >> (8 * h)) & 0xFFu);
+  }
+  *reinterpret_cast<u32x4_t*>(out + (long)tile * kMarlinTileWords + 4 * l) = o;
 }
 
 __global__ __launch_bounds__(256) void awq_to_marlin_kernel(
-    const uint32_t* __restrict__ in, uint32_t* __restrict__ out, int size_k,
-    int size_n, long total_words) {
-  const int n_tiles = size_n / kMarlinTileN;
-  const int in_stride = size_n / 8;
-  for (long idx = (long)blockIdx.x * blockDim.x + threadIdx.x; idx < total_words;
-       idx += (long)gridDim.x * blockDim.x) {
-    const long tile = idx / kMarlinTileWords;
-    const int word = (int)(idx % kMarlinTileWords);
-    const int kt = (int)(tile / n_tiles);
-    const int nt = (int)(tile % n_tiles);
-    uint32_t packed = 0;
-#pragma unroll
-    for (int slot = 0; slot < 8; ++slot) {
-      int row, col;
-      marlin_word_sources(word, slot, row, col);
-      const int k = kt * kMarlinTileK + row;
-      const int n = nt * kMarlinTileN + col;
-      // column n % 8 = 2*(p % 4) + p / 4 sits at nibble p = (n%8)/2 + 4*(n%2)
-      const int p = ((n & 7) >> 1) + 4 * (n & 1);
-      const uint32_t src = in[(long)k * in_stride + (n >> 3)];
-      packed |= ((src >> (4 * p)) & 0xFu) << (4 * slot);
-    }
-    out[idx] = packed;
+    const uint32_t* __restrict__ in, uint32_t* __restrict__ out, int size_n, uint32_t tiles_each, long in_each,
+    uint32_t total_tiles) {
+  __shared__ alignas(16) uint32_t lds[kRepackTiles * kRepackLdsStride];
+  const uint32_t n_tiles = size_n / kMarlinTileN;
+  const int sub = threadIdx.x >> 5, l = threadIdx.x & 31;
+  const uint32_t tile = blockIdx.x * kRepackTiles + sub;
+  const bool live = tile < total_tiles;
+  uint32_t* mine = lds + sub * kRepackLdsStride;
+  if (live) {
+    const uint32_t matrix = tile / tiles_each, t = tile - matrix * tiles_each;
+    const int kt = (int)(t / n_tiles), nt = (int)(t - kt * n_tiles);
+    const uint32_t* src = in + matrix * in_each + (long)(kt * kMarlinTileK + (l >> 1)) * (size_n / 8) +
+                          nt * (kMarlinTileN / 8) + 4 * (l & 1);
+    *reinterpret_cast<u32x4_t*>(mine + 4 * l) = *reinterpret_cast<const u32x4_t*>(src);   // row l / 2 of the tile: 8 words
   }
+  __syncthreads();
+  if (!live) return;
+  const int c = l >> 2, h = l & 3;
+  const int shift = 4 * ((c >> 1) + 4 * (c & 1));   // column n % 8 = c sits at nibble c / 2 + 4 (c % 2)
+  u32x4_t o;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const uint32_t* w = mine + 2 * h * 8 + 2 * j;   // rows 2h, 2h + 1 and eight further down; words 2j (columns 16j..) and 2j + 1
+    uint32_t b[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t* at = w + (i & 1) * 64 + (i >> 1);
+      b[i] = ((at[0] >> shift) & 0xFu) | (((at[8] >> shift) & 0xFu) << 4);
+    }
+    o[j] = interleave_nibbles(b[0], b[1], b[2], b[3]);
+  }
+  *reinterpret_cast<u32x4_t*>(out + (long)tile * kMarlinTileWords + 4 * l) = o;
 }
 
 // One thread per gfx950 word.  Word j of lane L of chunk c of strip s holds
@@ -365,6 +415,100 @@ __global__ __launch_bounds__(256) void int4_fp8_preprocess_kernel(const uint32_t
   }
 }
 
+// ---- checkpoint tensors around the codes -----------------------------------
+// marlin_permute_scales / marlin_permute_bias on 16-bit elements: inside every 64 columns
+// out[8 i + j] = in[i + 8 j] (groups along K), or inside every 32 columns
+// out[8 i + j] = in[2 i + {0, 1, 8, 9, 16, 17, 24, 25}[j]] (one group, bias).  A thread stores 16
+// bytes; its loads stay inside one 128-byte line.
+template <bool GROUPS>
+__global__ __launch_bounds__(256) void permute_scale_columns(const uint16_t* __restrict__ in,
+                                                             uint16_t* __restrict__ out, long vectors) {
+  const long v = (long)blockIdx.x * 256 + threadIdx.x;
+  if (v >= vectors) return;
+  uint32_t o[4];
+  if constexpr (GROUPS) {
+    const uint16_t* src = in + (v >> 3) * 64 + (v & 7);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o[j] = (uint32_t)src[16 * j] | ((uint32_t)src[16 * j + 8] << 16);
+  } else {
+    const uint16_t* src = in + (v >> 2) * 32 + 2 * (v & 3);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o[j] = (uint32_t)src[8 * j] | ((uint32_t)src[8 * j + 1] << 16);
+  }
+  *reinterpret_cast<uint4*>(out + 8 * v) = make_uint4(o[0], o[1], o[2], o[3]);
+}
+
+// Packed zero points -> Marlin zero points, (rows, N/8) words.  Nibble e of output word w is the code
+// of column 64 (w / 8) + w % 8 + 8 * i(e), i = {0, 2, 4, 6, 1, 3, 5, 7} (the column interleave of the
+// 16-bit dequantiser; the identity for 8-bit activations), i.e. always nibble w % 8 of a source word,
+// or nibble (w % 8) / 2 + 4 (w % 2) where the source has the AWQ order.
+__global__ __launch_bounds__(256) void pack_zero_points(const uint32_t* __restrict__ in, uint32_t* __restrict__ out,
+                                                        int words, long total, long row_stride, long word_stride,
+                                                        bool awq_order, bool a8) {
+  const long idx = (long)blockIdx.x * 256 + threadIdx.x;
+  if (idx >= total) return;
+  const long row = idx / words;
+  const int w = (int)(idx - row * words);
+  const int shift = 4 * (awq_order ? ((w & 7) >> 1) + 4 * (w & 1) : w & 7);
+  const uint32_t* src = in + row * row_stride + (long)(w & ~7) * word_stride;
+  uint32_t packed = 0;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const int from = a8 ? e : (e < 4 ? 2 * e : 2 * e - 7);
+    packed |= ((src[from * word_stride] >> shift) & 0xFu) << (4 * e);
+  }
+  out[idx] = packed;
+}
+
+// AutoAWQ codes (K, N/8) -> the GPTQ packing (K/8, N): a thread transposes the 8 x 8 nibbles of eight
+// rows of one word, three rounds of block swaps, and stores the eight columns side by side.
+__global__ __launch_bounds__(256) void awq_codes_to_gptq(const uint32_t* __restrict__ in, uint32_t* __restrict__ out,
+                                                         int words, long total) {
+  const long idx = (long)blockIdx.x * 256 + threadIdx.x;
+  if (idx >= total) return;
+  const long r = idx / words;
+  const int w = (int)(idx - r * words);
+  uint32_t x[8];
+#pragma unroll
+  for (int t = 0; t < 8; ++t) x[t] = in[(8 * r + t) * words + w];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t a = x[i], b = x[i + 4];
+    x[i] = (a & 0xFFFFu) | (b << 16);
+    x[i + 4] = (a >> 16) | (b & 0xFFFF0000u);
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int i = (q >> 1) * 4 + (q & 1);
+    const uint32_t a = x[i], b = x[i + 2];
+    x[i] = (a & 0x00FF00FFu) | ((b & 0x00FF00FFu) << 8);
+    x[i + 2] = ((a >> 8) & 0x00FF00FFu) | (b & 0xFF00FF00u);
+  }
+#pragma unroll
+  for (int i = 0; i < 8; i += 2) {
+    const uint32_t a = x[i], b = x[i + 1];
+    x[i] = (a & 0x0F0F0F0Fu) | ((b & 0x0F0F0F0Fu) << 4);
+    x[i + 1] = ((a >> 4) & 0x0F0F0F0Fu) | (b & 0xF0F0F0F0u);
+  }
+  // x[p] now holds nibble p of every row; column c sits at nibble c / 2 + 4 (c % 2)
+  uint32_t* dst = out + r * (8L * words) + 8 * w;
+  *reinterpret_cast<uint4*>(dst) = make_uint4(x[0], x[4], x[1], x[5]);
+  *reinterpret_cast<uint4*>(dst + 4) = make_uint4(x[2], x[6], x[3], x[7]);
+}
+
+// AutoAWQ zero points (G, N/8) -> plain column order, transposed: (N/8, G).
+__global__ __launch_bounds__(256) void awq_zeros_to_plain(const uint32_t* __restrict__ in, uint32_t* __restrict__ out,
+                                                          int groups, int words, long total) {
+  const long idx = (long)blockIdx.x * 256 + threadIdx.x;
+  if (idx >= total) return;
+  const long w = idx / groups;
+  const uint32_t z = in[(idx - w * groups) * words + w];
+  uint32_t packed = 0;
+#pragma unroll
+  for (int c = 0; c < 8; ++c) packed |= ((z >> (4 * ((c >> 1) + 4 * (c & 1)))) & 0xFu) << (4 * c);
+  out[idx] = packed;
+}
+
 int grid_for(long total_words) {
   long blocks = (total_words + 255) / 256;
   if (blocks > 256L * 32) blocks = 256L * 32;
@@ -380,9 +524,34 @@ int check_repack_shape(int64_t size_k, int64_t size_n, int num_bits) {
                 (long)size_k, kMarlinTileK);
   SONAR_REQUIRE(size_n % kMarlinTileN == 0, "size_n = %ld is not divisible by tile_n_size = %d",
                 (long)size_n, kMarlinTileN);
-  SONAR_REQUIRE(size_k * size_n / 8 < (1LL << 40), "weight too large");
+  SONAR_REQUIRE(size_k * size_n / 8 < (1LL << 37), "weight too large");   // half a terabyte of packed codes
   SONAR_REQUIRE(size_k < (1LL << 30) && size_n < (1LL << 30), "size_k / size_n too large");
   return SONAR_OK;
+}
+
+int check_experts(int64_t experts, int64_t size_k, int64_t size_n) {
+  SONAR_REQUIRE(experts >= 1 && experts * (size_k / kMarlinTileK) * (size_n / kMarlinTileN) < (1LL << 31),
+                "experts = %ld out of range", (long)experts);
+  return SONAR_OK;
+}
+
+int launch_gptq_to_marlin(const uint32_t* in, const int32_t* perm, uint32_t* out, int64_t experts, int64_t size_k,
+                          int64_t size_n, hipStream_t st) {
+  const long each = (size_k / kMarlinTileK) * (size_n / kMarlinTileN), total = experts * each;
+  const int blocks = (int)((total + kRepackTiles - 1) / kRepackTiles);
+  auto* kernel = perm ? gptq_to_marlin_kernel<true> : gptq_to_marlin_kernel<false>;
+  kernel<<<blocks, 256, 0, st>>>(in, perm, out, (int)size_k, (int)size_n, (uint32_t)each, size_k * size_n / 8,
+                                (uint32_t)total);
+  return launch_status("gptq_to_marlin_kernel");
+}
+
+int launch_awq_to_marlin(const uint32_t* in, uint32_t* out, int64_t experts, int64_t size_k, int64_t size_n,
+                         hipStream_t st) {
+  const long each = (size_k / kMarlinTileK) * (size_n / kMarlinTileN), total = experts * each;
+  const int blocks = (int)((total + kRepackTiles - 1) / kRepackTiles);
+  awq_to_marlin_kernel<<<blocks, 256, 0, st>>>(in, out, (int)size_n, (uint32_t)each, size_k * size_n / 8,
+                                              (uint32_t)total);
+  return launch_status("awq_to_marlin_kernel");
 }
 
 }  // namespace
@@ -409,14 +578,7 @@ extern "C" int sonar_gptq_marlin_repack(const uint32_t* b_q_weight, const int32_
                                                                     (int)size_n, words);
     return launch_status("gptq8_to_marlin_kernel");
   }
-  const long total = size_k * size_n / 8;
-  if (perm)
-    gptq_to_marlin_kernel<true><<<grid_for(total), 256, 0, st>>>(b_q_weight, perm, out, (int)size_k,
-                                                                (int)size_n, total);
-  else
-    gptq_to_marlin_kernel<false><<<grid_for(total), 256, 0, st>>>(b_q_weight, nullptr, out,
-                                                                 (int)size_k, (int)size_n, total);
-  return launch_status("gptq_to_marlin_kernel");
+  return launch_gptq_to_marlin(b_q_weight, perm, out, 1, size_k, size_n, st);
 }
 
 extern "C" int sonar_awq_marlin_repack(const uint32_t* b_q_weight, uint32_t* out, int64_t size_k,
@@ -424,10 +586,24 @@ extern "C" int sonar_awq_marlin_repack(const uint32_t* b_q_weight, uint32_t* out
   if (int rc = check_repack_shape(size_k, size_n, num_bits)) return rc;
   if (num_bits != 4) return fail(SONAR_E_UNSUPPORTED, "awq_marlin_repack: 8-bit AWQ weights are not built");
   SONAR_REQUIRE(b_q_weight && out, "b_q_weight and out must not be NULL");
-  const long total = size_k * size_n / 8;
-  awq_to_marlin_kernel<<<grid_for(total), 256, 0, (hipStream_t)stream>>>(b_q_weight, out, (int)size_k,
-                                                                        (int)size_n, total);
-  return launch_status("awq_to_marlin_kernel");
+  return launch_awq_to_marlin(b_q_weight, out, 1, size_k, size_n, (hipStream_t)stream);
+}
+
+// The stacked forms: matrix e at b_q_weight + e * K * N / 8 words (perm + e * K), one launch for all of them.
+extern "C" int sonar_gptq_marlin_moe_repack(const uint32_t* b_q_weight, const int32_t* perm, uint32_t* out,
+                                            int64_t experts, int64_t size_k, int64_t size_n, void* stream) {
+  if (int rc = check_repack_shape(size_k, size_n, 4)) return rc;
+  if (int rc = check_experts(experts, size_k, size_n)) return rc;
+  SONAR_REQUIRE(b_q_weight && out, "b_q_weight and out must not be NULL");
+  return launch_gptq_to_marlin(b_q_weight, perm, out, experts, size_k, size_n, (hipStream_t)stream);
+}
+
+extern "C" int sonar_awq_marlin_moe_repack(const uint32_t* b_q_weight, uint32_t* out, int64_t experts,
+                                           int64_t size_k, int64_t size_n, void* stream) {
+  if (int rc = check_repack_shape(size_k, size_n, 4)) return rc;
+  if (int rc = check_experts(experts, size_k, size_n)) return rc;
+  SONAR_REQUIRE(b_q_weight && out, "b_q_weight and out must not be NULL");
+  return launch_awq_to_marlin(b_q_weight, out, experts, size_k, size_n, (hipStream_t)stream);
 }
 
 extern "C" int sonar_marlin_to_gfx950(const uint32_t* marlin, uint32_t* out, int64_t size_k,
@@ -549,4 +725,58 @@ extern "C" int sonar_marlin_int4_fp8_preprocess(const uint32_t* qweight, const u
   int4_fp8_preprocess_kernel<<<grid_for(total), 256, 0, (hipStream_t)stream>>>(qweight, qzeros, out, words_per_row,
                                                                               (int)group_size, total);
   return launch_status("int4_fp8_preprocess_kernel");
+}
+
+// ---- checkpoint tensors around the codes -----------------------------------
+namespace {
+int blocks_of(int64_t items) { return (int)((items + 255) / 256); }
+}  // namespace
+
+extern "C" int sonar_marlin_permute_scales(const void* in, void* out, int64_t numel, int grouped, void* stream) {
+  SONAR_REQUIRE(numel >= 0 && numel % (grouped ? 64 : 32) == 0 && numel < (1LL << 38),
+                "the number of scales = %ld must be a multiple of %d", (long)numel, grouped ? 64 : 32);
+  if (numel == 0) return SONAR_OK;
+  SONAR_REQUIRE(in && out && in != out, "in and out must be distinct non-NULL buffers");
+  SONAR_REQUIRE((uintptr_t)out % 16 == 0, "out must be 16-byte aligned");
+  auto* kernel = grouped ? permute_scale_columns<true> : permute_scale_columns<false>;
+  kernel<<<blocks_of(numel / 8), 256, 0, (hipStream_t)stream>>>(static_cast<const uint16_t*>(in),
+                                                               static_cast<uint16_t*>(out), numel / 8);
+  return launch_status("permute_scale_columns");
+}
+
+extern "C" int sonar_marlin_pack_zero_points(const uint32_t* in, uint32_t* out, int64_t rows, int64_t size_n,
+                                             int64_t row_stride, int64_t word_stride, int awq_order, int is_a_8bit,
+                                             void* stream) {
+  SONAR_REQUIRE(rows >= 0 && size_n > 0 && size_n % 64 == 0 && size_n < (1LL << 30),
+                "size_n = %ld is not a positive multiple of 64", (long)size_n);
+  const int64_t total = rows * (size_n / 8);
+  SONAR_REQUIRE(total < (1LL << 38), "too many zero points");
+  if (total == 0) return SONAR_OK;
+  SONAR_REQUIRE(in && out && in != out, "in and out must be distinct non-NULL buffers");
+  pack_zero_points<<<blocks_of(total), 256, 0, (hipStream_t)stream>>>(in, out, (int)(size_n / 8), total, row_stride,
+                                                                     word_stride, awq_order != 0, is_a_8bit != 0);
+  return launch_status("pack_zero_points");
+}
+
+extern "C" int sonar_awq_to_gptq(const uint32_t* in, uint32_t* out, int64_t size_k, int64_t size_n, void* stream) {
+  SONAR_REQUIRE(size_k >= 0 && size_n > 0 && size_k % 8 == 0 && size_n % 8 == 0 && size_n < (1LL << 30) &&
+                    size_k < (1LL << 30), "size_k = %ld and size_n = %ld must be multiples of 8", (long)size_k, (long)size_n);
+  const int64_t total = size_k / 8 * (size_n / 8);
+  SONAR_REQUIRE(total < (1LL << 38), "weight too large");
+  if (total == 0) return SONAR_OK;
+  SONAR_REQUIRE(in && out && in != out, "in and out must be distinct non-NULL buffers");
+  awq_codes_to_gptq<<<blocks_of(total), 256, 0, (hipStream_t)stream>>>(in, out, (int)(size_n / 8), total);
+  return launch_status("awq_codes_to_gptq");
+}
+
+extern "C" int sonar_awq_zeros_to_plain(const uint32_t* in, uint32_t* out, int64_t groups, int64_t size_n,
+                                        void* stream) {
+  SONAR_REQUIRE(groups >= 0 && size_n > 0 && size_n % 8 == 0 && size_n < (1LL << 30) && groups < (1LL << 30),
+                "size_n = %ld must be a positive multiple of 8", (long)size_n);
+  const int64_t total = groups * (size_n / 8);
+  SONAR_REQUIRE(total < (1LL << 38), "too many zero points");
+  if (total == 0) return SONAR_OK;
+  SONAR_REQUIRE(in && out && in != out, "in and out must be distinct non-NULL buffers");
+  awq_zeros_to_plain<<<blocks_of(total), 256, 0, (hipStream_t)stream>>>(in, out, (int)groups, (int)(size_n / 8), total);
+  return launch_status("awq_zeros_to_plain");
 }

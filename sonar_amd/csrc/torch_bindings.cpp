@@ -372,6 +372,88 @@ Tensor awq_marlin_repack(const Tensor& b_q_weight, int64_t size_k, int64_t size_
   return out;
 }
 
+// Stacked 4-bit matrices (E, ...) in one launch; the loops of gptq_marlin_moe_repack and
+// awq_marlin_moe_repack (aphrodite/_custom_ops.py:1424-1461) copy every expert's result once more.
+Tensor moe_repack(const Tensor& b_q_weight, const OptTensor& perm, int64_t size_k, int64_t size_n, bool awq) {
+  TORCH_CHECK(size_k % 16 == 0, "size_k = ", size_k, " is not divisible by tile_k_size = ", 16);
+  TORCH_CHECK(size_n % 64 == 0, "size_n = ", size_n, " is not divisible by tile_n_size = ", 64);
+  TORCH_CHECK(b_q_weight.is_cuda() && b_q_weight.is_contiguous() && b_q_weight.scalar_type() == at::kInt,
+              "b_q_weight must be a contiguous int32 GPU tensor");
+  TORCH_CHECK(b_q_weight.dim() == 3 && b_q_weight.size(1) == (awq ? size_k : size_k / 8) &&
+                  b_q_weight.size(2) == (awq ? size_n / 8 : size_n),
+              "Shape mismatch: b_q_weight is ", b_q_weight.sizes(), ", size_k = ", size_k, ", size_n = ", size_n);
+  const int64_t experts = b_q_weight.size(0);
+  const bool has_perm = perm.has_value() && perm->numel() > 0;
+  if (has_perm) {
+    TORCH_CHECK(perm->is_cuda() && perm->is_contiguous() && perm->scalar_type() == at::kInt,
+                "perm must be a contiguous int32 GPU tensor");
+    TORCH_CHECK(perm->dim() == 2 && perm->size(0) == experts && perm->size(1) == size_k, "perm must be (E, size_k)");
+  }
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(b_q_weight.device());
+  Tensor out = at::empty({experts, size_k / 16, size_n * 2}, b_q_weight.options());
+  if (experts == 0) return out;
+  const uint32_t* src = static_cast<const uint32_t*>(b_q_weight.const_data_ptr());
+  uint32_t* dst = static_cast<uint32_t*>(out.mutable_data_ptr());
+  raise_if_failed(awq ? sonar_awq_marlin_moe_repack(src, dst, experts, size_k, size_n, current_stream(b_q_weight))
+                      : sonar_gptq_marlin_moe_repack(
+                            src, has_perm ? static_cast<const int32_t*>(perm->const_data_ptr()) : nullptr, dst, experts,
+                            size_k, size_n, current_stream(b_q_weight)));
+  forget_memory_of(out);
+  return out;
+}
+Tensor gptq_marlin_moe_repack(const Tensor& b_q_weight, const Tensor& perm, int64_t size_k, int64_t size_n) {
+  return moe_repack(b_q_weight, perm, size_k, size_n, false);
+}
+Tensor awq_marlin_moe_repack(const Tensor& b_q_weight, int64_t size_k, int64_t size_n) {
+  return moe_repack(b_q_weight, std::nullopt, size_k, size_n, true);
+}
+
+// The column order of marlin_permute_scales / marlin_permute_bias on 16-bit elements.
+Tensor permute_scales(const Tensor& s, bool grouped) {
+  TORCH_CHECK(s.is_cuda() && s.is_contiguous() && s.element_size() == 2, "s must be a contiguous 16-bit GPU tensor");
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(s.device());
+  Tensor out = at::empty_like(s);
+  raise_if_failed(sonar_marlin_permute_scales(s.const_data_ptr(), out.mutable_data_ptr(), s.numel(), grouped ? 1 : 0,
+                                              current_stream(s)));
+  return out;
+}
+
+// Zero points packed along N ((..., G, N/8), or (N/8, G) with `transposed`) -> Marlin zero points (..., G, N/8).
+Tensor pack_zero_points(const Tensor& zp, bool awq_order, bool transposed, bool is_a_8bit) {
+  TORCH_CHECK(zp.is_cuda() && zp.is_contiguous() && zp.scalar_type() == at::kInt && zp.dim() >= 2,
+              "zero points must be a contiguous int32 GPU tensor");
+  TORCH_CHECK(!transposed || zp.dim() == 2, "transposed zero points must be (N/8, G)");
+  const int64_t words = transposed ? zp.size(0) : zp.size(-1);
+  const int64_t rows = words ? zp.numel() / words : 0;
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(zp.device());
+  Tensor out = transposed ? at::empty({rows, words}, zp.options()) : at::empty_like(zp);
+  raise_if_failed(sonar_marlin_pack_zero_points(
+      static_cast<const uint32_t*>(zp.const_data_ptr()), static_cast<uint32_t*>(out.mutable_data_ptr()), rows,
+      words * 8, transposed ? 1 : words, transposed ? rows : 1, awq_order ? 1 : 0, is_a_8bit ? 1 : 0,
+      current_stream(zp)));
+  return out;
+}
+
+// AutoAWQ codes and zero points -> the GPTQ-like packing: ((K/8, N), (N/8, G)).
+std::tuple<Tensor, Tensor> awq_to_standard(const Tensor& qweight, const Tensor& qzeros) {
+  for (const Tensor* t : {&qweight, &qzeros})
+    TORCH_CHECK(t->is_cuda() && t->is_contiguous() && t->scalar_type() == at::kInt && t->dim() == 2,
+                "AWQ tensors must be contiguous two-dimensional int32 GPU tensors");
+  TORCH_CHECK(qweight.size(0) % 8 == 0, "AWQ weights have ", qweight.size(0), " rows, not a multiple of 8");
+  TORCH_CHECK(qweight.size(1) == qzeros.size(1), "AWQ weights and zero points differ in their columns");
+  const int64_t k = qweight.size(0), words = qweight.size(1), groups = qzeros.size(0);
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(qweight.device());
+  Tensor codes = at::empty({k / 8, words * 8}, qweight.options());
+  Tensor zeros = at::empty({words, groups}, qzeros.options());
+  raise_if_failed(sonar_awq_to_gptq(static_cast<const uint32_t*>(qweight.const_data_ptr()),
+                                    static_cast<uint32_t*>(codes.mutable_data_ptr()), k, words * 8,
+                                    current_stream(qweight)));
+  raise_if_failed(sonar_awq_zeros_to_plain(static_cast<const uint32_t*>(qzeros.const_data_ptr()),
+                                           static_cast<uint32_t*>(zeros.mutable_data_ptr()), groups, words * 8,
+                                           current_stream(qzeros)));
+  return {codes, zeros};
+}
+
 Tensor marlin_to_gfx950(const Tensor& b_q_weight, int64_t size_k, int64_t size_n) {
   TORCH_CHECK(b_q_weight.is_cuda() && b_q_weight.is_contiguous() && b_q_weight.scalar_type() == at::kInt,
               "b_q_weight must be a contiguous int32 GPU tensor");
@@ -1120,6 +1202,11 @@ TORCH_LIBRARY(sonar_amd, m) {
   m.def("swiglustep_and_mul(Tensor! out, Tensor input, float limit=7.0) -> ()");
   m.def("moe_sum(Tensor input, Tensor! output) -> ()");
   m.def("per_token_quant_int8(Tensor x) -> (Tensor, Tensor)");
+  m.def("gptq_marlin_moe_repack(Tensor b_q_weight, Tensor perm, SymInt size_k, SymInt size_n) -> Tensor");
+  m.def("awq_marlin_moe_repack(Tensor b_q_weight, SymInt size_k, SymInt size_n) -> Tensor");
+  m.def("permute_scales(Tensor s, bool grouped) -> Tensor");
+  m.def("pack_zero_points(Tensor zp, bool awq_order, bool transposed, bool is_a_8bit) -> Tensor");
+  m.def("awq_to_standard(Tensor qweight, Tensor qzeros) -> (Tensor, Tensor)");
   m.def("per_token_quant_fp8(Tensor x) -> (Tensor, Tensor)");
 }
 TORCH_LIBRARY_IMPL(sonar_amd, CUDA, m) {
@@ -1133,6 +1220,11 @@ TORCH_LIBRARY_IMPL(sonar_amd, CUDA, m) {
   m.impl("swiglustep_and_mul", &swiglustep_and_mul);
   m.impl("moe_sum", &moe_sum);
   m.impl("per_token_quant_int8", &per_token_quant_int8);
+  m.impl("gptq_marlin_moe_repack", &gptq_marlin_moe_repack);
+  m.impl("awq_marlin_moe_repack", &awq_marlin_moe_repack);
+  m.impl("permute_scales", &permute_scales);
+  m.impl("pack_zero_points", &pack_zero_points);
+  m.impl("awq_to_standard", &awq_to_standard);
   m.impl("per_token_quant_fp8", &per_token_quant_fp8);
 }
 

@@ -39,6 +39,12 @@ def convert_awq_to_standard_format(layer, w_q_name: str = "qweight", w_zp_name: 
     if size_bits != 4:
         raise NotImplementedError("AWQ conversion: 4-bit only")
     qw = getattr(layer, w_q_name)
+    zeros = getattr(layer, w_zp_name)
+    if qw.is_cuda and zeros.is_cuda and qw.dtype == zeros.dtype == torch.int32:
+        codes, zeros = torch.ops.sonar_amd.awq_to_standard(qw.contiguous(), zeros.contiguous())
+        setattr(layer, w_q_name, codes)
+        setattr(layer, w_zp_name, zeros)
+        return
     shifts = 4 * torch.tensor(_AWQ_SLOT_OF_COLUMN, dtype=torch.int32, device=qw.device)
     plain = 4 * torch.arange(8, dtype=torch.int32, device=qw.device)
 
@@ -116,6 +122,19 @@ class MarlinLinearKernel:
                            f"by group_size = {c.group_size}.")
         return True, None
 
+    def _zero_points_by_torch(self, zp: torch.Tensor, size_n: int, size_k: int, padded_n: int, padded_k: int,
+                              is_a_8bit: bool) -> torch.Tensor:
+        """Zero points that are unpacked, need padding or are not on the GPU."""
+        c = self.config
+        grouped_k = size_k // c.group_size if c.group_size != -1 else 1
+        padded_grouped_k = padded_k // c.group_size if c.group_size != -1 else 1
+        if zp.shape == (size_n // 8, grouped_k) and grouped_k != size_n // 8:
+            zp = zp.t().contiguous()      # packed along N and transposed (the converted AWQ form)
+        if zp.shape == (grouped_k, size_n // 8):
+            zp = unpack_cols(zp, c.weight_type.size_bits, grouped_k, size_n)
+        zp = marlin_pad_scales(zp, size_n, size_k, padded_n, padded_k, c.group_size)
+        return marlin_zero_points(zp, padded_grouped_k, padded_n, c.weight_type.size_bits, is_a_8bit=is_a_8bit)
+
     def process_weights_after_loading(self, layer) -> None:
         c = self.config
         device = getattr(layer, self.w_q_name).device
@@ -149,16 +168,15 @@ class MarlinLinearKernel:
 
         if c.zero_points:
             grouped_k = size_k // c.group_size if c.group_size != -1 else 1
-            padded_grouped_k = padded_k // c.group_size if c.group_size != -1 else 1
             zp = getattr(layer, self.w_zp_name)
-            if zp.shape == (size_n // 8, grouped_k) and grouped_k != size_n // 8:
-                zp = zp.t().contiguous()      # packed along N and transposed (the converted AWQ form)
-            if zp.shape == (grouped_k, size_n // 8):
-                zp = unpack_cols(zp, c.weight_type.size_bits, grouped_k, size_n)
-            zp = marlin_pad_scales(zp, size_n, size_k, padded_n, padded_k, c.group_size)
-            setattr(layer, self.w_zp_name,
-                    marlin_zero_points(zp, padded_grouped_k, padded_n, c.weight_type.size_bits,
-                                       is_a_8bit=is_a_8bit))
+            transposed = zp.shape == (size_n // 8, grouped_k) and grouped_k != size_n // 8
+            if ((transposed or zp.shape == (grouped_k, size_n // 8)) and (padded_n, padded_k) == (size_n, size_k)
+                    and size_n % 64 == 0 and c.weight_type.size_bits == 4 and zp.is_cuda
+                    and zp.dtype == torch.int32):
+                zp = torch.ops.sonar_amd.pack_zero_points(zp.contiguous(), False, transposed, is_a_8bit)
+            else:
+                zp = self._zero_points_by_torch(zp, size_n, size_k, padded_n, padded_k, is_a_8bit)
+            setattr(layer, self.w_zp_name, zp)
         else:
             setattr(layer, self.w_zp_name, marlin_make_empty_g_idx(device))
 

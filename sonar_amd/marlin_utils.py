@@ -242,10 +242,18 @@ def get_scale_perms():
     return scale_perm, scale_perm_single
 
 
+def _native_layout(t: torch.Tensor) -> bool:
+    """Whether the library's layout kernels take `t` (else the torch expressions below do)."""
+    return t.is_cuda and t.element_size() == 2 and t.numel() % 64 == 0 and not t.requires_grad
+
+
 def marlin_permute_scales(s: torch.Tensor, size_k: int, size_n: int, group_size: int,
                           is_a_8bit: bool = False) -> torch.Tensor:
+    grouped = group_size < size_k and group_size != -1 and not is_a_8bit
+    if _native_layout(s):
+        return torch.ops.sonar_amd.permute_scales(s.contiguous(), grouped).reshape((-1, size_n))
     scale_perm, scale_perm_single = get_scale_perms()
-    if group_size < size_k and group_size != -1 and not is_a_8bit:
+    if grouped:
         s = s.reshape((-1, len(scale_perm)))[:, scale_perm]
     else:
         s = s.reshape((-1, len(scale_perm_single)))[:, scale_perm_single]
@@ -253,6 +261,8 @@ def marlin_permute_scales(s: torch.Tensor, size_k: int, size_n: int, group_size:
 
 
 def marlin_permute_bias(s: torch.Tensor) -> torch.Tensor:
+    if _native_layout(s):
+        return torch.ops.sonar_amd.permute_scales(s.contiguous(), False)
     origin_shape = s.shape
     _, scale_perm_single = get_scale_perms()
     s = s.reshape((-1, len(scale_perm_single)))[:, scale_perm_single]
@@ -271,10 +281,12 @@ def marlin_act_int8_process_scales(s: torch.Tensor):
 
 def marlin_moe_permute_scales(s: torch.Tensor, size_k: int, size_n: int, group_size: int,
                               is_a_8bit: bool = False) -> torch.Tensor:
-    output = torch.empty_like(s)
-    for e in range(s.shape[0]):
-        output[e] = marlin_permute_scales(s[e], size_k, size_n, group_size, is_a_8bit)
-    return output
+    # the pattern repeats every 32 or 64 columns: the experts are so many more rows
+    return marlin_permute_scales(s, size_k, size_n, group_size, is_a_8bit).reshape(s.shape)
+
+
+def _packed_zero_points_on_gpu(zp: torch.Tensor, size_n: int) -> bool:
+    return zp.is_cuda and zp.dtype == torch.int32 and zp.is_contiguous() and zp.shape[-1] * 8 == size_n
 
 
 def marlin_zero_points(zp: torch.Tensor, size_k: int, size_n: int, num_bits: int,
@@ -292,6 +304,8 @@ def marlin_zero_points(zp: torch.Tensor, size_k: int, size_n: int, num_bits: int
 def awq_to_marlin_zero_points(q_zp_packed: torch.Tensor, size_k: int, size_n: int, num_bits: int,
                               is_a_8bit: bool = False) -> torch.Tensor:
     assert num_bits == 4
+    if _packed_zero_points_on_gpu(q_zp_packed, size_n) and q_zp_packed.shape[0] == size_k:
+        return torch.ops.sonar_amd.pack_zero_points(q_zp_packed, True, False, is_a_8bit)
     q_zp = unpack_cols(q_zp_packed, num_bits, size_k, size_n)
     undo = sorted(range(8), key=lambda i: _INTERLEAVE_4BIT[i])
     q_zp = q_zp.reshape((-1, 8))[:, undo].reshape((-1, size_n)).contiguous()
@@ -300,6 +314,8 @@ def awq_to_marlin_zero_points(q_zp_packed: torch.Tensor, size_k: int, size_n: in
 
 def moe_awq_to_marlin_zero_points(q_zp_packed: torch.Tensor, size_k: int, size_n: int, num_bits: int,
                                   is_a_8bit: bool = False) -> torch.Tensor:
+    if num_bits == 4 and _packed_zero_points_on_gpu(q_zp_packed, size_n):
+        return torch.ops.sonar_amd.pack_zero_points(q_zp_packed, True, False, is_a_8bit)
     output = torch.empty_like(q_zp_packed)
     for e in range(q_zp_packed.shape[0]):
         output[e] = awq_to_marlin_zero_points(q_zp_packed[e], size_k, size_n, num_bits, is_a_8bit)
@@ -311,6 +327,8 @@ def moe_packed_to_marlin_zero_points(q_zp_packed: torch.Tensor, size_k: int, siz
     """Per-expert zero points packed along columns in plain order (the
     compressed-tensors format, no AWQ interleave) to the op's layout
     (marlin_utils.py:538-559)."""
+    if num_bits == 4 and _packed_zero_points_on_gpu(q_zp_packed, size_n):
+        return torch.ops.sonar_amd.pack_zero_points(q_zp_packed, False, False, is_a_8bit)
     out = torch.empty_like(q_zp_packed)
     for e in range(q_zp_packed.shape[0]):
         out[e] = marlin_zero_points(unpack_cols(q_zp_packed[e], num_bits, size_k, size_n), size_k, size_n,

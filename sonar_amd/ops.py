@@ -54,6 +54,29 @@ def _register_fakes() -> None:
     reg("sonar_amd::per_token_quant_int8")(quant_fake(torch.int8))
     reg("sonar_amd::per_token_quant_fp8")(quant_fake(torch.float8_e4m3fn))
 
+    @reg("sonar_amd::gptq_marlin_moe_repack")
+    def _(b_q_weight, perm, size_k, size_n):
+        return torch.empty((b_q_weight.shape[0], size_k // 16, size_n * 2), dtype=b_q_weight.dtype,
+                           device=b_q_weight.device)
+
+    @reg("sonar_amd::awq_marlin_moe_repack")
+    def _(b_q_weight, size_k, size_n):
+        return torch.empty((b_q_weight.shape[0], size_k // 16, size_n * 2), dtype=b_q_weight.dtype,
+                           device=b_q_weight.device)
+
+    @reg("sonar_amd::permute_scales")
+    def _(s, grouped):
+        return torch.empty_like(s)
+
+    @reg("sonar_amd::pack_zero_points")
+    def _(zp, awq_order, transposed, is_a_8bit):
+        return zp.new_empty((zp.shape[1], zp.shape[0])) if transposed else torch.empty_like(zp)
+
+    @reg("sonar_amd::awq_to_standard")
+    def _(qweight, qzeros):
+        k, words = qweight.shape
+        return qweight.new_empty((k // 8, words * 8)), qzeros.new_empty((words, qzeros.shape[0]))
+
     @reg("_C::marlin_to_gfx950")
     def _(b_q_weight, size_k, size_n):
         return torch.empty_like(b_q_weight)
@@ -98,6 +121,8 @@ def gptq_marlin_moe_repack(b_q_weight: torch.Tensor, perm: torch.Tensor, size_k:
                            num_bits: int, is_a_8bit: bool = False) -> torch.Tensor:
     num_experts = b_q_weight.shape[0]
     assert size_k % 16 == 0
+    if num_bits == 4 and not is_a_8bit and b_q_weight.is_contiguous() and perm.is_contiguous():
+        return torch.ops.sonar_amd.gptq_marlin_moe_repack(b_q_weight, perm, size_k, size_n)
     output = torch.empty((num_experts, size_k // 16, size_n * (num_bits // 2)),
                          device=b_q_weight.device, dtype=b_q_weight.dtype)
     for e in range(num_experts):
@@ -109,6 +134,8 @@ def awq_marlin_moe_repack(b_q_weight: torch.Tensor, perm: torch.Tensor, size_k: 
                           num_bits: int, is_a_8bit: bool = False) -> torch.Tensor:
     num_experts = b_q_weight.shape[0]
     assert size_k % 16 == 0
+    if num_bits == 4 and not is_a_8bit and b_q_weight.is_contiguous():
+        return torch.ops.sonar_amd.awq_marlin_moe_repack(b_q_weight, size_k, size_n)
     output = torch.empty((num_experts, size_k // 16, size_n * (num_bits // 2)),
                          device=b_q_weight.device, dtype=b_q_weight.dtype)
     for e in range(num_experts):
