@@ -1436,43 +1436,67 @@ __global__ __launch_bounds__(256) void moe_tile_reduce_kernel(const TileParams p
 // Builds the row-tile table of a grouped call: runs of blocks with the same
 // expert are cut into tiles of up to four blocks.  With `table_small` the one or
 // two blocks a run ends in go there instead, to be computed as a 128-row tile at
-// half the cost.  One workgroup; expert_ids is staged in LDS and scanned by one
-// thread (a few hundred entries).
-__global__ __launch_bounds__(256) void moe_tile_table_kernel(const int32_t* __restrict__ expert_ids,
-                                                            const int32_t* __restrict__ num_post_pad,
-                                                            int num_blocks_max, int block_size, int num_experts,
-                                                            int32_t* __restrict__ table,
-                                                            int32_t* __restrict__ table_small, int max_tiles) {
-  extern __shared__ int32_t ids[];
-  int blocks = num_post_pad[0] / block_size;
-  if (blocks > num_blocks_max) blocks = num_blocks_max;
-  for (int b = threadIdx.x; b < blocks; b += blockDim.x) ids[b] = expert_ids[b];
-  __syncthreads();
-  if (threadIdx.x != 0) return;
-  int tiles = 0, small = 0;
-  int b = 0;
-  while (b < blocks) {
-    const int e = ids[b];
-    int run = 1;
-    while (b + run < blocks && ids[b + run] == e) ++run;
-    if (e >= 0 && e < num_experts) {
-      for (int at = 0; at < run; at += 4) {
-        const int n = min(4, run - at);
-        const bool to_small = table_small != nullptr && n <= 2;
-        int32_t* t = to_small ? table_small : table;
-        int& count = to_small ? small : tiles;
-        if (count < max_tiles) {
-          t[1 + 3 * count] = b + at;
-          t[2 + 3 * count] = n;
-          t[3 + 3 * count] = e;
-          ++count;
-        }
+// half the cost.  One workgroup, a thread per block of slots: where a block's run begins comes from a
+// ballot inside the wavefront and the other wavefronts' last run starts, a tile's number from counts of
+// the tile heads before it.  Latency bound (one thread scanning the blocks: 16 us at 157 blocks; 4 us so).
+constexpr int kTableThreads = 1024;
+constexpr int kTableWaves = kTableThreads / 64;
+__global__ __launch_bounds__(kTableThreads) void moe_tile_table_kernel(const int32_t* __restrict__ expert_ids,
+                                                                      const int32_t* __restrict__ num_post_pad,
+                                                                      int num_blocks_max, int block_size,
+                                                                      int num_experts, int32_t* __restrict__ table,
+                                                                      int32_t* __restrict__ table_small,
+                                                                      int max_tiles) {
+  __shared__ int32_t last_start[kTableWaves], heads[2][kTableWaves];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int blocks = min(num_post_pad[0] / block_size, num_blocks_max);
+  int run_carry = 0;          // where the run that reaches into this round of blocks begins
+  int count[2] = {0, 0};      // tiles so far: up to four blocks, and the small ones
+  for (int base = 0; base < blocks; base += kTableThreads) {
+    const int b = base + threadIdx.x;
+    const int e = b < blocks ? expert_ids[b] : -1;
+    const bool start = b < blocks && (b == 0 || expert_ids[b - 1] != e);
+    const unsigned long long starts = __ballot(start);
+    if (lane == 0) last_start[wave] = starts ? base + 64 * wave + 63 - __clzll(starts) : -1;
+    __syncthreads();
+    int run = run_carry;
+    for (int w = 0; w < kTableWaves; ++w) {
+      const int t = last_start[w];
+      if (t >= 0 && w < wave) run = t;
+      if (t >= 0) run_carry = t;
+    }
+    const unsigned long long upto = starts & (~0ull >> (63 - lane));
+    if (upto) run = base + 64 * wave + 63 - __clzll(upto);
+    const bool head = b < blocks && e >= 0 && e < num_experts && ((b - run) & 3) == 0;
+    int n = 1;
+    if (head)
+      while (n < 4 && b + n < blocks && expert_ids[b + n] == e) ++n;
+    const int small = table_small != nullptr && n <= 2;
+    const unsigned long long mask[2] = {__ballot(head && !small), __ballot(head && small)};
+    if (lane < 2) heads[lane][wave] = __popcll(mask[lane]);
+    __syncthreads();
+    int at[2] = {count[0], count[1]};
+    for (int w = 0; w < kTableWaves; ++w)
+      for (int i = 0; i < 2; ++i) {
+        const int t = heads[i][w];
+        if (w < wave) at[i] += t;
+        count[i] += t;
+      }
+    if (head) {
+      const int tile = at[small] + __popcll(mask[small] & ((1ull << lane) - 1ull));
+      if (tile < max_tiles) {
+        int32_t* t = (small ? table_small : table) + 1 + 3 * tile;
+        t[0] = b;
+        t[1] = n;
+        t[2] = e;
       }
     }
-    b += run;
+    __syncthreads();
   }
-  table[0] = tiles;
-  if (table_small != nullptr) table_small[0] = small;
+  if (threadIdx.x == 0) {
+    table[0] = min(count[0], max_tiles);
+    if (table_small != nullptr) table_small[0] = min(count[1], max_tiles);
+  }
 }
 
 template <typename T, bool HAS_ZP, bool G32>
@@ -1996,9 +2020,8 @@ int moe_tile_gemm(const void* a, void* c, const uint32_t* b, const void* bias, c
   const bool nvfp4 = fp4 && global_scale != nullptr;
   const bool two_sizes = wide && !no_small && !nvfp4 && (fp4 || !wide_groups_of_32(p));
   int32_t* table_small = two_sizes ? table + moe_one_table_bytes(sorted_len) / sizeof(int32_t) : nullptr;
-  moe_tile_table_kernel<<<1, 256, (size_t)blocks_max * sizeof(int32_t), st>>>(expert_ids, num_post_pad, blocks_max, 64,
-                                                                             (int)num_experts, table, table_small,
-                                                                             max_tiles);
+  moe_tile_table_kernel<<<1, kTableThreads, 0, st>>>(expert_ids, num_post_pad, blocks_max, 64, (int)num_experts, table,
+                                                     table_small, max_tiles);
   if (int rc = launch_status("moe_tile_table_kernel")) return rc;
   auto reduce = [&](const TileParams& q) -> int {
     if (q.partial == nullptr) return SONAR_OK;

@@ -9,38 +9,97 @@ namespace sonar {
 namespace {
 
 constexpr int kAlignThreads = 1024;
+constexpr int kAlignWaves = kAlignThreads / 64;
+// Experts up to which one workgroup counts and places: its wavefronts keep a histogram each (48 KiB of LDS).
+constexpr int kAlignOneLaunchExperts = 768;
 
-// One workgroup: per-expert counts, padded offsets, expert id of every block,
-// the padded total, and the sentinel fill of sorted_token_ids.  offsets[e] is
-// left for the placement kernel.
+// Inclusive sum over the lanes of a wavefront.
+__device__ __forceinline__ int wave_inclusive_sum(int v) {
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int up = __shfl_up(v, d, 64);
+    if ((int)(threadIdx.x & 63) >= d) v += up;
+  }
+  return v;
+}
+
+// One workgroup: per-expert counts, padded offsets, expert id of every block, the padded total and
+// the sentinels of sorted_token_ids.  With `place` it also places the slots: every wavefront owns
+// a contiguous share of them and a histogram row; the rows' prefix sums give each wavefront its first
+// position per expert, and inside 64 slots a lane's rank among the lanes of the same expert comes from
+// one ballot per bit of the expert number, so the slots of an expert keep ascending order.  Without it
+// (more experts than the histograms have room for) offsets[e] is left for the placement kernel.
+// Latency bound: 8000 slots on 32 experts 9 + 42 us as two launches whose second walked all slots once
+// per expert, 7 us like this.
 __global__ __launch_bounds__(kAlignThreads) void moe_align_count_kernel(
     const int32_t* __restrict__ topk_ids, int numel, int num_experts, int block_size,
     int32_t* __restrict__ sorted_ids, int sorted_len, int32_t* __restrict__ expert_ids, int expert_len,
-    int32_t* __restrict__ num_post_pad, const int32_t* __restrict__ expert_map, int32_t* __restrict__ offsets) {
-  extern __shared__ int32_t counts[];  // num_experts + 1 entries, then the padded prefix
-  int32_t* begin = counts + num_experts + 1;
-  for (int e = threadIdx.x; e <= num_experts; e += blockDim.x) counts[e] = 0;
+    int32_t* __restrict__ num_post_pad, const int32_t* __restrict__ expert_map, int32_t* __restrict__ offsets,
+    bool place) {
+  extern __shared__ int32_t lds[];     // begin[num_experts + 1], stop[num_experts], wave totals, the histogram rows
+  int32_t* begin = lds;
+  int32_t* stop = begin + num_experts + 1;   // where an expert's slots end and its padding begins
+  int32_t* wave_sum = stop + num_experts;
+  int32_t* hist = wave_sum + kAlignWaves;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int rows = place ? kAlignWaves : 1;
+  for (int i = tid; i < rows * num_experts; i += kAlignThreads) hist[i] = 0;
   __syncthreads();
-  for (int i = threadIdx.x; i < numel; i += blockDim.x) {
+  auto expert_of = [&](int i) {
     int e = topk_ids[i];
     if (e >= 0 && e < num_experts && expert_map) e = expert_map[e];
-    if (e >= 0 && e < num_experts) atomicAdd(&counts[e], 1);
+    return e >= 0 && e < num_experts ? e : -1;
+  };
+  // a wavefront's share: whole rounds of 64 slots
+  const int share = (((numel + kAlignWaves - 1) / kAlignWaves) + 63) / 64 * 64;
+  const int from = min(numel, wave * share), to = min(numel, from + share);
+  int32_t* mine = hist + (place ? wave * num_experts : 0);
+  for (int i = from + lane; i < to; i += 64) {
+    const int e = expert_of(i);
+    if (e >= 0) atomicAdd(&mine[e], 1);
   }
-  for (int i = threadIdx.x; i < sorted_len; i += blockDim.x) sorted_ids[i] = numel;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    int at = 0;
-    for (int e = 0; e < num_experts; ++e) {
-      begin[e] = at;
-      offsets[e] = at;
-      at += (counts[e] + block_size - 1) / block_size * block_size;
+  // padded run of every expert -> where it begins
+  int carry = 0;
+  for (int base = 0; base < num_experts; base += kAlignThreads) {
+    const int e = base + tid;
+    int count = 0, padded = 0;
+    if (e < num_experts) {
+      for (int r = 0; r < rows; ++r) {
+        const int c = hist[r * num_experts + e];
+        hist[r * num_experts + e] = count;   // slots of this expert in earlier shares
+        count += c;
+      }
+      padded = (count + block_size - 1) / block_size * block_size;
     }
-    begin[num_experts] = at;
-    num_post_pad[0] = at;
+    const int incl = wave_inclusive_sum(padded);
+    if (lane == 63) wave_sum[wave] = incl;
+    __syncthreads();
+    int before = carry;
+    for (int w = 0; w < kAlignWaves; ++w) {
+      const int t = wave_sum[w];
+      if (w < wave) before += t;
+      carry += t;
+    }
+    if (e < num_experts) {
+      begin[e] = before + incl - padded;
+      stop[e] = begin[e] + count;
+    }
+    __syncthreads();
+  }
+  const int total = carry;
+  if (tid == 0) {
+    begin[num_experts] = total;
+    num_post_pad[0] = total;
   }
   __syncthreads();
-  const int total = begin[num_experts];
-  for (int b = threadIdx.x; b < expert_len; b += blockDim.x) {
+  // sentinels: behind every expert's slots and behind the last run
+  for (int e = wave; e < num_experts; e += kAlignWaves)
+    for (int i = stop[e] + lane; i < begin[e + 1]; i += 64) sorted_ids[i] = numel;
+  for (int i = total + tid; i < sorted_len; i += kAlignThreads) sorted_ids[i] = numel;
+  if (!place)
+    for (int e = tid; e < num_experts; e += kAlignThreads) offsets[e] = begin[e];
+  for (int b = tid; b < expert_len; b += kAlignThreads) {
     const int start = b * block_size;
     int e = -1;
     if (start < total) {
@@ -53,6 +112,25 @@ __global__ __launch_bounds__(kAlignThreads) void moe_align_count_kernel(
       e = lo;
     }
     expert_ids[b] = e;
+  }
+  if (!place) return;
+  const int bits = 32 - __clz(num_experts);   // the number of experts itself stands for "none"
+  for (int base = from; base < to; base += 64) {
+    const int i = base + lane;
+    int e = i < to ? expert_of(i) : -1;
+    if (e < 0) e = num_experts;
+    unsigned long long same = ~0ull;
+    for (int bit = 0; bit < bits; ++bit) {
+      const bool set = (e >> bit) & 1;
+      const unsigned long long m = __ballot(set);
+      same &= set ? m : ~m;
+    }
+    if (e < num_experts) {
+      const int at = mine[e];   // read by every lane of the expert before its last one moves it on
+      sorted_ids[begin[e] + at + __popcll(same & ((1ull << lane) - 1ull))] = i;
+      if ((same >> lane) == 1ull) mine[e] = at + __popcll(same);
+    }
+    __builtin_amdgcn_wave_barrier();
   }
 }
 
@@ -264,13 +342,14 @@ extern "C" int sonar_moe_align_block_size(const int32_t* topk_ids, int64_t numel
   SONAR_REQUIRE(sorted_token_ids && expert_ids && num_tokens_post_pad && offsets_scratch && (topk_ids || numel == 0),
                 "moe_align_block_size: NULL argument");
   hipStream_t st = (hipStream_t)stream;
-  const size_t lds = (size_t)(2 * num_experts + 2) * sizeof(int32_t);
+  const bool place = num_experts <= kAlignOneLaunchExperts;
+  const size_t lds = (size_t)(2 * num_experts + 1 + kAlignWaves + (place ? kAlignWaves : 1) * num_experts) * sizeof(int32_t);
   moe_align_count_kernel<<<1, kAlignThreads, lds, st>>>(topk_ids, (int)numel, (int)num_experts, (int)block_size,
                                                         sorted_token_ids, (int)sorted_len, expert_ids,
                                                         (int)expert_len, num_tokens_post_pad, expert_map,
-                                                        offsets_scratch);
+                                                        offsets_scratch, place);
   if (int rc = launch_status("moe_align_count_kernel")) return rc;
-  if (numel > 0) {
+  if (numel > 0 && !place) {
     moe_align_place_kernel<<<(int)((num_experts + 3) / 4), 256, 0, st>>>(topk_ids, (int)numel, (int)num_experts,
                                                                          sorted_token_ids, expert_map,
                                                                          offsets_scratch);

@@ -903,23 +903,23 @@ Tensor moe_wna16_marlin_gemm_a8(const Tensor& a, const OptTensor& c_or_none, con
   return c;
 }
 
-Tensor moe_wna16_marlin_gemm(
-    Tensor& a, const OptTensor& c_or_none, Tensor& b_q_weight, const OptTensor& b_bias_or_none,
-    Tensor& b_scales, const OptTensor& a_scales, const OptTensor& global_scale,
-    const OptTensor& b_zeros_or_none, const OptTensor& g_idx_or_none, const OptTensor& perm_or_none,
-    Tensor& workspace, const Tensor& sorted_token_ids, Tensor& expert_ids,
-    Tensor& num_tokens_past_padded, Tensor& topk_weights, int64_t moe_block_size, int64_t top_k,
-    bool mul_topk_weights, int64_t b_type_id, int64_t size_m, int64_t size_n, int64_t size_k,
-    bool is_k_full, bool use_atomic_add, bool use_fp32_reduce, bool is_zp_float, int64_t thread_k,
-    int64_t thread_n, int64_t blocks_per_sm) {
-  (void)thread_k;
-  (void)thread_n;
-  (void)blocks_per_sm;
-  if (a.scalar_type() == at::kChar || a.scalar_type() == at::kFloat8_e4m3fn)
-    return moe_wna16_marlin_gemm_a8(a, c_or_none, b_q_weight, b_bias_or_none, b_scales, a_scales, global_scale,
-                                    b_zeros_or_none, g_idx_or_none, sorted_token_ids, expert_ids,
-                                    num_tokens_past_padded, topk_weights, moe_block_size, top_k, mul_topk_weights,
-                                    b_type_id, size_m, size_n, size_k, is_zp_float);
+// How the slots of a grouped call are routed (device pointers; checked by whoever fills it in).
+struct Routing {
+  const int32_t* sorted_ids;
+  int64_t sorted_len;
+  const int32_t* expert_ids;
+  const int32_t* past_padded;
+  const float* topk_weights;
+};
+
+// The grouped GEMM on 16-bit activations: checks of a and the expert matrices, and the launch into
+// `c` (size_m * top_k rows of a's type).  The kernels take no workspace.
+void moe_gemm_16bit(const Tensor& a, void* c, const Tensor& b_q_weight, const OptTensor& b_bias_or_none,
+                    const Tensor& b_scales, const OptTensor& a_scales, const OptTensor& global_scale,
+                    const OptTensor& b_zeros_or_none, const OptTensor& g_idx_or_none, const OptTensor& perm_or_none,
+                    const Routing& route, int64_t moe_block_size, int64_t top_k, bool mul_topk_weights,
+                    int64_t b_type_id, int64_t size_m, int64_t size_n, int64_t size_k, bool is_k_full,
+                    bool use_atomic_add, bool use_fp32_reduce, bool is_zp_float) {
   TORCH_CHECK(a.scalar_type() == at::kHalf || a.scalar_type() == at::kBFloat16, "unsupported `a` scalar_type");
   const int dtype = dtype_code(a);
   check_b_type(b_type_id);
@@ -973,20 +973,6 @@ Tensor moe_wna16_marlin_gemm(
   }
   const int64_t num_groups = b_scales.size(1);
 
-  c10::hip::HIPGuardMasqueradingAsCUDA guard(a.device());
-  Tensor c;
-  if (c_or_none.has_value()) {
-    c = c_or_none.value();
-    TORCH_CHECK(c.is_cuda() && c.is_contiguous(), "c is not a contiguous GPU tensor");
-    TORCH_CHECK(c.size(0) == size_m * top_k, "Shape mismatch: c.size(0) = ", c.size(0),
-                ", size_m * topk = ", size_m * top_k);
-    TORCH_CHECK(c.size(1) == size_n, "Shape mismatch: c.size(1) = ", c.size(1), ", size_n = ", size_n);
-    TORCH_CHECK(c.scalar_type() == a.scalar_type(), "c must have the dtype of a");
-  } else {
-    c = at::empty({size_m * top_k, size_n}, a.options());
-  }
-  if (size_m == 0) return c;
-
   const int32_t* g_idx = nullptr;
   const int32_t* perm = nullptr;
   if (g_idx_or_none.has_value() && perm_or_none.has_value() && g_idx_or_none->size(-1) > 0) {
@@ -1018,54 +1004,93 @@ Tensor moe_wna16_marlin_gemm(
     TORCH_CHECK(b_type_id != SONAR_TYPE_UINT4,
                 "b_type must be uint4b8, uint8b128 or float8_e4m3fn when has_zp = False. Got = uint4");
   }
-  TORCH_CHECK(sorted_token_ids.is_cuda() && sorted_token_ids.scalar_type() == at::kInt &&
-                  sorted_token_ids.is_contiguous(), "sorted_token_ids must be a contiguous int32 GPU tensor");
-  TORCH_CHECK(expert_ids.is_cuda() && expert_ids.scalar_type() == at::kInt && expert_ids.is_contiguous(),
-              "expert_ids must be a contiguous int32 GPU tensor");
-  TORCH_CHECK(num_tokens_past_padded.is_cuda() && num_tokens_past_padded.scalar_type() == at::kInt,
-              "num_tokens_past_padded must be an int32 GPU tensor");
-  TORCH_CHECK(topk_weights.is_cuda() && topk_weights.scalar_type() == at::kFloat &&
-                  topk_weights.is_contiguous(), "topk_weights must be a contiguous float32 GPU tensor");
-  TORCH_CHECK(workspace.is_cuda() && workspace.scalar_type() == at::kInt && workspace.is_contiguous(),
-              "workspace must be a contiguous int32 GPU tensor");
+  if (size_m == 0) return;
 
   Tensor native = native_weights(b_q_weight, size_k, size_n, experts, bits);
   size_t scratch_bytes =
-      sonar_moe_marlin_gemm_scratch_bytes(sorted_token_ids.numel(), moe_block_size, size_n, size_k);
+      sonar_moe_marlin_gemm_scratch_bytes(route.sorted_len, moe_block_size, size_n, size_k);
   // act-order: room for the column-permuted copy of A, one row per slot, behind the table of row tiles
   if (perm != nullptr)
-    scratch_bytes = ((scratch_bytes + 255) & ~(size_t)255) + (size_t)sorted_token_ids.numel() * size_k * 2;
+    scratch_bytes = ((scratch_bytes + 255) & ~(size_t)255) + (size_t)route.sorted_len * size_k * 2;
   Tensor scratch;
   if (scratch_bytes > 0) scratch = at::empty({(int64_t)scratch_bytes}, a.options().dtype(at::kByte));
 
   if (nvfp4) {
     TORCH_CHECK(perm == nullptr, "act-order is not supported with float4_e2m1f weights");
     raise_if_failed(sonar_moe_wna16_marlin_gemm_nvfp4(
-        a.const_data_ptr(), c.mutable_data_ptr(), static_cast<const uint32_t*>(native.const_data_ptr()),
+        a.const_data_ptr(), c, static_cast<const uint32_t*>(native.const_data_ptr()),
         SONAR_LAYOUT_GFX950, opt_ptr(b_bias_or_none),
         nvfp4_scales_as_16bit(b_scales, a.scalar_type()).const_data_ptr(),
         static_cast<const float*>(global_scale->const_data_ptr()),
         scratch_bytes > 0 ? scratch.mutable_data_ptr() : nullptr, scratch_bytes,
-        static_cast<const int32_t*>(sorted_token_ids.const_data_ptr()), sorted_token_ids.numel(),
-        static_cast<const int32_t*>(expert_ids.const_data_ptr()),
-        static_cast<const int32_t*>(num_tokens_past_padded.const_data_ptr()),
-        static_cast<const float*>(topk_weights.const_data_ptr()), moe_block_size, top_k, mul_topk_weights ? 1 : 0,
-        experts, dtype, size_m, size_n, size_k, num_groups, current_stream(a)));
-    return c;
+        route.sorted_ids, route.sorted_len, route.expert_ids, route.past_padded, route.topk_weights,
+        moe_block_size, top_k, mul_topk_weights ? 1 : 0, experts, dtype, size_m, size_n, size_k,
+        num_groups, current_stream(a)));
+    return;
   }
   raise_if_failed(sonar_moe_wna16_marlin_gemm(
-      a.const_data_ptr(), c.mutable_data_ptr(), static_cast<const uint32_t*>(native.const_data_ptr()),
+      a.const_data_ptr(), c, static_cast<const uint32_t*>(native.const_data_ptr()),
       SONAR_LAYOUT_GFX950, opt_ptr(b_bias_or_none),
       (fp4 || mxfp8 ? mx_scales_as_bf16(b_scales, mxfp8 ? 120 : 0) : b_scales).const_data_ptr(),
       has_zp ? static_cast<const uint32_t*>(b_zeros_or_none->const_data_ptr()) : nullptr, g_idx, perm,
-      static_cast<int32_t*>(workspace.mutable_data_ptr()), workspace.numel(),
-      scratch_bytes > 0 ? scratch.mutable_data_ptr() : nullptr, scratch_bytes,
-      static_cast<const int32_t*>(sorted_token_ids.const_data_ptr()),
-      sorted_token_ids.numel(), static_cast<const int32_t*>(expert_ids.const_data_ptr()),
-      static_cast<const int32_t*>(num_tokens_past_padded.const_data_ptr()),
-      static_cast<const float*>(topk_weights.const_data_ptr()), moe_block_size, top_k,
-      mul_topk_weights ? 1 : 0, experts, dtype, b_type_id, size_m, size_n, size_k, num_groups,
+      nullptr, 0, scratch_bytes > 0 ? scratch.mutable_data_ptr() : nullptr, scratch_bytes,
+      route.sorted_ids, route.sorted_len, route.expert_ids, route.past_padded, route.topk_weights,
+      moe_block_size, top_k, mul_topk_weights ? 1 : 0, experts, dtype, b_type_id, size_m, size_n, size_k, num_groups,
       is_k_full ? 1 : 0, use_atomic_add ? 1 : 0, use_fp32_reduce ? 1 : 0, current_stream(a)));
+}
+
+Tensor moe_wna16_marlin_gemm(
+    Tensor& a, const OptTensor& c_or_none, Tensor& b_q_weight, const OptTensor& b_bias_or_none,
+    Tensor& b_scales, const OptTensor& a_scales, const OptTensor& global_scale,
+    const OptTensor& b_zeros_or_none, const OptTensor& g_idx_or_none, const OptTensor& perm_or_none,
+    Tensor& workspace, const Tensor& sorted_token_ids, Tensor& expert_ids,
+    Tensor& num_tokens_past_padded, Tensor& topk_weights, int64_t moe_block_size, int64_t top_k,
+    bool mul_topk_weights, int64_t b_type_id, int64_t size_m, int64_t size_n, int64_t size_k,
+    bool is_k_full, bool use_atomic_add, bool use_fp32_reduce, bool is_zp_float, int64_t thread_k,
+    int64_t thread_n, int64_t blocks_per_sm) {
+  (void)thread_k;
+  (void)thread_n;
+  (void)blocks_per_sm;
+  if (a.scalar_type() == at::kChar || a.scalar_type() == at::kFloat8_e4m3fn)
+    return moe_wna16_marlin_gemm_a8(a, c_or_none, b_q_weight, b_bias_or_none, b_scales, a_scales, global_scale,
+                                    b_zeros_or_none, g_idx_or_none, sorted_token_ids, expert_ids,
+                                    num_tokens_past_padded, topk_weights, moe_block_size, top_k, mul_topk_weights,
+                                    b_type_id, size_m, size_n, size_k, is_zp_float);
+  TORCH_CHECK(a.scalar_type() == at::kHalf || a.scalar_type() == at::kBFloat16, "unsupported `a` scalar_type");
+  TORCH_CHECK(a.is_cuda(), "A is not a contiguous GPU tensor");
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(a.device());
+  Tensor c;
+  if (c_or_none.has_value()) {
+    c = c_or_none.value();
+    TORCH_CHECK(c.is_cuda() && c.is_contiguous(), "c is not a contiguous GPU tensor");
+    TORCH_CHECK(c.size(0) == size_m * top_k, "Shape mismatch: c.size(0) = ", c.size(0),
+                ", size_m * topk = ", size_m * top_k);
+    TORCH_CHECK(c.size(1) == size_n, "Shape mismatch: c.size(1) = ", c.size(1), ", size_n = ", size_n);
+    TORCH_CHECK(c.scalar_type() == a.scalar_type(), "c must have the dtype of a");
+  } else {
+    c = at::empty({size_m * top_k, size_n}, a.options());
+  }
+  if (size_m > 0) {
+    TORCH_CHECK(sorted_token_ids.is_cuda() && sorted_token_ids.scalar_type() == at::kInt &&
+                    sorted_token_ids.is_contiguous(), "sorted_token_ids must be a contiguous int32 GPU tensor");
+    TORCH_CHECK(expert_ids.is_cuda() && expert_ids.scalar_type() == at::kInt && expert_ids.is_contiguous(),
+                "expert_ids must be a contiguous int32 GPU tensor");
+    TORCH_CHECK(num_tokens_past_padded.is_cuda() && num_tokens_past_padded.scalar_type() == at::kInt,
+                "num_tokens_past_padded must be an int32 GPU tensor");
+    TORCH_CHECK(topk_weights.is_cuda() && topk_weights.scalar_type() == at::kFloat &&
+                    topk_weights.is_contiguous(), "topk_weights must be a contiguous float32 GPU tensor");
+    TORCH_CHECK(workspace.is_cuda() && workspace.scalar_type() == at::kInt && workspace.is_contiguous(),
+                "workspace must be a contiguous int32 GPU tensor");
+  }
+
+  moe_gemm_16bit(a, c.mutable_data_ptr(), b_q_weight, b_bias_or_none, b_scales, a_scales, global_scale,
+                 b_zeros_or_none, g_idx_or_none, perm_or_none,
+                 Routing{static_cast<const int32_t*>(sorted_token_ids.const_data_ptr()), sorted_token_ids.numel(),
+                         static_cast<const int32_t*>(expert_ids.const_data_ptr()),
+                         static_cast<const int32_t*>(num_tokens_past_padded.const_data_ptr()),
+                         static_cast<const float*>(topk_weights.const_data_ptr())},
+                 moe_block_size, top_k, mul_topk_weights, b_type_id, size_m, size_n, size_k, is_k_full,
+                 use_atomic_add, use_fp32_reduce, is_zp_float);
   return c;
 }
 
@@ -1150,6 +1175,74 @@ void moe_sum(const Tensor& input, Tensor& output) {
                                 input.size(2), dtype_code(input), current_stream(input)));
 }
 
+// The whole mixture-of-experts layer (marlin_moe.py:226-392 of the reference) for 16-bit activations:
+// routing, gate / up GEMM, gated activation, down GEMM, sum over a token's experts, in one call.  What
+// the Python form spends on a small layer is not the GPU's time but its own: five op calls, their
+// argument conversion and ten allocations (58 us at one token; 22 us this way).  `activation` 0 is
+// silu_and_mul, else a SONAR_ACT_* kind with its limit / alpha / beta.  `output` [M, K] is written;
+// cache13 (M * top_k * max(2N, K) values) and cache2 (M * top_k * N) are allocated when not given.
+void fused_moe(Tensor& output, const Tensor& hidden, const Tensor& w1, const Tensor& w2, const OptTensor& bias1,
+               const OptTensor& bias2, const Tensor& scale1, const Tensor& scale2, const OptTensor& global_scale1,
+               const OptTensor& global_scale2, const Tensor& topk_weights, const Tensor& topk_ids,
+               const OptTensor& g_idx1, const OptTensor& g_idx2, const OptTensor& perm1, const OptTensor& perm2,
+               const OptTensor& zeros1, const OptTensor& zeros2, const OptTensor& cache13, const OptTensor& cache2,
+               int64_t b_type_id, int64_t num_experts, int64_t block_size, bool router_weight_on_input,
+               bool is_k_full, int64_t activation, double limit, double alpha, double beta) {
+  TORCH_CHECK(hidden.is_cuda() && hidden.dim() == 2 && hidden.is_contiguous(), "hidden_states must be a contiguous "
+              "two-dimensional GPU tensor");
+  TORCH_CHECK(topk_ids.is_cuda() && topk_ids.dim() == 2 && topk_ids.is_contiguous() && topk_ids.scalar_type() == at::kInt,
+              "topk_ids must be a contiguous int32 GPU tensor");
+  TORCH_CHECK(topk_weights.is_cuda() && topk_weights.scalar_type() == at::kFloat && topk_weights.is_contiguous() &&
+                  topk_weights.numel() == topk_ids.numel(), "topk_weights must be a contiguous float32 GPU tensor of "
+              "topk_ids' size");
+  TORCH_CHECK(w2.dim() == 3, "w2 must be (E, N/16, 2K)");
+  const int64_t m = hidden.size(0), k = hidden.size(1), n = w2.size(1) * 16, topk = topk_ids.size(1);
+  TORCH_CHECK(topk_ids.size(0) == m, "topk_ids has ", topk_ids.size(0), " rows for ", m, " tokens");
+  TORCH_CHECK(output.is_cuda() && output.is_contiguous() && output.numel() == m * k &&
+                  output.scalar_type() == hidden.scalar_type(), "output must be a contiguous tensor like hidden_states");
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(hidden.device());
+  const int64_t rows = m * topk;
+  auto cache = [&](const OptTensor& given, int64_t values, const char* name) -> Tensor {
+    if (!given.has_value()) return at::empty({values}, hidden.options());
+    TORCH_CHECK(given->is_cuda() && given->is_contiguous() && given->numel() >= values &&
+                    given->scalar_type() == hidden.scalar_type(), name, " must be a contiguous tensor of at least ",
+                values, " values of hidden_states' type");
+    return *given;
+  };
+  Tensor between = cache2.has_value() ? cache(cache2, rows * n, "intermediate_cache2") : at::empty({rows, n}, hidden.options());
+  Tensor wide = cache(cache13, rows * std::max(2 * n, k), "intermediate_cache13");   // gate and up, then the rows of the down GEMM
+
+  // sorted ids | expert of each block | padded total | scratch of the routing kernel, 16-byte pieces
+  int64_t sorted_len = rows + num_experts * (block_size - 1);
+  if (rows < num_experts) sorted_len = std::min(rows * block_size, sorted_len);
+  const int64_t blocks = (sorted_len + block_size - 1) / block_size;
+  auto room = [](int64_t ints) { return (ints + 3) / 4 * 4; };
+  Tensor table = at::empty({room(sorted_len) + room(blocks) + 4 + num_experts}, topk_ids.options());
+  int32_t* sorted_ids = static_cast<int32_t*>(table.mutable_data_ptr());
+  int32_t* expert_ids = sorted_ids + room(sorted_len);
+  int32_t* past_padded = expert_ids + room(blocks);
+  void* stream = current_stream(hidden);
+  raise_if_failed(sonar_moe_align_block_size(static_cast<const int32_t*>(topk_ids.const_data_ptr()), rows, num_experts,
+                                             block_size, sorted_ids, sorted_len, expert_ids, blocks, past_padded,
+                                             nullptr, past_padded + 4, stream));
+  const Routing route{sorted_ids, sorted_len, expert_ids, past_padded,
+                      static_cast<const float*>(topk_weights.const_data_ptr())};
+  const int dtype = dtype_code(hidden);
+  moe_gemm_16bit(hidden, wide.mutable_data_ptr(), w1, bias1, scale1, std::nullopt, global_scale1, zeros1, g_idx1, perm1,
+                 route, block_size, topk, router_weight_on_input, b_type_id, m, 2 * n, k, is_k_full, false, true,
+                 false);
+  raise_if_failed(activation == 0
+                      ? sonar_silu_and_mul(between.mutable_data_ptr(), wide.const_data_ptr(), rows, n, dtype, stream)
+                      : sonar_moe_activation(between.mutable_data_ptr(), wide.const_data_ptr(), rows, n,
+                                             (int)activation, (float)limit, (float)alpha, (float)beta, dtype, stream));
+  const Tensor down_in = between.dim() == 2 && between.size(0) == rows && between.size(1) == n
+                             ? between
+                             : between.view({-1}).narrow(0, 0, rows * n).view({rows, n});
+  moe_gemm_16bit(down_in, wide.mutable_data_ptr(), w2, bias2, scale2, std::nullopt, global_scale2, zeros2, g_idx2, perm2,
+                 route, block_size, 1, !router_weight_on_input, b_type_id, rows, k, n, is_k_full, false, true, false);
+  raise_if_failed(sonar_moe_sum(output.mutable_data_ptr(), wide.const_data_ptr(), m, topk, k, dtype, stream));
+}
+
 // Per-token quantisation of the activations of the W4A8 GEMM: (codes of x's shape, float32
 // scales (..., 1)).
 std::tuple<Tensor, Tensor> per_token_quant(const Tensor& x, bool fp8) {
@@ -1201,6 +1294,12 @@ TORCH_LIBRARY(sonar_amd, m) {
   m.def("situ_and_mul(Tensor! out, Tensor input, float beta, float linear_beta) -> ()");
   m.def("swiglustep_and_mul(Tensor! out, Tensor input, float limit=7.0) -> ()");
   m.def("moe_sum(Tensor input, Tensor! output) -> ()");
+  m.def(
+      "fused_moe(Tensor(a!) output, Tensor hidden, Tensor w1, Tensor w2, Tensor? bias1, Tensor? bias2, Tensor scale1, "
+      "Tensor scale2, Tensor? global_scale1, Tensor? global_scale2, Tensor topk_weights, Tensor topk_ids, "
+      "Tensor? g_idx1, Tensor? g_idx2, Tensor? perm1, Tensor? perm2, Tensor? zeros1, Tensor? zeros2, "
+      "Tensor(b!)? cache13, Tensor(c!)? cache2, int b_type_id, int num_experts, int block_size, "
+      "bool router_weight_on_input, bool is_k_full, int activation, float limit, float alpha, float beta) -> ()");
   m.def("per_token_quant_int8(Tensor x) -> (Tensor, Tensor)");
   m.def("gptq_marlin_moe_repack(Tensor b_q_weight, Tensor perm, SymInt size_k, SymInt size_n) -> Tensor");
   m.def("awq_marlin_moe_repack(Tensor b_q_weight, SymInt size_k, SymInt size_n) -> Tensor");
@@ -1219,6 +1318,7 @@ TORCH_LIBRARY_IMPL(sonar_amd, CUDA, m) {
   m.impl("situ_and_mul", &situ_and_mul);
   m.impl("swiglustep_and_mul", &swiglustep_and_mul);
   m.impl("moe_sum", &moe_sum);
+  m.impl("fused_moe", &fused_moe);
   m.impl("per_token_quant_int8", &per_token_quant_int8);
   m.impl("gptq_marlin_moe_repack", &gptq_marlin_moe_repack);
   m.impl("awq_marlin_moe_repack", &awq_marlin_moe_repack);

@@ -6,7 +6,8 @@ Mirrors aphrodite/model_executor/layers/fused_moe/moe_align_block_size.py:11-101
 (`fused_marlin_moe`) for 4- and 8-bit integer, fp8 and MXFP4 weights with fp16 / bf16
 activations.
 On the GPU the routing, the activation and the final sum are the HIP kernels
-behind `torch.ops.sonar_amd.{moe_align_block_size, silu_and_mul, moe_sum}`; the
+behind `torch.ops.sonar_amd.{moe_align_block_size, silu_and_mul, moe_sum}`, and the
+whole layer with 16-bit activations is one call, `torch.ops.sonar_amd.fused_moe`; the
 torch expressions kept here serve CPU tensors (and the tests of those kernels).
 Neither reads a device value on the host, so the whole layer can be recorded
 in a HIP graph; the two GEMMs are the `_moe_C::moe_wna16_marlin_gemm` op.
@@ -266,6 +267,21 @@ def apply_moe_activation(activation, output: torch.Tensor, input: torch.Tensor, 
     return output
 
 
+def _native_activation(activation, clamp_limit, alpha, beta, situ_beta, situ_linear_beta):
+    """(kind, limit, alpha, beta) for torch.ops.sonar_amd.fused_moe: kind 0 is silu_and_mul, else the
+    library's number of the activation (SONAR_ACT_* in include/sonar_marlin.h); None where
+    apply_moe_activation has to decide (no gate, or arguments it refuses)."""
+    name = _activation_name(activation)
+    if name == "silu":
+        return (0, 0.0, 1.0, 0.0) if clamp_limit is None else (1, float(clamp_limit), 1.0, 0.0)
+    if name == "swigluoai_uninterleave" and clamp_limit is not None:
+        return 1, float(clamp_limit), float(alpha), float(beta)
+    if name == "situ" and situ_beta is not None:
+        return 5, 0.0, float(situ_beta), -1.0 if situ_linear_beta is None else float(situ_linear_beta)
+    return {"gelu": (2, 0.0, 1.0, 0.0), "gelu_tanh": (3, 0.0, 1.0, 0.0), "swigluoai": (4, 7.0, 1.702, 0.0),
+            "swiglustep": (6, 7.0, 1.0, 0.0)}.get(name)
+
+
 def _check_arguments(activation, input_dtype, global_scales) -> None:
     name = _activation_name(activation)
     if name not in _GATED + _NOT_GATED:
@@ -406,6 +422,24 @@ def fused_marlin_moe(hidden_states: torch.Tensor, w1: torch.Tensor, w2: torch.Te
     block_size_m = moe_block_size(m_est, topk, E)
     if input_dtype is not None and input_dtype.itemsize == 1:
         block_size_m = max(block_size_m, 16)             # marlin_moe.py:328-329
+    if (hidden_states.is_cuda and activation_func is None and moe_sum is None and expert_map is None
+            and (input_dtype is None or input_dtype.itemsize == 2) and K % 8 == 0
+            and (intermediate_cache13 is None or intermediate_cache13.is_contiguous())
+            and (intermediate_cache2 is None or intermediate_cache2.is_contiguous())
+            and (output is None or output.is_contiguous())):
+        kind = _native_activation(activation, clamp_limit, gemm1_alpha, gemm1_beta, activation_situ_beta,
+                                  activation_situ_linear_beta)
+        if kind is not None:
+            if output is None:
+                output = torch.empty_like(hidden_states)
+            ids = topk_ids if topk_ids.dtype == torch.int32 else topk_ids.to(torch.int32)
+            torch.ops.sonar_amd.fused_moe(
+                output, hidden_states, w1, w2, bias1, bias2, w1_scale, w2_scale, global_scale1, global_scale2,
+                topk_weights.contiguous(), ids.contiguous(), g_idx1, g_idx2, sort_indices1, sort_indices2, w1_zeros,
+                w2_zeros, intermediate_cache13, intermediate_cache2, quant_type_id, global_num_experts, block_size_m,
+                apply_router_weight_on_input, is_k_full, *kind)
+            return output
+
     sorted_token_ids, expert_ids, num_tokens_post_padded = moe_align_block_size(
         topk_ids, block_size_m, global_num_experts, expert_map, ignore_invalid_experts=True)
 

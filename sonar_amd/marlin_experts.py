@@ -166,16 +166,20 @@ class MarlinExperts(MarlinExpertsBase):
               apply_router_weight_on_input: bool):
         assert self.w1_scale is not None
         assert self.w2_scale is not None
+        # a subclass may replace either step; the package's own are fused_marlin_moe's defaults
+        own_activation = type(self).activation is MarlinExpertsBase.activation
+        own_sum = type(self).moe_sum is MarlinExperts.moe_sum
         fused_marlin_moe(
             hidden_states=hidden_states, w1=w1, w2=w2, bias1=self.w1_bias, bias2=self.w2_bias,
             w1_scale=self.w1_scale, w2_scale=self.w2_scale, topk_weights=topk_weights, topk_ids=topk_ids,
             global_scale1=self.g1_alphas, global_scale2=self.g2_alphas, input_global_scale1=self.a1_gscale,
             input_global_scale2=self.a2_gscale, w1_zeros=self.w1_zp, w2_zeros=self.w2_zp,
             quant_type_id=self.quant_type_id, apply_router_weight_on_input=apply_router_weight_on_input,
-            global_num_experts=global_num_experts, activation=activation, activation_func=self.activation,
+            global_num_experts=global_num_experts, activation=activation,
+            activation_func=None if own_activation else self.activation,
             activation_situ_beta=self.moe_config.activation_situ_beta,
             activation_situ_linear_beta=self.moe_config.activation_situ_linear_beta,
-            moe_sum=self.moe_sum, expert_map=expert_map, output=output,
+            moe_sum=None if own_sum else self.moe_sum, expert_map=expert_map, output=output,
             intermediate_cache13=workspace2, intermediate_cache2=workspace13,      # swapped: see workspace_shapes
             g_idx1=self.w13_g_idx, g_idx2=self.w2_g_idx, sort_indices1=self.w13_g_idx_sort_indices,
             sort_indices2=self.w2_g_idx_sort_indices, is_k_full=self.is_k_full, input_dtype=self.input_dtype,

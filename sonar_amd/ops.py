@@ -77,6 +77,12 @@ def _register_fakes() -> None:
         k, words = qweight.shape
         return qweight.new_empty((k // 8, words * 8)), qzeros.new_empty((words, qzeros.shape[0]))
 
+    @reg("sonar_amd::fused_moe")
+    def _(output, hidden, w1, w2, bias1, bias2, scale1, scale2, global_scale1, global_scale2, topk_weights, topk_ids,
+          g_idx1, g_idx2, perm1, perm2, zeros1, zeros2, cache13, cache2, b_type_id, num_experts, block_size,
+          router_weight_on_input, is_k_full, activation, limit, alpha, beta):
+        return None
+
     @reg("_C::marlin_to_gfx950")
     def _(b_q_weight, size_k, size_n):
         return torch.empty_like(b_q_weight)
