@@ -1,0 +1,429 @@
+// The GEMM between decode and prefill: from a few tens of rows up to where the tiles of the wide tile
+// kernel (gemm_tile.hip) fill the chip.  A workgroup owns 16 MB rows x 128 columns over the whole of K:
+// no partial tile goes through memory and no second launch sums them.
+//
+// Eight wavefronts: two strips of 64 columns x four ranges of K.  So every packed chunk is dequantised
+// exactly once in the workgroup, a wavefront's accumulators are small (16 MB registers), two wavefronts
+// share a SIMD (one's matrix instructions run beside the other's dequantisation), and the activations,
+// which the two strips share, are staged in LDS at half the bytes per matrix instruction of a one-strip
+// workgroup (at one strip the copies alone would need the whole 64 bytes per clock of a compute unit).
+//
+// What bounds it: issue slots of the vector unit.  Measured on this chip, a v_mfma_f32_16x16x32 takes 16 cycles of the
+// matrix pipe and 8 of the issue port when other vector instructions want it; those take 4.3 each (two-operand
+// logic, shifts and multiplies half of that).  A chunk (32 rows of a strip) costs 52 (fp16) to 68 (bf16) instructions
+// to dequantise and a few for its scales, beside 4 MB matrix instructions.  K = 4096, N = 8192, 64 rows, bf16:
+// 18.0 + 1.45 (MB - 2) us, of which about 6 are launch, first bytes and the sum over the ranges at the end.
+// Measured against the kernels it takes over from (us, before -> now):
+//   M   64, K 4096, N 28672, bf16: 29.1 -> 23.0      M  200, K 4096, N 6144, fp16, zero points: 24.6 -> 21.0
+//   M  333, K 2880, N  5760, bf16, groups of 32: 40.5 -> 21.7      M  512, K 4096, N 2048, bf16: 36 -> 20
+//   M  128, K 2048, N 20032, MXFP4: 47.6 -> 20.5     M   96, K 2048, N 20032, 8-bit codes: 48 -> 18.5
+// Tried and slower: one strip a workgroup with eight ranges (half the dequantisation per workgroup, but twice the
+// activation bytes through the copy path per matrix instruction: 200 rows above 23 us, 64 rows on N = 28672 31 us).
+//
+// Pipeline, per K step of 64 rows of each of the four ranges: the activations (LDS, copied by
+// LDS-DMA), two chunks of weights and the scales (registers) of step t + D - 1 are asked for during the
+// second half of step t, one operation behind a matrix instruction, and waited for in the middle of step
+// t + D - 2.  One barrier a step, in its middle: behind it stage t + 1 has landed for everyone and nobody
+// reads stage t - 1 any more, whose slot the copies of the second half fill.  The operands of the next half are
+// read behind the matrix instructions of their row block in this one, and each half dequantises the
+// chunk of the half after it, a pair of weights behind each matrix instruction (its last instruction one
+// matrix instruction later: the conversion to bf16 may not follow the multiply-adds at once).
+#include <algorithm>
+#include <cstdlib>
+#include <type_traits>
+#include <utility>
+
+#include "common.hpp"
+#include "dequant.hpp"
+#include "gemm_mid.hpp"
+
+namespace sonar {
+namespace {
+
+constexpr int kMidWaves = 8;
+constexpr int kMidStrips = 2;     // strips of a workgroup
+constexpr int kMidRanges = 4;     // ranges of K
+constexpr int kMidStepK = 64;     // rows of K a step takes from each range
+
+// Activation stages in LDS: MB x 8 KiB each.
+constexpr int mid_stages(int mb) { return mb <= 4 ? 4 : 3; }
+constexpr int mid_stage_bytes(int mb) { return mb * 8192; }
+constexpr int mid_sum_rows(int mb) { return mb < 4 ? mb : 4; }   // row blocks summed at a time at the end
+constexpr int mid_lds(int mb) {
+  const int stages = mid_stages(mb) * mid_stage_bytes(mb), sum = kMidWaves * mid_sum_rows(mb) * 4096;
+  return stages > sum ? stages : sum;
+}
+
+// How the scales come: one group, groups of 64 * 2^i rows (a scale row a step), or groups of 32 rows or less (a
+// scale row a chunk; NVFP4: two groups a chunk).
+enum MidGroups { kOneGroup = 0, kStepGroups = 1, kChunkGroups = 2 };
+
+template <typename T, int FMT>
+struct MidDequant {
+  static constexpr bool kF4 = FMT == kMidMxFp4 || FMT == kMidNvFp4;
+  static constexpr bool k8 = FMT == kMidInt8 || FMT == kMidFp8;
+  typedef typename Dq4Of<T, kF4, FMT == kMidNvFp4>::type D4;
+  typedef typename Dq8Of<T, FMT == kMidFp8>::type D8;
+  typedef typename std::conditional<k8, typename D8::Col, typename D4::Col>::type Col;
+};
+
+template <typename T, int FMT, int GROUPS, int MB>
+__global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void marlin_mid_gemm(
+    const MidParams p) {
+  typedef MidDequant<T, FMT> Fmt;
+  typedef typename Fmt::D4 D4;
+  typedef typename Fmt::D8 D8;
+  typedef typename Fmt::Col Col;
+  typedef typename Dq<T>::vec8 vec8;
+  constexpr bool kZero = FMT == kMidInt4Zp;
+  constexpr int D = mid_stages(MB);
+  constexpr int W = D - 1;                           // ring of the packed codes and scales in registers
+  constexpr int kStage = mid_stage_bytes(MB);
+  constexpr int kLoads = Fmt::k8 ? 4 : 2;            // 16-byte loads of packed codes per lane and step
+  constexpr int kScaleRows = GROUPS == kChunkGroups ? 2 : 1;
+  // memory operations per wavefront and step
+  constexpr int kOps = MB + kLoads + (GROUPS == kOneGroup ? 0 : kScaleRows * (kZero ? 2 : 1));
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col16 = lane & 15, kb = lane >> 4;
+  const int range = wave >> 1;
+  const uint32_t magic = magic_register();
+
+  // Workgroup ids congruent mod 8 run on one XCD: each XCD takes a contiguous run of tiles, the row tiles
+  // of a pair of strips next to each other, so the second to ask for a chunk finds it in that L2.
+  const int per_xcd = (p.tiles + 7) / 8;
+  const int tile = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= per_xcd || tile >= p.tiles) return;
+  const int tile_n = tile / p.tiles_m, tile_m = tile - tile_n * p.tiles_m;
+  const int m0 = tile_m * 16 * MB;
+  const int strips = p.size_n / kStripN;
+  // (the second strip of an odd last pair is the first again, and not stored)
+  const bool active = tile_n * kMidStrips + (wave & 1) < strips;
+  const int strip = __builtin_amdgcn_readfirstlane(active ? tile_n * kMidStrips + (wave & 1) : strips - 1);
+
+  const int steps = p.size_k / kMidStepK;
+  const int per_range = (steps + kMidRanges - 1) / kMidRanges;
+  const int k_first = range * per_range;
+
+  // ---- sources.  The activations of a range are copied by its own two wavefronts, MB copies each of 8 rows x
+  // one 128-byte line; piece q of row r sits at 16-byte slot q ^ r of the row, off the other rows' banks.
+  uint32_t a_off[MB];
+#pragma unroll
+  for (int i = 0; i < MB; ++i) {
+    int row = m0 + 8 * ((wave & 1) * MB + i) + (lane >> 3);
+    if (row >= p.size_m) row = p.size_m - 1;   // rows past M are computed and never stored
+    a_off[i] = (uint32_t)row * (uint32_t)(p.lda * 2) + 16 * ((lane & 7) ^ (lane >> 3));
+  }
+  const char* b_base = reinterpret_cast<const char*>(p.b) + (size_t)strip * p.chunks_per_strip * (Fmt::k8 ? 2048 : 1024);
+  const uint32_t b_off = 16 * lane;
+  const char* s_base = reinterpret_cast<const char*>(p.scales + (size_t)strip * kStripN);
+  const uint32_t s_off = 16 * (col16 & 7) + (FMT == kMidNvFp4 ? (kb >> 1) * (uint32_t)p.size_n * 2 : 0);
+  const char* z_base = reinterpret_cast<const char*>(p.zeros + (size_t)strip * (kStripN / 8));
+  const uint32_t z_off = 4 * (col16 & 7);
+  char* a_stage = smem + range * (MB * 2048);
+  const uint32_t a_lds = (uint32_t)(uintptr_t)(lds_void_t*)a_stage;
+
+  u32x4_t wq[W][kLoads];
+  u32x4_t sv[W][kScaleRows];
+  uint32_t zv[W][kScaleRows];
+
+  // Memory operation `op` (0..kOps-1) of step k: first the codes and scales into ring position R, then the
+  // activations into LDS slot `slot`.
+  auto issue_one = [&](const int R, const int slot, const int k, const int op) __attribute__((always_inline)) {
+    if (op < kLoads) {
+      const char* b_src = b_base + (size_t)k * (kLoads * 1024);
+      asm volatile("global_load_dwordx4 %0, %1, %2 offset:%3" : "=&v"(wq[R][op]) : "v"(b_off), "s"(b_src), "i"(op * 1024) : "memory");
+    } else if (op < kOps - MB) {
+      const int h = (op - kLoads) / (kZero ? 2 : 1);
+      const int g = GROUPS == kStepGroups ? k >> p.group_shift : (FMT == kMidNvFp4 ? 2 : 1) * (2 * k + h);
+      if (!kZero || (op - kLoads) % 2 == 0) {
+        const char* s_src = s_base + (size_t)g * p.size_n * 2;
+        asm volatile("global_load_dwordx4 %0, %1, %2" : "=&v"(sv[R][h]) : "v"(s_off), "s"(s_src) : "memory");
+      } else {
+        const char* z_src = z_base + (size_t)g * (p.size_n / 2);
+        asm volatile("global_load_dword %0, %1, %2" : "=&v"(zv[R][h]) : "v"(z_off), "s"(z_src) : "memory");
+      }
+    } else {
+      const int i = op - (kOps - MB);
+      const char* a_src = reinterpret_cast<const char*>(p.a) + (size_t)k * (kMidStepK * 2);
+      __builtin_amdgcn_global_load_lds((glb_void_t*)(a_src + a_off[i]),
+                                       (lds_void_t*)(a_stage + slot * kStage + ((wave & 1) * MB + i) * 1024), 16, 0, 0);
+    }
+  };
+  // until only the `n` youngest operations are outstanding; the registers of ring position R are in its hands
+  auto landed = [&](const int R, const int n) __attribute__((always_inline)) {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"i"(n) : "memory");
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) asm volatile("" : "+v"(wq[R][i]));
+    if constexpr (GROUPS != kOneGroup) {
+#pragma unroll
+      for (int h = 0; h < kScaleRows; ++h) {
+        asm volatile("" : "+v"(sv[R][h]));
+        if constexpr (kZero) asm volatile("" : "+v"(zv[R][h]));
+      }
+    }
+  };
+
+  Col cols[4];
+  auto set_col = [&](int j, uint16_t scale_bits, uint32_t zero_word) __attribute__((always_inline)) {
+    int z = 8;
+    if (kZero) z = (int)((zero_word >> (4 * (j + 4 * (col16 >> 3)))) & 0xFu);   // zero_point_shift(16 j + col16)
+    if constexpr (Fmt::k8) cols[j] = D8::make_col(scale_bits);
+    else cols[j] = D4::make_col(scale_bits, z);
+  };
+  // the constants of column block j from ring position R (chunk h of the step)
+  auto make_col = [&](const int R, const int h, const int j) __attribute__((always_inline)) {
+    if constexpr (GROUPS != kOneGroup) {
+      const u32x4_t& v = sv[R][GROUPS == kChunkGroups ? h : 0];
+      const uint32_t word = j == 0 ? v.x : j == 1 ? v.y : j == 2 ? v.z : v.w;
+      // column 16 j + col16 is slot 2 j + col16 / 8 of the lane's eight
+      const uint32_t bits = (col16 & 8) ? word >> 16 : word & 0xFFFFu;
+      set_col(j, (uint16_t)bits, kZero ? zv[R][GROUPS == kChunkGroups ? h : 0] : 0);
+    }
+  };
+  if constexpr (GROUPS == kOneGroup) {
+    const uint16_t* srow = p.scales + (size_t)strip * kStripN;
+    uint32_t zword = 0;
+    if (kZero) zword = p.zeros[(size_t)strip * (kStripN / 8) + (col16 & 7)];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) set_col(j, srow[scale_slot(16 * j + col16, false)], zword);
+  }
+
+  u32x4_t av[MB];
+  uint32_t wv[2][4][4];    // dequantised chunk of either half: four operand blocks of 16 columns
+  floatx4_t acc[4][MB];
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+#pragma unroll
+    for (int i = 0; i < MB; ++i) acc[j][i] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+
+  // Piece `q` (0..15) of dequantising chunk h of ring position R into wv[h].  A pair of 4-bit integer codes is
+  // finished by the piece after it (q = 16 finishes the last).
+  typename Dq<T>::Mid mid;
+  auto piece = [&](const int R, const int h, const int q) __attribute__((always_inline)) {
+    const int j = q >> 2, part = q & 3;
+    if constexpr (!Fmt::k8 && !Fmt::kF4) {
+      if (q > 0) wv[h][(q - 1) >> 2][(q - 1) & 3] = D4::stage3(mid, cols[(q - 1) >> 2]);
+    }
+    if (q == 16) return;
+    if (part == 0 && (GROUPS == kChunkGroups || h == 0)) make_col(R, h, j);
+    if constexpr (Fmt::k8) {
+      if (part & 1) return;
+      const u32x4_t& v = wq[R][2 * h + (part >> 1)];   // the low, then the high four of a lane's eight rows
+      const uint32_t word = j == 0 ? v.x : j == 1 ? v.y : j == 2 ? v.z : v.w;
+      const uint2 w = D8::word4(word, cols[j], magic);
+      wv[h][j][part] = w.x;
+      wv[h][j][part + 1] = w.y;
+    } else {
+      const u32x4_t& v = wq[R][h];
+      const uint32_t word = j == 0 ? v.x : j == 1 ? v.y : j == 2 ? v.z : v.w;
+      if constexpr (Fmt::kF4) {
+        if (part != 0) return;
+        const u32x4_t w = __builtin_bit_cast(u32x4_t, D4::word(word, cols[j], magic));
+        wv[h][j][0] = w.x, wv[h][j][1] = w.y, wv[h][j][2] = w.z, wv[h][j][3] = w.w;
+      } else {
+        mid = D4::stage2(D4::stage1(part < 2 ? word : word >> 8, part, magic), cols[j], part);
+      }
+    }
+  };
+  // operand lane (kb, col16) of row block 0, chunk h: piece 4 h + kb of row col16
+  uint32_t a_at[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+    a_at[h] = a_lds + (col16 >> 3) * 1024 + (col16 & 7) * 128 + (((4 * h + kb) ^ (col16 & 7)) * 16);
+#define SONAR_MID_READ(dst, base, off) \
+  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=&v"(dst) : "v"(base), "i"(off) : "memory")
+  // One half of a step: 4 MB matrix instructions on chunk H of the step in ring position R, LDS slot `slot`.
+  // Behind each, a share of the next half's dequantisation and (H = 1) of the memory operations of step `k_copy`;
+  // behind a row block's four, the read of its operand of the next half.
+  auto half_step = [&](const int R, const int H, const int slot, const int next_slot, const int fill,
+                       const int k_copy) __attribute__((always_inline)) {
+    const int NR = H ? (R + 1) % W : R, NH = H ^ 1;
+    const uint32_t a_next = a_at[NH] + (H ? next_slot : slot) * kStage;
+#pragma unroll
+    for (int i = 0; i < MB; ++i) {
+      // the operands of this half are the oldest reads, MB are outstanding at every row block
+      asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(av[i]) : "i"(MB - 1) : "memory");
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const vec8 w = __builtin_bit_cast(vec8, u32x4_t{wv[H][j][0], wv[H][j][1], wv[H][j][2], wv[H][j][3]});
+        acc[j][i] = Dq<T>::mfma(w, __builtin_bit_cast(vec8, av[i]), acc[j][i]);
+        const int at = 4 * i + j;
+#pragma unroll
+        for (int q = 0; q < 16; ++q)
+          if (q >= 16 * at / (4 * MB) && q < 16 * (at + 1) / (4 * MB)) piece(NR, NH, q);
+        if (H) {
+#pragma unroll
+          for (int o = 0; o < kOps; ++o)
+            if (o >= kOps * at / (4 * MB) && o < kOps * (at + 1) / (4 * MB)) issue_one(R, fill, k_copy, o);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      SONAR_MID_READ(av[i], a_next, i * 2048);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    piece(NR, NH, 16);
+  };
+
+  // ---- prologue: D - 1 steps asked for, the first one here
+#pragma unroll
+  for (int r = 0; r < W; ++r)
+#pragma unroll
+    for (int o = 0; o < kOps; ++o) issue_one(r, r, min(k_first + r, steps - 1), o);
+  landed(0, (W - 1) * kOps);
+  __builtin_amdgcn_s_barrier();
+#pragma unroll
+  for (int i = 0; i < MB; ++i) SONAR_MID_READ(av[i], a_at[0], i * 2048);
+#pragma unroll
+  for (int q = 0; q <= 16; ++q) piece(0, 0, q);
+
+  int slot = 0, fill = W;   // LDS slot of step t, and the one step t + D - 1 goes to
+  auto step = [&](const int R, int t) __attribute__((always_inline)) {
+    const bool live = k_first + t < steps;   // uniform; past the end of K only the copies are left to do
+    const int next_slot = slot == D - 1 ? 0 : slot + 1;
+    const int k_copy = min(k_first + t + W, steps - 1);
+    if (live) half_step(R, 0, slot, next_slot, 0, 0);
+    landed((R + 1) % W, (W - 2) * kOps);
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    if (live) {
+      half_step(R, 1, slot, next_slot, fill, k_copy);
+    } else {
+#pragma unroll
+      for (int o = 0; o < kOps; ++o) issue_one(R, fill, k_copy, o);
+    }
+    slot = next_slot;
+    fill = fill == D - 1 ? 0 : fill + 1;
+  };
+  for (int t = 0; t < per_range; t += W) {
+    step(0, t);
+    if (t + 1 < per_range) step(1, t + 1);
+    if constexpr (W > 2)
+      if (t + 2 < per_range) step(2, t + 2);
+  }
+  // copies and reads still under way must not outlive this point: LDS is used for the sums from here on
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+#pragma unroll
+  for (int i = 0; i < MB; ++i) asm volatile("" : "+v"(av[i]));
+#pragma unroll
+  for (int r = 0; r < W; ++r) {
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) asm volatile("" : "+v"(wq[r][i]));
+    if constexpr (GROUPS != kOneGroup) {
+#pragma unroll
+      for (int h = 0; h < kScaleRows; ++h) {
+        asm volatile("" : "+v"(sv[r][h]));
+        if constexpr (kZero) asm volatile("" : "+v"(zv[r][h]));
+      }
+    }
+  }
+#undef SONAR_MID_READ
+  __builtin_amdgcn_s_barrier();
+
+  // ---- the four ranges meet in LDS, mid_sum_rows(MB) row blocks at a time; a wavefront adds a quarter of
+  // its strip's accumulator tiles, in the order of the ranges
+  constexpr int kSum = mid_sum_rows(MB);
+  float4* sums = reinterpret_cast<float4*>(smem);
+  const float gs = FMT == kMidNvFp4 && p.global_scale ? p.global_scale[0] : 1.f;
+#pragma unroll
+  for (int round = 0; round < MB; round += kSum) {
+    if (round > 0) __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kSum; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (round + i < MB) {
+          const floatx4_t v = acc[j][round + i < MB ? round + i : 0];
+          sums[((wave * kSum + i) * 4 + j) * 64 + lane] = make_float4(v.x, v.y, v.z, v.w);
+        }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kSum; ++u) {
+      const int q = range * kSum + u;
+      const int i = round + (q >> 2), j = q & 3;
+      const int row = m0 + 16 * i + col16;
+      if (i >= MB || !active) continue;
+      floatx4_t v = floatx4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int g = 0; g < kMidRanges; ++g) {
+        const float4 s = sums[(((2 * g + (wave & 1)) * kSum + (q >> 2)) * 4 + j) * 64 + lane];
+        v += floatx4_t{s.x, s.y, s.z, s.w};
+      }
+      if (row >= p.size_m) continue;
+      if (FMT == kMidNvFp4) v = v * gs;
+      const int nl = 16 * j + 4 * kb;
+      float bias[4] = {0.f, 0.f, 0.f, 0.f};
+      if (p.bias) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) bias[r] = Dq<T>::to_float(p.bias[strip * kStripN + scale_slot(nl + r, false)]);
+      }
+      uint2 o;
+      o.x = (uint32_t)Dq<T>::from_float(v.x + bias[0]) | ((uint32_t)Dq<T>::from_float(v.y + bias[1]) << 16);
+      o.y = (uint32_t)Dq<T>::from_float(v.z + bias[2]) | ((uint32_t)Dq<T>::from_float(v.w + bias[3]) << 16);
+      *reinterpret_cast<uint2*>(p.c + (size_t)row * p.size_n + strip * kStripN + nl) = o;
+    }
+  }
+}
+
+template <typename T, int FMT, int GROUPS, int MB>
+int launch_mid_rows(const MidParams& p, hipStream_t st) {
+  static bool attr_set = false;   // raising the dynamic LDS limit is needed once per form
+  if (!attr_set) {
+    SONAR_HIP(hipFuncSetAttribute((const void*)marlin_mid_gemm<T, FMT, GROUPS, MB>,
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, mid_lds(MB)));
+    attr_set = true;
+  }
+  marlin_mid_gemm<T, FMT, GROUPS, MB><<<(p.tiles + 7) / 8 * 8, kMidWaves * 64, mid_lds(MB), st>>>(p);
+  return launch_status("marlin_mid_gemm");
+}
+
+template <typename T, int FMT, int GROUPS>
+int launch_mid(const MidParams& p, int row_blocks, hipStream_t st) {
+  switch (row_blocks) {
+    case 2: return launch_mid_rows<T, FMT, GROUPS, 2>(p, st);
+    case 3: return launch_mid_rows<T, FMT, GROUPS, 3>(p, st);
+    case 4: return launch_mid_rows<T, FMT, GROUPS, 4>(p, st);
+    case 5: return launch_mid_rows<T, FMT, GROUPS, 5>(p, st);
+    default: return launch_mid_rows<T, FMT, GROUPS, 6>(p, st);
+  }
+}
+
+template <typename T, int FMT>
+int launch_mid_groups(const MidParams& p, int row_blocks, hipStream_t st) {
+  if constexpr (FMT == kMidMxFp4 || FMT == kMidNvFp4) {
+    return launch_mid<T, FMT, kChunkGroups>(p, row_blocks, st);
+  } else {
+    if (p.num_groups == 1) return launch_mid<T, FMT, kOneGroup>(p, row_blocks, st);
+    if (p.group_shift >= 0) return launch_mid<T, FMT, kStepGroups>(p, row_blocks, st);
+    return launch_mid<T, FMT, kChunkGroups>(p, row_blocks, st);
+  }
+}
+
+template <typename T>
+int launch_mid_format(const MidParams& p, int format, int row_blocks, hipStream_t st) {
+  switch (format) {
+    case kMidInt4: return launch_mid_groups<T, kMidInt4>(p, row_blocks, st);
+    case kMidInt4Zp: return launch_mid_groups<T, kMidInt4Zp>(p, row_blocks, st);
+    case kMidInt8: return launch_mid_groups<T, kMidInt8>(p, row_blocks, st);
+    case kMidFp8: return launch_mid_groups<T, kMidFp8>(p, row_blocks, st);
+    case kMidNvFp4: return launch_mid_groups<T, kMidNvFp4>(p, row_blocks, st);
+    default:   // MXFP4: bf16 only, which the caller has checked
+      if constexpr (std::is_same<T, __bf16>::value) return launch_mid_groups<T, kMidMxFp4>(p, row_blocks, st);
+      return fail(SONAR_E_INVALID, "internal: MXFP4 weights with float16 activations");
+  }
+}
+
+}  // namespace
+
+int mid_gemm(MidParams p, int dtype, int format, int row_blocks, hipStream_t st) {
+  const int strips = p.size_n / kStripN;
+  p.tiles_m = (p.size_m + 16 * row_blocks - 1) / (16 * row_blocks);
+  p.tiles = p.tiles_m * ((strips + kMidStrips - 1) / kMidStrips);
+  return dtype == SONAR_DTYPE_F16 ? launch_mid_format<_Float16>(p, format, row_blocks, st)
+                                  : launch_mid_format<__bf16>(p, format, row_blocks, st);
+}
+
+}  // namespace sonar

@@ -1,0 +1,62 @@
+// Interface of gemm_mid.hip to the dispatchers.
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+namespace sonar {
+
+// Weight formats of the kernel in gemm_mid.hip.
+enum MidFormat { kMidInt4 = 0, kMidInt4Zp = 1, kMidInt8 = 2, kMidFp8 = 3, kMidMxFp4 = 4, kMidNvFp4 = 5 };
+
+struct MidParams {
+  const uint16_t* a;
+  long lda;                  // elements between rows of a
+  uint16_t* c;
+  const uint4* b;            // gfx950 streaming order
+  const uint16_t* bias;
+  const uint16_t* scales;
+  const uint32_t* zeros;
+  const float* global_scale;   // NVFP4
+  int size_m, size_n, size_k, num_groups;
+  int group_shift;           // log2 of the 64-row steps per group; -1: groups of 32 or 16 rows
+  int chunks_per_strip;
+  int tiles_m, tiles;        // filled in by mid_gemm
+};
+
+// Whether the kernel can run a call (no act-order gather; rows of a within 4 GiB; groups of 16, 32 or 64 * 2^i rows or
+// one group).
+inline bool mid_applies(int64_t size_m, int64_t size_k, int64_t lda, int64_t num_groups, int group_size) {
+  if (size_k % 64 != 0 || size_m * lda * 2 >= (1LL << 32)) return false;
+  if (num_groups == 1 || group_size == 16 || group_size == 32) return true;
+  const int per = group_size / 64;
+  return group_size % 64 == 0 && (per & (per - 1)) == 0;
+}
+
+// Microseconds a call takes in tiles of the best number of row blocks, which is returned in `row_blocks`.  A fit
+// of measured times (K = 2048 and 4096, N = 2048, 6144 and 20032, 17 to 768 rows, all formats, within 10 %): about
+// 6 us around the loop, per round of workgroups and 4096 rows of K 1.5 us for a row block's matrix instructions
+// and a time that depends on the format for the dequantisation, which the matrix instructions do not hide.
+inline double mid_estimate(int64_t size_m, int64_t size_n, int64_t size_k, int64_t num_groups, int dtype, int format,
+                           int cus, int& row_blocks) {
+  static const double kDequant[6][2] = {   // float16, bfloat16
+      {6.8, 8.8}, {8.3, 10.0}, {6.0, 10.2}, {8.0, 15.5}, {5.3, 5.3}, {9.0, 13.3}};
+  const double k = ((size_k / 64 + 3) / 4) * 256 / 4096.0;
+  const double dequant = kDequant[format][dtype == 0 ? 0 : 1] + (num_groups > 1 && size_k / num_groups == 32 && format != kMidMxFp4 ? 0.8 : 0.0);
+  double best = 1e30;
+  for (int mb = 2; mb <= 6; ++mb) {
+    const int64_t tiles = ((size_m + 16 * mb - 1) / (16 * mb)) * ((size_n + 127) / 128);
+    const int64_t rounds = (tiles + cus - 1) / cus;
+    const double us = 5.0 + rounds * (1.0 + k * (dequant + 1.5 * mb));
+    if (us < best) {
+      best = us;
+      row_blocks = mb;
+    }
+  }
+  return best;
+}
+
+// `row_blocks`: 16-row blocks of a tile, 2 to 6.
+int mid_gemm(MidParams p, int dtype, int format, int row_blocks, hipStream_t st);
+
+}  // namespace sonar

@@ -17,9 +17,11 @@
 // spins, nothing is atomic, and the result does not depend on timing.  Short
 // strips (K <= 4096) on a wide matrix get one workgroup each instead, which
 // shares nothing and needs no second kernel.
+#include <algorithm>
 #include <cstdlib>
 
 #include "dequant.hpp"
+#include "gemm_mid.hpp"
 #include "gemm_plan.hpp"
 #include "wave_reduce.hpp"
 
@@ -1730,6 +1732,15 @@ int moe_fast_gemm(const void* a, void* c, const uint32_t* b, const void* bias, c
 using namespace sonar;
 
 namespace {
+// The switches that single out an older path of the dense dispatch leave the kernel of gemm_mid.hip out as well.
+bool mid_switched_off() {
+  for (const char* name : {"SONAR_MARLIN_NO_MID", "SONAR_MARLIN_NO_FAST", "SONAR_MARLIN_NO_SLABS", "SONAR_MARLIN_NO_ROW_PAIRS",
+                           "SONAR_MARLIN_NO_HALF_WG", "SONAR_MARLIN_SPLIT", "SONAR_MARLIN_NO_INLINE_SUM",
+                           "SONAR_MARLIN_NO_TILE", "SONAR_MARLIN_NO_WIDE_TILE", "SONAR_MARLIN_NO_128_ROW_TILES",
+                           "SONAR_MARLIN_NO_ASYNC_TILE", "SONAR_MARLIN_MAX_K_SPLITS", "SONAR_MARLIN_NO_TWO_TILE_SIZES"})
+    if (getenv(name) != nullptr) return true;
+  return false;
+}
 size_t stream_scratch_bytes() { return (size_t)2 * cu_count() * kSlotFloat4 * sizeof(float4); }
 thread_local int32_t g_last_decode_launch[4] = {0, 0, 0, 0};
 }  // namespace
@@ -1887,6 +1898,44 @@ int marlin_gemm_any(const void* a, int64_t a_row_stride, void* c, const uint32_t
   // eight launches).
   const bool row_slabs = !use_tile && !slab_fast && size_m > 64 && strip_per_workgroup &&
                          total_units * n_strips < (1LL << 31);
+  // 17 rows and more: the kernel of gemm_mid.hip where it is estimated to be faster than what would run otherwise
+  static const char* mid_env = getenv("SONAR_MARLIN_MID_ROWS");   // debugging aid: its tiles of that many row blocks, always
+  static const bool no_mid = mid_switched_off();
+  if ((size_m > 16 || mid_env) && !no_mid && !chk.has_perm && !chk.row_groups && ((uintptr_t)b_scales) % 16 == 0 &&
+      mid_applies(size_m, size_k, a_row_stride, num_groups, chk.group_size)) {
+    const int format = chk.nvfp4 ? kMidNvFp4 : chk.fp4 ? kMidMxFp4 : chk.bits == 8 ? (chk.fp8 ? kMidFp8 : kMidInt8)
+                       : chk.has_zp ? kMidInt4Zp : kMidInt4;
+    int row_blocks;
+    const double mid_us = mid_estimate(size_m, size_n, size_k, num_groups, dtype, format, cus, row_blocks);
+    const double x = (double)size_n * size_k / (6144.0 * 4096.0), r = size_m / 64.0;
+    // (what the other kernels take, us: fits of measured times, see mid_estimate)
+    double us;
+    if (slab_fast)
+      us = 6.5 + 0.0245 * (size_k / 4096.0) * n_strips * ((size_m + 31) / 32) * (size_m <= 64 && n_strips < cus / 2 ? 0.6 : 1.0);
+    else if (use_tile)
+      us = 25.0 + 0.69e-9 * 2.0 * size_m * size_n * size_k;
+    else
+      us = size_m <= 64 ? 9.5 + x * (5.5 + 5.2 * r * r) : 11.0 + 10.7 * x * r;
+    if (mid_env) row_blocks = std::max(2, std::min(6, atoi(mid_env)));
+    if (mid_env || (mid_us < 0.93 * us && size_n * size_k >= 4 * 1000 * 1000)) {
+      MidParams q = {};
+      q.a = static_cast<const uint16_t*>(a);
+      q.lda = a_row_stride;
+      q.c = static_cast<uint16_t*>(c);
+      q.b = reinterpret_cast<const uint4*>(b_q_weight);
+      q.bias = static_cast<const uint16_t*>(b_bias);
+      q.scales = static_cast<const uint16_t*>(b_scales);
+      q.zeros = b_zeros;
+      q.global_scale = global_scale;
+      q.size_m = (int)size_m;
+      q.size_n = (int)size_n;
+      q.size_k = (int)size_k;
+      q.num_groups = (int)num_groups;
+      q.group_shift = chk.group_size < 64 ? -1 : 31 - __builtin_clz(chk.group_size / 64);
+      q.chunks_per_strip = p.chunks_per_strip;
+      return mid_gemm(q, dtype, format, row_blocks, st);
+    }
+  }
   p.parts = p.total_units < cus ? p.total_units : cus;
   if (strip_per_workgroup && row_slabs) p.parts = (int)n_strips;
   // One row block on a matrix with about as many strips as compute units: a workgroup per strip, so that
