@@ -15,8 +15,12 @@
 // four totals meet in LDS; wavefront w finishes column block w.  With K split
 // over several workgroups the raw totals go to scratch and a second kernel
 // adds them, so integer results never depend on the split.
+#include <cstdlib>
+#include <cstdio>
+
 #include "common.hpp"
 #include "dequant.hpp"
+#include "gemm_a8_block.hpp"
 
 namespace sonar {
 namespace {
@@ -882,6 +886,61 @@ int check_a8(int a_dtype, int dtype, int b_layout, int64_t b_type_id, int64_t si
   return SONAR_OK;
 }
 
+// The tile of the kernel in gemm_a8_block.hip for a call, or rows = 0 where the kernels above are to run.
+A8BlockShape block_shape(bool fp8, bool zero_points, bool float4, int64_t size_m, int64_t size_n, int64_t size_k,
+                         int64_t num_groups) {
+  A8BlockShape best = {0, 0, 0, 0};
+  static const char* forced = getenv("SONAR_MARLIN_A8_SHAPE");   // debugging aid: "rows,ranges,splits"; 0: never
+  if (size_k % 128 != 0 || float4) return best;
+  if (num_groups == 1 ? size_k > 65536 : fp8 && size_k / num_groups < 64) return best;
+  const int steps = (int)(size_k / 128), chunks = num_groups == 1 ? 0 : (int)(size_k / num_groups / kChunkK);
+  if (forced) {
+    if (sscanf(forced, "%d,%d,%d", &best.rows, &best.ranges, &best.splits) != 3) return A8BlockShape{0, 0, 0, 0};
+    best.strips = best.rows > 2 ? 4 : 2;
+  } else if (size_m > 16) {   // (to 16 rows the first kernel above is as fast or faster)
+    // Microseconds a call takes, a fit of measured times (int8 and fp8, groups of 32 to K, K = 1152 to 14336, N = 4096
+    // to 22976, 24 to 1000 rows; mostly within 15 %).  A step of two wavefronts of a SIMD: a time to dequantise plus
+    // one per row block, larger for smaller groups; one wavefront alone takes 0.55 of it.
+    double deq = 0.45, row = 0.5;
+    if (chunks == 0) deq = fp8 ? 0.8 : 0.2, row = fp8 ? 0.27 : 0.43;
+    else if (chunks == 1) deq = 0.8, row = 0.8;
+    else if (chunks == 2) deq = fp8 ? 0.8 : 0.6, row = fp8 ? 0.5 : 0.53;
+    else if (fp8) deq = 0.75, row = 0.38;
+    if (fp8 && zero_points) deq += 0.5;
+    static const struct { int rows, strips, ranges; double around; } kShapes[5] = {
+        {1, 2, 4, 5.0}, {2, 2, 4, 6.5}, {3, 4, 2, 10.0}, {3, 4, 1, 6.0}, {4, 4, 1, 7.0}};
+    double least = 1e30;
+    if (size_m <= 32)   // the first kernel: it reads the weights at a third of the rate of memory, and less
+      least = (5.5 + 0.19e-6 * size_n * size_k) * (chunks == 1 ? 1.5 : chunks == 2 ? 1.13 : chunks == 0 ? 0.87 : 1.0);
+    for (const auto& s : kShapes) {
+      if (s.rows > a8_max_row_blocks(fp8, zero_points, chunks)) continue;
+      const int64_t tiles = ((size_m + 32 * s.rows - 1) / (32 * s.rows)) * ((size_n / 64 + s.strips - 1) / s.strips);
+      // where the tiles leave compute units idle, K over several workgroups and a pass that adds their totals
+      for (int splits = 1; splits <= 8 && (splits == 1 || (tiles * splits <= 256 && steps >= 2 * splits * s.ranges)); ++splits) {
+        const int per = ((steps + splits - 1) / splits + s.ranges - 1) / s.ranges;
+        const double step = deq + row * s.rows, all = per * step + s.around;
+        double us = 1.0;
+        if (s.ranges > 1) {
+          us += (tiles * splits + 255) / 256 * all;
+        } else {
+          const int64_t rest = tiles * splits % 512;
+          us += tiles * splits / 512 * all;
+          if (rest > 256) us += all;
+          else if (rest > 0) us += 0.55 * per * step + s.around;
+        }
+        if (splits > 1) us += 5.0 + 2e-6 * size_m * size_n * splits;
+        if (us < least) least = us, best = A8BlockShape{s.rows, s.strips, s.ranges, splits};
+      }
+    }
+  }
+  if (best.rows) {
+    if (best.splits > steps) best.splits = steps;
+    const int per = (steps + best.splits - 1) / best.splits;
+    best.splits = (steps + per - 1) / per;
+  }
+  return best;
+}
+
 // One 32-row group of float4 weights is a "grouped" call even when K = 32.
 bool a8_grouped(int64_t b_type_id, int64_t num_groups) {
   return num_groups > 1 || b_type_id == SONAR_TYPE_FLOAT4_E2M1F;
@@ -957,8 +1016,14 @@ extern "C" int sonar_moe_wna16_marlin_gemm_a8(
 extern "C" size_t sonar_marlin_gemm_a8_scratch_bytes(int64_t size_m, int64_t size_n, int64_t size_k,
                                                      int64_t num_groups) {
   if (size_m <= 0 || size_n <= 0 || size_k < kChunkK || num_groups < 1) return 0;
-  const A8Plan plan = plan_a8(size_m, size_n, size_k, num_groups);
-  return plan.splits > 1 ? (size_t)plan.splits * size_m * size_n * 4 : 0;
+  // whatever the types: the most that any of them takes
+  int splits = 1;
+  for (int form = 0; form < 5; ++form) {
+    const A8BlockShape shape = block_shape(form & 1, form & 2, form == 4, size_m, size_n, size_k, num_groups);
+    const int s = shape.rows ? shape.splits : plan_a8(size_m, size_n, size_k, num_groups).splits;
+    if (s > splits) splits = s;
+  }
+  return splits > 1 ? (size_t)splits * size_m * size_n * 4 : 0;
 }
 
 extern "C" int sonar_marlin_gemm_a8(const void* a, int64_t a_row_stride, int a_dtype, void* c, const uint32_t* b_q_weight,
@@ -973,7 +1038,15 @@ extern "C" int sonar_marlin_gemm_a8(const void* a, int64_t a_row_stride, int a_d
                 "divisible by 8", (long)a_row_stride);
   SONAR_REQUIRE((uintptr_t)a % 16 == 0, "A must aligned to 16 bytes");
 
-  const A8Plan plan = plan_a8(size_m, size_n, size_k, num_groups);
+  A8Plan plan = plan_a8(size_m, size_n, size_k, num_groups);
+  A8BlockShape shape = block_shape(a_dtype == SONAR_ADTYPE_FP8, b_zeros != nullptr,
+                                   b_type_id == SONAR_TYPE_FLOAT4_E2M1F, size_m, size_n, size_k, num_groups);
+  if (shape.rows && (a_row_stride % 16 != 0 || size_m * a_row_stride >= (1LL << 32))) {
+    // rows it cannot copy: the older kernels, with the scratch there is
+    shape.rows = 0;
+    if (scratch_bytes < (size_t)plan.splits * size_m * size_n * 4) plan.splits = 1, plan.units_per_split = plan.units;
+  }
+  if (shape.rows) plan.splits = shape.splits;
   A8Params p;
   p.a = (const uint8_t*)a;
   p.a_row_stride = a_row_stride;
@@ -997,6 +1070,31 @@ extern "C" int sonar_marlin_gemm_a8(const void* a, int64_t a_row_stride, int a_d
                   (size_t)plan.splits * size_m * size_n * 4);
   const bool grouped = a8_grouped(b_type_id, num_groups);
   hipStream_t st = (hipStream_t)stream;
+  if (shape.rows) {
+    A8BlockParams b;
+    b.a = p.a;
+    b.lda = a_row_stride;
+    b.c = (uint16_t*)c;
+    b.w = b_q_weight;
+    b.scales = p.scales;
+    b.zeros = b_zeros;
+    b.a_scales = a_scales;
+    b.bias = p.bias;
+    b.size_m = p.m, b.size_n = p.n, b.size_k = (int)size_k;
+    b.group_chunks = num_groups > 1 ? (int)(size_k / num_groups) / kChunkK : 0;
+    b.bf16 = dtype == SONAR_DTYPE_BF16;
+    b.partial = p.partial;
+    if (int rc = a8_block_gemm(b, a_dtype == SONAR_ADTYPE_FP8, shape, st)) return rc;
+    if (shape.splits == 1) return SONAR_OK;
+    if (a_dtype == SONAR_ADTYPE_INT8) {
+      if (dtype == SONAR_DTYPE_F16) launch_a8_finish<ActInt8, _Float16>(p, grouped, st);
+      else launch_a8_finish<ActInt8, __bf16>(p, grouped, st);
+    } else {
+      if (dtype == SONAR_DTYPE_F16) launch_a8_finish<ActFp8, _Float16>(p, grouped, st);
+      else launch_a8_finish<ActFp8, __bf16>(p, grouped, st);
+    }
+    return launch_status("marlin_a8_finish_kernel");
+  }
   if (b_type_id == SONAR_TYPE_FLOAT4_E2M1F) {
     launch_a8<ActFp8F4, __bf16>(p, plan, grouped, st);   // bfloat16 outputs only (check_a8)
   } else if (a_dtype == SONAR_ADTYPE_INT8) {
