@@ -235,6 +235,10 @@ int sonar_marlin_gemm(const void* a, int64_t a_row_stride, void* c,
  *   x   dtype[rows][row_stride] (SONAR_DTYPE_F16, _BF16 or _F32); q [rows][cols]; scales float[rows] */
 int sonar_per_token_quant_int8(const void* x, int dtype, int64_t row_stride, int8_t* q,
                                float* scales, int64_t rows, int64_t cols, void* stream);
+/* Every scale times factor[0] (a float on the device, or NULL): the global scale of int8 group scales. */
+int sonar_per_token_quant_int8_scaled(const void* x, int dtype, int64_t row_stride, int8_t* q,
+                                      float* scales, const float* factor, int64_t rows,
+                                      int64_t cols, void* stream);
 int sonar_per_token_quant_fp8(const void* x, int dtype, int64_t row_stride, uint8_t* q,
                               float* scales, int64_t rows, int64_t cols, void* stream);
 

@@ -53,6 +53,8 @@ PROTOTYPES = {
     "sonar_gfx950_to_marlin_a8": (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_void_p]),
     "sonar_marlin_int4_fp8_preprocess": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_void_p]),
     "sonar_per_token_quant_int8": (c_int, [c_void_p, c_int, c_int64, c_void_p, c_void_p, c_int64, c_int64, c_void_p]),
+    "sonar_per_token_quant_int8_scaled": (c_int, [c_void_p, c_int, c_int64, c_void_p, c_void_p, c_void_p, c_int64, c_int64,
+                                                   c_void_p]),
     "sonar_per_token_quant_fp8": (c_int, [c_void_p, c_int, c_int64, c_void_p, c_void_p, c_int64, c_int64, c_void_p]),
     "sonar_marlin_gemm_a8_scratch_bytes": (c_size_t, [c_int64, c_int64, c_int64, c_int64]),
     "sonar_marlin_gemm_a8": (c_int, [c_void_p, c_int64, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p,
