@@ -503,6 +503,39 @@ Tensor marlin_int4_fp8_preprocess(const Tensor& qweight, const OptTensor& qzeros
   return output;
 }
 
+// Per-token quantisation of the activations of the W4A8 GEMM: (codes of x's shape, float32
+// scales (..., 1)), the int8 scales times `factor` if there is one.
+std::tuple<Tensor, Tensor> per_token_quant(const Tensor& x, bool fp8, const OptTensor& factor = std::nullopt) {
+  TORCH_CHECK(x.is_cuda(), "x is not on GPU");
+  TORCH_CHECK(x.dim() >= 1 && x.size(-1) > 0, "x must have a non-empty last dimension");
+  int dtype;
+  if (x.scalar_type() == at::kHalf) dtype = SONAR_DTYPE_F16;
+  else if (x.scalar_type() == at::kBFloat16) dtype = SONAR_DTYPE_BF16;
+  else if (x.scalar_type() == at::kFloat) dtype = SONAR_DTYPE_F32;
+  else TORCH_CHECK(false, "per-token quantisation takes float16, bfloat16 or float32; got ", x.scalar_type());
+  const int64_t cols = x.size(-1);
+  const Tensor x2 = x.reshape({-1, cols});
+  const Tensor src = x2.stride(1) == 1 ? x2 : x2.contiguous();
+  const int64_t rows = src.size(0);
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+  Tensor q = at::empty(x.sizes(), x.options().dtype(fp8 ? at::kFloat8_e4m3fn : at::kChar));
+  auto scale_shape = x.sizes().vec();
+  scale_shape.back() = 1;
+  Tensor scales = at::empty(scale_shape, x.options().dtype(at::kFloat));
+  if (fp8)
+    raise_if_failed(sonar_per_token_quant_fp8(src.const_data_ptr(), dtype, rows ? src.stride(0) : cols,
+                                              static_cast<uint8_t*>(q.mutable_data_ptr()),
+                                              static_cast<float*>(scales.mutable_data_ptr()), rows, cols,
+                                              current_stream(x)));
+  else
+    raise_if_failed(sonar_per_token_quant_int8_scaled(
+        src.const_data_ptr(), dtype, rows ? src.stride(0) : cols, static_cast<int8_t*>(q.mutable_data_ptr()),
+        static_cast<float*>(scales.mutable_data_ptr()),
+        factor.has_value() ? static_cast<const float*>(factor->const_data_ptr()) : nullptr, rows, cols,
+        current_stream(x)));
+  return {q, scales};
+}
+
 // ---------------------------------------------------------------- dense GEMM
 void check_b_type(int64_t b_type_id) {
   TORCH_CHECK_NOT_IMPLEMENTED(
@@ -619,13 +652,15 @@ Tensor marlin_gemm_a8(const Tensor& a, const OptTensor& c_or_none, const Tensor&
 
   Tensor native = native_weights(b_q_weight, size_k, size_n, 1, 4, /*a8=*/true);
   const size_t scratch_bytes = sonar_marlin_gemm_a8_scratch_bytes(size_m, size_n, size_k, num_groups);
-  Tensor scratch = at::empty({(int64_t)std::max<size_t>(scratch_bytes, 16)}, a.options().dtype(at::kByte));
+  Tensor scratch;
+  if (scratch_bytes > 0) scratch = at::empty({(int64_t)scratch_bytes}, a.options().dtype(at::kByte));
   raise_if_failed(sonar_marlin_gemm_a8(
       a.const_data_ptr(), a.stride(0), a_dtype, c.mutable_data_ptr(),
       static_cast<const uint32_t*>(native.const_data_ptr()), SONAR_LAYOUT_GFX950, opt_ptr(b_bias_or_none),
       b_scales.const_data_ptr(), static_cast<const float*>(a_scales->const_data_ptr()),
-      has_zp ? static_cast<const uint32_t*>(b_zeros_or_none->const_data_ptr()) : nullptr, scratch.mutable_data_ptr(),
-      scratch_bytes, dtype, b_type_id, size_m, size_n, size_k, num_groups, current_stream(a)));
+      has_zp ? static_cast<const uint32_t*>(b_zeros_or_none->const_data_ptr()) : nullptr,
+      scratch_bytes > 0 ? scratch.mutable_data_ptr() : nullptr, scratch_bytes, dtype, b_type_id, size_m, size_n, size_k,
+      num_groups, current_stream(a)));
   return c;
 }
 
@@ -789,6 +824,36 @@ Tensor marlin_gemm(const Tensor& a, const OptTensor& c_or_none, const Tensor& b_
       scratch_bytes, dtype, b_type_id, size_m, size_n, size_k, num_groups, is_k_full ? 1 : 0,
       use_atomic_add ? 1 : 0, use_fp32_reduce ? 1 : 0, current_stream(a)));
   return c;
+}
+
+// A linear layer on Marlin weights in one call: what apply_gptq_marlin_linear (marlin_utils.py:638-700),
+// apply_fp8_marlin_linear (marlin_utils_fp8.py:49-104) and apply_fp4_marlin_linear (marlin_utils_fp4.py:153-214)
+// do around the GEMM, for which a small call has no time in Python.  `act`: 0, or the type the activations are
+// quantised to (1: int8, their scales times `a_factor`; 2: float8_e4m3fn).
+Tensor marlin_linear(const Tensor& input, const Tensor& weight, const OptTensor& bias, const Tensor& scales,
+                     const OptTensor& a_factor, const OptTensor& global_scale, const OptTensor& zeros,
+                     const OptTensor& g_idx, const OptTensor& perm, const Tensor& workspace, int64_t b_type_id,
+                     int64_t size_n, int64_t size_k, bool is_k_full, bool use_fp32_reduce, int64_t act) {
+  TORCH_CHECK(input.dim() >= 1 && weight.dim() == 2, "input must have a dimension and the weight two");
+  const int64_t per_word = b_type_id == SONAR_TYPE_UINT8B128 || b_type_id == SONAR_TYPE_FLOAT8_E4M3FN ? 4 : 8;
+  const int64_t padded_k = weight.size(0) * 16, padded_n = weight.size(1) * per_word / 16;
+  Tensor x = input.dim() == 2 ? input : input.reshape({-1, input.size(-1)});
+  if (padded_k != size_k) x = at::constant_pad_nd(x, {0, padded_k - size_k});
+  OptTensor a_scales, c;
+  if (act != 0) {
+    if (b_type_id == SONAR_TYPE_FLOAT4_E2M1F) c = at::empty({x.size(0), padded_n}, input.options());
+    if (a_factor.has_value())
+      TORCH_CHECK(a_factor->is_cuda() && a_factor->scalar_type() == at::kFloat && a_factor->numel() == 1,
+                  "the factor of the activations' scales must be a float on the GPU");
+    std::tie(x, a_scales) = per_token_quant(x, act == 2, a_factor);
+  }
+  Tensor out = marlin_gemm(x, c, weight, bias, scales, a_scales, global_scale, zeros, g_idx, perm, workspace, b_type_id,
+                           x.size(0), padded_n, padded_k, is_k_full, false, use_fp32_reduce, false);
+  if (padded_n != size_n) out = out.narrow(-1, 0, size_n).contiguous();
+  if (input.dim() == 2) return out;
+  auto shape = input.sizes().vec();
+  shape.back() = size_n;
+  return out.reshape(shape);
 }
 
 // ---------------------------------------------------------------- grouped GEMM
@@ -1243,37 +1308,6 @@ void fused_moe(Tensor& output, const Tensor& hidden, const Tensor& w1, const Ten
   raise_if_failed(sonar_moe_sum(output.mutable_data_ptr(), wide.const_data_ptr(), m, topk, k, dtype, stream));
 }
 
-// Per-token quantisation of the activations of the W4A8 GEMM: (codes of x's shape, float32
-// scales (..., 1)).
-std::tuple<Tensor, Tensor> per_token_quant(const Tensor& x, bool fp8) {
-  TORCH_CHECK(x.is_cuda(), "x is not on GPU");
-  TORCH_CHECK(x.dim() >= 1 && x.size(-1) > 0, "x must have a non-empty last dimension");
-  int dtype;
-  if (x.scalar_type() == at::kHalf) dtype = SONAR_DTYPE_F16;
-  else if (x.scalar_type() == at::kBFloat16) dtype = SONAR_DTYPE_BF16;
-  else if (x.scalar_type() == at::kFloat) dtype = SONAR_DTYPE_F32;
-  else TORCH_CHECK(false, "per-token quantisation takes float16, bfloat16 or float32; got ", x.scalar_type());
-  const int64_t cols = x.size(-1);
-  const Tensor x2 = x.reshape({-1, cols});
-  const Tensor src = x2.stride(1) == 1 ? x2 : x2.contiguous();
-  const int64_t rows = src.size(0);
-  c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
-  Tensor q = at::empty(x.sizes(), x.options().dtype(fp8 ? at::kFloat8_e4m3fn : at::kChar));
-  auto scale_shape = x.sizes().vec();
-  scale_shape.back() = 1;
-  Tensor scales = at::empty(scale_shape, x.options().dtype(at::kFloat));
-  if (fp8)
-    raise_if_failed(sonar_per_token_quant_fp8(src.const_data_ptr(), dtype, rows ? src.stride(0) : cols,
-                                              static_cast<uint8_t*>(q.mutable_data_ptr()),
-                                              static_cast<float*>(scales.mutable_data_ptr()), rows, cols,
-                                              current_stream(x)));
-  else
-    raise_if_failed(sonar_per_token_quant_int8(src.const_data_ptr(), dtype, rows ? src.stride(0) : cols,
-                                               static_cast<int8_t*>(q.mutable_data_ptr()),
-                                               static_cast<float*>(scales.mutable_data_ptr()), rows, cols,
-                                               current_stream(x)));
-  return {q, scales};
-}
 std::tuple<Tensor, Tensor> per_token_quant_int8(const Tensor& x) { return per_token_quant(x, false); }
 std::tuple<Tensor, Tensor> per_token_quant_fp8(const Tensor& x) { return per_token_quant(x, true); }
 
@@ -1301,6 +1335,10 @@ TORCH_LIBRARY(sonar_amd, m) {
       "Tensor(b!)? cache13, Tensor(c!)? cache2, int b_type_id, int num_experts, int block_size, "
       "bool router_weight_on_input, bool is_k_full, int activation, float limit, float alpha, float beta) -> ()");
   m.def("per_token_quant_int8(Tensor x) -> (Tensor, Tensor)");
+  m.def(
+      "marlin_linear(Tensor input, Tensor weight, Tensor? bias, Tensor scales, Tensor? a_factor, Tensor? global_scale, "
+      "Tensor? zeros, Tensor? g_idx, Tensor? perm, Tensor workspace, int b_type_id, SymInt size_n, SymInt size_k, "
+      "bool is_k_full, bool use_fp32_reduce, int act) -> Tensor");
   m.def("gptq_marlin_moe_repack(Tensor b_q_weight, Tensor perm, SymInt size_k, SymInt size_n) -> Tensor");
   m.def("awq_marlin_moe_repack(Tensor b_q_weight, SymInt size_k, SymInt size_n) -> Tensor");
   m.def("permute_scales(Tensor s, bool grouped) -> Tensor");
@@ -1320,6 +1358,7 @@ TORCH_LIBRARY_IMPL(sonar_amd, CUDA, m) {
   m.impl("moe_sum", &moe_sum);
   m.impl("fused_moe", &fused_moe);
   m.impl("per_token_quant_int8", &per_token_quant_int8);
+  m.impl("marlin_linear", &marlin_linear);
   m.impl("gptq_marlin_moe_repack", &gptq_marlin_moe_repack);
   m.impl("awq_marlin_moe_repack", &awq_marlin_moe_repack);
   m.impl("permute_scales", &permute_scales);

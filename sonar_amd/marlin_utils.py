@@ -389,25 +389,13 @@ def apply_gptq_marlin_linear(input: torch.Tensor, weight: torch.Tensor, weight_s
                              bias: torch.Tensor | None = None,
                              use_fp32_reduce: bool = USE_FP32_REDUCE_DEFAULT,
                              input_dtype: torch.dtype | None = None) -> torch.Tensor:
-    reshaped_x = input.reshape(-1, input.shape[-1])
-    out_shape = input.shape[:-1] + (output_size_per_partition,)
-    padded_n, padded_k = marlin_repacked_nk(weight, wtype.size_bits)
-    reshaped_x = marlin_pad_dim(reshaped_x, input_size_per_partition, padded_k)
-    use_atomic_add = should_use_atomic_add_reduce(reshaped_x.size(0), padded_n, padded_k, input.device,
-                                                  input.dtype)
-    a_scales = None
+    act = 0
     if input_dtype == torch.int8:      # marlin_utils.py:671-680
         assert wtype == scalar_types.uint4b8, "W8A8-INT8 is not supported by marlin kernel."
-        reshaped_x, a_scales = marlin_quant_input(reshaped_x, input_dtype)
-        if input_global_scale is not None:
-            a_scales = a_scales * input_global_scale
+        act = 1
     elif input_dtype == torch.float8_e4m3fn:
         assert wtype == scalar_types.uint4b8, "INT8 weight + FP8 activation is not supported."
-        reshaped_x, a_scales = marlin_quant_input(reshaped_x, input_dtype)
-    output = ops.marlin_gemm(reshaped_x, None, weight, bias, weight_scale, a_scales, None, weight_zp, g_idx,
-                             g_idx_sort_indices, workspace, wtype, size_m=reshaped_x.shape[0],
-                             size_n=padded_n, size_k=padded_k, is_k_full=is_k_full,
-                             use_atomic_add=use_atomic_add, use_fp32_reduce=use_fp32_reduce,
-                             is_zp_float=False)
-    output = marlin_unpad_output(output, output_size_per_partition, padded_n)
-    return output.reshape(out_shape)
+        act = 2
+    return ops.marlin_linear(input, weight, bias, weight_scale, input_global_scale if act == 1 else None, None, weight_zp,
+                             g_idx, g_idx_sort_indices, workspace, wtype.id, output_size_per_partition,
+                             input_size_per_partition, is_k_full, use_fp32_reduce, act)

@@ -17,12 +17,12 @@ import torch
 
 from . import ops
 from .marlin_utils import (USE_FP32_REDUCE_DEFAULT, get_marlin_input_dtype, marlin_make_workspace_new,
-                           marlin_pad_dim, marlin_pad_qweight, marlin_pad_scales, marlin_padded_nk,
-                           marlin_permute_bias, marlin_permute_scales, marlin_quant_input, marlin_repacked_nk,
-                           marlin_unpad_output, should_use_atomic_add_reduce)
+                           marlin_pad_dim, marlin_pad_qweight, marlin_pad_scales, marlin_padded_nk, marlin_permute_bias,
+                           marlin_permute_scales)
 from .scalar_type import scalar_types
 
 MXFP4_GROUP_SIZE = 32
+_FP4_ID = scalar_types.float4_e2m1f.id
 FP4_MARLIN_SUPPORTED_GROUP_SIZES = [16]   # marlin_utils_fp4.py:29 (NVFP4)
 
 
@@ -95,28 +95,15 @@ def apply_fp4_marlin_linear(input: torch.Tensor, weight: torch.Tensor, weight_sc
                             size_k: int, bias: torch.Tensor | None = None, input_dtype: torch.dtype | None = None,
                             use_fp32_reduce: bool = USE_FP32_REDUCE_DEFAULT) -> torch.Tensor:
     """marlin_utils_fp4.py:153-214; with a global scale the weights are NVFP4."""
-    x = input.reshape(-1, input.shape[-1])
-    out_shape = input.shape[:-1] + (size_n,)
-    padded_n, padded_k = marlin_repacked_nk(weight, num_bits=4)
-    x = marlin_pad_dim(x, size_k, padded_k)
-    use_atomic_add = should_use_atomic_add_reduce(m=x.size(0), n=padded_n, k=padded_k, device=input.device,
-                                                  dtype=input.dtype)
-    a_scales, c = None, None
+    act = 0
     if input_dtype is not None and input_dtype.itemsize == 1:   # marlin_utils_fp4.py:185-191
         if weight_global_scale is not None:
             raise RuntimeError("NVFP4 weight + INT8/FP8 activation is not supported.")
         if input_dtype != torch.float8_e4m3fn:
             raise RuntimeError("MXFP4 weight + INT8 activation is not supported.")
-        # the op takes the output type from c in this mode (marlin.cu:576-590); the reference passes
-        # c = None here, which its op refuses
-        c = torch.empty((x.size(0), padded_n), dtype=input.dtype, device=input.device)
-        x, a_scales = marlin_quant_input(x, torch.float8_e4m3fn)
-    out = ops.marlin_gemm(a=x, c=c, b_q_weight=weight, b_bias=bias, b_scales=weight_scale, a_scales=a_scales,
-                          global_scale=weight_global_scale, b_zeros=None, g_idx=None, perm=None,
-                          workspace=workspace,
-                          b_q_type=scalar_types.float4_e2m1f, size_m=x.size(0), size_n=padded_n, size_k=padded_k,
-                          use_atomic_add=use_atomic_add, use_fp32_reduce=use_fp32_reduce)
-    return marlin_unpad_output(out, size_n, padded_n).reshape(out_shape)
+        act = 2   # (the result has the type of the input: the op wants it named in this mode, marlin.cu:576-590)
+    return ops.marlin_linear(input, weight, bias, weight_scale, None, weight_global_scale, None, None, None, workspace,
+                             _FP4_ID, size_n, size_k, True, use_fp32_reduce, act)
 
 
 def _set(layer, name: str, value: torch.Tensor) -> None:

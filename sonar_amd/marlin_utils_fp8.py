@@ -14,10 +14,11 @@ import torch.nn.functional as F
 
 from . import ops
 from .marlin_utils import (USE_FP32_REDUCE_DEFAULT, marlin_make_workspace_new, marlin_moe_padded_intermediate,
-                           marlin_pad_dim, marlin_pad_qweight, marlin_pad_scales, marlin_padded_nk,
-                           marlin_permute_bias, marlin_permute_scales, marlin_repacked_nk, marlin_unpad_output,
-                           should_use_atomic_add_reduce)
+                           marlin_pad_dim, marlin_pad_qweight, marlin_pad_scales, marlin_padded_nk, marlin_permute_bias,
+                           marlin_permute_scales)
 from .scalar_type import scalar_types
+
+_FP8_ID = scalar_types.float8_e4m3fn.id
 
 
 def is_fp8_marlin_supported() -> bool:
@@ -54,17 +55,8 @@ def apply_fp8_marlin_linear(input: torch.Tensor, weight: torch.Tensor, weight_sc
     """marlin_utils_fp8.py:49-104."""
     if input_dtype is not None and input_dtype.itemsize == 1:
         raise RuntimeError("Marlin W8A8 is not supported.")
-    x = input.reshape(-1, input.shape[-1])
-    out_shape = input.shape[:-1] + (size_n,)
-    padded_n, padded_k = marlin_repacked_nk(weight, num_bits=8)
-    x = marlin_pad_dim(x, size_k, padded_k)
-    use_atomic_add = should_use_atomic_add_reduce(m=x.size(0), n=padded_n, k=padded_k, device=input.device,
-                                                  dtype=input.dtype)
-    out = ops.marlin_gemm(a=x, c=None, b_q_weight=weight, b_bias=bias, b_scales=weight_scale, a_scales=None,
-                          global_scale=None, b_zeros=None, g_idx=None, perm=None, workspace=workspace,
-                          b_q_type=scalar_types.float8_e4m3fn, size_m=x.size(0), size_n=padded_n, size_k=padded_k,
-                          use_atomic_add=use_atomic_add, use_fp32_reduce=use_fp32_reduce)
-    return marlin_unpad_output(out, size_n, padded_n).reshape(out_shape)
+    return ops.marlin_linear(input, weight, bias, weight_scale, None, None, None, None, None, workspace, _FP8_ID, size_n,
+                             size_k, True, use_fp32_reduce, 0)
 
 
 def _set(layer, name: str, value: torch.Tensor) -> None:

@@ -45,6 +45,13 @@ def _register_fakes() -> None:
     def _(qweight, qzeros_or_none=None, inplace=False):
         return torch.empty_like(qweight)
 
+    @reg("sonar_amd::marlin_linear")
+    def _(input, weight, bias, scales, a_factor, global_scale, zeros, g_idx, perm, workspace, b_type_id, size_n, size_k,
+          is_k_full, use_fp32_reduce, act):
+        # with quantised activations the result has the type of 16-bit scales
+        dtype = scales.dtype if act and scales.element_size() == 2 else input.dtype
+        return torch.empty(input.shape[:-1] + (size_n,), dtype=dtype, device=input.device)
+
     def quant_fake(code_dtype):
         def fake(x):
             return (torch.empty(x.shape, dtype=code_dtype, device=x.device),
@@ -182,6 +189,9 @@ def marlin_gemm(a: torch.Tensor, c: torch.Tensor | None, b_q_weight: torch.Tenso
 
 
 gptq_marlin_gemm = marlin_gemm  # the op's older name
+
+# a linear layer in one op call (no reference counterpart): torch_bindings.cpp says what each argument is
+marlin_linear = torch.ops.sonar_amd.marlin_linear.default
 
 
 def moe_wna16_marlin_gemm(input: torch.Tensor, output: torch.Tensor | None, b_qweight: torch.Tensor,
