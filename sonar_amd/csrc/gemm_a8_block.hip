@@ -143,16 +143,17 @@ __global__ __launch_bounds__(64 * S * RG) __attribute__((amdgpu_waves_per_eu(2, 
 
   // Workgroup ids congruent mod 8 run on one XCD: each takes a contiguous run of tiles, the row tiles of the same
   // columns next to each other.
-  const int per_xcd = (p.tiles + 7) / 8;
-  const int tile = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-  if ((int)(blockIdx.x >> 3) >= per_xcd || tile >= p.tiles) return;
+  const int units = p.tiles * p.splits, per_xcd = (units + 7) / 8;
+  const int unit = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= per_xcd || unit >= units) return;
+  const int split = unit / p.tiles, tile = unit - split * p.tiles;
   const int tile_n = tile / p.tiles_m, tile_m = tile - tile_n * p.tiles_m;
   const int m0 = tile_m * 32 * R;
   const int strips = p.size_n / kStripN;
   const bool active = tile_n * S + ws < strips;   // strips past the last repeat it and are not stored
   const int strip = __builtin_amdgcn_readfirstlane(active ? tile_n * S + ws : strips - 1);
 
-  const int first = blockIdx.y * p.split_steps;            // of the steps this workgroup takes
+  const int first = split * p.split_steps;       // of the steps this workgroup takes
   const int all_steps = p.size_k / kStepK, steps = min(first + p.split_steps, all_steps);
   const int per_range = (steps - first + RG - 1) / RG;
   const int k_first = first + range * per_range;
@@ -452,8 +453,8 @@ __global__ __launch_bounds__(64 * S * RG) __attribute__((amdgpu_waves_per_eu(2, 
     if (row >= p.size_m || !active) return;
     if constexpr (kShifted) total >>= 4;
     const int col = strip * kStripN + 32 * j + l32;
-    if (gridDim.y > 1) {
-      p.partial[((size_t)blockIdx.y * p.size_m + row) * p.size_n + col] = a8_bits(total);
+    if (p.splits > 1) {
+      p.partial[((size_t)split * p.size_m + row) * p.size_n + col] = a8_bits(total);
       return;
     }
     float f = (float)total * p.a_scales[row];
@@ -518,9 +519,10 @@ int launch_a8_shape(A8BlockParams p, int splits, hipStream_t st) {
                                   hipFuncAttributeMaxDynamicSharedMemorySize, lds));
     attr_set = true;
   }
+  p.splits = splits;
   p.tiles_m = (p.size_m + 32 * R - 1) / (32 * R);
   p.tiles = p.tiles_m * ((p.size_n / kStripN + S - 1) / S);
-  marlin_a8_block<ACT, ZP, GC, R, S, RG><<<dim3((p.tiles + 7) / 8 * 8, splits), 64 * S * RG, lds, st>>>(p);
+  marlin_a8_block<ACT, ZP, GC, R, S, RG><<<(p.tiles * splits + 7) / 8 * 8, 64 * S * RG, lds, st>>>(p);
   return launch_status("marlin_a8_block");
 }
 

@@ -19,7 +19,7 @@ struct A8BlockParams {
   int group_chunks;          // 32-row chunks per group: 1 (int8 only), 2, 4; 0: channelwise
   int bf16;                  // output (and scale) type
   uint32_t* partial;         // [splits][M][N] raw totals when splits > 1
-  int tiles_m, tiles, split_steps;   // filled in by a8_block_gemm
+  int tiles_m, tiles, splits, split_steps;   // filled in by a8_block_gemm
 };
 
 // Tile of a workgroup: 32 * rows rows of C, 64 * strips columns, K in `ranges` parts; K split over `splits` workgroups,

@@ -1,6 +1,6 @@
 // The GEMM between decode and prefill: from a few tens of rows up to where the tiles of the wide tile
-// kernel (gemm_tile.hip) fill the chip.  A workgroup owns 16 MB rows x 128 columns over the whole of K:
-// no partial tile goes through memory and no second launch sums them.
+// kernel (gemm_tile.hip) fill the chip.  A workgroup owns 16 MB rows x 128 columns over the whole of K, so that no
+// partial tile goes through memory; where that leaves compute units idle, a part of K, and a second kernel adds the parts.
 //
 // Eight wavefronts: two strips of 64 columns x four ranges of K.  So every packed chunk is dequantised
 // exactly once in the workgroup, a wavefront's accumulators are small (16 MB registers), two wavefronts
@@ -17,6 +17,9 @@
 //   M   64, K 4096, N 28672, bf16: 29.1 -> 23.0      M  200, K 4096, N 6144, fp16, zero points: 24.6 -> 21.0
 //   M  333, K 2880, N  5760, bf16, groups of 32: 40.5 -> 21.7      M  512, K 4096, N 2048, bf16: 36 -> 20
 //   M  128, K 2048, N 20032, MXFP4: 47.6 -> 20.5     M   96, K 2048, N 20032, 8-bit codes: 48 -> 18.5
+// and with K split over workgroups, where there are fewer tiles than compute units:
+//   M  101, K 2048, N 1536, bf16, zero points: 27.8 -> 10.6      M  125, K 6528, N 4672, bf16: 44.5 -> 20.8
+//   M   76, K 9088, N 1920, MXFP4: 32.4 -> 14.5                  M   84, K 9088, N 2560, 8-bit codes: 32.5 -> 16.1
 // Tried and slower: one strip a workgroup with eight ranges (half the dequantisation per workgroup, but twice the
 // activation bytes through the copy path per matrix instruction: 200 rows above 23 us, 64 rows on N = 28672 31 us).
 //
@@ -93,9 +96,10 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
 
   // Workgroup ids congruent mod 8 run on one XCD: each XCD takes a contiguous run of tiles, the row tiles
   // of a pair of strips next to each other, so the second to ask for a chunk finds it in that L2.
-  const int per_xcd = (p.tiles + 7) / 8;
-  const int tile = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-  if ((int)(blockIdx.x >> 3) >= per_xcd || tile >= p.tiles) return;
+  const int units = p.tiles * p.splits, per_xcd = (units + 7) / 8;
+  const int unit = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= per_xcd || unit >= units) return;
+  const int split = unit / p.tiles, tile = unit - split * p.tiles;
   const int tile_n = tile / p.tiles_m, tile_m = tile - tile_n * p.tiles_m;
   const int m0 = tile_m * 16 * MB;
   const int strips = p.size_n / kStripN;
@@ -103,9 +107,10 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
   const bool active = tile_n * kMidStrips + (wave & 1) < strips;
   const int strip = __builtin_amdgcn_readfirstlane(active ? tile_n * kMidStrips + (wave & 1) : strips - 1);
 
-  const int steps = p.size_k / kMidStepK;
-  const int per_range = (steps + kMidRanges - 1) / kMidRanges;
-  const int k_first = range * per_range;
+  const int first = split * p.split_steps;   // of the steps this workgroup takes
+  const int steps = min(first + p.split_steps, p.size_k / kMidStepK);
+  const int per_range = (steps - first + kMidRanges - 1) / kMidRanges;
+  const int k_first = first + range * per_range;
 
   // ---- sources.  The activations of a range are copied by its own two wavefronts, MB copies each of 8 rows x
   // one 128-byte line; piece q of row r sits at 16-byte slot q ^ r of the row, off the other rows' banks.
@@ -353,8 +358,12 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
         v += floatx4_t{s.x, s.y, s.z, s.w};
       }
       if (row >= p.size_m) continue;
-      if (FMT == kMidNvFp4) v = v * gs;
       const int nl = 16 * j + 4 * kb;
+      if (p.splits > 1) {
+        p.partial[(((size_t)split * p.size_m + row) * p.size_n + strip * kStripN + nl) / 4] = make_float4(v.x, v.y, v.z, v.w);
+        continue;
+      }
+      if (FMT == kMidNvFp4) v = v * gs;
       float bias[4] = {0.f, 0.f, 0.f, 0.f};
       if (p.bias) {
 #pragma unroll
@@ -368,6 +377,33 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
   }
 }
 
+// Adds the totals of up to kMost K splits, four columns a thread, in the order of K.  (All loads are asked for before the
+// first is waited for: one after the other, seven splits took 5 us longer than two.)
+template <typename T, int kMost>
+__global__ __launch_bounds__(256) void marlin_mid_sum(const MidParams p) {
+  const size_t quads = (size_t)p.size_m * p.size_n / 4;
+  const float gs = p.global_scale ? p.global_scale[0] : 1.f;
+  for (size_t q = (size_t)blockIdx.x * 256 + threadIdx.x; q < quads; q += (size_t)gridDim.x * 256) {
+    float4 w[kMost];
+#pragma unroll
+    for (int s = 0; s < kMost; ++s) w[s] = p.partial[(s < p.splits ? s : 0) * quads + q];
+    float4 v = w[0];
+#pragma unroll
+    for (int s = 1; s < kMost; ++s)
+      if (s < p.splits) v.x += w[s].x, v.y += w[s].y, v.z += w[s].z, v.w += w[s].w;
+    const int col = (int)(4 * q % p.size_n), nl = col & (kStripN - 1);
+    float bias[4] = {0.f, 0.f, 0.f, 0.f};
+    if (p.bias) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) bias[r] = Dq<T>::to_float(p.bias[col - nl + scale_slot(nl + r, false)]);
+    }
+    uint2 o;
+    o.x = (uint32_t)Dq<T>::from_float(v.x * gs + bias[0]) | ((uint32_t)Dq<T>::from_float(v.y * gs + bias[1]) << 16);
+    o.y = (uint32_t)Dq<T>::from_float(v.z * gs + bias[2]) | ((uint32_t)Dq<T>::from_float(v.w * gs + bias[3]) << 16);
+    reinterpret_cast<uint2*>(p.c)[q] = o;
+  }
+}
+
 template <typename T, int FMT, int GROUPS, int MB>
 int launch_mid_rows(const MidParams& p, hipStream_t st) {
   static bool attr_set = false;   // raising the dynamic LDS limit is needed once per form
@@ -376,7 +412,7 @@ int launch_mid_rows(const MidParams& p, hipStream_t st) {
                                   hipFuncAttributeMaxDynamicSharedMemorySize, mid_lds(MB)));
     attr_set = true;
   }
-  marlin_mid_gemm<T, FMT, GROUPS, MB><<<(p.tiles + 7) / 8 * 8, kMidWaves * 64, mid_lds(MB), st>>>(p);
+  marlin_mid_gemm<T, FMT, GROUPS, MB><<<(p.tiles * p.splits + 7) / 8 * 8, kMidWaves * 64, mid_lds(MB), st>>>(p);
   return launch_status("marlin_mid_gemm");
 }
 
@@ -422,8 +458,22 @@ int mid_gemm(MidParams p, int dtype, int format, int row_blocks, hipStream_t st)
   const int strips = p.size_n / kStripN;
   p.tiles_m = (p.size_m + 16 * row_blocks - 1) / (16 * row_blocks);
   p.tiles = p.tiles_m * ((strips + kMidStrips - 1) / kMidStrips);
-  return dtype == SONAR_DTYPE_F16 ? launch_mid_format<_Float16>(p, format, row_blocks, st)
-                                  : launch_mid_format<__bf16>(p, format, row_blocks, st);
+  const int steps = p.size_k / kMidStepK;
+  p.split_steps = (steps + p.splits - 1) / p.splits;
+  p.splits = (steps + p.split_steps - 1) / p.split_steps;
+  const int rc = dtype == SONAR_DTYPE_F16 ? launch_mid_format<_Float16>(p, format, row_blocks, st)
+                                          : launch_mid_format<__bf16>(p, format, row_blocks, st);
+  if (rc || p.splits == 1) return rc;
+  const int blocks = (int)std::min<int64_t>(((int64_t)p.size_m * p.size_n / 4 + 255) / 256, 2048);
+  if (p.splits > kMidMostSplits) return fail(SONAR_E_INVALID, "internal: %d K splits", p.splits);
+  if (dtype == SONAR_DTYPE_F16) {
+    if (p.splits <= 4) marlin_mid_sum<_Float16, 4><<<blocks, 256, 0, st>>>(p);
+    else marlin_mid_sum<_Float16, kMidMostSplits><<<blocks, 256, 0, st>>>(p);
+  } else {
+    if (p.splits <= 4) marlin_mid_sum<__bf16, 4><<<blocks, 256, 0, st>>>(p);
+    else marlin_mid_sum<__bf16, kMidMostSplits><<<blocks, 256, 0, st>>>(p);
+  }
+  return launch_status("marlin_mid_sum");
 }
 
 }  // namespace sonar

@@ -9,6 +9,8 @@ namespace sonar {
 // Weight formats of the kernel in gemm_mid.hip.
 enum MidFormat { kMidInt4 = 0, kMidInt4Zp = 1, kMidInt8 = 2, kMidFp8 = 3, kMidMxFp4 = 4, kMidNvFp4 = 5 };
 
+constexpr int kMidMostSplits = 8;
+
 struct MidParams {
   const uint16_t* a;
   long lda;                  // elements between rows of a
@@ -21,7 +23,9 @@ struct MidParams {
   int size_m, size_n, size_k, num_groups;
   int group_shift;           // log2 of the 64-row steps per group; -1: groups of 32 or 16 rows
   int chunks_per_strip;
-  int tiles_m, tiles;        // filled in by mid_gemm
+  int splits;                // of K over workgroups; their totals go to `partial` and a second kernel adds them
+  float4* partial;           // [splits][M][N / 4]
+  int tiles_m, tiles, split_steps;   // filled in by mid_gemm
 };
 
 // Whether the kernel can run a call (no act-order gather; rows of a within 4 GiB; groups of 16, 32 or 64 * 2^i rows or
@@ -33,24 +37,31 @@ inline bool mid_applies(int64_t size_m, int64_t size_k, int64_t lda, int64_t num
   return group_size % 64 == 0 && (per & (per - 1)) == 0;
 }
 
-// Microseconds a call takes in tiles of the best number of row blocks, which is returned in `row_blocks`.  A fit
-// of measured times (K = 2048 and 4096, N = 2048, 6144 and 20032, 17 to 768 rows, all formats, within 10 %): about
-// 6 us around the loop, per round of workgroups and 4096 rows of K 1.5 us for a row block's matrix instructions
-// and a time that depends on the format for the dequantisation, which the matrix instructions do not hide.
+// Microseconds a call takes in tiles of the best number of row blocks and splits of K, which are returned in
+// `row_blocks` and `splits`.  A fit of measured times (K = 2048 and 4096, N = 2048, 6144 and 20032, 17 to 768 rows, all
+// formats, mostly within 15 %): 4 us around the loop of a round of workgroups, and per 4096 rows of K 1.5 us for a row
+// block's matrix instructions and a time that depends on the format for the dequantisation, which the matrix
+// instructions do not hide; more at the clock of a full chip than of a half empty one; no less than the weights take
+// from memory.  K is split where the tiles leave compute units idle, if the totals fit `room` bytes; the
+// pass that adds them is 3.3 us and its bytes.
 inline double mid_estimate(int64_t size_m, int64_t size_n, int64_t size_k, int64_t num_groups, int dtype, int format,
-                           int cus, int& row_blocks) {
+                           int cus, size_t room, int& row_blocks, int& splits) {
   static const double kDequant[6][2] = {   // float16, bfloat16
       {6.8, 8.8}, {8.3, 10.0}, {6.0, 10.2}, {8.0, 15.5}, {5.3, 5.3}, {9.0, 13.3}};
-  const double k = ((size_k / 64 + 3) / 4) * 256 / 4096.0;
   const double dequant = kDequant[format][dtype == 0 ? 0 : 1] + (num_groups > 1 && size_k / num_groups == 32 && format != kMidMxFp4 ? 0.8 : 0.0);
+  const int64_t steps = size_k / 64;
+  const double memory = 4.0 + size_n * size_k * (format == kMidInt8 || format == kMidFp8 ? 1.0 : 0.5) / 4.5e6;
   double best = 1e30;
   for (int mb = 2; mb <= 6; ++mb) {
     const int64_t tiles = ((size_m + 16 * mb - 1) / (16 * mb)) * ((size_n + 127) / 128);
-    const int64_t rounds = (tiles + cus - 1) / cus;
-    const double us = 5.0 + rounds * (1.0 + k * (dequant + 1.5 * mb));
-    if (us < best) {
-      best = us;
-      row_blocks = mb;
+    for (int n = 1; n <= kMidMostSplits; ++n) {
+      if (n > 1 && (tiles * n > cus || steps < 8 * n || (size_t)n * size_m * size_n * 4 > room)) break;
+      const double k = (((steps + n - 1) / n + 3) / 4) * 256 / 4096.0;
+      const int64_t groups = tiles * n, rounds = (groups + cus - 1) / cus;
+      double us = 1.5 + rounds * (4.0 + k * (dequant + 1.5 * mb) * (rounds > 2 ? 1.3 : 2 * groups > cus ? 1.1 : 0.85));
+      if (us < memory) us = memory;
+      if (n > 1) us += 3.3 + 2e-6 * n * size_m * size_n;
+      if (us < best) best = us, row_blocks = mb, splits = n;
     }
   }
   return best;

@@ -19,6 +19,7 @@
 // shares nothing and needs no second kernel.
 #include <algorithm>
 #include <cstdlib>
+#include <cstring>
 
 #include "dequant.hpp"
 #include "gemm_mid.hpp"
@@ -1905,19 +1906,34 @@ int marlin_gemm_any(const void* a, int64_t a_row_stride, void* c, const uint32_t
       mid_applies(size_m, size_k, a_row_stride, num_groups, chk.group_size)) {
     const int format = chk.nvfp4 ? kMidNvFp4 : chk.fp4 ? kMidMxFp4 : chk.bits == 8 ? (chk.fp8 ? kMidFp8 : kMidInt8)
                        : chk.has_zp ? kMidInt4Zp : kMidInt4;
-    int row_blocks;
-    const double mid_us = mid_estimate(size_m, size_n, size_k, num_groups, dtype, format, cus, row_blocks);
+    int row_blocks, splits;
+    const double mid_us = mid_estimate(size_m, size_n, size_k, num_groups, dtype, format, cus, base_scratch, row_blocks, splits);
     const double x = (double)size_n * size_k / (6144.0 * 4096.0), r = size_m / 64.0;
     // (what the other kernels take, us: fits of measured times, see mid_estimate)
     double us;
-    if (slab_fast)
+    if (slab_fast && n_strips < 64) {   // strips in as many pieces as powers of two divide their units: often one
+      int pieces = 1;
+      while (pieces < 8 && n_strips * 2 * pieces * ((size_m + 15) / 16) <= cus && (p.chunks_per_strip / 4) % (2 * pieces) == 0)
+        pieces *= 2;
+      us = 4.5 + 3.3 * (size_k / 4096.0) / pieces;
+    } else if (slab_fast) {
       us = 6.5 + 0.0245 * (size_k / 4096.0) * n_strips * ((size_m + 31) / 32) * (size_m <= 64 && n_strips < cus / 2 ? 0.6 : 1.0);
-    else if (use_tile)
-      us = 25.0 + 0.69e-9 * 2.0 * size_m * size_n * size_k;
-    else
-      us = size_m <= 64 ? 9.5 + x * (5.5 + 5.2 * r * r) : 11.0 + 10.7 * x * r;
-    if (mid_env) row_blocks = std::max(2, std::min(6, atoi(mid_env)));
-    if (mid_env || (mid_us < 0.93 * us && size_n * size_k >= 4 * 1000 * 1000)) {
+    } else if (use_tile) {
+      // us per 1e9 operations: the wide kernel on 4-bit codes, on others, and the kernel with eight wavefronts
+      const int64_t steps = size_k / 64, padding = (4 - steps % 4) % 4;
+      const bool wide = chk.fp4 || (num_groups > 1 && chk.group_size == 32) ? padding == 0 : padding * 10 <= steps;
+      const double rate = chk.bits == 8 ? 1.05 : chk.fp4 ? 0.78 : wide || (dtype == SONAR_DTYPE_F16 && !chk.has_zp) ? 0.72 : 1.5;
+      us = 25.0 + rate * 2e-9 * ((size_m + 127) / 128 * 128) * size_n * size_k;
+    } else {   // (few strips: shared between workgroups, and a second launch that adds the shares)
+      us = size_m <= 64 ? (n_strips < 64 ? 12.0 : 9.5) + x * (5.5 + 5.2 * r * r) : 11.0 + 10.7 * x * r;
+    }
+    if (mid_env) {   // "row blocks" or "row blocks,splits"
+      const char* comma = strchr(mid_env, ',');
+      row_blocks = std::max(2, std::min(6, atoi(mid_env)));
+      splits = comma ? std::max(1, std::min(kMidMostSplits, atoi(comma + 1))) : 1;
+      if ((size_t)splits * size_m * size_n * 4 > base_scratch || splits > size_k / 64) splits = 1;
+    }
+    if (mid_env || mid_us < 0.93 * us) {
       MidParams q = {};
       q.a = static_cast<const uint16_t*>(a);
       q.lda = a_row_stride;
@@ -1933,6 +1949,8 @@ int marlin_gemm_any(const void* a, int64_t a_row_stride, void* c, const uint32_t
       q.num_groups = (int)num_groups;
       q.group_shift = chk.group_size < 64 ? -1 : 31 - __builtin_clz(chk.group_size / 64);
       q.chunks_per_strip = p.chunks_per_strip;
+      q.splits = splits;
+      q.partial = static_cast<float4*>(scratch);
       return mid_gemm(q, dtype, format, row_blocks, st);
     }
   }

@@ -1,5 +1,6 @@
 """Child process of test_gpu_mid_rows: with SONAR_MARLIN_MID_ROWS set (read once per process) every
-dense call that the kernel of gemm_mid.hip can run goes to its tiles of that many row blocks, here at the
+dense call that the kernel of gemm_mid.hip can run goes to its tiles of that many row blocks ("rows,splits": with K
+split over workgroups as well), here at the
 edges of tiles, strips and K ranges, for every weight format, against the oracle."""
 from __future__ import annotations
 
@@ -25,7 +26,7 @@ def int4(m, k, n, g, dtype, zp, bias) -> None:
 
 
 def main() -> None:
-    rows = 16 * int(os.environ["SONAR_MARLIN_MID_ROWS"])
+    rows = 16 * int(os.environ["SONAR_MARLIN_MID_ROWS"].split(",")[0])
     # one step of K for four ranges; an odd last strip; a last tile of one row; ranges of unequal length; many tiles
     shapes = [(1, 64, 64), (rows, 320, 192), (rows + 1, 1344, 448), (2 * rows - 1, 512, 1088), (5 * rows + 3, 1024, 128)]
     for i, (m, k, n) in enumerate(shapes):
