@@ -211,7 +211,7 @@ struct DqF4Generic {
   }
   // codes in bits 12-15 and 28-31 of y -> two scaled values of T
   static __device__ __forceinline__ uint32_t pair(uint32_t y, float s) {
-    const half2_t h = __builtin_bit_cast(half2_t, (y & 0x80008000u) | ((y & 0x70007000u) >> 3));
+    const half2_t h = __builtin_bit_cast(half2_t, __builtin_bit_cast(uint32_t, __builtin_bit_cast(short2_t, y) >> 3) & 0x8e008e00u);
     return (uint32_t)Dq<T>::from_float((float)h.x * s) | ((uint32_t)Dq<T>::from_float((float)h.y * s) << 16);
   }
   static __device__ __forceinline__ vec8 word(uint32_t q, const Col& c, uint32_t) {
@@ -242,7 +242,7 @@ struct DqNvF4<_Float16> {
     return Col{b | (b << 16)};
   }
   static __device__ __forceinline__ uint32_t pair(uint32_t y, uint32_t s2) {
-    const half2_t h = __builtin_bit_cast(half2_t, (y & 0x80008000u) | ((y & 0x70007000u) >> 3));
+    const half2_t h = __builtin_bit_cast(half2_t, __builtin_bit_cast(uint32_t, __builtin_bit_cast(short2_t, y) >> 3) & 0x8e008e00u);
     return __builtin_bit_cast(uint32_t, h * __builtin_bit_cast(half2_t, s2));
   }
   static __device__ __forceinline__ vec8 word(uint32_t q, const Col& c, uint32_t) {
@@ -392,7 +392,7 @@ template <typename T>
 struct Dq8F;
 
 __device__ __forceinline__ uint32_t fp8_pair_as_fp16(uint32_t y) {  // codes in bits 8-15 and 24-31
-  return (y & 0x80008000u) | ((y & 0x7f007f00u) >> 1);
+  return __builtin_bit_cast(uint32_t, __builtin_bit_cast(short2_t, y) >> 1) & 0xbf80bf80u;   // (sign kept, its copy cleared)
 }
 
 template <>

@@ -20,6 +20,10 @@
 // and with K split over workgroups, where there are fewer tiles than compute units:
 //   M  101, K 2048, N 1536, bf16, zero points: 27.8 -> 10.6      M  125, K 6528, N 4672, bf16: 44.5 -> 20.8
 //   M   76, K 9088, N 1920, MXFP4: 32.4 -> 14.5                  M   84, K 9088, N 2560, 8-bit codes: 32.5 -> 16.1
+// Up to 16 rows of the formats that the decode kernel does not have take one row block and one strip a workgroup: eight
+// ranges of K, so that 64 columns are enough to keep a compute unit busy (two strips: 4096 x 11008 18.6 us, one: 17.3).
+//   M    8, K 4096, N 11008, fp8, bf16: 19.9 -> 17.3     M    8, K 2048, N 1536, 8-bit codes: 12.3 -> 7.4
+//   M    8, K 8192, N  8192, fp8, bf16: 30.5 -> 22.4     M    8, K 4096, N 28672, NVFP4: 33.3 -> 23.4
 // Tried and slower: one strip a workgroup with eight ranges (half the dequantisation per workgroup, but twice the
 // activation bytes through the copy path per matrix instruction: 200 rows above 23 us, 64 rows on N = 28672 31 us).
 //
@@ -44,13 +48,16 @@ namespace sonar {
 namespace {
 
 constexpr int kMidWaves = 8;
-constexpr int kMidStrips = 2;     // strips of a workgroup
-constexpr int kMidRanges = 4;     // ranges of K
+constexpr int mid_strips(int mb) { return mb == 1 ? 1 : 2; }                 // strips of a workgroup
+constexpr int mid_ranges(int mb) { return kMidWaves / mid_strips(mb); }      // ranges of K
 constexpr int kMidStepK = 64;     // rows of K a step takes from each range
 
-// Activation stages in LDS: MB x 8 KiB each.
-constexpr int mid_stages(int mb) { return mb <= 4 ? 4 : 3; }
-constexpr int mid_stage_bytes(int mb) { return mb * 8192; }
+// Activation stages in LDS.
+constexpr int mid_stages(int mb) { return mb > 1 && mb <= 4 ? 4 : 3; }
+// Wavefronts a SIMD: two (one workgroup a compute unit), or four for a single row block, whose loop is so short that two
+// workgroups are needed to keep enough bytes under way.
+constexpr int mid_waves_per_simd(int mb) { return mb == 1 ? 4 : 2; }
+constexpr int mid_stage_bytes(int mb) { return mid_ranges(mb) * mb * 2048; }
 constexpr int mid_sum_rows(int mb) { return mb < 4 ? mb : 4; }   // row blocks summed at a time at the end
 constexpr int mid_lds(int mb) {
   const int stages = mid_stages(mb) * mid_stage_bytes(mb), sum = kMidWaves * mid_sum_rows(mb) * 4096;
@@ -71,7 +78,7 @@ struct MidDequant {
 };
 
 template <typename T, int FMT, int GROUPS, int MB>
-__global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void marlin_mid_gemm(
+__global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(mid_waves_per_simd(MB), mid_waves_per_simd(MB)))) void marlin_mid_gemm(
     const MidParams p) {
   typedef MidDequant<T, FMT> Fmt;
   typedef typename Fmt::D4 D4;
@@ -82,16 +89,18 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
   constexpr int D = mid_stages(MB);
   constexpr int W = D - 1;                           // ring of the packed codes and scales in registers
   constexpr int kStage = mid_stage_bytes(MB);
+  constexpr int kMidStrips = mid_strips(MB), kMidRanges = mid_ranges(MB);
+  constexpr int kCopies = 2 * MB / kMidStrips;       // 8-row copies of activations per wavefront and step
   constexpr int kLoads = Fmt::k8 ? 4 : 2;            // 16-byte loads of packed codes per lane and step
   constexpr int kScaleRows = GROUPS == kChunkGroups ? 2 : 1;
   // memory operations per wavefront and step
-  constexpr int kOps = MB + kLoads + (GROUPS == kOneGroup ? 0 : kScaleRows * (kZero ? 2 : 1));
+  constexpr int kOps = kCopies + kLoads + (GROUPS == kOneGroup ? 0 : kScaleRows * (kZero ? 2 : 1));
   extern __shared__ __attribute__((aligned(1024))) char smem[];
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col16 = lane & 15, kb = lane >> 4;
-  const int range = wave >> 1;
+  const int range = wave / kMidStrips, strip_of = wave % kMidStrips;
   const uint32_t magic = magic_register();
 
   // Workgroup ids congruent mod 8 run on one XCD: each XCD takes a contiguous run of tiles, the row tiles
@@ -104,20 +113,20 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
   const int m0 = tile_m * 16 * MB;
   const int strips = p.size_n / kStripN;
   // (the second strip of an odd last pair is the first again, and not stored)
-  const bool active = tile_n * kMidStrips + (wave & 1) < strips;
-  const int strip = __builtin_amdgcn_readfirstlane(active ? tile_n * kMidStrips + (wave & 1) : strips - 1);
+  const bool active = tile_n * kMidStrips + strip_of < strips;
+  const int strip = __builtin_amdgcn_readfirstlane(active ? tile_n * kMidStrips + strip_of : strips - 1);
 
   const int first = split * p.split_steps;   // of the steps this workgroup takes
   const int steps = min(first + p.split_steps, p.size_k / kMidStepK);
   const int per_range = (steps - first + kMidRanges - 1) / kMidRanges;
   const int k_first = first + range * per_range;
 
-  // ---- sources.  The activations of a range are copied by its own two wavefronts, MB copies each of 8 rows x
+  // ---- sources.  The activations of a range are copied by its own wavefronts, kCopies copies each of 8 rows x
   // one 128-byte line; piece q of row r sits at 16-byte slot q ^ r of the row, off the other rows' banks.
-  uint32_t a_off[MB];
+  uint32_t a_off[kCopies];
 #pragma unroll
-  for (int i = 0; i < MB; ++i) {
-    int row = m0 + 8 * ((wave & 1) * MB + i) + (lane >> 3);
+  for (int i = 0; i < kCopies; ++i) {
+    int row = m0 + 8 * (strip_of * kCopies + i) + (lane >> 3);
     if (row >= p.size_m) row = p.size_m - 1;   // rows past M are computed and never stored
     a_off[i] = (uint32_t)row * (uint32_t)(p.lda * 2) + 16 * ((lane & 7) ^ (lane >> 3));
   }
@@ -140,7 +149,7 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
     if (op < kLoads) {
       const char* b_src = b_base + (size_t)k * (kLoads * 1024);
       asm volatile("global_load_dwordx4 %0, %1, %2 offset:%3" : "=&v"(wq[R][op]) : "v"(b_off), "s"(b_src), "i"(op * 1024) : "memory");
-    } else if (op < kOps - MB) {
+    } else if (op < kOps - kCopies) {
       const int h = (op - kLoads) / (kZero ? 2 : 1);
       const int g = GROUPS == kStepGroups ? k >> p.group_shift : (FMT == kMidNvFp4 ? 2 : 1) * (2 * k + h);
       if (!kZero || (op - kLoads) % 2 == 0) {
@@ -151,10 +160,10 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
         asm volatile("global_load_dword %0, %1, %2" : "=&v"(zv[R][h]) : "v"(z_off), "s"(z_src) : "memory");
       }
     } else {
-      const int i = op - (kOps - MB);
+      const int i = op - (kOps - kCopies);
       const char* a_src = reinterpret_cast<const char*>(p.a) + (size_t)k * (kMidStepK * 2);
       __builtin_amdgcn_global_load_lds((glb_void_t*)(a_src + a_off[i]),
-                                       (lds_void_t*)(a_stage + slot * kStage + ((wave & 1) * MB + i) * 1024), 16, 0, 0);
+                                       (lds_void_t*)(a_stage + slot * kStage + (strip_of * kCopies + i) * 1024), 16, 0, 0);
     }
   };
   // until only the `n` youngest operations are outstanding; the registers of ring position R are in its hands
@@ -347,14 +356,16 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < kSum; ++u) {
-      const int q = range * kSum + u;
+      constexpr int kEach = kSum * 4 / kMidRanges;   // accumulator tiles a wavefront adds
+      if (kEach > 0 ? u >= kEach : range >= 4 * kSum) continue;
+      const int q = kEach > 0 ? range * kEach + u : range;
       const int i = round + (q >> 2), j = q & 3;
       const int row = m0 + 16 * i + col16;
       if (i >= MB || !active) continue;
       floatx4_t v = floatx4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int g = 0; g < kMidRanges; ++g) {
-        const float4 s = sums[(((2 * g + (wave & 1)) * kSum + (q >> 2)) * 4 + j) * 64 + lane];
+        const float4 s = sums[(((kMidStrips * g + strip_of) * kSum + (q >> 2)) * 4 + j) * 64 + lane];
         v += floatx4_t{s.x, s.y, s.z, s.w};
       }
       if (row >= p.size_m) continue;
@@ -419,6 +430,8 @@ int launch_mid_rows(const MidParams& p, hipStream_t st) {
 template <typename T, int FMT, int GROUPS>
 int launch_mid(const MidParams& p, int row_blocks, hipStream_t st) {
   switch (row_blocks) {
+    case 1:
+      if constexpr (FMT == kMidInt8 || FMT == kMidFp8 || FMT == kMidNvFp4) return launch_mid_rows<T, FMT, GROUPS, 1>(p, st);
     case 2: return launch_mid_rows<T, FMT, GROUPS, 2>(p, st);
     case 3: return launch_mid_rows<T, FMT, GROUPS, 3>(p, st);
     case 4: return launch_mid_rows<T, FMT, GROUPS, 4>(p, st);
@@ -456,8 +469,10 @@ int launch_mid_format(const MidParams& p, int format, int row_blocks, hipStream_
 
 int mid_gemm(MidParams p, int dtype, int format, int row_blocks, hipStream_t st) {
   const int strips = p.size_n / kStripN;
+  // a single row block is built for the formats that the decode kernel does not have
+  if (row_blocks < 2 && (format == kMidInt4 || format == kMidInt4Zp || format == kMidMxFp4)) row_blocks = 2;
   p.tiles_m = (p.size_m + 16 * row_blocks - 1) / (16 * row_blocks);
-  p.tiles = p.tiles_m * ((strips + kMidStrips - 1) / kMidStrips);
+  p.tiles = p.tiles_m * ((strips + mid_strips(row_blocks) - 1) / mid_strips(row_blocks));
   const int steps = p.size_k / kMidStepK;
   p.split_steps = (steps + p.splits - 1) / p.splits;
   p.splits = (steps + p.split_steps - 1) / p.split_steps;

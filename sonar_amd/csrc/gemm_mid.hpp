@@ -67,7 +67,23 @@ inline double mid_estimate(int64_t size_m, int64_t size_n, int64_t size_k, int64
   return best;
 }
 
-// `row_blocks`: 16-row blocks of a tile, 2 to 6.
+// Up to 16 rows of 8-bit codes or NVFP4, which the decode kernel does not have: into how many parts K is split, in
+// tiles of one row block and one strip.  Never more workgroups than compute units (two on one share its vector unit:
+// K = 4096, N = 11008, fp8, 172 strips: 17.3 us, 19.3 with K in two), and as many parts as pay for the pass that adds them:
+// 1.2 us for 64 rows in each of a workgroup's eight ranges, 3 us for the pass (N = 4096, 64 strips, K = 1 / 2 / 4 parts:
+// 14.8 / 12.3 / 10.6 us; K = 1024, N = 1024: 6.4 / 6.8 / 6.9).
+inline int mid_splits_16_rows(int64_t size_n, int64_t size_k, int cus) {
+  const int64_t strips = size_n / 64, steps = size_k / 64;
+  double best = 1e30;
+  int splits = 1;
+  for (int n = 1; n <= kMidMostSplits && (n == 1 || (strips * n <= cus && steps >= 8 * n)); ++n) {
+    const double us = 1.2 * (((steps + n - 1) / n + 7) / 8) + (n > 1 ? 3.0 + 0.1 * n : 0.0);
+    if (us < best) best = us, splits = n;
+  }
+  return splits;
+}
+
+// `row_blocks`: 16-row blocks of a tile, 1 to 6.
 int mid_gemm(MidParams p, int dtype, int format, int row_blocks, hipStream_t st);
 
 }  // namespace sonar

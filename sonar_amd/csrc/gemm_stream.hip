@@ -1899,15 +1899,24 @@ int marlin_gemm_any(const void* a, int64_t a_row_stride, void* c, const uint32_t
   // eight launches).
   const bool row_slabs = !use_tile && !slab_fast && size_m > 64 && strip_per_workgroup &&
                          total_units * n_strips < (1LL << 31);
-  // 17 rows and more: the kernel of gemm_mid.hip where it is estimated to be faster than what would run otherwise
+  // 17 rows and more: the kernel of gemm_mid.hip where it is estimated to be faster than what would run otherwise;
+  // up to 16 rows of 8-bit codes and NVFP4 always (on 16 shapes from 1024 x 1024 to 14336 x 28672 1.05 to 2 times as
+  // fast as marlin_stream8_kernel and marlin_stream_kernel).
   static const char* mid_env = getenv("SONAR_MARLIN_MID_ROWS");   // debugging aid: its tiles of that many row blocks, always
   static const bool no_mid = mid_switched_off();
-  if ((size_m > 16 || mid_env) && !no_mid && !chk.has_perm && !chk.row_groups && ((uintptr_t)b_scales) % 16 == 0 &&
+  const bool one_block = size_m <= 16 && (chk.bits == 8 || chk.nvfp4);
+  if ((size_m > 16 || one_block || mid_env) && !no_mid && !chk.has_perm && !chk.row_groups && ((uintptr_t)b_scales) % 16 == 0 &&
       mid_applies(size_m, size_k, a_row_stride, num_groups, chk.group_size)) {
     const int format = chk.nvfp4 ? kMidNvFp4 : chk.fp4 ? kMidMxFp4 : chk.bits == 8 ? (chk.fp8 ? kMidFp8 : kMidInt8)
                        : chk.has_zp ? kMidInt4Zp : kMidInt4;
     int row_blocks, splits;
-    const double mid_us = mid_estimate(size_m, size_n, size_k, num_groups, dtype, format, cus, base_scratch, row_blocks, splits);
+    double mid_us = mid_estimate(size_m, size_n, size_k, num_groups, dtype, format, cus, base_scratch, row_blocks, splits);
+    if (one_block) {
+      mid_us = 0.0;
+      row_blocks = 1;
+      splits = mid_splits_16_rows(size_n, size_k, cus);
+      if ((size_t)splits * size_m * size_n * 4 > base_scratch) splits = 1;
+    }
     const double x = (double)size_n * size_k / (6144.0 * 4096.0), r = size_m / 64.0;
     // (what the other kernels take, us: fits of measured times, see mid_estimate)
     double us;
@@ -1929,7 +1938,7 @@ int marlin_gemm_any(const void* a, int64_t a_row_stride, void* c, const uint32_t
     }
     if (mid_env) {   // "row blocks" or "row blocks,splits"
       const char* comma = strchr(mid_env, ',');
-      row_blocks = std::max(2, std::min(6, atoi(mid_env)));
+      row_blocks = std::max(1, std::min(6, atoi(mid_env)));
       splits = comma ? std::max(1, std::min(kMidMostSplits, atoi(comma + 1))) : 1;
       if ((size_t)splits * size_m * size_n * 4 > base_scratch || splits > size_k / 64) splits = 1;
     }

@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
-@pytest.mark.parametrize("row_blocks", ["2", "3", "4", "5", "6", "2,3", "4,5"])
+@pytest.mark.parametrize("row_blocks", ["1", "2", "3", "4", "5", "6", "1,6", "2,3", "4,5"])
 def test_tiles_of_every_height_meet_the_oracle(row_blocks):
     env = dict(os.environ, SONAR_MARLIN_MID_ROWS=row_blocks)
     out = subprocess.run([sys.executable, "-u", "-m", "tests.mid_rows_child"], cwd=ROOT, env=env,
