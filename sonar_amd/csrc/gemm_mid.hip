@@ -22,8 +22,9 @@
 //   M   76, K 9088, N 1920, MXFP4: 32.4 -> 14.5                  M   84, K 9088, N 2560, 8-bit codes: 32.5 -> 16.1
 // Up to 16 rows of the formats that the decode kernel does not have take one row block and one strip a workgroup: eight
 // ranges of K, so that 64 columns are enough to keep a compute unit busy (two strips: 4096 x 11008 18.6 us, one: 17.3).
-//   M    8, K 4096, N 11008, fp8, bf16: 19.9 -> 17.3     M    8, K 2048, N 1536, 8-bit codes: 12.3 -> 7.4
-//   M    8, K 8192, N  8192, fp8, bf16: 30.5 -> 22.4     M    8, K 4096, N 28672, NVFP4: 33.3 -> 23.4
+//   M    8, K 4096, N 11008, fp8, bf16: 19.9 -> 14.8     M    8, K 2048, N 1536, 8-bit codes: 12.3 -> 7.2
+//   M    8, K 8192, N  8192, fp8, bf16: 30.5 -> 21.0     M    8, K 4096, N 28672, NVFP4: 33.3 -> 23.4
+// Tried without gain there: every workgroup starting its rows of K at another place (no channel conflicts to avoid).
 // Tried and slower: one strip a workgroup with eight ranges (half the dequantisation per workgroup, but twice the
 // activation bytes through the copy path per matrix instruction: 200 rows above 23 us, 64 rows on N = 28672 31 us).
 //
@@ -53,14 +54,17 @@ constexpr int mid_ranges(int mb) { return kMidWaves / mid_strips(mb); }      // 
 constexpr int kMidStepK = 64;     // rows of K a step takes from each range
 
 // Activation stages in LDS.
-constexpr int mid_stages(int mb) { return mb > 1 && mb <= 4 ? 4 : 3; }
-// Wavefronts a SIMD: two (one workgroup a compute unit), or four for a single row block, whose loop is so short that two
-// workgroups are needed to keep enough bytes under way.
-constexpr int mid_waves_per_simd(int mb) { return mb == 1 ? 4 : 2; }
+constexpr int mid_stages(int mb, bool deep) { return deep ? 5 : mb > 1 && mb <= 4 ? 4 : 3; }
+// Wavefronts a SIMD: two (one workgroup a compute unit), or four for a single row block with more workgroups than
+// compute units, `deep` without: its loop is so short that the bytes under way have to come from two workgroups or
+// a longer ring.  That ring pays from six steps a range on: K = 4096, N = 11008, fp8 (8 steps) 16.3 -> 14.8 us, K = 3072,
+// N = 16384 (6) 16.3 -> 15.6, but K = 2048, N = 8192 (4) 9.6 -> 10.2, K = 1024, N = 1024 (2) 5.1 -> 6.1.
+constexpr int kMidDeepSteps = 6;
+constexpr int mid_waves_per_simd(int mb, bool deep) { return mb == 1 && !deep ? 4 : 2; }
 constexpr int mid_stage_bytes(int mb) { return mid_ranges(mb) * mb * 2048; }
 constexpr int mid_sum_rows(int mb) { return mb < 4 ? mb : 4; }   // row blocks summed at a time at the end
-constexpr int mid_lds(int mb) {
-  const int stages = mid_stages(mb) * mid_stage_bytes(mb), sum = kMidWaves * mid_sum_rows(mb) * 4096;
+constexpr int mid_lds(int mb, bool deep) {
+  const int stages = mid_stages(mb, deep) * mid_stage_bytes(mb), sum = kMidWaves * mid_sum_rows(mb) * 4096;
   return stages > sum ? stages : sum;
 }
 
@@ -77,8 +81,8 @@ struct MidDequant {
   typedef typename std::conditional<k8, typename D8::Col, typename D4::Col>::type Col;
 };
 
-template <typename T, int FMT, int GROUPS, int MB>
-__global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(mid_waves_per_simd(MB), mid_waves_per_simd(MB)))) void marlin_mid_gemm(
+template <typename T, int FMT, int GROUPS, int MB, bool DEEP>
+__global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(mid_waves_per_simd(MB, DEEP), mid_waves_per_simd(MB, DEEP)))) void marlin_mid_gemm(
     const MidParams p) {
   typedef MidDequant<T, FMT> Fmt;
   typedef typename Fmt::D4 D4;
@@ -86,7 +90,13 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
   typedef typename Fmt::Col Col;
   typedef typename Dq<T>::vec8 vec8;
   constexpr bool kZero = FMT == kMidInt4Zp;
-  constexpr int D = mid_stages(MB);
+  // 8-bit codes go to the matrix cores as they are, which halves their instructions, and their scales into the fp32
+  // sums: at the end with one group; else group by group (`raw` to `acc`), which pays for a single row block only
+  // and has the operands of the matrix instruction the other way round, so that a lane's sums share a column.
+  // (K = 4096, N = 4096, 8 rows, fp8, one group / MXFP8: 10.6 -> 10.2 / 11.0 -> 10.6 us; K = 12288, N = 2560: 14.4 -> 14.0.)
+  constexpr bool kRaw = Fmt::k8 && std::is_same<T, __bf16>::value && (GROUPS == kOneGroup || MB == 1);
+  constexpr bool kFold = kRaw && GROUPS != kOneGroup;
+  constexpr int D = mid_stages(MB, DEEP);
   constexpr int W = D - 1;                           // ring of the packed codes and scales in registers
   constexpr int kStage = mid_stage_bytes(MB);
   constexpr int kMidStrips = mid_strips(MB), kMidRanges = mid_ranges(MB);
@@ -181,6 +191,7 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
   };
 
   Col cols[4];
+  float fold_scale[2][4];   // kFold: of the chunk or step that is multiplied and the one after it
   auto set_col = [&](int j, uint16_t scale_bits, uint32_t zero_word) __attribute__((always_inline)) {
     int z = 8;
     if (kZero) z = (int)((zero_word >> (4 * (j + 4 * (col16 >> 3)))) & 0xFu);   // zero_point_shift(16 j + col16)
@@ -194,10 +205,11 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
       const uint32_t word = j == 0 ? v.x : j == 1 ? v.y : j == 2 ? v.z : v.w;
       // column 16 j + col16 is slot 2 j + col16 / 8 of the lane's eight
       const uint32_t bits = (col16 & 8) ? word >> 16 : word & 0xFFFFu;
-      set_col(j, (uint16_t)bits, kZero ? zv[R][GROUPS == kChunkGroups ? h : 0] : 0);
+      if constexpr (kFold) fold_scale[GROUPS == kChunkGroups ? h : R % 2][j] = Raw8<FMT == kMidFp8>::column_scale((uint16_t)bits);
+      else set_col(j, (uint16_t)bits, kZero ? zv[R][GROUPS == kChunkGroups ? h : 0] : 0);
     }
   };
-  if constexpr (GROUPS == kOneGroup) {
+  if constexpr (GROUPS == kOneGroup && !kRaw) {
     const uint16_t* srow = p.scales + (size_t)strip * kStripN;
     uint32_t zword = 0;
     if (kZero) zword = p.zeros[(size_t)strip * (kStripN / 8) + (col16 & 7)];
@@ -212,6 +224,7 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
   for (int j = 0; j < 4; ++j)
 #pragma unroll
     for (int i = 0; i < MB; ++i) acc[j][i] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+  floatx4_t raw[4];
 
   // Piece `q` (0..15) of dequantising chunk h of ring position R into wv[h].  A pair of 4-bit integer codes is
   // finished by the piece after it (q = 16 finishes the last).
@@ -227,7 +240,9 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
       if (part & 1) return;
       const u32x4_t& v = wq[R][2 * h + (part >> 1)];   // the low, then the high four of a lane's eight rows
       const uint32_t word = j == 0 ? v.x : j == 1 ? v.y : j == 2 ? v.z : v.w;
-      const uint2 w = D8::word4(word, cols[j], magic);
+      uint2 w;
+      if constexpr (kRaw) w = Raw8<FMT == kMidFp8>::word4(word);
+      else w = D8::word4(word, cols[j], magic);
       wv[h][j][part] = w.x;
       wv[h][j][part + 1] = w.y;
     } else {
@@ -252,6 +267,11 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
   // One half of a step: 4 MB matrix instructions on chunk H of the step in ring position R, LDS slot `slot`.
   // Behind each, a share of the next half's dequantisation and (H = 1) of the memory operations of step `k_copy`;
   // behind a row block's four, the read of its operand of the next half.
+  auto fold = [&](const int R, const int H, const int j) __attribute__((always_inline)) {
+    const float s = fold_scale[GROUPS == kChunkGroups ? H : R % 2][j];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) acc[j][0][r] = __builtin_fmaf(raw[j][r], s, acc[j][0][r]);
+  };
   auto half_step = [&](const int R, const int H, const int slot, const int next_slot, const int fill,
                        const int k_copy) __attribute__((always_inline)) {
     const int NR = H ? (R + 1) % W : R, NH = H ^ 1;
@@ -263,8 +283,13 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const vec8 w = __builtin_bit_cast(vec8, u32x4_t{wv[H][j][0], wv[H][j][1], wv[H][j][2], wv[H][j][3]});
-        acc[j][i] = Dq<T>::mfma(w, __builtin_bit_cast(vec8, av[i]), acc[j][i]);
+        if constexpr (kFold)
+          raw[j] = Dq<T>::mfma(__builtin_bit_cast(vec8, av[i]), w,
+                               GROUPS == kChunkGroups || H == 0 ? floatx4_t{0.f, 0.f, 0.f, 0.f} : raw[j]);
+        else
+          acc[j][i] = Dq<T>::mfma(w, __builtin_bit_cast(vec8, av[i]), acc[j][i]);
         const int at = 4 * i + j;
+        if (kFold && j > 0 && (GROUPS == kChunkGroups || H == 1)) fold(R, H, j - 1);   // (one matrix instruction later)
 #pragma unroll
         for (int q = 0; q < 16; ++q)
           if (q >= 16 * at / (4 * MB) && q < 16 * (at + 1) / (4 * MB)) piece(NR, NH, q);
@@ -279,6 +304,7 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
       __builtin_amdgcn_sched_barrier(0);
     }
     piece(NR, NH, 16);
+    if (kFold && (GROUPS == kChunkGroups || H == 1)) fold(R, H, 3);
   };
 
   // ---- prologue: D - 1 steps asked for, the first one here
@@ -317,6 +343,8 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
     if (t + 1 < per_range) step(1, t + 1);
     if constexpr (W > 2)
       if (t + 2 < per_range) step(2, t + 2);
+    if constexpr (W > 3)
+      if (t + 3 < per_range) step(3, t + 3);
   }
   // copies and reads still under way must not outlive this point: LDS is used for the sums from here on
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
@@ -351,7 +379,13 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
       for (int j = 0; j < 4; ++j)
         if (round + i < MB) {
           const floatx4_t v = acc[j][round + i < MB ? round + i : 0];
-          sums[((wave * kSum + i) * 4 + j) * 64 + lane] = make_float4(v.x, v.y, v.z, v.w);
+          const int at = ((wave * kSum + i) * 4 + j) * 64;
+          if constexpr (kFold) {   // rows 4 kb .. + 3 of column col16: stored as the others, four columns of a row together
+#pragma unroll
+            for (int r = 0; r < 4; ++r) reinterpret_cast<float*>(sums)[4 * at + 16 * (4 * kb + r) + col16] = v[r];
+          } else {
+            sums[at + lane] = make_float4(v.x, v.y, v.z, v.w);
+          }
         }
     __syncthreads();
 #pragma unroll
@@ -365,11 +399,16 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
       floatx4_t v = floatx4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int g = 0; g < kMidRanges; ++g) {
-        const float4 s = sums[(((kMidStrips * g + strip_of) * kSum + (q >> 2)) * 4 + j) * 64 + lane];
+        const float4 s = sums[(((kMidStrips * g + strip_of) * kSum + (q >> 2)) * 4 + j) * 64 + (kFold ? 4 * col16 + kb : lane)];
         v += floatx4_t{s.x, s.y, s.z, s.w};
       }
       if (row >= p.size_m) continue;
       const int nl = 16 * j + 4 * kb;
+      if constexpr (kRaw && !kFold) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          v[r] *= Raw8<FMT == kMidFp8>::column_scale(p.scales[strip * kStripN + scale_slot(nl + r, false)]);
+      }
       if (p.splits > 1) {
         p.partial[(((size_t)split * p.size_m + row) * p.size_n + strip * kStripN + nl) / 4] = make_float4(v.x, v.y, v.z, v.w);
         continue;
@@ -415,15 +454,15 @@ __global__ __launch_bounds__(256) void marlin_mid_sum(const MidParams p) {
   }
 }
 
-template <typename T, int FMT, int GROUPS, int MB>
+template <typename T, int FMT, int GROUPS, int MB, bool DEEP = false>
 int launch_mid_rows(const MidParams& p, hipStream_t st) {
   static bool attr_set = false;   // raising the dynamic LDS limit is needed once per form
   if (!attr_set) {
-    SONAR_HIP(hipFuncSetAttribute((const void*)marlin_mid_gemm<T, FMT, GROUPS, MB>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, mid_lds(MB)));
+    SONAR_HIP(hipFuncSetAttribute((const void*)marlin_mid_gemm<T, FMT, GROUPS, MB, DEEP>,
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, mid_lds(MB, DEEP)));
     attr_set = true;
   }
-  marlin_mid_gemm<T, FMT, GROUPS, MB><<<(p.tiles * p.splits + 7) / 8 * 8, kMidWaves * 64, mid_lds(MB), st>>>(p);
+  marlin_mid_gemm<T, FMT, GROUPS, MB, DEEP><<<(p.tiles * p.splits + 7) / 8 * 8, kMidWaves * 64, mid_lds(MB, DEEP), st>>>(p);
   return launch_status("marlin_mid_gemm");
 }
 
@@ -431,7 +470,10 @@ template <typename T, int FMT, int GROUPS>
 int launch_mid(const MidParams& p, int row_blocks, hipStream_t st) {
   switch (row_blocks) {
     case 1:
-      if constexpr (FMT == kMidInt8 || FMT == kMidFp8 || FMT == kMidNvFp4) return launch_mid_rows<T, FMT, GROUPS, 1>(p, st);
+      if constexpr (FMT == kMidInt8 || FMT == kMidFp8 || FMT == kMidNvFp4) {
+        if (p.tiles * p.splits <= p.cus && p.split_steps >= kMidDeepSteps * mid_ranges(1)) return launch_mid_rows<T, FMT, GROUPS, 1, true>(p, st);
+        return launch_mid_rows<T, FMT, GROUPS, 1>(p, st);
+      }
     case 2: return launch_mid_rows<T, FMT, GROUPS, 2>(p, st);
     case 3: return launch_mid_rows<T, FMT, GROUPS, 3>(p, st);
     case 4: return launch_mid_rows<T, FMT, GROUPS, 4>(p, st);

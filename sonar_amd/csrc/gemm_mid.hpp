@@ -23,6 +23,7 @@ struct MidParams {
   int size_m, size_n, size_k, num_groups;
   int group_shift;           // log2 of the 64-row steps per group; -1: groups of 32 or 16 rows
   int chunks_per_strip;
+  int cus;                   // compute units
   int splits;                // of K over workgroups; their totals go to `partial` and a second kernel adds them
   float4* partial;           // [splits][M][N / 4]
   int tiles_m, tiles, split_steps;   // filled in by mid_gemm
@@ -69,9 +70,9 @@ inline double mid_estimate(int64_t size_m, int64_t size_n, int64_t size_k, int64
 
 // Up to 16 rows of 8-bit codes or NVFP4, which the decode kernel does not have: into how many parts K is split, in
 // tiles of one row block and one strip.  Never more workgroups than compute units (two on one share its vector unit:
-// K = 4096, N = 11008, fp8, 172 strips: 17.3 us, 19.3 with K in two), and as many parts as pay for the pass that adds them:
-// 1.2 us for 64 rows in each of a workgroup's eight ranges, 3 us for the pass (N = 4096, 64 strips, K = 1 / 2 / 4 parts:
-// 14.8 / 12.3 / 10.6 us; K = 1024, N = 1024: 6.4 / 6.8 / 6.9).
+// K = 4096, N = 11008, fp8, 172 strips: 14.8 us, 17.4 with K in two), and as many parts as pay for the pass that adds them:
+// about 1.2 us for 64 rows in each of a workgroup's eight ranges, 3 us for the pass (N = 4096, 64 strips, K = 1 / 2 / 4 parts:
+// 13.2 / 11.4 / 10.0 us; K = 1024, N = 1024: 5.1 / 6.4 / 6.5).
 inline int mid_splits_16_rows(int64_t size_n, int64_t size_k, int cus) {
   const int64_t strips = size_n / 64, steps = size_k / 64;
   double best = 1e30;

@@ -1958,6 +1958,7 @@ int marlin_gemm_any(const void* a, int64_t a_row_stride, void* c, const uint32_t
       q.num_groups = (int)num_groups;
       q.group_shift = chk.group_size < 64 ? -1 : 31 - __builtin_clz(chk.group_size / 64);
       q.chunks_per_strip = p.chunks_per_strip;
+      q.cus = cus;
       q.splits = splits;
       q.partial = static_cast<float4*>(scratch);
       return mid_gemm(q, dtype, format, row_blocks, st);

@@ -27,8 +27,9 @@ def int4(m, k, n, g, dtype, zp, bias) -> None:
 
 def main() -> None:
     rows = 16 * int(os.environ["SONAR_MARLIN_MID_ROWS"].split(",")[0])
-    # one step of K for four ranges; an odd last strip; a last tile of one row; ranges of unequal length; many tiles
-    shapes = [(1, 64, 64), (rows, 320, 192), (rows + 1, 1344, 448), (2 * rows - 1, 512, 1088), (5 * rows + 3, 1024, 128)]
+    # one step of K for four ranges; an odd last strip; a last tile of one row; ranges of unequal length; many tiles;
+    # ranges of 6 and 7 steps (the longer ring of a single row block)
+    shapes = [(1, 64, 64), (rows, 320, 192), (rows + 1, 1344, 448), (2 * rows - 1, 512, 1088), (5 * rows + 3, 1024, 128), (rows - 3, 3136, 192)]
     for i, (m, k, n) in enumerate(shapes):
         for dtype in ("fp16", "bf16"):
             for g in (-1, 32, 64) + ((256,) if k % 256 == 0 and k > 256 else ()):
