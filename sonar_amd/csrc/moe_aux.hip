@@ -30,7 +30,7 @@ __device__ __forceinline__ int wave_inclusive_sum(int v) {
 // one ballot per bit of the expert number, so the slots of an expert keep ascending order.  Without it
 // (more experts than the histograms have room for) offsets[e] is left for the placement kernel.
 // Latency bound: 8000 slots on 32 experts 9 + 42 us as two launches whose second walked all slots once
-// per expert, 7 us like this.
+// per expert, 7 us like this (14 us in a kernel trace of the whole layer, at the clock it runs at there).
 __global__ __launch_bounds__(kAlignThreads) void moe_align_count_kernel(
     const int32_t* __restrict__ topk_ids, int numel, int num_experts, int block_size,
     int32_t* __restrict__ sorted_ids, int sorted_len, int32_t* __restrict__ expert_ids, int expert_len,
