@@ -173,6 +173,30 @@ struct Dq<__bf16> {
   }
 };
 
+// The operand of kernels that feed the matrix cores integers and apply offset and scale to their fp32 sums: B + v, the
+// nibble OR-ed into the mantissa of B (7 instructions for a packed word).
+template <typename T>
+struct RawOperand;
+template <>
+struct RawOperand<_Float16> {
+  static constexpr uint32_t kMagic = 0x64006400u;  // 1024.0 twice
+  static constexpr uint32_t kOnes = 0x3c003c00u;
+  static constexpr float kBase = 1024.f;
+};
+template <>
+struct RawOperand<__bf16> {
+  static constexpr uint32_t kMagic = 0x43004300u;  // 128.0 twice
+  static constexpr uint32_t kOnes = 0x3f803f80u;
+  static constexpr float kBase = 128.f;
+};
+__device__ __forceinline__ u32x4_t raw_operand(uint32_t q, uint32_t magic) {
+  const uint32_t e0 = and_or(q, 0x000f000fu, magic);
+  const uint32_t e1 = and_or(q >> 4, 0x000f000fu, magic);
+  const uint32_t e2 = and_or(q >> 8, 0x000f000fu, magic);
+  const uint32_t e3 = and_or(q >> 12, 0x000f000fu, magic);
+  return u32x4_t{e0, e1, e2, e3};
+}
+
 // Per-lane constants of the four columns (j = 0..3) a lane dequantises, for
 // the group `g` of strip `strip`.
 template <typename T, bool HAS_ZP, typename D = Dq<T>>

@@ -13,8 +13,16 @@
 // logic, shifts and multiplies half of that).  A chunk (32 rows of a strip) costs 52 (fp16) to 68 (bf16) instructions
 // to dequantise and a few for its scales, beside 4 MB matrix instructions.  K = 4096, N = 8192, 64 rows, bf16:
 // 18.0 + 1.45 (MB - 2) us, of which about 6 are launch, first bytes and the sum over the ranges at the end.
+// Calls on 4-bit integers that would else run in the decode kernel's blocks of rows (one group or groups of 128 * 2^i
+// rows) feed the matrix cores the integers as that kernel does (kOneGroupRaw, kUnitGroupsRaw): 36 and 28
+// instructions a chunk, and per unit of 128 rows 16 (fp16) or 36 (bf16) a row block for the fold.  The error against
+// 64 bits is the output's own rounding (1.00 times it in fp16 and bf16; rounding each scaled weight: 1.28 times), and
+//   M   64, K 4096, N 28672, bf16: 22.6 -> 21.7      M  200, K 4096, N 6144, fp16, zero points: 20.4 -> 17.6
+//   M   80, K 4096, N 11008, bf16: 23.8 -> 18.4      M   17, K 2048, N 20032, bf16: 11.4 -> 10.0
+// against scaled weights or the decode kernel; but two sets of sums end at four row blocks, so that 65 to 96 rows lose
+// the single round of tiles they had on matrices of 129 to 256 pairs of strips (M 96, K 4096, N 28672: 30.3 -> 36; 45 in the decode kernel).
 // Measured against the kernels it takes over from (us, before -> now):
-//   M   64, K 4096, N 28672, bf16: 29.1 -> 23.0      M  200, K 4096, N 6144, fp16, zero points: 24.6 -> 21.0
+//   M   64, K 4096, N 28672, bf16: 29.1 -> 21.7      M  200, K 4096, N 6144, fp16, zero points: 24.6 -> 17.6
 //   M  333, K 2880, N  5760, bf16, groups of 32: 40.5 -> 21.7      M  512, K 4096, N 2048, bf16: 36 -> 20
 //   M  128, K 2048, N 20032, MXFP4: 47.6 -> 20.5     M   96, K 2048, N 20032, 8-bit codes: 48 -> 18.5
 // and with K split over workgroups, where there are fewer tiles than compute units:
@@ -69,8 +77,10 @@ constexpr int mid_lds(int mb, bool deep) {
 }
 
 // How the scales come: one group, groups of 64 * 2^i rows (a scale row a step), or groups of 32 rows or less (a
-// scale row a chunk; NVFP4: two groups a chunk).
-enum MidGroups { kOneGroup = 0, kStepGroups = 1, kChunkGroups = 2 };
+// scale row a chunk; NVFP4: two groups a chunk).  The last two are forms for 4-bit integers (MidParams::raw_codes): the
+// codes go to the matrix cores as integers, and the scale of one group or of groups of 128 * 2^i rows (a scale row a
+// unit of two steps) into the fp32 sums.
+enum MidGroups { kOneGroup = 0, kStepGroups = 1, kChunkGroups = 2, kOneGroupRaw = 3, kUnitGroupsRaw = 4 };
 
 template <typename T, int FMT>
 struct MidDequant {
@@ -96,6 +106,16 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
   // (K = 4096, N = 4096, 8 rows, fp8, one group / MXFP8: 10.6 -> 10.2 / 11.0 -> 10.6 us; K = 12288, N = 2560: 14.4 -> 14.0.)
   constexpr bool kRaw = Fmt::k8 && std::is_same<T, __bf16>::value && (GROUPS == kOneGroup || MB == 1);
   constexpr bool kFold = kRaw && GROUPS != kOneGroup;
+  // 4-bit integers that way: v - z in fp16 (nine instructions a word instead of 13), in bf16 128 + v (7 instead of 17), whose
+  // surplus (128 + z) * sum(a) comes off with the sum of the activations, one more matrix instruction with an operand of
+  // ones per row block and chunk.  The sums of a unit of 128 rows (`unit_sum`) are folded into `acc` behind the matrix instructions
+  // of the row block after them; with one group and fp16 nothing is folded and the scale waits for the end.  Both sets of
+  // sums are 16 registers a row block: with four the largest form has 256.
+  constexpr bool kBf16 = std::is_same<T, __bf16>::value;
+  constexpr bool kCodes = GROUPS == kOneGroupRaw || GROUPS == kUnitGroupsRaw;
+  constexpr bool kUnits = GROUPS == kUnitGroupsRaw || (GROUPS == kOneGroupRaw && kBf16);
+  constexpr bool kSwap = kFold || kCodes;            // activations are the row operand: a lane's sums share a column
+  constexpr bool kNoScales = GROUPS == kOneGroup || kCodes;   // none among the memory operations of every step
   constexpr int D = mid_stages(MB, DEEP);
   constexpr int W = D - 1;                           // ring of the packed codes and scales in registers
   constexpr int kStage = mid_stage_bytes(MB);
@@ -104,14 +124,14 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
   constexpr int kLoads = Fmt::k8 ? 4 : 2;            // 16-byte loads of packed codes per lane and step
   constexpr int kScaleRows = GROUPS == kChunkGroups ? 2 : 1;
   // memory operations per wavefront and step
-  constexpr int kOps = kCopies + kLoads + (GROUPS == kOneGroup ? 0 : kScaleRows * (kZero ? 2 : 1));
+  constexpr int kOps = kCopies + kLoads + (kNoScales ? 0 : kScaleRows * (kZero ? 2 : 1));
   extern __shared__ __attribute__((aligned(1024))) char smem[];
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col16 = lane & 15, kb = lane >> 4;
   const int range = wave / kMidStrips, strip_of = wave % kMidStrips;
-  const uint32_t magic = magic_register();
+  const uint32_t magic = magic_register(kCodes ? RawOperand<T>::kMagic : 0x64006400u);
 
   // Workgroup ids congruent mod 8 run on one XCD: each XCD takes a contiguous run of tiles, the row tiles
   // of a pair of strips next to each other, so the second to ask for a chunk finds it in that L2.
@@ -128,7 +148,8 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
 
   const int first = split * p.split_steps;   // of the steps this workgroup takes
   const int steps = min(first + p.split_steps, p.size_k / kMidStepK);
-  const int per_range = (steps - first + kMidRanges - 1) / kMidRanges;
+  int per_range = (steps - first + kMidRanges - 1) / kMidRanges;
+  if constexpr (kUnits) per_range = (per_range + 1) & ~1;   // whole units: the host has seen to it that `first` and `steps` are even
   const int k_first = first + range * per_range;
 
   // ---- sources.  The activations of a range are copied by its own wavefronts, kCopies copies each of 8 rows x
@@ -152,6 +173,8 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
   u32x4_t wq[W][kLoads];
   u32x4_t sv[W][kScaleRows];
   uint32_t zv[W][kScaleRows];
+  u32x4_t unit_sv;    // kUnitGroupsRaw: scales and zero points of a unit, asked for two steps before they are used
+  uint32_t unit_zv;
 
   // Memory operation `op` (0..kOps-1) of step k: first the codes and scales into ring position R, then the
   // activations into LDS slot `slot`.
@@ -176,12 +199,27 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
                                        (lds_void_t*)(a_stage + slot * kStage + (strip_of * kCopies + i) * 1024), 16, 0, 0);
     }
   };
+  // Scales of the unit of step `k`, behind whose first half they are taken from the registers, and zero points, which fp16
+  // needs for the unit after it.  Older than the other operations of their step.
+  auto issue_unit = [&](const int k) __attribute__((always_inline)) {
+    const int g = min(k, steps - 1) >> p.group_shift, gz = kBf16 ? g : min(k + 1, steps - 1) >> p.group_shift;
+    const char* s_src = s_base + (size_t)g * p.size_n * 2;
+    asm volatile("global_load_dwordx4 %0, %1, %2" : "=&v"(unit_sv) : "v"(s_off), "s"(s_src) : "memory");
+    if constexpr (kZero) {
+      const char* z_src = z_base + (size_t)gz * (p.size_n / 2);
+      asm volatile("global_load_dword %0, %1, %2" : "=&v"(unit_zv) : "v"(z_off), "s"(z_src) : "memory");
+    }
+  };
+  auto unit_landed = [&]() __attribute__((always_inline)) {
+    asm volatile("" : "+v"(unit_sv));
+    if constexpr (kZero) asm volatile("" : "+v"(unit_zv));
+  };
   // until only the `n` youngest operations are outstanding; the registers of ring position R are in its hands
   auto landed = [&](const int R, const int n) __attribute__((always_inline)) {
     asm volatile("s_waitcnt vmcnt(%0)" ::"i"(n) : "memory");
 #pragma unroll
     for (int i = 0; i < kLoads; ++i) asm volatile("" : "+v"(wq[R][i]));
-    if constexpr (GROUPS != kOneGroup) {
+    if constexpr (!kNoScales) {
 #pragma unroll
       for (int h = 0; h < kScaleRows; ++h) {
         asm volatile("" : "+v"(sv[R][h]));
@@ -198,9 +236,21 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
     if constexpr (Fmt::k8) cols[j] = D8::make_col(scale_bits);
     else cols[j] = D4::make_col(scale_bits, z);
   };
+  float unit_scale[4], unit_zero[4];   // kCodes: of the unit whose sums are folded next; bf16: z + 128 below zero
+  uint32_t next_zeros = 0;             // kUnitGroupsRaw in fp16: of the unit after it
+  auto zero_point = [&](int j, uint32_t word) __attribute__((always_inline)) {   // zero_point_shift(16 j + col16)
+    return (int)((word >> (4 * (j + 4 * (col16 >> 3)))) & 0xFu);
+  };
+  auto take_unit = [&](int j) __attribute__((always_inline)) {
+    const uint32_t word = j == 0 ? unit_sv.x : j == 1 ? unit_sv.y : j == 2 ? unit_sv.z : unit_sv.w;
+    unit_scale[j] = Dq<T>::to_float((uint16_t)((col16 & 8) ? word >> 16 : word));   // the slots of make_col
+    if constexpr (kZero && kBf16) unit_zero[j] = -RawOperand<T>::kBase - (float)zero_point(j, unit_zv);
+    if constexpr (kZero && !kBf16)
+      if (j == 3) asm volatile("v_mov_b32 %0, %1" : "=v"(next_zeros) : "v"(unit_zv));   // (a register of its own: unit_zv is loaded again)
+  };
   // the constants of column block j from ring position R (chunk h of the step)
   auto make_col = [&](const int R, const int h, const int j) __attribute__((always_inline)) {
-    if constexpr (GROUPS != kOneGroup) {
+    if constexpr (!kNoScales) {
       const u32x4_t& v = sv[R][GROUPS == kChunkGroups ? h : 0];
       const uint32_t word = j == 0 ? v.x : j == 1 ? v.y : j == 2 ? v.z : v.w;
       // column 16 j + col16 is slot 2 j + col16 / 8 of the lane's eight
@@ -217,6 +267,14 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
     for (int j = 0; j < 4; ++j) set_col(j, srow[scale_slot(16 * j + col16, false)], zword);
   }
 
+  uint16_t one_scale[4];   // kOneGroupRaw: as they were loaded, used when the first step has landed or later
+  uint32_t one_zeros = 0;
+  if constexpr (GROUPS == kOneGroupRaw) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) one_scale[j] = p.scales[(size_t)strip * kStripN + scale_slot(16 * j + col16, false)];
+    if (kZero) one_zeros = p.zeros[(size_t)strip * (kStripN / 8) + (col16 & 7)];
+  }
+
   u32x4_t av[MB];
   uint32_t wv[2][4][4];    // dequantised chunk of either half: four operand blocks of 16 columns
   floatx4_t acc[4][MB];
@@ -225,12 +283,31 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
     for (int i = 0; i < MB; ++i) acc[j][i] = floatx4_t{0.f, 0.f, 0.f, 0.f};
   floatx4_t raw[4];
+  floatx4_t unit_sum[kUnits ? 4 : 1][kUnits ? MB : 1], a_sum[kUnits ? MB : 1];   // of codes times activations, of activations
+  u32x4_t ones = u32x4_t{RawOperand<T>::kOnes, RawOperand<T>::kOnes, RawOperand<T>::kOnes, RawOperand<T>::kOnes};
+  if constexpr (kCodes && kBf16) asm("" : "+v"(ones));
 
   // Piece `q` (0..15) of dequantising chunk h of ring position R into wv[h].  A pair of 4-bit integer codes is
   // finished by the piece after it (q = 16 finishes the last).
   typename Dq<T>::Mid mid;
-  auto piece = [&](const int R, const int h, const int q) __attribute__((always_inline)) {
+  // (`odd`: the chunk's step is the second of its unit)
+  auto piece = [&](const int R, const int h, const bool odd, const int q) __attribute__((always_inline)) {
     const int j = q >> 2, part = q & 3;
+    if constexpr (kCodes) {
+      if (q == 16) return;
+      const u32x4_t& v = wq[R][h];
+      const uint32_t word = j == 0 ? v.x : j == 1 ? v.y : j == 2 ? v.z : v.w;
+      if constexpr (GROUPS == kUnitGroupsRaw)
+        if (part == 0 && odd && h == 1) take_unit(j);
+      if constexpr (kBf16) {
+        wv[h][j][part] = and_or(part ? word >> (4 * part) : word, 0x000f000fu, magic);
+      } else {
+        if constexpr (GROUPS == kUnitGroupsRaw && kZero)
+          if (part == 0 && !odd && h == 0) cols[j] = D4::make_col(0, zero_point(j, next_zeros));
+        wv[h][j][part] = __builtin_bit_cast(uint32_t, D4::stage2(D4::stage1(part < 2 ? word : word >> 8, part, magic), cols[j], part));
+      }
+      return;
+    }
     if constexpr (!Fmt::k8 && !Fmt::kF4) {
       if (q > 0) wv[h][(q - 1) >> 2][(q - 1) & 3] = D4::stage3(mid, cols[(q - 1) >> 2]);
     }
@@ -272,27 +349,60 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
     for (int r = 0; r < 4; ++r) acc[j][0][r] = __builtin_fmaf(raw[j][r], s, acc[j][0][r]);
   };
-  auto half_step = [&](const int R, const int H, const int slot, const int next_slot, const int fill,
-                       const int k_copy) __attribute__((always_inline)) {
+  // the sums of row block i, column block j of a unit
+  float surplus[4];
+  auto fold_unit = [&](const int i, const int j) __attribute__((always_inline)) {
+    if constexpr (kUnits) {
+      if constexpr (kBf16 && !kZero) {
+        if (j == 0) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) surplus[r] = (RawOperand<T>::kBase + 8.f) * a_sum[i][r];
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        float x = unit_sum[j][i][r];
+        if constexpr (kBf16 && kZero) x = __builtin_fmaf(unit_zero[j], a_sum[i][r], x);
+        else if constexpr (kBf16) x -= surplus[r];
+        if constexpr (GROUPS == kUnitGroupsRaw) acc[j][i][r] = __builtin_fmaf(x, unit_scale[j], acc[j][i][r]);
+        else acc[j][i][r] += x;
+      }
+    }
+  };
+  // (`odd`: the second step of a unit)
+  auto half_step = [&](const int R, const int H, const bool odd, const int slot, const int next_slot, const int fill,
+                       const int k_copy, const int k_unit) __attribute__((always_inline)) {
     const int NR = H ? (R + 1) % W : R, NH = H ^ 1;
+    const bool next_odd = odd != (H == 1), begins = !odd && H == 0, ends = odd && H == 1;   // of the unit
     const uint32_t a_next = a_at[NH] + (H ? next_slot : slot) * kStage;
 #pragma unroll
     for (int i = 0; i < MB; ++i) {
       // the operands of this half are the oldest reads, MB are outstanding at every row block
       asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(av[i]) : "i"(MB - 1) : "memory");
+      if constexpr (kUnits && kBf16)
+        a_sum[i] = Dq<T>::mfma(__builtin_bit_cast(vec8, av[i]), __builtin_bit_cast(vec8, ones),
+                               begins ? floatx4_t{0.f, 0.f, 0.f, 0.f} : a_sum[i]);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const vec8 w = __builtin_bit_cast(vec8, u32x4_t{wv[H][j][0], wv[H][j][1], wv[H][j][2], wv[H][j][3]});
-        if constexpr (kFold)
+        if constexpr (kUnits)
+          unit_sum[j][i] = Dq<T>::mfma(__builtin_bit_cast(vec8, av[i]), w,
+                                       begins ? floatx4_t{0.f, 0.f, 0.f, 0.f} : unit_sum[j][i]);
+        else if constexpr (kCodes)
+          acc[j][i] = Dq<T>::mfma(__builtin_bit_cast(vec8, av[i]), w, acc[j][i]);
+        else if constexpr (kFold)
           raw[j] = Dq<T>::mfma(__builtin_bit_cast(vec8, av[i]), w,
                                GROUPS == kChunkGroups || H == 0 ? floatx4_t{0.f, 0.f, 0.f, 0.f} : raw[j]);
         else
           acc[j][i] = Dq<T>::mfma(w, __builtin_bit_cast(vec8, av[i]), acc[j][i]);
         const int at = 4 * i + j;
         if (kFold && j > 0 && (GROUPS == kChunkGroups || H == 1)) fold(R, H, j - 1);   // (one matrix instruction later)
+        if (kUnits && ends && i > 0) fold_unit(i - 1, j);
 #pragma unroll
         for (int q = 0; q < 16; ++q)
-          if (q >= 16 * at / (4 * MB) && q < 16 * (at + 1) / (4 * MB)) piece(NR, NH, q);
+          if (q >= 16 * at / (4 * MB) && q < 16 * (at + 1) / (4 * MB)) piece(NR, NH, next_odd, q);
+        if constexpr (GROUPS == kUnitGroupsRaw)
+          if (ends && at == 0) issue_unit(k_unit);
         if (H) {
 #pragma unroll
           for (int o = 0; o < kOps; ++o)
@@ -303,48 +413,91 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
       SONAR_MID_READ(av[i], a_next, i * 2048);
       __builtin_amdgcn_sched_barrier(0);
     }
-    piece(NR, NH, 16);
+    piece(NR, NH, next_odd, 16);
+    if (kUnits && ends) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) fold_unit(MB - 1, j);
+    }
     if (kFold && (GROUPS == kChunkGroups || H == 1)) fold(R, H, 3);
   };
 
   // ---- prologue: D - 1 steps asked for, the first one here
+  if constexpr (GROUPS == kUnitGroupsRaw) {
+    if constexpr (kZero && !kBf16) {   // (the zero points of the first unit)
+      const char* z_src = z_base + (size_t)(min(k_first, steps - 1) >> p.group_shift) * (p.size_n / 2);
+      asm volatile("global_load_dword %0, %1, %2" : "=&v"(next_zeros) : "v"(z_off), "s"(z_src) : "memory");
+    }
+    issue_unit(k_first + 1);
+  }
 #pragma unroll
   for (int r = 0; r < W; ++r)
 #pragma unroll
     for (int o = 0; o < kOps; ++o) issue_one(r, r, min(k_first + r, steps - 1), o);
   landed(0, (W - 1) * kOps);
+  if constexpr (GROUPS == kUnitGroupsRaw) {
+    unit_landed();
+    asm volatile("" : "+v"(next_zeros));
+  }
+  if constexpr (kCodes && !kBf16 && !(GROUPS == kUnitGroupsRaw && kZero)) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) cols[j] = D4::make_col(0, kZero ? zero_point(j, one_zeros) : 8);
+  }
+  if constexpr (GROUPS == kOneGroupRaw && kBf16 && kZero) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) unit_zero[j] = -RawOperand<T>::kBase - (float)zero_point(j, one_zeros);
+  }
   __builtin_amdgcn_s_barrier();
 #pragma unroll
   for (int i = 0; i < MB; ++i) SONAR_MID_READ(av[i], a_at[0], i * 2048);
 #pragma unroll
-  for (int q = 0; q <= 16; ++q) piece(0, 0, q);
+  for (int q = 0; q <= 16; ++q) piece(0, 0, false, q);
 
   int slot = 0, fill = W;   // LDS slot of step t, and the one step t + D - 1 goes to
-  auto step = [&](const int R, int t) __attribute__((always_inline)) {
+  auto step = [&](const int R, const bool odd, int t) __attribute__((always_inline)) {
     const bool live = k_first + t < steps;   // uniform; past the end of K only the copies are left to do
     const int next_slot = slot == D - 1 ? 0 : slot + 1;
     const int k_copy = min(k_first + t + W, steps - 1);
-    if (live) half_step(R, 0, slot, next_slot, 0, 0);
+    if (live) half_step(R, 0, odd, slot, next_slot, 0, 0, 0);
     landed((R + 1) % W, (W - 2) * kOps);
+    if constexpr (GROUPS == kUnitGroupsRaw)
+      if (!odd) unit_landed();
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
     if (live) {
-      half_step(R, 1, slot, next_slot, fill, k_copy);
+      half_step(R, 1, odd, slot, next_slot, fill, k_copy, k_first + t + 2);
     } else {
+      if constexpr (GROUPS == kUnitGroupsRaw)
+        if (odd) issue_unit(k_first + t + 2);
 #pragma unroll
       for (int o = 0; o < kOps; ++o) issue_one(R, fill, k_copy, o);
     }
     slot = next_slot;
     fill = fill == D - 1 ? 0 : fill + 1;
   };
-  for (int t = 0; t < per_range; t += W) {
-    step(0, t);
-    if (t + 1 < per_range) step(1, t + 1);
-    if constexpr (W > 2)
-      if (t + 2 < per_range) step(2, t + 2);
-    if constexpr (W > 3)
-      if (t + 3 < per_range) step(3, t + 3);
+  if constexpr (kUnits) {   // units of two steps through a ring of three
+    static_assert(W == 3);
+    for (int t = 0; t < per_range; t += 6) {
+      step(0, false, t);
+      step(1, true, t + 1);
+      if (t + 2 < per_range) {
+        step(2, false, t + 2);
+        step(0, true, t + 3);
+      }
+      if (t + 4 < per_range) {
+        step(1, false, t + 4);
+        step(2, true, t + 5);
+      }
+    }
+  } else {
+    for (int t = 0; t < per_range; t += W) {
+      step(0, false, t);
+      if (t + 1 < per_range) step(1, false, t + 1);
+      if constexpr (W > 2)
+        if (t + 2 < per_range) step(2, false, t + 2);
+      if constexpr (W > 3)
+        if (t + 3 < per_range) step(3, false, t + 3);
+    }
   }
   // copies and reads still under way must not outlive this point: LDS is used for the sums from here on
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
@@ -354,7 +507,7 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
   for (int r = 0; r < W; ++r) {
 #pragma unroll
     for (int i = 0; i < kLoads; ++i) asm volatile("" : "+v"(wq[r][i]));
-    if constexpr (GROUPS != kOneGroup) {
+    if constexpr (!kNoScales) {
 #pragma unroll
       for (int h = 0; h < kScaleRows; ++h) {
         asm volatile("" : "+v"(sv[r][h]));
@@ -363,13 +516,25 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
     }
   }
 #undef SONAR_MID_READ
+  if constexpr (GROUPS == kUnitGroupsRaw) unit_landed();
   __builtin_amdgcn_s_barrier();
+  if constexpr (GROUPS == kOneGroupRaw) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[j][i][r] *= Dq<T>::to_float(one_scale[j]);
+  }
 
   // ---- the four ranges meet in LDS, mid_sum_rows(MB) row blocks at a time; a wavefront adds a quarter of
   // its strip's accumulator tiles, in the order of the ranges
   constexpr int kSum = mid_sum_rows(MB);
   float4* sums = reinterpret_cast<float4*>(smem);
   const float gs = FMT == kMidNvFp4 && p.global_scale ? p.global_scale[0] : 1.f;
+  // Row and first of four columns of a tile that a lane adds.  With kSwap a lane holds rows 4 kb .. + 3 of column col16 and
+  // stores them so that four columns of a row lie together; rows change places between the kb, off each other's banks.
+  const int tile_row = kSwap ? 4 * kb + ((col16 >> 2) ^ kb) : col16, tile_col = 4 * (kSwap ? lane & 3 : kb);
 #pragma unroll
   for (int round = 0; round < MB; round += kSum) {
     if (round > 0) __syncthreads();
@@ -380,9 +545,9 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
         if (round + i < MB) {
           const floatx4_t v = acc[j][round + i < MB ? round + i : 0];
           const int at = ((wave * kSum + i) * 4 + j) * 64;
-          if constexpr (kFold) {   // rows 4 kb .. + 3 of column col16: stored as the others, four columns of a row together
+          if constexpr (kSwap) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) reinterpret_cast<float*>(sums)[4 * at + 16 * (4 * kb + r) + col16] = v[r];
+            for (int r = 0; r < 4; ++r) reinterpret_cast<float*>(sums)[4 * at + 64 * kb + 16 * (r ^ kb) + col16] = v[r];
           } else {
             sums[at + lane] = make_float4(v.x, v.y, v.z, v.w);
           }
@@ -394,16 +559,16 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
       if (kEach > 0 ? u >= kEach : range >= 4 * kSum) continue;
       const int q = kEach > 0 ? range * kEach + u : range;
       const int i = round + (q >> 2), j = q & 3;
-      const int row = m0 + 16 * i + col16;
+      const int row = m0 + 16 * i + tile_row;
       if (i >= MB || !active) continue;
       floatx4_t v = floatx4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int g = 0; g < kMidRanges; ++g) {
-        const float4 s = sums[(((kMidStrips * g + strip_of) * kSum + (q >> 2)) * 4 + j) * 64 + (kFold ? 4 * col16 + kb : lane)];
+        const float4 s = sums[(((kMidStrips * g + strip_of) * kSum + (q >> 2)) * 4 + j) * 64 + lane];
         v += floatx4_t{s.x, s.y, s.z, s.w};
       }
       if (row >= p.size_m) continue;
-      const int nl = 16 * j + 4 * kb;
+      const int nl = 16 * j + tile_col;
       if constexpr (kRaw && !kFold) {
 #pragma unroll
         for (int r = 0; r < 4; ++r)
@@ -467,6 +632,15 @@ int launch_mid_rows(const MidParams& p, hipStream_t st) {
 }
 
 template <typename T, int FMT, int GROUPS>
+int launch_mid_raw(const MidParams& p, int row_blocks, hipStream_t st) {
+  switch (row_blocks) {
+    case 2: return launch_mid_rows<T, FMT, GROUPS, 2>(p, st);
+    case 3: return launch_mid_rows<T, FMT, GROUPS, 3>(p, st);
+    default: return launch_mid_rows<T, FMT, GROUPS, kMidMostRawRows>(p, st);
+  }
+}
+
+template <typename T, int FMT, int GROUPS>
 int launch_mid(const MidParams& p, int row_blocks, hipStream_t st) {
   switch (row_blocks) {
     case 1:
@@ -487,6 +661,11 @@ int launch_mid_groups(const MidParams& p, int row_blocks, hipStream_t st) {
   if constexpr (FMT == kMidMxFp4 || FMT == kMidNvFp4) {
     return launch_mid<T, FMT, kChunkGroups>(p, row_blocks, st);
   } else {
+    if constexpr (FMT == kMidInt4 || FMT == kMidInt4Zp) {
+      if (p.raw_codes)
+        return p.num_groups == 1 ? launch_mid_raw<T, FMT, kOneGroupRaw>(p, row_blocks, st)
+                                 : launch_mid_raw<T, FMT, kUnitGroupsRaw>(p, row_blocks, st);
+    }
     if (p.num_groups == 1) return launch_mid<T, FMT, kOneGroup>(p, row_blocks, st);
     if (p.group_shift >= 0) return launch_mid<T, FMT, kStepGroups>(p, row_blocks, st);
     return launch_mid<T, FMT, kChunkGroups>(p, row_blocks, st);
@@ -513,10 +692,12 @@ int mid_gemm(MidParams p, int dtype, int format, int row_blocks, hipStream_t st)
   const int strips = p.size_n / kStripN;
   // a single row block is built for the formats that the decode kernel does not have
   if (row_blocks < 2 && (format == kMidInt4 || format == kMidInt4Zp || format == kMidMxFp4)) row_blocks = 2;
+  if (p.raw_codes) row_blocks = std::min(row_blocks, kMidMostRawRows);
   p.tiles_m = (p.size_m + 16 * row_blocks - 1) / (16 * row_blocks);
   p.tiles = p.tiles_m * ((strips + mid_strips(row_blocks) - 1) / mid_strips(row_blocks));
   const int steps = p.size_k / kMidStepK;
   p.split_steps = (steps + p.splits - 1) / p.splits;
+  if (p.raw_codes) p.split_steps = (p.split_steps + 1) & ~1;   // whole units of 128 rows
   p.splits = (steps + p.split_steps - 1) / p.split_steps;
   const int rc = dtype == SONAR_DTYPE_F16 ? launch_mid_format<_Float16>(p, format, row_blocks, st)
                                           : launch_mid_format<__bf16>(p, format, row_blocks, st);

@@ -10,6 +10,7 @@ namespace sonar {
 enum MidFormat { kMidInt4 = 0, kMidInt4Zp = 1, kMidInt8 = 2, kMidFp8 = 3, kMidMxFp4 = 4, kMidNvFp4 = 5 };
 
 constexpr int kMidMostSplits = 8;
+constexpr int kMidMostRawRows = 4;   // row blocks of a tile with MidParams::raw_codes
 
 struct MidParams {
   const uint16_t* a;
@@ -26,6 +27,9 @@ struct MidParams {
   int cus;                   // compute units
   int splits;                // of K over workgroups; their totals go to `partial` and a second kernel adds them
   float4* partial;           // [splits][M][N / 4]
+  // 4-bit integers with one group or groups of 128 * 2^i rows, K % 128 == 0: feed the matrix cores the integers and apply
+  // scales to fp32 sums, as the decode kernel does, instead of rounding every scaled weight to 16 bits
+  bool raw_codes;
   int tiles_m, tiles, split_steps;   // filled in by mid_gemm
 };
 
@@ -44,24 +48,30 @@ inline bool mid_applies(int64_t size_m, int64_t size_k, int64_t lda, int64_t num
 // block's matrix instructions and a time that depends on the format for the dequantisation, which the matrix
 // instructions do not hide; more at the clock of a full chip than of a half empty one; no less than the weights take
 // from memory.  K is split where the tiles leave compute units idle, if the totals fit `room` bytes; the
-// pass that adds them is 3.3 us and its bytes.
+// pass that adds them is 3.3 us and its bytes.  `raw_codes` (see MidParams) has a fit of its own (K = 2048, 4096 and
+// 8192, N = 2048 to 20032, 17 to 256 rows: 90 % within 7 % below and 11 % above): fewer instructions a chunk for the
+// dequantisation, more a row block for the fold.
 inline double mid_estimate(int64_t size_m, int64_t size_n, int64_t size_k, int64_t num_groups, int dtype, int format,
-                           int cus, size_t room, int& row_blocks, int& splits) {
+                           bool raw_codes, int cus, size_t room, int& row_blocks, int& splits) {
   static const double kDequant[6][2] = {   // float16, bfloat16
       {6.8, 8.8}, {8.3, 10.0}, {6.0, 10.2}, {8.0, 15.5}, {5.3, 5.3}, {9.0, 13.3}};
   const double dequant = kDequant[format][dtype == 0 ? 0 : 1] + (num_groups > 1 && size_k / num_groups == 32 && format != kMidMxFp4 ? 0.8 : 0.0);
+  static const double kRaw[2][2][2] = {   // without and with zero points, float16 and bfloat16: a strip's share, a row block's
+      {{8.2, 1.83}, {6.2, 2.8}}, {{9.55, 1.77}, {6.7, 2.8}}};
+  const double* raw = kRaw[format == kMidInt4Zp][dtype == 0 ? 0 : 1];
   const int64_t steps = size_k / 64;
   const double memory = 4.0 + size_n * size_k * (format == kMidInt8 || format == kMidFp8 ? 1.0 : 0.5) / 4.5e6;
   double best = 1e30;
-  for (int mb = 2; mb <= 6; ++mb) {
+  for (int mb = 2; mb <= (raw_codes ? kMidMostRawRows : 6); ++mb) {
     const int64_t tiles = ((size_m + 16 * mb - 1) / (16 * mb)) * ((size_n + 127) / 128);
     for (int n = 1; n <= kMidMostSplits; ++n) {
       if (n > 1 && (tiles * n > cus || steps < 8 * n || (size_t)n * size_m * size_n * 4 > room)) break;
-      const double k = (((steps + n - 1) / n + 3) / 4) * 256 / 4096.0;
+      const double k = (raw_codes ? 2 * (((steps / 2 + n - 1) / n + 3) / 4) : ((steps + n - 1) / n + 3) / 4) * 256 / 4096.0;
       const int64_t groups = tiles * n, rounds = (groups + cus - 1) / cus;
       double us = 1.5 + rounds * (4.0 + k * (dequant + 1.5 * mb) * (rounds > 2 ? 1.3 : 2 * groups > cus ? 1.1 : 0.85));
+      if (raw_codes) us = 1.4 + rounds * (1.6 + 0.3 * mb + k * (raw[0] + raw[1] * mb) * (2 * groups > cus ? 1.08 : 0.9));
       if (us < memory) us = memory;
-      if (n > 1) us += 3.3 + 2e-6 * n * size_m * size_n;
+      if (n > 1) us += raw_codes ? 2.5 + 1.3e-6 * n * size_m * size_n : 3.3 + 2e-6 * n * size_m * size_n;
       if (us < best) best = us, row_blocks = mb, splits = n;
     }
   }

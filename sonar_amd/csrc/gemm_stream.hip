@@ -747,28 +747,6 @@ __device__ __forceinline__ void copy_activations(const StreamParams& p, const Fa
 // the last sum coming from one more MFMA per chunk with an all-ones operand.
 // Products and sums are exact or fp32, so the result differs from the
 // dequantise-then-multiply form only by not rounding (v - z) * s to 16 bits first.
-template <typename T>
-struct RawOperand;
-template <>
-struct RawOperand<_Float16> {
-  static constexpr uint32_t kMagic = 0x64006400u;  // 1024.0 twice
-  static constexpr uint32_t kOnes = 0x3c003c00u;
-  static constexpr float kBase = 1024.f;
-};
-template <>
-struct RawOperand<__bf16> {
-  static constexpr uint32_t kMagic = 0x43004300u;  // 128.0 twice
-  static constexpr uint32_t kOnes = 0x3f803f80u;
-  static constexpr float kBase = 128.f;
-};
-__device__ __forceinline__ u32x4_t raw_operand(uint32_t q, uint32_t magic) {
-  const uint32_t e0 = and_or(q, 0x000f000fu, magic);
-  const uint32_t e1 = and_or(q >> 4, 0x000f000fu, magic);
-  const uint32_t e2 = and_or(q >> 8, 0x000f000fu, magic);
-  const uint32_t e3 = and_or(q >> 12, 0x000f000fu, magic);
-  return u32x4_t{e0, e1, e2, e3};
-}
-
 // One unit's operands for the deferred-scale path, issued and awaited inside a
 // single asm block (a register must not be touched between the issue of the LDS
 // read that fills it and the counter wait): four weight chunks, four activation
@@ -1909,8 +1887,11 @@ int marlin_gemm_any(const void* a, int64_t a_row_stride, void* c, const uint32_t
       mid_applies(size_m, size_k, a_row_stride, num_groups, chk.group_size)) {
     const int format = chk.nvfp4 ? kMidNvFp4 : chk.fp4 ? kMidMxFp4 : chk.bits == 8 ? (chk.fp8 ? kMidFp8 : kMidInt8)
                        : chk.has_zp ? kMidInt4Zp : kMidInt4;
+    // What the decode kernel's blocks of rows would take keeps its precision: integers in the matrix cores, scales
+    // in fp32.  (The other kernels round scaled weights to 16 bits.)
+    const bool raw_codes = slab_fast || (mid_env && fast_shape && unit_group_shift >= -1);
     int row_blocks, splits;
-    double mid_us = mid_estimate(size_m, size_n, size_k, num_groups, dtype, format, cus, base_scratch, row_blocks, splits);
+    double mid_us = mid_estimate(size_m, size_n, size_k, num_groups, dtype, format, raw_codes, cus, base_scratch, row_blocks, splits);
     if (one_block) {
       mid_us = 0.0;
       row_blocks = 1;
@@ -1926,7 +1907,9 @@ int marlin_gemm_any(const void* a, int64_t a_row_stride, void* c, const uint32_t
         pieces *= 2;
       us = 4.5 + 3.3 * (size_k / 4096.0) / pieces;
     } else if (slab_fast) {
-      us = 6.5 + 0.0245 * (size_k / 4096.0) * n_strips * ((size_m + 31) / 32) * (size_m <= 64 && n_strips < cus / 2 ? 0.6 : 1.0);
+      // (measured / this, us: 17 rows, K 4096, N 6144 7.9 / 8.2; 64 rows, N 14336 18.6 / 18.9; 128 rows, N 14336 31.1 / 32.6; 128
+      // rows, K 2048, N 20032 27.2 / 24.4)
+      us = 5.3 + 0.0305 * (size_k / 4096.0) * n_strips * ((size_m + 31) / 32);
     } else if (use_tile) {
       // us per 1e9 operations: the wide kernel on 4-bit codes, on others, and the kernel with eight wavefronts
       const int64_t steps = size_k / 64, padding = (4 - steps % 4) % 4;
@@ -1942,7 +1925,7 @@ int marlin_gemm_any(const void* a, int64_t a_row_stride, void* c, const uint32_t
       splits = comma ? std::max(1, std::min(kMidMostSplits, atoi(comma + 1))) : 1;
       if ((size_t)splits * size_m * size_n * 4 > base_scratch || splits > size_k / 64) splits = 1;
     }
-    if (mid_env || mid_us < 0.93 * us) {
+    if (mid_env || mid_us < (raw_codes ? 1.0 : 0.93) * us) {
       MidParams q = {};
       q.a = static_cast<const uint16_t*>(a);
       q.lda = a_row_stride;
@@ -1960,6 +1943,7 @@ int marlin_gemm_any(const void* a, int64_t a_row_stride, void* c, const uint32_t
       q.chunks_per_strip = p.chunks_per_strip;
       q.cus = cus;
       q.splits = splits;
+      q.raw_codes = raw_codes && (!mid_env || row_blocks <= kMidMostRawRows);
       q.partial = static_cast<float4*>(scratch);
       return mid_gemm(q, dtype, format, row_blocks, st);
     }
