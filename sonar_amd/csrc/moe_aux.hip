@@ -344,6 +344,8 @@ extern "C" int sonar_moe_align_block_size(const int32_t* topk_ids, int64_t numel
   hipStream_t st = (hipStream_t)stream;
   const bool place = num_experts <= kAlignOneLaunchExperts;
   const size_t lds = (size_t)(2 * num_experts + 1 + kAlignWaves + (place ? kAlignWaves : 1) * num_experts) * sizeof(int32_t);
+  if (lds > 64 * 1024)   // from 5456 experts on (8192: 98372 bytes); HIP promises no more unasked, though ROCm 7.2 gives it
+    SONAR_HIP(hipFuncSetAttribute((const void*)moe_align_count_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   moe_align_count_kernel<<<1, kAlignThreads, lds, st>>>(topk_ids, (int)numel, (int)num_experts, (int)block_size,
                                                         sorted_token_ids, (int)sorted_len, expert_ids,
                                                         (int)expert_len, num_tokens_post_pad, expert_map,

@@ -442,6 +442,13 @@ def test_moe_align_kernel_matches_oracle(m, topk, e, bs):
     assert np.array_equal(expert_ids.cpu().numpy(), want_experts)
 
 
+# the histogram and the runs of all experts in LDS: the last count that fits a launch's ordinary 64 KiB, the first that does
+# not, and the most there may be
+@pytest.mark.parametrize("e", [5455, 5456, 8191, 8192])
+def test_moe_align_kernel_with_thousands_of_experts(e):
+    test_moe_align_kernel_matches_oracle(40, 4, e, 8)
+
+
 def test_moe_align_op_with_expert_map_matches_torch_expressions():
     from sonar_amd import fused_moe
     rng = np.random.default_rng(3)
