@@ -842,10 +842,15 @@ Tensor marlin_linear(const Tensor& input, const Tensor& weight, const OptTensor&
   OptTensor a_scales, c;
   if (act != 0) {
     if (b_type_id == SONAR_TYPE_FLOAT4_E2M1F) c = at::empty({x.size(0), padded_n}, input.options());
-    if (a_factor.has_value())
-      TORCH_CHECK(a_factor->is_cuda() && a_factor->scalar_type() == at::kFloat && a_factor->numel() == 1,
-                  "the factor of the activations' scales must be a float on the GPU");
-    std::tie(x, a_scales) = per_token_quant(x, act == 2, a_factor);
+    // one float on the GPU is multiplied in by the quantiser; anything else that a product with the scales takes (a
+    // number on the CPU, another type, one for every row), by the product
+    const bool fused = a_factor.has_value() && a_factor->device() == x.device() && a_factor->scalar_type() == at::kFloat &&
+                       a_factor->numel() == 1;
+    std::tie(x, a_scales) = per_token_quant(x, act == 2, fused ? a_factor : OptTensor());
+    if (a_factor.has_value() && !fused) {
+      c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+      a_scales = at::mul(*a_scales, *a_factor);
+    }
   }
   Tensor out = marlin_gemm(x, c, weight, bias, scales, a_scales, global_scale, zeros, g_idx, perm, workspace, b_type_id,
                            x.size(0), padded_n, padded_k, is_k_full, false, use_fp32_reduce, false);

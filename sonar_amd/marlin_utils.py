@@ -393,6 +393,8 @@ def apply_gptq_marlin_linear(input: torch.Tensor, weight: torch.Tensor, weight_s
     if input_dtype == torch.int8:      # marlin_utils.py:671-680
         assert wtype == scalar_types.uint4b8, "W8A8-INT8 is not supported by marlin kernel."
         act = 1
+        if input_global_scale is not None and not isinstance(input_global_scale, torch.Tensor):
+            input_global_scale = torch.tensor(input_global_scale)
     elif input_dtype == torch.float8_e4m3fn:
         assert wtype == scalar_types.uint4b8, "INT8 weight + FP8 activation is not supported."
         act = 2

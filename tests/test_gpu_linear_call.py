@@ -53,3 +53,25 @@ def test_linear_call_is_pad_quantise_multiply_unpad(shape, act, n, k):
                            scalar_types.uint4b8, a.shape[0], padded_n, padded_k, True, False, True, False)
     assert got.shape == shape + (n,) and got.is_contiguous()
     assert torch.equal(got.reshape(-1, n), want[:, :n])
+
+
+# what a product with the (rows, 1) scales of the activations takes
+@pytest.mark.parametrize("factor", [
+    lambda: torch.tensor(0.37), lambda: 0.37, lambda: torch.tensor([0.37], device="cuda"), lambda: torch.tensor(0.37, device="cuda"),
+    lambda: torch.tensor([0.37], device="cuda").half(), lambda: torch.tensor(0.37, device="cuda", dtype=torch.float64),
+    lambda: torch.linspace(0.2, 0.9, 5, device="cuda").unsqueeze(1), lambda: torch.full((1, 1), 0.37, device="cuda"),
+], ids=["cpu", "number", "float", "scalar", "half", "double_scalar", "per_row", "matrix"])
+def test_factor_of_the_activation_scales_in_every_form(factor):
+    m, n, k = 5, 128, 256
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    weight = torch.randint(-2 ** 31, 2 ** 31 - 1, (k // 16, 2 * n), dtype=torch.int32, device="cuda", generator=gen)
+    scales = (torch.rand((1, n), device="cuda", generator=gen) * 1e-2).half()
+    x = torch.randn((m, k), device="cuda", generator=gen).half()
+    empty = torch.empty(0, dtype=torch.int32, device="cuda")
+    workspace = mu.marlin_make_workspace_new(torch.device("cuda"))
+    got = mu.apply_gptq_marlin_linear(x, weight, scales, empty, empty, empty, workspace, scalar_types.uint4b8, n, k, True,
+                                      factor(), None, True, torch.int8)
+    a, a_scales = mu.marlin_quant_input(x, torch.int8)
+    want = ops.marlin_gemm(a, None, weight, None, scales, a_scales * factor(), None, empty, empty, empty, workspace,
+                           scalar_types.uint4b8, m, n, k, True, False, True, False)
+    assert torch.equal(got, want)
