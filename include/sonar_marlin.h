@@ -100,7 +100,8 @@ int sonar_marlin_last_decode_launch(int32_t* out, int n);
 /* GPTQ (K/8, N) int32, nibble k%8 of word [k/8][n] = code of W[k][n]
  * -> Marlin (K/16, 2N) int32; with num_bits == 8: (K/4, N) int32, byte k%4
  * -> Marlin (K/16, 4N) int32.  perm (int32[K], may be NULL) selects source
- * rows: output row k is source row perm[k].
+ * rows: output row k is source row perm[k].  Here and in the other functions that lay out weights and
+ * zero points, buffers of words may begin at any multiple of 4 bytes.
  * (gptq_marlin_repack, csrc/libtorch_stable/quantization/marlin/gptq_marlin_repack.cu:285-362) */
 int sonar_gptq_marlin_repack(const uint32_t* b_q_weight, const int32_t* perm,
                              uint32_t* out, int64_t size_k, int64_t size_n,
@@ -122,7 +123,7 @@ int sonar_awq_marlin_moe_repack(const uint32_t* b_q_weight, uint32_t* out, int64
 
 /* The checkpoint tensors around the codes.
  * marlin_permute_scales (grouped != 0: 64-column pattern; 0: the 32-column pattern of one group and
- * of marlin_permute_bias) on 16-bit elements, aphrodite quantization/utils/marlin_utils.py:404-434. */
+ * of marlin_permute_bias) on 16-bit elements (`out` 16-byte aligned), aphrodite quantization/utils/marlin_utils.py:404-434. */
 int sonar_marlin_permute_scales(const void* in, void* out, int64_t numel, int grouped, void* stream);
 /* Zero points packed along N, eight to a word, in plain or AWQ nibble order -> (rows, N/8) words in the
  * order the GEMM reads (marlin_utils.py:457-559: marlin_zero_points, awq_to_marlin_zero_points);

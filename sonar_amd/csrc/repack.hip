@@ -10,6 +10,10 @@ char* last_error_buffer() { return g_last_error; }
 
 namespace {
 
+// Four words from or to a caller's buffer, which need only be aligned as words (a view of a larger tensor): the loads and
+// stores of this chip take that, and the type makes the compiler choose instructions that do.
+typedef uint32_t words4_t __attribute__((ext_vector_type(4), aligned(4)));
+
 // Position of a weight inside a Marlin tile (16-bit activations, 4-bit
 // weights).  Word w = lane*4 + j of the tile; lane = 4*c + h, c = column % 8
 // inside the 16-column sub-tile j, h = (row % 8) / 2.  Nibble slot s of the
@@ -69,12 +73,12 @@ __global__ __launch_bounds__(256) void gptq_to_marlin_kernel(
 #pragma unroll
       for (int r = 0; r < 8; ++r) {
         const int k = rows[r];
-        const u32x4_t w = *reinterpret_cast<const u32x4_t*>(src + (long)(k >> 3) * size_n + col);
+        const u32x4_t w = *reinterpret_cast<const words4_t*>(src + (long)(k >> 3) * size_n + col);
 #pragma unroll
         for (int i = 0; i < 4; ++i) v[i] |= ((w[i] >> (4 * (k & 7))) & 0xFu) << (4 * r);
       }
     } else {
-      v = *reinterpret_cast<const u32x4_t*>(src + (long)(2 * kt + half) * size_n + col);
+      v = *reinterpret_cast<const words4_t*>(src + (long)(2 * kt + half) * size_n + col);
     }
     *reinterpret_cast<u32x4_t*>(mine + half * kMarlinTileN + col) = v;
   }
@@ -89,7 +93,7 @@ __global__ __launch_bounds__(256) void gptq_to_marlin_kernel(
     o[j] = interleave_nibbles((w[0] >> (8 * h)) & 0xFFu, (w[kMarlinTileN] >> (8 * h)) & 0xFFu,
                               (w[8] >> (8 * h)) & 0xFFu, (w[kMarlinTileN + 8] >> (8 * h)) & 0xFFu);
   }
-  *reinterpret_cast<u32x4_t*>(out + (long)tile * kMarlinTileWords + 4 * l) = o;
+  *reinterpret_cast<words4_t*>(out + (long)tile * kMarlinTileWords + 4 * l) = o;
 }
 
 __global__ __launch_bounds__(256) void awq_to_marlin_kernel(
@@ -106,7 +110,7 @@ __global__ __launch_bounds__(256) void awq_to_marlin_kernel(
     const int kt = (int)(t / n_tiles), nt = (int)(t - kt * n_tiles);
     const uint32_t* src = in + matrix * in_each + (long)(kt * kMarlinTileK + (l >> 1)) * (size_n / 8) +
                           nt * (kMarlinTileN / 8) + 4 * (l & 1);
-    *reinterpret_cast<u32x4_t*>(mine + 4 * l) = *reinterpret_cast<const u32x4_t*>(src);   // row l / 2 of the tile: 8 words
+    *reinterpret_cast<u32x4_t*>(mine + 4 * l) = *reinterpret_cast<const words4_t*>(src);   // row l / 2 of the tile: 8 words
   }
   __syncthreads();
   if (!live) return;
@@ -124,7 +128,7 @@ __global__ __launch_bounds__(256) void awq_to_marlin_kernel(
     }
     o[j] = interleave_nibbles(b[0], b[1], b[2], b[3]);
   }
-  *reinterpret_cast<u32x4_t*>(out + (long)tile * kMarlinTileWords + 4 * l) = o;
+  *reinterpret_cast<words4_t*>(out + (long)tile * kMarlinTileWords + 4 * l) = o;
 }
 
 // One thread per gfx950 word.  Word j of lane L of chunk c of strip s holds
@@ -492,8 +496,8 @@ __global__ __launch_bounds__(256) void awq_codes_to_gptq(const uint32_t* __restr
   }
   // x[p] now holds nibble p of every row; column c sits at nibble c / 2 + 4 (c % 2)
   uint32_t* dst = out + r * (8L * words) + 8 * w;
-  *reinterpret_cast<uint4*>(dst) = make_uint4(x[0], x[4], x[1], x[5]);
-  *reinterpret_cast<uint4*>(dst + 4) = make_uint4(x[2], x[6], x[3], x[7]);
+  *reinterpret_cast<words4_t*>(dst) = words4_t{x[0], x[4], x[1], x[5]};
+  *reinterpret_cast<words4_t*>(dst + 4) = words4_t{x[2], x[6], x[3], x[7]};
 }
 
 // AutoAWQ zero points (G, N/8) -> plain column order, transposed: (N/8, G).

@@ -37,6 +37,36 @@ def test_stacked_repack_is_the_repack_of_every_matrix(kind, experts, k, n):
     assert np.array_equal(got.cpu().numpy(), np.stack(want))
 
 
+# buffers that are aligned as words and no better: views that begin inside a larger tensor
+@pytest.mark.parametrize("offset", [1, 2, 3])
+def test_repack_of_views_that_begin_at_any_word(offset):
+    from sonar_amd import _lib, ops
+    from tests import gpu_util as gu
+    e, k, n = 2, 48, 192
+    rng = np.random.default_rng(offset)
+    words = e * k * n // 8
+    flat = _words(rng, words + 8).to(DEV)
+    perm = np.stack([rng.permutation(k) for _ in range(e)]).astype(np.int32)
+    none = torch.empty((e, 0), dtype=torch.int32, device=DEV)
+    gptq, awq = flat[offset:offset + words].view(e, k // 8, n), flat[offset:offset + words].view(e, k, n // 8)
+    assert gptq.data_ptr() % 16 == 4 * offset
+    host_gptq, host_awq = gptq.cpu().numpy(), awq.cpu().numpy()
+    for p, got in ((None, ops.gptq_marlin_moe_repack(gptq, none, k, n, 4)),
+                   (perm, ops.gptq_marlin_moe_repack(gptq, torch.from_numpy(perm).to(DEV), k, n, 4))):
+        want = np.stack([mo.gptq_marlin_repack(host_gptq[i], None if p is None else p[i], k, n) for i in range(e)])
+        assert np.array_equal(got.cpu().numpy(), want)
+    want = np.stack([mo.awq_marlin_repack(host_awq[i], k, n) for i in range(e)])
+    assert np.array_equal(ops.awq_marlin_moe_repack(awq, none, k, n, 4).cpu().numpy(), want)
+    codes, _ = torch.ops.sonar_amd.awq_to_standard(awq[0], awq[1][:2].contiguous())
+    assert np.array_equal(ops.gptq_marlin_repack(codes, none[0], k, n, 4).cpu().numpy(), want[0])
+    lib = _lib.load()
+    out = torch.empty(words + 4, dtype=torch.int32, device=DEV)[offset:offset + words]
+    _lib.check(lib.sonar_awq_marlin_moe_repack(gu.ptr(awq), gu.ptr(out), e, k, n, gu.stream()))
+    assert np.array_equal(out.cpu().numpy(), want.reshape(-1))
+    _lib.check(lib.sonar_awq_to_gptq(gu.ptr(awq), gu.ptr(out), k, n, gu.stream()))
+    assert torch.equal(out[:words // e], codes.reshape(-1))
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("rows,n,group", [(1, 64, -1), (3, 192, 128), (33, 1088, 64), (256, 4096, 32)])
 def test_permute_scales_and_bias(dtype, rows, n, group):
