@@ -9,14 +9,16 @@
 // column's 32 rows of a chunk in four lanes; v_permlane16_swap, one per two packed words, makes it two.
 //
 // What bounds it: with few rows the vector instructions that dequantise (9.5 per packed word, of which 2 put the
-// bytes into the order of K), with many rows power: the int8 instruction alone, on random operands, falls
-// to 21 ns (3.15 POP/s on the chip, of a nominal 5), and the multiply-adds of the group scales (16 per tile and
-// group) come on top.  R = 3 with 256 registers, R = 4 where the scales in flight leave room for it.
+// bytes into the order of K).  With many rows no unit alone: at 2048 rows, K 4096, N 11008, int8, the matrix pipes are 30 %
+// busy and vector issue 48 % (11.7 other vector instructions a matrix instruction: 16 multiply-adds of the group scales
+// per tile and group, and a wavefront dequantises its whole strip for 128 rows), and a third of the wavefronts' time is
+// waits and barriers; 1.35 POP/s, where the int8 instruction alone reaches 3.15 on random operands.  R = 3 with 256
+// registers, R = 4 where the scales in flight leave room for it.
 // Measured against the kernels it takes over from (us, before -> now):
 //   M  153, K 1152, N 22976, fp8:  42 -> 23       M  259, K 3456, N 20032, int8: 172 -> 40
 //   M  987, K 1664, N 12608, int8: 206 -> 55      M 2048, K 4096, N 11008, int8: 181 -> 137
 //   M 1929, K 3072, N 25216, int8, groups of 32, zero points: 1836 -> 536
-//   44 random shapes of 16 to 8192 rows, all formats: 1.93 times as fast (geometric mean)
+//   44 random shapes of 17 to 8192 rows: 1.69 times as fast (geometric mean; one, of 25 rows, 0.89)
 //
 // Pipeline, per step of 128 rows of K: activations (shared by the strips of a range) and packed codes (a wavefront's
 // own) go to LDS by LDS-DMA and the scales to registers, two steps ahead (three with one row block), and one

@@ -8,7 +8,9 @@
 // which the two strips share, are staged in LDS at half the bytes per matrix instruction of a one-strip
 // workgroup (at one strip the copies alone would need the whole 64 bytes per clock of a compute unit).
 //
-// What bounds it: issue slots of the vector unit.  Measured on this chip, a v_mfma_f32_16x16x32 takes 16 cycles of the
+// What bounds it: the sum of vector and matrix instructions, which two wavefronts a SIMD overlap in part, and the start and the
+// end.  (Counters at 64 to 333 rows: of the busy cycles vector issue fills 41 to 48 % and the matrix pipes 26 to 38 %; without
+// start and end 55 to 70 % and 35 to 50 %.)  Measured on this chip, a v_mfma_f32_16x16x32 takes 16 cycles of the
 // matrix pipe and 8 of the issue port when other vector instructions want it; those take 4.3 each (two-operand
 // logic, shifts and multiplies half of that).  A chunk (32 rows of a strip) costs 52 (fp16) to 68 (bf16) instructions
 // to dequantise and a few for its scales, beside 4 MB matrix instructions.  K = 4096, N = 8192, 64 rows, bf16:

@@ -44,7 +44,7 @@ inline bool mid_applies(int64_t size_m, int64_t size_k, int64_t lda, int64_t num
 
 // Microseconds a call takes in tiles of the best number of row blocks and splits of K, which are returned in
 // `row_blocks` and `splits`.  A fit of measured times (K = 2048 and 4096, N = 2048, 6144 and 20032, 17 to 768 rows, all
-// formats, mostly within 15 %): 4 us around the loop of a round of workgroups, and per 4096 rows of K 1.5 us for a row
+// formats, on weights that a cache holds, mostly within 15 %; from memory two rounds of tiles take 15 to 20 % more): 4 us around the loop of a round of workgroups, and per 4096 rows of K 1.5 us for a row
 // block's matrix instructions and a time that depends on the format for the dequantisation, which the matrix
 // instructions do not hide; more at the clock of a full chip than of a half empty one; no less than the weights take
 // from memory.  K is split where the tiles leave compute units idle, if the totals fit `room` bytes; the
