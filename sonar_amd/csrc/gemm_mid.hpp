@@ -44,13 +44,13 @@ inline bool mid_applies(int64_t size_m, int64_t size_k, int64_t lda, int64_t num
 
 // Microseconds a call takes in tiles of the best number of row blocks and splits of K, which are returned in
 // `row_blocks` and `splits`.  A fit of measured times (K = 2048 and 4096, N = 2048, 6144 and 20032, 17 to 768 rows, all
-// formats, on weights that a cache holds, mostly within 15 %; from memory two rounds of tiles take 15 to 20 % more): 4 us around the loop of a round of workgroups, and per 4096 rows of K 1.5 us for a row
-// block's matrix instructions and a time that depends on the format for the dequantisation, which the matrix
-// instructions do not hide; more at the clock of a full chip than of a half empty one; no less than the weights take
-// from memory.  K is split where the tiles leave compute units idle, if the totals fit `room` bytes; the
-// pass that adds them is 3.3 us and its bytes.  `raw_codes` (see MidParams) has a fit of its own (K = 2048, 4096 and
-// 8192, N = 2048 to 20032, 17 to 256 rows: 90 % within 7 % below and 11 % above): fewer instructions a chunk for the
-// dequantisation, more a row block for the fold.
+// formats, on weights that a cache holds, mostly within 15 %; from memory two rounds of tiles take 15 to 20 % more): 4 us
+// around the loop of a round of workgroups, and per 4096 rows of K 1.5 us for a row block's matrix instructions and a time
+// that depends on the format for the dequantisation, which the matrix instructions do not hide; more at the clock of a
+// full chip than of a half empty one; no less than the weights take from memory.  K is split where the tiles leave
+// compute units idle, if the totals fit `room` bytes; the pass that adds them is 3.3 us and its bytes.  `raw_codes` (see
+// MidParams) has a fit of its own (K = 1024 to 14336, N = 2048 to 28672, 17 to 256 rows, weights from memory: 90 % within
+// 6 % below and 13 % above): fewer instructions a chunk for the dequantisation, more a row block for the fold.
 inline double mid_estimate(int64_t size_m, int64_t size_n, int64_t size_k, int64_t num_groups, int dtype, int format,
                            bool raw_codes, int cus, size_t room, int& row_blocks, int& splits) {
   static const double kDequant[6][2] = {   // float16, bfloat16
@@ -69,9 +69,12 @@ inline double mid_estimate(int64_t size_m, int64_t size_n, int64_t size_k, int64
       const double k = (raw_codes ? 2 * (((steps / 2 + n - 1) / n + 3) / 4) : ((steps + n - 1) / n + 3) / 4) * 256 / 4096.0;
       const int64_t groups = tiles * n, rounds = (groups + cus - 1) / cus;
       double us = 1.5 + rounds * (4.0 + k * (dequant + 1.5 * mb) * (rounds > 2 ? 1.3 : 2 * groups > cus ? 1.1 : 0.85));
-      if (raw_codes) us = 1.4 + rounds * (1.6 + 0.3 * mb + k * (raw[0] + raw[1] * mb) * (2 * groups > cus ? 1.08 : 0.9));
+      if (raw_codes) {   // (one round: slower the more bytes its weights are)
+        const double slow = rounds > 1 ? 0.95 : (2 * groups > cus ? 0.86 : 0.8) + 2.5e-9 * size_n * size_k;
+        us = 1.4 + rounds * (2.4 + 0.3 * mb + k * (raw[0] + raw[1] * mb) * slow);
+      }
       if (us < memory) us = memory;
-      if (n > 1) us += raw_codes ? 2.5 + 1.3e-6 * n * size_m * size_n : 3.3 + 2e-6 * n * size_m * size_n;
+      if (n > 1) us += raw_codes ? 3.0 + 1.6e-6 * n * size_m * size_n : 3.3 + 2e-6 * n * size_m * size_n;
       if (us < best) best = us, row_blocks = mb, splits = n;
     }
   }

@@ -1720,6 +1720,25 @@ bool mid_switched_off() {
     if (getenv(name) != nullptr) return true;
   return false;
 }
+// Microseconds the decode kernel takes in blocks of rows: a fit of measured times (K = 1024 to 14336, N = 2048 to 28672, 17 to
+// 256 rows, weights from memory: 90 % within 7 %).  What counts is the launch: one block of 16 rows a workgroup while those
+// fit the compute units once (strips then in pieces), else two, and from there on the most workgroups on a compute unit.
+double decode_rows_estimate(int64_t size_m, int64_t n_strips, int64_t size_k, bool zero_points, int cus) {
+  const int64_t blocks16 = (size_m + 15) / 16, units = size_k / 128;
+  int pieces = 1;
+  if (size_m <= 64)
+    while (pieces < 8 && n_strips * 2 * pieces * blocks16 <= cus && units % (2 * pieces) == 0) pieces *= 2;
+  const bool pairs = n_strips * pieces * blocks16 > cus;
+  const int64_t workgroups = n_strips * pieces * (pairs ? (blocks16 + 1) / 2 : blocks16);
+  const double k = size_k / pieces / 1024.0, megabytes = n_strips * 64.0 * size_k / 2e6;
+  const int64_t most = (workgroups + cus - 1) / cus;
+  double us;
+  if (!pairs) us = 3.2 + 1.25 * k + (pieces > 1 ? 1.8 : 0.0);
+  else if (most == 1) us = 4.6 + 1.62 * k + 0.06 * megabytes;
+  else us = 2.6 + 1.2 * most + k * (0.2 + 1.4 * most) + (megabytes > 13.0 ? 0.06 * (megabytes - 13.0) : 0.0);
+  return zero_points ? 1.04 * us : us;
+}
+
 size_t stream_scratch_bytes() { return (size_t)2 * cu_count() * kSlotFloat4 * sizeof(float4); }
 thread_local int32_t g_last_decode_launch[4] = {0, 0, 0, 0};
 }  // namespace
@@ -1901,15 +1920,8 @@ int marlin_gemm_any(const void* a, int64_t a_row_stride, void* c, const uint32_t
     const double x = (double)size_n * size_k / (6144.0 * 4096.0), r = size_m / 64.0;
     // (what the other kernels take, us: fits of measured times, see mid_estimate)
     double us;
-    if (slab_fast && n_strips < 64) {   // strips in as many pieces as powers of two divide their units: often one
-      int pieces = 1;
-      while (pieces < 8 && n_strips * 2 * pieces * ((size_m + 15) / 16) <= cus && (p.chunks_per_strip / 4) % (2 * pieces) == 0)
-        pieces *= 2;
-      us = 4.5 + 3.3 * (size_k / 4096.0) / pieces;
-    } else if (slab_fast) {
-      // (measured / this, us: 17 rows, K 4096, N 6144 7.9 / 8.2; 64 rows, N 14336 18.6 / 18.9; 128 rows, N 14336 31.1 / 32.6; 128
-      // rows, K 2048, N 20032 27.2 / 24.4)
-      us = 5.3 + 0.0305 * (size_k / 4096.0) * n_strips * ((size_m + 31) / 32);
+    if (slab_fast) {
+      us = decode_rows_estimate(size_m, n_strips, size_k, chk.has_zp, cus);
     } else if (use_tile) {
       // us per 1e9 operations: the wide kernel on 4-bit codes, on others, and the kernel with eight wavefronts
       const int64_t steps = size_k / 64, padding = (4 - steps % 4) % 4;
