@@ -21,8 +21,11 @@
 // 64 bits is the output's own rounding (1.00 times it in fp16 and bf16; rounding each scaled weight: 1.28 times), and
 //   M   64, K 4096, N 28672, bf16: 22.6 -> 21.7      M  200, K 4096, N 6144, fp16, zero points: 20.4 -> 17.6
 //   M   80, K 4096, N 11008, bf16: 23.8 -> 18.4      M   17, K 2048, N 20032, bf16: 11.4 -> 10.0
-// against scaled weights or the decode kernel; but two sets of sums end at four row blocks, so that 65 to 96 rows lose
-// the single round of tiles they had on matrices of 129 to 256 pairs of strips (M 96, K 4096, N 28672: 30.3 -> 36; 45 in the decode kernel).
+// against scaled weights or the decode kernel.  But two sets of sums end at four row blocks, so that some calls lose the single
+// round of tiles of five or six that scaled weights have (fp16, scaled -> now, and the decode kernel):
+//   M   80, K 4096, N 28672: 27.9 -> 36.5, 45.0       M  144, K 4096, N 11008: 22.9 -> 27.9, 29.7
+// Five and six row blocks on four wavefronts with 512 registers each took 30 and 33 us in the first call with M 80 and 96, and
+// 1.5 times as long as eight wavefronts elsewhere.
 // Measured against the kernels it takes over from (us, before -> now):
 //   M   64, K 4096, N 28672, bf16: 29.1 -> 21.7      M  200, K 4096, N 6144, fp16, zero points: 24.6 -> 17.6
 //   M  333, K 2880, N  5760, bf16, groups of 32: 40.5 -> 21.7      M  512, K 4096, N 2048, bf16: 36 -> 20
