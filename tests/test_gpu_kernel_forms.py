@@ -89,6 +89,9 @@ def _without_the_mid_kernel() -> None:
                 tp.test_mxfp4_weights_dequant_bit_exact_and_gemm_within_tolerance(gu, m, 512, 192, m == 20)
             for zp, act in ((False, False), (True, False), (False, True)):
                 tp.test_marlin_gemm_within_tolerance(gu, dtype, m, 512, 192, 64, zp, act, m == 40)
+        # 132 strips x 2 pairs of row blocks: the decode kernel with four wavefronts
+        for g, zp in ((128, False), (-1, False), (128, True)):
+            tp.test_marlin_gemm_within_tolerance(gu, dtype, 40, 512, 8448, g, zp, False, zp)
         print("streaming", dtype, "ok", flush=True)
         for case in tp.TILE_CASES:
             if case[3] == 32:
