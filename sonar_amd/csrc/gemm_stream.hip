@@ -1923,10 +1923,8 @@ int marlin_gemm_any(const void* a, int64_t a_row_stride, void* c, const uint32_t
     if (slab_fast) {
       us = decode_rows_estimate(size_m, n_strips, size_k, chk.has_zp, cus);
     } else if (use_tile) {
-      // us per 1e9 operations: the wide kernel on 4-bit codes, on others, and the kernel with eight wavefronts
-      const int64_t steps = size_k / 64, padding = (4 - steps % 4) % 4;
-      const bool wide = chk.fp4 || (num_groups > 1 && chk.group_size == 32) ? padding == 0 : padding * 10 <= steps;
-      const double rate = chk.bits == 8 ? 1.05 : chk.fp4 ? 0.78 : wide || (dtype == SONAR_DTYPE_F16 && !chk.has_zp) ? 0.72 : 1.5;
+      // us per 1e9 operations of the wide kernel on 4-bit codes and on others
+      const double rate = chk.bits == 8 ? 1.05 : chk.fp4 ? 0.78 : 0.72;
       us = 25.0 + rate * 2e-9 * ((size_m + 127) / 128 * 128) * size_n * size_k;
     } else {   // (few strips: shared between workgroups, and a second launch that adds the shares)
       us = size_m <= 64 ? (n_strips < 64 ? 12.0 : 9.5) + x * (5.5 + 5.2 * r * r) : 11.0 + 10.7 * x * r;

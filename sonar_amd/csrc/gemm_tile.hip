@@ -812,9 +812,8 @@ __global__ __launch_bounds__(kTileWaves * 64) void marlin_tile_async_kernel(cons
 // bf16, a scale per 32 rows: one hardware conversion and half a byte permute behind each row
 // block), integer / 8-bit floating-point codes with a scale per 32 rows (MXFP8 among them), or NVFP4
 // (float4_e2m1f codes with a scale per 16 rows and a global scale, either activation type); no
-// act-order; dense and grouped (mixture-of-experts) calls.  K ranges that are not a
-// multiple of four steps are padded with steps of zeros (integer codes; taken only where that
-// is a small part of the range).
+// act-order; dense and grouped (mixture-of-experts) calls.  A pass of the loop is four steps, whose ring positions
+// are static; a K range that is no multiple of four steps leaves the last pass early.
 constexpr int kWideStages = 4;
 constexpr int kWideScaleRows = 16;   // a ring of 16 rows per wavefront: eight steps of one row, or of two (groups of 32 rows)
 // RB: row blocks of 16 rows a wavefront owns: 16 (a 256-row tile) or 8 (a 128-row tile, for
@@ -825,11 +824,6 @@ constexpr int wide_lds(int rb) { return wide_a(rb) + 4 * kWideScaleRows * 256; }
 // memory operations per wavefront and step: its blocks of A, the scale row (groups of 32 / 16 rows: two, one per
 // k block), two chunks (8-bit codes: four blocks)
 constexpr int wide_ops(int rb, bool fp4 = false, bool w8 = false) { return rb / 2 + (fp4 ? 2 : 1) + (w8 ? 4 : 2); }
-
-// One 128-byte line of zeros: what the copies of A fetch for the steps past the end of a K range that
-// is not a multiple of four steps (the loop always runs whole passes of four; those steps then add
-// zeros times the last step's weights).
-__device__ __attribute__((aligned(128))) const uint32_t kWideZeroLine[32] = {};
 
 // G32: a scale (and zero point) per 32 rows, i.e. one row of them per k block: MXFP4 always, integer codes when asked.
 // NV (with FP4): NVFP4, a scale per 16 rows: the row of a k block then holds two groups of 128 bytes (the copy
@@ -960,10 +954,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   auto issue_one = [&](int kt, int slot, int idx) __attribute__((always_inline)) {
     const int k = min(kt, k_tiles - 1);
     if (idx < RB / 2) {
-      // (the comparison is uniform: a pair of selects per copy)
-      const char* src = kt < k_tiles ? a_src[idx] + (long)k * (kTileK * 2)
-                                     : reinterpret_cast<const char*>(kWideZeroLine) + 16 * (lane & 7);
-      __builtin_amdgcn_global_load_lds((glb_void_t*)src,
+      __builtin_amdgcn_global_load_lds((glb_void_t*)(a_src[idx] + (long)k * (kTileK * 2)),
                                        (lds_void_t*)(smem + slot * kStage + ((RB / 2) * wave + idx) * kBlockBytes),
                                        16, 0, 0);
     } else if (idx < RB / 2 + (G32 ? 2 : 1)) {
@@ -1209,6 +1200,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
     chunk(R, 1, kt);
+    // the chunk of the next step is dequantised up to here: without this the compiler moves all of it behind the branch
+    // between the steps, where no matrix instruction hides it
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      asm volatile("" : "+v"(wb[0][j][0]), "+v"(wb[0][j][1]), "+v"(wb[0][j][2]), "+v"(wb[0][j][3]));
   };
 
   // ---- prologue: the scale row of the first step, then what steps k_first - 3 .. k_first - 1 would have issued
@@ -1252,13 +1248,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   for (int rb = 0; rb < kAhead; ++rb) SONAR_WIDE_READ(av[rb], a_base[0], rb * 2048);
   __builtin_amdgcn_sched_barrier(0);
 
-  // whole passes of four steps (the ring positions are static); steps past the end of the range
-  // multiply zeros
-  for (int kt = k_first; kt < k_tiles; kt += 4) {
+  for (int kt = k_first;; kt += 4) {
     step(0, kt);
+    if (kt + 1 >= k_tiles) break;
     step(1, kt + 1);
+    if (kt + 2 >= k_tiles) break;
     step(2, kt + 2);
+    if (kt + 3 >= k_tiles) break;
     step(3, kt + 3);
+    if (kt + 4 >= k_tiles) break;
   }
   // nothing in flight may outlive the wavefront (the copies of the steps past the end, the two
   // operand reads of the last half step), and the matrix pipeline drains before the results are read
@@ -1710,28 +1708,28 @@ int launch_tile(const TileParams& p, hipStream_t st) {
 }  // namespace
 
 namespace {
-// The wide form: groups of 64 * 2^i rows or one group; K ranges of a multiple of four steps, or long ones.
-// Groups of 32 rows: whole passes only.
-// Steps of zeros the wide kernel adds to a K range of `range` steps (at most a tenth of the range is accepted).
-int wide_padding(int range) { return (4 - range % 4) % 4; }
+// The wide form: groups of 32 or 64 * 2^i rows or one group, K of any number of steps.  (Passes of the loop were whole
+// before: up to three steps of zeros where that was at most a tenth of K, and eight wavefronts elsewhere.  Us, before ->
+// now: int4 with groups of 32, M = 4096, K = 2880, N = 5760 204 -> 142; AWQ, M = 4000, K = 1152, N = 6144 117 -> 71; NVFP4
+// bf16, M = 2048, K = 4480, N = 8192 148 -> 118; MXFP8, M = 3000, K = 2944, N = 6144 188 -> 168; int4, M = 2000, K = 2944,
+// N = 7808, once padded, 81.5 -> 78.3; 2000 tokens on 32 MXFP4 experts of 2880 x 2880, the whole layer 626 -> 543.)
 bool wide_applies(const TileParams& p) {
   static const bool no_wide = getenv("SONAR_MARLIN_NO_WIDE_TILE") != nullptr;   // debugging aid
   if (no_wide) return false;
-  // K ranges are rounded up to four steps with steps of zeros: not where that is a large part of the work
-  const int range = p.k_splits > 1 ? p.k_steps_per_split : p.size_k / kTileK;
-  if (wide_groups_of_32(p)) return wide_padding(range) == 0;
-  if (wide_padding(range) * 10 > range) return false;
-  if (p.num_groups == 1) return true;
+  if (p.num_groups == 1 || wide_groups_of_32(p)) return true;
   const int per_group = p.group_size / kTileK;   // steps per group: a power of two
   return p.group_size % kTileK == 0 && (per_group & (per_group - 1)) == 0;
 }
-// ... and for MXFP4 (groups of 32 rows, the caller has checked): the K ranges only.
+// ... and for MXFP4 and NVFP4 (groups of 32 and 16 rows, the caller has checked).  Dense MXFP4 calls whose 256-row tiles
+// leave a quarter of the compute units without one stay with eight wavefronts, at the higher clock of such a launch
+// the faster ones on these codes (M = 3000, K = 6656, N = 3072, 144 tiles: 127 us against 131; M = 2048, K = 4224, N = 5120,
+// 160 tiles: 85.6 against 88.4; but M = 2048, K = 6400, N = 7680, 240 tiles: 148 against 145, M = 4096, K = 4224, N = 8192,
+// 512 tiles: 215 against 201).
 bool wide_applies_fp4(const TileParams& p) {
   static const bool no_wide = getenv("SONAR_MARLIN_NO_WIDE_TILE") != nullptr;
-  const int range = p.k_splits > 1 ? p.k_steps_per_split : p.size_k / kTileK;
-  // (no padding here: the eight-wavefront kernel is as fast on these codes, and ahead once steps are wasted:
-  // K = 2880, N = 5760, M = 4096: 143 us against 156)
-  return !no_wide && wide_padding(range) == 0;
+  const bool few = p.tile_table == nullptr && p.global_scale == nullptr && p.tile_rows == kTileM && p.k_splits == 1 &&
+                   p.tile_count == 0 && p.tiles_m * p.tiles_n <= 192;
+  return !no_wide && !few;
 }
 // ... and for 8-bit codes (the same rule).
 bool wide_applies8(const TileParams& p) { return wide_applies(p); }
