@@ -474,6 +474,13 @@ int64_t sonar_debug_tile_schedule(int64_t size_m, int64_t size_n, int64_t size_k
 int64_t sonar_debug_moe_tile_schedule(int64_t row_tiles, int64_t max_row_tiles, int64_t size_n,
                                       int64_t size_k, int tile_rows, int with_partial,
                                       int32_t* out, int64_t out_rows);
+/* The same for a grouped call that runs both tile sizes in one launch, whose routing made `big`
+ * row tiles of three or four blocks and `small` of one or two: launch 0 are the 256-row tiles,
+ * launch 1 the 128-row ones.  chosen: the 256-row tiles that are halved, and the K ranges of
+ * the tiles of each size. */
+int64_t sonar_debug_moe_pair_schedule(int64_t big, int64_t small, int64_t max_row_tiles, int64_t size_n,
+                                      int64_t size_k, int with_partial, int32_t* chosen,
+                                      int32_t* out, int64_t out_rows);
 
 #ifdef __cplusplus
 }

@@ -50,8 +50,6 @@ struct TileParams {
   int tiles_m, tiles_n;
   int tile_rows;               // rows of a tile: 256 (128: marlin_tile_wide_kernel with 8 row blocks)
   int tile_band;               // rows of tiles per band of the tile numbering (tile_of_workgroup)
-  // the launch covers tiles [tile_begin, tile_begin + tile_count) of the numbering (tile_count 0: all of them)
-  int tile_begin, tile_count;
   // split K (k_splits > 1): workgroup (tile, split) of a split tile covers K steps
   // [split * k_steps_per_split, ...) and leaves its fp32 tile in `partial` for tile_reduce_kernel
   int k_splits, k_steps_per_split;
@@ -61,6 +59,12 @@ struct TileParams {
   const int32_t* sorted_ids;   // slot -> row id of C (row id / top_k of A), >= rows_total: padding
   const float* topk_weights;
   const int32_t* tile_table;   // [0]: number of row tiles, then (first block, blocks, expert) per tile
+  // launches with both tile sizes (marlin_tile_wide_pair_kernel): dense, the first `big_tiles` tiles of the 256-row
+  // numbering as they are and the others as two 128-row tiles each; grouped, `tile_table` of 256-row tiles and
+  // `table_small` of 128-row tiles (pair_word says what their first words hold)
+  int big_tiles;
+  const int32_t* table_small;
+  float4* partial_small;       // partial tiles of the 128-row tiles
   int rows_total, top_k, mul_topk;
   int a_by_slot;               // grouped: row of A = slot index (a column-permuted copy made per slot), else row id / top_k
   long expert_b_stride;        // uint4 units between experts in b
@@ -94,7 +98,7 @@ __host__ __device__ __forceinline__ void tile_coords(const TileParams& p, int ti
 }
 // Tiles of the launch, and those of them computed by one workgroup over the whole of K (the first ones).
 __host__ __device__ __forceinline__ int launch_tiles(const TileParams& p) {
-  return p.tile_count > 0 ? p.tile_count : p.tiles_m * p.tiles_n;
+  return p.tiles_m * p.tiles_n;
 }
 __host__ __device__ __forceinline__ int whole_tiles(const TileParams& p) {
   return p.k_splits > 1 ? p.whole_tiles : launch_tiles(p);
@@ -118,9 +122,7 @@ __host__ __device__ __forceinline__ bool tile_of_block(const TileParams& p, int 
   if (whole_k) {
     tile = xcd * whole_per_xcd + i;
     split = 0;
-    const bool mine = tile < whole;
-    tile += p.tile_begin;   // (a launch over a part of the numbering never splits K)
-    return mine;
+    return tile < whole;
   }
   // (a grouped launch is sized for the most tiles there could be: ids past this XCD's share do nothing)
   if (i - whole_per_xcd >= split_per_xcd) return false;
@@ -176,6 +178,147 @@ __host__ __device__ __forceinline__ TileParams live_tiles_of(const TileParams& p
   return live;
 }
 __device__ __forceinline__ TileParams live_tiles(const TileParams& p) { return live_tiles_of(p, p.tile_table[0]); }
+
+// ---- Launches with both tile sizes (marlin_tile_wide_pair_kernel).
+// What a 128-row tile takes of a 256-row tile's time.
+constexpr float kPairBig = 1.f, kPairSmall = 0.58f;
+// (A power of two, and floats below: these run in a kernel that is all latency.)
+constexpr int kPairCus = 256;
+// When the last of `big` longer and `small` shorter tiles ends, the longer ones started first and every tile on the compute
+// unit that is free first.
+__host__ __device__ __forceinline__ float pair_makespan(int big, float big_time, int small, float small_time) {
+  const int rounds = big / kPairCus, extra = big % kPairCus;
+  float t0 = rounds * big_time, t1 = t0 + big_time;      // compute units with `rounds` and one more of them
+  float end = extra > 0 ? t1 : t0;
+  if (small > 16 * kPairCus) return end + small * small_time * (1.f / kPairCus);
+  while (small > 0) {
+    const bool first = extra == 0 || t0 <= t1;
+    small -= first ? kPairCus - extra : extra;
+    (first ? t0 : t1) += small_time;
+    end = fmaxf(end, first ? t0 : t1);
+  }
+  return end;
+}
+// Steps of a range when K is cut into about `splits`, and the ranges there are then.
+__host__ __device__ __forceinline__ int pair_range(int k_steps, int splits) {
+  return splits > 1 ? ((k_steps + splits - 1) / splits + 3) / 4 * 4 : k_steps;
+}
+__host__ __device__ __forceinline__ int pair_ranges(int k_steps, int splits) {
+  const int range = pair_range(k_steps, splits);
+  return (k_steps + range - 1) / range;
+}
+// How a grouped call's rows are cut: of `big` 256-row and `small` 128-row row tiles at first, the last `halved` 256-row ones
+// become two 128-row tiles each, and K of the tiles of each size is cut into `splits[size]` ranges, whose partial tiles a second
+// kernel adds.
+struct PairPlan {
+  int halved, splits[2];
+};
+// The time that takes, and a little of the work it is (a launch with less of it leaves more of the power limit).
+__host__ __device__ __forceinline__ float pair_cost(int big, int small, const PairPlan& plan, int tiles_n, int k_steps) {
+  int tiles[2] = {(big - plan.halved) * tiles_n, (small + 2 * plan.halved) * tiles_n};
+  float time[2] = {kPairBig, kPairSmall}, extra = 0.f;
+  for (int i = 0; i < 2; ++i)
+    if (plan.splits[i] > 1) {   // (a K step of a 256-row tile is about 1.4 us, its start and end 13 us, the sum of the partial tiles 8 us)
+      tiles[i] *= plan.splits[i];
+      time[i] *= (k_steps / (float)plan.splits[i] + 11.f) / (k_steps + 9.f);
+      extra = 8.f / (1.4f * k_steps + 13.f);
+    }
+  const float work = (tiles[0] * time[0] + tiles[1] * time[1]) * (1.f / kPairCus);
+  return pair_makespan(tiles[0], time[0], tiles[1], time[1]) + extra + 0.125f * work;
+}
+// Whether the partial tiles of a plan have room: K is cut for all tiles of a size, while they are few.
+__host__ __device__ __forceinline__ bool pair_has_room(int big, int small, const PairPlan& plan, int tiles_n, int k_steps) {
+  const int tiles[2] = {(big - plan.halved) * tiles_n, (small + 2 * plan.halved) * tiles_n};
+  for (int i = 0; i < 2; ++i)
+    if (plan.splits[i] > 1 && (tiles[i] == 0 || tiles[i] > kLiveSplitTilesMax || tiles[i] * plan.splits[i] > kLiveSplitWorkMax ||
+                               k_steps < 8 * plan.splits[i]))
+      return false;
+  return true;
+}
+// Plans by number, at most 256: the first is none halved, nothing cut.
+__host__ __device__ __forceinline__ int pair_halved_step(int big, bool may_split) { return may_split ? big / 16 + 1 : big / 128 + 1; }
+__host__ __device__ __forceinline__ int pair_plans(int big, bool may_split) {
+  return (big / pair_halved_step(big, may_split) + 1) * (may_split ? 16 : 1);
+}
+__host__ __device__ __forceinline__ PairPlan pair_plan(int number, int big, bool may_split) {
+  PairPlan plan = {0, {1, 1}};
+  if (may_split) {
+    plan.splits[0] = number % 4 + 1;
+    plan.splits[1] = 1 << (number / 4 % 4);
+    number /= 16;
+  }
+  plan.halved = number * pair_halved_step(big, may_split);
+  return plan;
+}
+// The first word of a table of such a launch: its tiles, and above them the K ranges asked for less one.
+constexpr int kPairSplitShift = 27;
+__host__ __device__ __forceinline__ int pair_word(int tiles, int splits) { return tiles | ((splits - 1) << kPairSplitShift); }
+// The tiles of one size, from the first word of its table, in the terms that moe_tile_reduce_kernel reads.
+__host__ __device__ __forceinline__ TileParams pair_params(const TileParams& p, bool small, int word) {
+  TileParams q = p;
+  const int splits = (word >> kPairSplitShift) + 1, k_steps = p.size_k / kTileK;
+  q.tile_rows = small ? 128 : kTileM;
+  q.tile_table = small ? p.table_small : p.tile_table;
+  q.tiles_m = word & ((1 << kPairSplitShift) - 1);
+  q.tile_band = small ? 8 : 4;   // the same rows of A per band with either tile size
+  q.k_steps_per_split = pair_range(k_steps, splits);
+  q.k_splits = pair_ranges(k_steps, splits);
+  q.whole_tiles = 0;   // read only with k_splits > 1
+  if (small) q.partial = p.partial_small;
+  return q;
+}
+struct PairTile {
+  int rows, tile_m, tile_n, k_first, k_tiles;
+  int partial_at;   // -1: the whole of K
+};
+// Workgroup id -> tile.  Each XCD takes a contiguous run of the 256-row tiles and then one of the 128-row tiles.
+// Grouped: `big_word` and `small_word` are the first words of the two tables.  False: nothing to do.
+__host__ __device__ __forceinline__ bool pair_tile_of_block(const TileParams& p, int big_word, int small_word, int block,
+                                                            PairTile& out) {
+  const bool grouped = p.tile_table != nullptr;
+  const int xcd = block & 7, k_steps = p.size_k / kTileK;
+  int i = block >> 3;
+  TileParams q;
+  for (int size = 0; size < 2; ++size) {
+    int tiles, first = 0;
+    if (grouped) {
+      q = pair_params(p, size == 1, size == 1 ? small_word : big_word);
+      tiles = q.tiles_m * q.tiles_n;
+    } else {
+      q = p;
+      q.k_splits = 1;
+      tiles = p.big_tiles;
+      if (size == 1) {   // tile t of the 256-row numbering is tiles 2 t and 2 t + 1 of the 128-row one, in bands twice as high
+        q.tiles_m = 2 * p.tiles_m;
+        q.tile_band = 2 * p.tile_band;
+        first = 2 * p.big_tiles;
+        tiles = q.tiles_m * q.tiles_n - first;
+      }
+    }
+    const int work = tiles * q.k_splits;
+    const int begin = (int)((int64_t)work * xcd >> 3), end = (int)((int64_t)work * (xcd + 1) >> 3);
+    if (i < end - begin) {
+      i += begin;
+      const int split = q.k_splits > 1 ? i / tiles : 0;
+      out.rows = size == 1 ? 128 : kTileM;
+      out.partial_at = q.k_splits > 1 ? i : -1;
+      out.k_first = split * q.k_steps_per_split;
+      out.k_tiles = q.k_splits > 1 && out.k_first + q.k_steps_per_split < k_steps ? out.k_first + q.k_steps_per_split : k_steps;
+      tile_coords(q, first + i - split * tiles, out.tile_m, out.tile_n);
+      return grouped || out.tile_m * out.rows < p.size_m;   // (the second half of a ragged last tile may have no rows)
+    }
+    i -= end - begin;
+  }
+  return false;
+}
+inline int pair_grid(const TileParams& p, int max_tiles) {
+  if (p.tile_table == nullptr) {
+    const int smalls = 2 * (p.tiles_m * p.tiles_n - p.big_tiles);
+    return 8 * ((p.big_tiles + 7) / 8 + (smalls + 7) / 8);
+  }
+  // a tile has at least one block; K ranges: at most kLiveSplitWorkMax of either size
+  return 8 * ((max_tiles * p.tiles_n + 7) / 8 + 2 + (p.partial != nullptr ? 2 * kLiveSplitWorkMax / 8 : 0));
+}
 
 inline int tile_grid(const TileParams& p) {
   const int whole = whole_tiles(p);
@@ -829,10 +972,11 @@ constexpr int wide_ops(int rb, bool fp4 = false, bool w8 = false) { return rb / 
 // NV (with FP4): NVFP4, a scale per 16 rows: the row of a k block then holds two groups of 128 bytes (the copy
 // fetches one per half of the wavefront), and a lane, whose eight rows of a k block lie in one group, reads group
 // kb / 2; the global scale multiplies the sums at the end.
-template <typename T, bool HAS_ZP, bool GROUPED = false, int RB = 16, bool FP4 = false, int W8 = 0, bool G32 = FP4,
-          bool NV = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void marlin_tile_wide_kernel(
-    const TileParams p) {
+// The tile (tile_m, tile_n) of a launch, over K steps [k_first, k_tiles); `table`: of the row tiles of a grouped call;
+// partial_at: index of the workgroup's partial tile in `partial`, or -1 when it has the whole of K.
+template <typename T, bool HAS_ZP, bool GROUPED, int RB, bool FP4, int W8, bool G32, bool NV>
+__device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* table, float4* partial, const int tile_m,
+                                          const int tile_n, const int k_first, const int k_tiles, const int partial_at) {
   typedef typename Dq<T>::vec8 vec8;
   typedef typename Dq4Of<T, FP4, NV>::type D4;   // integer codes, or float4_e2m1f (MXFP4: bf16; NVFP4)
   typedef typename Dq8Of<T, W8 == 2>::type D8;   // 8-bit integer (W8 = 1) or floating-point (W8 = 2) codes
@@ -860,37 +1004,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   const uint32_t magic = magic_register();
   const bool grouped = p.num_groups > 1;
 
-  int tile, tile_m, tile_n, split;
-  bool whole_k;
-  int steps_per_split = p.k_steps_per_split;
-  int partial_at;   // without whole_k: index of this workgroup's partial tile, (split, split tile)
-  if (GROUPED) {
-    // The launch is sized for the most row tiles the routing could make; the tiles there are
-    // (tile_table[0]) are numbered here in bands of four row tiles, so that the 32 workgroups an
-    // XCD holds share 4 panels of A and 8 panels of W (of one expert where the routing is even),
-    // and every XCD gets its share of them.
-    // With room for partial tiles the K split is planned here too (plan_live_split).
-    const TileParams live = live_tiles(p);
-    if (live.tiles_m <= 0 || !tile_of_workgroup(live, tile, split, whole_k)) return;
-    tile_coords(live, tile, tile_m, tile_n);
-    steps_per_split = live.k_steps_per_split;
-    const int first_split = whole_tiles(live);
-    partial_at = split * (live.tiles_m * live.tiles_n - first_split) + tile - first_split;
-  } else {
-    if (!tile_of_workgroup(p, tile, split, whole_k)) return;
-    tile_coords(p, tile, tile_m, tile_n);
-    const int first_split = whole_tiles(p);
-    partial_at = split * (p.tiles_m * p.tiles_n - first_split) + tile - first_split;
-  }
   // Grouped calls: row tile t is up to four consecutive 64-slot blocks of one expert, listed in
   // tile_table; rows are slots of sorted_ids (as in marlin_tile_async_kernel).
   int first_slot = 0, tile_rows = kRows;
   long expert = 0;
   if (GROUPED) {
-    if (tile_m >= p.tile_table[0]) return;
-    first_slot = p.tile_table[1 + 3 * tile_m] * 64;
-    tile_rows = p.tile_table[2 + 3 * tile_m] * 64;
-    expert = p.tile_table[3 + 3 * tile_m];
+    first_slot = table[1 + 3 * tile_m] * 64;
+    tile_rows = table[2 + 3 * tile_m] * 64;
+    expert = table[3 + 3 * tile_m];
   }
   const int m0 = tile_m * kRows;
   const int strip0 = tile_n * (kTileN / kStripN);
@@ -934,10 +1055,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   char* sring = smem + kWideA + wave * (kWideScaleRows * 256);
   const uint32_t a_lds = (uint32_t)(uintptr_t)(lds_void_t*)smem;
   const uint32_t s_lds = (uint32_t)(uintptr_t)(lds_void_t*)sring;
-
-  // K steps [k_first, k_tiles) of this workgroup
-  const int k_first = whole_k ? 0 : split * steps_per_split;
-  const int k_tiles = whole_k ? p.size_k / kTileK : min(p.size_k / kTileK, k_first + steps_per_split);
 
   u32x4_t wq[kWideStages][2 * kChunkLoads];   // packed chunks in flight or waiting (8-bit: [2 b + h], h = high rows)
   // the scale row of step kt (clamped to the last step) into its ring position; MXFP4: the row of
@@ -1274,10 +1391,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 #undef SONAR_WIDE_READ
 
   if (!active) return;
-  if (!whole_k) {
+  if (partial_at >= 0) {
     // partial tile of this K range, in the order tile_reduce_kernel reads: 1-KiB blocks
     // (half of the rows, strip, column block, row block)
-    float4* dst = p.partial + ((size_t)partial_at * kRows + wave * 32) * 64 + lane;
+    float4* dst = partial + ((size_t)partial_at * kRows + wave * 32) * 64 + lane;
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb)
 #pragma unroll
@@ -1336,6 +1453,49 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   }
 }
 
+// One tile size.
+template <typename T, bool HAS_ZP, bool GROUPED = false, int RB = 16, bool FP4 = false, int W8 = 0, bool G32 = FP4,
+          bool NV = false>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void marlin_tile_wide_kernel(
+    const TileParams p) {
+  int tile, tile_m, tile_n, split;
+  bool whole_k;
+  // Grouped: the launch is sized for the most row tiles the routing could make; the tiles there are
+  // (tile_table[0]) are numbered here in bands of four row tiles, so that the 32 workgroups an
+  // XCD holds share 4 panels of A and 8 panels of W (of one expert where the routing is even),
+  // and every XCD gets its share of them.
+  // With room for partial tiles the K split is planned here too (plan_live_split).
+  TileParams live = p;
+  if (GROUPED) live = live_tiles(p);
+  if ((GROUPED && live.tiles_m <= 0) || !tile_of_workgroup(live, tile, split, whole_k)) return;
+  tile_coords(live, tile, tile_m, tile_n);
+  const int first_split = whole_tiles(live), k_steps = p.size_k / kTileK;
+  const int k_first = whole_k ? 0 : split * live.k_steps_per_split;
+  wide_tile<T, HAS_ZP, GROUPED, RB, FP4, W8, G32, NV>(
+      p, p.tile_table, p.partial, tile_m, tile_n, k_first, whole_k ? k_steps : min(k_steps, k_first + live.k_steps_per_split),
+      whole_k ? -1 : split * (live.tiles_m * live.tiles_n - first_split) + tile - first_split);
+}
+
+// Both tile sizes in one launch, the 256-row tiles first: the 128-row tiles start on the compute units that the last round
+// of 256-row tiles leaves idle, and there is one launch to wait for instead of two.  Us, before -> now: dense, M = 4096,
+// K = 4096, N = 6144, fp16, as two launches 167 -> 161; M = 4096, K = 2880, N = 5760 (368 tiles of 256 rows), int4 with groups of
+// 32 142 -> 120, MXFP4 131 -> 108; M = 4352, K = 8192, N = 4096 298 -> 229.  Mixture-of-experts layers, where two launches
+// and their sums of partial tiles followed each other: 8 experts 1408 x 3712, 2000 tokens 284 -> 195; 8 experts 3072 x 6784,
+// AWQ, 939 tokens 402 -> 298; 32 MXFP4 experts 2880 x 2880, 2000 tokens 543 -> 504; Mixtral-8x7B shapes, 2000 and 4096
+// tokens: level.
+template <typename T, bool HAS_ZP, bool GROUPED = false, bool FP4 = false, int W8 = 0, bool G32 = FP4>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void marlin_tile_wide_pair_kernel(
+    const TileParams p) {
+  PairTile t;
+  if (!pair_tile_of_block(p, GROUPED ? p.tile_table[0] : 0, GROUPED ? p.table_small[0] : 0, blockIdx.x, t)) return;
+  if (t.rows == kTileM)
+    wide_tile<T, HAS_ZP, GROUPED, 16, FP4, W8, G32, false>(p, p.tile_table, p.partial, t.tile_m, t.tile_n, t.k_first, t.k_tiles,
+                                                           t.partial_at);
+  else
+    wide_tile<T, HAS_ZP, GROUPED, 8, FP4, W8, G32, false>(p, p.table_small, p.partial_small, t.tile_m, t.tile_n, t.k_first,
+                                                          t.k_tiles, t.partial_at);
+}
+
 // Sums the partial tiles of the split tiles of a launch in split order, adds the
 // bias and writes C.  One wavefront per accumulator tile (16 rows x 16 columns).
 template <typename T>
@@ -1383,74 +1543,90 @@ template <typename T>
 __global__ __launch_bounds__(256) void moe_tile_reduce_kernel(const TileParams p) {
   const int lane = threadIdx.x & 63;
   const int col16 = lane & 15, kb = lane >> 4;
-  const int unit = blockIdx.x * 4 + (threadIdx.x >> 6);   // (split tile, 1-KiB block of the partial tile)
-  const TileParams live = live_tiles(p);
+  TileParams live;
+  if (p.table_small != nullptr) {   // of both tile sizes: the grid's second row adds those of the 128-row tiles
+    live = pair_params(p, blockIdx.y == 1, blockIdx.y == 1 ? p.table_small[0] : p.tile_table[0]);
+  } else {
+    live = live_tiles(p);
+  }
   if (live.tiles_m <= 0 || live.k_splits < 2) return;
   const int first_split = live.whole_tiles;
   const int tiles = live.tiles_m * live.tiles_n - first_split;
-  const int blocks = p.tile_rows;   // 1-KiB blocks per partial tile: 256 or 128
-  if (unit >= tiles * blocks) return;
-  const int tile = unit / blocks;
-  const int within = unit - tile * blocks;
-  const int half = within >> 7, wave = (within >> 5) & 3;
-  const int nb = (within >> 3) & 3, mb = within & 7;
-  int tile_m, tile_n;
-  tile_coords(live, first_split + tile, tile_m, tile_n);
-  const int strip = tile_n * (kTileN / kStripN) + wave;
-  if (strip * kStripN >= p.size_n) return;
-  const int first_slot = p.tile_table[1 + 3 * tile_m] * 64;
-  const int tile_rows = p.tile_table[2 + 3 * tile_m] * 64;
-  const long expert = p.tile_table[3 + 3 * tile_m];
-  const int r = 128 * half + 16 * mb + col16;
-  const int id = r < tile_rows ? p.sorted_ids[first_slot + r] : p.rows_total;
-  if ((unsigned)id >= (unsigned)p.rows_total) return;   // padding slot
-  floatx4_t acc = floatx4_t{0.f, 0.f, 0.f, 0.f};
-  for (int s = 0; s < live.k_splits; ++s) {
-    const float4 v = p.partial[((size_t)(s * tiles + tile) * blocks + within) * 64 + lane];
-    acc += floatx4_t{v.x, v.y, v.z, v.w};
-  }
-  if (p.global_scale) acc = acc * p.global_scale[expert];
-  const int nl = 16 * nb + 4 * kb;
-  float bias[4] = {0.f, 0.f, 0.f, 0.f};
-  if (p.bias) {
+  const int blocks = live.tile_rows;   // 1-KiB blocks per partial tile: 256 or 128
+  // units: (split tile, 1-KiB block of the partial tile)
+  for (int unit = blockIdx.x * 4 + (threadIdx.x >> 6); unit < tiles * blocks; unit += gridDim.x * 4) {
+    const int tile = unit / blocks;
+    const int within = unit - tile * blocks;
+    const int half = within >> 7, wave = (within >> 5) & 3;
+    const int nb = (within >> 3) & 3, mb = within & 7;
+    int tile_m, tile_n;
+    tile_coords(live, first_split + tile, tile_m, tile_n);
+    const int strip = tile_n * (kTileN / kStripN) + wave;
+    if (strip * kStripN >= p.size_n) continue;
+    const int first_slot = live.tile_table[1 + 3 * tile_m] * 64;
+    const int tile_rows = live.tile_table[2 + 3 * tile_m] * 64;
+    const long expert = live.tile_table[3 + 3 * tile_m];
+    const int r = 128 * half + 16 * mb + col16;
+    const int id = r < tile_rows ? p.sorted_ids[first_slot + r] : p.rows_total;
+    if ((unsigned)id >= (unsigned)p.rows_total) continue;   // padding slot
+    floatx4_t acc = floatx4_t{0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < live.k_splits; ++s) {
+      const float4 v = live.partial[((size_t)(s * tiles + tile) * blocks + within) * 64 + lane];
+      acc += floatx4_t{v.x, v.y, v.z, v.w};
+    }
+    if (p.global_scale) acc = acc * p.global_scale[expert];
+    const int nl = 16 * nb + 4 * kb;
+    float bias[4] = {0.f, 0.f, 0.f, 0.f};
+    if (p.bias) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      bias[i] = Dq<T>::to_float(p.bias[expert * p.expert_bias_stride + strip * kStripN + scale_slot(nl + i, false)]);
-  }
-  uint16_t o[4] = {Dq<T>::from_float(acc.x + bias[0]), Dq<T>::from_float(acc.y + bias[1]),
-                   Dq<T>::from_float(acc.z + bias[2]), Dq<T>::from_float(acc.w + bias[3])};
-  if (p.mul_topk) {
-    // rounded to the activation type, the product formed and rounded in that type (as in the kernel)
-    const float row_w = Dq<T>::to_float(Dq<T>::from_float(p.topk_weights[id]));
+      for (int i = 0; i < 4; ++i)
+        bias[i] = Dq<T>::to_float(p.bias[expert * p.expert_bias_stride + strip * kStripN + scale_slot(nl + i, false)]);
+    }
+    uint16_t o[4] = {Dq<T>::from_float(acc.x + bias[0]), Dq<T>::from_float(acc.y + bias[1]),
+                     Dq<T>::from_float(acc.z + bias[2]), Dq<T>::from_float(acc.w + bias[3])};
+    if (p.mul_topk) {
+      // rounded to the activation type, the product formed and rounded in that type (as in the kernel)
+      const float row_w = Dq<T>::to_float(Dq<T>::from_float(p.topk_weights[id]));
 #pragma unroll
-    for (int i = 0; i < 4; ++i) o[i] = Dq<T>::from_float(Dq<T>::to_float(o[i]) * row_w);
+      for (int i = 0; i < 4; ++i) o[i] = Dq<T>::from_float(Dq<T>::to_float(o[i]) * row_w);
+    }
+    uint2 packed;
+    packed.x = (uint32_t)o[0] | ((uint32_t)o[1] << 16);
+    packed.y = (uint32_t)o[2] | ((uint32_t)o[3] << 16);
+    *reinterpret_cast<uint2*>(p.c + (long)id * p.size_n + strip * kStripN + nl) = packed;
   }
-  uint2 packed;
-  packed.x = (uint32_t)o[0] | ((uint32_t)o[1] << 16);
-  packed.y = (uint32_t)o[2] | ((uint32_t)o[3] << 16);
-  *reinterpret_cast<uint2*>(p.c + (long)id * p.size_n + strip * kStripN + nl) = packed;
 }
 
 // Builds the row-tile table of a grouped call: runs of blocks with the same
 // expert are cut into tiles of up to four blocks.  With `table_small` the one or
 // two blocks a run ends in go there instead, to be computed as a 128-row tile at
-// half the cost.  One workgroup, a thread per block of slots: where a block's run begins comes from a
+// half the cost, and of the longer tiles as many are halved as makes the launch shortest
+// (pair_cost).  One workgroup, a thread per block of slots: where a block's run begins comes from a
 // ballot inside the wavefront and the other wavefronts' last run starts, a tile's number from counts of
 // the tile heads before it.  Latency bound (one thread scanning the blocks: 16 us at 157 blocks; 4 us so).
-constexpr int kTableThreads = 1024;
-constexpr int kTableWaves = kTableThreads / 64;
-__global__ __launch_bounds__(kTableThreads) void moe_tile_table_kernel(const int32_t* __restrict__ expert_ids,
+// (1024 threads for up to 256 blocks: 3 us longer, and the code of a kernel that runs once is fetched from memory.)
+template <int kTableWaves>
+__global__ __launch_bounds__(64 * kTableWaves) void moe_tile_table_kernel(const int32_t* __restrict__ expert_ids,
                                                                       const int32_t* __restrict__ num_post_pad,
                                                                       int num_blocks_max, int block_size,
                                                                       int num_experts, int32_t* __restrict__ table,
                                                                       int32_t* __restrict__ table_small,
-                                                                      int max_tiles) {
+                                                                      int max_tiles, int tiles_n, int k_steps,
+                                                                      int may_split) {
+  constexpr int kTableThreads = 64 * kTableWaves;
   __shared__ int32_t last_start[kTableWaves], heads[2][kTableWaves];
+  __shared__ unsigned long long best;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int blocks = min(num_post_pad[0] / block_size, num_blocks_max);
+  if (threadIdx.x == 0) best = ~0ull;
   int run_carry = 0;          // where the run that reaches into this round of blocks begins
   int count[2] = {0, 0};      // tiles so far: up to four blocks, and the small ones
-  for (int base = 0; base < blocks; base += kTableThreads) {
+  struct Tile {
+    int first, blocks, expert, number, small;
+    bool head;
+  };
+  // the tile that begins at this thread's block of the round from `base` on
+  auto scan = [&](int base) -> Tile {
     const int b = base + threadIdx.x;
     const int e = b < blocks ? expert_ids[b] : -1;
     const bool start = b < blocks && (b == 0 || expert_ids[b - 1] != e);
@@ -1480,20 +1656,54 @@ __global__ __launch_bounds__(kTableThreads) void moe_tile_table_kernel(const int
         if (w < wave) at[i] += t;
         count[i] += t;
       }
-    if (head) {
-      const int tile = at[small] + __popcll(mask[small] & ((1ull << lane) - 1ull));
-      if (tile < max_tiles) {
-        int32_t* t = (small ? table_small : table) + 1 + 3 * tile;
-        t[0] = b;
-        t[1] = n;
-        t[2] = e;
-      }
-    }
     __syncthreads();
+    return Tile{b, n, e, at[small] + (int)__popcll(mask[small] & ((1ull << lane) - 1ull)), small, head};
+  };
+  auto put = [&](int32_t* to, int i, int first, int num, int expert) {
+    if (i >= max_tiles) return;
+    int32_t* t = to + 1 + 3 * i;
+    t[0] = first;
+    t[1] = num;
+    t[2] = expert;
+  };
+  if (table_small == nullptr) {
+    for (int base = 0; base < blocks; base += kTableThreads) {
+      const Tile t = scan(base);
+      if (t.head) put(table, t.number, t.first, t.blocks, t.expert);
+    }
+    if (threadIdx.x == 0) table[0] = min(count[0], max_tiles);
+    return;
+  }
+  // two sizes: the tiles are counted first and written when it is known which are halved
+  Tile t = {};
+  for (int base = 0; base < blocks; base += kTableThreads) t = scan(base);
+  const int big = count[0], small = count[1], plans = pair_plans(big, may_split);
+  for (int i = threadIdx.x; i < plans; i += kTableThreads) {
+    const PairPlan plan = pair_plan(i, big, may_split);
+    if (!pair_has_room(big, small, plan, tiles_n, k_steps)) continue;
+    // (a positive float's bits order as it does)
+    const float cost = pair_cost(big, small, plan, tiles_n, k_steps);
+    atomicMin(&best, ((unsigned long long)__float_as_uint(cost) << 32) | (unsigned)i);
+  }
+  __syncthreads();
+  const PairPlan plan = pair_plan((int)(unsigned)best, big, may_split);
+  const int whole = big - plan.halved;
+  run_carry = count[0] = count[1] = 0;
+  for (int base = 0; base < blocks; base += kTableThreads) {
+    if (blocks > kTableThreads) t = scan(base);
+    if (!t.head) continue;
+    if (t.small) {
+      put(table_small, 2 * plan.halved + t.number, t.first, t.blocks, t.expert);
+    } else if (t.number < whole) {
+      put(table, t.number, t.first, t.blocks, t.expert);
+    } else {
+      put(table_small, 2 * (t.number - whole), t.first, 2, t.expert);
+      put(table_small, 2 * (t.number - whole) + 1, t.first + 2, t.blocks - 2, t.expert);
+    }
   }
   if (threadIdx.x == 0) {
-    table[0] = min(count[0], max_tiles);
-    if (table_small != nullptr) table_small[0] = min(count[1], max_tiles);
+    table[0] = pair_word(min(whole, max_tiles), plan.splits[0]);
+    table_small[0] = pair_word(min(small + 2 * plan.halved, max_tiles), plan.splits[1]);
   }
 }
 
@@ -1594,7 +1804,8 @@ int launch_tile_wide_fp4_rows(const TileParams& p, hipStream_t st) {
 }
 template <bool GROUPED>
 int launch_tile_wide_fp4(const TileParams& p, hipStream_t st) {
-  if (p.tile_rows == 128) return launch_tile_wide_fp4_rows<GROUPED, 8>(p, st);
+  if constexpr (!GROUPED)
+    if (p.tile_rows == 128) return launch_tile_wide_fp4_rows<false, 8>(p, st);
   return launch_tile_wide_fp4_rows<GROUPED, 16>(p, st);
 }
 // NVFP4: either activation type, groups of 16 rows, a global scale (one per expert when GROUPED)
@@ -1630,11 +1841,12 @@ int launch_tile_wide8_groups(const TileParams& p, hipStream_t st) {
 template <typename T, bool GROUPED>
 int launch_tile_wide8(const TileParams& p, bool fp8, hipStream_t st) {
   const bool g32 = wide_groups_of_32(p);
-  // 128-row tiles (dense calls with few tiles; the short ends of an expert's rows)
+  // 128-row tiles (dense calls with few tiles)
   if (p.tile_rows == 128 && g32) return fail(SONAR_E_INVALID, "internal: 8-bit codes with groups of 32 rows run on 256-row tiles");
-  if (p.tile_rows == 128)
-    return fp8 ? launch_tile_wide8_groups<T, GROUPED, 2, false, 8>(p, st)
-               : launch_tile_wide8_groups<T, GROUPED, 1, false, 8>(p, st);
+  if constexpr (!GROUPED)
+    if (p.tile_rows == 128)
+      return fp8 ? launch_tile_wide8_groups<T, false, 2, false, 8>(p, st)
+                 : launch_tile_wide8_groups<T, false, 1, false, 8>(p, st);
   if (fp8) return g32 ? launch_tile_wide8_groups<T, GROUPED, 2, true>(p, st)
                       : launch_tile_wide8_groups<T, GROUPED, 2, false>(p, st);
   return g32 ? launch_tile_wide8_groups<T, GROUPED, 1, true>(p, st)
@@ -1654,18 +1866,49 @@ int launch_tile_wide_g32_rows(const TileParams& p, hipStream_t st) {
 }
 template <typename T, bool HAS_ZP, bool GROUPED>
 int launch_tile_wide_g32(const TileParams& p, hipStream_t st) {
-  if constexpr (!GROUPED) {
+  if constexpr (!GROUPED)
     if (p.tile_rows == 128) return launch_tile_wide_g32_rows<T, HAS_ZP, false, 8>(p, st);
-  } else if (p.tile_rows == 128) {
-    return fail(SONAR_E_INVALID, "internal: grouped calls with groups of 32 rows run on 256-row tiles");
-  }
   return launch_tile_wide_g32_rows<T, HAS_ZP, GROUPED, 16>(p, st);
 }
 template <typename T, bool HAS_ZP, bool GROUPED = false>
 int launch_tile_wide(const TileParams& p, hipStream_t st) {
   if (wide_groups_of_32(p)) return launch_tile_wide_g32<T, HAS_ZP, GROUPED>(p, st);
-  if (p.tile_rows == 128) return launch_tile_wide_rows<T, HAS_ZP, GROUPED, 8>(p, st);
+  if constexpr (!GROUPED)   // (grouped: 128-row tiles run with the others in one launch)
+    if (p.tile_rows == 128) return launch_tile_wide_rows<T, HAS_ZP, false, 8>(p, st);
   return launch_tile_wide_rows<T, HAS_ZP, GROUPED, 16>(p, st);
+}
+
+// Both tile sizes; `max_row_tiles`: grouped calls, the most row tiles there can be.
+template <typename T, bool HAS_ZP, bool GROUPED, bool FP4, int W8, bool G32>
+int launch_pair_form(const TileParams& p, int max_row_tiles, hipStream_t st) {
+  static bool attr_set = false;
+  if (!attr_set) {
+    SONAR_HIP(hipFuncSetAttribute((const void*)marlin_tile_wide_pair_kernel<T, HAS_ZP, GROUPED, FP4, W8, G32>,
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, wide_lds(16)));
+    attr_set = true;
+  }
+  marlin_tile_wide_pair_kernel<T, HAS_ZP, GROUPED, FP4, W8, G32><<<pair_grid(p, max_row_tiles), 256, wide_lds(16), st>>>(p);
+  return SONAR_OK;
+}
+template <typename T, bool GROUPED>
+int launch_pair_type(const TileParams& p, int max_row_tiles, bool fp4, int bits, bool fp8, hipStream_t st) {
+  if constexpr (std::is_same<T, __bf16>::value)
+    if (fp4) return launch_pair_form<T, false, GROUPED, true, 0, true>(p, max_row_tiles, st);
+  if (fp4) return fail(SONAR_E_INVALID, "internal: MXFP4 weights with float16 activations");
+  if (bits == 8)
+    return fp8 ? launch_pair_form<T, false, GROUPED, false, 2, false>(p, max_row_tiles, st)
+               : launch_pair_form<T, false, GROUPED, false, 1, false>(p, max_row_tiles, st);
+  if (wide_groups_of_32(p))
+    return p.zeros ? launch_pair_form<T, true, GROUPED, false, 0, true>(p, max_row_tiles, st)
+                   : launch_pair_form<T, false, GROUPED, false, 0, true>(p, max_row_tiles, st);
+  return p.zeros ? launch_pair_form<T, true, GROUPED, false, 0, false>(p, max_row_tiles, st)
+                 : launch_pair_form<T, false, GROUPED, false, 0, false>(p, max_row_tiles, st);
+}
+template <bool GROUPED>
+int launch_pair(const TileParams& p, int max_row_tiles, int dtype, bool fp4, int bits, bool fp8, hipStream_t st) {
+  const int rc = dtype == SONAR_DTYPE_F16 ? launch_pair_type<_Float16, GROUPED>(p, max_row_tiles, fp4, bits, fp8, st)
+                                          : launch_pair_type<__bf16, GROUPED>(p, max_row_tiles, fp4, bits, fp8, st);
+  return rc ? rc : launch_status("marlin_tile_wide_pair_kernel");
 }
 
 template <typename T, bool HAS_ZP>
@@ -1728,7 +1971,7 @@ bool wide_applies(const TileParams& p) {
 bool wide_applies_fp4(const TileParams& p) {
   static const bool no_wide = getenv("SONAR_MARLIN_NO_WIDE_TILE") != nullptr;
   const bool few = p.tile_table == nullptr && p.global_scale == nullptr && p.tile_rows == kTileM && p.k_splits == 1 &&
-                   p.tile_count == 0 && p.tiles_m * p.tiles_n <= 192;
+                   p.tiles_m * p.tiles_n <= 192;
   return !no_wide && !few;
 }
 // ... and for 8-bit codes (the same rule).
@@ -1741,11 +1984,11 @@ bool tile_async_applies(bool has_perm, int64_t num_groups, int group_size) {
 }
 
 namespace {
-// What tile_gemm launches for a call the asynchronous tile kernels take: one launch (with
-// tile_reduce_kernel behind it when K is split), or two launches of the wide kernel.
+// What tile_gemm launches for a call the asynchronous tile kernels take: one tile size (with
+// tile_reduce_kernel behind it when K is split), or both sizes of the wide kernel.
 struct TileLaunches {
-  int count;          // 1 or 2; 0: an internal error
-  TileParams launch[2];
+  bool ok, pair;
+  TileParams launch;
 };
 
 // `p` arrives with the shape, the pointers and one 256-row launch over the whole of K filled in.
@@ -1753,7 +1996,8 @@ TileLaunches plan_tile_launches(TileParams p, int64_t size_m, int64_t size_n, in
                                 int group_size, void* partial, size_t partial_bytes, bool fp4, bool nvfp4, int bits,
                                 bool has_perm) {
   TileLaunches out;
-  out.count = 1;
+  out.ok = true;
+  out.pair = false;
   const int steps_per_group = group_size / kTileK;
   const bool wide128 = bits == 4 && !fp4 && !has_perm &&
                        (num_groups == 1 || (group_size % kTileK == 0 && (steps_per_group & (steps_per_group - 1)) == 0));
@@ -1792,38 +2036,31 @@ TileLaunches plan_tile_launches(TileParams p, int64_t size_m, int64_t size_n, in
       if (p.k_splits == 1) p.partial = nullptr;
     }
   }
-  out.launch[0] = p;
+  out.launch = p;
   if (p.tile_rows != kTileM && !(fp4 ? wide_applies_fp4(p) : wide_applies(p))) {
-    out.count = 0;   // 128-row tiles exist in the wide tile kernel only
+    out.ok = false;   // 128-row tiles exist in the wide tile kernel only
     return out;
   }
   auto takes_wide = [&](const TileParams& q) {
     return fp4 ? wide_applies_fp4(q) : (bits == 8 ? wide_applies8(q) : wide_applies(q));
   };
-  // More tiles than compute units with a short last round (M = 4096, N = 6144: 384 tiles of 256
-  // rows = 256 + 128): instead of cutting the K ranges of that round's tiles in two and summing
-  // partial tiles in a third launch, the full rounds run as they are and the last round runs in
-  // a second launch as twice as many 128-row tiles over the whole of K: nothing goes through
-  // scratch (163 + 18 us of split tiles and their sum before).  Tile t of the 256-row numbering
-  // is tiles 2 t and 2 t + 1 of the 128-row numbering with bands twice as high.
+  // More tiles than compute units with a last round that fills half of them or less (M = 4096, N = 6144: 384 tiles of 256
+  // rows = 256 + 128): the full rounds run as they are and the tiles of the last round as two 128-row tiles each, over
+  // the whole of K and in the same launch: nothing goes through scratch.  Tile t of the 256-row numbering is tiles 2 t and
+  // 2 t + 1 of the 128-row numbering with bands twice as high.
   static const bool no_two_sizes = getenv("SONAR_MARLIN_NO_TWO_TILE_SIZES") != nullptr;   // debugging aid
-  if (!no_two_sizes && !no_128 && rows128_ok && p.tile_rows == kTileM && plan.k_splits > 1 && plan.whole_tiles > 0 &&
-      (size_m - 1) % kTileM >= 128) {
-    TileParams big = p;
-    big.k_splits = 1;
-    big.k_steps_per_split = (int)(size_k / kTileK);
-    big.partial = nullptr;
-    big.tile_count = (int)plan.whole_tiles;
-    TileParams half = big;
-    half.tile_rows = 128;
-    half.tiles_m = 2 * p.tiles_m;
-    half.tile_band = 8;
-    half.tile_begin = 2 * (int)plan.whole_tiles;
-    half.tile_count = 2 * (p.tiles_m * p.tiles_n - (int)plan.whole_tiles);
-    if (takes_wide(big) && takes_wide(half)) {
-      out.count = 2;
-      out.launch[0] = big;
-      out.launch[1] = half;
+  const int tiles = p.tiles_m * p.tiles_n, last_round = tiles % 256;
+  // (Where K is long enough to be cut into three ranges or more, a short last round is shorter that way.)
+  if (!no_two_sizes && !no_128 && rows128_ok && p.tile_rows == kTileM && p.k_splits < 3 && tiles > 256 && last_round > 0 &&
+      last_round <= 128) {
+    TileParams both = p;
+    both.k_splits = 1;
+    both.k_steps_per_split = (int)(size_k / kTileK);
+    both.partial = nullptr;
+    both.big_tiles = tiles - last_round;
+    if (takes_wide(both)) {
+      out.pair = true;
+      out.launch = both;
     }
   }
   return out;
@@ -1841,7 +2078,6 @@ TileParams dense_tile_shape(int64_t size_m, int64_t size_n, int64_t size_k, int6
   p.tile_rows = kTileM;
   p.tiles_m = (int)((size_m + kTileM - 1) / kTileM);
   p.tile_band = 4;
-  p.tile_begin = p.tile_count = 0;
   p.tiles_n = (int)((size_n + kTileN - 1) / kTileN);
   p.k_splits = 1;
   p.whole_tiles = 0;  // read only with k_splits > 1
@@ -1874,7 +2110,7 @@ int tile_gemm(const void* a, int64_t a_row_stride, void* c, const uint32_t* b, c
       (!no_async || fp4 || bits == 8)) {   // float4 and 8-bit codes exist here only
     const TileLaunches plan = plan_tile_launches(p, size_m, size_n, size_k, num_groups, group_size, partial,
                                                  partial_bytes, fp4, nvfp4, bits, pm);
-    if (plan.count == 0)
+    if (!plan.ok)
       return fail(SONAR_E_INVALID, "internal: 128-row tiles exist in the wide tile kernel only");
     // the kernel a launch described by q takes
     auto launch = [&](const TileParams& q) -> int {
@@ -1900,13 +2136,8 @@ int tile_gemm(const void* a, int64_t a_row_stride, void* c, const uint32_t* b, c
       else
         return zp ? launch_tile_async<__bf16, true>(q, st) : launch_tile_async<__bf16, false>(q, st);
     };
-    if (plan.count == 2) {
-      if (int rc1 = launch(plan.launch[0])) return rc1;
-      if (int rc2 = launch_status("marlin_tile_wide_kernel")) return rc2;
-      if (int rc1 = launch(plan.launch[1])) return rc1;
-      return launch_status("marlin_tile_wide_kernel (128-row tiles)");
-    }
-    p = plan.launch[0];
+    p = plan.launch;
+    if (plan.pair) return launch_pair<false>(p, 0, dtype, fp4, bits, fp8, st);
     rc = launch(p);
     if (rc) return rc;
     if (int rc2 = launch_status("marlin_tile_async_kernel")) return rc2;
@@ -1968,8 +2199,7 @@ int moe_tile_gemm(const void* a, void* c, const uint32_t* b, const void* bias, c
                   size_t partial_bytes, hipStream_t st) {
   const int max_tiles = moe_tile_max(sorted_len, num_experts);
   const int blocks_max = (int)((sorted_len + 63) / 64);
-  TileParams p;
-  p.tile_begin = p.tile_count = 0;
+  TileParams p = {};
   p.global_scale = global_scale;   // NVFP4: one per expert
   p.a = static_cast<const uint16_t*>(a);
   p.lda = size_k;
@@ -2012,42 +2242,39 @@ int moe_tile_gemm(const void* a, void* c, const uint32_t* b, const void* bias, c
   if (wide && !no_live_split && partial != nullptr && partial_need > 0 && partial_bytes >= partial_need &&
       ((uintptr_t)partial) % 16 == 0)
     p.partial = static_cast<float4*>(partial);
-  // ... and computes the one or two blocks an expert's rows end in as a 128-row tile, in a launch of
-  // its own (the forms that have 128-row tiles: not NVFP4, not groups of 32 rows but MXFP4's)
+  // ... and computes the one or two blocks an expert's rows end in as a 128-row tile, and others where that makes the launch
+  // shorter (marlin_tile_wide_pair_kernel; not NVFP4, and not 8-bit codes with groups of 32 rows)
   static const bool no_small = getenv("SONAR_MARLIN_NO_MOE_128_ROW_TILES") != nullptr;   // debugging aid
   const bool nvfp4 = fp4 && global_scale != nullptr;
-  const bool two_sizes = wide && !no_small && !nvfp4 && (fp4 || !wide_groups_of_32(p));
+  const bool two_sizes = wide && !no_small && !nvfp4 && !(bits == 8 && wide_groups_of_32(p));
   int32_t* table_small = two_sizes ? table + moe_one_table_bytes(sorted_len) / sizeof(int32_t) : nullptr;
-  moe_tile_table_kernel<<<1, kTableThreads, 0, st>>>(expert_ids, num_post_pad, blocks_max, 64, (int)num_experts, table,
-                                                     table_small, max_tiles);
+  if (two_sizes) {
+    // tiles are cut along K only while they are few (and the second kernel is launched only where they may be): not when
+    // the rows nearly fill the chip wherever they go, or, with a long K, fill it twice
+    const int64_t least_tiles = (int64_t)(p.rows_total + 255) / 256 * p.tiles_n;
+    if (least_tiles > (size_k >= 64 * kTileK ? 512 : 192)) p.partial = nullptr;
+    if (p.partial != nullptr)
+      p.partial_small = reinterpret_cast<float4*>(static_cast<char*>(partial) + moe_partial_bytes_of(kTileM));
+  }
+  auto build_table = [&](auto kernel, int threads) {
+    kernel<<<1, threads, 0, st>>>(expert_ids, num_post_pad, blocks_max, 64, (int)num_experts, table, table_small, max_tiles,
+                                  p.tiles_n, (int)(size_k / kTileK), p.partial != nullptr);
+  };
+  if (blocks_max <= 256) build_table(moe_tile_table_kernel<4>, 256);
+  else build_table(moe_tile_table_kernel<16>, 1024);
   if (int rc = launch_status("moe_tile_table_kernel")) return rc;
   auto reduce = [&](const TileParams& q) -> int {
     if (q.partial == nullptr) return SONAR_OK;
     const int64_t tiles = std::min<int64_t>((int64_t)max_tiles * q.tiles_n, kLiveSplitTilesMax);
-    const int blocks = (int)(tiles * (q.tile_rows / 4));
+    const dim3 blocks((unsigned)std::min<int64_t>(tiles * (q.tile_rows / 4), 1024), q.table_small != nullptr ? 2 : 1);
     if (dtype == SONAR_DTYPE_F16) moe_tile_reduce_kernel<_Float16><<<blocks, 256, 0, st>>>(q);
     else moe_tile_reduce_kernel<__bf16><<<blocks, 256, 0, st>>>(q);
     return launch_status("moe_tile_reduce_kernel");
   };
   if (two_sizes) {
-    TileParams q = p;
-    q.tile_rows = 128;
-    q.tile_table = table_small;
-    if (p.partial != nullptr)
-      q.partial = reinterpret_cast<float4*>(static_cast<char*>(partial) + moe_partial_bytes_of(kTileM));
-    int rc;
-    if (fp4)
-      rc = launch_tile_wide_fp4<true>(q, st);
-    else if (bits == 8)
-      rc = dtype == SONAR_DTYPE_F16 ? launch_tile_wide8<_Float16, true>(q, fp8, st)
-                                    : launch_tile_wide8<__bf16, true>(q, fp8, st);
-    else if (dtype == SONAR_DTYPE_F16)
-      rc = zeros ? launch_tile_wide<_Float16, true, true>(q, st) : launch_tile_wide<_Float16, false, true>(q, st);
-    else
-      rc = zeros ? launch_tile_wide<__bf16, true, true>(q, st) : launch_tile_wide<__bf16, false, true>(q, st);
-    if (rc) return rc;
-    if (int rc2 = launch_status("tile kernel (grouped, 128-row tiles)")) return rc2;
-    if (int rc2 = reduce(q)) return rc2;
+    p.table_small = table_small;
+    if (int rc = launch_pair<true>(p, max_tiles, dtype, fp4, bits, fp8, st)) return rc;
+    return reduce(p);
   }
   int rc;
   if (fp4 && global_scale != nullptr && wide_applies_fp4(p))
@@ -2108,6 +2335,21 @@ int64_t schedule_rows(const sonar::TileParams& p, const sonar::TileParams& mappe
   }
   return at;
 }
+// A launch with both tile sizes, reported as launch 0 (256-row tiles) and launch 1.
+int64_t pair_schedule_rows(const sonar::TileParams& p, int big_word, int small_word, int grid, int32_t* out, int64_t out_rows) {
+  using namespace sonar;
+  int64_t at = 0;
+  for (int block = 0; block < grid; ++block) {
+    PairTile t;
+    if (!pair_tile_of_block(p, big_word, small_word, block, t)) continue;
+    if (at < out_rows) {
+      const int32_t row[6] = {t.rows == kTileM ? 0 : 1, t.rows, t.tile_m, t.tile_n, t.k_first, t.k_tiles};
+      std::copy(row, row + 6, out + 6 * at);
+    }
+    ++at;
+  }
+  return at;
+}
 }  // namespace
 
 // A dense call (4-bit integer codes, no act-order) with room for every partial tile.
@@ -2121,9 +2363,8 @@ extern "C" int64_t sonar_debug_tile_schedule(int64_t size_m, int64_t size_n, int
   const TileLaunches plan =
       plan_tile_launches(dense_tile_shape(size_m, size_n, size_k, num_groups, group_size), size_m, size_n, size_k,
                          num_groups, group_size, &never_read, ~(size_t)0, false, false, 4, false);
-  int64_t at = 0;
-  for (int l = 0; l < plan.count; ++l) at = schedule_rows(plan.launch[l], plan.launch[l], l, out, out_rows, at);
-  return at;
+  if (!plan.pair) return schedule_rows(plan.launch, plan.launch, 0, out, out_rows, 0);
+  return pair_schedule_rows(plan.launch, 0, 0, pair_grid(plan.launch, 0), out, out_rows);
 }
 
 // A grouped call whose routing made `row_tiles` row tiles of `tile_rows` rows, launched for up to
@@ -2143,4 +2384,36 @@ extern "C" int64_t sonar_debug_moe_tile_schedule(int64_t row_tiles, int64_t max_
   p.tile_table = &no_table;
   if (with_partial && moe_tile_partial_bytes(size_k) > 0) p.partial = &never_read;
   return schedule_rows(p, live_tiles_of(p, (int)row_tiles), 0, out, out_rows, 0);
+}
+
+// A grouped call whose routing made `big` row tiles of three or four blocks and `small` of one or two, with both tile
+// sizes in one launch, for up to `max_row_tiles` blocks.  What the device would choose comes back in `chosen`: 256-row tiles
+// that are halved, K ranges of the tiles of each size.
+extern "C" int64_t sonar_debug_moe_pair_schedule(int64_t big, int64_t small, int64_t max_row_tiles, int64_t size_n,
+                                                 int64_t size_k, int with_partial, int32_t* chosen, int32_t* out,
+                                                 int64_t out_rows) {
+  using namespace sonar;
+  if (big < 0 || small < 0 || 3 * big + small > max_row_tiles || size_n <= 0 || size_k <= 0 || size_k % kTileK != 0)
+    return -1;
+  static float4 never_read;
+  static int32_t no_table;
+  TileParams p = dense_tile_shape(max_row_tiles * kTileM, size_n, size_k, 1, (int)size_k);
+  p.tiles_m = (int)max_row_tiles;
+  p.tile_table = p.table_small = &no_table;
+  const int k_steps = p.size_k / kTileK;
+  if (with_partial && moe_tile_partial_bytes(size_k) > 0) p.partial = &never_read;
+  const bool may_split = p.partial != nullptr;
+  float best = 0.f;
+  PairPlan plan = pair_plan(0, (int)big, may_split);
+  for (int i = 0; i < pair_plans((int)big, may_split); ++i) {
+    const PairPlan one = pair_plan(i, (int)big, may_split);
+    if (!pair_has_room((int)big, (int)small, one, p.tiles_n, k_steps)) continue;
+    const float cost = pair_cost((int)big, (int)small, one, p.tiles_n, k_steps);
+    if (i == 0 || cost < best) best = cost, plan = one;
+  }
+  chosen[0] = plan.halved;
+  chosen[1] = plan.splits[0];
+  chosen[2] = plan.splits[1];
+  return pair_schedule_rows(p, pair_word((int)big - plan.halved, plan.splits[0]),
+                            pair_word((int)small + 2 * plan.halved, plan.splits[1]), pair_grid(p, (int)max_row_tiles), out, out_rows);
 }
