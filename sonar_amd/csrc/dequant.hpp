@@ -197,6 +197,19 @@ __device__ __forceinline__ u32x4_t raw_operand(uint32_t q, uint32_t magic) {
   return u32x4_t{e0, e1, e2, e3};
 }
 
+// The integers v - z themselves in fp16: the instructions of Dq<_Float16>::word() without the scale.
+__device__ __forceinline__ half8_t exact_operand(uint32_t q, uint32_t z, uint32_t magic) {
+  const half2_t r16 = half2_t{(_Float16)0.0625f, (_Float16)0.0625f};
+  const half2_t c0 = __builtin_bit_cast(half2_t, 0x64006400u + z * 0x00010001u);   // 1024 + z
+  const half2_t c1 = __builtin_bit_cast(half2_t, 0xD400D400u + z * 0x00100010u);   // -(64 + z)
+  const half2_t d0 = __builtin_bit_cast(half2_t, and_or(q, 0x000f000fu, magic)) - c0;
+  const half2_t d1 = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, and_or(q, 0x00f000f0u, magic)), r16, c1);
+  q >>= 8;
+  const half2_t d2 = __builtin_bit_cast(half2_t, and_or(q, 0x000f000fu, magic)) - c0;
+  const half2_t d3 = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, and_or(q, 0x00f000f0u, magic)), r16, c1);
+  return half8_t{d0.x, d0.y, d1.x, d1.y, d2.x, d2.y, d3.x, d3.y};
+}
+
 // Per-lane constants of the four columns (j = 0..3) a lane dequantises, for
 // the group `g` of strip `strip`.
 template <typename T, bool HAS_ZP, typename D = Dq<T>>

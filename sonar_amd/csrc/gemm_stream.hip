@@ -20,6 +20,7 @@
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>
+#include <type_traits>
 
 #include "dequant.hpp"
 #include "gemm_mid.hpp"
@@ -682,7 +683,7 @@ struct FastLane {
 template <int MB, int GPU>
 __device__ __forceinline__ void copy_weights(const StreamParams& p, const FastLane<MB>& fl, int strip, int unit,
                                              char* slot, int lane, int unit_group_shift) {
-  const uint4* gq = p.b + (size_t)(unsigned)(strip * p.chunks_per_strip + unit * 4) * 64 + lane;
+  const char* gq = reinterpret_cast<const char*>(p.b + (size_t)(unsigned)(strip * p.chunks_per_strip + unit * 4) * 64) + 16u * (uint32_t)lane;
   lds_void_t* lq = (lds_void_t*)slot;
   // `nt_weights` (a launch whose workgroups each read their weights once, on a matrix of 10 MB or
   // more): the copies carry the non-temporal bit, which streams the weights past the caches and
@@ -727,118 +728,57 @@ __device__ __forceinline__ void copy_activations(const StreamParams& p, const Fa
                                                  char* slot) {
   const char* ga = reinterpret_cast<const char*>(p.a) + (long)unit * (4 * kChunkK * 2);
 #pragma unroll
-  for (int mb = 0; mb < MB; ++mb) {
-    char* s = slot + 4096 * mb;
-    __builtin_amdgcn_global_load_lds((glb_void_t*)(ga + fl.a_off[2 * mb]), (lds_void_t*)(s), 16, 0, 0);
-    __builtin_amdgcn_global_load_lds((glb_void_t*)(ga + fl.a_off[2 * mb + 1]), (lds_void_t*)(s + 1024), 16, 0, 0);
-    __builtin_amdgcn_global_load_lds((glb_void_t*)(ga + 128 + fl.a_off[2 * mb]), (lds_void_t*)(s + 2048), 16, 0, 0);
-    __builtin_amdgcn_global_load_lds((glb_void_t*)(ga + 128 + fl.a_off[2 * mb + 1]), (lds_void_t*)(s + 3072), 16, 0, 0);
+  for (int h = 0; h < 2 * MB; ++h) {
+    // Eight rows that do not exist are not copied: what their places in LDS hold goes into rows of the sums that are
+    // not stored.  (The copies of a compute unit share 64 bytes a clock.  Four decoder layers of 7424 / 9472 / 25984, one
+    // row: 365 -> 359 us.)
+    if (h > 0 && 8 * h >= p.size_m) break;
+    char* s = slot + 4096 * (h >> 1) + 1024 * (h & 1);
+    __builtin_amdgcn_global_load_lds((glb_void_t*)(ga + fl.a_off[h]), (lds_void_t*)(s), 16, 0, 0);
+    __builtin_amdgcn_global_load_lds((glb_void_t*)(ga + 128 + fl.a_off[h]), (lds_void_t*)(s + 2048), 16, 0, 0);
   }
 }
 
 // Forming (v - z) * s per weight costs 13 VALU instructions per packed word in
 // fp16 and 17 in bf16 (gfx950 has no packed bf16 arithmetic), more than the
 // matrix work of a 16-row tile is worth.  The fast kernel instead feeds the
-// matrix cores the exact integers B + v (the nibble OR-ed into the mantissa of
-// B = 1024.0 in fp16, 128.0 in bf16: 7 instructions per word) and folds offset
-// and scale into the accumulator once per 128-row unit, which lies inside one
-// group:
-//   sum_k (v_k - z) s a_k = s * (sum_k (B + v_k) a_k - (B + z) * sum_k a_k),
+// matrix cores exact integers and applies the scales to fp32 sums once per 128-row unit, which lies inside one
+// group: in fp16 v - z (9 instructions a word), in bf16 128 + v (the nibble OR-ed into the mantissa of 128.0: 7
+// instructions) with
+//   sum_k (v_k - z) s a_k = s * (sum_k (128 + v_k) a_k - (128 + z) * sum_k a_k),
 // the last sum coming from one more MFMA per chunk with an all-ones operand.
 // Products and sums are exact or fp32, so the result differs from the
 // dequantise-then-multiply form only by not rounding (v - z) * s to 16 bits first.
-// One unit's operands for the deferred-scale path, issued and awaited inside a
-// single asm block (a register must not be touched between the issue of the LDS
-// read that fills it and the counter wait): four weight chunks, four activation
-// slices, the lane's four zero-point words, and the 16 scales of the output
-// rows the lane holds (column 16 j + 4 (lane / 16) + r of the strip, register
-// 4 j + r).  O0..O15 are the byte offsets of those scales from `s_at`.
-#define SONAR_UNIT_READS(O0, O1, O2, O3, O4, O5, O6, O7, O8, O9, O10, O11, O12, O13, O14, O15)      \
-  asm volatile(                                                                                    \
-      "ds_read_b128 %0, %25\n\t"                                                                   \
-      "ds_read_b128 %1, %25 offset:1024\n\t"                                                       \
-      "ds_read_b128 %2, %25 offset:2048\n\t"                                                       \
-      "ds_read_b128 %3, %25 offset:3072\n\t"                                                       \
-      "ds_read_b128 %4, %26\n\t"                                                                   \
-      "ds_read_b128 %5, %29\n\t"                                                                   \
-      "ds_read_b128 %6, %26 offset:2048\n\t"                                                       \
-      "ds_read_b128 %7, %29 offset:2048\n\t"                                                       \
-      "ds_read_b128 %8, %27\n\t"                                                                   \
-      "ds_read_u16 %9, %28 offset:" #O0 "\n\tds_read_u16 %10, %28 offset:" #O1 "\n\t"              \
-      "ds_read_u16 %11, %28 offset:" #O2 "\n\tds_read_u16 %12, %28 offset:" #O3 "\n\t"             \
-      "ds_read_u16 %13, %28 offset:" #O4 "\n\tds_read_u16 %14, %28 offset:" #O5 "\n\t"             \
-      "ds_read_u16 %15, %28 offset:" #O6 "\n\tds_read_u16 %16, %28 offset:" #O7 "\n\t"             \
-      "ds_read_u16 %17, %28 offset:" #O8 "\n\tds_read_u16 %18, %28 offset:" #O9 "\n\t"             \
-      "ds_read_u16 %19, %28 offset:" #O10 "\n\tds_read_u16 %20, %28 offset:" #O11 "\n\t"           \
-      "ds_read_u16 %21, %28 offset:" #O12 "\n\tds_read_u16 %22, %28 offset:" #O13 "\n\t"           \
-      "ds_read_u16 %23, %28 offset:" #O14 "\n\tds_read_u16 %24, %28 offset:" #O15 "\n\t"           \
-      "s_waitcnt lgkmcnt(0)"                                                                       \
-      : "=&v"(q0), "=&v"(q1), "=&v"(q2), "=&v"(q3), "=&v"(a0), "=&v"(a1), "=&v"(a2), "=&v"(a3),    \
-        "=&v"(row_z), "=&v"(row_s[0]), "=&v"(row_s[1]), "=&v"(row_s[2]), "=&v"(row_s[3]),          \
-        "=&v"(row_s[4]), "=&v"(row_s[5]), "=&v"(row_s[6]), "=&v"(row_s[7]), "=&v"(row_s[8]),       \
-        "=&v"(row_s[9]), "=&v"(row_s[10]), "=&v"(row_s[11]), "=&v"(row_s[12]), "=&v"(row_s[13]),   \
-        "=&v"(row_s[14]), "=&v"(row_s[15])                                                         \
-      : "v"(q_at), "v"(a_at), "v"(z_at), "v"(s_at), "v"(a_at ^ 64u)                                \
-      : "memory")
+// (fp16 with 1024 + v: the surplus is eight times as large against sums that are rounded at the same place, and the error
+// of K = 128 on activations with a mean reached 1.05 times the rounding of the output.)
+// The activations are the row operand of the matrix instructions: a lane's sums are four rows of one column, so that it
+// needs one scale (and zero point) a column block, and the surplus (B + z) sum_k a_k of those rows, which no column
+// changes without zero points, is what the sums of a unit start from.  (With the weights as the row operand a lane had
+// four columns: 16 scales to read and to widen and 32 multiply-adds a unit instead of 4 and 16, in bf16 332 instructions a
+// unit instead of 237.  Us, before -> now: four decoder layers of 4096 / 6144 / 14336, 16 rows, bf16 169 -> 164; AWQ with
+// groups of 64, K = 10368, N = 8256, 5 rows 19.0 -> 15.3; groups of 32, K = 6144, N = 3136, 16 rows 8.1 -> 7.4; 16 MXFP4 experts
+// 2560 x 10368, 29 tokens 184 -> 148; 16 tokens on Mixtral-8x7B experts 127 -> 123.  Two activation slots a wavefront,
+// filled as early as the weights': no change.)
 
-// The same with the 16 scales fetched as four 16-byte vectors (grouped scales, whose
-// permuted row holds the scales of columns 16 j + 4 (lane / 16) + r, j = 0..3, as the
-// low (lane / 32 == 0) or high 16 bits of the four words at byte 64 ((lane / 16) & 1) + 16 r):
-// 4 LDS instructions instead of 16.
-#define SONAR_UNIT_READS_VEC()                                                                     \
-  asm volatile(                                                                                    \
-      "ds_read_b128 %0, %13\n\t"                                                                   \
-      "ds_read_b128 %1, %13 offset:1024\n\t"                                                       \
-      "ds_read_b128 %2, %13 offset:2048\n\t"                                                       \
-      "ds_read_b128 %3, %13 offset:3072\n\t"                                                       \
-      "ds_read_b128 %4, %14\n\t"                                                                   \
-      "ds_read_b128 %5, %17\n\t"                                                                   \
-      "ds_read_b128 %6, %14 offset:2048\n\t"                                                       \
-      "ds_read_b128 %7, %17 offset:2048\n\t"                                                       \
-      "ds_read_b128 %8, %15\n\t"                                                                   \
-      "ds_read_b128 %9, %16\n\t"                                                                   \
-      "ds_read_b128 %10, %16 offset:16\n\t"                                                        \
-      "ds_read_b128 %11, %16 offset:32\n\t"                                                        \
-      "ds_read_b128 %12, %16 offset:48\n\t"                                                        \
-      "s_waitcnt lgkmcnt(0)"                                                                       \
-      : "=&v"(q0), "=&v"(q1), "=&v"(q2), "=&v"(q3), "=&v"(a0), "=&v"(a1), "=&v"(a2), "=&v"(a3),    \
-        "=&v"(row_z), "=&v"(sv0), "=&v"(sv1), "=&v"(sv2), "=&v"(sv3)                               \
-      : "v"(q_at), "v"(a_at), "v"(z_at), "v"(sv_at), "v"(a_at ^ 64u)                               \
-      : "memory")
-
-// The activation operands of a second block of 16 rows (4 KiB after the first).
-#define SONAR_UNIT_READS_ROWS2(B0, B1, B2, B3)                                                      \
-  asm volatile(                                                                                    \
-      "ds_read_b128 %0, %4 offset:4096\n\t"                                                        \
-      "ds_read_b128 %1, %5 offset:4096\n\t"                                                        \
-      "ds_read_b128 %2, %4 offset:6144\n\t"                                                        \
-      "ds_read_b128 %3, %5 offset:6144\n\t"                                                        \
-      "s_waitcnt lgkmcnt(0)"                                                                       \
-      : "=&v"(B0), "=&v"(B1), "=&v"(B2), "=&v"(B3)                                                 \
-      : "v"(a_at), "v"(a_at ^ 64u)                                                                 \
-      : "memory")
-
-// Zero-point words and the 16 scales of one more group of the unit (GI = 1..3, 256 bytes per group).
-#define SONAR_GROUP_READS(GI)                                                                       \
-  asm volatile(                                                                                    \
-      "ds_read_b128 %0, %17\n\t"                                                                   \
-      "ds_read_u16 %1, %18\n\tds_read_u16 %2, %18 offset:16\n\t"                                  \
-      "ds_read_u16 %3, %18 offset:32\n\tds_read_u16 %4, %18 offset:48\n\t"                        \
-      "ds_read_u16 %5, %18 offset:4\n\tds_read_u16 %6, %18 offset:20\n\t"                         \
-      "ds_read_u16 %7, %18 offset:36\n\tds_read_u16 %8, %18 offset:52\n\t"                        \
-      "ds_read_u16 %9, %18 offset:8\n\tds_read_u16 %10, %18 offset:24\n\t"                        \
-      "ds_read_u16 %11, %18 offset:40\n\tds_read_u16 %12, %18 offset:56\n\t"                      \
-      "ds_read_u16 %13, %18 offset:12\n\tds_read_u16 %14, %18 offset:28\n\t"                      \
-      "ds_read_u16 %15, %18 offset:44\n\tds_read_u16 %16, %18 offset:60\n\t"                      \
-      "s_waitcnt lgkmcnt(0)"                                                                       \
-      : "=&v"(more_z[GI - 1]), "=&v"(more_s[GI - 1][0]), "=&v"(more_s[GI - 1][1]),                  \
-        "=&v"(more_s[GI - 1][2]), "=&v"(more_s[GI - 1][3]), "=&v"(more_s[GI - 1][4]),                \
-        "=&v"(more_s[GI - 1][5]), "=&v"(more_s[GI - 1][6]), "=&v"(more_s[GI - 1][7]),                \
-        "=&v"(more_s[GI - 1][8]), "=&v"(more_s[GI - 1][9]), "=&v"(more_s[GI - 1][10]),               \
-        "=&v"(more_s[GI - 1][11]), "=&v"(more_s[GI - 1][12]), "=&v"(more_s[GI - 1][13]),             \
-        "=&v"(more_s[GI - 1][14]), "=&v"(more_s[GI - 1][15])                                         \
-      : "v"(z_at + 256u * (GI)), "v"(s_at + 256u * (GI))                                           \
-      : "memory")
+// Four rows of one column per lane -> four columns of one row: lane 16 q + 4 u + v of a tile of the matrix cores holds rows
+// 4 q .. 4 q + 3 of column 4 u + v, and afterwards columns 4 u .. 4 u + 3 of row 4 q + v, which is what the functions
+// above call lane (4 q + v) + 16 u.
+__device__ __forceinline__ int quad_lane(int lane) { return (lane >> 4) * 4 + (lane & 3) + 16 * ((lane >> 2) & 3); }
+__device__ __forceinline__ floatx4_t quad_transpose(floatx4_t x, int lane) {
+  auto swap = [](float v, auto ctrl) {
+    return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), decltype(ctrl)::value, 0xf, 0xf, true));
+  };
+  typedef std::integral_constant<int, 0xB1> Next;   // quad_perm [1, 0, 3, 2]
+  typedef std::integral_constant<int, 0x4E> Pair;   // quad_perm [2, 3, 0, 1]
+  const bool odd = lane & 1, high = lane & 2;
+  const float a = swap(odd ? x.x : x.y, Next()), b = swap(odd ? x.z : x.w, Next());
+  if (odd) x.x = a, x.z = b;
+  else x.y = a, x.w = b;
+  const float c = swap(high ? x.x : x.z, Pair()), d = swap(high ? x.y : x.w, Pair());
+  if (high) x.x = c, x.y = d;
+  else x.z = c, x.w = d;
+  return x;
+}
 
 // MB blocks of 16 rows per workgroup (1 or 2): the weights of a unit are pulled
 // out of LDS and turned into operands once and multiplied with every block.
@@ -856,8 +796,8 @@ __device__ __forceinline__ void copy_activations(const StreamParams& p, const Fa
 // strip's ticket.  (A third weight slot per wavefront was measured slower than two on every
 // Llama-3-8B shape: M = 16, down 12.2 against 11.4 us, gate_up 19.1 against 17.4.)
 template <typename T, bool HAS_ZP, int kFastWaves, int MB, bool GROUPED = false, int GPU = 1, bool FP4 = false>
-__global__ __launch_bounds__(kFastWaves * 64) void marlin_stream_fast_kernel(const StreamParams params,
-                                                                             const int unit_group_shift) {
+__global__ __launch_bounds__(kFastWaves * 64, 2) void marlin_stream_fast_kernel(const StreamParams params,
+                                                                                const int unit_group_shift) {
   typedef typename Dq<T>::vec8 vec8;
   constexpr int kWaveLds = wave_lds(MB, GPU);
   constexpr int kSlotBytes = slot_bytes(GPU);
@@ -874,7 +814,7 @@ __global__ __launch_bounds__(kFastWaves * 64) void marlin_stream_fast_kernel(con
     asm volatile("" ::"s"(p.a), "s"(p.lda), "s"(p.c), "s"(p.b), "s"(p.bias), "s"(p.scales), "s"(p.zeros),
                  "s"(p.scratch), "s"(p.size_m), "s"(p.size_n), "s"(p.num_groups), "s"(p.chunks_per_strip),
                  "s"(p.units_per_strip), "s"(p.parts), "s"(p.slabs), "s"(p.grid_parts), "s"(p.tickets),
-                 "s"(p.ticket_stride), "s"(p.xcd_ranges), "s"(p.piece_shift), "s"(p.piece_units),
+                 "s"(p.ticket_stride), "s"(p.xcd_ranges), "s"(p.piece_shift), "s"(p.piece_units), "s"(p.nt_weights),
                  "s"(unit_group_shift));
   int part, slab;
   if constexpr (GROUPED) {   // strip-major inside a block of slots
@@ -885,7 +825,7 @@ __global__ __launch_bounds__(kFastWaves * 64) void marlin_stream_fast_kernel(con
   }
   if (part >= p.parts) return;
   const int lane = threadIdx.x & 63;
-  int row_id[MB] = {};  // grouped calls: the row of C that row (lane & 15) of block of rows mb goes to, or -1
+  int row_id[MB] = {};  // grouped calls: the row of C that row (quad_lane & 15) of block of rows mb goes to, or -1
   if constexpr (GROUPED) {
     // `slab` names the block of slots and the 32 rows of it; the whole workgroup leaves together
     const int block = slab / p.sub_blocks;
@@ -897,9 +837,9 @@ __global__ __launch_bounds__(kFastWaves * 64) void marlin_stream_fast_kernel(con
     p.scales += expert * p.expert_s_stride;
     if (HAS_ZP) p.zeros += expert * p.expert_z_stride;
     if (p.bias) p.bias += expert * p.expert_bias_stride;
-    p.size_m = 16 * MB;
+    p.size_m = min(16 * MB, p.block_size - row0);
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) row_id[mb] = moe_row_id(p, block, row0 + 16 * mb + (lane & 15));
+    for (int mb = 0; mb < MB; ++mb) row_id[mb] = moe_row_id(p, block, row0 + 16 * mb + (quad_lane(lane) & 15));
     // nothing but padding in these rows (the tail of an expert's last block): every
     // wavefront sees the same ids, so the workgroup leaves as one
     bool any_row = false;
@@ -953,14 +893,16 @@ __global__ __launch_bounds__(kFastWaves * 64) void marlin_stream_fast_kernel(con
   // chunks 2 and 3 (+ 4096 for the second block of rows).
   const uint32_t a_at = ring_lds + kWaveA + (col16 >> 3) * 1024 + (col16 & 7) * 128 +
                         ((uint32_t)((lane >> 4) ^ (col16 & 7)) * 16);
-  // where the scales / zero points of this lane's output rows sit inside a weight slot
-  const int q4 = lane >> 4;
-  const uint32_t row_s_off = kSlotS + (grouped ? 64 * (q4 & 1) + 2 * (q4 >> 1) : 32 * (q4 & 1) + 4 * (q4 >> 1));
-  const uint32_t row_z_off = kSlotS + 128 + 16 * (q4 & 1);
-  const uint32_t row_z_shift = 16 * (q4 >> 1);
-  // bfloat16 scales of one group per unit: row_s holds float bits
-  constexpr bool kVecScales = sizeof(typename Dq<T>::vec8) == 16 && __is_same(T, __bf16) && GPU == 1;
-  const uint32_t scale_half = (q4 >> 1) ? 0x07060c0cu : 0x05040c0cu;   // byte selector: high or low 16 bits, shifted up
+  // Where the scales of this lane's columns 16 j + col16 (j = 0..3) sit inside a weight slot, and their zero points: four bits
+  // each of the 16 from z_shift on.
+  const int q4 = col16 >> 2, r4 = col16 & 3;
+  uint32_t s_at[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    s_at[j] = ring_lds + kSlotS + (grouped ? 64 * (q4 & 1) + 16 * r4 + 4 * j + 2 * (q4 >> 1)
+                                           : 32 * (q4 & 1) + 4 * (q4 >> 1) + 64 * (j >> 1) + 8 * (j & 1) + 16 * (r4 >> 1) + 2 * (r4 & 1));
+  const uint32_t z_at = ring_lds + kSlotS + 128 + 16 * (q4 & 1) + 4 * r4, z_shift = 16 * (q4 >> 1);
+  const uint32_t q_at = ring_lds + lane * 16;
   const uint32_t magic = magic_register(RawOperand<T>::kMagic);
   u32x4_t ones = u32x4_t{RawOperand<T>::kOnes, RawOperand<T>::kOnes, RawOperand<T>::kOnes, RawOperand<T>::kOnes};
   asm("" : "+v"(ones));
@@ -975,7 +917,6 @@ __global__ __launch_bounds__(kFastWaves * 64) void marlin_stream_fast_kernel(con
     copy_activations<MB>(p, fl, unit, ring + kWaveA);
   }
   if (mine > 1) copy_weights<MB, GPU>(p, fl, strip, unit + kFastWaves, ring + kSlotBytes, lane, unit_group_shift);
-  int c_slot = 0;
 
   floatx4_t acc[MB][4];
 #pragma unroll
@@ -983,103 +924,129 @@ __global__ __launch_bounds__(kFastWaves * 64) void marlin_stream_fast_kernel(con
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[mb][j] = floatx4_t{0.f, 0.f, 0.f, 0.f};
 
-  for (int left = mine; left > 0; --left) {
-    // One unit: wait for its copies, pull them into registers, start the
-    // copies of the units after it, then do the arithmetic.
-    const uint32_t slot_lds = ring_lds + c_slot * kSlotBytes;
-    u32x4_t q0, q1, q2, q3, a0, a1, a2, a3;
-    u32x4_t b0 = u32x4_t{0u, 0u, 0u, 0u}, b1 = b0, b2 = b0, b3 = b0;  // second block of rows
-    uint32_t row_s[16];
-    u32x4_t row_z = u32x4_t{0u, 0u, 0u, 0u};
-    uint32_t more_s[GPU > 1 ? GPU - 1 : 1][16];   // the other groups of the unit
-    u32x4_t more_z[GPU > 1 ? GPU - 1 : 1];
-    if (left > 1) {
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kWeightCopies) : "memory");
-    } else {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    }
-    {
-      const uint32_t q_at = slot_lds + lane * 16;
-      const uint32_t z_at = slot_lds + row_z_off, s_at = slot_lds + row_s_off;
-      if (kVecScales && grouped) {   // bfloat16: the float bits of a scale are a byte permute of its word
-        const uint32_t sv_at = slot_lds + kSlotS + 64 * (q4 & 1);
-        u32x4_t sv0, sv1, sv2, sv3;
-        SONAR_UNIT_READS_VEC();
-        const u32x4_t sv[4] = {sv0, sv1, sv2, sv3};
+  // Scales as they are read: in bf16 into the upper half of registers whose lower half stays zero, which makes them floats.
+  constexpr bool kBf16 = __is_same(T, __bf16);
+  constexpr bool kSurplus = kBf16 && !FP4;   // bf16 integers come as 128 + v
+  uint32_t sbits[GPU][4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+  for (int gi = 0; gi < GPU; ++gi)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) row_s[4 * j + r] = __builtin_amdgcn_perm(sv[r][j], 0u, scale_half);
-      } else if (grouped) {  // scale of (j, r) at byte 16 r + 4 j past s_at
-        SONAR_UNIT_READS(0, 16, 32, 48, 4, 20, 36, 52, 8, 24, 40, 56, 12, 28, 44, 60);
-      } else {        // at byte 64 (j >> 1) + 8 (j & 1) + 16 (r >> 1) + 2 (r & 1)
-        SONAR_UNIT_READS(0, 2, 16, 18, 8, 10, 24, 26, 64, 66, 80, 82, 72, 74, 88, 90);
-      }
-      if (kVecScales && !grouped) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) row_s[i] <<= 16;
-      }
-      if constexpr (MB == 2) SONAR_UNIT_READS_ROWS2(b0, b1, b2, b3);
-      if constexpr (GPU >= 2) SONAR_GROUP_READS(1);
-      if constexpr (GPU == 4) {
-        SONAR_GROUP_READS(2);
-        SONAR_GROUP_READS(3);
-      }
+    for (int j = 0; j < 4; ++j) {
+      sbits[gi][j] = 0;
+      asm("" : "+v"(sbits[gi][j]));
     }
-    if (left > 1) {
-      copy_activations<MB>(p, fl, unit + kFastWaves, ring + kWaveA);
-      if (left > 2)
-        copy_weights<MB, GPU>(p, fl, strip, unit + 2 * kFastWaves, ring + c_slot * kSlotBytes, lane,
-                              unit_group_shift);
-    }
-    unit += kFastWaves;
-    c_slot ^= 1;
 
-    const u32x4_t qs[4] = {q0, q1, q2, q3};
-    const u32x4_t as[2][4] = {{a0, a1, a2, a3}, {b0, b1, b2, b3}};
-    const floatx4_t zero4 = floatx4_t{0.f, 0.f, 0.f, 0.f};
-    floatx4_t part_sum[MB][4], asum[MB];
+  // One unit, in weight slot `slot`: wait for its copies, read its operands in the order of their use, start the copies of the
+  // units after it as soon as what they overwrite has been read, and multiply what has arrived meanwhile.
+  constexpr int kScaleReads = GPU * (HAS_ZP ? 5 : 4);
+  constexpr auto most = [](int n) { return n < 15 ? n : 15; };   // what lgkmcnt can say
+  auto work = [&](const int slot, const int left) __attribute__((always_inline)) {
+    u32x4_t a[MB][4], q[4];
+    uint32_t zbits[GPU];
+    if (left > 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kWeightCopies) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int cc = 0; cc < 4; ++cc)
+        asm volatile("ds_read_b128 %0, %1 offset:%2" : "=&v"(a[mb][cc]) : "v"(cc & 1 ? a_at ^ 64u : a_at), "i"(2048 * (cc >> 1) + 4096 * mb) : "memory");
+#pragma unroll
+    for (int cc = 0; cc < 4; ++cc)
+      asm volatile("ds_read_b128 %0, %1 offset:%2" : "=&v"(q[cc]) : "v"(q_at), "i"(slot * kSlotBytes + 1024 * cc) : "memory");
+#pragma unroll
+    for (int gi = 0; gi < GPU; ++gi) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if constexpr (kBf16)
+          asm volatile("ds_read_u16_d16_hi %0, %1 offset:%2" : "+v"(sbits[gi][j]) : "v"(s_at[j]), "i"(slot * kSlotBytes + 256 * gi) : "memory");
+        else
+          asm volatile("ds_read_u16 %0, %1 offset:%2" : "=&v"(sbits[gi][j]) : "v"(s_at[j]), "i"(slot * kSlotBytes + 256 * gi) : "memory");
+      }
+      if constexpr (HAS_ZP)
+        asm volatile("ds_read_b32 %0, %1 offset:%2" : "=&v"(zbits[gi]) : "v"(z_at), "i"(slot * kSlotBytes + 256 * gi) : "memory");
+    }
+    // the activations
+    asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(most(4 + kScaleReads)) : "memory");
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int cc = 0; cc < 4; ++cc) asm volatile("" : "+v"(a[mb][cc]));
+    if (left > 1) copy_activations<MB>(p, fl, unit + kFastWaves, ring + kWaveA);
     constexpr int kChunksPerGroup = 4 / GPU;
+    const floatx4_t zero4 = floatx4_t{0.f, 0.f, 0.f, 0.f};
+    floatx4_t a_sum[GPU][MB];
+    if constexpr (kSurplus) {
+#pragma unroll
+      for (int gi = 0; gi < GPU; ++gi)
+#pragma unroll
+        for (int cg = 0; cg < kChunksPerGroup; ++cg)
+#pragma unroll
+          for (int mb = 0; mb < MB; ++mb)
+            a_sum[gi][mb] = Dq<T>::mfma(__builtin_bit_cast(vec8, a[mb][gi * kChunksPerGroup + cg]), __builtin_bit_cast(vec8, ones),
+                                        cg == 0 ? zero4 : a_sum[gi][mb]);
+    }
+    // the codes, then scales and zero points: the slot is free
+    asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(most(kScaleReads)) : "memory");
+#pragma unroll
+    for (int cc = 0; cc < 4; ++cc) asm volatile("" : "+v"(q[cc]));
+    auto zero_point = [&](int gi, int j) __attribute__((always_inline)) -> uint32_t {
+      return HAS_ZP ? (zbits[gi] >> (z_shift + 4 * j)) & 0xFu : 8u;
+    };
+    auto unpack = [&](int cc, int j) __attribute__((always_inline)) {
+      const uint32_t word = j == 0 ? q[cc].x : j == 1 ? q[cc].y : j == 2 ? q[cc].z : q[cc].w;
+      if constexpr (FP4) return DqF4<T>::word(word, typename DqF4<T>::Col{1.0f}, magic);
+      else if constexpr (kBf16) return __builtin_bit_cast(vec8, raw_operand(word, magic));
+      else return exact_operand(word, zero_point(cc / kChunksPerGroup, j), magic);
+    };
+    vec8 first[4];   // chunk 0: unpacked while the scales and the sums of the activations are under way
+    if constexpr (!HAS_ZP || kBf16) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) first[j] = unpack(0, j);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int gi = 0; gi < GPU; ++gi) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) asm volatile("" : "+v"(sbits[gi][j]));
+      if constexpr (HAS_ZP) asm volatile("" : "+v"(zbits[gi]));
+    }
+    if (left > 2)
+      copy_weights<MB, GPU>(p, fl, strip, unit + 2 * kFastWaves, ring + slot * kSlotBytes, lane, unit_group_shift);
+    unit += kFastWaves;
+    floatx4_t sum[MB][4];
 #pragma unroll
     for (int gi = 0; gi < GPU; ++gi) {
 #pragma unroll
       for (int cg = 0; cg < kChunksPerGroup; ++cg) {
         const int cc = gi * kChunksPerGroup + cg;
-        const uint32_t words[4] = {qs[cc].x, qs[cc].y, qs[cc].z, qs[cc].w};
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          vec8 wv;
-          if constexpr (FP4) wv = DqF4<T>::word(words[j], typename DqF4<T>::Col{1.0f}, magic);
-          else wv = __builtin_bit_cast(vec8, raw_operand(words[j], magic));
+          const vec8 w = cc == 0 && (!HAS_ZP || kBf16) ? first[j] : unpack(cc, j);
+          if (cg == 0) {   // what the sums of the group start from
 #pragma unroll
-          for (int mb = 0; mb < MB; ++mb)
-            part_sum[mb][j] = Dq<T>::mfma(wv, __builtin_bit_cast(vec8, as[mb][cc]), cg == 0 ? zero4 : part_sum[mb][j]);
-        }
-        if constexpr (!FP4) {
+            for (int mb = 0; mb < MB; ++mb) {
+              if constexpr (kSurplus) sum[mb][j] = a_sum[gi][mb] * -(RawOperand<T>::kBase + (float)zero_point(gi, j));
+              else sum[mb][j] = zero4;
+            }
+          }
 #pragma unroll
-          for (int mb = 0; mb < MB; ++mb)
-            asum[mb] = Dq<T>::mfma(__builtin_bit_cast(vec8, ones), __builtin_bit_cast(vec8, as[mb][cc]),
-                                   cg == 0 ? zero4 : asum[mb]);
+          for (int mb = 0; mb < MB; ++mb) sum[mb][j] = Dq<T>::mfma(__builtin_bit_cast(vec8, a[mb][cc]), w, sum[mb][j]);
         }
       }
-      // scale and offset of this group (the whole unit when GPU == 1)
-      const u32x4_t gz = gi == 0 ? row_z : more_z[gi == 0 ? 0 : gi - 1];
-      const uint32_t zrow[4] = {gz.x >> row_z_shift, gz.y >> row_z_shift, gz.z >> row_z_shift, gz.w >> row_z_shift};
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+      for (int j = 0; j < 4; ++j) {
+        const float sc = kBf16 ? __uint_as_float(sbits[gi][j]) : Dq<T>::to_float((uint16_t)sbits[gi][j]);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const uint32_t sbits = gi == 0 ? row_s[4 * j + r] : more_s[gi == 0 ? 0 : gi - 1][4 * j + r];
-          const float sc = (kVecScales && gi == 0) ? __uint_as_float(sbits) : Dq<T>::to_float((uint16_t)sbits);
-          float off = -(RawOperand<T>::kBase + 8.f);
-          if (HAS_ZP) off = -RawOperand<T>::kBase - (float)((zrow[r] >> (4 * j)) & 0xFu);
+        for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-          for (int mb = 0; mb < MB; ++mb) {
-            if constexpr (FP4) acc[mb][j][r] = __builtin_fmaf(sc, part_sum[mb][j][r], acc[mb][j][r]);
-            else acc[mb][j][r] = __builtin_fmaf(sc, __builtin_fmaf(off, asum[mb][r], part_sum[mb][j][r]), acc[mb][j][r]);
-          }
-        }
+          for (int r = 0; r < 4; ++r) acc[mb][j][r] = __builtin_fmaf(sc, sum[mb][j][r], acc[mb][j][r]);
+      }
     }
+  };
+  for (int left = mine; left > 0; left -= 2) {   // two units a pass, so that the slots are constants
+    work(0, left);
+    if (left == 1) break;
+    work(1, left - 1);
   }
 
   // The cross-wavefront sum: in each pass every wavefront parks kPark of its tiles in
@@ -1141,13 +1108,14 @@ __global__ __launch_bounds__(kFastWaves * 64) void marlin_stream_fast_kernel(con
         sum += t2;
         sum += t3;
       }
-      const int j = jb + wave;
+      const int j = jb + wave, at = quad_lane(lane);
+      sum = quad_transpose(sum, lane);
       if constexpr (GROUPED) {
-        finish_block_grouped<T>(p, row_id[mb], strip, lane, j, sum);
+        finish_block_grouped<T>(p, row_id[mb], strip, at, j, sum);
       } else if (pieces == 1) {
-        store_c_block<T>(p, p.c + (long)(16 * mb) * p.size_n, p.size_m - 16 * mb, strip, lane, j, sum);
+        store_c_block<T>(p, p.c + (long)(16 * mb) * p.size_n, p.size_m - 16 * mb, strip, at, j, sum);
       } else {
-        store_partial_block(p, part, first, (slab * MB + mb) * 4 + j, lane, sum);
+        store_partial_block(p, part, first, (slab * MB + mb) * 4 + j, at, sum);
       }
     }
   }
@@ -1189,9 +1157,6 @@ __global__ __launch_bounds__(kFastWaves * 64) void marlin_stream_fast_kernel(con
     }
   }
 }
-#undef SONAR_UNIT_READS_VEC
-#undef SONAR_UNIT_READS_ROWS2
-#undef SONAR_GROUP_READS
 
 // ---------------------------------------------------------------------------
 // Second pass over the strips that were split between workgroups: adds the
