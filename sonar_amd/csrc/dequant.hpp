@@ -384,13 +384,18 @@ struct Dq8<_Float16> {
     return Col{half2_t{s, s}};
   }
   static __device__ __forceinline__ uint2 word4(uint32_t q, const Col& c, uint32_t magic) {
-    const half2_t off = half2_t{(_Float16)1152.f, (_Float16)1152.f};
-    const uint32_t lo = and_or(q, 0x00ff00ffu, magic);
-    const uint32_t hi = and_or(q >> 8, 0x00ff00ffu, magic);
-    const half2_t w0 = (__builtin_bit_cast(half2_t, lo) - off) * c.s;
-    const half2_t w1 = (__builtin_bit_cast(half2_t, hi) - off) * c.s;
-    return make_uint2(__builtin_bit_cast(uint32_t, w0), __builtin_bit_cast(uint32_t, w1));
+    return make_uint2(stage3(stage2(stage1(q, 0, magic), c), c), stage3(stage2(stage1(q, 1, magic), c), c));
   }
+  // word4() a few instructions at a time, for kernels that place them themselves: register `part` (0, 1) of it is
+  // stage3(stage2(stage1(q, part, magic), c), c)
+  typedef half2_t Mid;
+  static __device__ __forceinline__ uint32_t stage1(uint32_t q, int part, uint32_t magic) {
+    return and_or(part ? q >> 8 : q, 0x00ff00ffu, magic);
+  }
+  static __device__ __forceinline__ Mid stage2(uint32_t x, const Col&) {
+    return __builtin_bit_cast(half2_t, x) - half2_t{(_Float16)1152.f, (_Float16)1152.f};
+  }
+  static __device__ __forceinline__ uint32_t stage3(Mid y, const Col& c) { return __builtin_bit_cast(uint32_t, y * c.s); }
 };
 
 template <>
@@ -405,12 +410,19 @@ struct Dq8<__bf16> {
     return c;
   }
   static __device__ __forceinline__ uint2 word4(uint32_t q, const Col& c, uint32_t magic) {
-    const uint32_t lo = and_or(q, 0x00ff00ffu, magic);
-    const uint32_t hi = and_or(q >> 8, 0x00ff00ffu, magic);
-    // (1024 + v) * s - 1152 s: both products and their sum are exact in fp32
-    const bf16x2_t w0 = Dq<__bf16>::pair(lo, c.s, c.c0);
-    const bf16x2_t w1 = Dq<__bf16>::pair(hi, c.s, c.c0);
-    return make_uint2(__builtin_bit_cast(uint32_t, w0), __builtin_bit_cast(uint32_t, w1));
+    return make_uint2(stage3(stage2(stage1(q, 0, magic), c), c), stage3(stage2(stage1(q, 1, magic), c), c));
+  }
+  typedef floatx2_t Mid;
+  static __device__ __forceinline__ uint32_t stage1(uint32_t q, int part, uint32_t magic) {
+    return and_or(part ? q >> 8 : q, 0x00ff00ffu, magic);
+  }
+  // (1024 + v) * s - 1152 s: both products and their sum are exact in fp32
+  static __device__ __forceinline__ Mid stage2(uint32_t x, const Col& c) {
+    const half2_t h = __builtin_bit_cast(half2_t, x);
+    return floatx2_t{__builtin_fmaf((float)h.x, c.s, c.c0), __builtin_fmaf((float)h.y, c.s, c.c0)};
+  }
+  static __device__ __forceinline__ uint32_t stage3(Mid y, const Col&) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(y, bf16x2_t));
   }
 };
 
@@ -436,11 +448,13 @@ template <>
 struct Dq8F<_Float16> {
   typedef Dq8<_Float16>::Col Col;
   static __device__ __forceinline__ Col make_col(uint16_t scale_bits) { return Dq8<_Float16>::make_col(scale_bits); }
-  static __device__ __forceinline__ uint2 word4(uint32_t q, const Col& c, uint32_t) {
-    const half2_t w0 = __builtin_bit_cast(half2_t, fp8_pair_as_fp16(q << 8)) * c.s;
-    const half2_t w1 = __builtin_bit_cast(half2_t, fp8_pair_as_fp16(q)) * c.s;
-    return make_uint2(__builtin_bit_cast(uint32_t, w0), __builtin_bit_cast(uint32_t, w1));
+  static __device__ __forceinline__ uint2 word4(uint32_t q, const Col& c, uint32_t magic) {
+    return make_uint2(stage3(stage2(stage1(q, 0, magic), c), c), stage3(stage2(stage1(q, 1, magic), c), c));
   }
+  typedef half2_t Mid;
+  static __device__ __forceinline__ uint32_t stage1(uint32_t q, int part, uint32_t) { return part ? q : q << 8; }
+  static __device__ __forceinline__ Mid stage2(uint32_t x, const Col&) { return __builtin_bit_cast(half2_t, fp8_pair_as_fp16(x)); }
+  static __device__ __forceinline__ uint32_t stage3(Mid y, const Col& c) { return __builtin_bit_cast(uint32_t, y * c.s); }
 };
 
 template <>
@@ -451,14 +465,17 @@ struct Dq8F<__bf16> {
   static __device__ __forceinline__ Col make_col(uint16_t scale_bits) {
     return Col{__builtin_bit_cast(float, (uint32_t)scale_bits << 16) * 0x1p-112f};
   }
-  static __device__ __forceinline__ bf16x2_t scaled(uint32_t fp16_pair, float s) {
-    const half2_t h = __builtin_bit_cast(half2_t, fp16_pair);
-    return __builtin_convertvector(floatx2_t{(float)h.x * s, (float)h.y * s}, bf16x2_t);
+  static __device__ __forceinline__ uint2 word4(uint32_t q, const Col& c, uint32_t magic) {
+    return make_uint2(stage3(stage2(stage1(q, 0, magic), c), c), stage3(stage2(stage1(q, 1, magic), c), c));
   }
-  static __device__ __forceinline__ uint2 word4(uint32_t q, const Col& c, uint32_t) {
-    const bf16x2_t w0 = scaled(fp8_pair_as_fp16(q << 8), c.s);
-    const bf16x2_t w1 = scaled(fp8_pair_as_fp16(q), c.s);
-    return make_uint2(__builtin_bit_cast(uint32_t, w0), __builtin_bit_cast(uint32_t, w1));
+  typedef floatx2_t Mid;
+  static __device__ __forceinline__ uint32_t stage1(uint32_t q, int part, uint32_t) { return fp8_pair_as_fp16(part ? q : q << 8); }
+  static __device__ __forceinline__ Mid stage2(uint32_t x, const Col& c) {
+    const half2_t h = __builtin_bit_cast(half2_t, x);
+    return floatx2_t{(float)h.x * c.s, (float)h.y * c.s};
+  }
+  static __device__ __forceinline__ uint32_t stage3(Mid y, const Col&) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(y, bf16x2_t));
   }
 };
 

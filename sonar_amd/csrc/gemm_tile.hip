@@ -1184,18 +1184,26 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
       if (rb == 0 && (B == 0 || G32)) scales_start(kt + 1, B);
       const uint32_t qw = word_of(q4, j);
       if constexpr (W8 != 0) {
-        // behind every second row block, half a column block (four rows of 16 columns) in one piece
+        // a register of half a column block (two of four rows of 16 columns; with 8 row blocks: both), spread over three
+        // matrix instructions.  (Half a column block in one piece behind every second row block, 14 instructions behind
+        // one that hides four: fp8, bf16, M = 2000, K = 2944, N = 8832 167 -> 133 us; M = 1323, K = N = 8832 235 -> 203; MXFP8,
+        // M = 3000, K = 2944, N = 6144 168 -> 150; uint8b128, M = 1000, K = 4096, N = 6144 68 -> 58.)
+        const int piece = RB == 8 ? rb : rb >> 1, jj = piece >> 1, half = piece & 1, first = RB == 8 ? 0 : rb & 1;
+        const uint32_t w8 = word_of(half ? q4h : q4, jj);
         mfma(B, 0, rb);
-        if (RB == 8 || (rb & 1) == 0) {   // (with 8 row blocks: behind every row block)
-          const int piece = RB == 8 ? rb : rb >> 1;
-          const int jj = piece >> 1, half = piece & 1;
-          const uint2 w = D8::word4(word_of(half ? q4h : q4, jj), cols[set][jj], magic);
-          wb[NB][jj][2 * half] = w.x;
-          wb[NB][jj][2 * half + 1] = w.y;
-        }
+        const uint32_t x = D8::stage1(w8, first, magic);
+        uint32_t x2 = 0;
+        if (RB == 8) x2 = D8::stage1(w8, 1, magic);
         __builtin_amdgcn_sched_barrier(0);
         mfma(B, 1, rb);
+        const typename D8::Mid y = D8::stage2(x, cols[set][jj]);
+        typename D8::Mid y2 = y;
+        if (RB == 8) y2 = D8::stage2(x2, cols[set][jj]);
+        __builtin_amdgcn_sched_barrier(0);
         mfma(B, 2, rb);
+        wb[NB][jj][2 * half + first] = D8::stage3(y, cols[set][jj]);
+        if (RB == 8) wb[NB][jj][2 * half + 1] = D8::stage3(y2, cols[set][jj]);
+        __builtin_amdgcn_sched_barrier(0);
         mfma(B, 3, rb);
       } else if constexpr (NV && std::is_same<T, _Float16>::value) {
         // the pair of codes read as fp16 numbers (value * 2^-14) times scale * 2^14 in one packed multiply
