@@ -1373,15 +1373,21 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
   for (int rb = 0; rb < kAhead; ++rb) SONAR_WIDE_READ(av[rb], a_base[0], rb * 2048);
   __builtin_amdgcn_sched_barrier(0);
 
-  for (int kt = k_first;; kt += 4) {
+  // Whole passes without a branch between their steps, then up to three steps.  (With a branch behind every step: int4, M = 8192,
+  // K = 4096, N = 28672 1520 us against 1498, M = 4000, K = 1152, N = 6144 71 against 64.)
+  int kt = k_first;
+  for (; kt + 4 <= k_tiles; kt += 4) {
     step(0, kt);
-    if (kt + 1 >= k_tiles) break;
     step(1, kt + 1);
-    if (kt + 2 >= k_tiles) break;
     step(2, kt + 2);
-    if (kt + 3 >= k_tiles) break;
     step(3, kt + 3);
-    if (kt + 4 >= k_tiles) break;
+  }
+  if (kt < k_tiles) {
+    step(0, kt);
+    if (kt + 1 < k_tiles) {
+      step(1, kt + 1);
+      if (kt + 2 < k_tiles) step(2, kt + 2);
+    }
   }
   // nothing in flight may outlive the wavefront (the copies of the steps past the end, the two
   // operand reads of the last half step), and the matrix pipeline drains before the results are read
