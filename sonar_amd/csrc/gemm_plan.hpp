@@ -96,6 +96,24 @@ inline bool plan_prefers_128_rows(int64_t size_m, int64_t size_n, int64_t size_k
   return tiles256 <= (size_k <= 8192 ? 128 : 32);
 }
 
+// Microseconds the tile kernels take: rounds of workgroups, each 11.2 us around its loop and `step` us per 64 rows of K for a
+// 256-row tile (0.58 of both for a 128-row one), 3.3 us for the launch, and for K in ranges a second launch and its bytes.  A fit
+// of 168 random calls of 220 to 8192 rows in all formats: 90 % within 14 % below and 13 % above.  `rows128`: the call's
+// format has 128-row tiles.
+inline double tile_estimate(int64_t size_m, int64_t size_n, int64_t size_k, double step, bool rows128) {
+  const bool small = rows128 && plan_prefers_128_rows(size_m, size_n, size_k);
+  const int64_t rows = small ? 128 : 256, steps = size_k / 64, tiles = ((size_m + rows - 1) / rows) * ((size_n + 255) / 256);
+  const GemmPlan plan = plan_gemm(size_m, size_n, size_k, true, (int)rows);
+  const double unit = small ? 0.58 : 1.0, whole = unit * (step * steps + 11.2);
+  const double range = unit * (step * plan.k_steps_per_split + 11.2), sum = 1.1 + 1.24e-6 * plan.k_splits * size_m * size_n;
+  if (plan.k_splits > 1 && plan.whole_tiles == 0) return 3.3 + (tiles * plan.k_splits + 255) / 256 * range + sum;
+  const int64_t last = tiles % 256;
+  double us = 3.3 + tiles / 256 * whole;
+  if (last > 128 || (last > 0 && plan.k_splits < 3 && (tiles < 256 || !rows128))) us += whole;
+  else if (last > 0) us += plan.k_splits >= 3 ? range + 1.1 : 0.58 * whole;
+  return us;
+}
+
 // Scratch for the partial tiles of either tiling.
 inline size_t plan_partial_bytes_any(int64_t size_m, int64_t size_n, int64_t size_k) {
   const bool r = plan_rows_97_128(size_m, size_n, size_k, true);

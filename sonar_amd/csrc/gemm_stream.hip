@@ -1888,9 +1888,13 @@ int marlin_gemm_any(const void* a, int64_t a_row_stride, void* c, const uint32_t
     if (slab_fast) {
       us = decode_rows_estimate(size_m, n_strips, size_k, chk.has_zp, cus);
     } else if (use_tile) {
-      // us per 1e9 operations of the wide kernel on 4-bit codes and on others
-      const double rate = chk.bits == 8 ? 1.05 : chk.fp4 ? 0.78 : 0.72;
-      us = 25.0 + rate * 2e-9 * ((size_m + 127) / 128 * 128) * size_n * size_k;
+      const double step = chk.bits == 8 ? 1.27 : chk.nvfp4 ? 1.30 : chk.fp4 ? 1.14 : 1.21;
+      us = tile_estimate(size_m, size_n, size_k, step, !chk.nvfp4 && !(chk.bits == 8 && num_groups > 1 && chk.group_size == 32));
+      // what mid_estimate lacks, with K in one piece, on the calls tile_estimate was fitted to (a time that grows with the operations alone, and 0.93 for
+      // either kernel: 2.7 % slower than the better of the two on 147 random calls, at worst 1.6 times; so 0.6 %, 1.3 times)
+      static const double kSlow[6][2] = {{1.12, 1.10}, {1.18, 1.10}, {1.30, 1.12}, {1.13, 1.05}, {1.22, 1.22}, {1.03, 1.0}};
+      if (splits > 1) mid_us *= 0.94;
+      else mid_us *= format == kMidFp8 && num_groups > 1 && chk.group_size == 32 ? 0.97 : kSlow[format][dtype == SONAR_DTYPE_F16 ? 0 : 1];
     } else {   // (few strips: shared between workgroups, and a second launch that adds the shares)
       us = size_m <= 64 ? (n_strips < 64 ? 12.0 : 9.5) + x * (5.5 + 5.2 * r * r) : 11.0 + 10.7 * x * r;
     }
@@ -1900,7 +1904,7 @@ int marlin_gemm_any(const void* a, int64_t a_row_stride, void* c, const uint32_t
       splits = comma ? std::max(1, std::min(kMidMostSplits, atoi(comma + 1))) : 1;
       if ((size_t)splits * size_m * size_n * 4 > base_scratch || splits > size_k / 64) splits = 1;
     }
-    if (mid_env || mid_us < (raw_codes ? 1.0 : 0.93) * us) {
+    if (mid_env || mid_us < (raw_codes || use_tile ? 1.0 : 0.93) * us) {
       MidParams q = {};
       q.a = static_cast<const uint16_t*>(a);
       q.lda = a_row_stride;
