@@ -125,6 +125,15 @@ int sonar_awq_marlin_moe_repack(const uint32_t* b_q_weight, uint32_t* out, int64
  * marlin_permute_scales (grouped != 0: 64-column pattern; 0: the 32-column pattern of one group and
  * of marlin_permute_bias) on 16-bit elements (`out` 16-byte aligned), aphrodite quantization/utils/marlin_utils.py:404-434. */
 int sonar_marlin_permute_scales(const void* in, void* out, int64_t numel, int grouped, void* stream);
+
+/* sonar_gptq_marlin_repack (4-bit codes, no act-order), sonar_marlin_permute_scales of the
+ * (groups, size_n) scales, sonar_marlin_pack_zero_points of zero points in plain order ((groups,
+ * size_n / 8), or with zeros_transposed its transpose; NULL: none) and a workspace of zeros, as one
+ * launch. */
+int sonar_load_gptq_linear(const uint32_t* codes, uint32_t* codes_out, const void* scales, void* scales_out,
+                           const uint32_t* zeros, uint32_t* zeros_out, uint32_t* workspace,
+                           int64_t workspace_words, int64_t size_k, int64_t size_n, int64_t groups,
+                           int grouped, int zeros_transposed, void* stream);
 /* Zero points packed along N, eight to a word, in plain or AWQ nibble order -> (rows, N/8) words in the
  * order the GEMM reads (marlin_utils.py:457-559: marlin_zero_points, awq_to_marlin_zero_points);
  * in[row * row_stride + word * word_stride]. */

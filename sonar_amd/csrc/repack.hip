@@ -52,13 +52,12 @@ __device__ __forceinline__ uint32_t interleave_nibbles(uint32_t b0, uint32_t b1,
 // With HAS_PERM (act-order) the sixteen rows of a tile come from sixteen words of different rows: a
 // half wavefront reads each as 256 bytes and leaves the selected nibbles in LDS in the source's own packing.
 template <bool HAS_PERM>
-__global__ __launch_bounds__(256) void gptq_to_marlin_kernel(
-    const uint32_t* __restrict__ in, const int32_t* __restrict__ perm, uint32_t* __restrict__ out, int size_k,
-    int size_n, uint32_t tiles_each, long in_each, uint32_t total_tiles) {
-  __shared__ alignas(16) uint32_t lds[kRepackTiles * kRepackLdsStride];
+__device__ __forceinline__ void gptq_tiles(uint32_t* lds, const uint32_t block, const uint32_t* __restrict__ in,
+                                           const int32_t* __restrict__ perm, uint32_t* __restrict__ out, int size_k,
+                                           int size_n, uint32_t tiles_each, long in_each, uint32_t total_tiles) {
   const uint32_t n_tiles = size_n / kMarlinTileN;
   const int sub = threadIdx.x >> 5, l = threadIdx.x & 31;
-  const uint32_t tile = blockIdx.x * kRepackTiles + sub;
+  const uint32_t tile = block * kRepackTiles + sub;
   const bool live = tile < total_tiles;
   uint32_t* mine = lds + sub * kRepackLdsStride;
   if (live) {
@@ -94,6 +93,13 @@ __global__ __launch_bounds__(256) void gptq_to_marlin_kernel(
                               (w[8] >> (8 * h)) & 0xFFu, (w[kMarlinTileN + 8] >> (8 * h)) & 0xFFu);
   }
   *reinterpret_cast<words4_t*>(out + (long)tile * kMarlinTileWords + 4 * l) = o;
+}
+template <bool HAS_PERM>
+__global__ __launch_bounds__(256) void gptq_to_marlin_kernel(
+    const uint32_t* __restrict__ in, const int32_t* __restrict__ perm, uint32_t* __restrict__ out, int size_k,
+    int size_n, uint32_t tiles_each, long in_each, uint32_t total_tiles) {
+  __shared__ alignas(16) uint32_t lds[kRepackTiles * kRepackLdsStride];
+  gptq_tiles<HAS_PERM>(lds, blockIdx.x, in, perm, out, size_k, size_n, tiles_each, in_each, total_tiles);
 }
 
 __global__ __launch_bounds__(256) void awq_to_marlin_kernel(
@@ -425,10 +431,8 @@ __global__ __launch_bounds__(256) void int4_fp8_preprocess_kernel(const uint32_t
 // out[8 i + j] = in[2 i + {0, 1, 8, 9, 16, 17, 24, 25}[j]] (one group, bias).  A thread stores 16
 // bytes; its loads stay inside one 128-byte line.
 template <bool GROUPS>
-__global__ __launch_bounds__(256) void permute_scale_columns(const uint16_t* __restrict__ in,
-                                                             uint16_t* __restrict__ out, long vectors) {
-  const long v = (long)blockIdx.x * 256 + threadIdx.x;
-  if (v >= vectors) return;
+__device__ __forceinline__ void permute_scale_vector(const uint16_t* __restrict__ in, uint16_t* __restrict__ out,
+                                                     const long v) {
   uint32_t o[4];
   if constexpr (GROUPS) {
     const uint16_t* src = in + (v >> 3) * 64 + (v & 7);
@@ -441,16 +445,19 @@ __global__ __launch_bounds__(256) void permute_scale_columns(const uint16_t* __r
   }
   *reinterpret_cast<uint4*>(out + 8 * v) = make_uint4(o[0], o[1], o[2], o[3]);
 }
+template <bool GROUPS>
+__global__ __launch_bounds__(256) void permute_scale_columns(const uint16_t* __restrict__ in,
+                                                             uint16_t* __restrict__ out, long vectors) {
+  const long v = (long)blockIdx.x * 256 + threadIdx.x;
+  if (v < vectors) permute_scale_vector<GROUPS>(in, out, v);
+}
 
 // Packed zero points -> Marlin zero points, (rows, N/8) words.  Nibble e of output word w is the code
 // of column 64 (w / 8) + w % 8 + 8 * i(e), i = {0, 2, 4, 6, 1, 3, 5, 7} (the column interleave of the
 // 16-bit dequantiser; the identity for 8-bit activations), i.e. always nibble w % 8 of a source word,
 // or nibble (w % 8) / 2 + 4 (w % 2) where the source has the AWQ order.
-__global__ __launch_bounds__(256) void pack_zero_points(const uint32_t* __restrict__ in, uint32_t* __restrict__ out,
-                                                        int words, long total, long row_stride, long word_stride,
-                                                        bool awq_order, bool a8) {
-  const long idx = (long)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= total) return;
+__device__ __forceinline__ void pack_zero_word(const uint32_t* __restrict__ in, uint32_t* __restrict__ out, const long idx,
+                                               int words, long row_stride, long word_stride, bool awq_order, bool a8) {
   const long row = idx / words;
   const int w = (int)(idx - row * words);
   const int shift = 4 * (awq_order ? ((w & 7) >> 1) + 4 * (w & 1) : w & 7);
@@ -462,6 +469,58 @@ __global__ __launch_bounds__(256) void pack_zero_points(const uint32_t* __restri
     packed |= ((src[from * word_stride] >> shift) & 0xFu) << (4 * e);
   }
   out[idx] = packed;
+}
+__global__ __launch_bounds__(256) void pack_zero_points(const uint32_t* __restrict__ in, uint32_t* __restrict__ out,
+                                                        int words, long total, long row_stride, long word_stride,
+                                                        bool awq_order, bool a8) {
+  const long idx = (long)blockIdx.x * 256 + threadIdx.x;
+  if (idx < total) pack_zero_word(in, out, idx, words, row_stride, word_stride, awq_order, a8);
+}
+
+// A GPTQ-like projection as one launch: codes, scales, zero points (when it has any) and the tickets of its workspace, which
+// start at zero.  A workgroup's number says which of the four it works on; each is the body of the kernel that does it
+// alone.  Up to about 40 MB of codes a load is bound by the host, which made three or four operator calls with a launch
+// each; one call takes 4096x4096 from 31 us to 18 (a copy of its bytes: 3), the same with AWQ's conversion before it from
+// 46 to 27, and 14336x28672, where the three launches followed one another, from 76 to 71 (its bytes: 82 at the rate of a
+// large copy, part of them in the memory-side cache).
+struct LoadLinear {
+  const uint32_t* codes;
+  uint32_t* codes_out;
+  int size_k, size_n;
+  uint32_t tiles, code_blocks;
+  const uint16_t* scales;
+  uint16_t* scales_out;
+  long vectors;
+  uint32_t scale_blocks;
+  const uint32_t* zeros;
+  uint32_t* zeros_out;
+  long zero_words, zero_row_stride, zero_word_stride;
+  uint32_t zero_blocks;
+  uint32_t* workspace;
+  int workspace_words;
+};
+template <bool GROUPS>
+__global__ __launch_bounds__(256) void load_linear_kernel(const LoadLinear p) {
+  __shared__ alignas(16) uint32_t lds[kRepackTiles * kRepackLdsStride];
+  uint32_t block = blockIdx.x;
+  if (block < p.code_blocks) {
+    gptq_tiles<false>(lds, block, p.codes, nullptr, p.codes_out, p.size_k, p.size_n, p.tiles, 0, p.tiles);
+    return;
+  }
+  block -= p.code_blocks;
+  if (block < p.scale_blocks) {
+    const long v = (long)block * 256 + threadIdx.x;
+    if (v < p.vectors) permute_scale_vector<GROUPS>(p.scales, p.scales_out, v);
+    return;
+  }
+  block -= p.scale_blocks;
+  if (block < p.zero_blocks) {
+    const long w = (long)block * 256 + threadIdx.x;
+    if (w < p.zero_words)
+      pack_zero_word(p.zeros, p.zeros_out, w, p.size_n / 8, p.zero_row_stride, p.zero_word_stride, false, false);
+    return;
+  }
+  for (int i = threadIdx.x; i < p.workspace_words; i += 256) p.workspace[i] = 0;
 }
 
 // AutoAWQ codes (K, N/8) -> the GPTQ packing (K/8, N): a thread transposes the 8 x 8 nibbles of eight
@@ -760,6 +819,48 @@ extern "C" int sonar_marlin_pack_zero_points(const uint32_t* in, uint32_t* out, 
   pack_zero_points<<<blocks_of(total), 256, 0, (hipStream_t)stream>>>(in, out, (int)(size_n / 8), total, row_stride,
                                                                      word_stride, awq_order != 0, is_a_8bit != 0);
   return launch_status("pack_zero_points");
+}
+
+extern "C" int sonar_load_gptq_linear(const uint32_t* codes, uint32_t* codes_out, const void* scales, void* scales_out,
+                                      const uint32_t* zeros, uint32_t* zeros_out, uint32_t* workspace,
+                                      int64_t workspace_words, int64_t size_k, int64_t size_n, int64_t groups, int grouped,
+                                      int zeros_transposed, void* stream) {
+  if (int rc = check_repack_shape(size_k, size_n, 4)) return rc;
+  if (int rc = check_experts(1, size_k, size_n)) return rc;
+  SONAR_REQUIRE(groups >= 1 && groups * size_n < (1LL << 38), "num_groups = %ld out of range", (long)groups);
+  SONAR_REQUIRE(codes && codes_out && codes != codes_out && scales && scales_out && scales != scales_out,
+                "codes, scales and their outputs must be distinct non-NULL buffers");
+  SONAR_REQUIRE((zeros == nullptr) == (zeros_out == nullptr) && (zeros == nullptr || zeros != zeros_out),
+                "zero points and their output must be given together, as distinct buffers");
+  SONAR_REQUIRE(workspace_words >= 0 && workspace_words < (1LL << 20) && (workspace || workspace_words == 0),
+                "workspace of %ld words is out of range", (long)workspace_words);
+  SONAR_REQUIRE((uintptr_t)scales_out % 16 == 0, "out must be 16-byte aligned");
+  LoadLinear p = {};
+  p.codes = codes;
+  p.codes_out = codes_out;
+  p.size_k = (int)size_k;
+  p.size_n = (int)size_n;
+  p.tiles = (uint32_t)((size_k / kMarlinTileK) * (size_n / kMarlinTileN));
+  p.code_blocks = (p.tiles + kRepackTiles - 1) / kRepackTiles;
+  p.scales = static_cast<const uint16_t*>(scales);
+  p.scales_out = static_cast<uint16_t*>(scales_out);
+  p.vectors = groups * size_n / 8;
+  p.scale_blocks = (uint32_t)((p.vectors + 255) / 256);
+  if (zeros) {
+    p.zeros = zeros;
+    p.zeros_out = zeros_out;
+    p.zero_words = groups * (size_n / 8);
+    p.zero_row_stride = zeros_transposed ? 1 : size_n / 8;
+    p.zero_word_stride = zeros_transposed ? groups : 1;
+    p.zero_blocks = (uint32_t)((p.zero_words + 255) / 256);
+  }
+  p.workspace = workspace;
+  p.workspace_words = (int)workspace_words;
+  const int64_t blocks = (int64_t)p.code_blocks + p.scale_blocks + p.zero_blocks + (workspace_words > 0);
+  SONAR_REQUIRE(blocks < (1LL << 31), "weight too large");
+  auto* kernel = grouped ? load_linear_kernel<true> : load_linear_kernel<false>;
+  kernel<<<(int)blocks, 256, 0, (hipStream_t)stream>>>(p);
+  return launch_status("load_linear_kernel");
 }
 
 extern "C" int sonar_awq_to_gptq(const uint32_t* in, uint32_t* out, int64_t size_k, int64_t size_n, void* stream) {

@@ -434,6 +434,38 @@ Tensor pack_zero_points(const Tensor& zp, bool awq_order, bool transposed, bool 
   return out;
 }
 
+// The tensors of a 4-bit GPTQ-like projection ((K/8, N) codes, (G, N) 16-bit scales, zero points (G, N/8) or (N/8, G) packed
+// along N, or none) -> what the GEMM takes, and a workspace of zeros: (codes, scales, zero points, workspace).
+std::tuple<Tensor, Tensor, Tensor, Tensor> load_gptq_linear(const Tensor& qweight, const Tensor& scales, const OptTensor& zeros,
+                                                            bool grouped, bool transposed) {
+  TORCH_CHECK(qweight.is_cuda() && qweight.is_contiguous() && qweight.scalar_type() == at::kInt && qweight.dim() == 2,
+              "qweight must be a contiguous two-dimensional int32 GPU tensor");
+  const int64_t size_k = qweight.size(0) * 8, size_n = qweight.size(1);
+  TORCH_CHECK(scales.is_cuda() && scales.is_contiguous() && scales.element_size() == 2 && scales.dim() == 2 &&
+                  scales.size(1) == size_n && scales.size(0) >= 1 && scales.device() == qweight.device(),
+              "scales must be a contiguous 16-bit (groups, N) tensor on the GPU of qweight");
+  const int64_t groups = scales.size(0);
+  if (zeros.has_value())
+    TORCH_CHECK(zeros->is_cuda() && zeros->is_contiguous() && zeros->scalar_type() == at::kInt && zeros->dim() == 2 &&
+                    zeros->size(transposed ? 1 : 0) == groups && zeros->size(transposed ? 0 : 1) == size_n / 8 &&
+                    zeros->device() == qweight.device(),
+                "zero points must be a contiguous int32 tensor, packed along N, on the GPU of qweight");
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(qweight.device());
+  Tensor codes_out = at::empty({size_k / 16, size_n * 2}, qweight.options());
+  Tensor scales_out = at::empty_like(scales);
+  Tensor zeros_out = at::empty({zeros.has_value() ? groups : 0, size_n / 8}, qweight.options());
+  Tensor workspace = at::empty({at::cuda::getCurrentDeviceProperties()->multiProcessorCount}, qweight.options());
+  raise_if_failed(sonar_load_gptq_linear(
+      static_cast<const uint32_t*>(qweight.const_data_ptr()), static_cast<uint32_t*>(codes_out.mutable_data_ptr()),
+      scales.const_data_ptr(), scales_out.mutable_data_ptr(),
+      zeros.has_value() ? static_cast<const uint32_t*>(zeros->const_data_ptr()) : nullptr,
+      zeros.has_value() ? static_cast<uint32_t*>(zeros_out.mutable_data_ptr()) : nullptr,
+      static_cast<uint32_t*>(workspace.mutable_data_ptr()), workspace.numel(), size_k, size_n, groups, grouped ? 1 : 0,
+      transposed ? 1 : 0, current_stream(qweight)));
+  forget_memory_of(codes_out);
+  return {codes_out, scales_out, zeros_out, workspace};
+}
+
 // AutoAWQ codes and zero points -> the GPTQ-like packing: ((K/8, N), (N/8, G)).
 std::tuple<Tensor, Tensor> awq_to_standard(const Tensor& qweight, const Tensor& qzeros) {
   for (const Tensor* t : {&qweight, &qzeros})
@@ -1349,6 +1381,8 @@ TORCH_LIBRARY(sonar_amd, m) {
   m.def("permute_scales(Tensor s, bool grouped) -> Tensor");
   m.def("pack_zero_points(Tensor zp, bool awq_order, bool transposed, bool is_a_8bit) -> Tensor");
   m.def("awq_to_standard(Tensor qweight, Tensor qzeros) -> (Tensor, Tensor)");
+  m.def("load_gptq_linear(Tensor qweight, Tensor scales, Tensor? zeros, bool grouped, bool transposed) -> "
+        "(Tensor, Tensor, Tensor, Tensor)");
   m.def("per_token_quant_fp8(Tensor x) -> (Tensor, Tensor)");
 }
 TORCH_LIBRARY_IMPL(sonar_amd, CUDA, m) {
@@ -1369,6 +1403,7 @@ TORCH_LIBRARY_IMPL(sonar_amd, CUDA, m) {
   m.impl("permute_scales", &permute_scales);
   m.impl("pack_zero_points", &pack_zero_points);
   m.impl("awq_to_standard", &awq_to_standard);
+  m.impl("load_gptq_linear", &load_gptq_linear);
   m.impl("per_token_quant_fp8", &per_token_quant_fp8);
 }
 

@@ -135,7 +135,46 @@ class MarlinLinearKernel:
         zp = marlin_pad_scales(zp, size_n, size_k, padded_n, padded_k, c.group_size)
         return marlin_zero_points(zp, padded_grouped_k, padded_n, c.weight_type.size_bits, is_a_8bit=is_a_8bit)
 
+    def _load_in_one_launch(self, layer) -> bool:
+        """process_weights_after_loading for tensors already in the layout that the kernels of the general path read: 4-bit
+        codes (K/8, N), 16-bit scales (G, N), zero points packed along N, all contiguous on one GPU, no act-order, no
+        padding.  False: nothing was touched."""
+        c = self.config
+        size_k, size_n = c.partition_weight_shape
+        if (c.has_g_idx or c.weight_type.size_bits != 4 or c.act_type.itemsize != 2 or size_n % 64 or size_k % 128
+                or hasattr(self, "workspace")):
+            return False
+        w_q, w_s = getattr(layer, self.w_q_name), getattr(layer, self.w_s_name)
+        groups = 1 if c.group_size == -1 else size_k // c.group_size
+        if (groups < 1 or w_q.dtype != torch.int32 or w_q.shape != (size_k // 8, size_n) or w_s.shape != (groups, size_n)
+                or w_s.element_size() != 2 or not w_s.is_floating_point() or w_s.requires_grad or not w_q.is_cuda
+                or w_s.device != w_q.device or not w_q.is_contiguous() or not w_s.is_contiguous()
+                or getattr(w_q, "input_dim", 0) != 0 or getattr(w_s, "input_dim", 0) != 0):
+            return False
+        zeros, transposed = None, False
+        if c.zero_points:
+            zeros = getattr(layer, self.w_zp_name)
+            transposed = zeros.shape == (size_n // 8, groups) and groups != size_n // 8
+            if (not transposed and zeros.shape != (groups, size_n // 8)) or (
+                    zeros.dtype != torch.int32 or zeros.device != w_q.device or not zeros.is_contiguous()):
+                return False
+        codes, scales, zeros, self.workspace = torch.ops.sonar_amd.load_gptq_linear(
+            w_q, w_s, zeros, c.group_size != -1 and c.group_size < size_k, transposed)
+        device = codes.device
+        self.is_k_full = True
+        setattr(layer, self.w_gidx_name, marlin_make_empty_g_idx(device))
+        layer.g_idx_sort_indices = marlin_make_empty_g_idx(device)
+        setattr(layer, self.w_zp_name, zeros if c.zero_points else marlin_make_empty_g_idx(device))
+        setattr(layer, self.w_q_name, codes)
+        setattr(layer, self.w_s_name, scales)
+        layer.input_global_scale = None
+        if getattr(layer, "bias", None) is not None:
+            layer.bias = marlin_permute_bias(layer.bias)
+        return True
+
     def process_weights_after_loading(self, layer) -> None:
+        if self._load_in_one_launch(layer):
+            return
         c = self.config
         device = getattr(layer, self.w_q_name).device
         is_a_8bit = c.act_type is not None and c.act_type.itemsize == 1

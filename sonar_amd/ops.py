@@ -84,6 +84,13 @@ def _register_fakes() -> None:
         k, words = qweight.shape
         return qweight.new_empty((k // 8, words * 8)), qzeros.new_empty((words, qzeros.shape[0]))
 
+    @reg("sonar_amd::load_gptq_linear")
+    def _(qweight, scales, zeros, grouped, transposed):
+        k, n = qweight.shape[0] * 8, qweight.shape[1]
+        return (qweight.new_empty((k // 16, n * 2)), torch.empty_like(scales),
+                qweight.new_empty((0 if zeros is None else scales.shape[0], n // 8)),
+                qweight.new_empty((torch.cuda.get_device_properties(qweight.device).multi_processor_count,)))
+
     @reg("sonar_amd::fused_moe")
     def _(output, hidden, w1, w2, bias1, bias2, scale1, scale2, global_scale1, global_scale2, topk_weights, topk_ids,
           g_idx1, g_idx2, perm1, perm2, zeros1, zeros2, cache13, cache2, b_type_id, num_experts, block_size,
