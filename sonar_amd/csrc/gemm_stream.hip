@@ -785,7 +785,8 @@ __device__ __forceinline__ floatx4_t quad_transpose(floatx4_t x, int lane) {
 // GROUPED: one workgroup per (block of slots, strip) of a mixture-of-experts
 // call; the rows of A are gathered and the rows of C scattered through
 // sorted_ids, everything else is the dense kernel on the expert's matrices.
-// GPU: groups per 128-row unit (2 or 4 for groups of 64 or 32 rows, else 1).
+// GPU: groups per 128-row unit (2 or 4 for groups of 64 or 32 rows, else 1).  With two blocks of rows and four sets of
+// scales it holds 170 to 216 registers, so two wavefronts fit a SIMD as with one set.
 // FP4 (with GPU = 4, no zero points): float4_e2m1f codes; the operands are the
 // converted values themselves, so only the scale is left for after the unit.
 // A workgroup works on one piece of one strip (StreamParams::piece_shift / piece_units):
@@ -1387,16 +1388,16 @@ void launch_stream8_mb(const StreamParams& p, bool fp8, hipStream_t st) {
   else launch_stream8_gidx<T, false, false>(p, st);
 }
 
-template <typename T, bool HAS_ZP, int WAVES, int MB, bool GROUPED, int GPU>
+template <typename T, bool HAS_ZP, int WAVES, int MB, bool GROUPED, int GPU, bool FP4 = false>
 int launch_fast_groups(const StreamParams& p, int unit_group_shift, hipStream_t st) {
   static bool attr_set = false;  // raising the dynamic LDS limit is needed once per kernel
   if (!attr_set) {
-    SONAR_HIP(hipFuncSetAttribute((const void*)marlin_stream_fast_kernel<T, HAS_ZP, WAVES, MB, GROUPED, GPU>,
+    SONAR_HIP(hipFuncSetAttribute((const void*)marlin_stream_fast_kernel<T, HAS_ZP, WAVES, MB, GROUPED, GPU, FP4>,
                                   hipFuncAttributeMaxDynamicSharedMemorySize, fast_lds_bytes(WAVES, MB, GPU)));
     attr_set = true;
   }
   const int lds = fast_lds_bytes(WAVES, MB, GPU);
-  marlin_stream_fast_kernel<T, HAS_ZP, WAVES, MB, GROUPED, GPU>
+  marlin_stream_fast_kernel<T, HAS_ZP, WAVES, MB, GROUPED, GPU, FP4>
       <<<p.grid_parts * p.slabs, WAVES * 64, lds, st>>>(p, unit_group_shift);
   return SONAR_OK;
 }
@@ -1405,36 +1406,21 @@ int launch_fast_groups(const StreamParams& p, int unit_group_shift, hipStream_t 
 template <typename T, bool HAS_ZP, int WAVES, int MB, bool GROUPED>
 int launch_fast_waves(const StreamParams& p, int unit_group_shift, hipStream_t st) {
   if (unit_group_shift <= -2) {
-    // several sets of scales per unit and two blocks of rows do not fit the register file (and were measured
-    // slower than the general kernel): callers pass one block of rows
-    if constexpr (MB == 1) {
-      return unit_group_shift == -2 ? launch_fast_groups<T, HAS_ZP, WAVES, 1, GROUPED, 2>(p, unit_group_shift, st)
-                                    : launch_fast_groups<T, HAS_ZP, WAVES, 1, GROUPED, 4>(p, unit_group_shift, st);
-    } else {
+    if constexpr (MB == 1 || GROUPED) {
+      return unit_group_shift == -2 ? launch_fast_groups<T, HAS_ZP, WAVES, MB, GROUPED, 2>(p, unit_group_shift, st)
+                                    : launch_fast_groups<T, HAS_ZP, WAVES, MB, GROUPED, 4>(p, unit_group_shift, st);
+    } else {   // dense calls of more than 16 rows are the mid-size kernel's
       return fail(SONAR_E_INVALID, "internal: groups of 32 / 64 rows with two blocks of rows per workgroup");
     }
   }
   return launch_fast_groups<T, HAS_ZP, WAVES, MB, GROUPED, 1>(p, unit_group_shift, st);
 }
 
-// MXFP4: bf16, four groups of 32 rows per unit, one block of 16 rows per workgroup
-template <int WAVES, bool GROUPED>
-int launch_fast_fp4_waves(const StreamParams& p, hipStream_t st) {
-  static bool attr_set = false;
-  if (!attr_set) {
-    SONAR_HIP(hipFuncSetAttribute((const void*)marlin_stream_fast_kernel<__bf16, false, WAVES, 1, GROUPED, 4, true>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, fast_lds_bytes(WAVES, 1, 4)));
-    attr_set = true;
-  }
-  const int lds = fast_lds_bytes(WAVES, 1, 4);
-  marlin_stream_fast_kernel<__bf16, false, WAVES, 1, GROUPED, 4, true>
-      <<<p.grid_parts * p.slabs, WAVES * 64, lds, st>>>(p, -4);
-  return SONAR_OK;
-}
-
-template <bool GROUPED>
+// MXFP4: bf16, four groups of 32 rows per unit; two blocks of 16 rows in grouped calls only
+template <bool GROUPED, int MB = 1>
 int launch_fast_fp4(const StreamParams& p, bool half_workgroups, hipStream_t st) {
-  return half_workgroups ? launch_fast_fp4_waves<4, GROUPED>(p, st) : launch_fast_fp4_waves<8, GROUPED>(p, st);
+  return half_workgroups ? launch_fast_groups<__bf16, false, 4, MB, GROUPED, 4, true>(p, -4, st)
+                         : launch_fast_groups<__bf16, false, 8, MB, GROUPED, 4, true>(p, -4, st);
 }
 
 // `row_blocks`: blocks of 16 rows per workgroup (1 or 2).
@@ -1579,7 +1565,9 @@ bool moe_fast_applies(bool has_perm, int64_t moe_block_size, int64_t sorted_len,
   if (no_fast || has_perm || size_k % (4 * kChunkK) != 0 || !fast_group_shift(num_groups, group_size, shift) ||
       a_rows * size_k * 2 >= (1LL << 31) || n_strips * units * n_strips >= (1LL << 31))
     return false;
-  if (shift <= -2 && moe_block_size > 16) return false;   // groups of 32 / 64 rows: one block of 16 rows only
+  // (Groups of 32 / 64 rows in blocks of more than 16 slots, us of a layer in the general kernel and here: 32 MXFP4 experts
+  // 3584 x 2688, 24 rows an expert 279 / 170; 8 of 4096 x 14336, 39 rows 476 / 366; 8 with integer codes and groups of 32,
+  // 4096 x 6912, 22 rows 270 / 127, 38 rows 325 / 194; 16 with groups of 64, 2816 x 2816, 41 rows 222 / 137.)
   if (moe_block_size < 64) return true;
   // 64-slot blocks also have the tile kernel, which wins once the experts have
   // rows enough for its tiles.  Measured on Mixtral shapes (8 experts, top 2;
@@ -1589,9 +1577,12 @@ bool moe_fast_applies(bool has_perm, int64_t moe_block_size, int64_t sorted_len,
   // against 272 / 132; 1144 slots: down 150 against 137; 1272 slots: down 178
   // against 141.  The tile kernel launches at least experts x N / 256
   // workgroups; where that is under one per compute unit (down) it stays
-  // behind a little longer.
+  // behind a little longer.  Four sets of scales a unit cost this kernel more than
+  // the tile kernel: MXFP4, 4096 x 6912, 884 slots 188 us a layer against 195, 944
+  // slots 203 against 198, 994 slots 229 against 200 (with only the down GEMM here 197);
+  // 1024 x 1408, 984 slots (88 and 32 tiles) 41 against 62.
   const int64_t tile_workgroups = num_experts * ((size_n + 255) / 256);
-  return sorted_len <= (tile_workgroups < cu_count() ? 1100 : 1000);
+  return sorted_len <= (tile_workgroups < cu_count() ? 1100 : shift == -4 ? 900 : 1000);
 }
 
 // Called by sonar_moe_wna16_marlin_gemm when moe_fast_applies: one workgroup
@@ -1659,8 +1650,8 @@ int moe_fast_gemm(const void* a, void* c, const uint32_t* b, const void* bias, c
   p.nt_weights = !no_nt && p.sub_blocks == 1 && p.slabs <= 2 * num_experts &&
                  num_experts * size_k * size_n / 2 >= 10 * 1000 * 1000;
   int rc;
-  if (fp4)   // bf16, groups of 32 rows, blocks of at most 16 slots: moe_fast_applies has seen to it
-    rc = launch_fast_fp4<true>(p, half, st);
+  if (fp4)   // bf16, groups of 32 rows
+    rc = row_blocks == 2 ? launch_fast_fp4<true, 2>(p, half, st) : launch_fast_fp4<true>(p, half, st);
   else if (dtype == SONAR_DTYPE_F16)
     rc = zeros ? launch_fast<_Float16, true, true>(p, unit_group_shift, half, row_blocks, st)
                : launch_fast<_Float16, false, true>(p, unit_group_shift, half, row_blocks, st);
