@@ -10,6 +10,8 @@
 // routing weight when asked (marlin_template.h:1883-1909).  K is never split
 // across workgroups, so nothing is reduced through memory and results do not
 // depend on the launch: scratch and workspace are not used.
+// Calls with few rows per expert and K % 128 == 0 on 4-bit codes go to the decode kernel in grouped form instead
+// (gemm_stream.hip), 64-slot blocks of many rows to the tile kernels (gemm_tile.hip).
 #include <cstdlib>
 
 #include "common.hpp"
@@ -27,7 +29,7 @@ int moe_tile_gemm(const void* a, void* c, const uint32_t* b, const void* bias, c
                   size_t partial_bytes, hipStream_t st);
 size_t moe_tile_table_bytes(int64_t sorted_len, int64_t num_experts);
 size_t moe_tile_partial_bytes(int64_t size_k);
-// gemm_stream.hip: the 16-row decode kernel in grouped form, for few rows per expert
+// gemm_stream.hip: the decode kernel in grouped form, for few rows per expert
 bool moe_fast_applies(bool has_perm, int64_t moe_block_size, int64_t sorted_len, int64_t num_experts,
                       int64_t a_rows, int64_t size_n, int64_t size_k, int64_t num_groups, int group_size);
 int moe_fast_gemm(const void* a, void* c, const uint32_t* b, const void* bias, const void* scales,

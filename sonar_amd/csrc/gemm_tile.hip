@@ -511,15 +511,16 @@ __global__ __launch_bounds__(kTileWaves * 64) void marlin_tile_kernel(const Tile
 // phase 4kt+4.
 // LDS is read from asm blocks only (the compiler cannot tell which LDS bytes a
 // copy writes and would otherwise wait for all copies before any LDS access).
-// Needs groups of 32 rows or a multiple of 64 (or one group) and no act-order.
+// Needs groups of a multiple of 64 rows (or one group) and no act-order, or MXFP4: what the wide kernel does not take
+// (groups of 192 rows and the like, and dense MXFP4 calls of few tiles).
 constexpr int kAsyncStages = 3;
-// G32: groups of 32 rows, i.e. one group per k block: a stage then carries two
-// scale / zero-point rows (256 bytes each) and takes one copy more.
+// g32: groups of 32 rows (MXFP4), i.e. one group per k block: a stage then carries two
+// scale rows (256 bytes each) and takes one copy more.
 constexpr int wave_stage(bool g32) { return 2 * kBlockBytes + (g32 ? 512 : 256); }   // two weight chunks + scale rows
 constexpr int kAsyncA = kAsyncStages * kStageA;
 constexpr int async_lds(bool g32) { return kAsyncA + kTileWaves * kAsyncStages * wave_stage(g32); }
 constexpr int async_copies(bool g32) { return g32 ? 8 : 7; }
-// 8-bit codes (W8 = 1: uint8b128, 2: float8_e4m3fn): a K step of a strip is four 1-KiB blocks
+// 8-bit codes (W8: uint8b128): a K step of a strip is four 1-KiB blocks
 // of 16 rows (block 2 b holds the low four, block 2 b + 1 the high four of the eight
 // consecutive rows of a lane's operand of k block b).  Private rings of that size would not
 // fit, so the two wavefronts of a strip (one per group of rows) share one ring: the
@@ -527,21 +528,18 @@ constexpr int async_copies(bool g32) { return g32 ? 8 : 7; }
 // 1, the same number of copies per stage as with 4-bit codes.  The barriers that order the
 // shared stages of A order these too: group 1 reads k block 0 one phase after group 0 has
 // waited for its copies, group 0 reads k block 1 two barriers after group 1 has.
-constexpr int strip_stage8(bool g32) { return 4 * kBlockBytes + (g32 ? 512 : 256); }
-constexpr int async_lds8(bool g32) { return kAsyncA + (kTileN / kStripN) * kAsyncStages * strip_stage8(g32); }
+constexpr int strip_stage8() { return 4 * kBlockBytes + 256; }
+constexpr int async_lds8() { return kAsyncA + (kTileN / kStripN) * kAsyncStages * strip_stage8(); }
 
-// NV (with G32 and FP4): NVFP4, groups of 16 rows.  The scale rows of a stage then hold four
-// groups of 128 bytes (a copy fetches two rows, one per half of the wavefront), and a lane,
-// whose eight rows of a k block lie in one group, reads the row of group 2 b + kb / 2.
-template <typename T, bool HAS_ZP, bool GROUPED, bool G32 = false, bool FP4 = false, int W8 = 0, bool NV = false>
+template <typename T, bool HAS_ZP, bool GROUPED, bool FP4 = false, bool W8 = false>
 __global__ __launch_bounds__(kTileWaves * 64) void marlin_tile_async_kernel(const TileParams p) {
   typedef typename Dq<T>::vec8 vec8;
-  typedef typename Dq4Of<T, FP4, NV>::type D4;   // integer codes, or float4_e2m1f (MXFP4 / NVFP4: with G32)
-  static_assert(!NV || (G32 && FP4 && !HAS_ZP && W8 == 0), "NVFP4 is float4 codes with groups of 16 rows");
-  typedef typename Dq8Of<T, W8 == 2>::type D8;   // 8-bit integer or floating-point codes (W8 != 0)
-  typedef typename std::conditional<W8 != 0, typename D8::Col, typename D4::Col>::type Col;
-  static_assert(W8 == 0 || (!HAS_ZP && !FP4), "8-bit codes are symmetric");
-  constexpr int kWaveStage = W8 ? strip_stage8(G32) : wave_stage(G32);
+  typedef typename Dq4Of<T, FP4, false>::type D4;   // integer codes, or float4_e2m1f (MXFP4)
+  typedef typename Dq8Of<T, false>::type D8;
+  typedef typename std::conditional<W8, typename D8::Col, typename D4::Col>::type Col;
+  static_assert(!W8 || (!HAS_ZP && !FP4), "8-bit codes are symmetric");
+  constexpr bool G32 = FP4;
+  constexpr int kWaveStage = W8 ? strip_stage8() : wave_stage(G32);
   constexpr int kWeightBytes = (W8 ? 4 : 2) * kBlockBytes;   // packed weights of a stage, scale rows behind them
   constexpr int kAsyncCopies = async_copies(G32);
   extern __shared__ __attribute__((aligned(1024))) char smem[];
@@ -613,7 +611,6 @@ __global__ __launch_bounds__(kTileWaves * 64) void marlin_tile_async_kernel(cons
   } else {
     s_src = reinterpret_cast<const char*>(p.scales + expert * p.expert_s_stride + strip * kStripN) + 4 * (lane & 31);
     s_group_stride = (long)p.size_n * 2;
-    if (NV) s_src += (lane >> 5) * s_group_stride;   // the upper half of the wavefront fetches the next group's row
   }
   // the weight ring: private to the wavefront, or shared by the two wavefronts of a strip (8-bit codes)
   char* wring = smem + kAsyncA + (W8 ? wn : wave) * (kAsyncStages * kWaveStage);
@@ -642,8 +639,7 @@ __global__ __launch_bounds__(kTileWaves * 64) void marlin_tile_async_kernel(cons
     }
     // the scale rows (with a shared ring both wavefronts of the strip copy them: the same bytes twice)
     if (G32) {   // idx 6 / 7: the rows of groups 2 kt and 2 kt + 1
-      __builtin_amdgcn_global_load_lds((glb_void_t*)(s_src + (long)((NV ? 4 : 2) * kt + (NV ? 2 : 1) * (idx - 6)) *
-                                                                 s_group_stride),
+      __builtin_amdgcn_global_load_lds((glb_void_t*)(s_src + (long)(2 * kt + idx - 6) * s_group_stride),
                                        (lds_void_t*)(sw + kWeightBytes + 256 * (idx - 6)), 4, 0, 0);
       return;
     }
@@ -697,8 +693,8 @@ __global__ __launch_bounds__(kTileWaves * 64) void marlin_tile_async_kernel(cons
   auto raw_start = [&](int slot, int b, bool with_scales) {
     const uint32_t w_at = w_lds + slot * kWaveStage;
     const uint32_t q_at = w_at + (W8 ? 2 * b : b) * kBlockBytes + lane * 16;
-    const uint32_t r_at = w_at + (NV ? 128 * (2 * b + (kb >> 1)) : (G32 ? 256 * b : 0));   // this k block's scale row
-    if constexpr (W8 != 0) asm volatile("ds_read_b128 %0, %1 offset:1024" : "=&v"(qhigh) : "v"(q_at) : "memory");
+    const uint32_t r_at = w_at + (G32 ? 256 * b : 0);   // this k block's scale row
+    if constexpr (W8) asm volatile("ds_read_b128 %0, %1 offset:1024" : "=&v"(qhigh) : "v"(q_at) : "memory");
     if (with_scales) {
       asm volatile(
           "ds_read_b128 %0, %6\n\t"
@@ -709,7 +705,7 @@ __global__ __launch_bounds__(kTileWaves * 64) void marlin_tile_async_kernel(cons
           "ds_read_b32 %5, %11"
           : "=&v"(qraw), "=&v"(sb0), "=&v"(sb1), "=&v"(sb2), "=&v"(sb3), "=&v"(zw)
           : "v"(q_at), "v"(r_at + s_off[0]), "v"(r_at + s_off[1]), "v"(r_at + s_off[2]), "v"(r_at + s_off[3]),
-            "v"(NV ? r_at + s_off[0] : r_at + z_off)
+            "v"(r_at + z_off)
           : "memory");
     } else {
       asm volatile("ds_read_b128 %0, %1" : "=&v"(qraw) : "v"(q_at) : "memory");
@@ -719,7 +715,7 @@ __global__ __launch_bounds__(kTileWaves * 64) void marlin_tile_async_kernel(cons
   // and dequantises it, then waits for the operands of A the last multiply
   // phase started to read.
   auto fetch = [&](int slot, int b, bool with_scales) {
-    if constexpr (W8 != 0) {
+    if constexpr (W8) {
       asm volatile("s_waitcnt lgkmcnt(0)"
                    : "+v"(qraw), "+v"(qhigh), "+v"(sb0), "+v"(sb1), "+v"(sb2), "+v"(sb3), "+v"(zw)
                    :
@@ -734,7 +730,7 @@ __global__ __launch_bounds__(kTileWaves * 64) void marlin_tile_async_kernel(cons
       const uint32_t sbits[4] = {sb0, sb1, sb2, sb3};
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        if constexpr (W8 != 0) {
+        if constexpr (W8) {
           cols[j] = D8::make_col((uint16_t)sbits[j]);
         } else {
           int z = 8;
@@ -743,7 +739,7 @@ __global__ __launch_bounds__(kTileWaves * 64) void marlin_tile_async_kernel(cons
         }
       }
     }
-    if constexpr (W8 != 0) {
+    if constexpr (W8) {
       const uint32_t lo[4] = {qraw.x, qraw.y, qraw.z, qraw.w}, hi[4] = {qhigh.x, qhigh.y, qhigh.z, qhigh.w};
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -799,7 +795,7 @@ __global__ __launch_bounds__(kTileWaves * 64) void marlin_tile_async_kernel(cons
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kAsyncCopies) : "memory");  // stage k_first has landed
   // a shared ring: the blocks of k block 0 are the copies of the strip's wavefront of group 0,
   // which the wavefront of group 1 may read only behind a barrier that follows that wait
-  if constexpr (W8 != 0) phase_end();
+  if constexpr (W8) phase_end();
   raw_start(0, 0, true);
   phase_end();
   {
@@ -848,7 +844,7 @@ __global__ __launch_bounds__(kTileWaves * 64) void marlin_tile_async_kernel(cons
   }
   if (wm == 0) phase_end();  // the barrier that ends group 1's last phase
   // the last copies and the last read started by raw_start must not outlive the wavefront
-  if constexpr (W8 != 0) {
+  if constexpr (W8) {
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)"
                  : "+v"(qraw), "+v"(qhigh), "+v"(sb0), "+v"(sb1), "+v"(sb2), "+v"(sb3), "+v"(zw)::"memory");
   } else {
@@ -894,8 +890,6 @@ __global__ __launch_bounds__(kTileWaves * 64) void marlin_tile_async_kernel(cons
     }
   }
   const uint16_t* bias_src = p.bias ? p.bias + expert * p.expert_bias_stride + strip * kStripN : nullptr;
-  float gs = 1.f;   // NVFP4: the global scale multiplies the sum before anything else (marlin_template.h:1661-1665)
-  if (NV && p.global_scale) gs = p.global_scale[GROUPED ? expert : 0];
 #pragma unroll
   for (int nb = 0; nb < 4; ++nb) {
     const int n = strip * kStripN + 16 * nb + 4 * kb;
@@ -907,7 +901,7 @@ __global__ __launch_bounds__(kTileWaves * 64) void marlin_tile_async_kernel(cons
 #pragma unroll
     for (int mb = 0; mb < 8; ++mb) {
       if (c_row[mb] < 0) continue;
-      const floatx4_t v = NV ? acc[nb][mb] * gs : acc[nb][mb];
+      const floatx4_t v = acc[nb][mb];
       uint16_t o[4] = {Dq<T>::from_float(v.x + bias[0]), Dq<T>::from_float(v.y + bias[1]),
                        Dq<T>::from_float(v.z + bias[2]), Dq<T>::from_float(v.w + bias[3])};
       if (GROUPED && p.mul_topk) {
@@ -956,7 +950,7 @@ __global__ __launch_bounds__(kTileWaves * 64) void marlin_tile_async_kernel(cons
 // block), integer / 8-bit floating-point codes with a scale per 32 rows (MXFP8 among them), or NVFP4
 // (float4_e2m1f codes with a scale per 16 rows and a global scale, either activation type); no
 // act-order; dense and grouped (mixture-of-experts) calls.  A pass of the loop is four steps, whose ring positions
-// are static; a K range that is no multiple of four steps leaves the last pass early.
+// are static; up to three steps that are no whole pass follow the loop.
 constexpr int kWideStages = 4;
 constexpr int kWideScaleRows = 16;   // a ring of 16 rows per wavefront: eight steps of one row, or of two (groups of 32 rows)
 // RB: row blocks of 16 rows a wavefront owns: 16 (a 256-row tile) or 8 (a 128-row tile, for
@@ -1735,106 +1729,55 @@ __global__ __launch_bounds__(64 * kTableWaves) void moe_tile_table_kernel(const 
   }
 }
 
-template <typename T, bool HAS_ZP, bool G32>
-int launch_tile_async_groups(const TileParams& p, hipStream_t st) {
+template <typename T, bool HAS_ZP, bool GROUPED, bool FP4 = false, bool W8 = false>
+int launch_tile_async(const TileParams& p, hipStream_t st) {
+  constexpr int kLds = W8 ? async_lds8() : async_lds(FP4);
   static bool attr_set = false;  // raising the dynamic LDS limit is needed once per kernel
   if (!attr_set) {
-    SONAR_HIP(hipFuncSetAttribute((const void*)marlin_tile_async_kernel<T, HAS_ZP, false, G32>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, async_lds(G32)));
+    SONAR_HIP(hipFuncSetAttribute((const void*)marlin_tile_async_kernel<T, HAS_ZP, GROUPED, FP4, W8>,
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, kLds));
     attr_set = true;
   }
-  const int grid = tile_grid(p);
-  marlin_tile_async_kernel<T, HAS_ZP, false, G32><<<grid, kTileWaves * 64, async_lds(G32), st>>>(p);
+  marlin_tile_async_kernel<T, HAS_ZP, GROUPED, FP4, W8><<<tile_grid(p), kTileWaves * 64, kLds, st>>>(p);
   return SONAR_OK;
 }
-
-// MXFP4: bf16, groups of 32 rows, float4_e2m1f codes
-int launch_tile_async_fp4(const TileParams& p, hipStream_t st) {
-  static bool attr_set = false;
-  if (!attr_set) {
-    SONAR_HIP(hipFuncSetAttribute((const void*)marlin_tile_async_kernel<__bf16, false, false, true, true>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, async_lds(true)));
-    attr_set = true;
-  }
-  marlin_tile_async_kernel<__bf16, false, false, true, true><<<tile_grid(p), kTileWaves * 64, async_lds(true), st>>>(p);
-  return SONAR_OK;
+// groups of a multiple of 64 rows that is no power of two times 64
+template <bool GROUPED>
+int launch_tile_async_type(const TileParams& p, int dtype, int bits, hipStream_t st) {
+  if (bits == 8)
+    return dtype == SONAR_DTYPE_F16 ? launch_tile_async<_Float16, false, GROUPED, false, true>(p, st)
+                                    : launch_tile_async<__bf16, false, GROUPED, false, true>(p, st);
+  if (dtype == SONAR_DTYPE_F16)
+    return p.zeros ? launch_tile_async<_Float16, true, GROUPED>(p, st) : launch_tile_async<_Float16, false, GROUPED>(p, st);
+  return p.zeros ? launch_tile_async<__bf16, true, GROUPED>(p, st) : launch_tile_async<__bf16, false, GROUPED>(p, st);
 }
 
-// NVFP4: either activation type, groups of 16 rows, a global scale (one per expert when GROUPED)
-template <typename T, bool GROUPED = false>
-int launch_tile_async_nvfp4(const TileParams& p, hipStream_t st) {
-  static bool attr_set = false;
-  if (!attr_set) {
-    SONAR_HIP(hipFuncSetAttribute((const void*)marlin_tile_async_kernel<T, false, GROUPED, true, true, 0, true>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, async_lds(true)));
-    attr_set = true;
-  }
-  marlin_tile_async_kernel<T, false, GROUPED, true, true, 0, true>
-      <<<tile_grid(p), kTileWaves * 64, async_lds(true), st>>>(p);
-  return SONAR_OK;
-}
-
-int launch_tile_grouped_fp4(const TileParams& p, hipStream_t st) {
-  static bool attr_set = false;
-  if (!attr_set) {
-    SONAR_HIP(hipFuncSetAttribute((const void*)marlin_tile_async_kernel<__bf16, false, true, true, true>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, async_lds(true)));
-    attr_set = true;
-  }
-  marlin_tile_async_kernel<__bf16, false, true, true, true><<<tile_grid(p), kTileWaves * 64, async_lds(true), st>>>(p);
-  return SONAR_OK;
-}
-
-// 8-bit codes (W8 = 1: uint8b128, 2: float8_e4m3fn), dense or grouped
-template <typename T, bool GROUPED, bool G32, int W8>
-int launch_tile_async8_groups(const TileParams& p, hipStream_t st) {
-  static bool attr_set = false;
-  if (!attr_set) {
-    SONAR_HIP(hipFuncSetAttribute((const void*)marlin_tile_async_kernel<T, false, GROUPED, G32, false, W8>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, async_lds8(G32)));
-    attr_set = true;
-  }
-  marlin_tile_async_kernel<T, false, GROUPED, G32, false, W8>
-      <<<tile_grid(p), kTileWaves * 64, async_lds8(G32), st>>>(p);
-  return SONAR_OK;
-}
-template <typename T, bool GROUPED>
-int launch_tile_async8(const TileParams& p, bool fp8, hipStream_t st) {
-  const bool g32 = p.num_groups > 1 && p.group_size == 32;
-  if (fp8) return g32 ? launch_tile_async8_groups<T, GROUPED, true, 2>(p, st)
-                      : launch_tile_async8_groups<T, GROUPED, false, 2>(p, st);
-  return g32 ? launch_tile_async8_groups<T, GROUPED, true, 1>(p, st)
-             : launch_tile_async8_groups<T, GROUPED, false, 1>(p, st);
-}
-
-template <typename T, bool HAS_ZP, bool GROUPED, int RB>
+// (Grouped calls: marlin_tile_wide_pair_kernel, but for NVFP4 and 8-bit codes with groups of 32 rows.)
+template <typename T, bool HAS_ZP, int RB>
 int launch_tile_wide_rows(const TileParams& p, hipStream_t st) {
   static bool attr_set = false;
   if (!attr_set) {
-    SONAR_HIP(hipFuncSetAttribute((const void*)marlin_tile_wide_kernel<T, HAS_ZP, GROUPED, RB>,
+    SONAR_HIP(hipFuncSetAttribute((const void*)marlin_tile_wide_kernel<T, HAS_ZP, false, RB>,
                                   hipFuncAttributeMaxDynamicSharedMemorySize, wide_lds(RB)));
     attr_set = true;
   }
-  marlin_tile_wide_kernel<T, HAS_ZP, GROUPED, RB><<<tile_grid(p), 256, wide_lds(RB), st>>>(p);
+  marlin_tile_wide_kernel<T, HAS_ZP, false, RB><<<tile_grid(p), 256, wide_lds(RB), st>>>(p);
   return SONAR_OK;
 }
 // MXFP4: bf16, groups of 32 rows, float4_e2m1f codes
-template <bool GROUPED, int RB>
+template <int RB>
 int launch_tile_wide_fp4_rows(const TileParams& p, hipStream_t st) {
   static bool attr_set = false;
   if (!attr_set) {
-    SONAR_HIP(hipFuncSetAttribute((const void*)marlin_tile_wide_kernel<__bf16, false, GROUPED, RB, true>,
+    SONAR_HIP(hipFuncSetAttribute((const void*)marlin_tile_wide_kernel<__bf16, false, false, RB, true>,
                                   hipFuncAttributeMaxDynamicSharedMemorySize, wide_lds(RB)));
     attr_set = true;
   }
-  marlin_tile_wide_kernel<__bf16, false, GROUPED, RB, true><<<tile_grid(p), 256, wide_lds(RB), st>>>(p);
+  marlin_tile_wide_kernel<__bf16, false, false, RB, true><<<tile_grid(p), 256, wide_lds(RB), st>>>(p);
   return SONAR_OK;
 }
-template <bool GROUPED>
 int launch_tile_wide_fp4(const TileParams& p, hipStream_t st) {
-  if constexpr (!GROUPED)
-    if (p.tile_rows == 128) return launch_tile_wide_fp4_rows<false, 8>(p, st);
-  return launch_tile_wide_fp4_rows<GROUPED, 16>(p, st);
+  return p.tile_rows == 128 ? launch_tile_wide_fp4_rows<8>(p, st) : launch_tile_wide_fp4_rows<16>(p, st);
 }
 // NVFP4: either activation type, groups of 16 rows, a global scale (one per expert when GROUPED)
 template <typename T, bool GROUPED, int RB>
@@ -1871,39 +1814,32 @@ int launch_tile_wide8(const TileParams& p, bool fp8, hipStream_t st) {
   const bool g32 = wide_groups_of_32(p);
   // 128-row tiles (dense calls with few tiles)
   if (p.tile_rows == 128 && g32) return fail(SONAR_E_INVALID, "internal: 8-bit codes with groups of 32 rows run on 256-row tiles");
-  if constexpr (!GROUPED)
+  if (g32) return fp8 ? launch_tile_wide8_groups<T, GROUPED, 2, true>(p, st) : launch_tile_wide8_groups<T, GROUPED, 1, true>(p, st);
+  if constexpr (!GROUPED) {
     if (p.tile_rows == 128)
       return fp8 ? launch_tile_wide8_groups<T, false, 2, false, 8>(p, st)
                  : launch_tile_wide8_groups<T, false, 1, false, 8>(p, st);
-  if (fp8) return g32 ? launch_tile_wide8_groups<T, GROUPED, 2, true>(p, st)
-                      : launch_tile_wide8_groups<T, GROUPED, 2, false>(p, st);
-  return g32 ? launch_tile_wide8_groups<T, GROUPED, 1, true>(p, st)
-             : launch_tile_wide8_groups<T, GROUPED, 1, false>(p, st);
+    return fp8 ? launch_tile_wide8_groups<T, false, 2, false>(p, st) : launch_tile_wide8_groups<T, false, 1, false>(p, st);
+  }
+  return fail(SONAR_E_INVALID, "internal: a grouped call of one tile size");
 }
 // 4-bit integer codes with groups of 32 rows
-template <typename T, bool HAS_ZP, bool GROUPED, int RB>
+template <typename T, bool HAS_ZP, int RB>
 int launch_tile_wide_g32_rows(const TileParams& p, hipStream_t st) {
   static bool attr_set = false;
   if (!attr_set) {
-    SONAR_HIP(hipFuncSetAttribute((const void*)marlin_tile_wide_kernel<T, HAS_ZP, GROUPED, RB, false, 0, true>,
+    SONAR_HIP(hipFuncSetAttribute((const void*)marlin_tile_wide_kernel<T, HAS_ZP, false, RB, false, 0, true>,
                                   hipFuncAttributeMaxDynamicSharedMemorySize, wide_lds(RB)));
     attr_set = true;
   }
-  marlin_tile_wide_kernel<T, HAS_ZP, GROUPED, RB, false, 0, true><<<tile_grid(p), 256, wide_lds(RB), st>>>(p);
+  marlin_tile_wide_kernel<T, HAS_ZP, false, RB, false, 0, true><<<tile_grid(p), 256, wide_lds(RB), st>>>(p);
   return SONAR_OK;
 }
-template <typename T, bool HAS_ZP, bool GROUPED>
-int launch_tile_wide_g32(const TileParams& p, hipStream_t st) {
-  if constexpr (!GROUPED)
-    if (p.tile_rows == 128) return launch_tile_wide_g32_rows<T, HAS_ZP, false, 8>(p, st);
-  return launch_tile_wide_g32_rows<T, HAS_ZP, GROUPED, 16>(p, st);
-}
-template <typename T, bool HAS_ZP, bool GROUPED = false>
+template <typename T, bool HAS_ZP>
 int launch_tile_wide(const TileParams& p, hipStream_t st) {
-  if (wide_groups_of_32(p)) return launch_tile_wide_g32<T, HAS_ZP, GROUPED>(p, st);
-  if constexpr (!GROUPED)   // (grouped: 128-row tiles run with the others in one launch)
-    if (p.tile_rows == 128) return launch_tile_wide_rows<T, HAS_ZP, false, 8>(p, st);
-  return launch_tile_wide_rows<T, HAS_ZP, GROUPED, 16>(p, st);
+  if (wide_groups_of_32(p))
+    return p.tile_rows == 128 ? launch_tile_wide_g32_rows<T, HAS_ZP, 8>(p, st) : launch_tile_wide_g32_rows<T, HAS_ZP, 16>(p, st);
+  return p.tile_rows == 128 ? launch_tile_wide_rows<T, HAS_ZP, 8>(p, st) : launch_tile_wide_rows<T, HAS_ZP, 16>(p, st);
 }
 
 // Both tile sizes; `max_row_tiles`: grouped calls, the most row tiles there can be.
@@ -1939,30 +1875,6 @@ int launch_pair(const TileParams& p, int max_row_tiles, int dtype, bool fp4, int
   return rc ? rc : launch_status("marlin_tile_wide_pair_kernel");
 }
 
-template <typename T, bool HAS_ZP>
-int launch_tile_async(const TileParams& p, hipStream_t st) {
-  return (p.num_groups > 1 && p.group_size == 32) ? launch_tile_async_groups<T, HAS_ZP, true>(p, st)
-                                                  : launch_tile_async_groups<T, HAS_ZP, false>(p, st);
-}
-
-template <typename T, bool HAS_ZP, bool G32>
-int launch_tile_grouped_groups(const TileParams& p, hipStream_t st) {
-  static bool attr_set = false;
-  if (!attr_set) {
-    SONAR_HIP(hipFuncSetAttribute((const void*)marlin_tile_async_kernel<T, HAS_ZP, true, G32>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, async_lds(G32)));
-    attr_set = true;
-  }
-  marlin_tile_async_kernel<T, HAS_ZP, true, G32><<<tile_grid(p), kTileWaves * 64, async_lds(G32), st>>>(p);
-  return SONAR_OK;
-}
-
-template <typename T, bool HAS_ZP>
-int launch_tile_grouped(const TileParams& p, hipStream_t st) {
-  return (p.num_groups > 1 && p.group_size == 32) ? launch_tile_grouped_groups<T, HAS_ZP, true>(p, st)
-                                                  : launch_tile_grouped_groups<T, HAS_ZP, false>(p, st);
-}
-
 template <typename T, bool HAS_ZP, bool HAS_PERM>
 int launch_tile(const TileParams& p, hipStream_t st) {
   static bool attr_set = false;  // raising the dynamic LDS limit is needed once per kernel
@@ -1986,8 +1898,9 @@ namespace {
 // N = 7808, once padded, 81.5 -> 78.3; 2000 tokens on 32 MXFP4 experts of 2880 x 2880, the whole layer 626 -> 543.)
 bool wide_applies(const TileParams& p) {
   static const bool no_wide = getenv("SONAR_MARLIN_NO_WIDE_TILE") != nullptr;   // debugging aid
+  if (wide_groups_of_32(p)) return true;
   if (no_wide) return false;
-  if (p.num_groups == 1 || wide_groups_of_32(p)) return true;
+  if (p.num_groups == 1) return true;
   const int per_group = p.group_size / kTileK;   // steps per group: a power of two
   return p.group_size % kTileK == 0 && (per_group & (per_group - 1)) == 0;
 }
@@ -1998,12 +1911,12 @@ bool wide_applies(const TileParams& p) {
 // 512 tiles: 215 against 201).
 bool wide_applies_fp4(const TileParams& p) {
   static const bool no_wide = getenv("SONAR_MARLIN_NO_WIDE_TILE") != nullptr;
-  const bool few = p.tile_table == nullptr && p.global_scale == nullptr && p.tile_rows == kTileM && p.k_splits == 1 &&
-                   p.tiles_m * p.tiles_n <= 192;
+  if (p.tile_table != nullptr || p.global_scale != nullptr) return true;
+  const bool few = p.tile_rows == kTileM && p.k_splits == 1 && p.tiles_m * p.tiles_n <= 192;
   return !no_wide && !few;
 }
-// ... and for 8-bit codes (the same rule).
-bool wide_applies8(const TileParams& p) { return wide_applies(p); }
+// ... and for 8-bit codes (the same rule; floating-point ones come in groups of 32 or 128 rows or one).
+bool wide_applies8(const TileParams& p, bool fp8) { return fp8 || wide_applies(p); }
 }  // namespace
 
 // The asynchronous tile kernel needs groups of 32 rows or a multiple of 64 and no gather of A.
@@ -2070,7 +1983,7 @@ TileLaunches plan_tile_launches(TileParams p, int64_t size_m, int64_t size_n, in
     return out;
   }
   auto takes_wide = [&](const TileParams& q) {
-    return fp4 ? wide_applies_fp4(q) : (bits == 8 ? wide_applies8(q) : wide_applies(q));
+    return fp4 ? wide_applies_fp4(q) : wide_applies(q);
   };
   // More tiles than compute units with a last round that fills half of them or less (M = 4096, N = 6144: 384 tiles of 256
   // rows = 256 + 128): the full rounds run as they are and the tiles of the last round as two 128-row tiles each, over
@@ -2142,27 +2055,17 @@ int tile_gemm(const void* a, int64_t a_row_stride, void* c, const uint32_t* b, c
       return fail(SONAR_E_INVALID, "internal: 128-row tiles exist in the wide tile kernel only");
     // the kernel a launch described by q takes
     auto launch = [&](const TileParams& q) -> int {
-      if (nvfp4 && wide_applies_fp4(q))
+      if (nvfp4)
         return dtype == SONAR_DTYPE_F16 ? launch_tile_wide_nvfp4<_Float16, false>(q, st)
-                                    : launch_tile_wide_nvfp4<__bf16, false>(q, st);
-      else if (nvfp4)
-        return dtype == SONAR_DTYPE_F16 ? launch_tile_async_nvfp4<_Float16>(q, st) : launch_tile_async_nvfp4<__bf16>(q, st);
-      else if (fp4)   // the caller has checked: bf16, groups of 32 rows, no zero points
-        return wide_applies_fp4(q) ? launch_tile_wide_fp4<false>(q, st) : launch_tile_async_fp4(q, st);
-      else if (bits == 8 && wide_applies8(q))
+                                        : launch_tile_wide_nvfp4<__bf16, false>(q, st);
+      if (fp4)   // the caller has checked: bf16, groups of 32 rows, no zero points
+        return wide_applies_fp4(q) ? launch_tile_wide_fp4(q, st) : launch_tile_async<__bf16, false, false, true>(q, st);
+      if (bits == 8 && wide_applies8(q, fp8))   // symmetric 8-bit codes: the caller has checked
         return dtype == SONAR_DTYPE_F16 ? launch_tile_wide8<_Float16, false>(q, fp8, st)
-                                    : launch_tile_wide8<__bf16, false>(q, fp8, st);
-      else if (bits == 8)   // symmetric 8-bit codes: the caller has checked
-        return dtype == SONAR_DTYPE_F16 ? launch_tile_async8<_Float16, false>(q, fp8, st)
-                                    : launch_tile_async8<__bf16, false>(q, fp8, st);
-      else if (wide_applies(q) && dtype == SONAR_DTYPE_F16)
-        return zp ? launch_tile_wide<_Float16, true>(q, st) : launch_tile_wide<_Float16, false>(q, st);
-      else if (wide_applies(q))
-        return zp ? launch_tile_wide<__bf16, true>(q, st) : launch_tile_wide<__bf16, false>(q, st);
-      else if (dtype == SONAR_DTYPE_F16)
-        return zp ? launch_tile_async<_Float16, true>(q, st) : launch_tile_async<_Float16, false>(q, st);
-      else
-        return zp ? launch_tile_async<__bf16, true>(q, st) : launch_tile_async<__bf16, false>(q, st);
+                                        : launch_tile_wide8<__bf16, false>(q, fp8, st);
+      if (bits == 8 || !wide_applies(q)) return launch_tile_async_type<false>(q, dtype, bits, st);
+      if (dtype == SONAR_DTYPE_F16) return zp ? launch_tile_wide<_Float16, true>(q, st) : launch_tile_wide<_Float16, false>(q, st);
+      return zp ? launch_tile_wide<__bf16, true>(q, st) : launch_tile_wide<__bf16, false>(q, st);
     };
     p = plan.launch;
     if (plan.pair) return launch_pair<false>(p, 0, dtype, fp4, bits, fp8, st);
@@ -2265,16 +2168,15 @@ int moe_tile_gemm(const void* a, void* c, const uint32_t* b, const void* bias, c
   // The wide kernel splits the tiles of a short last round (or all of them when they are few) along
   // K, given room for their partial tiles; moe_tile_reduce_kernel sums them.
   static const bool no_live_split = getenv("SONAR_MARLIN_NO_MOE_K_SPLIT") != nullptr;   // debugging aid
-  const bool wide = fp4 ? wide_applies_fp4(p) : (bits == 8 ? wide_applies8(p) : wide_applies(p));
+  const bool wide = fp4 ? wide_applies_fp4(p) : (bits == 8 ? wide_applies8(p, fp8) : wide_applies(p));
   const size_t partial_need = moe_tile_partial_bytes(size_k);
   if (wide && !no_live_split && partial != nullptr && partial_need > 0 && partial_bytes >= partial_need &&
       ((uintptr_t)partial) % 16 == 0)
     p.partial = static_cast<float4*>(partial);
   // ... and computes the one or two blocks an expert's rows end in as a 128-row tile, and others where that makes the launch
   // shorter (marlin_tile_wide_pair_kernel; not NVFP4, and not 8-bit codes with groups of 32 rows)
-  static const bool no_small = getenv("SONAR_MARLIN_NO_MOE_128_ROW_TILES") != nullptr;   // debugging aid
   const bool nvfp4 = fp4 && global_scale != nullptr;
-  const bool two_sizes = wide && !no_small && !nvfp4 && !(bits == 8 && wide_groups_of_32(p));
+  const bool two_sizes = wide && !nvfp4 && !(bits == 8 && wide_groups_of_32(p));
   int32_t* table_small = two_sizes ? table + moe_one_table_bytes(sorted_len) / sizeof(int32_t) : nullptr;
   if (two_sizes) {
     // tiles are cut along K only while they are few (and the second kernel is launched only where they may be): not when
@@ -2305,28 +2207,14 @@ int moe_tile_gemm(const void* a, void* c, const uint32_t* b, const void* bias, c
     return reduce(p);
   }
   int rc;
-  if (fp4 && global_scale != nullptr && wide_applies_fp4(p))
+  if (nvfp4)
     rc = dtype == SONAR_DTYPE_F16 ? launch_tile_wide_nvfp4<_Float16, true>(p, st)
                                   : launch_tile_wide_nvfp4<__bf16, true>(p, st);
-  else if (fp4 && global_scale != nullptr)
-    rc = dtype == SONAR_DTYPE_F16 ? launch_tile_async_nvfp4<_Float16, true>(p, st)
-                                  : launch_tile_async_nvfp4<__bf16, true>(p, st);
-  else if (fp4)
-    rc = wide_applies_fp4(p) ? launch_tile_wide_fp4<true>(p, st) : launch_tile_grouped_fp4(p, st);
-  else if (bits == 8 && wide_applies8(p))
+  else if (wide)   // 8-bit codes with groups of 32 rows
     rc = dtype == SONAR_DTYPE_F16 ? launch_tile_wide8<_Float16, true>(p, fp8, st)
                                   : launch_tile_wide8<__bf16, true>(p, fp8, st);
-  else if (bits == 8)
-    rc = dtype == SONAR_DTYPE_F16 ? launch_tile_async8<_Float16, true>(p, fp8, st)
-                                  : launch_tile_async8<__bf16, true>(p, fp8, st);
-  else if (wide_applies(p) && dtype == SONAR_DTYPE_F16)
-    rc = zeros ? launch_tile_wide<_Float16, true, true>(p, st) : launch_tile_wide<_Float16, false, true>(p, st);
-  else if (wide_applies(p))
-    rc = zeros ? launch_tile_wide<__bf16, true, true>(p, st) : launch_tile_wide<__bf16, false, true>(p, st);
-  else if (dtype == SONAR_DTYPE_F16)
-    rc = zeros ? launch_tile_grouped<_Float16, true>(p, st) : launch_tile_grouped<_Float16, false>(p, st);
   else
-    rc = zeros ? launch_tile_grouped<__bf16, true>(p, st) : launch_tile_grouped<__bf16, false>(p, st);
+    rc = launch_tile_async_type<true>(p, dtype, bits, st);
   if (rc) return rc;
   if (int rc2 = launch_status("tile kernel (grouped)")) return rc2;
   return reduce(p);
