@@ -1582,7 +1582,12 @@ bool moe_fast_applies(bool has_perm, int64_t moe_block_size, int64_t sorted_len,
   // slots 203 against 198, 994 slots 229 against 200 (with only the down GEMM here 197);
   // 1024 x 1408, 984 slots (88 and 32 tiles) 41 against 62.
   const int64_t tile_workgroups = num_experts * ((size_n + 255) / 256);
-  return sorted_len <= (tile_workgroups < cu_count() ? 1100 : shift == -4 ? 900 : 1000);
+  // Nine to sixteen experts and fewer tiles than compute units: up to about 60 rows an expert
+  // (us of a layer, tile kernel / here: 16 experts, AWQ, 2944 x 1024, 44 / 60 rows an expert 82 / 65 and 83 / 76; int4,
+  // 1024 x 10112, 50 rows 249 / 174; MXFP4, 2816 x 1024, 50 rows 79 / 68; 4096 x 1792, 60 rows level.  32 experts have twice
+  // the workgroups and lose: int4, 1792 x 896, 47 rows 69 / 78.)
+  if (tile_workgroups < cu_count()) return sorted_len <= (num_experts <= 16 ? std::max<int64_t>(1100, 125 * num_experts) : 1100);
+  return sorted_len <= (shift == -4 ? 900 : 1000);
 }
 
 // Called by sonar_moe_wna16_marlin_gemm when moe_fast_applies: one workgroup

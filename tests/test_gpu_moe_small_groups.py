@@ -30,3 +30,10 @@ def test_integer_codes_in_the_general_kernel(slots, dtype, zp, group):
 @pytest.mark.parametrize("k,n", [(512, 256), (1152, 4096), (192, 256)])
 def test_mxfp4(tokens, k, n):
     tm.test_full_size_grouped_gemm_agrees_with_dense_rows(tokens, k, n, "mxfp4")
+
+
+# sixteen experts in blocks of 64 slots, few strips: 1908 slots in the decode kernel, 2048 in the tile kernel
+@pytest.mark.parametrize("dtype,zp,group", [("fp16", True, 128), ("bf16", False, 32)])
+@pytest.mark.parametrize("tokens", [450, 520])
+def test_sixteen_experts(tokens, dtype, zp, group):
+    tm.test_moe_gemm_within_tolerance((tokens, 16, 2, 384, 192, group, dtype, zp, False, zp, 64, True))
