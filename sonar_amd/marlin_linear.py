@@ -35,13 +35,15 @@ def convert_awq_to_standard_format(layer, w_q_name: str = "qweight", w_zp_name: 
     layers/quantization/auto_awq.py:93-153): qweight (K, N/8), packed along N
     with AWQ's interleaved nibble order, becomes (K/8, N) packed along K in
     plain order; qzeros (G, N/8) in the same AWQ packing becomes (N/8, G),
-    packed along N in plain order and transposed."""
+    packed along N in plain order and transposed.  The result says so in
+    `input_dim` / `output_dim`, because its shape does not where G == N/8."""
     if size_bits != 4:
         raise NotImplementedError("AWQ conversion: 4-bit only")
     qw = getattr(layer, w_q_name)
     zeros = getattr(layer, w_zp_name)
     if qw.is_cuda and zeros.is_cuda and qw.dtype == zeros.dtype == torch.int32:
         codes, zeros = torch.ops.sonar_amd.awq_to_standard(qw.contiguous(), zeros.contiguous())
+        zeros.input_dim, zeros.output_dim = 1, 0
         setattr(layer, w_q_name, codes)
         setattr(layer, w_zp_name, zeros)
         return
@@ -56,7 +58,9 @@ def convert_awq_to_standard_format(layer, w_q_name: str = "qweight", w_zp_name: 
         return (q << plain[None, :, None]).sum(dim=1, dtype=torch.int32).contiguous()
 
     setattr(layer, w_q_name, pack_dim0(codes(qw)))
-    setattr(layer, w_zp_name, pack_dim0(codes(getattr(layer, w_zp_name)).t().contiguous()))
+    zeros = pack_dim0(codes(zeros).t().contiguous())
+    zeros.input_dim, zeros.output_dim = 1, 0
+    setattr(layer, w_zp_name, zeros)
 
 
 @dataclass
@@ -85,6 +89,15 @@ def _input_major(x: torch.Tensor, rows: int, cols: int) -> torch.Tensor:
         x = x.t()
     assert x.shape == (rows, cols), f"expected {(rows, cols)} or its transpose, got {tuple(x.shape)}"
     return x
+
+
+def _zero_points_are_transposed(zp: torch.Tensor, groups: int, size_n: int) -> bool:
+    """Whether zero points packed along N lie as (N/8, G) instead of (G, N/8).  Where both fit (G == N/8) what the
+    tensor says of itself (`input_dim`, `output_dim`) decides, without that (G, N/8)."""
+    if zp.shape != (size_n // 8, groups):
+        return False
+    input_dim, output_dim = getattr(zp, "input_dim", None), getattr(zp, "output_dim", None)
+    return groups != size_n // 8 or input_dim == 1 or (input_dim is None and output_dim == 0)
 
 
 class MarlinLinearKernel:
@@ -128,7 +141,7 @@ class MarlinLinearKernel:
         c = self.config
         grouped_k = size_k // c.group_size if c.group_size != -1 else 1
         padded_grouped_k = padded_k // c.group_size if c.group_size != -1 else 1
-        if zp.shape == (size_n // 8, grouped_k) and grouped_k != size_n // 8:
+        if _zero_points_are_transposed(zp, grouped_k, size_n):
             zp = zp.t().contiguous()      # packed along N and transposed (the converted AWQ form)
         if zp.shape == (grouped_k, size_n // 8):
             zp = unpack_cols(zp, c.weight_type.size_bits, grouped_k, size_n)
@@ -154,7 +167,7 @@ class MarlinLinearKernel:
         zeros, transposed = None, False
         if c.zero_points:
             zeros = getattr(layer, self.w_zp_name)
-            transposed = zeros.shape == (size_n // 8, groups) and groups != size_n // 8
+            transposed = _zero_points_are_transposed(zeros, groups, size_n)
             if (not transposed and zeros.shape != (groups, size_n // 8)) or (
                     zeros.dtype != torch.int32 or zeros.device != w_q.device or not zeros.is_contiguous()):
                 return False
@@ -208,7 +221,7 @@ class MarlinLinearKernel:
         if c.zero_points:
             grouped_k = size_k // c.group_size if c.group_size != -1 else 1
             zp = getattr(layer, self.w_zp_name)
-            transposed = zp.shape == (size_n // 8, grouped_k) and grouped_k != size_n // 8
+            transposed = _zero_points_are_transposed(zp, grouped_k, size_n)
             if ((transposed or zp.shape == (grouped_k, size_n // 8)) and (padded_n, padded_k) == (size_n, size_k)
                     and size_n % 64 == 0 and c.weight_type.size_bits == 4 and zp.is_cuda
                     and zp.dtype == torch.int32):
