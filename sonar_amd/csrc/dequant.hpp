@@ -483,6 +483,7 @@ struct Dq8F<__bf16> {
 // Nine (fp8) and seven instructions (integers) for four codes, beside 15 and 13 with the scale.  Rows as word4 above.
 template <bool FP8>
 struct Raw8 {   // v - 128: the code with its top bit turned is the number as a signed byte
+  static constexpr uint16_t kOne = 0x3f80;   // the scale bits for which Dq8<__bf16> leaves the code as it is
   static __device__ __forceinline__ float column_scale(uint16_t scale_bits) { return __uint_as_float((uint32_t)scale_bits << 16); }
   static __device__ __forceinline__ uint2 word4(uint32_t q) {
     // bytes 0..3 of a word are rows 0, 2, 1, 3
@@ -503,6 +504,7 @@ struct Dq8Of<T, true> {
 
 template <>
 struct Raw8<true> {   // the scale arrives times 2^120 (see Dq8F)
+  static constexpr uint16_t kOne = 0x7b80;
   static __device__ __forceinline__ float column_scale(uint16_t scale_bits) {
     return __uint_as_float((uint32_t)scale_bits << 16) * 0x1p-120f;
   }

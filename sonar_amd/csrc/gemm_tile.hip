@@ -962,6 +962,20 @@ constexpr int wide_lds(int rb) { return wide_a(rb) + 4 * kWideScaleRows * 256; }
 // k block), two chunks (8-bit codes: four blocks)
 constexpr int wide_ops(int rb, bool fp4 = false, bool w8 = false) { return rb / 2 + (fp4 ? 2 : 1) + (w8 ? 4 : 2); }
 
+// A scale row of ones in bf16: what 8-bit codes with one scale a column are dequantised with.  Every code is a bf16 number, so
+// the matrix cores get it exact and the column's scale goes into the fp32 sums, as in marlin_mid_gemm, between which and this
+// kernel the estimates choose.  (Error against 64 bits in units of the output's rounding, scaled weights rounded to bf16: 1.38
+// to 1.41, so: 1.00.  A row of ones instead of a form without scales: the same instructions in the loop, and no branch.)
+template <bool FP8>
+struct OnesRow {
+  uint16_t bits[kStripN];
+  constexpr OnesRow() : bits() {
+    for (int i = 0; i < kStripN; ++i) bits[i] = Raw8<FP8>::kOne;
+  }
+};
+__device__ __attribute__((aligned(128))) const OnesRow<false> kOnesInt8 = {};
+__device__ __attribute__((aligned(128))) const OnesRow<true> kOnesFp8 = {};
+
 // G32: a scale (and zero point) per 32 rows, i.e. one row of them per k block: MXFP4 always, integer codes when asked.
 // NV (with FP4): NVFP4, a scale per 16 rows: the row of a k block then holds two groups of 128 bytes (the copy
 // fetches one per half of the wavefront), and a lane, whose eight rows of a k block lie in one group, reads group
@@ -997,6 +1011,7 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
   const int kb = lane >> 4;
   const uint32_t magic = magic_register();
   const bool grouped = p.num_groups > 1;
+  constexpr bool kScaleSums = W8 != 0 && !G32 && std::is_same<T, __bf16>::value;   // with one group (OnesRow)
 
   // Grouped calls: row tile t is up to four consecutive 64-slot blocks of one expert, listed in
   // tile_table; rows are slots of sorted_ids (as in marlin_tile_async_kernel).
@@ -1043,6 +1058,8 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
     s_src = reinterpret_cast<const char*>(p.scales + expert * p.expert_s_stride + strip * kStripN) + 4 * (lane & 31);
     s_group_stride = (long)p.size_n * 2;
     if (NV) s_src += (lane >> 5) * s_group_stride;   // the upper half of the wavefront fetches the next group's row
+    if (kScaleSums && !grouped)
+      s_src = (W8 == 2 ? reinterpret_cast<const char*>(&kOnesFp8) : reinterpret_cast<const char*>(&kOnesInt8)) + 4 * (lane & 31);
   }
   // steps per group as a shift (the host checks: group_size = 64 * 2^i)
   const int group_shift = grouped ? 31 - __builtin_clz(p.group_size / kTileK) : 0;
@@ -1399,6 +1416,15 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
 #undef SONAR_WIDE_READ
 
   if (!active) return;
+  floatx4_t sum_scale[4];
+  if constexpr (kScaleSums) {
+    const uint16_t* row = p.scales + expert * p.expert_s_stride + strip * kStripN;
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        sum_scale[nb][r] = grouped ? 1.f : Raw8<W8 == 2>::column_scale(row[scale_slot(16 * nb + 4 * kb + r, false)]);
+  }
   if (partial_at >= 0) {
     // partial tile of this K range, in the order tile_reduce_kernel reads: 1-KiB blocks
     // (half of the rows, strip, column block, row block)
@@ -1408,7 +1434,7 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
 #pragma unroll
       for (int mb = 0; mb < RB; ++mb) {
         if (mb < kAgprBlocks) asm volatile("" : "+a"(acc[nb][mb]));   // still in its AGPRs here
-        const floatx4_t v = acc[nb][mb];
+        const floatx4_t v = kScaleSums ? acc[nb][mb] * sum_scale[nb] : acc[nb][mb];
         dst[((mb >> 3) * 128 + nb * 8 + (mb & 7)) * 64] = make_float4(v.x, v.y, v.z, v.w);
         __builtin_amdgcn_sched_barrier(0);   // one accumulator at a time leaves the AGPRs
       }
@@ -1458,7 +1484,7 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
     for (int nb = 0; nb < 4; ++nb) {
       if (mb < kAgprBlocks) asm volatile("" : "+a"(acc[nb][mb]));   // still in its AGPRs here
       if (c_row >= 0) {
-        const floatx4_t v = NV ? acc[nb][mb] * gs : acc[nb][mb];
+        const floatx4_t v = kScaleSums ? acc[nb][mb] * sum_scale[nb] : NV ? acc[nb][mb] * gs : acc[nb][mb];
         uint16_t o[4] = {Dq<T>::from_float(v.x + bias[nb][0]), Dq<T>::from_float(v.y + bias[nb][1]),
                          Dq<T>::from_float(v.z + bias[nb][2]), Dq<T>::from_float(v.w + bias[nb][3])};
         if (GROUPED && p.mul_topk) {
