@@ -490,6 +490,8 @@ int64_t sonar_debug_moe_tile_schedule(int64_t row_tiles, int64_t max_row_tiles, 
 int64_t sonar_debug_moe_pair_schedule(int64_t big, int64_t small, int64_t max_row_tiles, int64_t size_n,
                                       int64_t size_k, int with_partial, int32_t* chosen,
                                       int32_t* out, int64_t out_rows);
+/* What the choice between marlin_mid_gemm and the tile kernels takes the latter's time to be (us; 4-bit integer codes). */
+double sonar_debug_tile_estimate(int64_t size_m, int64_t size_n, int64_t size_k);
 
 #ifdef __cplusplus
 }

@@ -86,24 +86,32 @@ inline size_t plan_partial_bytes(const GemmPlan& plan, int64_t size_m, int64_t s
 // from 48 tiles on (measured at K = 14336, N = 4096, 128-row against 256-row tiles: M = 256:
 // 44.4 against 50.9 us; 384: 62.0 against 75.4; 512: 72.7 against 74.6; 768: 109 against 101;
 // 1024: 126 against 120).
-inline bool plan_prefers_128_rows(int64_t size_m, int64_t size_n, int64_t size_k, bool rows_97_128 = false) {
+inline bool plan_prefers_128_rows(int64_t size_m, int64_t size_n, int64_t size_k) {
   const int64_t tiles256 = ((size_m + 255) / 256) * ((size_n + 255) / 256);
   // up to 128 rows (calls that plan_gemm gives to the tile kernel at all: a long K, or rows_97_128) half of a
   // 256-row tile would be padding (K = 14336, N = 4096, M = 72 / 96 / 128: 47.3 / 47.8 / 49.0 -> 29.8 / 30.0 /
   // 30.0 us; K = 8192, N = 8192, M = 65 / 128: 54.4 / 52.9 -> 32.3 / 32.7)
-  (void)rows_97_128;
   if (size_m <= 128) return size_m > 64 && tiles256 <= 128;
   return tiles256 <= (size_k <= 8192 ? 128 : 32);
 }
 
+// What the tile kernels are launched with, given room for the partial tiles.  `rows128`: the call's format has 128-row tiles.
+inline GemmPlan tile_plan(int64_t size_m, int64_t size_n, int64_t size_k, bool rows128, bool rows_97_128) {
+  if (rows128 && plan_prefers_128_rows(size_m, size_n, size_k)) {
+    const GemmPlan plan = plan_gemm(size_m, size_n, size_k, true, 128, rows_97_128);
+    if (plan.tile) return plan;
+  }
+  return plan_gemm(size_m, size_n, size_k, true, 256, rows_97_128);
+}
+
 // Microseconds the tile kernels take: rounds of workgroups, each 11.2 us around its loop and `step` us per 64 rows of K for a
 // 256-row tile (0.58 of both for a 128-row one), 3.3 us for the launch, and for K in ranges a second launch and its bytes.  A fit
-// of 168 random calls of 220 to 8192 rows in all formats: 90 % within 14 % below and 13 % above.  `rows128`: the call's
-// format has 128-row tiles.
-inline double tile_estimate(int64_t size_m, int64_t size_n, int64_t size_k, double step, bool rows128) {
-  const bool small = rows128 && plan_prefers_128_rows(size_m, size_n, size_k);
-  const int64_t rows = small ? 128 : 256, steps = size_k / 64, tiles = ((size_m + rows - 1) / rows) * ((size_n + 255) / 256);
-  const GemmPlan plan = plan_gemm(size_m, size_n, size_k, true, (int)rows);
+// of 168 random calls of 220 to 8192 rows in all formats: 90 % within 14 % below and 13 % above.
+constexpr double kTileStepInt4 = 1.21;   // `step` of 4-bit integer codes
+inline double tile_estimate(int64_t size_m, int64_t size_n, int64_t size_k, double step, bool rows128, bool rows_97_128) {
+  const GemmPlan plan = tile_plan(size_m, size_n, size_k, rows128, rows_97_128);
+  const bool small = plan.tile_rows == 128;
+  const int64_t rows = plan.tile_rows, steps = size_k / 64, tiles = ((size_m + rows - 1) / rows) * ((size_n + 255) / 256);
   const double unit = small ? 0.58 : 1.0, whole = unit * (step * steps + 11.2);
   const double range = unit * (step * plan.k_steps_per_split + 11.2), sum = 1.1 + 1.24e-6 * plan.k_splits * size_m * size_n;
   if (plan.k_splits > 1 && plan.whole_tiles == 0) return 3.3 + (tiles * plan.k_splits + 255) / 256 * range + sum;

@@ -1884,8 +1884,9 @@ int marlin_gemm_any(const void* a, int64_t a_row_stride, void* c, const uint32_t
     if (slab_fast) {
       us = decode_rows_estimate(size_m, n_strips, size_k, chk.has_zp, cus);
     } else if (use_tile) {
-      const double step = chk.bits == 8 ? 1.27 : chk.nvfp4 ? 1.30 : chk.fp4 ? 1.14 : 1.21;
-      us = tile_estimate(size_m, size_n, size_k, step, !chk.nvfp4 && !(chk.bits == 8 && num_groups > 1 && chk.group_size == 32));
+      const double step = chk.bits == 8 ? 1.27 : chk.nvfp4 ? 1.30 : chk.fp4 ? 1.14 : kTileStepInt4;
+      us = tile_estimate(size_m, size_n, size_k, step, !chk.nvfp4 && !(chk.bits == 8 && num_groups > 1 && chk.group_size == 32),
+                         rows_97_128);
       // what mid_estimate lacks, with K in one piece, on the calls tile_estimate was fitted to (a time that grows with the operations alone, and 0.93 for
       // either kernel: 2.7 % slower than the better of the two on 147 random calls, at worst 1.6 times; so 0.6 %, 1.3 times)
       static const double kSlow[6][2] = {{1.12, 1.10}, {1.18, 1.10}, {1.30, 1.12}, {1.13, 1.05}, {1.22, 1.22}, {1.03, 1.0}};

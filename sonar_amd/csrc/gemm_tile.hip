@@ -1969,24 +1969,24 @@ TileLaunches plan_tile_launches(TileParams p, int64_t size_m, int64_t size_n, in
   const bool wide128 = bits == 4 && !fp4 && !has_perm &&
                        (num_groups == 1 || (group_size % kTileK == 0 && (steps_per_group & (steps_per_group - 1)) == 0));
   const bool rows_97_128 = plan_rows_97_128(size_m, size_n, size_k, wide128);
-  GemmPlan plan = plan_gemm(size_m, size_n, size_k, true, 256, rows_97_128);
   // few tiles and a call the wide kernel takes: 128-row tiles
   static const bool no_128 = getenv("SONAR_MARLIN_NO_128_ROW_TILES") != nullptr;   // debugging aid
   // (not for NVFP4 and 8-bit codes with groups of 32 rows, whose heavier dequantisation wants the 16 row blocks
   // to hide behind: M = 512, K = 4096, N = 11008: NVFP4 69.9 us against 68.7, MXFP8 91.8 against 82.2)
   const bool rows128_ok = !nvfp4 && !(bits == 8 && num_groups > 1 && group_size == 32);
-  if (!no_128 && rows128_ok && plan_prefers_128_rows(size_m, size_n, size_k, rows_97_128)) {
-    const GemmPlan plan128 = plan_gemm(size_m, size_n, size_k, true, 128, rows_97_128);
+  GemmPlan plan = tile_plan(size_m, size_n, size_k, rows128_ok && !no_128, rows_97_128);
+  if (plan.tile_rows == 128) {
     TileParams probe = p;
     probe.tile_rows = 128;
-    probe.k_splits = plan128.k_splits;
-    probe.k_steps_per_split = plan128.k_steps_per_split;
-    if (plan128.tile && (fp4 ? wide_applies_fp4(probe) : wide_applies(probe)) &&
-        (plan128.k_splits == 1 || (partial != nullptr && partial_bytes >= plan_partial_bytes(plan128, size_m, size_n)))) {
-      plan = plan128;
+    probe.k_splits = plan.k_splits;
+    probe.k_steps_per_split = plan.k_steps_per_split;
+    if ((fp4 ? wide_applies_fp4(probe) : wide_applies(probe)) &&
+        (plan.k_splits == 1 || (partial != nullptr && partial_bytes >= plan_partial_bytes(plan, size_m, size_n)))) {
       p.tile_rows = 128;
       p.tiles_m = (int)((size_m + 127) / 128);
       p.tile_band = 8;   // the same rows of A per band as four 256-row tiles
+    } else {
+      plan = tile_plan(size_m, size_n, size_k, false, rows_97_128);
     }
   }
   if (plan.k_splits > 1 && partial != nullptr && partial_bytes >= plan_partial_bytes(plan, size_m, size_n)) {
@@ -2293,6 +2293,12 @@ int64_t pair_schedule_rows(const sonar::TileParams& p, int big_word, int small_w
   return at;
 }
 }  // namespace
+
+// What the choice between the mid-size and the tile kernels takes the latter's time to be, in us, for 4-bit integer codes.
+extern "C" double sonar_debug_tile_estimate(int64_t size_m, int64_t size_n, int64_t size_k) {
+  using namespace sonar;
+  return tile_estimate(size_m, size_n, size_k, kTileStepInt4, true, plan_rows_97_128(size_m, size_n, size_k, true));
+}
 
 // A dense call (4-bit integer codes, no act-order) with room for every partial tile.
 extern "C" int64_t sonar_debug_tile_schedule(int64_t size_m, int64_t size_n, int64_t size_k, int64_t num_groups,
