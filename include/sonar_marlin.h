@@ -492,6 +492,10 @@ int64_t sonar_debug_moe_pair_schedule(int64_t big, int64_t small, int64_t max_ro
                                       int32_t* out, int64_t out_rows);
 /* What the choice between marlin_mid_gemm and the tile kernels takes the latter's time to be (us; 4-bit integer codes). */
 double sonar_debug_tile_estimate(int64_t size_m, int64_t size_n, int64_t size_k);
+/* Which of the two that choice falls on (1: marlin_mid_gemm) for a call of more than 64 rows that either could run, integer or
+ * fp8 codes, 256 compute units; -1 for arguments out of range. */
+int sonar_debug_mid_beats_tiles(int64_t size_m, int64_t size_n, int64_t size_k, int64_t num_groups, int dtype,
+                                int64_t b_type_id);
 
 #ifdef __cplusplus
 }

@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "gemm_plan.hpp"
+
 namespace sonar {
 
 // Weight formats of the kernel in gemm_mid.hip.
@@ -79,6 +81,30 @@ inline double mid_estimate(int64_t size_m, int64_t size_n, int64_t size_k, int64
     }
   }
   return best;
+}
+
+// Whether a call that the tile kernels could take runs in this kernel, whose time mid_estimate puts at `mid_us`, with K in
+// `splits` ranges.
+// What mid_estimate lacks on the calls tile_estimate was fitted to, with K in one piece: kSlow.  (A time of the tile kernels that
+// grows with the operations alone, and 0.93 for either kernel: 2.7 % slower than the better of the two on 147 random calls, at
+// worst 1.6 times; so 0.6 %, 1.3 times.)
+// 8-bit codes with one scale a column in bf16 have factors of their own: this kernel multiplies them unscaled, with fewer
+// instructions than mid_estimate's fit of all 8-bit codes, and the tile kernels take longer for fp8 codes in bf16 than
+// tile_estimate has it (199 random calls of 65 to 3000 rows: slower than the better of the two by 5.6 % (fp8) and 1.4 % (integers),
+// at worst 1.5 times, with the other formats' factors; so 0.3 % and 0.5 %, 1.17 times.  Us, before -> now: fp8, M = 271,
+// K = 6144, N = 6400 51.4 -> 34.9; M = 134, K = 3968, N = 26240 71.8 -> 53.0; integers, M = 196, K = 1664, N = 11392
+// 29.9 -> 24.0).
+inline bool mid_beats_tiles(double mid_us, int splits, int64_t size_m, int64_t size_n, int64_t size_k, int64_t num_groups,
+                            int group_size, bool float16, int format, bool rows_97_128) {
+  static const double kStep[6] = {kTileStepInt4, kTileStepInt4, 1.27, 1.27, 1.14, 1.30};
+  static const double kSlow[6][2] = {   // float16, bfloat16
+      {1.12, 1.10}, {1.18, 1.10}, {1.30, 1.12}, {1.13, 1.05}, {1.22, 1.22}, {1.03, 1.0}};
+  const bool is_8bit = format == kMidInt8 || format == kMidFp8, groups_of_32 = num_groups > 1 && group_size == 32;
+  if (is_8bit && num_groups == 1 && !float16) mid_us *= format == kMidFp8 ? 0.77 : 0.92;
+  else if (splits > 1) mid_us *= 0.94;
+  else mid_us *= format == kMidFp8 && groups_of_32 ? 0.97 : kSlow[format][float16 ? 0 : 1];
+  const bool rows128 = format != kMidNvFp4 && !(is_8bit && groups_of_32);
+  return mid_us < tile_estimate(size_m, size_n, size_k, kStep[format], rows128, rows_97_128);
 }
 
 // Up to 16 rows of 8-bit codes or NVFP4, which the decode kernel does not have: into how many parts K is split, in

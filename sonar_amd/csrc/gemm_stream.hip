@@ -1878,22 +1878,16 @@ int marlin_gemm_any(const void* a, int64_t a_row_stride, void* c, const uint32_t
       splits = mid_splits_16_rows(size_n, size_k, cus);
       if ((size_t)splits * size_m * size_n * 4 > base_scratch) splits = 1;
     }
-    const double x = (double)size_n * size_k / (6144.0 * 4096.0), r = size_m / 64.0;
-    // (what the other kernels take, us: fits of measured times, see mid_estimate)
-    double us;
+    bool take;
     if (slab_fast) {
-      us = decode_rows_estimate(size_m, n_strips, size_k, chk.has_zp, cus);
+      take = mid_us < decode_rows_estimate(size_m, n_strips, size_k, chk.has_zp, cus);
     } else if (use_tile) {
-      const double step = chk.bits == 8 ? 1.27 : chk.nvfp4 ? 1.30 : chk.fp4 ? 1.14 : kTileStepInt4;
-      us = tile_estimate(size_m, size_n, size_k, step, !chk.nvfp4 && !(chk.bits == 8 && num_groups > 1 && chk.group_size == 32),
-                         rows_97_128);
-      // what mid_estimate lacks, with K in one piece, on the calls tile_estimate was fitted to (a time that grows with the operations alone, and 0.93 for
-      // either kernel: 2.7 % slower than the better of the two on 147 random calls, at worst 1.6 times; so 0.6 %, 1.3 times)
-      static const double kSlow[6][2] = {{1.12, 1.10}, {1.18, 1.10}, {1.30, 1.12}, {1.13, 1.05}, {1.22, 1.22}, {1.03, 1.0}};
-      if (splits > 1) mid_us *= 0.94;
-      else mid_us *= format == kMidFp8 && num_groups > 1 && chk.group_size == 32 ? 0.97 : kSlow[format][dtype == SONAR_DTYPE_F16 ? 0 : 1];
-    } else {   // (few strips: shared between workgroups, and a second launch that adds the shares)
-      us = size_m <= 64 ? (n_strips < 64 ? 12.0 : 9.5) + x * (5.5 + 5.2 * r * r) : 11.0 + 10.7 * x * r;
+      take = mid_beats_tiles(mid_us, splits, size_m, size_n, size_k, num_groups, chk.group_size, dtype == SONAR_DTYPE_F16, format,
+                             rows_97_128);
+    } else {   // (the general kernels, us: a fit of measured times; few strips: shared between workgroups, and a second launch)
+      const double x = (double)size_n * size_k / (6144.0 * 4096.0), r = size_m / 64.0;
+      const double us = size_m <= 64 ? (n_strips < 64 ? 12.0 : 9.5) + x * (5.5 + 5.2 * r * r) : 11.0 + 10.7 * x * r;
+      take = mid_us < (raw_codes ? 1.0 : 0.93) * us;
     }
     if (mid_env) {   // "row blocks" or "row blocks,splits"
       const char* comma = strchr(mid_env, ',');
@@ -1901,7 +1895,7 @@ int marlin_gemm_any(const void* a, int64_t a_row_stride, void* c, const uint32_t
       splits = comma ? std::max(1, std::min(kMidMostSplits, atoi(comma + 1))) : 1;
       if ((size_t)splits * size_m * size_n * 4 > base_scratch || splits > size_k / 64) splits = 1;
     }
-    if (mid_env || mid_us < (raw_codes || use_tile ? 1.0 : 0.93) * us) {
+    if (mid_env || take) {
       MidParams q = {};
       q.a = static_cast<const uint16_t*>(a);
       q.lda = a_row_stride;
@@ -2073,6 +2067,19 @@ extern "C" int sonar_marlin_last_decode_launch(int32_t* out, int n) {
   int i = 0;
   for (; out != nullptr && i < n && i < 4; ++i) out[i] = g_last_decode_launch[i];
   return i;
+}
+
+extern "C" int sonar_debug_mid_beats_tiles(int64_t size_m, int64_t size_n, int64_t size_k, int64_t num_groups, int dtype,
+                                           int64_t b_type_id) {
+  if (size_m <= 64 || size_n <= 0 || size_k <= 0 || num_groups < 1) return -1;
+  const int format = b_type_id == SONAR_TYPE_FLOAT8_E4M3FN ? kMidFp8 : b_type_id == SONAR_TYPE_UINT8B128 ? kMidInt8
+                     : b_type_id == SONAR_TYPE_UINT4 ? kMidInt4Zp : b_type_id == SONAR_TYPE_UINT4B8 ? kMidInt4 : -1;
+  if (format < 0) return -1;
+  int row_blocks, splits;
+  const double us = mid_estimate(size_m, size_n, size_k, num_groups, dtype, format, false, 256,
+                                 sonar_marlin_gemm_scratch_bytes(size_m, size_n, size_k), row_blocks, splits);
+  return mid_beats_tiles(us, splits, size_m, size_n, size_k, num_groups, (int)(size_k / num_groups), dtype == SONAR_DTYPE_F16, format,
+                         plan_rows_97_128(size_m, size_n, size_k, format == kMidInt4 || format == kMidInt4Zp)) ? 1 : 0;
 }
 
 extern "C" int sonar_marlin_gemm(const void* a, int64_t a_row_stride, void* c,

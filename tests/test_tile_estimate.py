@@ -41,3 +41,19 @@ def test_random_shapes():
             seen += 1
             assert _lib.load().sonar_debug_tile_estimate(m, n, k) == pytest.approx(want, rel=1e-6), (m, n, k)
     assert seen > 200
+
+
+# us in marlin_mid_gemm and in the tile kernels: one of the two at least a sixth faster
+@pytest.mark.parametrize("code,dtype,group,m,k,n,mid,tile", [
+    ("fp8", "bf16", -1, 271, 6144, 6400, 34.9, 51.2), ("fp8", "bf16", -1, 134, 3968, 26240, 53.0, 70.5),
+    ("fp8", "bf16", -1, 504, 4480, 2752, 25.9, 34.4), ("fp8", "bf16", -1, 1270, 6656, 1472, 34.9, 46.4),
+    ("fp8", "bf16", -1, 818, 3840, 5376, 51.9, 67.4), ("fp8", "bf16", -1, 274, 8832, 15104, 97.8, 129.1),
+    ("uint8b128", "bf16", -1, 196, 1664, 11392, 24.0, 31.2), ("uint8b128", "bf16", -1, 123, 8832, 16128, 42.5, 48.9),
+    ("uint8b128", "bf16", -1, 207, 7296, 8448, 39.3, 49.3), ("uint8b128", "bf16", -1, 125, 13440, 17472, 104.8, 77.2),
+    ("uint8b128", "fp16", 128, 122, 13056, 22016, 130.6, 104.7), ("uint8b128", "fp16", 128, 203, 4352, 10688, 28.7, 37.7),
+    ("uint4", "fp16", 64, 113, 6656, 16640, 60.8, 45.1), ("uint4b8", "bf16", -1, 187, 5888, 10304, 30.7, 44.7)])
+def test_choice_between_the_mid_size_and_the_tile_kernels(code, dtype, group, m, k, n, mid, tile):
+    types = {"fp8": _lib.TYPE_FLOAT8_E4M3FN, "uint8b128": _lib.TYPE_UINT8B128, "uint4": _lib.TYPE_UINT4, "uint4b8": _lib.TYPE_UINT4B8}
+    dtypes = {"fp16": _lib.DTYPE_F16, "bf16": _lib.DTYPE_BF16}
+    chosen = _lib.load().sonar_debug_mid_beats_tiles(m, n, k, 1 if group == -1 else k // group, dtypes[dtype], types[code])
+    assert chosen == int(mid < tile)
