@@ -1725,6 +1725,7 @@ __global__ __launch_bounds__(64 * kTableWaves) void moe_tile_table_kernel(const 
   // two sizes: the tiles are counted first and written when it is known which are halved
   Tile t = {};
   for (int base = 0; base < blocks; base += kTableThreads) t = scan(base);
+  __syncthreads();   // `best` is set (scan() has barriers of its own, but there may be no block)
   const int big = count[0], small = count[1], plans = pair_plans(big, may_split);
   for (int i = threadIdx.x; i < plans; i += kTableThreads) {
     const PairPlan plan = pair_plan(i, big, may_split);
