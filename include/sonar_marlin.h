@@ -472,8 +472,9 @@ int sonar_moe_activation(void* out, const void* in, int64_t rows, int64_t d, int
 
 /* Diagnostics for host-side tests; no counterpart in the reference.  The tile kernels'
  * launches for a dense call (4-bit integer codes, no act-order, room for every partial
- * tile), or for a grouped call whose routing made `row_tiles` row tiles of `tile_rows`
- * rows out of at most `max_row_tiles`: one row of six int32 per workgroup that has
+ * tile), or for a grouped call of one tile size (256 rows: NVFP4, and 8-bit codes with
+ * groups of 32 rows) whose routing made `row_tiles` row tiles out of at most
+ * `max_row_tiles`: one row of six int32 per workgroup that has
  * work (launch, rows of a tile, row tile, column tile, first K step, end of its K
  * steps), from the planning and mapping code the launches and the kernels run.
  * Returns the number of such workgroups (rows beyond out_rows are counted, not
@@ -481,8 +482,7 @@ int sonar_moe_activation(void* out, const void* in, int64_t rows, int64_t d, int
 int64_t sonar_debug_tile_schedule(int64_t size_m, int64_t size_n, int64_t size_k,
                                   int64_t num_groups, int32_t* out, int64_t out_rows);
 int64_t sonar_debug_moe_tile_schedule(int64_t row_tiles, int64_t max_row_tiles, int64_t size_n,
-                                      int64_t size_k, int tile_rows, int with_partial,
-                                      int32_t* out, int64_t out_rows);
+                                      int64_t size_k, int with_partial, int32_t* out, int64_t out_rows);
 /* The same for a grouped call that runs both tile sizes in one launch, whose routing made `big`
  * row tiles of three or four blocks and `small` of one or two: launch 0 are the 256-row tiles,
  * launch 1 the 128-row ones.  chosen: the 256-row tiles that are halved, and the K ranges of

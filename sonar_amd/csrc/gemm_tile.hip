@@ -168,7 +168,7 @@ __host__ __device__ __forceinline__ LiveSplit plan_live_split(int tiles, int k_s
 __host__ __device__ __forceinline__ TileParams live_tiles_of(const TileParams& p, int row_tiles) {
   TileParams live = p;
   live.tiles_m = row_tiles;
-  live.tile_band = p.tile_rows == kTileM ? 4 : 8;   // the same rows of A per band with either tile size
+  live.tile_band = 4;
   if (p.partial != nullptr) {
     const LiveSplit s = plan_live_split(live.tiles_m * live.tiles_n, p.size_k / kTileK);
     live.k_splits = s.splits;
@@ -2316,19 +2316,15 @@ extern "C" int64_t sonar_debug_tile_schedule(int64_t size_m, int64_t size_n, int
   return pair_schedule_rows(plan.launch, 0, 0, pair_grid(plan.launch, 0), out, out_rows);
 }
 
-// A grouped call whose routing made `row_tiles` row tiles of `tile_rows` rows, launched for up to
+// A grouped call of one tile size whose routing made `row_tiles` row tiles, launched for up to
 // `max_row_tiles` of them; `with_partial`: the call has room for partial tiles.
 extern "C" int64_t sonar_debug_moe_tile_schedule(int64_t row_tiles, int64_t max_row_tiles, int64_t size_n,
-                                                 int64_t size_k, int tile_rows, int with_partial, int32_t* out,
-                                                 int64_t out_rows) {
+                                                 int64_t size_k, int with_partial, int32_t* out, int64_t out_rows) {
   using namespace sonar;
-  if (row_tiles < 0 || row_tiles > max_row_tiles || size_n <= 0 || size_k <= 0 || size_k % kTileK != 0 ||
-      (tile_rows != kTileM && tile_rows != 128))
-    return -1;
+  if (row_tiles < 0 || row_tiles > max_row_tiles || size_n <= 0 || size_k <= 0 || size_k % kTileK != 0) return -1;
   static float4 never_read;
   static int32_t no_table;
-  TileParams p = dense_tile_shape(max_row_tiles * tile_rows, size_n, size_k, 1, (int)size_k);
-  p.tile_rows = tile_rows;
+  TileParams p = dense_tile_shape(max_row_tiles * kTileM, size_n, size_k, 1, (int)size_k);
   p.tiles_m = (int)max_row_tiles;
   p.tile_table = &no_table;
   if (with_partial && moe_tile_partial_bytes(size_k) > 0) p.partial = &never_read;
