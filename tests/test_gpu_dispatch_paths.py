@@ -28,11 +28,10 @@ SWITCHES = [
     "SONAR_MARLIN_NO_128_ROW_TILES", # the wide tile kernel with 256-row tiles only
     "SONAR_MARLIN_NO_ASYNC_TILE",    # the register-staged tile kernel
     "SONAR_MARLIN_MAX_K_SPLITS=1",   # no split K in the tile kernel
-    "SONAR_MARLIN_NO_TWO_TILE_SIZES",  # a short last round of tiles cut along K instead of a second launch of 128-row tiles
+    "SONAR_MARLIN_NO_TWO_TILE_SIZES",  # a short last round of tiles cut along K instead of halved into 128-row tiles
     "SONAR_MARLIN_NO_MOE_TILE",      # the grouped streaming kernel for 64-slot blocks
     "SONAR_MARLIN_NO_MOE_FAST",      # ... and for blocks of up to 32 slots
     "SONAR_MARLIN_NO_MOE_K_SPLIT",   # the grouped wide tile kernel never cuts its tiles along K
-    "SONAR_MARLIN_NO_MOE_128_ROW_TILES",   # ... and computes the short ends of the experts' rows as 256-row tiles
     "SONAR_MARLIN_NO_MOE_PERMUTED_COPY",   # act-order experts: the gathering kernel although scratch has room
 ]
 

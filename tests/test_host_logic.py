@@ -241,27 +241,42 @@ def test_kernels_with_hand_counted_waits_do_not_spill():
     if not os.path.exists(hipcc):
         pytest.skip("hipcc not available")
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-    watched = [("gemm_tile.hip", "marlin_tile_async_kernel"), ("gemm_tile.hip", "marlin_tile_wide_kernel"),
-               ("gemm_stream.hip", "marlin_stream_fast_kernel")]
-    for src, kernel in watched:
+    watched = {"gemm_tile.hip": ["marlin_tile_async_kernel", "marlin_tile_wide_kernel", "marlin_tile_wide_pair_kernel"],
+               "gemm_stream.hip": ["marlin_stream_fast_kernel"]}
+    for src, kernels in watched.items():
         out = subprocess.run(
             [hipcc, "-O3", "--offload-arch=gfx950", "-std=c++17", "-Xclang", "-target-feature", "-Xclang",
              "-packed-fp32-ops", "-I", os.path.join(root, "include"), "-I", os.path.join(root, "sonar_amd", "csrc"),
              "-c", "--offload-device-only", "-Rpass-analysis=kernel-resource-usage",
              os.path.join(root, "sonar_amd", "csrc", src), "-o", os.devnull],
-            capture_output=True, text=True, timeout=600)
+            capture_output=True, text=True, timeout=900)
         assert out.returncode == 0, out.stderr[-2000:]
         name = None
-        seen = 0
+        seen = dict.fromkeys(kernels, 0)
         for line in out.stderr.splitlines():
             m = re.search(r"Function Name: (\S+)", line)
             if m:
                 name = m.group(1)
             m = re.search(r"VGPRs Spill: (\d+)", line)
-            if m and name and kernel in name:
-                seen += 1
-                assert int(m.group(1)) == 0, f"{name} spills {m.group(1)} VGPRs"
-        assert seen >= 4, f"no resource report for {kernel}"
+            if m and name:
+                for kernel in kernels:
+                    if kernel in name:
+                        seen[kernel] += 1
+                        assert int(m.group(1)) == 0, f"{name} spills {m.group(1)} VGPRs"
+        assert min(seen.values()) >= 4, f"no resource report for some of {seen}"
+
+
+def test_switches_of_the_dispatch_tests_exist():
+    """A switch that the library does not read would run the default path under another name."""
+    import glob
+    import re
+
+    from tests import test_gpu_dispatch_paths
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    sources = "".join(open(f).read() for f in glob.glob(os.path.join(root, "sonar_amd", "csrc", "*.h*")))
+    read = set(re.findall(r'getenv\("(\w+)"\)', sources))
+    for switch in filter(None, test_gpu_dispatch_paths.SWITCHES):
+        assert switch.partition("=")[0] in read, switch
 
 
 KERNEL_FORMS = {
