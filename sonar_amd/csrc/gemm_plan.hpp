@@ -104,10 +104,11 @@ inline GemmPlan tile_plan(int64_t size_m, int64_t size_n, int64_t size_k, bool r
   return plan_gemm(size_m, size_n, size_k, true, 256, rows_97_128);
 }
 
+constexpr double kTileStepInt4 = 1.21;   // tile_estimate's `step` of 4-bit integer codes
+
 // Microseconds the tile kernels take: rounds of workgroups, each 11.2 us around its loop and `step` us per 64 rows of K for a
 // 256-row tile (0.58 of both for a 128-row one), 3.3 us for the launch, and for K in ranges a second launch and its bytes.  A fit
 // of 168 random calls of 220 to 8192 rows in all formats: 90 % within 14 % below and 13 % above.
-constexpr double kTileStepInt4 = 1.21;   // `step` of 4-bit integer codes
 inline double tile_estimate(int64_t size_m, int64_t size_n, int64_t size_k, double step, bool rows128, bool rows_97_128) {
   const GemmPlan plan = tile_plan(size_m, size_n, size_k, rows128, rows_97_128);
   const bool small = plan.tile_rows == 128;

@@ -9,7 +9,7 @@
 // are dealt round-robin to the workgroup's wavefronts; each wavefront keeps
 // MB x 4 accumulator tiles (16 rows x 16 columns) and feeds
 // v_mfma_f32_16x16x32 with the dequantised weights as the row operand and the
-// activations as the column operand.  At the end of every strip segment the
+// activations as the column operand (marlin_stream_fast_kernel: integers, and the other way round).  At the end of every strip segment the
 // wavefronts' tiles are summed through LDS.  A segment that covers the whole K
 // of its strip is rounded and written to C.  A partial segment is written as
 // an fp32 tile to scratch memory; a second, tiny kernel adds the (two to five)

@@ -135,12 +135,14 @@ class MarlinLinearKernel:
                            f"by group_size = {c.group_size}.")
         return True, None
 
+    def _num_groups(self, size_k: int) -> int:
+        return 1 if self.config.group_size == -1 else size_k // self.config.group_size
+
     def _zero_points_by_torch(self, zp: torch.Tensor, size_n: int, size_k: int, padded_n: int, padded_k: int,
                               is_a_8bit: bool) -> torch.Tensor:
         """Zero points that are unpacked, need padding or are not on the GPU."""
         c = self.config
-        grouped_k = size_k // c.group_size if c.group_size != -1 else 1
-        padded_grouped_k = padded_k // c.group_size if c.group_size != -1 else 1
+        grouped_k, padded_grouped_k = self._num_groups(size_k), self._num_groups(padded_k)
         if _zero_points_are_transposed(zp, grouped_k, size_n):
             zp = zp.t().contiguous()      # packed along N and transposed (the converted AWQ form)
         if zp.shape == (grouped_k, size_n // 8):
@@ -158,7 +160,7 @@ class MarlinLinearKernel:
                 or hasattr(self, "workspace")):
             return False
         w_q, w_s = getattr(layer, self.w_q_name), getattr(layer, self.w_s_name)
-        groups = 1 if c.group_size == -1 else size_k // c.group_size
+        groups = self._num_groups(size_k)
         if (groups < 1 or w_q.dtype != torch.int32 or w_q.shape != (size_k // 8, size_n) or w_s.shape != (groups, size_n)
                 or w_s.element_size() != 2 or not w_s.is_floating_point() or w_s.requires_grad or not w_q.is_cuda
                 or w_s.device != w_q.device or not w_q.is_contiguous() or not w_s.is_contiguous()
@@ -219,7 +221,7 @@ class MarlinLinearKernel:
             layer.g_idx_sort_indices = marlin_make_empty_g_idx(device)
 
         if c.zero_points:
-            grouped_k = size_k // c.group_size if c.group_size != -1 else 1
+            grouped_k = self._num_groups(size_k)
             zp = getattr(layer, self.w_zp_name)
             transposed = _zero_points_are_transposed(zp, grouped_k, size_n)
             if ((transposed or zp.shape == (grouped_k, size_n // 8)) and (padded_n, padded_k) == (size_n, size_k)
@@ -247,7 +249,7 @@ class MarlinLinearKernel:
         w_s = marlin_permute_scales(
             marlin_pad_scales(w_s.contiguous(), size_n, size_k, padded_n, padded_k, c.group_size),
             size_k=padded_k, size_n=padded_n, group_size=c.group_size, is_a_8bit=is_a_8bit)
-        num_groups = 1 if c.group_size == -1 else size_k // c.group_size
+        num_groups = self._num_groups(size_k)
         layer.input_global_scale = None
         if c.act_type == torch.int8 and num_groups > 1:   # marlin.py:156-163
             w_s, input_global_scale = marlin_act_int8_process_scales(w_s)
