@@ -91,13 +91,18 @@ def _input_major(x: torch.Tensor, rows: int, cols: int) -> torch.Tensor:
     return x
 
 
-def _zero_points_are_transposed(zp: torch.Tensor, groups: int, size_n: int) -> bool:
+def _zero_points_are_transposed(zp: torch.Tensor, scales: torch.Tensor, groups: int, size_n: int) -> bool:
     """Whether zero points packed along N lie as (N/8, G) instead of (G, N/8).  Where both fit (G == N/8) what the
-    tensor says of itself (`input_dim`, `output_dim`) decides, without that (G, N/8)."""
+    tensor says of itself (`input_dim`, `output_dim`) decides; without that they lie as the scales do, which
+    compressed-tensors checkpoints hold as (N, G)."""
     if zp.shape != (size_n // 8, groups):
         return False
+    if groups != size_n // 8:
+        return True
     input_dim, output_dim = getattr(zp, "input_dim", None), getattr(zp, "output_dim", None)
-    return groups != size_n // 8 or input_dim == 1 or (input_dim is None and output_dim == 0)
+    if input_dim is None and output_dim is None:
+        return scales.shape == (size_n, groups)
+    return input_dim == 1 or (input_dim is None and output_dim == 0)
 
 
 class MarlinLinearKernel:
@@ -140,11 +145,9 @@ class MarlinLinearKernel:
 
     def _zero_points_by_torch(self, zp: torch.Tensor, size_n: int, size_k: int, padded_n: int, padded_k: int,
                               is_a_8bit: bool) -> torch.Tensor:
-        """Zero points that are unpacked, need padding or are not on the GPU."""
+        """Zero points that are unpacked, need padding or are not on the GPU; packed ones as (G, N/8)."""
         c = self.config
         grouped_k, padded_grouped_k = self._num_groups(size_k), self._num_groups(padded_k)
-        if _zero_points_are_transposed(zp, grouped_k, size_n):
-            zp = zp.t().contiguous()      # packed along N and transposed (the converted AWQ form)
         if zp.shape == (grouped_k, size_n // 8):
             zp = unpack_cols(zp, c.weight_type.size_bits, grouped_k, size_n)
         zp = marlin_pad_scales(zp, size_n, size_k, padded_n, padded_k, c.group_size)
@@ -169,7 +172,7 @@ class MarlinLinearKernel:
         zeros, transposed = None, False
         if c.zero_points:
             zeros = getattr(layer, self.w_zp_name)
-            transposed = _zero_points_are_transposed(zeros, groups, size_n)
+            transposed = _zero_points_are_transposed(zeros, w_s, groups, size_n)
             if (not transposed and zeros.shape != (groups, size_n // 8)) or (
                     zeros.dtype != torch.int32 or zeros.device != w_q.device or not zeros.is_contiguous()):
                 return False
@@ -223,12 +226,13 @@ class MarlinLinearKernel:
         if c.zero_points:
             grouped_k = self._num_groups(size_k)
             zp = getattr(layer, self.w_zp_name)
-            transposed = _zero_points_are_transposed(zp, grouped_k, size_n)
+            transposed = _zero_points_are_transposed(zp, getattr(layer, self.w_s_name), grouped_k, size_n)
             if ((transposed or zp.shape == (grouped_k, size_n // 8)) and (padded_n, padded_k) == (size_n, size_k)
                     and size_n % 64 == 0 and c.weight_type.size_bits == 4 and zp.is_cuda
                     and zp.dtype == torch.int32):
                 zp = torch.ops.sonar_amd.pack_zero_points(zp.contiguous(), False, transposed, is_a_8bit)
             else:
+                zp = zp.t().contiguous() if transposed else zp
                 zp = self._zero_points_by_torch(zp, size_n, size_k, padded_n, padded_k, is_a_8bit)
             setattr(layer, self.w_zp_name, zp)
         else:

@@ -26,13 +26,17 @@ def _converted(k, n, group, device):
 
 
 @pytest.mark.parametrize("k,n,group", SQUARE + [(1024, 256, 64), (256, 192, 64)])
-def test_general_path(k, n, group):
+def test_orientation(k, n, group):
     layer, kernel, want = _converted(k, n, group, "cpu")
-    assert torch.equal(kernel._zero_points_by_torch(layer.qzeros, n, k, n, k, False), want)
-    # without a mark a tensor that fits both ways is (G, N/8), as before there was one
-    plain = mu.pack_cols(torch.arange(k // group * n, dtype=torch.int32).reshape(k // group, n) % 16, 4, k // group, n)
-    codes = mu.unpack_cols(plain, 4, k // group, n)
-    assert torch.equal(kernel._zero_points_by_torch(plain, n, k, n, k, False), mu.marlin_zero_points(codes, k // group, n, 4))
+    groups = k // group
+    assert ml._zero_points_are_transposed(layer.qzeros, layer.scales, groups, n)
+    assert torch.equal(kernel._zero_points_by_torch(layer.qzeros.t().contiguous(), n, k, n, k, False), want)
+    # without a mark a tensor that fits both ways lies as the scales do: (G, N/8) in GPTQ's layout, (N/8, G) beside (N, G)
+    plain = torch.empty((groups, n // 8), dtype=torch.int32)
+    assert not ml._zero_points_are_transposed(plain, layer.scales, groups, n)
+    assert ml._zero_points_are_transposed(plain.t().contiguous(), layer.scales.t().contiguous(), groups, n)
+    plain.input_dim, plain.output_dim = 0, 1
+    assert not ml._zero_points_are_transposed(plain, layer.scales.t().contiguous(), groups, n)
 
 
 @pytest.mark.gpu
@@ -46,3 +50,20 @@ def test_loading(k, n, group, one_launch):
     if not one_launch:
         kernel.process_weights_after_loading(layer)
     assert torch.equal(layer.qzeros.cpu(), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("k,n,group", [(2048, 128, 128), (512, 128, 32), (4096, 256, 128), (256, 192, 64)])
+def test_compressed_tensors_layout(k, n, group):
+    """(N, K/8) codes, (N, G) scales and (N/8, G) zero points, without marks: loaded as the same tensors in GPTQ's layout are.
+    (Where K/8 == N the codes need marks: a square tensor of codes is (K/8, N).)"""
+    other, _, want = _converted(k, n, group, "cuda:0")
+    config = ml.MPLinearLayerConfig((k, n), (k, n), scalar_types.uint4, torch.float16, group, True, False)
+    gptq = SimpleNamespace(**{**vars(other), "qzeros": other.qzeros.t().contiguous()})
+    packed = SimpleNamespace(qweight=other.qweight.t().contiguous(), scales=other.scales.t().contiguous(), bias=None,
+                             qzeros=other.qzeros.clone())   # (a clone has no marks)
+    for layer in (gptq, packed):
+        ml.MarlinLinearKernel(config).process_weights_after_loading(layer)
+    assert torch.equal(gptq.qzeros.cpu(), want)
+    for name in ("qweight", "scales", "qzeros"):
+        assert torch.equal(getattr(packed, name), getattr(gptq, name)), name
