@@ -9,14 +9,17 @@
 // column's 32 rows of a chunk in four lanes; v_permlane16_swap, one per two packed words, makes it two.
 //
 // What bounds it: with few rows the vector instructions that dequantise (9.5 per packed word, of which 2 put the
-// bytes into the order of K).  With many rows no unit alone: at 2048 rows, K 4096, N 11008, int8, the matrix pipes are 30 %
-// busy and vector issue 48 % (11.7 other vector instructions a matrix instruction: 16 multiply-adds of the group scales
-// per tile and group, and a wavefront dequantises its whole strip for 128 rows), and a third of the wavefronts' time is
-// waits and barriers; 1.35 POP/s, where the int8 instruction alone reaches 3.15 on random operands.  R = 3 with 256
+// bytes into the order of K).  With many rows the issue of instructions: beside matrix instructions a SIMD starts one
+// instruction of its wavefronts every 4.7 cycles, and 9.4 other vector instructions go with a matrix instruction (16
+// multiply-adds of the group scales per tile and group, and a wavefront dequantises its whole strip for 128 rows); at 2048
+// rows, K 4096, N 11008, int8, 1.5 POP/s, where the int8 instruction alone reaches 3.15 on random operands.  R = 3 with 256
 // registers, R = 4 where the scales in flight leave room for it.
 // Measured against the kernels it takes over from (us, before -> now):
 //   M  153, K 1152, N 22976, fp8:  42 -> 23       M  259, K 3456, N 20032, int8: 172 -> 40
 //   M  987, K 1664, N 12608, int8: 206 -> 55      M 2048, K 4096, N 11008, int8: 181 -> 137
+// and since rows of C leave as whole lines (they were 2-byte stores from a lane's column):
+//   M 1024, K 4096, N  8192, int8: 67 -> 56       M 2048, K 4096, N 11008, int8: 146 -> 124 (the same box)
+//   M   64, K 4096, N 11008, int8, 64 rows a tile: 18.8 -> 17.2      M 1213, K 1152, N 6336: 39 -> 24 with the quantisation
 //   M 1929, K 3072, N 25216, int8, groups of 32, zero points: 1836 -> 536
 //   44 random shapes of 17 to 8192 rows: 1.69 times as fast (geometric mean; one, of 25 rows, 0.89)
 //
@@ -42,13 +45,14 @@ typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
 
 constexpr int kStepK = 128;        // rows of K a step takes from each range: four chunks
 constexpr int kStepBytes = 4096;   // LDS bytes of 32 rows of A, or of a strip's packed codes, of a step
+constexpr int kTurnRow = 144;      // bytes between rows of results in LDS: the halves of a wavefront write to banks of their own
 
 // Steps between asking for a stage and using it.  One row block is bound by memory and its steps are short.
 constexpr int a8_ahead(int rows) { return rows == 1 ? 3 : 2; }
 constexpr int a8_lds(int rows, int strips, int ranges) {
   const int stages = (ranges * (a8_ahead(rows) + 1) * rows + strips * ranges * a8_ahead(rows)) * kStepBytes;
-  const int sum = ranges > 1 ? strips * ranges * 8192 : 0;
-  return stages > sum ? stages : sum;
+  const int end = (ranges > 1 ? strips * ranges * 8192 : 0) + strips * 32 * kTurnRow + 32 * rows * 4;
+  return stages > end ? stages : end;
 }
 
 // A chunk's word (rows 8 b .. 8 b + 7 of a column, nibbles in the order {0, 2, 4, 6, 1, 3, 5, 7}) -> eight operand
@@ -449,36 +453,77 @@ __global__ __launch_bounds__(64 * S * RG) __attribute__((amdgpu_waves_per_eu(2, 
     if (GC == 0) col_scale[j] = a8_number(p.scales[slot], bf16);
     if (p.bias) bias[j] = a8_number(p.bias[slot], bf16);
   }
-  auto store = [&](scalar_t total, int row, int j) __attribute__((always_inline)) {
+  auto number = [&](scalar_t total, float row_scale, int j) __attribute__((always_inline)) -> uint16_t {
     // every step rounds to fp32 as written; contraction would fuse them
 #pragma clang fp contract(off)
-    if (row >= p.size_m || !active) return;
     if constexpr (kShifted) total >>= 4;
-    const int col = strip * kStripN + 32 * j + l32;
-    if (p.splits > 1) {
-      p.partial[((size_t)split * p.size_m + row) * p.size_n + col] = a8_bits(total);
-      return;
-    }
-    float f = (float)total * p.a_scales[row];
+    float f = (float)total * row_scale;
     if (GC == 0) f *= col_scale[j];
     f += bias[j];
-    p.c[(size_t)row * p.size_n + col] =
-        bf16 ? __builtin_bit_cast(uint16_t, (__bf16)f) : __builtin_bit_cast(uint16_t, (_Float16)f);
+    return bf16 ? __builtin_bit_cast(uint16_t, (__bf16)f) : __builtin_bit_cast(uint16_t, (_Float16)f);
   };
+  auto store_raw = [&](scalar_t total, int row, int j) __attribute__((always_inline)) {
+    if (row >= p.size_m || !active) return;
+    if constexpr (kShifted) total >>= 4;
+    p.partial[((size_t)split * p.size_m + row) * p.size_n + strip * kStripN + 32 * j + l32] = a8_bits(total);
+  };
+  // Rows of C leave as whole 128-byte lines, turned in LDS: 2-byte stores straight from a lane's column, each behind the
+  // load of its row's scale, took 44 to 54 thousand cycles for 128 x 256 results, a third of the kernel; this takes 10.
+  char* sums_end = smem + (RG > 1 ? kWaves * 8192 : 0);
+  char* turn = sums_end + (RG > 1 ? ws : wave) * (32 * kTurnRow);
+  float* row_scale = reinterpret_cast<float*>(sums_end + (RG > 1 ? S : kWaves) * (32 * kTurnRow));
+  const bool wide = (reinterpret_cast<uintptr_t>(p.c) & 15) == 0;
+  auto turn_in = [&](scalar_t total, int row, float by, int j) __attribute__((always_inline)) {
+    *reinterpret_cast<uint16_t*>(turn + row * kTurnRow + 64 * j + 2 * l32) = number(total, by, j);
+  };
+  // rows 8 q .. 8 q + 7 of row block rb
+  auto turn_out = [&](int rb, int q) __attribute__((always_inline)) {
+    const int r = 8 * q + (lane >> 3), row = m0 + 32 * rb + r;
+    const uint4 v = *reinterpret_cast<const uint4*>(turn + r * kTurnRow + 16 * (lane & 7));
+    if (row >= p.size_m || !active) return;
+    uint16_t* to = p.c + (size_t)row * p.size_n + strip * kStripN + 8 * (lane & 7);
+    if (wide) {
+      *reinterpret_cast<uint4*>(to) = v;
+    } else {
+      const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+      for (int e = 0; e < 8; ++e) to[e] = (uint16_t)(w[e >> 1] >> (16 * (e & 1)));
+    }
+  };
+  __syncthreads();   // the stages are nobody's any more
+  if (p.splits == 1)
+    for (int r = threadIdx.x; r < 32 * R; r += 64 * kWaves) row_scale[r] = p.a_scales[min(m0 + r, p.size_m - 1)];
   if constexpr (RG == 1) {
+    if (p.splits > 1) {
 #pragma unroll
-    for (int rb = 0; rb < R; ++rb)
+      for (int rb = 0; rb < R; ++rb)
 #pragma unroll
-      for (int i = 0; i < 16; ++i)
+        for (int i = 0; i < 16; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) store(acc[rb][j][i], m0 + 32 * rb + 8 * (i >> 2) + 4 * half + (i & 3), j);
+          for (int j = 0; j < 2; ++j) store_raw(acc[rb][j][i], m0 + 32 * rb + 8 * (i >> 2) + 4 * half + (i & 3), j);
+      return;
+    }
+    __syncthreads();   // the rows' scales
+#pragma unroll
+    for (int rb = 0; rb < R; ++rb) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const float4 by = *reinterpret_cast<const float4*>(row_scale + 32 * rb + 8 * q + 4 * half);
+        const float bys[4] = {by.x, by.y, by.z, by.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) turn_in(acc[rb][j][4 * q + i], 8 * q + 4 * half + i, bys[i], j);
+      }
+      // only this wavefront writes and reads here, and its LDS operations complete in order
+#pragma unroll
+      for (int q = 0; q < 4; ++q) turn_out(rb, q);
+    }
   } else {
     // the ranges meet in LDS, a row block at a time; a wavefront adds 1/RG of its strip's tiles
     uint4* sums = reinterpret_cast<uint4*>(smem);
-    __syncthreads();
 #pragma unroll
     for (int rb = 0; rb < R; ++rb) {
-      if (rb > 0) __syncthreads();
 #pragma unroll
       for (int q = 0; q < 8; ++q) {   // four elements of tile q / 4
         const acc_t& v = acc[rb][q >> 2];
@@ -500,12 +545,27 @@ __global__ __launch_bounds__(64 * S * RG) __attribute__((amdgpu_waves_per_eu(2, 
           a8_from_bits(s.z, v), total[2] += v;
           a8_from_bits(s.w, v), total[3] += v;
         }
-        const int row = m0 + 32 * rb + 8 * (q & 3) + 4 * half;
+        const int r = 8 * (q & 3) + 4 * half;
+        if (p.splits > 1) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          if (q >> 2) store(total[i], row + i, 1);
-          else store(total[i], row + i, 0);
+          for (int i = 0; i < 4; ++i) {
+            if (q >> 2) store_raw(total[i], m0 + 32 * rb + r + i, 1);
+            else store_raw(total[i], m0 + 32 * rb + r + i, 0);
+          }
+        } else {
+          const float4 by = *reinterpret_cast<const float4*>(row_scale + 32 * rb + r);
+          const float bys[4] = {by.x, by.y, by.z, by.w};
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            if (q >> 2) turn_in(total[i], r + i, bys[i], 1);
+            else turn_in(total[i], r + i, bys[i], 0);
+          }
         }
+      }
+      __syncthreads();   // the sums have been read, the rows of all ranges stand
+      if (p.splits == 1) {
+#pragma unroll
+        for (int u = 0; u < 4 / RG; ++u) turn_out(rb, range * (4 / RG) + u);
       }
     }
   }
