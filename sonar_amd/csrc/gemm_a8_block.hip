@@ -260,6 +260,7 @@ __global__ __launch_bounds__(64 * S * RG) __attribute__((amdgpu_waves_per_eu(2, 
     // lanes 16 .. 31 and 48 .. 63 hold rows 8 .. 15 and 24 .. 31 of the left sixteen columns of the half, which the
     // others hold the rows before of: swapped with the right sixteen columns, a lane has 16 rows of one column
     const auto y = __builtin_amdgcn_permlane16_swap(xw[j][c].x, xw[j][c].y, false, false);
+    xw[j][c] = u32x2_t{y[0], y[1]};   // (in place: as copies they took eight instructions and registers a half)
     if constexpr (ZP && GC != 0) {
       if (c % GC == 0) zb[j] = ACT::zero_bytes((zv[ring][c / GC] >> (nibble + 16 * j)) & 15u);
     }
@@ -445,11 +446,14 @@ __global__ __launch_bounds__(64 * S * RG) __attribute__((amdgpu_waves_per_eu(2, 
 #undef SONAR_A8_READ_W
 
   // ---- results.  Element i of a tile: row 8 (i / 4) + 4 half + i % 4, column l32.
+  int at_end = lane;   // a register of its own: what is computed from it is not kept through the loop
+  asm volatile("" : "+v"(at_end));
+  const int end_l32 = at_end & 31, end_half = at_end >> 5;
   const bool bf16 = p.bf16 != 0;
   float col_scale[2] = {1.f, 1.f}, bias[2] = {0.f, 0.f};
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
-    const int slot = strip * kStripN + scale_slot(32 * j + l32, false);
+    const int slot = strip * kStripN + scale_slot(32 * j + end_l32, false);
     if (GC == 0) col_scale[j] = a8_number(p.scales[slot], bf16);
     if (p.bias) bias[j] = a8_number(p.bias[slot], bf16);
   }
@@ -465,7 +469,7 @@ __global__ __launch_bounds__(64 * S * RG) __attribute__((amdgpu_waves_per_eu(2, 
   auto store_raw = [&](scalar_t total, int row, int j) __attribute__((always_inline)) {
     if (row >= p.size_m || !active) return;
     if constexpr (kShifted) total >>= 4;
-    p.partial[((size_t)split * p.size_m + row) * p.size_n + strip * kStripN + 32 * j + l32] = a8_bits(total);
+    p.partial[((size_t)split * p.size_m + row) * p.size_n + strip * kStripN + 32 * j + end_l32] = a8_bits(total);
   };
   // Rows of C leave as whole 128-byte lines, turned in LDS: 2-byte stores straight from a lane's column, each behind the
   // load of its row's scale, took 44 to 54 thousand cycles for 128 x 256 results, a third of the kernel; this takes 10.
@@ -474,14 +478,14 @@ __global__ __launch_bounds__(64 * S * RG) __attribute__((amdgpu_waves_per_eu(2, 
   float* row_scale = reinterpret_cast<float*>(sums_end + (RG > 1 ? S : kWaves) * (32 * kTurnRow));
   const bool wide = (reinterpret_cast<uintptr_t>(p.c) & 15) == 0;
   auto turn_in = [&](scalar_t total, int row, float by, int j) __attribute__((always_inline)) {
-    *reinterpret_cast<uint16_t*>(turn + row * kTurnRow + 64 * j + 2 * l32) = number(total, by, j);
+    *reinterpret_cast<uint16_t*>(turn + row * kTurnRow + 64 * j + 2 * end_l32) = number(total, by, j);
   };
   // rows 8 q .. 8 q + 7 of row block rb
   auto turn_out = [&](int rb, int q) __attribute__((always_inline)) {
-    const int r = 8 * q + (lane >> 3), row = m0 + 32 * rb + r;
-    const uint4 v = *reinterpret_cast<const uint4*>(turn + r * kTurnRow + 16 * (lane & 7));
+    const int r = 8 * q + (at_end >> 3), row = m0 + 32 * rb + r;
+    const uint4 v = *reinterpret_cast<const uint4*>(turn + r * kTurnRow + 16 * (at_end & 7));
     if (row >= p.size_m || !active) return;
-    uint16_t* to = p.c + (size_t)row * p.size_n + strip * kStripN + 8 * (lane & 7);
+    uint16_t* to = p.c + (size_t)row * p.size_n + strip * kStripN + 8 * (at_end & 7);
     if (wide) {
       *reinterpret_cast<uint4*>(to) = v;
     } else {
@@ -500,7 +504,7 @@ __global__ __launch_bounds__(64 * S * RG) __attribute__((amdgpu_waves_per_eu(2, 
 #pragma unroll
         for (int i = 0; i < 16; ++i)
 #pragma unroll
-          for (int j = 0; j < 2; ++j) store_raw(acc[rb][j][i], m0 + 32 * rb + 8 * (i >> 2) + 4 * half + (i & 3), j);
+          for (int j = 0; j < 2; ++j) store_raw(acc[rb][j][i], m0 + 32 * rb + 8 * (i >> 2) + 4 * end_half + (i & 3), j);
       return;
     }
     __syncthreads();   // the rows' scales
@@ -508,12 +512,12 @@ __global__ __launch_bounds__(64 * S * RG) __attribute__((amdgpu_waves_per_eu(2, 
     for (int rb = 0; rb < R; ++rb) {
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const float4 by = *reinterpret_cast<const float4*>(row_scale + 32 * rb + 8 * q + 4 * half);
+        const float4 by = *reinterpret_cast<const float4*>(row_scale + 32 * rb + 8 * q + 4 * end_half);
         const float bys[4] = {by.x, by.y, by.z, by.w};
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
-          for (int j = 0; j < 2; ++j) turn_in(acc[rb][j][4 * q + i], 8 * q + 4 * half + i, bys[i], j);
+          for (int j = 0; j < 2; ++j) turn_in(acc[rb][j][4 * q + i], 8 * q + 4 * end_half + i, bys[i], j);
       }
       // only this wavefront writes and reads here, and its LDS operations complete in order
 #pragma unroll
@@ -529,7 +533,7 @@ __global__ __launch_bounds__(64 * S * RG) __attribute__((amdgpu_waves_per_eu(2, 
         const acc_t& v = acc[rb][q >> 2];
         const int i = 4 * (q & 3);
         const scalar_t v0 = v[i], v1 = v[i + 1], v2 = v[i + 2], v3 = v[i + 3];
-        sums[(wave * 8 + q) * 64 + lane] = make_uint4(a8_bits(v0), a8_bits(v1), a8_bits(v2), a8_bits(v3));
+        sums[(wave * 8 + q) * 64 + at_end] = make_uint4(a8_bits(v0), a8_bits(v1), a8_bits(v2), a8_bits(v3));
       }
       __syncthreads();
 #pragma unroll
@@ -538,14 +542,14 @@ __global__ __launch_bounds__(64 * S * RG) __attribute__((amdgpu_waves_per_eu(2, 
         scalar_t total[4] = {0, 0, 0, 0};
 #pragma unroll
         for (int g = 0; g < RG; ++g) {
-          const uint4 s = sums[((g * S + ws) * 8 + q) * 64 + lane];
+          const uint4 s = sums[((g * S + ws) * 8 + q) * 64 + at_end];
           scalar_t v;
           a8_from_bits(s.x, v), total[0] += v;
           a8_from_bits(s.y, v), total[1] += v;
           a8_from_bits(s.z, v), total[2] += v;
           a8_from_bits(s.w, v), total[3] += v;
         }
-        const int r = 8 * (q & 3) + 4 * half;
+        const int r = 8 * (q & 3) + 4 * end_half;
         if (p.splits > 1) {
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
