@@ -1415,6 +1415,7 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
 #undef SONAR_WIDE_LANDED
 #undef SONAR_WIDE_READ
 
+  __builtin_amdgcn_s_barrier();   // nobody reads the stages of A any more
   if (!active) return;
   floatx4_t sum_scale[4];
   if constexpr (kScaleSums) {
@@ -1452,9 +1453,14 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
   // Grouped: the rows of C, and their weights, of all row blocks at once.  (One row block after the other, every one waited
   // for two loads, and the sixteen waits took about 15 us: 32 MXFP4 experts 2880 x 2880, 2000 tokens 504 -> 470 us; 8
   // experts 1280 x 1408, 3655 tokens 279 -> 259; 8 experts 2816 x 1280, 1254 tokens 130 -> 117.)
-  int ids[GROUPED ? RB : 1];
+  int ids[GROUPED ? RB : 1], c_rows[GROUPED ? 2 * RB : 1];   // of the rows that this lane computes, and stores
   float weights[GROUPED ? RB : 1];
   if constexpr (GROUPED) {
+#pragma unroll
+    for (int i = 0; i < 2 * RB; ++i) {
+      const int r = 8 * i + (lane >> 3);
+      c_rows[i] = r < tile_rows ? p.sorted_ids[first_slot + r] : -1;   // (rows_total or more: padding slot)
+    }
 #pragma unroll
     for (int mb = 0; mb < RB; ++mb) {
       const int r = 16 * mb + col16;
@@ -1466,37 +1472,62 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
       weights[mb] = p.mul_topk && ids[mb] >= 0 ? p.topk_weights[ids[mb]] : 1.f;
     }
   }
+  // Rows leave as whole 128-byte lines, turned in the stages of A, which are nobody's any more: a wavefront's rows x 128 bytes,
+  // 16-byte piece q of row r at slot q ^ (r % 8).  (8-byte pieces straight from the accumulators were 32
+  // bytes a row and store: M = 8192, K = 4096, N = 28672, fp16 1442 -> 1412 us; MXFP8, M = 4000, K = 2048, N = 6016 112 -> 107; NVFP4,
+  // M = 2222, K = 4096, N = 8192 148 -> 142; 32 MXFP4 experts 2880 x 2880, 2000 tokens 496 -> 492, Mixtral-8x7B shapes, 4096 tokens
+  // 2515 -> 2487.)
+  const uint32_t turn = a_lds + wave * (kRows * 128);
+  uint32_t turn_in[4];
+#pragma unroll
+  for (int nb = 0; nb < 4; ++nb)
+    turn_in[nb] = turn + col16 * 128 + (((2 * nb + (kb >> 1)) ^ (col16 & 7)) * 16) + 8 * (kb & 1);
 #pragma unroll
   for (int mb = 0; mb < RB; ++mb) {
-    // the row of C this lane writes for this row block
-    const int r = 16 * mb + col16;
-    long c_row = -1;
+    // the routing weight is rounded to the activation type and the product is
+    // formed and rounded in that type (marlin_template.h(moe):1893-1897)
     float row_w = 1.f;
-    if constexpr (GROUPED) {
-      c_row = ids[mb];
-      // the routing weight is rounded to the activation type and the product is
-      // formed and rounded in that type (marlin_template.h(moe):1893-1897)
-      row_w = Dq<T>::to_float(Dq<T>::from_float(weights[mb]));
-    } else if (m0 + r < p.size_m) {
-      c_row = m0 + r;
-    }
+    if constexpr (GROUPED) row_w = Dq<T>::to_float(Dq<T>::from_float(weights[mb]));
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) {
       if (mb < kAgprBlocks) asm volatile("" : "+a"(acc[nb][mb]));   // still in its AGPRs here
-      if (c_row >= 0) {
-        const floatx4_t v = kScaleSums ? acc[nb][mb] * sum_scale[nb] : NV ? acc[nb][mb] * gs : acc[nb][mb];
-        uint16_t o[4] = {Dq<T>::from_float(v.x + bias[nb][0]), Dq<T>::from_float(v.y + bias[nb][1]),
-                         Dq<T>::from_float(v.z + bias[nb][2]), Dq<T>::from_float(v.w + bias[nb][3])};
-        if (GROUPED && p.mul_topk) {
+      const floatx4_t v = kScaleSums ? acc[nb][mb] * sum_scale[nb] : NV ? acc[nb][mb] * gs : acc[nb][mb];
+      uint16_t o[4] = {Dq<T>::from_float(v.x + bias[nb][0]), Dq<T>::from_float(v.y + bias[nb][1]),
+                       Dq<T>::from_float(v.z + bias[nb][2]), Dq<T>::from_float(v.w + bias[nb][3])};
+      if (GROUPED && p.mul_topk) {
 #pragma unroll
-          for (int i = 0; i < 4; ++i) o[i] = Dq<T>::from_float(Dq<T>::to_float(o[i]) * row_w);
-        }
-        uint2 packed;
-        packed.x = (uint32_t)o[0] | ((uint32_t)o[1] << 16);
-        packed.y = (uint32_t)o[2] | ((uint32_t)o[3] << 16);
-        *reinterpret_cast<uint2*>(p.c + c_row * p.size_n + strip * kStripN + 16 * nb + 4 * kb) = packed;
+        for (int i = 0; i < 4; ++i) o[i] = Dq<T>::from_float(Dq<T>::to_float(o[i]) * row_w);
       }
+      const uint2 packed = make_uint2((uint32_t)o[0] | ((uint32_t)o[1] << 16), (uint32_t)o[2] | ((uint32_t)o[3] << 16));
+      asm volatile("ds_write_b64 %0, %1 offset:%2" ::"v"(turn_in[nb]), "v"(packed), "i"(mb * 2048) : "memory");
       __builtin_amdgcn_sched_barrier(0);   // one accumulator at a time leaves the AGPRs
+    }
+  }
+  const int r8 = lane >> 3;
+  const uint32_t turn_out = turn + r8 * 128 + (((lane & 7) ^ r8) * 16);
+  uint16_t* c_strip = p.c + strip * kStripN + 8 * (lane & 7);
+  const bool c_aligned = (reinterpret_cast<uintptr_t>(p.c) & 15) == 0;
+#pragma unroll
+  for (int i = 0; i < 2 * RB; i += 4) {
+    u32x4_t line[4];   // (a wavefront's LDS operations complete in order)
+    asm volatile(
+        "ds_read_b128 %0, %4 offset:%5\n\tds_read_b128 %1, %4 offset:%6\n\t"
+        "ds_read_b128 %2, %4 offset:%7\n\tds_read_b128 %3, %4 offset:%8\n\ts_waitcnt lgkmcnt(0)"
+        : "=&v"(line[0]), "=&v"(line[1]), "=&v"(line[2]), "=&v"(line[3])
+        : "v"(turn_out), "i"(i * 1024), "i"(i * 1024 + 1024), "i"(i * 1024 + 2048), "i"(i * 1024 + 3072)
+        : "memory");
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int row = GROUPED ? c_rows[i + u] : m0 + 8 * (i + u) + r8;
+      if ((unsigned)row < (unsigned)(GROUPED ? p.rows_total : p.size_m)) {
+        uint16_t* to = c_strip + (long)row * p.size_n;
+        if (c_aligned) {
+          *reinterpret_cast<u32x4_t*>(to) = line[u];
+        } else {
+          *reinterpret_cast<uint2*>(to) = make_uint2(line[u].x, line[u].y);
+          *reinterpret_cast<uint2*>(to + 4) = make_uint2(line[u].z, line[u].w);
+        }
+      }
     }
   }
 }
