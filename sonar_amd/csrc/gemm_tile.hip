@@ -1453,14 +1453,9 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
   // Grouped: the rows of C, and their weights, of all row blocks at once.  (One row block after the other, every one waited
   // for two loads, and the sixteen waits took about 15 us: 32 MXFP4 experts 2880 x 2880, 2000 tokens 504 -> 470 us; 8
   // experts 1280 x 1408, 3655 tokens 279 -> 259; 8 experts 2816 x 1280, 1254 tokens 130 -> 117.)
-  int ids[GROUPED ? RB : 1], c_rows[GROUPED ? 2 * RB : 1];   // of the rows that this lane computes, and stores
+  int ids[GROUPED ? RB : 1];
   float weights[GROUPED ? RB : 1];
   if constexpr (GROUPED) {
-#pragma unroll
-    for (int i = 0; i < 2 * RB; ++i) {
-      const int r = 8 * i + (lane >> 3);
-      c_rows[i] = r < tile_rows ? p.sorted_ids[first_slot + r] : -1;   // (rows_total or more: padding slot)
-    }
 #pragma unroll
     for (int mb = 0; mb < RB; ++mb) {
       const int r = 16 * mb + col16;
@@ -1475,8 +1470,8 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
   // Rows leave as whole 128-byte lines, turned in the stages of A, which are nobody's any more: a wavefront's rows x 128 bytes,
   // 16-byte piece q of row r at slot q ^ (r % 8).  (8-byte pieces straight from the accumulators were 32
   // bytes a row and store: M = 8192, K = 4096, N = 28672, fp16 1442 -> 1412 us; MXFP8, M = 4000, K = 2048, N = 6016 112 -> 107; NVFP4,
-  // M = 2222, K = 4096, N = 8192 148 -> 142; 32 MXFP4 experts 2880 x 2880, 2000 tokens 496 -> 492, Mixtral-8x7B shapes, 4096 tokens
-  // 2515 -> 2487.)
+  // M = 2222, K = 4096, N = 8192 148 -> 142; 32 MXFP4 experts 2880 x 2880, 2000 tokens 475 -> 462; 8 experts 1024 x 2688, AWQ, 6002
+  // tokens 533 -> 513; Mixtral-8x7B shapes, 4096 tokens 2515 -> 2487.)
   const uint32_t turn = a_lds + wave * (kRows * 128);
   uint32_t turn_in[4];
 #pragma unroll
@@ -1486,6 +1481,7 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
   for (int mb = 0; mb < RB; ++mb) {
     // the routing weight is rounded to the activation type and the product is
     // formed and rounded in that type (marlin_template.h(moe):1893-1897)
+    if (GROUPED && __builtin_amdgcn_ballot_w64(ids[mb] >= 0) == 0) continue;   // sixteen padding slots
     float row_w = 1.f;
     if constexpr (GROUPED) row_w = Dq<T>::to_float(Dq<T>::from_float(weights[mb]));
 #pragma unroll
@@ -1509,6 +1505,11 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
   const bool c_aligned = (reinterpret_cast<uintptr_t>(p.c) & 15) == 0;
 #pragma unroll
   for (int i = 0; i < 2 * RB; i += 4) {
+    int ids_out[4];   // of the rows that this lane stores
+    if constexpr (GROUPED) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) ids_out[u] = __shfl(ids[(i + u) >> 1], 8 * (u & 1) + r8);
+    }
     u32x4_t line[4];   // (a wavefront's LDS operations complete in order)
     asm volatile(
         "ds_read_b128 %0, %4 offset:%5\n\tds_read_b128 %1, %4 offset:%6\n\t"
@@ -1518,7 +1519,7 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
         : "memory");
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const int row = GROUPED ? c_rows[i + u] : m0 + 8 * (i + u) + r8;
+      const int row = GROUPED ? ids_out[u] : m0 + 8 * (i + u) + r8;
       if ((unsigned)row < (unsigned)(GROUPED ? p.rows_total : p.size_m)) {
         uint16_t* to = c_strip + (long)row * p.size_n;
         if (c_aligned) {
