@@ -96,7 +96,7 @@ struct MidDequant {
   typedef typename std::conditional<k8, typename D8::Col, typename D4::Col>::type Col;
 };
 
-template <typename T, int FMT, int GROUPS, int MB, bool DEEP>
+template <typename T, int FMT, int GROUPS, int MB, bool DEEP, bool GROUPED = false>
 __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(mid_waves_per_simd(MB, DEEP), mid_waves_per_simd(MB, DEEP)))) void marlin_mid_gemm(
     const MidParams p) {
   typedef MidDequant<T, FMT> Fmt;
@@ -140,13 +140,18 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
 
   // Workgroup ids congruent mod 8 run on one XCD: each XCD takes a contiguous run of tiles, the row tiles
   // of a pair of strips next to each other, so the second to ask for a chunk finds it in that L2.
-  const int units = p.tiles * p.splits, per_xcd = (units + 7) / 8;
+  // (Grouped: of the blocks that the routing has made, one after the other, so that those of an expert share its chunks.)
+  const int strips = p.size_n / kStripN;
+  const int tiles_m = GROUPED ? min(p.tiles_m, p.num_post_pad[0] / p.block_size) : p.tiles_m;
+  const int tiles = GROUPED ? tiles_m * ((strips + kMidStrips - 1) / kMidStrips) : p.tiles;
+  const int units = tiles * p.splits, per_xcd = (units + 7) / 8;
   const int unit = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
   if ((int)(blockIdx.x >> 3) >= per_xcd || unit >= units) return;
-  const int split = unit / p.tiles, tile = unit - split * p.tiles;
-  const int tile_n = tile / p.tiles_m, tile_m = tile - tile_n * p.tiles_m;
+  const int split = unit / tiles, tile = unit - split * tiles;
+  const int tile_n = tile / tiles_m, tile_m = tile - tile_n * tiles_m;
   const int m0 = tile_m * 16 * MB;
-  const int strips = p.size_n / kStripN;
+  const int expert = GROUPED ? p.expert_ids[tile_m] : 0;
+  if (GROUPED && (unsigned)expert >= (unsigned)p.num_experts) return;
   // (the second strip of an odd last pair is the first again, and not stored)
   const bool active = tile_n * kMidStrips + strip_of < strips;
   const int strip = __builtin_amdgcn_readfirstlane(active ? tile_n * kMidStrips + strip_of : strips - 1);
@@ -163,14 +168,22 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
   for (int i = 0; i < kCopies; ++i) {
     int row = m0 + 8 * (strip_of * kCopies + i) + (lane >> 3);
-    if (row >= p.size_m) row = p.size_m - 1;   // rows past M are computed and never stored
+    if constexpr (GROUPED) {   // (padding slots read row 0 and are not stored)
+      const int id = row < p.sorted_len ? p.sorted_ids[row] : p.rows_total;
+      row = (unsigned)id < (unsigned)p.rows_total ? (p.a_by_slot ? row : id / p.top_k) : 0;
+    } else if (row >= p.size_m) {
+      row = p.size_m - 1;   // rows past M are computed and never stored
+    }
     a_off[i] = (uint32_t)row * (uint32_t)(p.lda * 2) + 16 * ((lane & 7) ^ (lane >> 3));
   }
-  const char* b_base = reinterpret_cast<const char*>(p.b) + (size_t)strip * p.chunks_per_strip * (Fmt::k8 ? 2048 : 1024);
+  const uint16_t* scales = p.scales + (GROUPED ? expert * p.expert_s_stride : 0) + (size_t)strip * kStripN;
+  const uint32_t* zeros = p.zeros + (GROUPED ? expert * p.expert_z_stride : 0) + (size_t)strip * (kStripN / 8);
+  const char* b_base = reinterpret_cast<const char*>(p.b + (GROUPED ? expert * p.expert_b_stride : 0)) +
+                       (size_t)strip * p.chunks_per_strip * (Fmt::k8 ? 2048 : 1024);
   const uint32_t b_off = 16 * lane;
-  const char* s_base = reinterpret_cast<const char*>(p.scales + (size_t)strip * kStripN);
+  const char* s_base = reinterpret_cast<const char*>(scales);
   const uint32_t s_off = 16 * (col16 & 7) + (FMT == kMidNvFp4 ? (kb >> 1) * (uint32_t)p.size_n * 2 : 0);
-  const char* z_base = reinterpret_cast<const char*>(p.zeros + (size_t)strip * (kStripN / 8));
+  const char* z_base = reinterpret_cast<const char*>(zeros);
   const uint32_t z_off = 4 * (col16 & 7);
   char* a_stage = smem + range * (MB * 2048);
   const uint32_t a_lds = (uint32_t)(uintptr_t)(lds_void_t*)a_stage;
@@ -265,19 +278,18 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
     }
   };
   if constexpr (GROUPS == kOneGroup && !kRaw) {
-    const uint16_t* srow = p.scales + (size_t)strip * kStripN;
     uint32_t zword = 0;
-    if (kZero) zword = p.zeros[(size_t)strip * (kStripN / 8) + (col16 & 7)];
+    if (kZero) zword = zeros[col16 & 7];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) set_col(j, srow[scale_slot(16 * j + col16, false)], zword);
+    for (int j = 0; j < 4; ++j) set_col(j, scales[scale_slot(16 * j + col16, false)], zword);
   }
 
   uint16_t one_scale[4];   // kOneGroupRaw: as they were loaded, used when the first step has landed or later
   uint32_t one_zeros = 0;
   if constexpr (GROUPS == kOneGroupRaw) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) one_scale[j] = p.scales[(size_t)strip * kStripN + scale_slot(16 * j + col16, false)];
-    if (kZero) one_zeros = p.zeros[(size_t)strip * (kStripN / 8) + (col16 & 7)];
+    for (int j = 0; j < 4; ++j) one_scale[j] = scales[scale_slot(16 * j + col16, false)];
+    if (kZero) one_zeros = zeros[col16 & 7];
   }
 
   u32x4_t av[MB];
@@ -564,34 +576,47 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
       if (kEach > 0 ? u >= kEach : range >= 4 * kSum) continue;
       const int q = kEach > 0 ? range * kEach + u : range;
       const int i = round + (q >> 2), j = q & 3;
-      const int row = m0 + 16 * i + tile_row;
+      int row = m0 + 16 * i + tile_row;
       if (i >= MB || !active) continue;
+      float row_w = 1.f;
+      if constexpr (GROUPED) {
+        row = row < p.sorted_len ? p.sorted_ids[row] : p.rows_total;
+        if ((unsigned)row >= (unsigned)p.rows_total) row = p.rows_total;   // padding slot
+        // the routing weight is rounded to the activation type and the product is formed and rounded in that type
+        // (marlin_template.h(moe):1893-1897)
+        if (p.mul_topk && row < p.rows_total) row_w = Dq<T>::to_float(Dq<T>::from_float(p.topk_weights[row]));
+      }
       floatx4_t v = floatx4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int g = 0; g < kMidRanges; ++g) {
         const float4 s = sums[(((kMidStrips * g + strip_of) * kSum + (q >> 2)) * 4 + j) * 64 + lane];
         v += floatx4_t{s.x, s.y, s.z, s.w};
       }
-      if (row >= p.size_m) continue;
+      if (row >= (GROUPED ? p.rows_total : p.size_m)) continue;
       const int nl = 16 * j + tile_col;
       if constexpr (kRaw && !kFold) {
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          v[r] *= Raw8<FMT == kMidFp8>::column_scale(p.scales[strip * kStripN + scale_slot(nl + r, false)]);
+          v[r] *= Raw8<FMT == kMidFp8>::column_scale(scales[scale_slot(nl + r, false)]);
       }
-      if (p.splits > 1) {
+      if (!GROUPED && p.splits > 1) {
         p.partial[(((size_t)split * p.size_m + row) * p.size_n + strip * kStripN + nl) / 4] = make_float4(v.x, v.y, v.z, v.w);
         continue;
       }
       if (FMT == kMidNvFp4) v = v * gs;
       float bias[4] = {0.f, 0.f, 0.f, 0.f};
       if (p.bias) {
+        const uint16_t* bias_row = p.bias + (GROUPED ? expert * p.expert_bias_stride : 0) + strip * kStripN;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) bias[r] = Dq<T>::to_float(p.bias[strip * kStripN + scale_slot(nl + r, false)]);
+        for (int r = 0; r < 4; ++r) bias[r] = Dq<T>::to_float(bias_row[scale_slot(nl + r, false)]);
       }
-      uint2 o;
-      o.x = (uint32_t)Dq<T>::from_float(v.x + bias[0]) | ((uint32_t)Dq<T>::from_float(v.y + bias[1]) << 16);
-      o.y = (uint32_t)Dq<T>::from_float(v.z + bias[2]) | ((uint32_t)Dq<T>::from_float(v.w + bias[3]) << 16);
+      uint16_t n[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        n[r] = Dq<T>::from_float(v[r] + bias[r]);
+        if (GROUPED && p.mul_topk) n[r] = Dq<T>::from_float(Dq<T>::to_float(n[r]) * row_w);
+      }
+      const uint2 o = make_uint2((uint32_t)n[0] | ((uint32_t)n[1] << 16), (uint32_t)n[2] | ((uint32_t)n[3] << 16));
       *reinterpret_cast<uint2*>(p.c + (size_t)row * p.size_n + strip * kStripN + nl) = o;
     }
   }
@@ -624,15 +649,15 @@ __global__ __launch_bounds__(256) void marlin_mid_sum(const MidParams p) {
   }
 }
 
-template <typename T, int FMT, int GROUPS, int MB, bool DEEP = false>
+template <typename T, int FMT, int GROUPS, int MB, bool DEEP = false, bool GROUPED = false>
 int launch_mid_rows(const MidParams& p, hipStream_t st) {
   static bool attr_set = false;   // raising the dynamic LDS limit is needed once per form
   if (!attr_set) {
-    SONAR_HIP(hipFuncSetAttribute((const void*)marlin_mid_gemm<T, FMT, GROUPS, MB, DEEP>,
+    SONAR_HIP(hipFuncSetAttribute((const void*)marlin_mid_gemm<T, FMT, GROUPS, MB, DEEP, GROUPED>,
                                   hipFuncAttributeMaxDynamicSharedMemorySize, mid_lds(MB, DEEP)));
     attr_set = true;
   }
-  marlin_mid_gemm<T, FMT, GROUPS, MB, DEEP><<<(p.tiles * p.splits + 7) / 8 * 8, kMidWaves * 64, mid_lds(MB, DEEP), st>>>(p);
+  marlin_mid_gemm<T, FMT, GROUPS, MB, DEEP, GROUPED><<<(p.tiles * p.splits + 7) / 8 * 8, kMidWaves * 64, mid_lds(MB, DEEP), st>>>(p);
   return launch_status("marlin_mid_gemm");
 }
 
@@ -691,7 +716,36 @@ int launch_mid_format(const MidParams& p, int format, int row_blocks, hipStream_
   }
 }
 
+template <typename T, int FMT, int GROUPS>
+int launch_mid_moe(const MidParams& p, hipStream_t st) {
+  switch (p.block_size) {
+    case 32: return launch_mid_rows<T, FMT, GROUPS, 2, false, true>(p, st);
+    case 48: return launch_mid_rows<T, FMT, GROUPS, 3, false, true>(p, st);
+    case 64: return launch_mid_rows<T, FMT, GROUPS, 4, false, true>(p, st);
+    default: return fail(SONAR_E_INVALID, "internal: blocks of %d slots", p.block_size);
+  }
+}
+
+template <typename T>
+int launch_mid_moe_format(const MidParams& p, int format, hipStream_t st) {
+  if (format == kMidInt4)
+    return p.num_groups == 1 ? launch_mid_moe<T, kMidInt4, kOneGroupRaw>(p, st) : launch_mid_moe<T, kMidInt4, kUnitGroupsRaw>(p, st);
+  if (format == kMidInt4Zp)
+    return p.num_groups == 1 ? launch_mid_moe<T, kMidInt4Zp, kOneGroupRaw>(p, st) : launch_mid_moe<T, kMidInt4Zp, kUnitGroupsRaw>(p, st);
+  if constexpr (std::is_same<T, __bf16>::value)
+    if (format == kMidMxFp4) return launch_mid_moe<T, kMidMxFp4, kChunkGroups>(p, st);
+  return fail(SONAR_E_INVALID, "internal: format %d of expert weights", format);
+}
+
 }  // namespace
+
+int mid_moe_gemm(MidParams p, int dtype, int format, int blocks, hipStream_t st) {
+  p.splits = 1;
+  p.tiles_m = blocks;
+  p.tiles = blocks * ((p.size_n / kStripN + mid_strips(2) - 1) / mid_strips(2));
+  p.split_steps = p.size_k / kMidStepK;
+  return dtype == SONAR_DTYPE_F16 ? launch_mid_moe_format<_Float16>(p, format, st) : launch_mid_moe_format<__bf16>(p, format, st);
+}
 
 int mid_gemm(MidParams p, int dtype, int format, int row_blocks, hipStream_t st) {
   const int strips = p.size_n / kStripN;

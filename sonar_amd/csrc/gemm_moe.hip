@@ -15,6 +15,7 @@
 #include <cstdlib>
 
 #include "common.hpp"
+#include "gemm_mid.hpp"
 #include "dequant.hpp"
 #include "wave_reduce.hpp"
 
@@ -29,7 +30,8 @@ int moe_tile_gemm(const void* a, void* c, const uint32_t* b, const void* bias, c
                   size_t partial_bytes, hipStream_t st);
 size_t moe_tile_table_bytes(int64_t sorted_len, int64_t num_experts);
 size_t moe_tile_partial_bytes(int64_t size_k);
-// gemm_stream.hip: the decode kernel in grouped form, for few rows per expert
+// gemm_stream.hip: compute units of the current device; the decode kernel in grouped form, for few rows per expert
+int cu_count();
 bool moe_fast_applies(bool has_perm, int64_t moe_block_size, int64_t sorted_len, int64_t num_experts,
                       int64_t a_rows, int64_t size_n, int64_t size_k, int64_t num_groups, int group_size);
 int moe_fast_gemm(const void* a, void* c, const uint32_t* b, const void* bias, const void* scales,
@@ -526,6 +528,30 @@ void launch_moe_mb(const MoeParams& p, bool has_perm, int grid, hipStream_t st) 
 
 using namespace sonar;
 
+// Whether a grouped call runs in marlin_mid_gemm, which dequantises a chunk once for all slots of a block and two strips:
+// 4-bit integers with one group or groups of 128 * 2^i rows, MXFP4.  Otherwise the decode kernel (32 slots at a time) or the tile
+// kernels (128 and 256 rows) run.  120 random GEMMs of 8 to 64 experts, us there / here:
+//   blocks of 48 slots: 1.2 times as fast (geometric mean; lowest 0.94, with a quarter of a round of workgroups or less):
+//     8 experts, 30 slots each, K = 7552, N = 3200, MXFP4 53 / 29; 32 of 39, 2560 x 5760, AWQ 117 / 90; 64 of 42, 768 x 4864 123 / 98
+//   blocks of 64, up to 56 slots an expert, so that most experts are one block: 1.2 times (lowest 0.90): 16 of 48, 4352 x 9344,
+//     AWQ 189 / 134; 32 of 48, 1024 x 896 25 / 12; with more slots, while it is one round of workgroups: 8 of 78, 640 x 1920
+//     19 / 11; 8 of 110, 7040 x 2816 94 / 70; but in 3.5 rounds 16 of 107, 1152 x 3584 26 / 44
+//   blocks of 32: as fast as the decode kernel, whose copies ask for more bytes at a time, but for half a round to a round of
+//     workgroups: 16 of 24, 3456 x 1792, AWQ 20.4 / 16.7; 16 of 17, 4608 x 1152, MXFP4 24.7 / 18.6; 64 of 20, 1408 x 2048 39 / 41
+static bool moe_mid_applies(int64_t moe_block_size, int64_t rows_total, int64_t num_experts, int64_t a_rows, int64_t size_n,
+                            int64_t size_k, int64_t num_groups, int group_size, bool fp4) {
+  static const bool no_mid = getenv("SONAR_MARLIN_NO_MOE_MID") != nullptr;  // debugging aid
+  if (no_mid || moe_block_size < 32 || !mid_applies(a_rows, size_k, size_k, num_groups, group_size)) return false;
+  if (!fp4 && (size_k % 128 != 0 || (num_groups > 1 && group_size % 128 != 0))) return false;
+  // blocks there will be where the routing is even, and rounds of workgroups (a pair of strips each)
+  const int64_t slots = rows_total / num_experts, blocks = num_experts * (slots <= moe_block_size - 8 ? 1 : slots / 56 + 1);
+  const double rounds = (double)(blocks * ((size_n + 127) / 128)) / cu_count();
+  if (slots < moe_block_size * 3 / 8) return false;   // mostly padding: the decode kernel leaves 32 slots of it out
+  if (moe_block_size == 32) return rounds >= 0.5 && rounds <= 1.0;
+  if (moe_block_size == 48) return rounds >= 0.25;
+  return slots <= 56 || rounds <= 1.0;
+}
+
 // the table of row tiles, rounded up so that what follows it is aligned
 static size_t moe_table_room(int64_t sorted_len) {
   return (moe_tile_table_bytes(sorted_len, 0) + 255) & ~(size_t)255;
@@ -671,6 +697,40 @@ int moe_gemm_any(
     return fail(SONAR_E_INVALID,
                 "act-order with 8-bit expert weights needs sorted_len * size_k * 2 more scratch bytes "
                 "(the column-permuted copy of A per slot)");
+  if (!bits8 && !row_groups && !nvfp4 && !has_perm &&
+      moe_mid_applies(moe_block_size, size_m * top_k, num_experts, a_rows, size_n, size_k, num_groups, group_size, fp4)) {
+    MidParams m = {};
+    m.a = static_cast<const uint16_t*>(a);
+    m.lda = size_k;
+    m.c = static_cast<uint16_t*>(c);
+    m.b = reinterpret_cast<const uint4*>(b_q_weight);
+    m.bias = static_cast<const uint16_t*>(b_bias);
+    m.scales = static_cast<const uint16_t*>(b_scales);
+    m.zeros = b_zeros;
+    m.size_m = (int)size_m, m.size_n = (int)size_n, m.size_k = (int)size_k, m.num_groups = (int)num_groups;
+    m.group_shift = -1;
+    if (!fp4 && num_groups > 1)
+      for (int per = group_size / 64; per > 0; per >>= 1) ++m.group_shift;   // (moe_mid_applies: 64 * 2^i rows)
+    m.chunks_per_strip = (int)(size_k / kChunkK);
+    m.raw_codes = !fp4;
+    m.sorted_ids = sorted_token_ids;
+    m.expert_ids = expert_ids;
+    m.num_post_pad = num_tokens_past_padded;
+    m.topk_weights = topk_weights;
+    m.block_size = (int)moe_block_size;
+    m.top_k = (int)top_k;
+    m.mul_topk = mul_topk_weights ? 1 : 0;
+    m.num_experts = (int)num_experts;
+    m.rows_total = (int)(size_m * top_k);
+    m.sorted_len = (int)sorted_len;
+    m.a_by_slot = a_by_slot;
+    m.expert_b_stride = (long)(size_n / kStripN) * m.chunks_per_strip * 64;
+    m.expert_s_stride = (long)num_groups * size_n;
+    m.expert_z_stride = (long)num_groups * (size_n / 8);
+    m.expert_bias_stride = size_n;
+    return mid_moe_gemm(m, dtype, fp4 ? kMidMxFp4 : has_zp ? kMidInt4Zp : kMidInt4,
+                        (int)((sorted_len + moe_block_size - 1) / moe_block_size), st);
+  }
   // Few rows per expert: the decode kernel, one workgroup per strip and 32 slots of a block
   if (!bits8 && !row_groups && !nvfp4 &&
       moe_fast_applies(has_perm, moe_block_size, sorted_len, num_experts, a_rows, size_n, size_k, num_groups,

@@ -1299,6 +1299,8 @@ __global__ __launch_bounds__(256) void marlin_dequant8_kernel(const uint4* __res
   }
 }
 
+}  // namespace
+
 int cu_count() {
   static int cached = 0;
   if (cached == 0) {
@@ -1310,6 +1312,8 @@ int cu_count() {
   }
   return cached;
 }
+
+namespace {
 
 // A'[m][k] = A[m][perm[k]]: with act-order weights (rows in sorted-group order)
 // the GEMM on A' is a plain grouped GEMM, which every kernel here runs without
