@@ -57,6 +57,21 @@ typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void lds_void_t;
 typedef __attribute__((address_space(1))) const void glb_void_t;
 
+// Asynchronous copy of BYTES (4 or 16) a lane from `base` + the lane's `off` to LDS, lane after lane from byte `lds` on; `base` and
+// `lds` are the wavefront's.  (The builtin takes 64-bit addresses a lane, which hold up the wavefront's other instructions some
+// 20 cycles more.)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"   // m0 is a reserved register: that it changes is what the clobber says
+template <int BYTES>
+__device__ __forceinline__ void copy_to_lds(uint32_t lds, uint32_t off, const char* base) {
+  static_assert(BYTES == 4 || BYTES == 16, "");
+  if constexpr (BYTES == 16)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory", "m0");
+  else
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory", "m0");
+}
+#pragma clang diagnostic pop
+
 // ---- layout constants -----------------------------------------------------
 // Marlin order: tiles of 16 (k) x 64 (n), 128 words each, stored k-tile major.
 constexpr int kMarlinTileK = 16;

@@ -95,6 +95,9 @@ inline bool plan_prefers_128_rows(int64_t size_m, int64_t size_n, int64_t size_k
   return tiles256 <= (size_k <= 8192 ? 128 : 32);
 }
 
+// Whether the rows of a tile are within the 32-bit offsets that the wide tile kernel copies a dense call's A with.
+inline bool tile_rows_within_32_bits(int64_t a_row_stride) { return a_row_stride < (int64_t)1 << 23; }
+
 // What the tile kernels are launched with, given room for the partial tiles.  `rows128`: the call's format has 128-row tiles.
 inline GemmPlan tile_plan(int64_t size_m, int64_t size_n, int64_t size_k, bool rows128, bool rows_97_128) {
   if (rows128 && plan_prefers_128_rows(size_m, size_n, size_k)) {

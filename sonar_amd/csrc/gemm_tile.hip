@@ -1020,7 +1020,7 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
   if (GROUPED) {
     first_slot = table[1 + 3 * tile_m] * 64;
     tile_rows = table[2 + 3 * tile_m] * 64;
-    expert = table[3 + 3 * tile_m];
+    expert = __builtin_amdgcn_readfirstlane(table[3 + 3 * tile_m]);
   }
   const int m0 = tile_m * kRows;
   const int strip0 = tile_n * (kTileN / kStripN);
@@ -1030,7 +1030,11 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
   const int strip = strip0 + (active ? wave : strips_here - 1);
 
   // ---- sources (regions of A as in marlin_tile_async_kernel; wavefront w fills RB / 2 regions)
-  const char* a_src[RB / 2];
+  // Memory operations take a scalar base and a 32-bit offset a lane where they can: with a 64-bit address a lane each holds up the
+  // wavefront's other instructions 20 cycles longer.  (M = 8192, K = 4096, N = 28672, fp16 1357 -> 1343 us; one tile alone 74.2 -> 73.4.)
+  // Dense calls: 256 rows of A are within 32 bits (tile_rows_within_32_bits); the rows of a grouped tile may be anywhere.
+  const char* a_rows = reinterpret_cast<const char*>(p.a + (GROUPED ? 0 : (long)m0 * p.lda));
+  typename std::conditional<GROUPED, const char*, uint32_t>::type a_src[RB / 2];
 #pragma unroll
   for (int i = 0; i < RB / 2; ++i) {
     const int region = (RB / 2) * wave + i;
@@ -1045,22 +1049,20 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
       row = m0 + in_tile;
       if (row >= p.size_m) row = p.size_m - 1;   // rows past M are computed and never stored
     }
-    a_src[i] = reinterpret_cast<const char*>(p.a) + ((long)row * p.lda + 8 * ((lane & 7) ^ r8)) * 2;
+    if constexpr (GROUPED) a_src[i] = a_rows + ((long)row * p.lda + 8 * ((lane & 7) ^ r8)) * 2;
+    else a_src[i] = (uint32_t)(row - m0) * (uint32_t)(p.lda * 2) + 16 * ((lane & 7) ^ r8);
   }
-  const uint4* b_src = p.b + expert * p.expert_b_stride +
-                       (size_t)(unsigned)(strip * p.chunks_per_strip) * (64 * kChunkLoads) + lane;
-  const char* s_src;
-  long s_group_stride;
-  if (HAS_ZP && lane >= 32) {
-    s_src = reinterpret_cast<const char*>(p.zeros + expert * p.expert_z_stride + strip * 8 + (lane & 7));
-    s_group_stride = (long)(p.size_n / 8) * 4;
-  } else {
-    s_src = reinterpret_cast<const char*>(p.scales + expert * p.expert_s_stride + strip * kStripN) + 4 * (lane & 31);
-    s_group_stride = (long)p.size_n * 2;
-    if (NV) s_src += (lane >> 5) * s_group_stride;   // the upper half of the wavefront fetches the next group's row
-    if (kScaleSums && !grouped)
-      s_src = (W8 == 2 ? reinterpret_cast<const char*>(&kOnesFp8) : reinterpret_cast<const char*>(&kOnesInt8)) + 4 * (lane & 31);
-  }
+  const char* b_base = reinterpret_cast<const char*>(p.b + expert * p.expert_b_stride) +
+                       (size_t)(unsigned)(strip * p.chunks_per_strip) * (1024 * kChunkLoads);
+  const uint32_t b_off = 16 * lane;
+  // (zero points: the lower half of the wavefront copies scales, the upper half zero points, from bases of their own)
+  const char* s_base = reinterpret_cast<const char*>(p.scales + expert * p.expert_s_stride + strip * kStripN);
+  if (kScaleSums && !grouped) s_base = W8 == 2 ? reinterpret_cast<const char*>(&kOnesFp8) : reinterpret_cast<const char*>(&kOnesInt8);
+  const char* z_src = reinterpret_cast<const char*>(p.zeros + expert * p.expert_z_stride + strip * 8 + (lane & 7));
+  const long s_group_stride = (long)p.size_n * 2;
+  const long sz_group_stride = HAS_ZP && lane >= 32 ? (long)(p.size_n / 8) * 4 : s_group_stride;
+  const char* sz_src = HAS_ZP && lane >= 32 ? z_src : s_base + 4 * (lane & 31);
+  const uint32_t s_lane = 4 * (lane & 31) + (NV ? (lane >> 5) * (uint32_t)s_group_stride : 0);   // (NVFP4: the next group's row)
   // steps per group as a shift (the host checks: group_size = 64 * 2^i)
   const int group_shift = grouped ? 31 - __builtin_clz(p.group_size / kTileK) : 0;
   char* sring = smem + kWideA + wave * (kWideScaleRows * 256);
@@ -1074,23 +1076,28 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
     const int k = min(kt, k_tiles - 1);
     const int grp = G32 ? (NV ? 2 : 1) * (2 * k + h) : (grouped ? k >> group_shift : 0);
     const int at = G32 ? 2 * (kt - k_first) + h : kt - k_first;
-    __builtin_amdgcn_global_load_lds((glb_void_t*)(s_src + (long)grp * s_group_stride),
-                                     (lds_void_t*)(sring + (at & (kWideScaleRows - 1)) * 256), 4, 0, 0);
+    if constexpr (HAS_ZP)
+      __builtin_amdgcn_global_load_lds((glb_void_t*)(sz_src + (long)grp * sz_group_stride),
+                                       (lds_void_t*)(sring + (at & (kWideScaleRows - 1)) * 256), 4, 0, 0);
+    else
+      copy_to_lds<4>(s_lds + (at & (kWideScaleRows - 1)) * 256, s_lane, s_base + grp * s_group_stride);
   };
   // memory operation `idx` (0..kWideOps-1) issued for step kt into ring position `slot`: first the
   // blocks of A of step kt, then the scale row of step kt + 1, then the two chunks of step kt
   auto issue_one = [&](int kt, int slot, int idx) __attribute__((always_inline)) {
     const int k = min(kt, k_tiles - 1);
     if (idx < RB / 2) {
-      __builtin_amdgcn_global_load_lds((glb_void_t*)(a_src[idx] + (long)k * (kTileK * 2)),
-                                       (lds_void_t*)(smem + slot * kStage + ((RB / 2) * wave + idx) * kBlockBytes),
-                                       16, 0, 0);
+      const uint32_t to = slot * kStage + ((RB / 2) * wave + idx) * kBlockBytes;
+      if constexpr (GROUPED)
+        __builtin_amdgcn_global_load_lds((glb_void_t*)(a_src[idx] + (long)k * (kTileK * 2)), (lds_void_t*)(smem + to), 16, 0, 0);
+      else
+        copy_to_lds<16>(a_lds + to, a_src[idx], a_rows + (long)k * (kTileK * 2));
     } else if (idx < RB / 2 + (G32 ? 2 : 1)) {
       issue_scales(kt + 1, idx - RB / 2);
     } else {
       const int c = idx - RB / 2 - (G32 ? 2 : 1);
-      const uint4* g = b_src + (size_t)(2 * kChunkLoads * k + c) * 64;
-      asm volatile("global_load_dwordx4 %0, %1, off" : "=&v"(wq[slot][c]) : "v"(g) : "memory");
+      asm volatile("global_load_dwordx4 %0, %1, %2 offset:%3"
+                   : "=&v"(wq[slot][c]) : "v"(b_off), "s"(b_base + (size_t)k * (2048 * kChunkLoads)), "i"(c * 1024) : "memory");
     }
   };
 

@@ -67,3 +67,17 @@ def test_grouped(mul_topk):
                                   use_atomic_add=False, use_fp32_reduce=True, is_zp_float=False)
         want = c.clone() if want is None else want
         assert torch.equal(c, want) and bool((want != -7.0).all()) and _untouched(whole, first, m * top_k * n)
+
+
+def test_rows_of_a_too_far_apart_for_32_bit_offsets():
+    """Rows 16 MiB apart: the kernels that take such calls, against the same rows side by side (two roundings to fp16 differ)."""
+    m, k, n, dtype = 150, 8192, 1088, torch.float16
+    gen = torch.Generator(device=DEV).manual_seed(1)
+    q, s = _weights(gen, 1, k, n, dtype)
+    far = torch.empty_strided((m, k), (1 << 23, 1), dtype=dtype, device=DEV)
+    far.copy_(torch.randn((m, k), device=DEV, generator=gen))
+    empty = torch.empty(0, dtype=torch.int32, device=DEV)
+    ws = mu.marlin_make_workspace_new(torch.device(DEV))
+    got, want = (ops.marlin_gemm(a, None, q[0], None, s[0], None, None, empty, empty, empty, ws, scalar_types.uint4b8, m, n, k,
+                                 True, False, True, False).double() for a in (far, far.contiguous()))
+    assert float((got - want).norm() / want.norm()) < 2e-3
