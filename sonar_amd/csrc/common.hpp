@@ -70,6 +70,18 @@ __device__ __forceinline__ void copy_to_lds(uint32_t lds, uint32_t off, const ch
   else
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory", "m0");
 }
+// Four copies of 1 KiB that follow one another in memory and in LDS (the offset of the instruction counts for both).
+// NT: non-temporal.
+template <bool NT>
+__device__ __forceinline__ void copy_4k_to_lds(uint32_t lds, uint32_t off, const char* base) {
+#define SONAR_COPY_4K(NT_BIT)                                                                                              \
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" NT_BIT                                      \
+               "\n\tglobal_load_lds_dwordx4 %1, %2 offset:1024" NT_BIT "\n\tglobal_load_lds_dwordx4 %1, %2 offset:2048" NT_BIT \
+               "\n\tglobal_load_lds_dwordx4 %1, %2 offset:3072" NT_BIT ::"s"(lds), "v"(off), "s"(base) : "memory", "m0")
+  if constexpr (NT) SONAR_COPY_4K(" nt");
+  else SONAR_COPY_4K("");
+#undef SONAR_COPY_4K
+}
 #pragma clang diagnostic pop
 
 // ---- layout constants -----------------------------------------------------

@@ -20,6 +20,8 @@
 // and since rows of C leave as whole lines (they were 2-byte stores from a lane's column):
 //   M 1024, K 4096, N  8192, int8: 67 -> 56       M 2048, K 4096, N 11008, int8: 146 -> 124 (the same box)
 //   M   64, K 4096, N 11008, int8, 64 rows a tile: 18.8 -> 17.2      M 1213, K 1152, N 6336: 39 -> 24 with the quantisation
+// and since copies have a scalar base and 32-bit offsets:
+//   M 2048, K 4096, N 11008, int8, with the quantisation: 118.3 -> 116.6
 //   M 1929, K 3072, N 25216, int8, groups of 32, zero points: 1836 -> 536
 //   44 random shapes of 17 to 8192 rows: 1.69 times as fast (geometric mean; one, of 25 rows, 0.89)
 //
@@ -182,17 +184,14 @@ __global__ __launch_bounds__(64 * S * RG) __attribute__((amdgpu_waves_per_eu(2, 
   char* a_stage = smem + range * (kRing * R * kStepBytes);
   char* w_stage = smem + RG * kRing * R * kStepBytes + wave * (kAhead * kStepBytes);
   const uint32_t a_lds = (uint32_t)(uintptr_t)(lds_void_t*)a_stage;
-  const uint32_t w_lds = (uint32_t)(uintptr_t)(lds_void_t*)w_stage + 16 * lane;
+  const uint32_t w_stage_lds = (uint32_t)(uintptr_t)(lds_void_t*)w_stage, w_lds = w_stage_lds + 16 * lane;
 
   // uint16 scales of both column halves and zero-point words of the steps in flight
   uint32_t sv[kRing][kGroups ? kGroups : 1][2], zv[kRing][kGroups ? kGroups : 1];
   auto issue_w = [&](const int ring, int wslot, int k) __attribute__((always_inline)) {
     k = min(k_first + k, steps - 1);
     const char* src = b_base + (size_t)k * kStepBytes;
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-      __builtin_amdgcn_global_load_lds((glb_void_t*)(src + c * 1024 + b_off),
-                                       (lds_void_t*)(w_stage + wslot * kStepBytes + c * 1024), 16, 0, 0);
+    copy_4k_to_lds<false>(w_stage_lds + wslot * kStepBytes, b_off, src);
 #pragma unroll
     for (int g = 0; g < kGroups; ++g) {
       const char* s_src = s_base + (size_t)(k * kGroups + g) * p.size_n * 2;
@@ -208,9 +207,7 @@ __global__ __launch_bounds__(64 * S * RG) __attribute__((amdgpu_waves_per_eu(2, 
     const char* src = reinterpret_cast<const char*>(p.a) + (size_t)min(k_first + k, steps - 1) * kStepK;
 #pragma unroll
     for (int i = 0; i < kLoadsA; ++i)
-      __builtin_amdgcn_global_load_lds(
-          (glb_void_t*)(src + a_off[i]),
-          (lds_void_t*)(a_stage + ring * (R * kStepBytes) + (ws * kLoadsA + i) * 1024), 16, 0, 0);
+      copy_to_lds<16>(a_lds + ring * (R * kStepBytes) + (ws * kLoadsA + i) * 1024, a_off[i], src);
   };
   // until only the `n` youngest operations are outstanding; the registers of ring position `ring` have landed
   auto landed = [&](const int ring, const int n) __attribute__((always_inline)) {

@@ -26,6 +26,7 @@
 //   M   80, K 4096, N 28672: 27.9 -> 36.5, 45.0       M  144, K 4096, N 11008: 22.9 -> 27.9, 29.7
 // Five and six row blocks on four wavefronts with 512 registers each took 30 and 33 us in the first call with M 80 and 96, and
 // 1.5 times as long as eight wavefronts elsewhere.
+// (Copies of activations by asm with a scalar base: the first two 22.1 -> 21.7 and 17.8 -> 17.5.)
 // Measured against the kernels it takes over from (us, before -> now):
 //   M   64, K 4096, N 28672, bf16: 29.1 -> 21.7      M  200, K 4096, N 6144, fp16, zero points: 24.6 -> 17.6
 //   M  333, K 2880, N  5760, bf16, groups of 32: 40.5 -> 21.7      M  512, K 4096, N 2048, bf16: 36 -> 20
@@ -213,8 +214,7 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
     } else {
       const int i = op - (kOps - kCopies);
       const char* a_src = reinterpret_cast<const char*>(p.a) + (size_t)k * (kMidStepK * 2);
-      __builtin_amdgcn_global_load_lds((glb_void_t*)(a_src + a_off[i]),
-                                       (lds_void_t*)(a_stage + slot * kStage + (strip_of * kCopies + i) * 1024), 16, 0, 0);
+      copy_to_lds<16>(a_lds + slot * kStage + (strip_of * kCopies + i) * 1024, a_off[i], a_src);
     }
   };
   // Scales of the unit of step `k`, behind whose first half they are taken from the registers, and zero points, which fp16

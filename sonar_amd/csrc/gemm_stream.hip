@@ -673,18 +673,19 @@ __device__ __forceinline__ int moe_row_id(const StreamParams& p, int block, int 
 template <int MB>
 struct FastLane {
   uint32_t a_off[2 * MB];  // byte offset of the 16 bytes this lane copies from rows 8h..8h+7 of a 64-column slice of A
-  const char* s_ptr;    // this lane's dword of the scale / zero-point row of (group 0, strip 0)
+  const char* s_ptr;    // (zero points) this lane's dword of the scale / zero-point row of (group 0, strip 0)
   long s_group_stride;  // bytes between groups for s_ptr
   int s_strip_stride;   // bytes between strips for s_ptr
 };
 
+// Copies have a scalar base and 32-bit offsets, and the four of a unit's codes one address: four decoder layers of 4096 / 6144 /
+// 14336, 16 rows 164.9 -> 163.5 us.
 // unit_group_shift: s >= 0 for groups of 128 * 2^s rows, -1 for one group; with
 // GPU > 1 the unit holds groups GPU * unit .. GPU * unit + GPU - 1.
-template <int MB, int GPU>
+template <bool HAS_ZP, int MB, int GPU>
 __device__ __forceinline__ void copy_weights(const StreamParams& p, const FastLane<MB>& fl, int strip, int unit,
-                                             char* slot, int lane, int unit_group_shift) {
-  const char* gq = reinterpret_cast<const char*>(p.b + (size_t)(unsigned)(strip * p.chunks_per_strip + unit * 4) * 64) + 16u * (uint32_t)lane;
-  lds_void_t* lq = (lds_void_t*)slot;
+                                             uint32_t slot, int lane, int unit_group_shift) {
+  const char* gq = reinterpret_cast<const char*>(p.b + (size_t)(unsigned)(strip * p.chunks_per_strip + unit * 4) * 64);
   // `nt_weights` (a launch whose workgroups each read their weights once, on a matrix of 10 MB or
   // more): the copies carry the non-temporal bit, which streams the weights past the caches and
   // leaves the activations and the partial tiles there.  Measured on the four GEMMs of a
@@ -695,24 +696,20 @@ __device__ __forceinline__ void copy_weights(const StreamParams& p, const FastLa
   // stands for "the model's weights do not fit the caches": matrices of a few MB may well be
   // found there by the next call.  With several blocks of rows the later ones count on finding
   // the chunk in the L2, and those copies stay plain.
-  constexpr int kNonTemporal = 2;
-  if (p.nt_weights) {
-    __builtin_amdgcn_global_load_lds((glb_void_t*)gq, lq, 16, 0, kNonTemporal);
-    __builtin_amdgcn_global_load_lds((glb_void_t*)gq, lq, 16, 1024, kNonTemporal);
-    __builtin_amdgcn_global_load_lds((glb_void_t*)gq, lq, 16, 2048, kNonTemporal);
-    __builtin_amdgcn_global_load_lds((glb_void_t*)gq, lq, 16, 3072, kNonTemporal);
-  } else {
-    __builtin_amdgcn_global_load_lds((glb_void_t*)gq, lq, 16, 0, 0);
-    __builtin_amdgcn_global_load_lds((glb_void_t*)gq, lq, 16, 1024, 0);
-    __builtin_amdgcn_global_load_lds((glb_void_t*)gq, lq, 16, 2048, 0);
-    __builtin_amdgcn_global_load_lds((glb_void_t*)gq, lq, 16, 3072, 0);
-  }
+  if (p.nt_weights) copy_4k_to_lds<true>(slot, 16 * lane, gq);
+  else copy_4k_to_lds<false>(slot, 16 * lane, gq);
   const int g = GPU > 1 ? unit * GPU : (unit_group_shift >= 0 ? (unit >> unit_group_shift) : 0);
-  const char* gs = fl.s_ptr + (long)g * fl.s_group_stride + (long)strip * fl.s_strip_stride;
+  if constexpr (HAS_ZP) {   // the halves of the wavefront copy from bases of their own
+    const char* gs = fl.s_ptr + (long)g * fl.s_group_stride + (long)strip * fl.s_strip_stride;
 #pragma unroll
-  for (int gi = 0; gi < GPU; ++gi)
-    __builtin_amdgcn_global_load_lds((glb_void_t*)(gs + gi * fl.s_group_stride),
-                                     (lds_void_t*)(slot + kSlotS + 256 * gi), 4, 0, 0);
+    for (int gi = 0; gi < GPU; ++gi)
+      __builtin_amdgcn_global_load_lds((glb_void_t*)(gs + gi * fl.s_group_stride),
+                                       (lds_void_t*)(uintptr_t)(slot + kSlotS + 256 * gi), 4, 0, 0);
+  } else {
+    const char* gs = reinterpret_cast<const char*>(p.scales + (long)g * p.size_n + strip * kStripN);
+#pragma unroll
+    for (int gi = 0; gi < GPU; ++gi) copy_to_lds<4>(slot + kSlotS + 256 * gi, 4 * (lane & 31), gs + (long)gi * p.size_n * 2);
+  }
 }
 
 // The 16 x 128 slice of A of one unit and block of 16 rows, as four regions of
@@ -725,7 +722,7 @@ __device__ __forceinline__ void copy_weights(const StreamParams& p, const FastLa
 // reads (16 rows, one piece each) off each other's banks.
 template <int MB>
 __device__ __forceinline__ void copy_activations(const StreamParams& p, const FastLane<MB>& fl, int unit,
-                                                 char* slot) {
+                                                 uint32_t slot) {
   const char* ga = reinterpret_cast<const char*>(p.a) + (long)unit * (4 * kChunkK * 2);
 #pragma unroll
   for (int h = 0; h < 2 * MB; ++h) {
@@ -733,9 +730,9 @@ __device__ __forceinline__ void copy_activations(const StreamParams& p, const Fa
     // not stored.  (The copies of a compute unit share 64 bytes a clock.  Four decoder layers of 7424 / 9472 / 25984, one
     // row: 365 -> 359 us.)
     if (h > 0 && 8 * h >= p.size_m) break;
-    char* s = slot + 4096 * (h >> 1) + 1024 * (h & 1);
-    __builtin_amdgcn_global_load_lds((glb_void_t*)(ga + fl.a_off[h]), (lds_void_t*)(s), 16, 0, 0);
-    __builtin_amdgcn_global_load_lds((glb_void_t*)(ga + 128 + fl.a_off[h]), (lds_void_t*)(s + 2048), 16, 0, 0);
+    const uint32_t s = slot + 4096 * (h >> 1) + 1024 * (h & 1);
+    copy_to_lds<16>(s, fl.a_off[h], ga);
+    copy_to_lds<16>(s + 2048, fl.a_off[h], ga + 128);
   }
 }
 
@@ -854,8 +851,7 @@ __global__ __launch_bounds__(kFastWaves * 64, 2) void marlin_stream_fast_kernel(
   }
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col16 = lane & 15;
-  char* ring = smem + wave * kWaveLds;
-  const uint32_t ring_lds = (uint32_t)(uintptr_t)(lds_void_t*)ring;
+  const uint32_t ring_lds = (uint32_t)(uintptr_t)(lds_void_t*)smem + wave * kWaveLds;
   const uint32_t red_lds = (uint32_t)(uintptr_t)(lds_void_t*)smem;
 
   // this workgroup's piece and this wavefront's share of it: units unit, unit + kFastWaves, ...
@@ -882,7 +878,7 @@ __global__ __launch_bounds__(kFastWaves * 64, 2) void marlin_stream_fast_kernel(
       fl.s_ptr = reinterpret_cast<const char*>(p.zeros + (lane & 7));
       fl.s_group_stride = (long)(p.size_n / 8) * 4;
       fl.s_strip_stride = 8 * 4;
-    } else {
+    } else if (HAS_ZP) {
       fl.s_ptr = reinterpret_cast<const char*>(p.scales) + 4 * (lane & 31);
       fl.s_group_stride = (long)p.size_n * 2;
       fl.s_strip_stride = kStripN * 2;
@@ -914,10 +910,10 @@ __global__ __launch_bounds__(kFastWaves * 64, 2) void marlin_stream_fast_kernel(
   // younger than A(x) are those of weights(x+W), so "at most that many outstanding"
   // means weights(x) and A(x) have landed.
   if (mine > 0) {
-    copy_weights<MB, GPU>(p, fl, strip, unit, ring, lane, unit_group_shift);
-    copy_activations<MB>(p, fl, unit, ring + kWaveA);
+    copy_weights<HAS_ZP, MB, GPU>(p, fl, strip, unit, ring_lds, lane, unit_group_shift);
+    copy_activations<MB>(p, fl, unit, ring_lds + kWaveA);
   }
-  if (mine > 1) copy_weights<MB, GPU>(p, fl, strip, unit + kFastWaves, ring + kSlotBytes, lane, unit_group_shift);
+  if (mine > 1) copy_weights<HAS_ZP, MB, GPU>(p, fl, strip, unit + kFastWaves, ring_lds + kSlotBytes, lane, unit_group_shift);
 
   floatx4_t acc[MB][4];
 #pragma unroll
@@ -972,7 +968,7 @@ __global__ __launch_bounds__(kFastWaves * 64, 2) void marlin_stream_fast_kernel(
     for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
       for (int cc = 0; cc < 4; ++cc) asm volatile("" : "+v"(a[mb][cc]));
-    if (left > 1) copy_activations<MB>(p, fl, unit + kFastWaves, ring + kWaveA);
+    if (left > 1) copy_activations<MB>(p, fl, unit + kFastWaves, ring_lds + kWaveA);
     constexpr int kChunksPerGroup = 4 / GPU;
     const floatx4_t zero4 = floatx4_t{0.f, 0.f, 0.f, 0.f};
     floatx4_t a_sum[GPU][MB];
@@ -1012,7 +1008,7 @@ __global__ __launch_bounds__(kFastWaves * 64, 2) void marlin_stream_fast_kernel(
       if constexpr (HAS_ZP) asm volatile("" : "+v"(zbits[gi]));
     }
     if (left > 2)
-      copy_weights<MB, GPU>(p, fl, strip, unit + 2 * kFastWaves, ring + slot * kSlotBytes, lane, unit_group_shift);
+      copy_weights<HAS_ZP, MB, GPU>(p, fl, strip, unit + 2 * kFastWaves, ring_lds + slot * kSlotBytes, lane, unit_group_shift);
     unit += kFastWaves;
     floatx4_t sum[MB][4];
 #pragma unroll
