@@ -80,12 +80,12 @@ struct StreamParams {
   // workgroup ids are dealt to the parts so that consecutive parts (which share
   // strips and rows of A) have ids congruent mod 8, i.e. sit on one XCD
   int xcd_ranges;
-  // fast kernel only: piece_units > 0 says that every strip is cut into 2^piece_shift
-  // pieces of piece_units units, part (strip << piece_shift) + i being piece i: the
-  // kernel then finds its range with shifts instead of the divisions of the general
-  // split (a wavefront's scalar unit is shared with seven others: the index arithmetic
-  // of the general split alone took about 0.4 us before the first copy was issued)
-  int piece_shift, piece_units;
+  // fast kernel only: every strip is cut into `pieces` pieces of whole units, part strip * pieces + i being piece i, units
+  // i * units_per_strip / pieces and on.  The kernel divides by a multiplication with piece_recip = 2^32 / pieces, rounded up
+  // (a wavefront's scalar unit is shared with seven others: the divisions of the general split took about 0.4 us before the
+  // first copy was issued); one piece needs none.
+  int pieces;
+  unsigned piece_recip;
   int nt_weights;   // fast kernel only: copy the weights with the non-temporal bit
   // grouped (mixture-of-experts) calls of the fast kernel only: workgroup
   // block * grid_parts + strip works on the slots [block * block_size, ...) of
@@ -812,7 +812,7 @@ __global__ __launch_bounds__(kFastWaves * 64, 2) void marlin_stream_fast_kernel(
     asm volatile("" ::"s"(p.a), "s"(p.lda), "s"(p.c), "s"(p.b), "s"(p.bias), "s"(p.scales), "s"(p.zeros),
                  "s"(p.scratch), "s"(p.size_m), "s"(p.size_n), "s"(p.num_groups), "s"(p.chunks_per_strip),
                  "s"(p.units_per_strip), "s"(p.parts), "s"(p.slabs), "s"(p.grid_parts), "s"(p.tickets),
-                 "s"(p.ticket_stride), "s"(p.xcd_ranges), "s"(p.piece_shift), "s"(p.piece_units), "s"(p.nt_weights),
+                 "s"(p.ticket_stride), "s"(p.xcd_ranges), "s"(p.pieces), "s"(p.piece_recip), "s"(p.nt_weights),
                  "s"(unit_group_shift));
   int part, slab;
   if constexpr (GROUPED) {   // strip-major inside a block of slots
@@ -855,10 +855,16 @@ __global__ __launch_bounds__(kFastWaves * 64, 2) void marlin_stream_fast_kernel(
   const uint32_t red_lds = (uint32_t)(uintptr_t)(lds_void_t*)smem;
 
   // this workgroup's piece and this wavefront's share of it: units unit, unit + kFastWaves, ...
-  const int strip = part >> p.piece_shift;
-  const int pieces = 1 << p.piece_shift;
-  int unit = (part & (pieces - 1)) * p.piece_units + wave;
-  const int mine = wave < p.piece_units ? (p.piece_units - wave + kFastWaves - 1) / kFastWaves : 0;
+  const int pieces = GROUPED ? 1 : p.pieces;
+  int strip = part, first_unit = 0, end_unit = p.units_per_strip;
+  if (pieces > 1) {   // (part < 2^16 and units < 2^28 here: the products with the reciprocal are exact)
+    strip = __umulhi(part, p.piece_recip);
+    const int at = (part - strip * pieces) * p.units_per_strip;
+    first_unit = __umulhi(at, p.piece_recip);
+    end_unit = __umulhi(at + p.units_per_strip, p.piece_recip);
+  }
+  int unit = first_unit + wave;
+  const int mine = unit < end_unit ? (end_unit - unit + kFastWaves - 1) / kFastWaves : 0;
   const bool grouped = p.num_groups > 1;
 
   FastLane<MB> fl;
@@ -1051,7 +1057,7 @@ __global__ __launch_bounds__(kFastWaves * 64, 2) void marlin_stream_fast_kernel(
   // wavefront order and finishes it.
   int first = 0, last = 0;   // the workgroups that share this strip
   if constexpr (!GROUPED) {
-    first = strip << p.piece_shift;
+    first = strip * pieces;
     last = first + pieces - 1;
   }
 #pragma unroll
@@ -1621,8 +1627,8 @@ int moe_fast_gemm(const void* a, void* c, const uint32_t* b, const void* bias, c
   p.sub_blocks = moe_block_size > 32 ? 2 : 1;
   p.slabs = (int)((sorted_len + moe_block_size - 1) / moe_block_size) * p.sub_blocks;   // blocks of slots x halves
   p.grid_parts = n_strips;
-  p.piece_shift = 0;
-  p.piece_units = p.units_per_strip;
+  p.pieces = 1;
+  p.piece_recip = 0;
   p.sorted_ids = sorted_ids;
   p.expert_ids = expert_ids;
   p.num_post_pad = num_post_pad;
@@ -1681,17 +1687,36 @@ bool mid_switched_off() {
     if (getenv(name) != nullptr) return true;
   return false;
 }
+// How many pieces the strips of a decode launch are cut into: `units` of 128 rows a strip, `workgroups` with one piece, at most
+// `room` of them.  In thousandths of what a round of the eight wavefronts takes (0.7 us): a launch takes as many rounds as its
+// longest piece, a little for every unit and workgroup, and with pieces 2.2 rounds for the partial tiles, the ticket and the
+// last workgroup's sum, 0.3 more when that needs a second set of loads.  Fitted to 196 shapes (K = 1024 to 14336, N = 1024 to 8192, 1 to
+// 32 rows, gptq, AWQ and MXFP4, weights from memory) timed with one to eight pieces each: 0.5 % above the best of them on average;
+// 5, 6 and 7 pieces are never much better.  Against the largest power of two that divides the units and fits (us, before -> now):
+//   K 13952, N 4160, 8 rows, AWQ (109 units): 17.1 -> 11.7     K 10368, N 1280, 8 rows, MXFP4 (81): 14.0 -> 7.7
+//   K  1536, N 7488, 1 row,  AWQ (12 units):   6.4 ->  4.7     K  1024, N 2432, 16 rows (8): 5.3 -> 4.1
+// over all 196 shapes 0.90 times the time, two 2 and 4 % longer.
+int decode_pieces(int units, int64_t workgroups, int64_t room, int most) {
+  int best = 1;
+  int64_t least = INT64_MAX;
+  for (const int pieces : {1, 2, 3, 4, 8}) {
+    if (pieces > 1 && (pieces > most || pieces > units || workgroups * pieces > room)) break;
+    const int64_t longest = (units + pieces - 1) / pieces;
+    const int64_t cost = 1000 * ((longest + 7) / 8) + 20 * longest + workgroups * pieces + (pieces > 1 ? 2200 : 0) + (pieces > 4 ? 300 : 0);
+    if (cost < least) least = cost, best = pieces;
+  }
+  return best;
+}
+
 // Microseconds the decode kernel takes in blocks of rows: a fit of measured times (K = 1024 to 14336, N = 2048 to 28672, 17 to
 // 256 rows, weights from memory: 90 % within 7 %).  What counts is the launch: one block of 16 rows a workgroup while those
 // fit the compute units once (strips then in pieces), else two, and from there on the most workgroups on a compute unit.
 double decode_rows_estimate(int64_t size_m, int64_t n_strips, int64_t size_k, bool zero_points, int cus) {
   const int64_t blocks16 = (size_m + 15) / 16, units = size_k / 128;
-  int pieces = 1;
-  if (size_m <= 64)
-    while (pieces < 8 && n_strips * 2 * pieces * blocks16 <= cus && units % (2 * pieces) == 0) pieces *= 2;
+  const int pieces = size_m <= 64 ? decode_pieces((int)units, n_strips * blocks16, cus, 8) : 1;
   const bool pairs = n_strips * pieces * blocks16 > cus;
   const int64_t workgroups = n_strips * pieces * (pairs ? (blocks16 + 1) / 2 : blocks16);
-  const double k = size_k / pieces / 1024.0, megabytes = n_strips * 64.0 * size_k / 2e6;
+  const double k = (units + pieces - 1) / pieces / 8.0, megabytes = n_strips * 64.0 * size_k / 2e6;
   const int64_t most = (workgroups + cus - 1) / cus;
   double us;
   if (!pairs) us = 3.2 + 1.25 * k + (pieces > 1 ? 1.8 : 0.0);
@@ -1932,8 +1957,8 @@ int marlin_gemm_any(const void* a, int64_t a_row_stride, void* c, const uint32_t
   p.tickets = nullptr;
   p.ticket_stride = 1;
   p.xcd_ranges = 0;
-  p.piece_shift = 0;
-  p.piece_units = 0;
+  p.pieces = 1;
+  p.piece_recip = 0;
 
   if (use_tile) {
     const size_t used = stream_scratch_bytes();
@@ -1943,9 +1968,8 @@ int marlin_gemm_any(const void* a, int64_t a_row_stride, void* c, const uint32_t
   }
 
   // The fast kernel: up to 16 rows, or more rows in blocks of 16 or 32 (slab_fast), all in
-  // one launch.  Every strip is cut into the same number of pieces, a power of two, as many
-  // as keep the launch at one workgroup per compute unit (a Llama-3-8B attention output
-  // projection at M <= 16: 64 strips x 4 pieces), and the pieces of a strip are summed inside
+  // one launch.  Every strip is cut into the same number of pieces (decode_pieces; a Llama-3-8B
+  // attention output projection at M <= 16: 64 strips x 4 pieces), and the pieces of a strip are summed inside
   // the kernel (tickets in the workspace; the fix-up launch when the workspace is too small
   // for them).  With more strips than compute units every strip is one workgroup of four
   // wavefronts, three of which fit a compute unit.
@@ -1958,19 +1982,14 @@ int marlin_gemm_any(const void* a, int64_t a_row_stride, void* c, const uint32_t
     p.c = static_cast<uint16_t*>(c);
     p.size_m = (int)size_m;
     const int blocks16 = (int)((size_m + 15) / 16);
-    int shift = 0;
     // a scratch slot holds the partial tiles of four blocks of 16 rows, a ticket field counts to 15
     if (size_m <= 64) {
-      while (shift < 3 && n_strips * (2 << shift) * blocks16 <= cus && p.units_per_strip % (2 << shift) == 0 &&
-             n_strips * (2 << shift) * blocks16 <= workspace_len)
-        ++shift;
-      if (split_env)
-        while (shift > 0 && (1 << shift) > atoi(split_env)) --shift;
+      p.pieces = decode_pieces(p.units_per_strip, n_strips * blocks16, std::min<int64_t>(cus, workspace_len),
+                               split_env ? atoi(split_env) : 8);
+      if (p.pieces > 1) p.piece_recip = 0xffffffffu / (unsigned)p.pieces + 1;
     }
-    p.piece_shift = shift;
-    p.piece_units = p.units_per_strip >> shift;
-    p.parts = (int)(n_strips << shift);
-    SONAR_REQUIRE(n_strips << shift < (1LL << 30), "size_n = %ld is too large", (long)size_n);
+    p.parts = (int)n_strips * p.pieces;
+    SONAR_REQUIRE(n_strips < (1LL << 30), "size_n = %ld is too large", (long)size_n);
     // Two blocks of rows per workgroup once one block each would make more
     // workgroups than compute units: the weights are then fetched from L2 and
     // unpacked once for 32 rows.
@@ -1980,7 +1999,7 @@ int marlin_gemm_any(const void* a, int64_t a_row_stride, void* c, const uint32_t
     p.grid_parts = p.slabs > 1 ? (p.parts + 7) / 8 * 8 : p.parts;
     // more workgroups than compute units: small ones, three per compute unit
     const bool half = !no_half && (int64_t)p.parts * p.slabs > cus;
-    const bool split = shift > 0;
+    const bool split = p.pieces > 1;
     // a split strip leaves one set of partial tiles per contributor in scratch slot `part` or `parts + part`
     if (split)
       SONAR_REQUIRE((size_t)2 * p.parts * kSlotFloat4 * sizeof(float4) <= stream_scratch_bytes() &&
@@ -1998,7 +2017,7 @@ int marlin_gemm_any(const void* a, int64_t a_row_stride, void* c, const uint32_t
     p.nt_weights = !no_nt && p.slabs == 1 && size_k * size_n / 2 >= 10 * 1000 * 1000;
     g_last_decode_launch[0] = p.grid_parts * p.slabs;
     g_last_decode_launch[1] = half ? 256 : 512;
-    g_last_decode_launch[2] = 1 << shift;
+    g_last_decode_launch[2] = p.pieces;
     g_last_decode_launch[3] = p.nt_weights;
     int rc;
     if (chk.fp4)   // groups of 32 rows: never in blocks of rows (slab_fast is off), so one block of 16 rows
@@ -2011,7 +2030,7 @@ int marlin_gemm_any(const void* a, int64_t a_row_stride, void* c, const uint32_t
                       : launch_fast<__bf16, false>(p, unit_group_shift, half, row_blocks, st);
     if (rc) return rc;
     if (int rc2 = launch_status("marlin_stream_fast_kernel")) return rc2;
-    if (split && !inline_sum) {   // the fix-up kernel reads the split as ranges of units: part i = units [i, i + 1) * piece_units
+    if (split && !inline_sum) {   // the fix-up kernel reads the split as ranges of units, which the pieces of all strips are in a row
       p.total_units = (int)total_units;
       if (dtype == SONAR_DTYPE_F16) launch_fixup<_Float16>(p, st);
       else launch_fixup<__bf16>(p, st);
