@@ -416,6 +416,25 @@ int sonar_moe_wna16_marlin_gemm_nvfp4(
     int64_t num_experts, int dtype, int64_t size_m, int64_t size_n,
     int64_t size_k, int64_t num_groups, void* stream);
 
+/* A grouped GEMM whose result goes through a gated activation (the first of a mixture-of-experts layer's two; marlin_moe.py:134-180
+ * of the reference, two calls there).  Where the kernel of the call can form the activation itself, gated
+ * dtype[size_m * top_k][size_n / 2] is written, c is left as it was and *gated_written is 1; the bits are those of the GEMM and the
+ * activation after one another.  Otherwise *gated_written is 0 and c holds the GEMM's result.  `activation` 0 is sonar_silu_and_mul,
+ * else a SONAR_ACT_* kind with its limit and alpha (formed here: 0 and SONAR_ACT_SWIGLUOAI).  gated must not overlap the inputs.
+ * global_scale != NULL: NVFP4.  The other arguments as for sonar_moe_wna16_marlin_gemm. */
+int sonar_moe_wna16_marlin_gemm_gated(
+    const void* a, void* c, const uint32_t* b_q_weight, int b_layout,
+    const void* b_bias, const void* b_scales, const float* global_scale,
+    const uint32_t* b_zeros, const int32_t* g_idx, const int32_t* perm,
+    void* scratch, size_t scratch_bytes, const int32_t* sorted_token_ids,
+    int64_t sorted_len, const int32_t* expert_ids,
+    const int32_t* num_tokens_past_padded, const float* topk_weights,
+    int64_t moe_block_size, int64_t top_k, int mul_topk_weights,
+    int64_t num_experts, int dtype, int64_t b_type_id, int64_t size_m,
+    int64_t size_n, int64_t size_k, int64_t num_groups, int is_k_full,
+    void* gated, int activation, float limit, float alpha, int* gated_written,
+    void* stream);
+
 /* The small kernels around the two grouped GEMMs of a mixture-of-experts layer.
  * They have counterparts in every build of the reference (also on ROCm):
  *   sonar_moe_align_block_size -> _moe_C::moe_align_block_size

@@ -20,6 +20,7 @@
 
 #include "dequant.hpp"
 #include "gemm_plan.hpp"
+#include "moe_activation.hpp"
 
 namespace sonar {
 namespace {
@@ -69,6 +70,11 @@ struct TileParams {
   int a_by_slot;               // grouped: row of A = slot index (a column-permuted copy made per slot), else row id / top_k
   long expert_b_stride;        // uint4 units between experts in b
   long expert_s_stride, expert_z_stride, expert_bias_stride;  // elements between experts
+  // grouped, wide kernel: the gated activation of C, (rows_total, size_n / 2), in place of C; `gated_halves`: silu_and_mul of the
+  // columns' two halves, else swigluoai_and_mul of alternating columns
+  uint16_t* gated;
+  int gated_halves;
+  float gated_limit, gated_alpha;
 };
 
 // 16 bytes (8 consecutive k) of row `row` of A, gathered through perm when given.
@@ -976,6 +982,86 @@ struct OnesRow {
 __device__ __attribute__((aligned(128))) const OnesRow<false> kOnesInt8 = {};
 __device__ __attribute__((aligned(128))) const OnesRow<true> kOnesFp8 = {};
 
+// The end of a grouped tile whose rows go through the gated activation: the rows lie turned in LDS as wide_tile left them, a
+// wavefront's at wave * kRows * 128, and every value is rounded as the GEMM's result would be, so that the bits are those of
+// the GEMM and the activation after one another.  Bound by vector instructions (20 to 30 a result).  A launch and two passes over
+// the rows of gate and up less; us a layer, activation in a launch of its own -> here: Mixtral-8x7B shapes, 4096 tokens 2500 -> 2395,
+// 2000 tokens 1310 -> 1255; 8 experts 1024 x 2688, AWQ, 6002 tokens 298 -> 273; 16 of 2048 x 2816, 3000 tokens, top 4 481 -> 450; 64
+// MXFP4 experts 2048 x 768, 4000 tokens, top 8 437 -> 426; 32 of 2880 x 2880, swigluoai, 2000 tokens, top 4 480 -> 465 (of which the
+// tiles take 15 us longer and the activation took 30), 6000 tokens 1171 -> 1131.
+//   alternating columns: a wavefront's own 64 columns are 32 results; `strip` is its strip
+//   halves: wavefronts 0 and 1 have two strips of the gate half, 2 and 3 the same strips of the up half; wavefront w
+//   then takes half w / 2 of the rows of strip `strip` + w % 2
+// The ids of the rows go through `ids_lds`, 1 KiB of the wavefront's own, so that the rows are a loop: unrolled, its code would be
+// fetched once a tile (with the division and expf of the library as well: 467 us for the 2000 tokens above that take 457
+// with a launch of their own).
+template <typename T, int RB>
+__device__ __forceinline__ void store_gated(const TileParams& p, uint32_t a_lds, uint32_t ids_lds, int wave, int lane, int strip,
+                                            const int (&ids)[RB]) {
+  constexpr int kRows = 16 * RB;
+  const int r8 = lane >> 3;
+#pragma unroll
+  for (int mb = 0; mb < RB; ++mb)
+    asm volatile("ds_write_b32 %0, %1 offset:%2" ::"v"(ids_lds + 4 * (lane & 15)), "v"(ids[mb]), "i"(mb * 64) : "memory");
+  const bool halves = p.gated_halves != 0;
+  uint32_t at = a_lds + r8 * 128 + (((lane & 7) ^ r8) * 16), row_at = ids_lds + 4 * r8;
+  if (halves) {
+    at += (wave & 1) * (kRows * 128) + (wave >> 1) * (RB * 1024);
+    row_at += (wave >> 1) * (8 * RB * 4);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();   // the rows of the other wavefronts
+  } else {
+    at += wave * (kRows * 128);
+  }
+  uint16_t* to_strip = p.gated + (halves ? (strip + (wave & 1)) * kStripN + 8 * (lane & 7) : strip * (kStripN / 2) + 4 * (lane & 7));
+  const int steps = halves ? RB / 4 : RB / 2;   // of 32 rows
+#pragma unroll 1
+  for (int i = 0; i < steps; ++i, at += 4096, row_at += 128) {
+    u32x4_t g[4], v[4];
+    int row[4];
+#define SONAR_READ_ROWS(IDS)                                                                                       \
+  "ds_read_b32 %4, " IDS "\n\tds_read_b32 %5, " IDS " offset:32\n\tds_read_b32 %6, " IDS " offset:64\n\t"          \
+  "ds_read_b32 %7, " IDS " offset:96\n\t"
+#define SONAR_READ_LINES(A, B, C, D, AT)                                                                           \
+  "ds_read_b128 " A ", " AT "\n\tds_read_b128 " B ", " AT " offset:1024\n\tds_read_b128 " C ", " AT " offset:2048\n\t" \
+  "ds_read_b128 " D ", " AT " offset:3072\n\t"
+#define SONAR_LINES_AND_ROWS "=&v"(g[0]), "=&v"(g[1]), "=&v"(g[2]), "=&v"(g[3]), "=&v"(row[0]), "=&v"(row[1]), "=&v"(row[2]), "=&v"(row[3])
+    if (halves) {
+      asm volatile(SONAR_READ_ROWS("%12") SONAR_READ_LINES("%0", "%1", "%2", "%3", "%13")
+                       SONAR_READ_LINES("%8", "%9", "%10", "%11", "%14") "s_waitcnt lgkmcnt(0)"
+                   : SONAR_LINES_AND_ROWS, "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3])
+                   : "v"(row_at), "v"(at), "v"(at + 2 * (kRows * 128))
+                   : "memory");
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        u32x4_t o;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          o[j] = (uint32_t)silu_times<T>((uint16_t)g[u][j], (uint16_t)v[u][j]) |
+                 ((uint32_t)silu_times<T>((uint16_t)(g[u][j] >> 16), (uint16_t)(v[u][j] >> 16)) << 16);
+        if (row[u] >= 0) *reinterpret_cast<u32x4_t*>(to_strip + (long)row[u] * (p.size_n / 2)) = o;
+      }
+    } else {
+      asm volatile(SONAR_READ_ROWS("%8") SONAR_READ_LINES("%0", "%1", "%2", "%3", "%9") "s_waitcnt lgkmcnt(0)"
+                   : SONAR_LINES_AND_ROWS
+                   : "v"(row_at), "v"(at)
+                   : "memory");
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        uint32_t o[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          o[j] = swiglu_oai<T>((uint16_t)g[u][j], (uint16_t)(g[u][j] >> 16), p.gated_limit, p.gated_alpha);
+        if (row[u] >= 0)
+          *reinterpret_cast<uint2*>(to_strip + (long)row[u] * (p.size_n / 2)) = make_uint2(o[0] | (o[1] << 16), o[2] | (o[3] << 16));
+      }
+    }
+#undef SONAR_READ_ROWS
+#undef SONAR_READ_LINES
+#undef SONAR_LINES_AND_ROWS
+  }
+}
+
 // G32: a scale (and zero point) per 32 rows, i.e. one row of them per k block: MXFP4 always, integer codes when asked.
 // NV (with FP4): NVFP4, a scale per 16 rows: the row of a k block then holds two groups of 128 bytes (the copy
 // fetches one per half of the wavefront), and a lane, whose eight rows of a k block lie in one group, reads group
@@ -1027,7 +1113,10 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
   const int strips_here = min(kTileN / kStripN, p.size_n / kStripN - strip0);
   const bool active = wave < strips_here;
   // a wavefront past the last strip works on the last strip again and stores nothing
-  const int strip = strip0 + (active ? wave : strips_here - 1);
+  int strip = strip0 + (active ? wave : strips_here - 1);
+  // silu_and_mul at the end: a tile is 128 columns of the gate and the same 128 of the up half (the host checks: all strips are there)
+  if (GROUPED && p.gated != nullptr && p.gated_halves)
+    strip = 2 * tile_n + (wave & 1) + (wave >> 1) * (p.size_n / (2 * kStripN));
 
   // ---- sources (regions of A as in marlin_tile_async_kernel; wavefront w fills RB / 2 regions)
   // Memory operations take a scalar base and a 32-bit offset a lane where they can: with a 64-bit address a lane each holds up the
@@ -1507,6 +1596,12 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
     }
   }
   const int r8 = lane >> 3;
+  if constexpr (GROUPED) {
+    if (p.gated != nullptr) {
+      store_gated<T, RB>(p, a_lds, s_lds, wave, lane, p.gated_halves ? 2 * tile_n : strip, ids);
+      return;
+    }
+  }
   const uint32_t turn_out = turn + r8 * 128 + (((lane & 7) ^ r8) * 16);
   uint16_t* c_strip = p.c + strip * kStripN + 8 * (lane & 7);
   const bool c_aligned = (reinterpret_cast<uintptr_t>(p.c) & 15) == 0;
@@ -2193,7 +2288,7 @@ int moe_tile_gemm(const void* a, void* c, const uint32_t* b, const void* bias, c
                   const int32_t* num_post_pad, const float* topk_weights, int64_t top_k, int mul_topk,
                   int64_t num_experts, int32_t* table, int dtype, int64_t size_m, int64_t size_n, int64_t size_k,
                   int64_t num_groups, int group_size, int a_by_slot, bool fp4, int bits, bool fp8, void* partial,
-                  size_t partial_bytes, hipStream_t st) {
+                  size_t partial_bytes, GatedOutput* gated, hipStream_t st) {
   const int max_tiles = moe_tile_max(sorted_len, num_experts);
   const int blocks_max = (int)((sorted_len + 63) / 64);
   TileParams p = {};
@@ -2251,6 +2346,15 @@ int moe_tile_gemm(const void* a, void* c, const uint32_t* b, const void* bias, c
     if (least_tiles > (size_k >= 64 * kTileK ? 512 : 192)) p.partial = nullptr;
     if (p.partial != nullptr)
       p.partial_small = reinterpret_cast<float4*>(static_cast<char*>(partial) + moe_partial_bytes_of(kTileM));
+  }
+  // The activation at the end of the tiles that are not cut along K (those cut are summed by another kernel)
+  if (gated != nullptr && wide && p.partial == nullptr && ((uintptr_t)gated->out) % 16 == 0 &&
+      (gated->kind == 0 ? size_n % (2 * 2 * kStripN) == 0 : gated->kind == SONAR_ACT_SWIGLUOAI && gated->limit > 0.f)) {
+    p.gated = static_cast<uint16_t*>(gated->out);
+    p.gated_halves = gated->kind == 0;
+    p.gated_limit = gated->limit;
+    p.gated_alpha = gated->alpha;
+    gated->done = true;
   }
   auto build_table = [&](auto kernel, int threads) {
     kernel<<<1, threads, 0, st>>>(expert_ids, num_post_pad, blocks_max, 64, (int)num_experts, table, table_small, max_tiles,

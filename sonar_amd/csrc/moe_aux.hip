@@ -4,6 +4,7 @@
 // csrc/libtorch_stable/moe/moe_align_sum_kernels.cu:626-725,759+ and the
 // silu_and_mul of csrc/libtorch_stable/activation_kernels.cu for fp16 / bf16.
 #include "common.hpp"
+#include "moe_activation.hpp"
 
 namespace sonar {
 namespace {
@@ -181,15 +182,6 @@ __global__ __launch_bounds__(256) void moe_align_place_kernel(const int32_t* __r
   }
 }
 
-template <typename T>
-__device__ __forceinline__ float to_f32(uint16_t b);
-template <>
-__device__ __forceinline__ float to_f32<_Float16>(uint16_t b) { return (float)__builtin_bit_cast(_Float16, b); }
-template <>
-__device__ __forceinline__ float to_f32<__bf16>(uint16_t b) { return __builtin_bit_cast(float, (uint32_t)b << 16); }
-template <typename T>
-__device__ __forceinline__ uint16_t from_f32(float f) { return __builtin_bit_cast(uint16_t, (T)f); }
-
 // out[r][c] = T(T(silu(x[r][c])) * x[r][d + c]): the activation is rounded to
 // the tensor type before the product, as act_and_mul does.
 template <typename T>
@@ -209,10 +201,7 @@ __global__ __launch_bounds__(256) void silu_and_mul_kernel(uint16_t* __restrict_
       uint32_t o = 0;
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        const float x = to_f32<T>((uint16_t)(gw[w] >> (16 * h)));
-        const float y = to_f32<T>((uint16_t)(uw[w] >> (16 * h)));
-        const float s = to_f32<T>(from_f32<T>(x / (1.0f + __expf(-x))));
-        o |= (uint32_t)from_f32<T>(s * y) << (16 * h);
+        o |= (uint32_t)silu_times<T>((uint16_t)(gw[w] >> (16 * h)), (uint16_t)(uw[w] >> (16 * h))) << (16 * h);
       }
       ow[w] = o;
     }
@@ -252,9 +241,7 @@ __device__ __forceinline__ uint16_t gated_activation(uint16_t gate_bits, uint16_
     const float act = to_f32<T>(from_f32<T>(0.5f * gate * (1.0f + tanhf(inner))));
     return from_f32<T>(act * up);
   } else if constexpr (KIND == kSwigluOai) {
-    const float g = fminf(gate, limit);
-    const float u = fmaxf(fminf(up, limit), -limit);
-    return from_f32<T>((u + 1.0f) * g / (1.0f + expf(-g * alpha)));
+    return swiglu_oai<T>(gate_bits, up_bits, limit, alpha);
   } else if constexpr (KIND == kSitu) {
     const float gate_out = alpha * tanhf(gate * (1.0f / alpha)) / (1.0f + expf(-gate));
     const float up_out = beta > 0.0f ? beta * tanhf(up * (1.0f / beta)) : up;

@@ -1014,14 +1014,22 @@ struct Routing {
   const float* topk_weights;
 };
 
+// A gated activation that a grouped GEMM may write to `out` in place of its result (sonar_moe_wna16_marlin_gemm_gated).
+struct Gated {
+  void* out;
+  int activation;
+  float limit, alpha;
+  int written;
+};
+
 // The grouped GEMM on 16-bit activations: checks of a and the expert matrices, and the launch into
-// `c` (size_m * top_k rows of a's type).  The kernels take no workspace.
+// `c` (size_m * top_k rows of a's type) or `gated`.  The kernels take no workspace.
 void moe_gemm_16bit(const Tensor& a, void* c, const Tensor& b_q_weight, const OptTensor& b_bias_or_none,
                     const Tensor& b_scales, const OptTensor& a_scales, const OptTensor& global_scale,
                     const OptTensor& b_zeros_or_none, const OptTensor& g_idx_or_none, const OptTensor& perm_or_none,
                     const Routing& route, int64_t moe_block_size, int64_t top_k, bool mul_topk_weights,
                     int64_t b_type_id, int64_t size_m, int64_t size_n, int64_t size_k, bool is_k_full,
-                    bool use_atomic_add, bool use_fp32_reduce, bool is_zp_float) {
+                    bool use_atomic_add, bool use_fp32_reduce, bool is_zp_float, Gated* gated = nullptr) {
   TORCH_CHECK(a.scalar_type() == at::kHalf || a.scalar_type() == at::kBFloat16, "unsupported `a` scalar_type");
   const int dtype = dtype_code(a);
   check_b_type(b_type_id);
@@ -1117,6 +1125,21 @@ void moe_gemm_16bit(const Tensor& a, void* c, const Tensor& b_q_weight, const Op
   Tensor scratch;
   if (scratch_bytes > 0) scratch = at::empty({(int64_t)scratch_bytes}, a.options().dtype(at::kByte));
 
+  if (gated != nullptr) {
+    TORCH_CHECK(!nvfp4 || perm == nullptr, "act-order is not supported with float4_e2m1f weights");
+    const Tensor scales = nvfp4 ? nvfp4_scales_as_16bit(b_scales, a.scalar_type())
+                                : fp4 || mxfp8 ? mx_scales_as_bf16(b_scales, mxfp8 ? 120 : 0) : b_scales;
+    raise_if_failed(sonar_moe_wna16_marlin_gemm_gated(
+        a.const_data_ptr(), c, static_cast<const uint32_t*>(native.const_data_ptr()), SONAR_LAYOUT_GFX950,
+        opt_ptr(b_bias_or_none), scales.const_data_ptr(),
+        nvfp4 ? static_cast<const float*>(global_scale->const_data_ptr()) : nullptr,
+        has_zp ? static_cast<const uint32_t*>(b_zeros_or_none->const_data_ptr()) : nullptr, g_idx, perm,
+        scratch_bytes > 0 ? scratch.mutable_data_ptr() : nullptr, scratch_bytes, route.sorted_ids, route.sorted_len,
+        route.expert_ids, route.past_padded, route.topk_weights, moe_block_size, top_k, mul_topk_weights ? 1 : 0, experts,
+        dtype, b_type_id, size_m, size_n, size_k, num_groups, is_k_full ? 1 : 0, gated->out, gated->activation,
+        gated->limit, gated->alpha, &gated->written, current_stream(a)));
+    return;
+  }
   if (nvfp4) {
     TORCH_CHECK(perm == nullptr, "act-order is not supported with float4_e2m1f weights");
     raise_if_failed(sonar_moe_wna16_marlin_gemm_nvfp4(
@@ -1330,13 +1353,21 @@ void fused_moe(Tensor& output, const Tensor& hidden, const Tensor& w1, const Ten
   const Routing route{sorted_ids, sorted_len, expert_ids, past_padded,
                       static_cast<const float*>(topk_weights.const_data_ptr())};
   const int dtype = dtype_code(hidden);
+  // The GEMM may form the activation itself; not where its input would be overwritten meanwhile.
+  auto range = [](const Tensor& t, int64_t values) {
+    const auto at = reinterpret_cast<uintptr_t>(t.const_data_ptr());
+    return std::make_pair(at, at + (uintptr_t)values * 2);
+  };
+  const auto in = range(hidden, m * k), mid = range(between, rows * n);
+  Gated gated{between.mutable_data_ptr(), (int)activation, (float)limit, (float)alpha, 0};
   moe_gemm_16bit(hidden, wide.mutable_data_ptr(), w1, bias1, scale1, std::nullopt, global_scale1, zeros1, g_idx1, perm1,
                  route, block_size, topk, router_weight_on_input, b_type_id, m, 2 * n, k, is_k_full, false, true,
-                 false);
-  raise_if_failed(activation == 0
-                      ? sonar_silu_and_mul(between.mutable_data_ptr(), wide.const_data_ptr(), rows, n, dtype, stream)
-                      : sonar_moe_activation(between.mutable_data_ptr(), wide.const_data_ptr(), rows, n,
-                                             (int)activation, (float)limit, (float)alpha, (float)beta, dtype, stream));
+                 false, in.first < mid.second && mid.first < in.second ? nullptr : &gated);
+  if (!gated.written)
+    raise_if_failed(activation == 0
+                        ? sonar_silu_and_mul(between.mutable_data_ptr(), wide.const_data_ptr(), rows, n, dtype, stream)
+                        : sonar_moe_activation(between.mutable_data_ptr(), wide.const_data_ptr(), rows, n,
+                                               (int)activation, (float)limit, (float)alpha, (float)beta, dtype, stream));
   const Tensor down_in = between.dim() == 2 && between.size(0) == rows && between.size(1) == n
                              ? between
                              : between.view({-1}).narrow(0, 0, rows * n).view({rows, n});

@@ -1,0 +1,94 @@
+"""The grouped tile kernels form the gated activation of their rows themselves: a layer gives the bits of the GEMM and the
+activation kernel after one another, in every weight format, with both tile sizes, a ragged last tile of columns (alternating gate
+and up only: halves need whole tiles), experts without rows, a bias and the routing weight on the input; the gate and up rows are
+not written then.  Activations and widths that the tiles do not take, and tiles cut along K, go the old way."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from sonar_amd import fused_moe
+from sonar_amd.scalar_type import scalar_types
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+def _experts(gen, kind, e, k, n, dtype):
+    """Random experts in the Marlin layout: weights, scales, zero points."""
+    words = 4 if kind == "uint8b128" else 2
+    q = torch.randint(-2 ** 31, 2 ** 31 - 1, (e, k // 16, words * n), dtype=torch.int32, device=DEV, generator=gen)
+    if kind == "mxfp4":
+        s = torch.randint(117, 122, (e, k // 32, n), dtype=torch.uint8, device=DEV, generator=gen).view(torch.float8_e8m0fnu)
+    else:
+        s = (torch.rand((e, k // 64, n), device=DEV, generator=gen) * 9e-3 + 1e-3).to(dtype)
+        s = s / 16 if kind == "uint8b128" else s
+    z = None
+    if kind == "uint4":
+        z = torch.randint(-2 ** 31, 2 ** 31 - 1, (e, k // 64, n // 8), dtype=torch.int32, device=DEV, generator=gen)
+    return q, s, z
+
+
+@pytest.mark.parametrize("kind,dtype", [("uint4b8", torch.float16), ("uint4", torch.bfloat16), ("mxfp4", torch.bfloat16),
+                                        ("uint8b128", torch.float16)])
+@pytest.mark.parametrize("activation,inter,k,in_tiles", [("silu", 384, 320, True), ("silu", 320, 320, False),
+                                                         ("swigluoai", 384, 192, True), ("swigluoai", 352, 320, True),
+                                                         ("gelu", 384, 320, False), ("silu", 384, 1024, False)])
+@pytest.mark.parametrize("on_input", [False, True])
+def test_layer(kind, dtype, activation, inter, k, in_tiles, on_input):
+    if kind != "mxfp4" and inter % 64:   # the down projection's groups
+        inter = 448
+    m, e, top_k = 1500 if kind == "mxfp4" else 700, 6, 2   # (MXFP4: more than marlin_mid_gemm takes)
+    gen = torch.Generator(device=DEV).manual_seed(inter + k)
+    w1, s1, z1 = _experts(gen, kind, e, k, 2 * inter, dtype)
+    w2, s2, z2 = _experts(gen, kind, e, inter, k, dtype)
+    bias1 = (torch.randn((e, 2 * inter), device=DEV, generator=gen) * 0.1).to(dtype)
+    x = torch.randn((m, k), device=DEV, generator=gen).to(dtype)
+    logits = torch.randn((m, e), device=DEV, generator=gen)
+    logits[:, 0] += 3.0    # most tokens: tiles of 256 rows
+    logits[:, 2] -= 100.0  # none
+    weights, ids = torch.topk(torch.softmax(logits, dim=1), top_k, dim=1)
+    weights, ids = weights.contiguous(), ids.to(torch.int32)
+    wtype = {"uint4b8": scalar_types.uint4b8, "uint4": scalar_types.uint4, "mxfp4": scalar_types.float4_e2m1f,
+             "uint8b128": scalar_types.uint8b128}[kind]
+    assert fused_moe.moe_block_size(m, top_k, e) == 64 and 2 * inter > k or k == 1024
+
+    def layer(**kw):
+        return fused_moe.fused_marlin_moe(x, w1, w2, bias1, None, s1, s2, weights, ids, wtype.id, on_input,
+                                          activation=activation, w1_zeros=z1, w2_zeros=z2, **kw)
+
+    rows = m * top_k
+    cache13 = torch.full((rows * max(2 * inter, k),), -7.0, dtype=dtype, device=DEV)
+    cache2 = torch.empty((rows * inter,), dtype=dtype, device=DEV)
+    got = layer(intermediate_cache13=cache13, intermediate_cache2=cache2)
+    if 2 * inter > k:
+        assert bool((cache13[rows * k:] == -7.0).all()) == in_tiles
+    between = torch.empty((rows, inter), dtype=dtype, device=DEV)
+
+    def after(name, out, rows_in, **kw):   # a function of the caller's own: two calls, the GEMM and the activation
+        fused_moe.apply_moe_activation(name, out, rows_in, **kw)
+        between.copy_(out)
+
+    want = layer(activation_func=after)
+    assert bool(torch.isfinite(want.float()).all())
+    assert torch.equal(cache2.view(rows, inter), between)
+    assert torch.equal(got, want)
+
+
+def test_input_in_the_place_of_the_rows_between():
+    """hidden_states inside intermediate_cache2: the GEMM reads all of it before anything is written there."""
+    m, e, top_k, k, inter, dtype = 700, 3, 2, 320, 384, torch.bfloat16
+    gen = torch.Generator(device=DEV).manual_seed(1)
+    w1, s1, _ = _experts(gen, "uint4b8", e, k, 2 * inter, dtype)
+    w2, s2, _ = _experts(gen, "uint4b8", e, inter, k, dtype)
+    cache2 = torch.empty((m * top_k * inter,), dtype=dtype, device=DEV)
+    x = torch.randn((m, k), device=DEV, generator=gen).to(dtype)
+    inside = cache2[:m * k].view(m, k)
+    weights, ids = torch.topk(torch.rand((m, e), device=DEV, generator=gen), top_k, dim=1)
+    weights, ids = weights.contiguous(), ids.to(torch.int32)
+    want = fused_moe.fused_marlin_moe(x, w1, w2, None, None, s1, s2, weights, ids, scalar_types.uint4b8.id)
+    inside.copy_(x)
+    got = fused_moe.fused_marlin_moe(inside, w1, w2, None, None, s1, s2, weights, ids, scalar_types.uint4b8.id,
+                                     intermediate_cache2=cache2)
+    assert torch.equal(got, want)
