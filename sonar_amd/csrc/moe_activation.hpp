@@ -34,7 +34,7 @@ __device__ __forceinline__ uint16_t silu_times(uint16_t gate_bits, uint16_t up_b
 // swigluoai_and_mul: T((u + 1) g / (1 + exp(-alpha g))), g = min(gate, limit), u = clamp(up, -limit, limit).  The power of two
 // takes -alpha log2(e) g with what its rounding leaves, so that the exponential is as close as expf's (which spends twice the
 // instructions).  Against expf and a division: 51 -> 39 instructions a result in the kernel of moe_aux.hip; the same relative error
-// against 64 bits (fp16 2.07e-4, bf16 1.66e-3), 14 of 524288 results in a tie rounded the other way.
+// against 64 bits (fp16 2.07e-4, bf16 1.66e-3), 8 of 1048576 results in a tie rounded the other way.
 template <typename T>
 __device__ __forceinline__ uint16_t swiglu_oai(uint16_t gate_bits, uint16_t up_bits, float limit, float alpha) {
   constexpr float kLog2e = 1.44269504f, kLog2eRest = 1.92596303e-8f, kLn2 = 0.693147181f;

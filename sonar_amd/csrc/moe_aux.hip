@@ -3,6 +3,8 @@
 // activation, and the sum over a token's experts.  They restate
 // csrc/libtorch_stable/moe/moe_align_sum_kernels.cu:626-725,759+ and the
 // silu_and_mul of csrc/libtorch_stable/activation_kernels.cu for fp16 / bf16.
+#include <algorithm>
+
 #include "common.hpp"
 #include "moe_activation.hpp"
 
@@ -11,8 +13,12 @@ namespace {
 
 constexpr int kAlignThreads = 1024;
 constexpr int kAlignWaves = kAlignThreads / 64;
-// Experts up to which one workgroup counts and places: its wavefronts keep a histogram each (48 KiB of LDS).
+// Experts up to which one launch counts and places: a workgroup's wavefronts keep a histogram each (54 KiB of LDS with two more).
 constexpr int kAlignOneLaunchExperts = 768;
+// Workgroups of a launch: one up to 5000 slots (counting the other segments costs one more round trip; us, one workgroup against
+// one for every 1024 slots, back to back: 2508 slots, 8 experts 5.5 / 6.9, 4000 6.1 / 6.9, 8192 8.8 / 7.3, 8000 on 32 9.2 / 7.3, 32000
+// on 64 31.6 / 9.5, 65536 on 256 67.6 / 12.7), and up to 64, after which they take longer segments (131072 on 64: 114 -> 20).
+constexpr int kAlignOneWorkgroup = 5000, kAlignMost = 64;
 
 // Inclusive sum over the lanes of a wavefront.
 __device__ __forceinline__ int wave_inclusive_sum(int v) {
@@ -24,16 +30,21 @@ __device__ __forceinline__ int wave_inclusive_sum(int v) {
   return v;
 }
 
-// One workgroup: per-expert counts, padded offsets, expert id of every block, the padded total and
+// Per-expert counts, padded offsets, expert id of every block, the padded total and
 // the sentinels of sorted_token_ids.  With `place` it also places the slots: every wavefront owns
-// a contiguous share of them and a histogram row; the rows' prefix sums give each wavefront its first
+// a contiguous share of its workgroup's and a histogram row; the rows' prefix sums give each wavefront its first
 // position per expert, and inside 64 slots a lane's rank among the lanes of the same expert comes from
 // one ballot per bit of the expert number, so the slots of an expert keep ascending order.  Without it
 // (more experts than the histograms have room for) offsets[e] is left for the placement kernel.
-// Latency bound: 8000 slots on 32 experts 9 + 42 us as two launches whose second walked all slots once
-// per expert, 7 us like this (14 us in a kernel trace of the whole layer, at the clock it runs at there).  Eight rounds of
-// slots are read at a time and, up to 8192 slots, once (one round after the other, twice: the whole layer of 2000 tokens on 32 experts
-// 488 us, 484 now; 8192 tokens with eight experts each 590 and 555).
+// Several workgroups take a segment of the slots each and count all of them: two more rows hold what lies before and behind the
+// segment, so that nobody waits for another, and placing, whose scattered stores one compute unit takes long for, is spread.
+// Latency bound with few slots, which one workgroup takes (kAlignOneWorkgroup); with many by their counting.  8000 slots on 32
+// experts: 9 + 42 us as two launches whose second walked all slots once per expert, 9.2 in one workgroup (eight rounds of slots
+// read at a time and, up to 8192 slots, once), 7.3 like this; a layer of 4000 tokens on 64 experts, top 8 427 -> 404.
+__host__ __device__ __forceinline__ int align_share(int numel, int workgroups) {   // slots of a wavefront
+  const int per_wave = (int)(((long)numel + (long)workgroups * kAlignWaves - 1) / ((long)workgroups * kAlignWaves));
+  return (per_wave + 63) / 64 * 64;
+}
 template <int kBatch>
 __global__ __launch_bounds__(kAlignThreads) void moe_align_count_kernel(
     const int32_t* __restrict__ topk_ids, int numel, int num_experts, int block_size,
@@ -46,7 +57,8 @@ __global__ __launch_bounds__(kAlignThreads) void moe_align_count_kernel(
   int32_t* wave_sum = stop + num_experts;
   int32_t* hist = wave_sum + kAlignWaves;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int rows = place ? kAlignWaves : 1;
+  const int many = gridDim.x > 1 ? 1 : 0;   // rows of the histogram: slots before the segment, the wavefronts' shares, slots behind
+  const int rows = place ? kAlignWaves + 2 * many : 1;
   for (int i = tid; i < rows * num_experts; i += kAlignThreads) hist[i] = 0;
   __syncthreads();
   // The experts (-1: none) of up to kBatch rounds of 64 slots from `base` on, all asked for before the first is waited for.
@@ -65,10 +77,45 @@ __global__ __launch_bounds__(kAlignThreads) void moe_align_count_kernel(
       if (held[r] >= num_experts) held[r] = -1;   // (and none of a map's negative ones)
     }
   };
-  // a wavefront's share: whole rounds of 64 slots
-  const int share = (((numel + kAlignWaves - 1) / kAlignWaves) + 63) / 64 * 64;
-  const int from = min(numel, wave * share), to = min(numel, from + share);
-  int32_t* mine = hist + (place ? wave * num_experts : 0);
+  // a wavefront's share of the segment: whole rounds of 64 slots
+  const int share = align_share(numel, gridDim.x);
+  const int segment = min(numel, (int)blockIdx.x * kAlignWaves * share), segment_end = min(numel, segment + kAlignWaves * share);
+  const int from = min(segment_end, segment + wave * share), to = min(segment_end, from + share);
+  int32_t* mine = hist + (place ? (many + wave) * num_experts : 0);
+  if (many) {
+    // the other slots, in any order, four a load where topk_ids lies so
+    const bool vectors = (reinterpret_cast<uintptr_t>(topk_ids) & 15) == 0;
+    auto count_others = [&](int lo, int hi, int32_t* row) {
+      for (int base = lo; base < hi; base += 16 * kAlignThreads) {
+        int4 v[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int at = base + 4 * (kAlignThreads * r + tid);
+          if (vectors && at + 4 <= hi) {
+            v[r] = *reinterpret_cast<const int4*>(topk_ids + at);
+          } else {
+            v[r].x = at < hi ? topk_ids[at] : -1;
+            v[r].y = at + 1 < hi ? topk_ids[at + 1] : -1;
+            v[r].z = at + 2 < hi ? topk_ids[at + 2] : -1;
+            v[r].w = at + 3 < hi ? topk_ids[at + 3] : -1;
+          }
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int e4[4] = {v[r].x, v[r].y, v[r].z, v[r].w};
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            int e = e4[j];
+            if (e < 0 || e >= num_experts) continue;
+            if (expert_map) e = expert_map[e];
+            if (e >= 0 && e < num_experts) atomicAdd(&row[e], 1);
+          }
+        }
+      }
+    };
+    count_others(0, segment, hist);
+    count_others(segment_end, numel, hist + (kAlignWaves + 1) * num_experts);
+  }
   for (int base = from; base < to; base += 64 * kBatch) {
     fetch(base, to);
 #pragma unroll
@@ -109,16 +156,17 @@ __global__ __launch_bounds__(kAlignThreads) void moe_align_count_kernel(
   const int total = carry;
   if (tid == 0) {
     begin[num_experts] = total;
-    num_post_pad[0] = total;
+    if (blockIdx.x == 0) num_post_pad[0] = total;
   }
   __syncthreads();
-  // sentinels: behind every expert's slots and behind the last run
-  for (int e = wave; e < num_experts; e += kAlignWaves)
+  // sentinels: behind every expert's slots and behind the last run (each workgroup some of them, and of the blocks)
+  const int all_waves = gridDim.x * kAlignWaves, all_threads = gridDim.x * kAlignThreads;
+  for (int e = blockIdx.x * kAlignWaves + wave; e < num_experts; e += all_waves)
     for (int i = stop[e] + lane; i < begin[e + 1]; i += 64) sorted_ids[i] = numel;
-  for (int i = total + tid; i < sorted_len; i += kAlignThreads) sorted_ids[i] = numel;
+  for (int i = total + blockIdx.x * kAlignThreads + tid; i < sorted_len; i += all_threads) sorted_ids[i] = numel;
   if (!place)
     for (int e = tid; e < num_experts; e += kAlignThreads) offsets[e] = begin[e];
-  for (int b = tid; b < expert_len; b += kAlignThreads) {
+  for (int b = blockIdx.x * kAlignThreads + tid; b < expert_len; b += all_threads) {
     const int start = b * block_size;
     int e = -1;
     if (start < total) {
@@ -352,12 +400,16 @@ extern "C" int sonar_moe_align_block_size(const int32_t* topk_ids, int64_t numel
                 "moe_align_block_size: NULL argument");
   hipStream_t st = (hipStream_t)stream;
   const bool place = num_experts <= kAlignOneLaunchExperts;
-  const size_t lds = (size_t)(2 * num_experts + 1 + kAlignWaves + (place ? kAlignWaves : 1) * num_experts) * sizeof(int32_t);
+  // a workgroup for every 1024 slots: a round of 64 a wavefront
+  const int workgroups =
+      place && numel > kAlignOneWorkgroup ? (int)std::min<int64_t>((numel + kAlignThreads - 1) / kAlignThreads, kAlignMost) : 1;
+  const size_t lds = (size_t)(2 * num_experts + 1 + kAlignWaves +
+                              (place ? kAlignWaves + (workgroups > 1 ? 2 : 0) : 1) * num_experts) * sizeof(int32_t);
   // (eight rounds at a time: 0.4 us longer where a wavefront has one)
-  auto* count = numel > 64 * kAlignWaves ? moe_align_count_kernel<8> : moe_align_count_kernel<1>;
+  auto* count = align_share((int)numel, workgroups) > 64 ? moe_align_count_kernel<8> : moe_align_count_kernel<1>;
   if (lds > 64 * 1024)   // from 5456 experts on (8192: 98372 bytes); HIP promises no more unasked, though ROCm 7.2 gives it
     SONAR_HIP(hipFuncSetAttribute((const void*)count, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  count<<<1, kAlignThreads, lds, st>>>(topk_ids, (int)numel, (int)num_experts, (int)block_size, sorted_token_ids,
+  count<<<workgroups, kAlignThreads, lds, st>>>(topk_ids, (int)numel, (int)num_experts, (int)block_size, sorted_token_ids,
                                        (int)sorted_len, expert_ids, (int)expert_len, num_tokens_post_pad, expert_map,
                                        offsets_scratch, place);
   if (int rc = launch_status("moe_align_count_kernel")) return rc;
