@@ -421,7 +421,19 @@ int sonar_moe_wna16_marlin_gemm_nvfp4(
  * dtype[size_m * top_k][size_n / 2] is written, c is left as it was and *gated_written is 1; the bits are those of the GEMM and the
  * activation after one another.  Otherwise *gated_written is 0 and c holds the GEMM's result.  `activation` 0 is sonar_silu_and_mul,
  * else a SONAR_ACT_* kind with its limit and alpha (formed here: 0 and SONAR_ACT_SWIGLUOAI).  gated must not overlap the inputs.
- * global_scale != NULL: NVFP4.  The other arguments as for sonar_moe_wna16_marlin_gemm. */
+ * global_scale != NULL: NVFP4.  The other arguments as for sonar_moe_wna16_marlin_gemm.
+ * next (may be NULL): sizes of the layer's next GEMM over the same routing, experts of the same type, and `table` of table_bytes
+ * (sonar_moe_marlin_gemm_scratch_bytes(sorted_len, moe_block_size, size_n, 64)) of device memory, where this call may lay down what
+ * that GEMM otherwise begins with; that call, on the same stream and with the routing unchanged, gets the struct as `ready`. */
+typedef struct {
+  int32_t* table;
+  size_t table_bytes;
+  int64_t size_n, size_k, num_groups;
+  /* written by the call */
+  int built, tiles_n, k_steps, may_split;
+  const int32_t* expert_ids;
+  int64_t sorted_len;
+} sonar_moe_tables;
 int sonar_moe_wna16_marlin_gemm_gated(
     const void* a, void* c, const uint32_t* b_q_weight, int b_layout,
     const void* b_bias, const void* b_scales, const float* global_scale,
@@ -433,7 +445,7 @@ int sonar_moe_wna16_marlin_gemm_gated(
     int64_t num_experts, int dtype, int64_t b_type_id, int64_t size_m,
     int64_t size_n, int64_t size_k, int64_t num_groups, int is_k_full,
     void* gated, int activation, float limit, float alpha, int* gated_written,
-    void* stream);
+    sonar_moe_tables* next, const sonar_moe_tables* ready, void* stream);
 
 /* The small kernels around the two grouped GEMMs of a mixture-of-experts layer.
  * They have counterparts in every build of the reference (also on ROCm):

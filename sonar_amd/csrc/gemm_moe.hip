@@ -28,7 +28,7 @@ int moe_tile_gemm(const void* a, void* c, const uint32_t* b, const void* bias, c
                   const int32_t* num_post_pad, const float* topk_weights, int64_t top_k, int mul_topk,
                   int64_t num_experts, int32_t* table, int dtype, int64_t size_m, int64_t size_n, int64_t size_k,
                   int64_t num_groups, int group_size, int a_by_slot, bool fp4, int bits, bool fp8, void* partial,
-                  size_t partial_bytes, GatedOutput* gated, hipStream_t st);
+                  size_t partial_bytes, const MoeLayerCall& layer, hipStream_t st);
 size_t moe_tile_table_bytes(int64_t sorted_len, int64_t num_experts);
 size_t moe_tile_partial_bytes(int64_t size_k);
 // gemm_stream.hip: compute units of the current device; the decode kernel in grouped form, for few rows per expert
@@ -578,7 +578,7 @@ int moe_gemm_any(
     const int32_t* num_tokens_past_padded, const float* topk_weights, int64_t moe_block_size,
     int64_t top_k, int mul_topk_weights, int64_t num_experts, int dtype, int64_t b_type_id,
     int64_t size_m, int64_t size_n, int64_t size_k, int64_t num_groups, int is_k_full, void* stream,
-    GatedOutput* gated = nullptr) {
+    const MoeLayerCall& layer = {}) {
   const bool nvfp4 = global_scale != nullptr;
   SONAR_REQUIRE(b_layout == SONAR_LAYOUT_GFX950, "unknown b_layout = %d", b_layout);
   SONAR_REQUIRE(dtype == SONAR_DTYPE_F16 || dtype == SONAR_DTYPE_BF16, "unsupported `a` scalar_type");
@@ -749,7 +749,7 @@ int moe_gemm_any(
                          num_tokens_past_padded, topk_weights, top_k, mul_topk_weights ? 1 : 0, num_experts,
                          static_cast<int32_t*>(scratch), dtype, size_m, size_n, size_k, num_groups, group_size,
                          a_by_slot, fp4, bits8 ? 8 : 4, fp8, static_cast<char*>(scratch) + moe_table_room(sorted_len),
-                         scratch_bytes > moe_table_room(sorted_len) ? scratch_bytes - moe_table_room(sorted_len) : 0, gated, st);
+                         scratch_bytes > moe_table_room(sorted_len) ? scratch_bytes - moe_table_room(sorted_len) : 0, layer, st);
 
   MoeParams p;
   p.a = static_cast<const uint16_t*>(a);
@@ -852,13 +852,22 @@ extern "C" int sonar_moe_wna16_marlin_gemm_gated(
     const int32_t* expert_ids, const int32_t* num_tokens_past_padded, const float* topk_weights, int64_t moe_block_size,
     int64_t top_k, int mul_topk_weights, int64_t num_experts, int dtype, int64_t b_type_id, int64_t size_m,
     int64_t size_n, int64_t size_k, int64_t num_groups, int is_k_full, void* gated, int activation, float limit,
-    float alpha, int* gated_written, void* stream) {
+    float alpha, int* gated_written, sonar_moe_tables* next, const sonar_moe_tables* ready, void* stream) {
   SONAR_REQUIRE(gated_written != nullptr, "gated_written must not be NULL");
   GatedOutput out = {gated, activation, limit, alpha, false};
+  if (next != nullptr) {
+    SONAR_REQUIRE(next != ready && next->table != nullptr && ((uintptr_t)next->table) % 4 == 0 && next->size_n > 0 &&
+                  next->size_n < (1LL << 30) && next->size_k > 0 && next->size_k < (1LL << 30), "next: bad table or sizes");
+    next->built = 0;
+  }
+  MoeLayerCall layer;
+  layer.gated = gated != nullptr ? &out : nullptr;
+  layer.next = next;
+  layer.ready = ready;
   const int rc = moe_gemm_any(a, c, b_q_weight, b_layout, b_bias, b_scales, global_scale, b_zeros, g_idx, perm, scratch,
                               scratch_bytes, sorted_token_ids, sorted_len, expert_ids, num_tokens_past_padded, topk_weights,
                               moe_block_size, top_k, mul_topk_weights, num_experts, dtype, b_type_id, size_m, size_n, size_k,
-                              num_groups, is_k_full, stream, gated != nullptr ? &out : nullptr);
+                              num_groups, is_k_full, stream, layer);
   *gated_written = out.done ? 1 : 0;
   return rc;
 }

@@ -1787,14 +1787,24 @@ __global__ __launch_bounds__(256) void moe_tile_reduce_kernel(const TileParams p
 // ballot inside the wavefront and the other wavefronts' last run starts, a tile's number from counts of
 // the tile heads before it.  Latency bound (one thread scanning the blocks: 16 us at 157 blocks; 4 us so).
 // (1024 threads for up to 256 blocks: 3 us longer, and the code of a kernel that runs once is fetched from memory.)
+// The second workgroup does the same for the layer's other GEMM (a launch of 5 to 9 us less;
+// us a layer: 64 MXFP4 experts 2048 x 768, 4000 tokens, top 8 405 -> 397; 8 experts 2816 x 1280, 1254 tokens 122 -> 118; 8 of
+// 1024 x 2688, AWQ, 6002 tokens 274 -> 269).
+struct TableJob {
+  int32_t *table, *table_small;
+  int tiles_n, k_steps, may_split;
+};
 template <int kTableWaves>
 __global__ __launch_bounds__(64 * kTableWaves) void moe_tile_table_kernel(const int32_t* __restrict__ expert_ids,
                                                                       const int32_t* __restrict__ num_post_pad,
                                                                       int num_blocks_max, int block_size,
-                                                                      int num_experts, int32_t* __restrict__ table,
-                                                                      int32_t* __restrict__ table_small,
-                                                                      int max_tiles, int tiles_n, int k_steps,
-                                                                      int may_split) {
+                                                                      int num_experts, int max_tiles, const TableJob first,
+                                                                      const TableJob second) {
+  int32_t* __restrict__ table = blockIdx.x == 0 ? first.table : second.table;
+  int32_t* __restrict__ table_small = blockIdx.x == 0 ? first.table_small : second.table_small;
+  const int tiles_n = blockIdx.x == 0 ? first.tiles_n : second.tiles_n;
+  const int k_steps = blockIdx.x == 0 ? first.k_steps : second.k_steps;
+  const int may_split = blockIdx.x == 0 ? first.may_split : second.may_split;
   constexpr int kTableThreads = 64 * kTableWaves;
   __shared__ int32_t last_start[kTableWaves], heads[2][kTableWaves];
   __shared__ unsigned long long best;
@@ -2288,7 +2298,7 @@ int moe_tile_gemm(const void* a, void* c, const uint32_t* b, const void* bias, c
                   const int32_t* num_post_pad, const float* topk_weights, int64_t top_k, int mul_topk,
                   int64_t num_experts, int32_t* table, int dtype, int64_t size_m, int64_t size_n, int64_t size_k,
                   int64_t num_groups, int group_size, int a_by_slot, bool fp4, int bits, bool fp8, void* partial,
-                  size_t partial_bytes, GatedOutput* gated, hipStream_t st) {
+                  size_t partial_bytes, const MoeLayerCall& layer, hipStream_t st) {
   const int max_tiles = moe_tile_max(sorted_len, num_experts);
   const int blocks_max = (int)((sorted_len + 63) / 64);
   TileParams p = {};
@@ -2329,7 +2339,10 @@ int moe_tile_gemm(const void* a, void* c, const uint32_t* b, const void* bias, c
   // The wide kernel splits the tiles of a short last round (or all of them when they are few) along
   // K, given room for their partial tiles; moe_tile_reduce_kernel sums them.
   static const bool no_live_split = getenv("SONAR_MARLIN_NO_MOE_K_SPLIT") != nullptr;   // debugging aid
-  const bool wide = fp4 ? wide_applies_fp4(p) : (bits == 8 ? wide_applies8(p, fp8) : wide_applies(p));
+  auto is_wide = [&](const TileParams& q) {
+    return fp4 ? wide_applies_fp4(q) : (bits == 8 ? wide_applies8(q, fp8) : wide_applies(q));
+  };
+  const bool wide = is_wide(p);
   const size_t partial_need = moe_tile_partial_bytes(size_k);
   if (wide && !no_live_split && partial != nullptr && partial_need > 0 && partial_bytes >= partial_need &&
       ((uintptr_t)partial) % 16 == 0)
@@ -2337,17 +2350,21 @@ int moe_tile_gemm(const void* a, void* c, const uint32_t* b, const void* bias, c
   // ... and computes the one or two blocks an expert's rows end in as a 128-row tile, and others where that makes the launch
   // shorter (marlin_tile_wide_pair_kernel; not NVFP4, and not 8-bit codes with groups of 32 rows)
   const bool nvfp4 = fp4 && global_scale != nullptr;
-  const bool two_sizes = wide && !nvfp4 && !(bits == 8 && wide_groups_of_32(p));
+  auto has_two_sizes = [&](const TileParams& q) { return is_wide(q) && !nvfp4 && !(bits == 8 && wide_groups_of_32(q)); };
+  const bool two_sizes = has_two_sizes(p);
   int32_t* table_small = two_sizes ? table + moe_one_table_bytes(sorted_len) / sizeof(int32_t) : nullptr;
+  // tiles are cut along K only while they are few (and the second kernel is launched only where they may be): not when
+  // the rows nearly fill the chip wherever they go, or, with a long K, fill it twice
+  auto few_tiles = [](const TileParams& q) {
+    return (int64_t)(q.rows_total + 255) / 256 * q.tiles_n <= (q.size_k >= 64 * kTileK ? 512 : 192);
+  };
   if (two_sizes) {
-    // tiles are cut along K only while they are few (and the second kernel is launched only where they may be): not when
-    // the rows nearly fill the chip wherever they go, or, with a long K, fill it twice
-    const int64_t least_tiles = (int64_t)(p.rows_total + 255) / 256 * p.tiles_n;
-    if (least_tiles > (size_k >= 64 * kTileK ? 512 : 192)) p.partial = nullptr;
+    if (!few_tiles(p)) p.partial = nullptr;
     if (p.partial != nullptr)
       p.partial_small = reinterpret_cast<float4*>(static_cast<char*>(partial) + moe_partial_bytes_of(kTileM));
   }
   // The activation at the end of the tiles that are not cut along K (those cut are summed by another kernel)
+  GatedOutput* gated = layer.gated;
   if (gated != nullptr && wide && p.partial == nullptr && ((uintptr_t)gated->out) % 16 == 0 &&
       (gated->kind == 0 ? size_n % (2 * 2 * kStripN) == 0 : gated->kind == SONAR_ACT_SWIGLUOAI && gated->limit > 0.f)) {
     p.gated = static_cast<uint16_t*>(gated->out);
@@ -2356,13 +2373,37 @@ int moe_tile_gemm(const void* a, void* c, const uint32_t* b, const void* bias, c
     p.gated_alpha = gated->alpha;
     gated->done = true;
   }
-  auto build_table = [&](auto kernel, int threads) {
-    kernel<<<1, threads, 0, st>>>(expert_ids, num_post_pad, blocks_max, 64, (int)num_experts, table, table_small, max_tiles,
-                                  p.tiles_n, (int)(size_k / kTileK), p.partial != nullptr);
-  };
-  if (blocks_max <= 256) build_table(moe_tile_table_kernel<4>, 256);
-  else build_table(moe_tile_table_kernel<16>, 1024);
-  if (int rc = launch_status("moe_tile_table_kernel")) return rc;
+  TableJob job = {table, table_small, p.tiles_n, (int)(size_k / kTileK), p.partial != nullptr}, next_job = {};
+  const sonar_moe_tables* ready = layer.ready;
+  if (two_sizes && ready != nullptr && ready->built && ready->expert_ids == expert_ids && ready->sorted_len == sorted_len &&
+      ready->tiles_n == job.tiles_n && ready->k_steps == job.k_steps && ready->may_split == job.may_split) {
+    p.tile_table = table = ready->table;
+    table_small = table + moe_one_table_bytes(sorted_len) / sizeof(int32_t);
+  } else {
+    // the layer's next GEMM, if it is one for both tile sizes as well, with the room for partial tiles it would be given
+    sonar_moe_tables* next = layer.next;
+    if (two_sizes && next != nullptr && next->size_k % kTileK == 0 && next->num_groups > 0 &&
+        next->table_bytes >= moe_tile_table_bytes(sorted_len, num_experts)) {
+      TileParams q = p;
+      q.size_n = (int)next->size_n, q.size_k = (int)next->size_k;
+      q.num_groups = (int)next->num_groups, q.group_size = (int)(next->size_k / next->num_groups);
+      q.tiles_n = (int)((next->size_n + kTileN - 1) / kTileN);
+      if (has_two_sizes(q)) {
+        next_job = {next->table, next->table + moe_one_table_bytes(sorted_len) / sizeof(int32_t), q.tiles_n, q.size_k / kTileK,
+                    !no_live_split && moe_tile_partial_bytes(q.size_k) > 0 && few_tiles(q)};
+        next->expert_ids = expert_ids, next->sorted_len = sorted_len;
+        next->tiles_n = next_job.tiles_n, next->k_steps = next_job.k_steps, next->may_split = next_job.may_split;
+        next->built = 1;
+      }
+    }
+    auto build_table = [&](auto kernel, int threads) {
+      kernel<<<next_job.table != nullptr ? 2 : 1, threads, 0, st>>>(expert_ids, num_post_pad, blocks_max, 64, (int)num_experts,
+                                                                    max_tiles, job, next_job);
+    };
+    if (blocks_max <= 256) build_table(moe_tile_table_kernel<4>, 256);
+    else build_table(moe_tile_table_kernel<16>, 1024);
+    if (int rc = launch_status("moe_tile_table_kernel")) return rc;
+  }
   auto reduce = [&](const TileParams& q) -> int {
     if (q.partial == nullptr) return SONAR_OK;
     const int64_t tiles = std::min<int64_t>((int64_t)max_tiles * q.tiles_n, kLiveSplitTilesMax);

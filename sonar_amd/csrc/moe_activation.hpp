@@ -55,4 +55,11 @@ struct GatedOutput {
   bool done;             // set by a call that wrote `out`, which then left c as it was
 };
 
+// What one grouped GEMM of a layer may do for another one of the same routing, or have had done for it.
+struct MoeLayerCall {
+  GatedOutput* gated = nullptr;
+  sonar_moe_tables* next = nullptr;          // build the row tiles of that GEMM in this call's launch
+  const sonar_moe_tables* ready = nullptr;   // this GEMM's, if an earlier call has built them
+};
+
 }  // namespace sonar

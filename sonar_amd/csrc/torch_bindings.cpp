@@ -1014,22 +1014,25 @@ struct Routing {
   const float* topk_weights;
 };
 
-// A gated activation that a grouped GEMM may write to `out` in place of its result (sonar_moe_wna16_marlin_gemm_gated).
-struct Gated {
-  void* out;
-  int activation;
-  float limit, alpha;
-  int written;
+// What sonar_moe_wna16_marlin_gemm_gated takes beyond the GEMM: a gated activation that it may write to `out` in place of its
+// result, and the row tiles of the layer's next GEMM or its own.
+struct InLayer {
+  void* out = nullptr;
+  int activation = 0;
+  float limit = 0, alpha = 0;
+  int written = 0;
+  sonar_moe_tables* next = nullptr;
+  const sonar_moe_tables* ready = nullptr;
 };
 
 // The grouped GEMM on 16-bit activations: checks of a and the expert matrices, and the launch into
-// `c` (size_m * top_k rows of a's type) or `gated`.  The kernels take no workspace.
+// `c` (size_m * top_k rows of a's type) or `layer->out`.  The kernels take no workspace.
 void moe_gemm_16bit(const Tensor& a, void* c, const Tensor& b_q_weight, const OptTensor& b_bias_or_none,
                     const Tensor& b_scales, const OptTensor& a_scales, const OptTensor& global_scale,
                     const OptTensor& b_zeros_or_none, const OptTensor& g_idx_or_none, const OptTensor& perm_or_none,
                     const Routing& route, int64_t moe_block_size, int64_t top_k, bool mul_topk_weights,
                     int64_t b_type_id, int64_t size_m, int64_t size_n, int64_t size_k, bool is_k_full,
-                    bool use_atomic_add, bool use_fp32_reduce, bool is_zp_float, Gated* gated = nullptr) {
+                    bool use_atomic_add, bool use_fp32_reduce, bool is_zp_float, InLayer* layer = nullptr) {
   TORCH_CHECK(a.scalar_type() == at::kHalf || a.scalar_type() == at::kBFloat16, "unsupported `a` scalar_type");
   const int dtype = dtype_code(a);
   check_b_type(b_type_id);
@@ -1125,7 +1128,7 @@ void moe_gemm_16bit(const Tensor& a, void* c, const Tensor& b_q_weight, const Op
   Tensor scratch;
   if (scratch_bytes > 0) scratch = at::empty({(int64_t)scratch_bytes}, a.options().dtype(at::kByte));
 
-  if (gated != nullptr) {
+  if (layer != nullptr) {
     TORCH_CHECK(!nvfp4 || perm == nullptr, "act-order is not supported with float4_e2m1f weights");
     const Tensor scales = nvfp4 ? nvfp4_scales_as_16bit(b_scales, a.scalar_type())
                                 : fp4 || mxfp8 ? mx_scales_as_bf16(b_scales, mxfp8 ? 120 : 0) : b_scales;
@@ -1136,8 +1139,8 @@ void moe_gemm_16bit(const Tensor& a, void* c, const Tensor& b_q_weight, const Op
         has_zp ? static_cast<const uint32_t*>(b_zeros_or_none->const_data_ptr()) : nullptr, g_idx, perm,
         scratch_bytes > 0 ? scratch.mutable_data_ptr() : nullptr, scratch_bytes, route.sorted_ids, route.sorted_len,
         route.expert_ids, route.past_padded, route.topk_weights, moe_block_size, top_k, mul_topk_weights ? 1 : 0, experts,
-        dtype, b_type_id, size_m, size_n, size_k, num_groups, is_k_full ? 1 : 0, gated->out, gated->activation,
-        gated->limit, gated->alpha, &gated->written, current_stream(a)));
+        dtype, b_type_id, size_m, size_n, size_k, num_groups, is_k_full ? 1 : 0, layer->out, layer->activation,
+        layer->limit, layer->alpha, &layer->written, layer->next, layer->ready, current_stream(a)));
     return;
   }
   if (nvfp4) {
@@ -1342,7 +1345,8 @@ void fused_moe(Tensor& output, const Tensor& hidden, const Tensor& w1, const Ten
   if (rows < num_experts) sorted_len = std::min(rows * block_size, sorted_len);
   const int64_t blocks = (sorted_len + block_size - 1) / block_size;
   auto room = [](int64_t ints) { return (ints + 3) / 4 * 4; };
-  Tensor table = at::empty({room(sorted_len) + room(blocks) + 4 + num_experts}, topk_ids.options());
+  const size_t tiles_bytes = sonar_moe_marlin_gemm_scratch_bytes(sorted_len, block_size, k, 64);   // and the down GEMM's row tiles
+  Tensor table = at::empty({room(sorted_len) + room(blocks) + 4 + room(num_experts) + (int64_t)(tiles_bytes / 4)}, topk_ids.options());
   int32_t* sorted_ids = static_cast<int32_t*>(table.mutable_data_ptr());
   int32_t* expert_ids = sorted_ids + room(sorted_len);
   int32_t* past_padded = expert_ids + room(blocks);
@@ -1359,11 +1363,18 @@ void fused_moe(Tensor& output, const Tensor& hidden, const Tensor& w1, const Ten
     return std::make_pair(at, at + (uintptr_t)values * 2);
   };
   const auto in = range(hidden, m * k), mid = range(between, rows * n);
-  Gated gated{between.mutable_data_ptr(), (int)activation, (float)limit, (float)alpha, 0};
+  sonar_moe_tables tables = {};
+  tables.table = past_padded + 4 + room(num_experts);
+  tables.table_bytes = tiles_bytes;
+  tables.size_n = k, tables.size_k = n, tables.num_groups = scale2.dim() == 3 ? scale2.size(1) : 0;
+  InLayer gate_up, down;
+  if (!(in.first < mid.second && mid.first < in.second)) gate_up.out = between.mutable_data_ptr();
+  gate_up.activation = (int)activation, gate_up.limit = (float)limit, gate_up.alpha = (float)alpha;
+  if (tiles_bytes > 0 && k > 0 && n > 0) gate_up.next = &tables, down.ready = &tables;
   moe_gemm_16bit(hidden, wide.mutable_data_ptr(), w1, bias1, scale1, std::nullopt, global_scale1, zeros1, g_idx1, perm1,
                  route, block_size, topk, router_weight_on_input, b_type_id, m, 2 * n, k, is_k_full, false, true,
-                 false, in.first < mid.second && mid.first < in.second ? nullptr : &gated);
-  if (!gated.written)
+                 false, &gate_up);
+  if (!gate_up.written)
     raise_if_failed(activation == 0
                         ? sonar_silu_and_mul(between.mutable_data_ptr(), wide.const_data_ptr(), rows, n, dtype, stream)
                         : sonar_moe_activation(between.mutable_data_ptr(), wide.const_data_ptr(), rows, n,
@@ -1372,7 +1383,7 @@ void fused_moe(Tensor& output, const Tensor& hidden, const Tensor& w1, const Ten
                              ? between
                              : between.view({-1}).narrow(0, 0, rows * n).view({rows, n});
   moe_gemm_16bit(down_in, wide.mutable_data_ptr(), w2, bias2, scale2, std::nullopt, global_scale2, zeros2, g_idx2, perm2,
-                 route, block_size, 1, !router_weight_on_input, b_type_id, rows, k, n, is_k_full, false, true, false);
+                 route, block_size, 1, !router_weight_on_input, b_type_id, rows, k, n, is_k_full, false, true, false, &down);
   raise_if_failed(sonar_moe_sum(output.mutable_data_ptr(), wide.const_data_ptr(), m, topk, k, dtype, stream));
 }
 

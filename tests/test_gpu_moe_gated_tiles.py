@@ -1,7 +1,8 @@
 """The grouped tile kernels form the gated activation of their rows themselves: a layer gives the bits of the GEMM and the
 activation kernel after one another, in every weight format, with both tile sizes, a ragged last tile of columns (alternating gate
 and up only: halves need whole tiles), experts without rows, a bias and the routing weight on the input; the gate and up rows are
-not written then.  Activations and widths that the tiles do not take, and tiles cut along K, go the old way."""
+not written then.  The row tiles of both GEMMs of a layer come from one launch, whichever of them may cut its tiles along K.
+Activations and widths that the tiles do not take, and tiles cut along K, go the old way."""
 from __future__ import annotations
 
 import pytest
@@ -34,7 +35,8 @@ def _experts(gen, kind, e, k, n, dtype):
                                         ("uint8b128", torch.float16)])
 @pytest.mark.parametrize("activation,inter,k,in_tiles", [("silu", 384, 320, True), ("silu", 320, 320, False),
                                                          ("swigluoai", 384, 192, True), ("swigluoai", 352, 320, True),
-                                                         ("gelu", 384, 320, False), ("silu", 384, 1024, False)])
+                                                         ("gelu", 384, 320, False), ("silu", 384, 1024, False),
+                                                         ("silu", 1024, 320, True), ("gelu", 1024, 1024, False)])
 @pytest.mark.parametrize("on_input", [False, True])
 def test_layer(kind, dtype, activation, inter, k, in_tiles, on_input):
     if kind != "mxfp4" and inter % 64:   # the down projection's groups
@@ -74,6 +76,19 @@ def test_layer(kind, dtype, activation, inter, k, in_tiles, on_input):
     assert bool(torch.isfinite(want.float()).all())
     assert torch.equal(cache2.view(rows, inter), between)
     assert torch.equal(got, want)
+
+
+def test_many_blocks():
+    """More blocks of slots than the smaller form of the table kernel has threads."""
+    m, e, top_k, k, inter, dtype = 9001, 5, 2, 320, 1024, torch.bfloat16
+    gen = torch.Generator(device=DEV).manual_seed(2)
+    w1, s1, _ = _experts(gen, "uint4b8", e, k, 2 * inter, dtype)
+    w2, s2, _ = _experts(gen, "uint4b8", e, inter, k, dtype)
+    x = torch.randn((m, k), device=DEV, generator=gen).to(dtype)
+    weights, ids = torch.topk(torch.rand((m, e), device=DEV, generator=gen), top_k, dim=1)
+    args = (x, w1, w2, None, None, s1, s2, weights.contiguous(), ids.to(torch.int32), scalar_types.uint4b8.id)
+    assert torch.equal(fused_moe.fused_marlin_moe(*args),
+                       fused_moe.fused_marlin_moe(*args, activation_func=fused_moe.apply_moe_activation))
 
 
 def test_input_in_the_place_of_the_rows_between():
