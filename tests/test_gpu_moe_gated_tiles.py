@@ -2,7 +2,7 @@
 activation kernel after one another, in every weight format, with both tile sizes, a ragged last tile of columns (alternating gate
 and up only: halves need whole tiles), experts without rows, a bias and the routing weight on the input; the gate and up rows are
 not written then.  The row tiles of both GEMMs of a layer come from one launch, whichever of them may cut its tiles along K.
-Activations and widths that the tiles do not take, and tiles cut along K, go the old way."""
+Activations and widths that the tiles do not take go the old way."""
 from __future__ import annotations
 
 import pytest
@@ -35,7 +35,7 @@ def _experts(gen, kind, e, k, n, dtype):
                                         ("uint8b128", torch.float16)])
 @pytest.mark.parametrize("activation,inter,k,in_tiles", [("silu", 384, 320, True), ("silu", 320, 320, False),
                                                          ("swigluoai", 384, 192, True), ("swigluoai", 352, 320, True),
-                                                         ("gelu", 384, 320, False), ("silu", 384, 1024, False),
+                                                         ("gelu", 384, 320, False), ("silu", 1024, 1024, True), ("swigluoai", 576, 1024, True),
                                                          ("silu", 1024, 320, True), ("gelu", 1024, 1024, False)])
 @pytest.mark.parametrize("on_input", [False, True])
 def test_layer(kind, dtype, activation, inter, k, in_tiles, on_input):
