@@ -99,7 +99,9 @@ struct MidDequant {
 
 template <typename T, int FMT, int GROUPS, int MB, bool DEEP, bool GROUPED = false>
 __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(mid_waves_per_simd(MB, DEEP), mid_waves_per_simd(MB, DEEP)))) void marlin_mid_gemm(
-    const MidParams p) {
+    const typename std::conditional<GROUPED, MidMoeParams, MidParams>::type p) {
+  MidMoe moe = {};
+  if constexpr (GROUPED) moe = p.moe;
   typedef MidDequant<T, FMT> Fmt;
   typedef typename Fmt::D4 D4;
   typedef typename Fmt::D8 D8;
@@ -143,7 +145,7 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
   // of a pair of strips next to each other, so the second to ask for a chunk finds it in that L2.
   // (Grouped: of the blocks that the routing has made, one after the other, so that those of an expert share its chunks.)
   const int strips = p.size_n / kStripN;
-  const int tiles_m = GROUPED ? min(p.tiles_m, p.num_post_pad[0] / p.block_size) : p.tiles_m;
+  const int tiles_m = GROUPED ? min(p.tiles_m, moe.num_post_pad[0] / moe.block_size) : p.tiles_m;
   const int tiles = GROUPED ? tiles_m * ((strips + kMidStrips - 1) / kMidStrips) : p.tiles;
   const int units = tiles * p.splits, per_xcd = (units + 7) / 8;
   const int unit = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
@@ -151,8 +153,8 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
   const int split = unit / tiles, tile = unit - split * tiles;
   const int tile_n = tile / tiles_m, tile_m = tile - tile_n * tiles_m;
   const int m0 = tile_m * 16 * MB;
-  const int expert = GROUPED ? p.expert_ids[tile_m] : 0;
-  if (GROUPED && (unsigned)expert >= (unsigned)p.num_experts) return;
+  const int expert = GROUPED ? moe.expert_ids[tile_m] : 0;
+  if (GROUPED && (unsigned)expert >= (unsigned)moe.num_experts) return;
   // (the second strip of an odd last pair is the first again, and not stored)
   const bool active = tile_n * kMidStrips + strip_of < strips;
   const int strip = __builtin_amdgcn_readfirstlane(active ? tile_n * kMidStrips + strip_of : strips - 1);
@@ -170,16 +172,16 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
   for (int i = 0; i < kCopies; ++i) {
     int row = m0 + 8 * (strip_of * kCopies + i) + (lane >> 3);
     if constexpr (GROUPED) {   // (padding slots read row 0 and are not stored)
-      const int id = row < p.sorted_len ? p.sorted_ids[row] : p.rows_total;
-      row = (unsigned)id < (unsigned)p.rows_total ? (p.a_by_slot ? row : id / p.top_k) : 0;
+      const int id = row < moe.sorted_len ? moe.sorted_ids[row] : moe.rows_total;
+      row = (unsigned)id < (unsigned)moe.rows_total ? (moe.a_by_slot ? row : id / moe.top_k) : 0;
     } else if (row >= p.size_m) {
       row = p.size_m - 1;   // rows past M are computed and never stored
     }
     a_off[i] = (uint32_t)row * (uint32_t)(p.lda * 2) + 16 * ((lane & 7) ^ (lane >> 3));
   }
-  const uint16_t* scales = p.scales + (GROUPED ? expert * p.expert_s_stride : 0) + (size_t)strip * kStripN;
-  const uint32_t* zeros = p.zeros + (GROUPED ? expert * p.expert_z_stride : 0) + (size_t)strip * (kStripN / 8);
-  const char* b_base = reinterpret_cast<const char*>(p.b + (GROUPED ? expert * p.expert_b_stride : 0)) +
+  const uint16_t* scales = p.scales + (GROUPED ? expert * moe.expert_s_stride : 0) + (size_t)strip * kStripN;
+  const uint32_t* zeros = p.zeros + (GROUPED ? expert * moe.expert_z_stride : 0) + (size_t)strip * (kStripN / 8);
+  const char* b_base = reinterpret_cast<const char*>(p.b + (GROUPED ? expert * moe.expert_b_stride : 0)) +
                        (size_t)strip * p.chunks_per_strip * (Fmt::k8 ? 2048 : 1024);
   const uint32_t b_off = 16 * lane;
   const char* s_base = reinterpret_cast<const char*>(scales);
@@ -580,11 +582,11 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
       if (i >= MB || !active) continue;
       float row_w = 1.f;
       if constexpr (GROUPED) {
-        row = row < p.sorted_len ? p.sorted_ids[row] : p.rows_total;
-        if ((unsigned)row >= (unsigned)p.rows_total) row = p.rows_total;   // padding slot
+        row = row < moe.sorted_len ? moe.sorted_ids[row] : moe.rows_total;
+        if ((unsigned)row >= (unsigned)moe.rows_total) row = moe.rows_total;   // padding slot
         // the routing weight is rounded to the activation type and the product is formed and rounded in that type
         // (marlin_template.h(moe):1893-1897)
-        if (p.mul_topk && row < p.rows_total) row_w = Dq<T>::to_float(Dq<T>::from_float(p.topk_weights[row]));
+        if (moe.mul_topk && row < moe.rows_total) row_w = Dq<T>::to_float(Dq<T>::from_float(moe.topk_weights[row]));
       }
       floatx4_t v = floatx4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -592,7 +594,7 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
         const float4 s = sums[(((kMidStrips * g + strip_of) * kSum + (q >> 2)) * 4 + j) * 64 + lane];
         v += floatx4_t{s.x, s.y, s.z, s.w};
       }
-      if (row >= (GROUPED ? p.rows_total : p.size_m)) continue;
+      if (row >= (GROUPED ? moe.rows_total : p.size_m)) continue;
       const int nl = 16 * j + tile_col;
       if constexpr (kRaw && !kFold) {
 #pragma unroll
@@ -606,7 +608,7 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
       if (FMT == kMidNvFp4) v = v * gs;
       float bias[4] = {0.f, 0.f, 0.f, 0.f};
       if (p.bias) {
-        const uint16_t* bias_row = p.bias + (GROUPED ? expert * p.expert_bias_stride : 0) + strip * kStripN;
+        const uint16_t* bias_row = p.bias + (GROUPED ? expert * moe.expert_bias_stride : 0) + strip * kStripN;
 #pragma unroll
         for (int r = 0; r < 4; ++r) bias[r] = Dq<T>::to_float(bias_row[scale_slot(nl + r, false)]);
       }
@@ -614,7 +616,7 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         n[r] = Dq<T>::from_float(v[r] + bias[r]);
-        if (GROUPED && p.mul_topk) n[r] = Dq<T>::from_float(Dq<T>::to_float(n[r]) * row_w);
+        if (GROUPED && moe.mul_topk) n[r] = Dq<T>::from_float(Dq<T>::to_float(n[r]) * row_w);
       }
       const uint2 o = make_uint2((uint32_t)n[0] | ((uint32_t)n[1] << 16), (uint32_t)n[2] | ((uint32_t)n[3] << 16));
       *reinterpret_cast<uint2*>(p.c + (size_t)row * p.size_n + strip * kStripN + nl) = o;
@@ -650,7 +652,7 @@ __global__ __launch_bounds__(256) void marlin_mid_sum(const MidParams p) {
 }
 
 template <typename T, int FMT, int GROUPS, int MB, bool DEEP = false, bool GROUPED = false>
-int launch_mid_rows(const MidParams& p, hipStream_t st) {
+int launch_mid_rows(const typename std::conditional<GROUPED, MidMoeParams, MidParams>::type& p, hipStream_t st) {
   static bool attr_set = false;   // raising the dynamic LDS limit is needed once per form
   if (!attr_set) {
     SONAR_HIP(hipFuncSetAttribute((const void*)marlin_mid_gemm<T, FMT, GROUPS, MB, DEEP, GROUPED>,
@@ -717,17 +719,17 @@ int launch_mid_format(const MidParams& p, int format, int row_blocks, hipStream_
 }
 
 template <typename T, int FMT, int GROUPS>
-int launch_mid_moe(const MidParams& p, hipStream_t st) {
-  switch (p.block_size) {
+int launch_mid_moe(const MidMoeParams& p, hipStream_t st) {
+  switch (p.moe.block_size) {
     case 32: return launch_mid_rows<T, FMT, GROUPS, 2, false, true>(p, st);
     case 48: return launch_mid_rows<T, FMT, GROUPS, 3, false, true>(p, st);
     case 64: return launch_mid_rows<T, FMT, GROUPS, 4, false, true>(p, st);
-    default: return fail(SONAR_E_INVALID, "internal: blocks of %d slots", p.block_size);
+    default: return fail(SONAR_E_INVALID, "internal: blocks of %d slots", p.moe.block_size);
   }
 }
 
 template <typename T>
-int launch_mid_moe_format(const MidParams& p, int format, hipStream_t st) {
+int launch_mid_moe_format(const MidMoeParams& p, int format, hipStream_t st) {
   if (format == kMidInt4)
     return p.num_groups == 1 ? launch_mid_moe<T, kMidInt4, kOneGroupRaw>(p, st) : launch_mid_moe<T, kMidInt4, kUnitGroupsRaw>(p, st);
   if (format == kMidInt4Zp)
@@ -739,7 +741,7 @@ int launch_mid_moe_format(const MidParams& p, int format, hipStream_t st) {
 
 }  // namespace
 
-int mid_moe_gemm(MidParams p, int dtype, int format, int blocks, hipStream_t st) {
+int mid_moe_gemm(MidMoeParams p, int dtype, int format, int blocks, hipStream_t st) {
   p.splits = 1;
   p.tiles_m = blocks;
   p.tiles = blocks * ((p.size_n / kStripN + mid_strips(2) - 1) / mid_strips(2));

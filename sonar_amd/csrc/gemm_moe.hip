@@ -701,7 +701,7 @@ int moe_gemm_any(
                 "(the column-permuted copy of A per slot)");
   if (!bits8 && !row_groups && !nvfp4 && !has_perm &&
       moe_mid_applies(moe_block_size, size_m * top_k, num_experts, a_rows, size_n, size_k, num_groups, group_size, fp4)) {
-    MidParams m = {};
+    MidMoeParams m = {};
     m.a = static_cast<const uint16_t*>(a);
     m.lda = size_k;
     m.c = static_cast<uint16_t*>(c);
@@ -715,21 +715,21 @@ int moe_gemm_any(
       for (int per = group_size / 64; per > 0; per >>= 1) ++m.group_shift;   // (moe_mid_applies: 64 * 2^i rows)
     m.chunks_per_strip = (int)(size_k / kChunkK);
     m.raw_codes = !fp4;
-    m.sorted_ids = sorted_token_ids;
-    m.expert_ids = expert_ids;
-    m.num_post_pad = num_tokens_past_padded;
-    m.topk_weights = topk_weights;
-    m.block_size = (int)moe_block_size;
-    m.top_k = (int)top_k;
-    m.mul_topk = mul_topk_weights ? 1 : 0;
-    m.num_experts = (int)num_experts;
-    m.rows_total = (int)(size_m * top_k);
-    m.sorted_len = (int)sorted_len;
-    m.a_by_slot = a_by_slot;
-    m.expert_b_stride = (long)(size_n / kStripN) * m.chunks_per_strip * 64;
-    m.expert_s_stride = (long)num_groups * size_n;
-    m.expert_z_stride = (long)num_groups * (size_n / 8);
-    m.expert_bias_stride = size_n;
+    m.moe.sorted_ids = sorted_token_ids;
+    m.moe.expert_ids = expert_ids;
+    m.moe.num_post_pad = num_tokens_past_padded;
+    m.moe.topk_weights = topk_weights;
+    m.moe.block_size = (int)moe_block_size;
+    m.moe.top_k = (int)top_k;
+    m.moe.mul_topk = mul_topk_weights ? 1 : 0;
+    m.moe.num_experts = (int)num_experts;
+    m.moe.rows_total = (int)(size_m * top_k);
+    m.moe.sorted_len = (int)sorted_len;
+    m.moe.a_by_slot = a_by_slot;
+    m.moe.expert_b_stride = (long)(size_n / kStripN) * m.chunks_per_strip * 64;
+    m.moe.expert_s_stride = (long)num_groups * size_n;
+    m.moe.expert_z_stride = (long)num_groups * (size_n / 8);
+    m.moe.expert_bias_stride = size_n;
     return mid_moe_gemm(m, dtype, fp4 ? kMidMxFp4 : has_zp ? kMidInt4Zp : kMidInt4,
                         (int)((sorted_len + moe_block_size - 1) / moe_block_size), st);
   }
