@@ -43,8 +43,10 @@ __device__ __forceinline__ uint16_t swiglu_oai(uint16_t gate_bits, uint16_t up_b
   const float u = fmaxf(fminf(to_f32<T>(up_bits), limit), -limit);
   const float t = g * hi;
   const float rest = __builtin_fmaf(g, lo, __builtin_fmaf(g, hi, -t));
-  // (beyond 1e7 `rest` is no small number any more and the power of two 0 or infinite: only its sign could go wrong)
-  return from_f32<T>(over_one_plus((u + 1.0f) * g, fabsf(__builtin_amdgcn_exp2f(t) * __builtin_fmaf(rest, kLn2, 1.0f))));
+  // (Where the power of two is 0 or infinite it is the exponential; `rest` is no small number there, but large, infinite or NaN:
+  // the minimum and the absolute value keep the product 0 or infinite.)
+  const float correction = fminf(__builtin_fmaf(rest, kLn2, 1.0f), 2.0f);
+  return from_f32<T>(over_one_plus((u + 1.0f) * g, fabsf(__builtin_amdgcn_exp2f(t) * correction)));
 }
 
 // Where a grouped GEMM may leave its activation instead of its result.

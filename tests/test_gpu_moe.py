@@ -542,6 +542,38 @@ def test_gated_activation_kernels(name, kind, limit, alpha, beta, kw, dtype):
     assert np.all(np.abs(cpu.float().numpy() - want) <= tol)
 
 
+# a limit within the range of the gates, one beyond which the exponent overflows (bf16), and none
+@pytest.mark.parametrize("limit", [7.0, 2e38, float("inf")])
+@pytest.mark.parametrize("alpha", [1.702, 1.0, 0.25])
+@pytest.mark.parametrize("dtype", ["fp16", "bf16"])
+def test_swigluoai_of_extreme_gates(dtype, alpha, limit):
+    """Gates whose exponential is 0 or infinite, infinities and NaN: what the clamp and a division of floats give."""
+    lib = _lib.load()
+    tops = [6e4] if dtype == "fp16" else [6e4, 1e8, 2.5e12, 1e30, 1.3e38, 1.5e38, 3e38]
+    gates = [s * v for v in [0.0, 1e-5, 5.0, 40.0, 88.0, 104.0, 400.0, float("inf"), *tops] for s in (1.0, -1.0)] + [float("nan")]
+    ups = [0.5, -3.0, 0.0, -1.0, 6e4, float("inf"), float("-inf"), float("nan")]
+    pairs = np.array([(g, u) for g in gates for u in ups], dtype=np.float32)
+    x32 = mo.round_to_dtype(pairs, dtype)
+    x = gu.dev_bits16(x32.reshape(1, -1), dtype)
+    out = torch.empty((1, len(pairs)), dtype=x.dtype, device=gu.DEV)
+    _lib.check(lib.sonar_moe_activation(gu.ptr(out), gu.ptr(x), 1, len(pairs), 4, limit, alpha, 0.0,
+                                        gu.dtype_code(dtype), gu.stream()))
+    with np.errstate(all="ignore"):
+        g = np.fmin(x32[:, 0], np.float32(limit))       # (a NaN goes, as with fminf)
+        u = np.fmax(np.fmin(x32[:, 1], np.float32(limit)), np.float32(-limit))
+        e = np.exp((g * np.float32(-alpha)).astype(np.float64)).astype(np.float32)
+        n = (u + np.float32(1.0)) * g
+        want = mo.round_to_dtype(n / (np.float32(1.0) + e), dtype)
+    got = gu.host_f32(out)[0]
+    same = (got == want) | (np.isnan(got) & np.isnan(want))
+    ulp = 2.0 ** (-10 if dtype == "fp16" else -7)
+    least = 2.0 ** -24 if dtype == "fp16" else 2.0 ** -125   # of a result; below it the last places of `e` are lost
+    with np.errstate(all="ignore"):
+        near = np.isfinite(got) & np.isfinite(want) & (np.abs(got - want) <= ulp * np.abs(want) + least)
+    bad = ~(same | near)
+    assert not bad.any(), list(zip(x32[bad].tolist(), got[bad].tolist(), want[bad].tolist()))[:8]
+
+
 def test_gated_activation_rejections():
     lib = _lib.load()
     x = torch.zeros((4, 32), dtype=torch.float16, device=gu.DEV)
