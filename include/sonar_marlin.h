@@ -97,6 +97,15 @@ const char* sonar_marlin_version(void);
  * and returns the number of entries written (at most n). */
 int sonar_marlin_last_decode_launch(int32_t* out, int n);
 
+/* The kernel that the calling thread's last grouped GEMM on 16-bit activations ran in (no counterpart in the reference; for
+ * tests that are about one of them). */
+#define SONAR_GROUPED_NONE 0      /* nothing to do, or refused */
+#define SONAR_GROUPED_GENERAL 1   /* marlin_moe_kernel, marlin_moe8_kernel */
+#define SONAR_GROUPED_DECODE 2    /* marlin_stream_fast_kernel */
+#define SONAR_GROUPED_MID 3       /* marlin_mid_gemm */
+#define SONAR_GROUPED_TILE 4      /* the tile kernels */
+int sonar_marlin_last_grouped_kernel(void);
+
 /* GPTQ (K/8, N) int32, nibble k%8 of word [k/8][n] = code of W[k][n]
  * -> Marlin (K/16, 2N) int32; with num_bits == 8: (K/4, N) int32, byte k%4
  * -> Marlin (K/16, 4N) int32.  perm (int32[K], may be NULL) selects source

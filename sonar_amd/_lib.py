@@ -27,11 +27,14 @@ E_INVALID = -1
 E_UNSUPPORTED = -2
 E_RUNTIME = -3
 
+GROUPED_GENERAL, GROUPED_DECODE, GROUPED_MID, GROUPED_TILE = 1, 2, 3, 4   # what sonar_marlin_last_grouped_kernel answers
+
 # name -> (restype, argtypes); must list every symbol include/sonar_marlin.h declares
 PROTOTYPES = {
     "sonar_marlin_last_error": (c_char_p, []),
     "sonar_marlin_version": (c_char_p, []),
     "sonar_marlin_last_decode_launch": (c_int, [c_void_p, c_int]),
+    "sonar_marlin_last_grouped_kernel": (c_int, []),
     "sonar_debug_tile_schedule": (c_int64, [c_int64, c_int64, c_int64, c_int64, c_void_p, c_int64]),
     "sonar_debug_moe_tile_schedule": (c_int64, [c_int64, c_int64, c_int64, c_int64, c_int, c_void_p, c_int64]),
     "sonar_debug_moe_pair_schedule": (c_int64, [c_int64, c_int64, c_int64, c_int64, c_int64, c_int, c_void_p, c_void_p, c_int64]),

@@ -569,6 +569,8 @@ extern "C" size_t sonar_moe_marlin_gemm_scratch_bytes(int64_t sorted_len, int64_
 }
 
 namespace {
+thread_local int g_last_grouped_kernel = SONAR_GROUPED_NONE;
+
 // The grouped GEMM behind sonar_moe_wna16_marlin_gemm (global_scale == nullptr) and its NVFP4 form.
 int moe_gemm_any(
     const void* a, void* c, const uint32_t* b_q_weight, int b_layout, const void* b_bias,
@@ -579,6 +581,7 @@ int moe_gemm_any(
     int64_t top_k, int mul_topk_weights, int64_t num_experts, int dtype, int64_t b_type_id,
     int64_t size_m, int64_t size_n, int64_t size_k, int64_t num_groups, int is_k_full, void* stream,
     const MoeLayerCall& layer = {}) {
+  g_last_grouped_kernel = SONAR_GROUPED_NONE;
   const bool nvfp4 = global_scale != nullptr;
   SONAR_REQUIRE(b_layout == SONAR_LAYOUT_GFX950, "unknown b_layout = %d", b_layout);
   SONAR_REQUIRE(dtype == SONAR_DTYPE_F16 || dtype == SONAR_DTYPE_BF16, "unsupported `a` scalar_type");
@@ -730,27 +733,33 @@ int moe_gemm_any(
     m.moe.expert_s_stride = (long)num_groups * size_n;
     m.moe.expert_z_stride = (long)num_groups * (size_n / 8);
     m.moe.expert_bias_stride = size_n;
+    g_last_grouped_kernel = SONAR_GROUPED_MID;
     return mid_moe_gemm(m, dtype, fp4 ? kMidMxFp4 : has_zp ? kMidInt4Zp : kMidInt4,
                         (int)((sorted_len + moe_block_size - 1) / moe_block_size), st);
   }
   // Few rows per expert: the decode kernel, one workgroup per strip and 32 slots of a block
   if (!bits8 && !row_groups && !nvfp4 &&
       moe_fast_applies(has_perm, moe_block_size, sorted_len, num_experts, a_rows, size_n, size_k, num_groups,
-                       group_size))
+                       group_size)) {
+    g_last_grouped_kernel = SONAR_GROUPED_DECODE;
     return moe_fast_gemm(a, c, b_q_weight, b_bias, b_scales, b_zeros, sorted_token_ids, sorted_len, expert_ids,
                          num_tokens_past_padded, topk_weights, moe_block_size, top_k, mul_topk_weights ? 1 : 0,
                          num_experts, dtype, size_m, size_n, size_k, num_groups, group_size, a_by_slot, fp4, st);
+  }
   static const bool no_tile = getenv("SONAR_MARLIN_NO_MOE_TILE") != nullptr;  // debugging aid
   // Full blocks of 64 slots mean many rows per expert: the MFMA-tiled kernel
   if (moe_block_size == 64 && !has_perm && !row_groups && !no_tile && size_k % 64 == 0 &&
       (num_groups == 1 || group_size % 64 == 0 || group_size == 32 || nvfp4) && scratch != nullptr &&
-      scratch_bytes >= moe_tile_table_bytes(sorted_len, num_experts) && ((uintptr_t)scratch) % 4 == 0)
+      scratch_bytes >= moe_tile_table_bytes(sorted_len, num_experts) && ((uintptr_t)scratch) % 4 == 0) {
+    g_last_grouped_kernel = SONAR_GROUPED_TILE;
     return moe_tile_gemm(a, c, b_q_weight, b_bias, b_scales, global_scale, b_zeros, sorted_token_ids, sorted_len, expert_ids,
                          num_tokens_past_padded, topk_weights, top_k, mul_topk_weights ? 1 : 0, num_experts,
                          static_cast<int32_t*>(scratch), dtype, size_m, size_n, size_k, num_groups, group_size,
                          a_by_slot, fp4, bits8 ? 8 : 4, fp8, static_cast<char*>(scratch) + moe_table_room(sorted_len),
                          scratch_bytes > moe_table_room(sorted_len) ? scratch_bytes - moe_table_room(sorted_len) : 0, layer, st);
+  }
 
+  g_last_grouped_kernel = SONAR_GROUPED_GENERAL;
   MoeParams p;
   p.a = static_cast<const uint16_t*>(a);
   p.c = static_cast<uint16_t*>(c);
@@ -811,6 +820,8 @@ int moe_gemm_any(
   return launch_status("marlin_moe_kernel");
 }
 }  // namespace
+
+extern "C" int sonar_marlin_last_grouped_kernel() { return g_last_grouped_kernel; }
 
 extern "C" int sonar_moe_wna16_marlin_gemm(
     const void* a, void* c, const uint32_t* b_q_weight, int b_layout, const void* b_bias,

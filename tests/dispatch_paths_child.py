@@ -90,7 +90,11 @@ def dense_8bit() -> None:
 
 
 def grouped() -> None:
+    from sonar_amd import _lib
     from tests import test_gpu_moe as tm
+    lib = _lib.load()
+    switched_off = {kernel for switch, kernel in (("MID", _lib.GROUPED_MID), ("TILE", _lib.GROUPED_TILE),
+                                                  ("FAST", _lib.GROUPED_DECODE)) if "SONAR_MARLIN_NO_MOE_" + switch in os.environ}
     for case in [(300, 4, 2, 256, 256, 128, "fp16", False, False, False, 64, True),
                  (700, 8, 2, 512, 128, 64, "bf16", True, False, True, 64, False),
                  (900, 3, 2, 2048, 256, 128, "bf16", True, False, True, 64, False),   # K split on the device
@@ -100,6 +104,11 @@ def grouped() -> None:
                  (50, 4, 2, 512, 128, 128, "bf16", False, True, False, 16, True)]:     # act-order
         print("grouped", case, flush=True)
         tm.test_moe_gemm_within_tolerance(case)   # raises on a mismatch
+        ran = lib.sonar_marlin_last_grouped_kernel()
+        assert ran not in switched_off, (case, ran)
+        if switched_off and case[10] == 64 and case[0] > 300:
+            want = _lib.GROUPED_GENERAL if _lib.GROUPED_TILE in switched_off else _lib.GROUPED_TILE
+            assert ran == want, (case, ran)
     # NVFP4 experts on 64-slot blocks: the tile kernels, or the general grouped kernel when they are switched off
     from tests import test_gpu_ops as to
     to.test_prepare_nvfp4_moe_layer_and_fused_marlin_moe((1500, 4, 2, 256, 128), "fp16")

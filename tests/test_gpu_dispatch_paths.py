@@ -29,6 +29,7 @@ SWITCHES = [
     "SONAR_MARLIN_NO_ASYNC_TILE",    # the register-staged tile kernel
     "SONAR_MARLIN_MAX_K_SPLITS=1",   # no split K in the tile kernel
     "SONAR_MARLIN_NO_TWO_TILE_SIZES",  # a short last round of tiles cut along K instead of halved into 128-row tiles
+    "SONAR_MARLIN_NO_MOE_MID",       # blocks of 32 slots and more in the decode and tile kernels, as with the switches below
     "SONAR_MARLIN_NO_MOE_TILE",      # the grouped streaming kernel for 64-slot blocks
     "SONAR_MARLIN_NO_MOE_FAST",      # ... and for blocks of up to 32 slots
     "SONAR_MARLIN_NO_MOE_K_SPLIT",   # the grouped wide tile kernel never cuts its tiles along K
@@ -42,6 +43,8 @@ def test_every_dispatch_path_meets_the_oracle(switch):
     if switch:
         name, _, value = switch.partition("=")
         env[name] = value or "1"
+        if name.startswith("SONAR_MARLIN_NO_MOE_"):   # the kernel in front of those that the others are about
+            env["SONAR_MARLIN_NO_MOE_MID"] = "1"
     out = subprocess.run([sys.executable, "-u", "-m", "tests.dispatch_paths_child"], cwd=ROOT, env=env,
                          capture_output=True, text=True, timeout=110)
     assert out.returncode == 0 and "all paths ok" in out.stdout, out.stdout[-1500:] + out.stderr[-1500:]

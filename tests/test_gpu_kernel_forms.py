@@ -18,7 +18,7 @@ from tests import test_gpu_parity as tp
 pytestmark = pytest.mark.gpu
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-SWITCHES = ("SONAR_MARLIN_NO_MID=1", "SONAR_MARLIN_A8_SHAPE=0", "SONAR_MARLIN_NO_MOE_TILE=1")
+SWITCHES = ("SONAR_MARLIN_NO_MID=1", "SONAR_MARLIN_A8_SHAPE=0", "SONAR_MARLIN_NO_MOE_TILE=1", "SONAR_MARLIN_NO_MOE_MID=1")
 
 
 @pytest.mark.parametrize("switch", SWITCHES)
@@ -121,7 +121,43 @@ def _without_the_grouped_tile_kernel() -> None:
     to.test_prepare_nvfp4_moe_layer_and_fused_marlin_moe((110, 4, 2, 256, 128), "bf16")
 
 
+def _without_the_grouped_mid_kernel() -> None:
+    """Blocks of 32 slots and more of 4-bit codes that marlin_mid_gemm takes: in the kernels that the cases are named after."""
+    from sonar_amd import _lib
+    from tests import test_gpu_moe_small_groups as ts
+    last = _lib.load().sonar_marlin_last_grouped_kernel
+
+    def ran(kernel, call, *args):
+        call(*args)
+        assert last() == kernel, (call.__name__, args, last())
+        print(call.__name__, args, "ok", flush=True)
+
+    for case in [(700, 4, 2, 1024, 320, 128, "fp16", False, False, False, 64, True),      # K split in both tile sizes
+                 (900, 3, 2, 2048, 256, 128, "bf16", True, False, True, 64, False),
+                 (650, 2, 2, 1024, 256, 128, "fp16", False, True, False, 64, True),       # act-order: rows of A by slot
+                 (1100, 2, 1, 128, 512, 128, "bf16", False, False, True, 64, False),
+                 (600, 4, 2, 512, 256, 128, "fp16", True, False, True, 64, True),
+                 (700, 4, 2, 512, 256, -1, "bf16", False, False, False, 64, True),
+                 (700, 2, 2, 640, 256, 128, "fp16", False, False, True, 64, True)]:
+        ran(_lib.GROUPED_TILE, tm.test_moe_gemm_within_tolerance, case)
+    ran(_lib.GROUPED_TILE, tm.test_full_size_grouped_gemm_agrees_with_dense_rows, 700, 2048, 1024, "uint4b8/fp16")
+    ran(_lib.GROUPED_TILE, tm.test_full_size_grouped_gemm_agrees_with_dense_rows, 700, 4096, 2048, "mxfp4")
+    ran(_lib.GROUPED_TILE, tm.test_tile_kernel_with_expert_ids_that_are_not_grouped_by_expert, 128)
+    ran(_lib.GROUPED_GENERAL, tm.test_full_size_grouped_gemm_agrees_with_dense_rows, 300, 512, 256, "mxfp4!")
+    for dtype, zp in (("bf16", False), ("fp16", False), ("fp16", True), ("bf16", True)):
+        ran(_lib.GROUPED_GENERAL, tm.test_moe_tiled_and_streaming_kernels_agree, dtype, zp, 128)
+    for tokens in (100, 150, 190):
+        ran(_lib.GROUPED_DECODE, ts.test_mxfp4, tokens, 1152, 4096)
+    ran(_lib.GROUPED_DECODE, ts.test_sixteen_experts, 450, "fp16", True, 128)
+    ran(_lib.GROUPED_TILE, ts.test_sixteen_experts, 520, "fp16", True, 128)
+    for case in [(200, 4, 2, 256, 1024, 128, "bf16", True, False, False, 32, True),
+                 (150, 4, 2, 256, 256, 128, "fp16", False, False, False, 48, True),
+                 (120, 4, 2, 512, 1024, 128, "fp16", True, False, True, 64, True)]:
+        ran(_lib.GROUPED_DECODE, tm.test_moe_gemm_within_tolerance, case)
+
+
 if __name__ == "__main__":
     {"SONAR_MARLIN_NO_MID": _without_the_mid_kernel, "SONAR_MARLIN_A8_SHAPE": _without_the_w4a8_block_kernel,
-     "SONAR_MARLIN_NO_MOE_TILE": _without_the_grouped_tile_kernel}[sys.argv[1]]()
+     "SONAR_MARLIN_NO_MOE_TILE": _without_the_grouped_tile_kernel,
+     "SONAR_MARLIN_NO_MOE_MID": _without_the_grouped_mid_kernel}[sys.argv[1]]()
     print("all forms ok", flush=True)

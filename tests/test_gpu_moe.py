@@ -97,14 +97,18 @@ MOE_CASES = [
     (150, 4, 2, 256, 256, 128, "fp16", False, False, False, 48, True),
     (222, 3, 2, 288, 128, 32, "bf16", False, False, False, 64, True),
     (5, 64, 6, 256, 128, 128, "fp16", False, False, False, 16, True),
-    # 64-slot blocks with groups of at least 64 rows: the MFMA-tiled grouped kernel
+    # 64-slot blocks: the decode, mid-size or tile kernel by format and size (each by name: test_gpu_kernel_forms)
     (300, 4, 2, 512, 256, 128, "fp16", False, False, False, 64, True),
     (513, 3, 2, 256, 320, 64, "bf16", True, False, True, 64, True),
     (90, 8, 2, 384, 128, -1, "fp16", False, False, False, 64, False),
     (1100, 2, 1, 128, 512, 128, "bf16", False, False, True, 64, False),
     (900, 2, 2, 256, 512, 32, "fp16", True, False, True, 64, True),      # groups of 32 rows in the tile kernel
     # K of 16 steps or more in whole passes of four: the wide kernel cuts its few tiles along K on the device
-    # (fp32 partial tiles through scratch, moe_tile_reduce_kernel); act-order through the permuted copy
+    # (fp32 partial tiles through scratch, moe_tile_reduce_kernel); act-order through the permuted copy.  Groups of 128 rows
+    # go to marlin_mid_gemm, of 64 to the tile kernel
+    (700, 4, 2, 1024, 320, 64, "fp16", False, False, False, 64, True),
+    (900, 3, 2, 2048, 256, 64, "bf16", True, False, True, 64, False),
+    (650, 2, 2, 1024, 256, 64, "fp16", False, True, False, 64, True),
     (700, 4, 2, 1024, 320, 128, "fp16", False, False, False, 64, True),
     (900, 3, 2, 2048, 256, 128, "bf16", True, False, True, 64, False),
     (640, 5, 2, 1280, 192, 64, "bf16", False, False, True, 64, True),
@@ -585,19 +589,21 @@ def test_gated_activation_rejections():
 
 
 @pytest.mark.parametrize("dtype,zp", [("bf16", False), ("fp16", False), ("fp16", True), ("bf16", True)])
-def test_moe_tiled_and_streaming_kernels_agree(dtype, zp):
-    """The same 64-slot-block call (more slots than the decode kernel takes) with
-    and without the scratch the tiled kernel needs for its table takes two
-    different kernels; both meet the tolerance against the reference and each
-    other."""
+def test_moe_tiled_and_streaming_kernels_agree(dtype, zp, group=64):
+    """The same 64-slot-block call (more slots than the decode kernel takes, groups
+    that marlin_mid_gemm does not) with and without the scratch the tiled kernel
+    needs for its table takes two different kernels; both meet the tolerance against
+    the reference and each other."""
     m, e, top_k, k, n, bs = 700, 4, 2, 512, 256, 64
-    ex = Experts(91, e, k, n, 128, dtype, zero_points=zp)
+    ex = Experts(91, e, k, n, group, dtype, zero_points=zp)
     topk_ids, topk_w = route(7, m, e, top_k)
     sorted_ids, expert_ids, past = mo.moe_align_block_size(topk_ids, bs, e)
     a32 = mo.make_activations(4, m, k, dtype)
     a = gu.dev_bits16(a32, dtype)
     tiled = gu.host_f32(ex.gemm(a, sorted_ids, expert_ids, int(past[0]), topk_w, bs, top_k, m, True, scratch=True))
+    assert _lib.load().sonar_marlin_last_grouped_kernel() == _lib.GROUPED_TILE
     streamed = gu.host_f32(ex.gemm(a, sorted_ids, expert_ids, int(past[0]), topk_w, bs, top_k, m, True, scratch=False))
+    assert _lib.load().sonar_marlin_last_grouped_kernel() == _lib.GROUPED_GENERAL
     want = ex.reference(a32, sorted_ids, expert_ids, int(past[0]), bs, top_k, m, topk_w)
     for got in (tiled, streamed):
         ok, *worst = mo.gemm_tolerance_ok(got, want)
@@ -633,14 +639,14 @@ def test_full_size_grouped_tile_gemm_agrees_with_dense_rows():
             assert err <= 1e-2 * scale, (t, j, err, scale)
 
 
-def test_tile_kernel_with_expert_ids_that_are_not_grouped_by_expert():
+def test_tile_kernel_with_expert_ids_that_are_not_grouped_by_expert(group=64):
     """64-slot blocks whose experts alternate, with blocks of absent experts (-1) in
     between: every block is a run of its own, more runs than experts.  The table of
     row tiles has an entry per block, so no block may be dropped."""
-    m, e, top_k, k, n, bs = 64 * 14, 3, 1, 256, 256, 64
-    ex = Experts(301, e, k, n, 128, "bf16")
+    m, e, top_k, k, n, bs = 64 * 20, 3, 1, 256, 256, 64   # (1100 slots and fewer: the decode kernel)
+    ex = Experts(301, e, k, n, group, "bf16")
     blocks = m // bs
-    pattern = [0, 1, -1, 2, 0, -1, 1, 2, 0, 1, 2, -1, 0, 2]
+    pattern = [0, 1, -1, 2, 0, -1, 1, 2, 0, 1, 2, -1, 0, 2, 2, -1, 2, 1, 1, 0]
     assert len(pattern) == blocks
     expert_ids = np.array(pattern, dtype=np.int32)
     rng = np.random.default_rng(5)
@@ -649,6 +655,7 @@ def test_tile_kernel_with_expert_ids_that_are_not_grouped_by_expert():
     a32 = mo.make_activations(9, m, k, "bf16")
     a = gu.dev_bits16(a32, "bf16")
     got = gu.host_f32(ex.gemm(a, sorted_ids, expert_ids, m, weights, bs, top_k, m, True))
+    assert _lib.load().sonar_marlin_last_grouped_kernel() == _lib.GROUPED_TILE
     want = ex.reference(a32, sorted_ids, expert_ids, m, bs, top_k, m, weights)
     written = np.concatenate([sorted_ids[b * bs:(b + 1) * bs] for b in range(blocks) if pattern[b] >= 0])
     ok, *worst = mo.gemm_tolerance_ok(got[written], want[written])
