@@ -702,7 +702,8 @@ int moe_gemm_any(
     return fail(SONAR_E_INVALID,
                 "act-order with 8-bit expert weights needs sorted_len * size_k * 2 more scratch bytes "
                 "(the column-permuted copy of A per slot)");
-  if (!bits8 && !row_groups && !nvfp4 && !has_perm &&
+  // (Its scales are 16-byte loads, as in the dense call; the other kernels copy them in pieces of 4.)
+  if (!bits8 && !row_groups && !nvfp4 && !has_perm && ((uintptr_t)b_scales) % 16 == 0 &&
       moe_mid_applies(moe_block_size, size_m * top_k, num_experts, a_rows, size_n, size_k, num_groups, group_size, fp4)) {
     MidMoeParams m = {};
     m.a = static_cast<const uint16_t*>(a);

@@ -5,7 +5,11 @@ against the dense call."""
 from __future__ import annotations
 
 import pytest
+import torch
 
+from oracle import marlin_oracle as mo
+from sonar_amd import _lib
+from tests import gpu_util as gu
 from tests import test_gpu_moe as tm
 
 pytestmark = pytest.mark.gpu
@@ -39,3 +43,22 @@ def test_uneven_routing(slots):
 @pytest.mark.parametrize("k,n", [(192, 4160), (1152, 2112)])
 def test_mxfp4(tokens, k, n):
     tm.test_full_size_grouped_gemm_agrees_with_dense_rows(tokens, k, n, "mxfp4")
+
+
+# the kernel reads scales 16 bytes a lane; the others take them at any 4
+@pytest.mark.parametrize("offset", [2, 4, 8])   # elements of two bytes
+@pytest.mark.parametrize("zp", [False, True])
+def test_scales_at_fewer_than_16_bytes(offset, zp):
+    m, e, top_k, k, n, slots = 200, 8, 2, 256, 2112, 64
+    ex = tm.Experts(9, e, k, n, 128, "fp16", zp)
+    sorted_ids, expert_ids, past = mo.moe_align_block_size(tm.route(3, m, e, top_k)[0], slots, e)
+    a32 = mo.make_activations(4, m, k, "fp16")
+    want = ex.reference(a32, sorted_ids, expert_ids, int(past[0]), slots, top_k, m, None)
+    room = torch.empty(ex.scales.numel() + offset, dtype=ex.scales.dtype, device=gu.DEV)
+    moved = room[offset:].view(ex.scales.shape).copy_(ex.scales)
+    for scales, kernel in ((ex.scales, _lib.GROUPED_MID), (moved, _lib.GROUPED_MID if offset == 8 else _lib.GROUPED_DECODE)):
+        ex.scales = scales
+        got = gu.host_f32(ex.gemm(gu.dev_bits16(a32, "fp16"), sorted_ids, expert_ids, int(past[0]), None, slots, top_k, m, False))
+        assert _lib.load().sonar_marlin_last_grouped_kernel() == kernel
+        ok, *worst = mo.gemm_tolerance_ok(got, want)
+        assert ok, worst
