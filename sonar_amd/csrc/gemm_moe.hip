@@ -12,6 +12,7 @@
 // depend on the launch: scratch and workspace are not used.
 // Calls with few rows per expert and K % 128 == 0 on 4-bit codes go to the decode kernel in grouped form instead
 // (gemm_stream.hip), 64-slot blocks of many rows to the tile kernels (gemm_tile.hip).
+#include <cmath>
 #include <cstdlib>
 
 #include "common.hpp"
@@ -530,27 +531,50 @@ void launch_moe_mb(const MoeParams& p, bool has_perm, int grid, hipStream_t st) 
 using namespace sonar;
 
 // Whether a grouped call runs in marlin_mid_gemm, which dequantises a chunk once for all slots of a block and two strips:
-// 4-bit integers with one group or groups of 128 * 2^i rows, MXFP4.  Otherwise the decode kernel (32 slots at a time) or the tile
-// kernels (128 and 256 rows) run.  120 random GEMMs of 8 to 64 experts, us there / here:
-//   blocks of 48 slots: 1.2 times as fast (geometric mean; lowest 0.94, with a quarter of a round of workgroups or less):
-//     8 experts, 30 slots each, K = 7552, N = 3200, MXFP4 53 / 29; 32 of 39, 2560 x 5760, AWQ 117 / 90; 64 of 42, 768 x 4864 123 / 98
-//   blocks of 64, up to 56 slots an expert, so that most experts are one block: 1.2 times (lowest 0.90): 16 of 48, 4352 x 9344,
-//     AWQ 189 / 134; 32 of 48, 1024 x 896 25 / 12; with more slots, while it is one round of workgroups: 8 of 78, 640 x 1920
-//     19 / 11; 8 of 110, 7040 x 2816 94 / 70; but in 3.5 rounds 16 of 107, 1152 x 3584 26 / 44
-//   blocks of 32: as fast as the decode kernel, whose copies ask for more bytes at a time, but for half a round to a round of
-//     workgroups: 16 of 24, 3456 x 1792, AWQ 20.4 / 16.7; 16 of 17, 4608 x 1152, MXFP4 24.7 / 18.6; 64 of 20, 1408 x 2048 39 / 41
+// 4-bit integers with one group or groups of 128 * 2^i rows, MXFP4.  Otherwise it runs in the decode kernel (`decode`: 32 slots at a
+// time), in the tile kernels (`tiles`: 128 and 256 rows, the activation at their end) or in the general kernel.  Timed on 359 random
+// layers of 8 to 64 experts, 13 to 135 slots each, either GEMM forced both ways (graph replays; quoted: the layer's us there / here).
+// Against the decode kernel:
+//   fewer than half a round of workgroups of integer codes, or a quarter of MXFP4, are too few wavefronts here: 8 experts of
+//     51 slots, down 8448 x 1024 92 / 108; of 40, gate and up 1280 x 1024 30.1 / 32.6
+//   blocks of 32: as fast, but for half a round to a round: 16 of 22, down 5632 x 1152 91 / 83; with just half a round only from
+//     21 slots on (8 of 18, gate and up 3584 x 2048 36 / 40), and a full round has a second as soon as an expert has a second
+//     block: 32 of 25, down 8064 x 1024 192 / 200
+//   blocks of 48: 1.16 times as fast; 64 of 41, 1024 x 3584 312 / 245; 32 of 41, MXFP4, 1280 x 768 73 / 55
+//   blocks of 64, up to 56 slots an expert: 8 of 53, MXFP4, 4096 x 10752 281 / 217; integer codes are level or behind from one round
+//     to one and a quarter: 16 of 44, AWQ, gate and up 4096 x 2560 84 / 88
+// Against the tile kernels, up to 56 slots: always for one round (32 of 50, AWQ, down 2048 x 384 70 / 61), else as the rounds
+//   of both say, the second blocks of uneven routing counted.  A fit of 131 GEMMs: it loses 0.3 % of a layer on average against
+//   the better of the two; always here 2.6 %, never 5.9 %.  32 of 51, 2560 x 1280 147 / 110; but 64 of 56, AWQ, 3840 x 512
+//   143 / 174, and 32 of 56, down 1152 x 2048 93 / 102 (256 tiles, one round of them).
+// More slots: while it is one round of workgroups (8 of 79, 1536 x 640 62 / 41; 8 of 111, MXFP4, down 4864 x 1536 103 / 96).
+// The general kernel (MXFP4 with K of no whole units) is never ahead: 16 of 35, 1472 x 704 54 / 37.
+// Blocks of 32 and 48 slots that are nearly full on average were not timed (the rule for block sizes makes none).
 static bool moe_mid_applies(int64_t moe_block_size, int64_t rows_total, int64_t num_experts, int64_t a_rows, int64_t size_n,
-                            int64_t size_k, int64_t num_groups, int group_size, bool fp4) {
+                            int64_t size_k, int64_t num_groups, int group_size, bool fp4, bool decode, bool tiles) {
   static const bool no_mid = getenv("SONAR_MARLIN_NO_MOE_MID") != nullptr;  // debugging aid
   if (no_mid || moe_block_size < 32 || !mid_applies(a_rows, size_k, size_k, num_groups, group_size)) return false;
   if (!fp4 && (size_k % 128 != 0 || (num_groups > 1 && group_size % 128 != 0))) return false;
-  // blocks there will be where the routing is even, and rounds of workgroups (a pair of strips each)
-  const int64_t slots = rows_total / num_experts, blocks = num_experts * (slots <= moe_block_size - 8 ? 1 : slots / 56 + 1);
-  const double rounds = (double)(blocks * ((size_n + 127) / 128)) / cu_count();
+  const int64_t slots = rows_total / num_experts, cus = cu_count();
   if (slots < moe_block_size * 3 / 8) return false;   // mostly padding: the decode kernel leaves 32 slots of it out
+  if (moe_block_size < 64 && 10 * slots >= 9 * moe_block_size) return false;
+  // rounds of workgroups (a pair of strips each) with the blocks there are where the routing is even
+  const int64_t pairs = (size_n + 127) / 128;
+  const double rounds = (double)(num_experts * (slots <= 56 ? 1 : slots / 56 + 1) * pairs) / cus;
+  if (slots > 56) return rounds <= 1.0;
+  if (decode) {
+    if (moe_block_size == 32) return rounds >= 0.5 && (rounds > 0.5 || slots > 20) && rounds < 1.0;
+    if (fp4) return rounds > 0.25;
+    return rounds >= 0.5 && (moe_block_size == 48 || rounds <= 1.0 || rounds > 1.25);
+  }
   if (moe_block_size == 32) return rounds >= 0.5 && rounds <= 1.0;
   if (moe_block_size == 48) return rounds >= 0.25;
-  return slots <= 56 || rounds <= 1.0;
+  if (!tiles || rounds <= 1.0) return true;
+  const double more = slots > 44 ? 0.0009 * (slots - 44) * (slots - 44) : 0.0;   // second blocks, for each first one
+  const double mid_rounds = std::ceil(rounds * (1.0 + more) - 0.06);
+  const double tile_rounds = (double)((num_experts * ((size_n + 255) / 256) + cus - 1) / cus);
+  const double k = size_k * 1e-3;
+  return mid_rounds * (2.3 + 5.4 * k) < tile_rounds * (14.8 * k - 2.4) + 4.5;
 }
 
 // the table of row tiles, rounded up so that what follows it is aligned
@@ -702,9 +726,17 @@ int moe_gemm_any(
     return fail(SONAR_E_INVALID,
                 "act-order with 8-bit expert weights needs sorted_len * size_k * 2 more scratch bytes "
                 "(the column-permuted copy of A per slot)");
+  const bool decode = !bits8 && !row_groups && !nvfp4 &&
+                      moe_fast_applies(has_perm, moe_block_size, sorted_len, num_experts, a_rows, size_n, size_k, num_groups,
+                                       group_size);
+  static const bool no_tile = getenv("SONAR_MARLIN_NO_MOE_TILE") != nullptr;  // debugging aid
+  const bool tiles = moe_block_size == 64 && !has_perm && !row_groups && !no_tile && size_k % 64 == 0 &&
+                     (num_groups == 1 || group_size % 64 == 0 || group_size == 32 || nvfp4) && scratch != nullptr &&
+                     scratch_bytes >= moe_tile_table_bytes(sorted_len, num_experts) && ((uintptr_t)scratch) % 4 == 0;
   // (Its scales are 16-byte loads, as in the dense call; the other kernels copy them in pieces of 4.)
   if (!bits8 && !row_groups && !nvfp4 && !has_perm && ((uintptr_t)b_scales) % 16 == 0 &&
-      moe_mid_applies(moe_block_size, size_m * top_k, num_experts, a_rows, size_n, size_k, num_groups, group_size, fp4)) {
+      moe_mid_applies(moe_block_size, size_m * top_k, num_experts, a_rows, size_n, size_k, num_groups, group_size, fp4,
+                      decode, tiles)) {
     MidMoeParams m = {};
     m.a = static_cast<const uint16_t*>(a);
     m.lda = size_k;
@@ -739,19 +771,14 @@ int moe_gemm_any(
                         (int)((sorted_len + moe_block_size - 1) / moe_block_size), st);
   }
   // Few rows per expert: the decode kernel, one workgroup per strip and 32 slots of a block
-  if (!bits8 && !row_groups && !nvfp4 &&
-      moe_fast_applies(has_perm, moe_block_size, sorted_len, num_experts, a_rows, size_n, size_k, num_groups,
-                       group_size)) {
+  if (decode) {
     g_last_grouped_kernel = SONAR_GROUPED_DECODE;
     return moe_fast_gemm(a, c, b_q_weight, b_bias, b_scales, b_zeros, sorted_token_ids, sorted_len, expert_ids,
                          num_tokens_past_padded, topk_weights, moe_block_size, top_k, mul_topk_weights ? 1 : 0,
                          num_experts, dtype, size_m, size_n, size_k, num_groups, group_size, a_by_slot, fp4, st);
   }
-  static const bool no_tile = getenv("SONAR_MARLIN_NO_MOE_TILE") != nullptr;  // debugging aid
   // Full blocks of 64 slots mean many rows per expert: the MFMA-tiled kernel
-  if (moe_block_size == 64 && !has_perm && !row_groups && !no_tile && size_k % 64 == 0 &&
-      (num_groups == 1 || group_size % 64 == 0 || group_size == 32 || nvfp4) && scratch != nullptr &&
-      scratch_bytes >= moe_tile_table_bytes(sorted_len, num_experts) && ((uintptr_t)scratch) % 4 == 0) {
+  if (tiles) {
     g_last_grouped_kernel = SONAR_GROUPED_TILE;
     return moe_tile_gemm(a, c, b_q_weight, b_bias, b_scales, global_scale, b_zeros, sorted_token_ids, sorted_len, expert_ids,
                          num_tokens_past_padded, topk_weights, top_k, mul_topk_weights ? 1 : 0, num_experts,

@@ -14,35 +14,58 @@ from tests import test_gpu_moe as tm
 
 pytestmark = pytest.mark.gpu
 
-# tokens, experts, K, N and slots of a block (top 2): half a round to a round of workgroups with blocks of 32, a quarter and more
-# with 48; 64 rows and less an expert, and 100 (two blocks)
-SHAPES = [(42, 4, 384, 4160, 32), (80, 4, 256, 2112, 48), (70, 3, 128, 2880, 48), (100, 4, 640, 320, 64), (200, 4, 128, 192, 64)]
+# tokens, experts, K, N and slots of a block (top 2): half a round to a round of workgroups on 256 compute units; most experts are
+# one block, and in the last shape two
+SHAPES = [(42, 4, 384, 4160, 32), (160, 8, 256, 2112, 48), (120, 6, 128, 2880, 48), (200, 8, 640, 2112, 64), (200, 4, 128, 192, 64)]
+
+
+def _ran(call, *args):
+    call(*args)
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert _lib.load().sonar_marlin_last_grouped_kernel() == _lib.GROUPED_MID
 
 
 @pytest.mark.parametrize("m,e,k,n,slots", SHAPES)
 @pytest.mark.parametrize("group", [-1, 128])
 @pytest.mark.parametrize("dtype,zp", [("fp16", False), ("fp16", True), ("bf16", False), ("bf16", True)])
 def test_integer_codes(m, e, k, n, slots, group, dtype, zp):
-    tm.test_moe_gemm_within_tolerance((m, e, 2, k, n, group, dtype, zp, False, zp, slots, not zp))
+    _ran(tm.test_moe_gemm_within_tolerance, (m, e, 2, k, n, group, dtype, zp, False, zp, slots, not zp))
 
 
 @pytest.mark.parametrize("m,e,k,n,slots", SHAPES)
 def test_act_order(m, e, k, n, slots):
     if k > 128:
-        tm.test_moe_gemm_within_tolerance((m, e, 2, k, n, 128, "bf16", False, True, True, slots, True))
+        _ran(tm.test_moe_gemm_within_tolerance, (m, e, 2, k, n, 128, "bf16", False, True, True, slots, True))
 
 
 # an expert with no rows, one with a single block, one with many: the routing of `route` over more experts than tokens reach
 @pytest.mark.parametrize("slots", [48, 64])
 def test_uneven_routing(slots):
-    tm.test_moe_gemm_within_tolerance((230, 8, 1, 256, 1088, 128, "bf16", True, False, False, slots, True))
+    _ran(tm.test_moe_gemm_within_tolerance, (230, 8, 1, 256, 2112, 128, "bf16", True, False, False, slots, True))
 
 
-# 25, 37 and 47 rows an expert are blocks of 32, 48 and 64 slots
+# 25, 37 and 47 rows an expert are blocks of 32, 48 and 64 slots; K of an odd number of steps, and of whole units
 @pytest.mark.parametrize("tokens", [100, 150, 190])
-@pytest.mark.parametrize("k,n", [(192, 4160), (1152, 2112)])
+@pytest.mark.parametrize("k,n", [(192, 2112), (1152, 2112)])
 def test_mxfp4(tokens, k, n):
-    tm.test_full_size_grouped_gemm_agrees_with_dense_rows(tokens, k, n, "mxfp4")
+    _ran(tm.test_full_size_grouped_gemm_agrees_with_dense_rows, tokens, k, n, "mxfp4")
+
+
+# the edges of the rule: experts, tokens (top 2), K, N, slots of a block, zero points, and the kernel
+RULE = [(8, 72, 128, 2048, 32, False, "DECODE"), (8, 100, 128, 2048, 32, False, "MID"), (8, 100, 128, 2112, 32, False, "MID"), (8, 100, 128, 4096, 32, True, "DECODE"),
+        (8, 120, 128, 1920, 48, True, "DECODE"), (8, 120, 128, 1984, 48, False, "MID"), (8, 120, 128, 8320, 48, False, "MID"),
+        (8, 180, 128, 2048, 48, False, "DECODE"),    # 45 slots an expert: nearly full blocks
+        (8, 200, 128, 4096, 64, True, "MID"), (8, 200, 128, 4224, 64, True, "DECODE"), (8, 200, 128, 5248, 64, True, "MID"),
+        (32, 800, 128, 1024, 64, False, "MID"), (32, 800, 128, 2048, 64, False, "TILE"),   # one round, and a short K in two
+        (32, 830, 1152, 1216, 64, False, "MID"), (32, 896, 1152, 2048, 64, False, "TILE")]  # 1.25 rounds; 2 of more blocks than experts
+
+
+@pytest.mark.parametrize("e,m,k,n,slots,zp,kernel", RULE)
+def test_rule(e, m, k, n, slots, zp, kernel):
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("rounds of workgroups on 256 compute units")
+    tm.test_moe_gemm_within_tolerance((m, e, 2, k, n, 128, "bf16", zp, False, False, slots, False))
+    assert _lib.load().sonar_marlin_last_grouped_kernel() == getattr(_lib, "GROUPED_" + kernel)
 
 
 # the kernel reads scales 16 bytes a lane; the others take them at any 4
