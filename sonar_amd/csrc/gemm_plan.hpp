@@ -95,8 +95,9 @@ inline bool plan_prefers_128_rows(int64_t size_m, int64_t size_n, int64_t size_k
   return tiles256 <= (size_k <= 8192 ? 128 : 32);
 }
 
-// Whether the rows of a tile are within the 32-bit offsets that the wide tile kernel copies a dense call's A with.
-inline bool tile_rows_within_32_bits(int64_t a_row_stride) { return a_row_stride < (int64_t)1 << 23; }
+// Whether the 64 rows of a dense call's A that a wavefront of the wide tile kernel copies are within 32-bit offsets of the first.
+// (The other tile kernels have 64-bit addresses.)
+inline bool wide_rows_within_32_bits(int64_t a_row_stride) { return a_row_stride < (int64_t)1 << 25; }
 
 // What the tile kernels are launched with, given room for the partial tiles.  `rows128`: the call's format has 128-row tiles.
 inline GemmPlan tile_plan(int64_t size_m, int64_t size_n, int64_t size_k, bool rows128, bool rows_97_128) {

@@ -1872,8 +1872,11 @@ int marlin_gemm_any(const void* a, int64_t a_row_stride, void* c, const uint32_t
   const size_t tile_room = base_scratch > stream_scratch_bytes() ? base_scratch - stream_scratch_bytes() : 0;
   const bool tile_starved = make_do && size_m <= 128 && plan.k_splits > 1 &&
                             tile_room < plan_partial_bytes_any(size_m, size_n, size_k);
+  // (rows of A too far apart for the wide tile kernel: the other tile kernels where they have the format, else the streaming ones)
+  const bool only_wide = chk.fp8 || chk.nvfp4 || (!chk.fp4 && !chk.has_perm && num_groups > 1 && chk.group_size == 32);
   const bool use_tile = plan.tile && !no_tile && !chk.row_groups && ((chk.bits == 4 && !chk.fp4) || async_tile) &&
-                        !(slab_fast && p.unit_chunks == 4) && !tile_starved && tile_rows_within_32_bits(a_row_stride);
+                        !(slab_fast && p.unit_chunks == 4) && !tile_starved &&
+                        (!only_wide || wide_rows_within_32_bits(a_row_stride));
   // More than 64 rows in the general kernels (8-bit codes, is_k_full = false,
   // the tile path switched off) on a matrix of short strips: one workgroup per
   // strip as well, so that every 64-row slab can run in the same launch and the

@@ -1121,8 +1121,10 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
   // ---- sources (regions of A as in marlin_tile_async_kernel; wavefront w fills RB / 2 regions)
   // Memory operations take a scalar base and a 32-bit offset a lane where they can: with a 64-bit address a lane each holds up the
   // wavefront's other instructions 20 cycles longer.  (M = 8192, K = 4096, N = 28672, fp16 1357 -> 1343 us; one tile alone 74.2 -> 73.4.)
-  // Dense calls: 256 rows of A are within 32 bits (tile_rows_within_32_bits); the rows of a grouped tile may be anywhere.
-  const char* a_rows = reinterpret_cast<const char*>(p.a + (GROUPED ? 0 : (long)m0 * p.lda));
+  // Dense calls: a wavefront's rows of A are within 32 bits of its first (wide_rows_within_32_bits); the rows of a grouped tile
+  // may be anywhere.
+  const int a_first = GROUPED ? 0 : min(m0 + 4 * RB * wave, p.size_m - 1);
+  const char* a_rows = reinterpret_cast<const char*>(p.a + (long)a_first * p.lda);
   typename std::conditional<GROUPED, const char*, uint32_t>::type a_src[RB / 2];
 #pragma unroll
   for (int i = 0; i < RB / 2; ++i) {
@@ -1139,7 +1141,7 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
       if (row >= p.size_m) row = p.size_m - 1;   // rows past M are computed and never stored
     }
     if constexpr (GROUPED) a_src[i] = a_rows + ((long)row * p.lda + 8 * ((lane & 7) ^ r8)) * 2;
-    else a_src[i] = (uint32_t)(row - m0) * (uint32_t)(p.lda * 2) + 16 * ((lane & 7) ^ r8);
+    else a_src[i] = (uint32_t)(row - a_first) * (uint32_t)(p.lda * 2) + 16 * ((lane & 7) ^ r8);
   }
   const char* b_base = reinterpret_cast<const char*>(p.b + expert * p.expert_b_stride) +
                        (size_t)(unsigned)(strip * p.chunks_per_strip) * (1024 * kChunkLoads);
@@ -2091,8 +2093,10 @@ namespace {
 // now: int4 with groups of 32, M = 4096, K = 2880, N = 5760 204 -> 142; AWQ, M = 4000, K = 1152, N = 6144 117 -> 71; NVFP4
 // bf16, M = 2048, K = 4480, N = 8192 148 -> 118; MXFP8, M = 3000, K = 2944, N = 6144 188 -> 168; int4, M = 2000, K = 2944,
 // N = 7808, once padded, 81.5 -> 78.3; 2000 tokens on 32 MXFP4 experts of 2880 x 2880, the whole layer 626 -> 543.)
+bool wide_takes_rows(const TileParams& p) { return p.tile_table != nullptr || wide_rows_within_32_bits(p.lda); }
 bool wide_applies(const TileParams& p) {
   static const bool no_wide = getenv("SONAR_MARLIN_NO_WIDE_TILE") != nullptr;   // debugging aid
+  if (!wide_takes_rows(p)) return false;
   if (wide_groups_of_32(p)) return true;
   if (no_wide) return false;
   if (p.num_groups == 1) return true;
@@ -2108,7 +2112,7 @@ bool wide_applies_fp4(const TileParams& p) {
   static const bool no_wide = getenv("SONAR_MARLIN_NO_WIDE_TILE") != nullptr;
   if (p.tile_table != nullptr || p.global_scale != nullptr) return true;
   const bool few = p.tile_rows == kTileM && p.k_splits == 1 && p.tiles_m * p.tiles_n <= 192;
-  return !no_wide && !few;
+  return !no_wide && !few && wide_takes_rows(p);
 }
 // ... and for 8-bit codes (the same rule; floating-point ones come in groups of 32 or 128 rows or one).
 bool wide_applies8(const TileParams& p, bool fp8) { return fp8 || wide_applies(p); }

@@ -70,14 +70,43 @@ def test_grouped(mul_topk):
 
 
 def test_rows_of_a_too_far_apart_for_32_bit_offsets():
-    """Rows 16 MiB apart: the kernels that take such calls, against the same rows side by side (two roundings to fp16 differ)."""
+    """Rows 64 MiB apart: the kernels that take such calls, against the same rows side by side (two roundings to fp16 differ)."""
     m, k, n, dtype = 150, 8192, 1088, torch.float16
     gen = torch.Generator(device=DEV).manual_seed(1)
     q, s = _weights(gen, 1, k, n, dtype)
-    far = torch.empty_strided((m, k), (1 << 23, 1), dtype=dtype, device=DEV)
+    far = torch.empty_strided((m, k), (1 << 25, 1), dtype=dtype, device=DEV)
     far.copy_(torch.randn((m, k), device=DEV, generator=gen))
     empty = torch.empty(0, dtype=torch.int32, device=DEV)
     ws = mu.marlin_make_workspace_new(torch.device(DEV))
     got, want = (ops.marlin_gemm(a, None, q[0], None, s[0], None, None, empty, empty, empty, ws, scalar_types.uint4b8, m, n, k,
                                  True, False, True, False).double() for a in (far, far.contiguous()))
     assert float((got - want).norm() / want.norm()) < 2e-3
+
+
+# the row strides up to which the wide tile kernel's 32-bit offsets reach, and the first beyond: both tile sizes, ragged rows
+@pytest.mark.parametrize("wtype", ["uint4b8", "uint8b128", "float8_e4m3fn"])
+@pytest.mark.parametrize("m,k,n", [(200, 512, 32832), (400, 256, 8256)])
+def test_strides_of_rows_of_a(wtype, m, k, n):
+    dtype = torch.float16
+    gen = torch.Generator(device=DEV).manual_seed(m)
+    words = 2 if wtype == "uint4b8" else 4
+    q = torch.randint(-2 ** 31, 2 ** 31 - 1, (k // 16, words * n), dtype=torch.int32, device=DEV, generator=gen) & 0x77777777
+    s = (torch.rand((k // 128, n), device=DEV, generator=gen) * (1e-3 if words == 4 else 9e-3) + 1e-4).to(dtype)
+    near = torch.randn((m, k), device=DEV, generator=gen).to(dtype)
+    empty = torch.empty(0, dtype=torch.int32, device=DEV)
+    ws = mu.marlin_make_workspace_new(torch.device(DEV))
+
+    def call(a):
+        return ops.marlin_gemm(a, None, q, None, s, None, None, empty, empty, empty, ws, getattr(scalar_types, wtype), m, n, k,
+                               True, False, True, False)
+
+    want = call(near)
+    assert bool(torch.isfinite(want).all())
+    for stride in (1 << 23, (1 << 25) - 8, 1 << 25):
+        far = torch.empty_strided((m, k), (stride, 1), dtype=dtype, device=DEV)
+        got = call(far.copy_(near))
+        del far
+        if stride < 1 << 25:
+            assert torch.equal(got, want), stride
+        else:   # another kernel: two roundings to fp16 differ
+            assert float((got.double() - want.double()).norm() / want.double().norm()) < 2e-3
