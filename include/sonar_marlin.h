@@ -433,7 +433,8 @@ int sonar_moe_wna16_marlin_gemm_nvfp4(
  * global_scale != NULL: NVFP4.  The other arguments as for sonar_moe_wna16_marlin_gemm.
  * next (may be NULL): sizes of the layer's next GEMM over the same routing, experts of the same type, and `table` of table_bytes
  * (sonar_moe_marlin_gemm_scratch_bytes(sorted_len, moe_block_size, size_n, 64)) of device memory, where this call may lay down what
- * that GEMM otherwise begins with; that call, on the same stream and with the routing unchanged, gets the struct as `ready`. */
+ * that GEMM otherwise begins with; that call, on the same stream and with the routing unchanged, gets the struct as `ready`, which is
+ * then spent: another call with it builds its own. */
 typedef struct {
   int32_t* table;
   size_t table_bytes;
@@ -454,7 +455,7 @@ int sonar_moe_wna16_marlin_gemm_gated(
     int64_t num_experts, int dtype, int64_t b_type_id, int64_t size_m,
     int64_t size_n, int64_t size_k, int64_t num_groups, int is_k_full,
     void* gated, int activation, float limit, float alpha, int* gated_written,
-    sonar_moe_tables* next, const sonar_moe_tables* ready, void* stream);
+    sonar_moe_tables* next, sonar_moe_tables* ready, void* stream);
 
 /* The small kernels around the two grouped GEMMs of a mixture-of-experts layer.
  * They have counterparts in every build of the reference (also on ROCm):

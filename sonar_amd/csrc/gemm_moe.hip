@@ -891,7 +891,7 @@ extern "C" int sonar_moe_wna16_marlin_gemm_gated(
     const int32_t* expert_ids, const int32_t* num_tokens_past_padded, const float* topk_weights, int64_t moe_block_size,
     int64_t top_k, int mul_topk_weights, int64_t num_experts, int dtype, int64_t b_type_id, int64_t size_m,
     int64_t size_n, int64_t size_k, int64_t num_groups, int is_k_full, void* gated, int activation, float limit,
-    float alpha, int* gated_written, sonar_moe_tables* next, const sonar_moe_tables* ready, void* stream) {
+    float alpha, int* gated_written, sonar_moe_tables* next, sonar_moe_tables* ready, void* stream) {
   SONAR_REQUIRE(gated_written != nullptr, "gated_written must not be NULL");
   GatedOutput out = {gated, activation, limit, alpha, false};
   if (next != nullptr) {

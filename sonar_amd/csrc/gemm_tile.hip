@@ -2402,10 +2402,11 @@ int moe_tile_gemm(const void* a, void* c, const uint32_t* b, const void* bias, c
     gated->done = true;
   }
   TableJob job = {table, table_small, p.tiles_n, (int)(size_k / kTileK), p.partial != nullptr}, next_job = {};
-  const sonar_moe_tables* ready = layer.ready;
+  sonar_moe_tables* ready = layer.ready;
   if (two_sizes && ready != nullptr && ready->built && ready->expert_ids == expert_ids && ready->sorted_len == sorted_len &&
       ready->tiles_n == job.tiles_n && ready->k_steps == job.k_steps && ready->may_split == job.may_split) {
     p.tile_table = table = ready->table;
+    ready->built = 0;   // (the routing may change in place before another call)
     table_small = table + moe_one_table_bytes(sorted_len) / sizeof(int32_t);
   } else {
     // the layer's next GEMM, if it is one for both tile sizes as well, with the room for partial tiles it would be given

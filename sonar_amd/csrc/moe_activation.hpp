@@ -61,7 +61,7 @@ struct GatedOutput {
 struct MoeLayerCall {
   GatedOutput* gated = nullptr;
   sonar_moe_tables* next = nullptr;          // build the row tiles of that GEMM in this call's launch
-  const sonar_moe_tables* ready = nullptr;   // this GEMM's, if an earlier call has built them
+  sonar_moe_tables* ready = nullptr;         // this GEMM's, if an earlier call has built them
 };
 
 }  // namespace sonar

@@ -1022,7 +1022,7 @@ struct InLayer {
   float limit = 0, alpha = 0;
   int written = 0;
   sonar_moe_tables* next = nullptr;
-  const sonar_moe_tables* ready = nullptr;
+  sonar_moe_tables* ready = nullptr;
 };
 
 // The grouped GEMM on 16-bit activations: checks of a and the expert matrices, and the launch into

@@ -5,11 +5,17 @@ not written then.  The row tiles of both GEMMs of a layer come from one launch, 
 Activations and widths that the tiles do not take go the old way."""
 from __future__ import annotations
 
+import ctypes
+
+import numpy as np
 import pytest
 import torch
 
-from sonar_amd import fused_moe
+from oracle import marlin_oracle as mo
+from sonar_amd import _lib, fused_moe
 from sonar_amd.scalar_type import scalar_types
+from tests import gpu_util as gu
+from tests import test_gpu_moe as tm
 
 pytestmark = pytest.mark.gpu
 
@@ -107,3 +113,46 @@ def test_input_in_the_place_of_the_rows_between():
     got = fused_moe.fused_marlin_moe(inside, w1, w2, None, None, s1, s2, weights, ids, scalar_types.uint4b8.id,
                                      intermediate_cache2=cache2)
     assert torch.equal(got, want)
+
+
+class _Tables(ctypes.Structure):
+    _fields_ = [("table", ctypes.c_void_p), ("table_bytes", ctypes.c_size_t), ("size_n", ctypes.c_int64), ("size_k", ctypes.c_int64),
+                ("num_groups", ctypes.c_int64), ("built", ctypes.c_int), ("tiles_n", ctypes.c_int), ("k_steps", ctypes.c_int),
+                ("may_split", ctypes.c_int), ("expert_ids", ctypes.c_void_p), ("sorted_len", ctypes.c_int64)]
+
+
+def test_row_tiles_laid_down_by_another_call_are_used_once():
+    """A second call with the same struct, the routing changed in place meanwhile, has to build its own."""
+    lib = _lib.load()
+    m, e, top_k, k, n, bs = 1400, 4, 1, 256, 320, 64
+    ex = tm.Experts(7, e, k, n, 64, "bf16")
+    a = torch.randn((m, k), device=DEV, generator=torch.Generator(device=DEV).manual_seed(4)).to(torch.bfloat16)
+    routes = []
+    for seed in (1, 2):   # the second: most slots of the last expert
+        ids = tm.route(seed, m, e, top_k)[0]
+        if seed == 2:
+            ids[:1000] = e - 1
+        routes.append(mo.moe_align_block_size(ids, bs, e))
+    sid, eid, npp = (gu.dev_i32(np.asarray(x).reshape(-1)) for x in routes[0])
+    tables = _Tables(size_n=n, size_k=k, num_groups=ex.groups)
+    room = torch.empty(lib.sonar_moe_marlin_gemm_scratch_bytes(sid.numel(), bs, n, 64), dtype=torch.uint8, device=DEV)
+    tables.table, tables.table_bytes = room.data_ptr(), room.numel()
+
+    def call(next_call=None, ready=None):
+        c = torch.zeros((m, n), dtype=torch.bfloat16, device=DEV)
+        scratch = torch.empty(lib.sonar_moe_marlin_gemm_scratch_bytes(sid.numel(), bs, n, k), dtype=torch.uint8, device=DEV)
+        written = ctypes.c_int(-1)
+        _lib.check(lib.sonar_moe_wna16_marlin_gemm_gated(
+            gu.ptr(a), gu.ptr(c), gu.ptr(ex.native), _lib.LAYOUT_GFX950, None, gu.ptr(ex.scales), None, None, None, None, gu.ptr(scratch),
+            scratch.numel(), gu.ptr(sid), sid.numel(), gu.ptr(eid), gu.ptr(npp), None, bs, top_k, 0, e, _lib.DTYPE_BF16, ex.b_type, m,
+            n, k, ex.groups, 1, None, 0, 0.0, 0.0, ctypes.byref(written), next_call, ready, gu.stream()))
+        torch.cuda.synchronize()
+        assert written.value == 0 and lib.sonar_marlin_last_grouped_kernel() == _lib.GROUPED_TILE
+        return c
+
+    want = call()
+    assert torch.equal(call(next_call=ctypes.byref(tables)), want) and tables.built == 1
+    assert torch.equal(call(ready=ctypes.byref(tables)), want) and tables.built == 0
+    for t, x in zip((sid, eid, npp), routes[1]):
+        t.copy_(gu.dev_i32(np.asarray(x).reshape(-1)))
+    assert torch.equal(call(ready=ctypes.byref(tables)), call())
