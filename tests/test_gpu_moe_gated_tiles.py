@@ -1,5 +1,6 @@
 """The grouped tile kernels form the gated activation of their rows themselves: a layer gives the bits of the GEMM and the
-activation kernel after one another, in every weight format, with both tile sizes, a ragged last tile of columns (alternating gate
+activation kernel after one another, in every weight format and kind of launch (both tile sizes; one, for NVFP4 and 8-bit codes with
+groups of 32 rows), with a ragged last tile of columns (alternating gate
 and up only: halves need whole tiles), experts without rows, a bias and the routing weight on the input; the gate and up rows are
 not written then.  The row tiles of both GEMMs of a layer come from one launch, whichever of them may cut its tiles along K.
 Activations and widths that the tiles do not take go the old way."""
@@ -24,10 +25,17 @@ DEV = "cuda:0"
 
 def _experts(gen, kind, e, k, n, dtype):
     """Random experts in the Marlin layout: weights, scales, zero points."""
-    words = 4 if kind == "uint8b128" else 2
+    words = 2 if kind in ("uint4b8", "uint4", "mxfp4", "nvfp4") else 4
     q = torch.randint(-2 ** 31, 2 ** 31 - 1, (e, k // 16, words * n), dtype=torch.int32, device=DEV, generator=gen)
     if kind == "mxfp4":
         s = torch.randint(117, 122, (e, k // 32, n), dtype=torch.uint8, device=DEV, generator=gen).view(torch.float8_e8m0fnu)
+    elif kind == "nvfp4":   # as the loading leaves them: the upper bytes of 1 to 4 times 2^7 in fp16, shifted by one
+        s = torch.randint(0xB0, 0xC0, (e, k // 16, n), dtype=torch.uint8, device=DEV, generator=gen).view(torch.float8_e4m3fn)
+    elif kind == "fp8":     # a scale a column, the codes' exponent bias in it; no code that is NaN
+        q &= 0x77777777
+        s = (torch.rand((e, 1, n), device=DEV, generator=gen) * 2.56e-2 + 2.56e-3).to(dtype)
+    elif kind == "uint8b128g32":
+        s = ((torch.rand((e, k // 32, n), device=DEV, generator=gen) * 9e-3 + 1e-3) / 16).to(dtype)
     else:
         s = (torch.rand((e, k // 64, n), device=DEV, generator=gen) * 9e-3 + 1e-3).to(dtype)
         s = s / 16 if kind == "uint8b128" else s
@@ -45,6 +53,18 @@ def _experts(gen, kind, e, k, n, dtype):
                                                          ("silu", 1024, 320, True), ("gelu", 1024, 1024, False)])
 @pytest.mark.parametrize("on_input", [False, True])
 def test_layer(kind, dtype, activation, inter, k, in_tiles, on_input):
+    _check_layer(kind, dtype, activation, inter, k, in_tiles, on_input)
+
+
+@pytest.mark.parametrize("kind,dtype", [("nvfp4", torch.float16), ("nvfp4", torch.bfloat16), ("uint8b128g32", torch.bfloat16),
+                                        ("fp8", torch.float16)])
+@pytest.mark.parametrize("activation,inter,k,in_tiles", [("silu", 384, 320, True), ("swigluoai", 384, 192, True),
+                                                         ("swigluoai", 576, 1024, True), ("silu", 320, 320, False)])
+def test_layer_of_other_formats(kind, dtype, activation, inter, k, in_tiles):
+    _check_layer(kind, dtype, activation, inter, k, in_tiles, inter == 384)
+
+
+def _check_layer(kind, dtype, activation, inter, k, in_tiles, on_input):
     if kind != "mxfp4" and inter % 64:   # the down projection's groups
         inter = 448
     m, e, top_k = 1500 if kind == "mxfp4" else 700, 6, 2   # (MXFP4: more than marlin_mid_gemm takes)
@@ -59,12 +79,18 @@ def test_layer(kind, dtype, activation, inter, k, in_tiles, on_input):
     weights, ids = torch.topk(torch.softmax(logits, dim=1), top_k, dim=1)
     weights, ids = weights.contiguous(), ids.to(torch.int32)
     wtype = {"uint4b8": scalar_types.uint4b8, "uint4": scalar_types.uint4, "mxfp4": scalar_types.float4_e2m1f,
-             "uint8b128": scalar_types.uint8b128}[kind]
+             "uint8b128": scalar_types.uint8b128, "uint8b128g32": scalar_types.uint8b128, "fp8": scalar_types.float8_e4m3fn,
+             "nvfp4": scalar_types.float4_e2m1f}[kind]
+    global_scale = None
+    if kind == "nvfp4":
+        global_scale = torch.rand(e, device=DEV, generator=gen) * 1e-3 + 1e-3
+        global_scale *= 2.0 ** (7 if dtype == torch.float16 else 119)
     assert fused_moe.moe_block_size(m, top_k, e) == 64 and 2 * inter > k or k == 1024
 
     def layer(**kw):
         return fused_moe.fused_marlin_moe(x, w1, w2, bias1, None, s1, s2, weights, ids, wtype.id, on_input,
-                                          activation=activation, w1_zeros=z1, w2_zeros=z2, **kw)
+                                          activation=activation, w1_zeros=z1, w2_zeros=z2, global_scale1=global_scale,
+                                          global_scale2=global_scale, **kw)
 
     rows = m * top_k
     cache13 = torch.full((rows * max(2 * inter, k),), -7.0, dtype=dtype, device=DEV)
