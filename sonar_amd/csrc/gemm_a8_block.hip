@@ -9,21 +9,21 @@
 // column's 32 rows of a chunk in four lanes; v_permlane16_swap, one per two packed words, makes it two.
 //
 // What bounds it: with few rows the vector instructions that dequantise (9.5 per packed word, of which 2 put the
-// bytes into the order of K).  With many rows the issue of instructions: beside matrix instructions a SIMD starts one
-// instruction of its wavefronts every 4.7 cycles, and 9.4 other vector instructions go with a matrix instruction (16
-// multiply-adds of the group scales per tile and group, and a wavefront dequantises its whole strip for 128 rows); at 2048
-// rows, K 4096, N 11008, int8, 1.5 POP/s, where the int8 instruction alone reaches 3.15 on random operands.  R = 3 with 256
-// registers, R = 4 where the scales in flight leave room for it.
+// bytes into the order of K).  With many rows vector instructions and waits: at 2048 rows, K 4096, N 11008, int8, 10.0 other vector
+// instructions go with a matrix instruction (16 multiply-adds of the group scales per tile and group, and a wavefront
+// dequantises its whole strip for 128 rows), vector issue fills 57 % of the cycles, the matrix pipes 41 %, a fifth of the
+// wavefronts' time is waits, and 13 % of the cycles are bank conflicts; 1.5 POP/s, where the int8 instruction alone reaches 3.15 on
+// random operands.  R = 3 with 256 registers, R = 4 where the scales in flight leave room for it.
 // Measured against the kernels it takes over from (us, before -> now):
 //   M  153, K 1152, N 22976, fp8:  42 -> 23       M  259, K 3456, N 20032, int8: 172 -> 40
 //   M  987, K 1664, N 12608, int8: 206 -> 55      M 2048, K 4096, N 11008, int8: 181 -> 137
+//   M 1929, K 3072, N 25216, int8, groups of 32, zero points: 1836 -> 536
+//   44 random shapes of 17 to 8192 rows: 1.69 times as fast (geometric mean; one, of 25 rows, 0.89)
 // and since rows of C leave as whole lines (they were 2-byte stores from a lane's column):
 //   M 1024, K 4096, N  8192, int8: 67 -> 56       M 2048, K 4096, N 11008, int8: 146 -> 124 (the same box)
 //   M   64, K 4096, N 11008, int8, 64 rows a tile: 18.8 -> 17.2      M 1213, K 1152, N 6336: 39 -> 24 with the quantisation
 // and since copies have a scalar base and 32-bit offsets:
 //   M 2048, K 4096, N 11008, int8, with the quantisation: 118.3 -> 116.6
-//   M 1929, K 3072, N 25216, int8, groups of 32, zero points: 1836 -> 536
-//   44 random shapes of 17 to 8192 rows: 1.69 times as fast (geometric mean; one, of 25 rows, 0.89)
 //
 // Pipeline, per step of 128 rows of K: activations (shared by the strips of a range) and packed codes (a wavefront's
 // own) go to LDS by LDS-DMA and the scales to registers, two steps ahead (three with one row block), and one

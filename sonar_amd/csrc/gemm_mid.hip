@@ -26,7 +26,8 @@
 //   M   80, K 4096, N 28672: 27.9 -> 36.5, 45.0       M  144, K 4096, N 11008: 22.9 -> 27.9, 29.7
 // Five and six row blocks on four wavefronts with 512 registers each took 30 and 33 us in the first call with M 80 and 96, and
 // 1.5 times as long as eight wavefronts elsewhere.
-// (Copies of activations by asm with a scalar base: the first two 22.1 -> 21.7 and 17.8 -> 17.5.)
+// (Copies of activations by asm with a scalar base, the trees before and after in turn: the first two 22.8 -> 22.5 and 18.1 -> 17.9
+// with the host, where two runs of one tree differ by up to 0.1.)
 // Measured against the kernels it takes over from (us, before -> now):
 //   M   64, K 4096, N 28672, bf16: 29.1 -> 21.7      M  200, K 4096, N 6144, fp16, zero points: 24.6 -> 17.6
 //   M  333, K 2880, N  5760, bf16, groups of 32: 40.5 -> 21.7      M  512, K 4096, N 2048, bf16: 36 -> 20

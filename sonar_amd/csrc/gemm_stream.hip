@@ -678,8 +678,9 @@ struct FastLane {
   int s_strip_stride;   // bytes between strips for s_ptr
 };
 
-// Copies have a scalar base and 32-bit offsets, and the four of a unit's codes one address: four decoder layers of 4096 / 6144 /
-// 14336, 16 rows 164.9 -> 163.5 us.
+// Copies have a scalar base and 32-bit offsets, and the four of a unit's codes one address (four decoder layers of 4096 / 6144 /
+// 14336, 16 rows, with the trees before and after in turn twice: 165.5 -> 164.2 and 167.0 -> 166.3 us, hardly more than two runs
+// of one tree differ by).
 // unit_group_shift: s >= 0 for groups of 128 * 2^s rows, -1 for one group; with
 // GPU > 1 the unit holds groups GPU * unit .. GPU * unit + GPU - 1.
 template <bool HAS_ZP, int MB, int GPU>
@@ -786,8 +787,8 @@ __device__ __forceinline__ floatx4_t quad_transpose(floatx4_t x, int lane) {
 // scales it holds 170 to 216 registers, so two wavefronts fit a SIMD as with one set.
 // FP4 (with GPU = 4, no zero points): float4_e2m1f codes; the operands are the
 // converted values themselves, so only the scale is left for after the unit.
-// A workgroup works on one piece of one strip (StreamParams::piece_shift / piece_units):
-// units unit0 .. unit0 + piece_units - 1 of strip `part >> piece_shift`, dealt round-robin
+// A workgroup works on one piece of one strip (StreamParams::pieces): units
+// i * units_per_strip / pieces and on of strip `part / pieces`, i = part % pieces, dealt round-robin
 // to its wavefronts.  It sums its wavefronts once, at the end (the tiles of that sum are
 // parked on top of the copy rings, every copy having been consumed by then), and either
 // writes C (the piece is the whole strip) or leaves fp32 partial tiles and draws the

@@ -224,7 +224,9 @@ __host__ __device__ __forceinline__ float pair_cost(int big, int small, const Pa
   int tiles[2] = {(big - plan.halved) * tiles_n, (small + 2 * plan.halved) * tiles_n};
   float time[2] = {kPairBig, kPairSmall}, extra = 0.f;
   for (int i = 0; i < 2; ++i)
-    if (plan.splits[i] > 1) {   // (a K step of a 256-row tile is about 1.4 us, its start and end 13 us, the sum of the partial tiles 8 us)
+    // (a K step of a 256-row tile is about 1.4 us, its start and end 13 us, the sum of the partial tiles 8 us: as measured with
+    // results stored from the registers; whole lines have made the end shorter since, and a gated activation longer)
+    if (plan.splits[i] > 1) {
       tiles[i] *= plan.splits[i];
       time[i] *= (k_steps / (float)plan.splits[i] + 11.f) / (k_steps + 9.f);
       extra = 8.f / (1.4f * k_steps + 13.f);
@@ -1120,7 +1122,7 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
 
   // ---- sources (regions of A as in marlin_tile_async_kernel; wavefront w fills RB / 2 regions)
   // Memory operations take a scalar base and a 32-bit offset a lane where they can: with a 64-bit address a lane each holds up the
-  // wavefront's other instructions 20 cycles longer.  (M = 8192, K = 4096, N = 28672, fp16 1357 -> 1343 us; one tile alone 74.2 -> 73.4.)
+  // wavefront's other instructions 20 cycles longer.  (M = 8192, K = 4096, N = 28672, fp16 1368 -> 1355 us; one tile alone 74.2 -> 73.4.)
   // Dense calls: a wavefront's rows of A are within 32 bits of its first (wide_rows_within_32_bits); the rows of a grouped tile
   // may be anywhere.
   const int a_first = GROUPED ? 0 : min(m0 + 4 * RB * wave, p.size_m - 1);
@@ -2088,12 +2090,13 @@ int launch_tile(const TileParams& p, hipStream_t st) {
 }  // namespace
 
 namespace {
+// (grouped calls: 64-bit addresses)
+bool wide_takes_rows(const TileParams& p) { return p.tile_table != nullptr || wide_rows_within_32_bits(p.lda); }
 // The wide form: groups of 32 or 64 * 2^i rows or one group, K of any number of steps.  (Passes of the loop were whole
 // before: up to three steps of zeros where that was at most a tenth of K, and eight wavefronts elsewhere.  Us, before ->
 // now: int4 with groups of 32, M = 4096, K = 2880, N = 5760 204 -> 142; AWQ, M = 4000, K = 1152, N = 6144 117 -> 71; NVFP4
 // bf16, M = 2048, K = 4480, N = 8192 148 -> 118; MXFP8, M = 3000, K = 2944, N = 6144 188 -> 168; int4, M = 2000, K = 2944,
 // N = 7808, once padded, 81.5 -> 78.3; 2000 tokens on 32 MXFP4 experts of 2880 x 2880, the whole layer 626 -> 543.)
-bool wide_takes_rows(const TileParams& p) { return p.tile_table != nullptr || wide_rows_within_32_bits(p.lda); }
 bool wide_applies(const TileParams& p) {
   static const bool no_wide = getenv("SONAR_MARLIN_NO_WIDE_TILE") != nullptr;   // debugging aid
   if (!wide_takes_rows(p)) return false;
