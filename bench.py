@@ -202,7 +202,7 @@ def launch_floors(torch, time_graph):
 
 def cpu_baseline(threads: int):
     """The layer's CPU path (int4 dequantise + fp32 torch.matmul) from the
-    oracle at M = 16: `value` on the o_proj shape (BASELINE configuration 1), and
+    oracle at M = 16: `value` on the o_proj shape, and
     the same on the other three projection shapes under `layer` (a bounded sample:
     one layer's four GEMMs, 2 + 5 runs each, 20 to 30 s of CPU work)."""
     import numpy as np
@@ -451,7 +451,7 @@ def main() -> int:
                          "a counter run has a kernel of known traffic to scale FETCH_SIZE / WRITE_SIZE by")
     args = ap.parse_args()
     if args.gpus != 1:
-        print("bench.py: this build runs on one GPU only (the GEMM is rank-local; no multi-GPU path "
+        print("bench.py: runs on one GPU only (the GEMM is rank-local; no multi-GPU path "
               "exists); run with --gpus 1", file=sys.stderr)
         return 2
     if not 1 <= args.m <= 64:

@@ -1,7 +1,7 @@
 """CPU oracle for the Marlin W4A16 path.  TEST INFRASTRUCTURE ONLY.
 
 This module restates, in plain numpy, the algorithms the reference implements
-for its Marlin-family W4A16 GEMM.  It is the checker that the HIP kernels are
+for its Marlin-family W4A16 GEMM.  It is what the HIP kernels are
 compared against.  Nothing in the shipped package imports it: only tests,
 ``__graft_entry__.smoke()`` and the ``cpu_baseline`` leg of ``bench.py`` do.
 
@@ -29,7 +29,7 @@ reference checkout).  How each function is pinned (none is "parity unpinned"):
                            fused_moe/moe_align_block_size.py:60-73 and set
                            equality per expert
                            (tests/kernels/moe/test_moe_align_block_size.py)
-* gfx950 layout            this build's own format: inverse round trip and
+* gfx950 layout            the package's own format: inverse round trip and
                            decode-to-(K,N) equality with the Marlin decode
 * 8-bit weights (W8A16)    the same pinning as the 4-bit functions: recipe
                            (get_weight_perm(8), interleave [0,2,1,3]) against
@@ -904,7 +904,7 @@ def nvfp4_process_global_scale(global_scale: float, dtype: str, scale_factor: fl
 
 
 def nvfp4_kernel_scales(scale_bytes: np.ndarray, dtype: str) -> np.ndarray:
-    """The block scales as this build's kernels take them: the kernel-side reading
+    """The block scales as the package's kernels take them: the kernel-side reading
     of a byte times 2^-(exponent bias), the factor the reference's dequantised
     code carries (dequant.h:397-470: a code read as fp16 / bf16 is value *
     2^-bias).  Plain marlin_permute_scales order (the 0, 2, 1, 3 reorder undone).
@@ -993,7 +993,7 @@ def stable_sort_g_idx(g_idx: np.ndarray):
 
 
 # --------------------------------------------------------------------------
-# gfx950 streaming layout (this build's own format; no reference counterpart)
+# gfx950 streaming layout (the package's own format; no reference counterpart)
 # --------------------------------------------------------------------------
 # The (K,N) code matrix is cut into 64-column strips; a strip is a contiguous
 # run of K/32 one-KiB chunks, chunk c covering rows [32c, 32c+32).  Inside a
@@ -1111,7 +1111,7 @@ def gemm_reference(a32: np.ndarray, w32: np.ndarray, bias32: np.ndarray | None =
 
 
 def gemm_tolerance_ok(out32: np.ndarray, ref32: np.ndarray):
-    """The acceptance rule of this build: max|err| <= 1e-2*max|ref| and
+    """The acceptance rule of the GEMM tests: max|err| <= 1e-2*max|ref| and
     |err| <= 1e-2*max|ref| + 1e-2*|ref| elementwise.  Returns (ok, max_err,
     max_ref)."""
     err = np.abs(out32.astype(np.float64) - ref32.astype(np.float64))
