@@ -100,7 +100,7 @@ inline double mid_estimate(int64_t size_m, int64_t size_n, int64_t size_k, int64
 }
 
 // Whether a call that the tile kernels could take runs in this kernel, whose time mid_estimate puts at `mid_us`, with K in
-// `splits` ranges.
+// `splits` ranges.  `twin`: tile_twin_applies.
 // What mid_estimate lacks on the calls tile_estimate was fitted to, with K in one piece: kSlow.  (A time of the tile kernels that
 // grows with the operations alone, and 0.93 for either kernel: 2.7 % slower than the better of the two on 147 random calls, at
 // worst 1.6 times; so 0.6 %, 1.3 times.)
@@ -111,8 +111,8 @@ inline double mid_estimate(int64_t size_m, int64_t size_n, int64_t size_k, int64
 // K = 6144, N = 6400 51.4 -> 34.9; M = 134, K = 3968, N = 26240 71.8 -> 53.0; integers, M = 196, K = 1664, N = 11392
 // 29.9 -> 24.0).
 inline bool mid_beats_tiles(double mid_us, int splits, int64_t size_m, int64_t size_n, int64_t size_k, int64_t num_groups,
-                            int group_size, bool float16, int format, bool rows_97_128) {
-  static const double kStep[6] = {kTileStepInt4, kTileStepInt4, 1.27, 1.27, 1.14, 1.30};
+                            int group_size, bool float16, int format, bool rows_97_128, bool twin) {
+  static const double kStep[6] = {kTileStepInt4, kTileStepInt4, 1.27, 1.27, kTileStepMxFp4, 1.30};
   static const double kSlow[6][2] = {   // float16, bfloat16
       {1.12, 1.10}, {1.18, 1.10}, {1.30, 1.12}, {1.13, 1.05}, {1.22, 1.22}, {1.03, 1.0}};
   const bool is_8bit = format == kMidInt8 || format == kMidFp8, groups_of_32 = num_groups > 1 && group_size == 32;
@@ -120,6 +120,9 @@ inline bool mid_beats_tiles(double mid_us, int splits, int64_t size_m, int64_t s
   else if (splits > 1) mid_us *= 0.94;
   else mid_us *= format == kMidFp8 && groups_of_32 ? 0.97 : kSlow[format][float16 ? 0 : 1];
   const bool rows128 = format != kMidNvFp4 && !(is_8bit && groups_of_32);
+  if (twin && twin_pays(size_m, size_n, size_k, float16, format == kMidMxFp4, rows128, rows_97_128) &&
+      twin_estimate(size_m, size_n, size_k, float16, format == kMidMxFp4) <= mid_us)
+    return false;
   return mid_us < tile_estimate(size_m, size_n, size_k, kStep[format], rows128, rows_97_128);
 }
 

@@ -108,7 +108,7 @@ inline GemmPlan tile_plan(int64_t size_m, int64_t size_n, int64_t size_k, bool r
   return plan_gemm(size_m, size_n, size_k, true, 256, rows_97_128);
 }
 
-constexpr double kTileStepInt4 = 1.21;   // tile_estimate's `step` of 4-bit integer codes
+constexpr double kTileStepInt4 = 1.21, kTileStepMxFp4 = 1.14;   // `step` of tile_estimate
 
 // Microseconds the tile kernels take: rounds of workgroups, each 11.2 us around its loop and `step` us per 64 rows of K for a
 // 256-row tile (0.58 of both for a 128-row one), 3.3 us for the launch, and for K in ranges a second launch and its bytes.  A fit
@@ -125,6 +125,27 @@ inline double tile_estimate(int64_t size_m, int64_t size_n, int64_t size_k, doub
   if (last > 128 || (last > 0 && plan.k_splits < 3 && (tiles < 256 || !rows128))) us += whole;
   else if (last > 0) us += plan.k_splits >= 3 ? range + 1.1 : 0.58 * whole;
   return us;
+}
+
+// Microseconds of marlin_tile_twin_kernel (128-row tiles over the whole of K, two at a time on a compute unit): so many pairs of tiles
+// as a compute unit gets, and a single one where their number is odd.  A fit of 156 random calls of 256 to 8192 rows, K = 512 to
+// 7168: 80 % within 9 %.  Taken where this is below tile_estimate, it is 0.7 % (float16), 1.0 % (bfloat16 integers) and 0.1 % (MXFP4)
+// above the better of the two on those, no call more than 1.7 % slower than before.
+inline double twin_estimate(int64_t size_m, int64_t size_n, int64_t size_k, bool float16, bool fp4) {
+  const double pair_step = fp4 ? 1.25 : float16 ? 1.34 : 1.41, one_step = fp4 ? 0.78 : float16 ? 0.93 : 1.02;
+  const int64_t steps = size_k / 64, tiles = ((size_m + 127) / 128) * ((size_n + 255) / 256), most = (tiles + 255) / 256;
+  return 3.3 + most / 2 * (pair_step * steps + 6.4) + most % 2 * (one_step * steps + 1.0);
+}
+// Whether a dense call that could have such tiles has them: where 256-row tiles would run otherwise (more than half a round of them),
+// and the estimates say so; by 3 % where it is at most one round of them, as both take a round then (M = 2834, K = 2304, N = 4352, AWQ,
+// fp16: 56.5 us there, 58.8 here; M = 2755, K = 1664, N = 3712, groups of 32 39.5 / 41.0).  On 246 random calls in turn with the
+// tree before, 0.965 times the time: M = 332, K = 3200, N = 17728, AWQ, fp16 (140 tiles of 256 rows, 210 of 128) 64.5 -> 43.0; M = 855,
+// K = 1024, N = 17472, MXFP4 (276 / 483) 48.2 -> 32.4; M = 4000, K = 512, N = 28672 148 -> 115; M = 569, K = 2944, N = 24512, bf16 110 -> 75.
+inline bool twin_pays(int64_t size_m, int64_t size_n, int64_t size_k, bool float16, bool fp4, bool rows128, bool rows_97_128) {
+  const double least = ((size_m + 255) / 256) * ((size_n + 255) / 256) <= 256 ? 0.97 : 1.0;
+  return tile_plan(size_m, size_n, size_k, rows128, rows_97_128).tile_rows == 256 &&
+         twin_estimate(size_m, size_n, size_k, float16, fp4) <
+             least * tile_estimate(size_m, size_n, size_k, fp4 ? kTileStepMxFp4 : kTileStepInt4, rows128, rows_97_128);
 }
 
 // Scratch for the partial tiles of either tiling.

@@ -36,6 +36,7 @@ int tile_gemm(const void* a, int64_t a_row_stride, void* c, const uint32_t* b, c
               int64_t size_n, int64_t size_k, int64_t num_groups, int group_size, void* partial,
               size_t partial_bytes, bool fp4, int bits, bool fp8, hipStream_t st);
 bool tile_async_applies(bool has_perm, int64_t num_groups, int group_size);
+bool tile_twin_applies(int bits, bool nvfp4, int64_t num_groups, int group_size, int64_t a_row_stride);
 
 namespace {
 
@@ -1912,7 +1913,7 @@ int marlin_gemm_any(const void* a, int64_t a_row_stride, void* c, const uint32_t
       take = mid_us < decode_rows_estimate(size_m, n_strips, size_k, chk.has_zp, cus);
     } else if (use_tile) {
       take = mid_beats_tiles(mid_us, splits, size_m, size_n, size_k, num_groups, chk.group_size, dtype == SONAR_DTYPE_F16, format,
-                             rows_97_128);
+                             rows_97_128, tile_twin_applies(chk.bits, chk.nvfp4, num_groups, chk.group_size, a_row_stride));
     } else {   // (the general kernels, us: a fit of measured times; few strips: shared between workgroups, and a second launch)
       const double x = (double)size_n * size_k / (6144.0 * 4096.0), r = size_m / 64.0;
       const double us = size_m <= 64 ? (n_strips < 64 ? 12.0 : 9.5) + x * (5.5 + 5.2 * r * r) : 11.0 + 10.7 * x * r;
@@ -2102,7 +2103,8 @@ extern "C" int sonar_debug_mid_beats_tiles(int64_t size_m, int64_t size_n, int64
   const double us = mid_estimate(size_m, size_n, size_k, num_groups, dtype, format, false, 256,
                                  sonar_marlin_gemm_scratch_bytes(size_m, size_n, size_k), row_blocks, splits);
   return mid_beats_tiles(us, splits, size_m, size_n, size_k, num_groups, (int)(size_k / num_groups), dtype == SONAR_DTYPE_F16, format,
-                         plan_rows_97_128(size_m, size_n, size_k, format == kMidInt4 || format == kMidInt4Zp)) ? 1 : 0;
+                         plan_rows_97_128(size_m, size_n, size_k, format == kMidInt4 || format == kMidInt4Zp),
+                         tile_twin_applies(format == kMidInt4 || format == kMidInt4Zp ? 4 : 8, false, num_groups, (int)(size_k / num_groups), size_k)) ? 1 : 0;
 }
 
 extern "C" int sonar_marlin_gemm(const void* a, int64_t a_row_stride, void* c,

@@ -1068,9 +1068,10 @@ __device__ __forceinline__ void store_gated(const TileParams& p, uint32_t a_lds,
 // NV (with FP4): NVFP4, a scale per 16 rows: the row of a k block then holds two groups of 128 bytes (the copy
 // fetches one per half of the wavefront), and a lane, whose eight rows of a k block lie in one group, reads group
 // kb / 2; the global scale multiplies the sums at the end.
+// TWIN (with RB = 8): the form of marlin_tile_twin_kernel.
 // The tile (tile_m, tile_n) of a launch, over K steps [k_first, k_tiles); `table`: of the row tiles of a grouped call;
 // partial_at: index of the workgroup's partial tile in `partial`, or -1 when it has the whole of K.
-template <typename T, bool HAS_ZP, bool GROUPED, int RB, bool FP4, int W8, bool G32, bool NV>
+template <typename T, bool HAS_ZP, bool GROUPED, int RB, bool FP4, int W8, bool G32, bool NV, bool TWIN = false>
 __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* table, float4* partial, const int tile_m,
                                           const int tile_n, const int k_first, const int k_tiles, const int partial_at) {
   typedef typename Dq<T>::vec8 vec8;
@@ -1087,6 +1088,7 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
   static_assert(!NV || (FP4 && RB == 16), "NVFP4 is float4 codes; 256-row tiles");
   static_assert(!(W8 != 0 && G32) || RB == 16, "8-bit codes with groups of 32 rows: 256-row tiles");
   static_assert(RB == 16 || RB == 8, "256-row tiles or 128-row tiles");
+  static_assert(!TWIN || (RB == 8 && W8 == 0 && !NV), "4-bit integers and MXFP4");
   constexpr int kRows = 16 * RB;
   constexpr int kStage = wide_stage(RB), kWideA = wide_a(RB), kWideOps = wide_ops(RB, G32, W8 != 0);
   constexpr int kAgprBlocks = RB == 16 ? 14 : RB;   // row blocks whose accumulators sit in AGPRs
@@ -1127,7 +1129,8 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
   // may be anywhere.
   const int a_first = GROUPED ? 0 : min(m0 + 4 * RB * wave, p.size_m - 1);
   const char* a_rows = reinterpret_cast<const char*>(p.a + (long)a_first * p.lda);
-  typename std::conditional<GROUPED, const char*, uint32_t>::type a_src[RB / 2];
+  constexpr bool kFarRows = GROUPED && !TWIN;
+  typename std::conditional<kFarRows, const char*, uint32_t>::type a_src[RB / 2];
 #pragma unroll
   for (int i = 0; i < RB / 2; ++i) {
     const int region = (RB / 2) * wave + i;
@@ -1142,7 +1145,7 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
       row = m0 + in_tile;
       if (row >= p.size_m) row = p.size_m - 1;   // rows past M are computed and never stored
     }
-    if constexpr (GROUPED) a_src[i] = a_rows + ((long)row * p.lda + 8 * ((lane & 7) ^ r8)) * 2;
+    if constexpr (kFarRows) a_src[i] = a_rows + ((long)row * p.lda + 8 * ((lane & 7) ^ r8)) * 2;
     else a_src[i] = (uint32_t)(row - a_first) * (uint32_t)(p.lda * 2) + 16 * ((lane & 7) ^ r8);
   }
   const char* b_base = reinterpret_cast<const char*>(p.b + expert * p.expert_b_stride) +
@@ -1153,7 +1156,7 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
   if (kScaleSums && !grouped) s_base = W8 == 2 ? reinterpret_cast<const char*>(&kOnesFp8) : reinterpret_cast<const char*>(&kOnesInt8);
   const char* z_src = reinterpret_cast<const char*>(p.zeros + expert * p.expert_z_stride + strip * 8 + (lane & 7));
   const long s_group_stride = (long)p.size_n * 2;
-  const long sz_group_stride = HAS_ZP && lane >= 32 ? (long)(p.size_n / 8) * 4 : s_group_stride;
+  const uint32_t sz_group_stride = HAS_ZP && lane >= 32 ? (uint32_t)p.size_n / 2 : (uint32_t)s_group_stride;
   const char* sz_src = HAS_ZP && lane >= 32 ? z_src : s_base + 4 * (lane & 31);
   const uint32_t s_lane = 4 * (lane & 31) + (NV ? (lane >> 5) * (uint32_t)s_group_stride : 0);   // (NVFP4: the next group's row)
   // steps per group as a shift (the host checks: group_size = 64 * 2^i)
@@ -1170,7 +1173,7 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
     const int grp = G32 ? (NV ? 2 : 1) * (2 * k + h) : (grouped ? k >> group_shift : 0);
     const int at = G32 ? 2 * (kt - k_first) + h : kt - k_first;
     if constexpr (HAS_ZP)
-      __builtin_amdgcn_global_load_lds((glb_void_t*)(sz_src + (long)grp * sz_group_stride),
+      __builtin_amdgcn_global_load_lds((glb_void_t*)(sz_src + (uint64_t)(uint32_t)grp * sz_group_stride),
                                        (lds_void_t*)(sring + (at & (kWideScaleRows - 1)) * 256), 4, 0, 0);
     else
       copy_to_lds<4>(s_lds + (at & (kWideScaleRows - 1)) * 256, s_lane, s_base + grp * s_group_stride);
@@ -1181,7 +1184,7 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
     const int k = min(kt, k_tiles - 1);
     if (idx < RB / 2) {
       const uint32_t to = slot * kStage + ((RB / 2) * wave + idx) * kBlockBytes;
-      if constexpr (GROUPED)
+      if constexpr (kFarRows)
         __builtin_amdgcn_global_load_lds((glb_void_t*)(a_src[idx] + (long)k * (kTileK * 2)), (lds_void_t*)(smem + to), 16, 0, 0);
       else
         copy_to_lds<16>(a_lds + to, a_src[idx], a_rows + (long)k * (kTileK * 2));
@@ -1196,7 +1199,7 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
 
   uint32_t s_off[4];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) s_off[j] = 2 * scale_slot(16 * j + col16, grouped);
+  for (int j = 0; j < 4; ++j) s_off[j] = 2 * scale_slot(16 * j + col16, TWIN || grouped);
   const uint32_t z_off = 128 + 4 * zero_point_word(col16);
   // operand lane (kb, col16) of row block 0, k block b of stage 0: piece 4 b + kb of row col16
   uint32_t a_base[2];
@@ -1209,6 +1212,10 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
   for (int nb = 0; nb < 4; ++nb)
 #pragma unroll
     for (int mb = 0; mb < RB; ++mb) {
+      if constexpr (TWIN) {   // (copies of one register of zeros need that register beside the 128 AGPRs there are)
+        asm volatile("s_nop 1\n\tv_mfma_f32_16x16x32_f16 %0, %1, %1, 0" : "=a"(acc[nb][mb]) : "v"(u32x4_t{0, 0, 0, 0}));
+        continue;
+      }
       acc[nb][mb] = floatx4_t{0.f, 0.f, 0.f, 0.f};
       // the zeros sit where the MFMAs will hold the accumulator, so that the value has one home
       // on every path to the stores
@@ -1216,11 +1223,14 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
       else asm volatile("" : "+v"(acc[nb][mb]));
     }
 
-  constexpr int kAhead = 4;   // operands of A are read this many row blocks ahead
-  u32x4_t av[8];          // row block rb in av[rb & 7]
+  constexpr int kAhead = TWIN ? 3 : 4, kAv = TWIN ? 4 : 8;   // operands of A are read this many row blocks ahead
+  u32x4_t av[kAv];        // row block rb in av[rb % kAv]
   uint32_t wb[2][4][4];   // dequantised chunk of k block b: four operand blocks of 16 columns, four pairs each
   uint32_t sb0 = 0, sb1 = 0, sb2 = 0, sb3 = 0, zw = 0;
-  Col cols[2][4];         // by the parity of the step (MXFP4: of the k block)
+  // a shift more for two nibbles of a word, and half the constants, which would not fit the registers
+  constexpr bool kOneForm = TWIN && HAS_ZP && std::is_same<T, __bf16>::value;
+  constexpr int kColSets = TWIN ? 1 : 2;
+  Col cols[kColSets][4];  // by the parity of the step (MXFP4: of the k block); TWIN: a column block's are replaced behind its last use
 
 #define SONAR_WIDE_READ(dst, base, off) \
   asm volatile("ds_read_b128 %0, %1 offset:%2" : "=&v"(dst) : "v"(base), "i"(off) : "memory")
@@ -1229,6 +1239,18 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
   auto scales_start = [&](int kt, int h) __attribute__((always_inline)) {
     const uint32_t r_at = s_lds + ((G32 ? 2 * (kt - k_first) + h : kt - k_first) & (kWideScaleRows - 1)) * 256 +
                           (NV ? 128 * (kb >> 1) : 0);
+    if constexpr (TWIN) {
+      asm volatile(
+          "ds_read_u16 %0, %5\n\t"
+          "ds_read_u16 %1, %5 offset:4\n\t"
+          "ds_read_u16 %2, %5 offset:8\n\t"
+          "ds_read_u16 %3, %5 offset:12\n\t"
+          "ds_read_b32 %4, %6"
+          : "=&v"(sb0), "=&v"(sb1), "=&v"(sb2), "=&v"(sb3), "=&v"(zw)
+          : "v"(r_at + s_off[0]), "v"(HAS_ZP ? r_at + z_off : r_at + s_off[0])
+          : "memory");
+      return;
+    }
     asm volatile(
         "ds_read_u16 %0, %5\n\t"
         "ds_read_u16 %1, %6\n\t"
@@ -1244,8 +1266,8 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
     const uint32_t sbits = j == 0 ? sb0 : j == 1 ? sb1 : j == 2 ? sb2 : sb3;
     int z = 8;
     if (HAS_ZP) z = (int)((zw >> zero_point_shift(16 * j + col16)) & 0xFu);
-    if constexpr (W8 != 0) cols[set][j] = D8::make_col((uint16_t)sbits);
-    else cols[set][j] = D4::make_col((uint16_t)sbits, z);
+    if constexpr (W8 != 0) cols[set % kColSets][j] = D8::make_col((uint16_t)sbits);
+    else cols[set % kColSets][j] = D4::make_col((uint16_t)sbits, z);
   };
   auto word_of = [](const u32x4_t& q, int j) __attribute__((always_inline)) -> uint32_t {
     return j == 0 ? q.x : j == 1 ? q.y : j == 2 ? q.z : q.w;
@@ -1254,11 +1276,11 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
   auto mfma = [&](int B, int j, int rb) __attribute__((always_inline)) {
     const u32x4_t w = u32x4_t{wb[B][j][0], wb[B][j][1], wb[B][j][2], wb[B][j][3]};
     if constexpr (std::is_same<T, _Float16>::value) {
-      if (rb < kAgprBlocks) asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(acc[j][rb]) : "v"(w), "v"(av[rb & 7]));
-      else asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(acc[j][rb]) : "v"(w), "v"(av[rb & 7]));
+      if (rb < kAgprBlocks) asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(acc[j][rb]) : "v"(w), "v"(av[rb % kAv]));
+      else asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(acc[j][rb]) : "v"(w), "v"(av[rb % kAv]));
     } else {
-      if (rb < kAgprBlocks) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[j][rb]) : "v"(w), "v"(av[rb & 7]));
-      else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc[j][rb]) : "v"(w), "v"(av[rb & 7]));
+      if (rb < kAgprBlocks) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[j][rb]) : "v"(w), "v"(av[rb % kAv]));
+      else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc[j][rb]) : "v"(w), "v"(av[rb % kAv]));
     }
   };
 
@@ -1283,14 +1305,14 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
       const int j = (kPairs * rb) >> 2, part = (kPairs * rb) & 3;
       // reads started after the one of this row block: those of the next kAhead - 1 row blocks,
       // and the five scale reads of slot 0 (first half; MXFP4: either half)
-      if ((B == 0 || G32) && rb >= 1 && rb <= kAhead) SONAR_WIDE_LANDED(kAhead - 1 + 5, av[rb & 7]);
-      else SONAR_WIDE_LANDED(kAhead - 1, av[rb & 7]);
+      if ((B == 0 || G32) && rb >= 1 && rb <= kAhead) SONAR_WIDE_LANDED(kAhead - 1 + 5, av[rb % kAv]);
+      else SONAR_WIDE_LANDED(kAhead - 1, av[rb % kAv]);
       // behind this wait the scale reads of slot 0 have landed: from here on the registers they fill
       // hold the scales (without this the compiler is free to use them any time after slot 0)
       if ((B == 0 || G32) && rb == (kAhead + 1 < RB ? kAhead + 1 : RB - 1))
         asm volatile("" : "+v"(sb0), "+v"(sb1), "+v"(sb2), "+v"(sb3), "+v"(zw) : : "memory");
-      if (rb + kAhead < RB) SONAR_WIDE_READ(av[(rb + kAhead) & 7], a_cur, (rb + kAhead) * 2048);
-      else SONAR_WIDE_READ(av[(rb + kAhead) & 7], a_next, (rb + kAhead - RB) * 2048);
+      if (rb + kAhead < RB) SONAR_WIDE_READ(av[(rb + kAhead) % kAv], a_cur, (rb + kAhead) * 2048);
+      else SONAR_WIDE_READ(av[(rb + kAhead) % kAv], a_next, (rb + kAhead - RB) * 2048);
       // the scales of the step after this one (MXFP4: of its k block B, two half steps ahead)
       if (rb == 0 && (B == 0 || G32)) scales_start(kt + 1, B);
       const uint32_t qw = word_of(q4, j);
@@ -1307,13 +1329,13 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
         if (RB == 8) x2 = D8::stage1(w8, 1, magic);
         __builtin_amdgcn_sched_barrier(0);
         mfma(B, 1, rb);
-        const typename D8::Mid y = D8::stage2(x, cols[set][jj]);
+        const typename D8::Mid y = D8::stage2(x, cols[set % kColSets][jj]);
         typename D8::Mid y2 = y;
-        if (RB == 8) y2 = D8::stage2(x2, cols[set][jj]);
+        if (RB == 8) y2 = D8::stage2(x2, cols[set % kColSets][jj]);
         __builtin_amdgcn_sched_barrier(0);
         mfma(B, 2, rb);
-        wb[NB][jj][2 * half + first] = D8::stage3(y, cols[set][jj]);
-        if (RB == 8) wb[NB][jj][2 * half + 1] = D8::stage3(y2, cols[set][jj]);
+        wb[NB][jj][2 * half + first] = D8::stage3(y, cols[set % kColSets][jj]);
+        if (RB == 8) wb[NB][jj][2 * half + 1] = D8::stage3(y2, cols[set % kColSets][jj]);
         __builtin_amdgcn_sched_barrier(0);
         mfma(B, 3, rb);
       } else if constexpr (NV && std::is_same<T, _Float16>::value) {
@@ -1328,14 +1350,14 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
         __builtin_amdgcn_sched_barrier(0);
         mfma(B, 2, rb);
         wb[NB][j][part] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, hbits) *
-                                                           __builtin_bit_cast(half2_t, cols[set][j].s2));
+                                                           __builtin_bit_cast(half2_t, cols[set % kColSets][j].s2));
         __builtin_amdgcn_sched_barrier(0);
         mfma(B, 3, rb);
       } else if constexpr (FP4 && kPairs == 2) {
         // MXFP4 with 8 row blocks: the conversions of an even and an odd part (rows (0,2) and (1,3), or (4,6) and
         // (5,7)) and their two byte permutes behind one row block
         mfma(B, 0, rb);
-        const float sc = cols[set][j].s;
+        const float sc = cols[set % kColSets][j].s;
         const uint32_t r_e = __builtin_bit_cast(uint32_t, part == 0 ? __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(qw, sc, 0)
                                                                     : __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(qw, sc, 1));
         __builtin_amdgcn_sched_barrier(0);
@@ -1353,7 +1375,7 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
         // column), the two values times the scale in fp32; behind the second and the fourth, the two byte
         // permutes that cut the products back to bf16 and put four rows in order (DqNvF4<__bf16>::word)
         mfma(B, 0, rb);
-        const float sc = cols[set][j].s;
+        const float sc = cols[set % kColSets][j].s;
         const uint32_t r = __builtin_bit_cast(
             uint32_t, part == 0   ? __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(qw, 1.0f, 0)
                       : part == 1 ? __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(qw, 1.0f, 2)
@@ -1378,7 +1400,7 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
         // one hardware conversion per row block (two rows of the column each: (0,2), (1,3), (4,6),
         // (5,7)); behind the second and the fourth, the two byte permutes that put four rows in order
         mfma(B, 0, rb);
-        const float sc = cols[set][j].s;
+        const float sc = cols[set % kColSets][j].s;
         const uint32_t r = __builtin_bit_cast(
             uint32_t, part == 0   ? __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(qw, sc, 0)
                       : part == 1 ? __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(qw, sc, 2)
@@ -1397,16 +1419,16 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
         mfma(B, 0, rb);
         const uint32_t x = Dq<T>::stage1(part < 2 ? qw : qw >> 8, part, magic);
         uint32_t x2 = 0;
-        if (kPairs == 2) x2 = Dq<T>::stage1(part < 2 ? qw : qw >> 8, part + 1, magic);
+        if (kPairs == 2) x2 = kOneForm ? Dq<T>::stage1(qw >> (part < 2 ? 4 : 12), part, magic) : Dq<T>::stage1(part < 2 ? qw : qw >> 8, part + 1, magic);
         __builtin_amdgcn_sched_barrier(0);
         mfma(B, 1, rb);
-        const Mid y = Dq<T>::stage2(x, cols[set][j], part);
+        const Mid y = Dq<T>::stage2(x, cols[set % kColSets][j], part);
         Mid y2 = y;
-        if (kPairs == 2) y2 = Dq<T>::stage2(x2, cols[set][j], part + 1);
+        if (kPairs == 2) y2 = Dq<T>::stage2(x2, cols[set % kColSets][j], kOneForm ? part : part + 1);
         __builtin_amdgcn_sched_barrier(0);
         mfma(B, 2, rb);
-        wb[NB][j][part] = Dq<T>::stage3(y, cols[set][j]);
-        if (kPairs == 2) wb[NB][j][part + 1] = Dq<T>::stage3(y2, cols[set][j]);
+        wb[NB][j][part] = Dq<T>::stage3(y, cols[set % kColSets][j]);
+        if (kPairs == 2) wb[NB][j][part + 1] = Dq<T>::stage3(y2, cols[set % kColSets][j]);
         __builtin_amdgcn_sched_barrier(0);
         mfma(B, 3, rb);
       }
@@ -1455,12 +1477,13 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
   asm volatile("s_waitcnt vmcnt(%2)" : "+v"(wq[0][0]), "+v"(wq[0][1]) : "n"(2 * kWideOps) : "memory");
   if constexpr (W8 != 0) asm volatile("" : "+v"(wq[0][2]), "+v"(wq[0][3]) : : "memory");
   __builtin_amdgcn_s_barrier();
-  if (G32) {   // the constants of k block 1 of the first step; those of k block 0 below
+  auto second_block = [&]() __attribute__((always_inline)) {   // the constants of k block 1 of the first step
     scales_start(k_first, 1);
     asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(sb0), "+v"(sb1), "+v"(sb2), "+v"(sb3), "+v"(zw) : : "memory");
 #pragma unroll
     for (int j = 0; j < 4; ++j) make_col(1, j);
-  }
+  };
+  if (G32 && !TWIN) second_block();
   scales_start(k_first, 0);
   asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(sb0), "+v"(sb1), "+v"(sb2), "+v"(sb3), "+v"(zw) : : "memory");
 #pragma unroll
@@ -1480,6 +1503,7 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
     wb[0][j][2] = w.z;
     wb[0][j][3] = w.w;
   }
+  if (G32 && TWIN) second_block();
 #pragma unroll
   for (int rb = 0; rb < kAhead; ++rb) SONAR_WIDE_READ(av[rb], a_base[0], rb * 2048);
   __builtin_amdgcn_sched_barrier(0);
@@ -1509,7 +1533,7 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
 #pragma unroll
     for (int c = 0; c < 2 * kChunkLoads; ++c) asm volatile("" : "+v"(wq[i][c]) : : "memory");
 #pragma unroll
-  for (int i = 0; i < 8; ++i) asm volatile("" : "+v"(av[i]) : : "memory");
+  for (int i = 0; i < kAv; ++i) asm volatile("" : "+v"(av[i]) : : "memory");
   asm volatile("" : "+v"(sb0), "+v"(sb1), "+v"(sb2), "+v"(sb3), "+v"(zw) : : "memory");
   __builtin_amdgcn_sched_barrier(0);
 #undef SONAR_WIDE_LANDED
@@ -1526,7 +1550,7 @@ __device__ __forceinline__ void wide_tile(const TileParams& p, const int32_t* ta
       for (int r = 0; r < 4; ++r)
         sum_scale[nb][r] = grouped ? 1.f : Raw8<W8 == 2>::column_scale(row[scale_slot(16 * nb + 4 * kb + r, false)]);
   }
-  if (partial_at >= 0) {
+  if (!TWIN && partial_at >= 0) {
     // partial tile of this K range, in the order tile_reduce_kernel reads: 1-KiB blocks
     // (half of the rows, strip, column block, row block)
     float4* dst = partial + ((size_t)partial_at * kRows + wave * 32) * 64 + lane;
@@ -1682,6 +1706,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
                                                           t.k_tiles, t.partial_at);
 }
 
+// 128-row tiles alone, two workgroups a compute unit: while one starts or ends, the other multiplies.  A 256-row tile takes 11 to 13 us
+// around its loop (first bytes, results turned and stored, the gated activation), as long as 8 to 10 steps of K, with nothing
+// beside it; and the last round is finer.  Each wavefront has 256 registers, the 128 accumulators in AGPRs and at most 128 more: four
+// operands of A instead of eight, one set of column constants (a column block's are replaced behind its last use), 32-bit
+// offsets of A, a scale row read from one address (several groups only), and no partial tiles: K is never cut here.  The price is
+// that every weight is dequantised once for 128 rows: per matrix instruction 1.7 other vector instructions in float16, 1.2 for
+// MXFP4, 2.3 for integers in bfloat16.  Us, before -> now (bits equal): twin_pays and is_twin have the figures.
+template <typename T, bool HAS_ZP, bool GROUPED, bool FP4, bool G32>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void marlin_tile_twin_kernel(const TileParams p) {
+  int tile, tile_m, tile_n, split;
+  bool whole_k;
+  TileParams live = p;
+  if (GROUPED) live.tiles_m = p.tile_table[0], live.tile_band = 8;
+  if ((GROUPED && live.tiles_m <= 0) || !tile_of_workgroup(live, tile, split, whole_k)) return;
+  tile_coords(live, tile, tile_m, tile_n);
+  wide_tile<T, HAS_ZP, GROUPED, 8, FP4, 0, G32, false, true>(p, p.tile_table, nullptr, tile_m, tile_n, 0, p.size_k / kTileK, -1);
+}
+
 // Sums the partial tiles of the split tiles of a launch in split order, adds the
 // bias and writes C.  One wavefront per accumulator tile (16 rows x 16 columns).
 template <typename T>
@@ -1820,8 +1862,10 @@ __global__ __launch_bounds__(256) void moe_tile_reduce_kernel(const TileParams p
 // 1024 x 2688, AWQ, 6002 tokens 274 -> 269).
 struct TableJob {
   int32_t *table, *table_small;
-  int tiles_n, k_steps, may_split;
+  int tiles_n, k_steps, may_split;   // may_split: 0, 1 (two sizes: K may be cut), or
 };
+constexpr int kTwinTiles = 2;        // 128-row tiles alone, in `table`
+
 template <int kTableWaves>
 __global__ __launch_bounds__(64 * kTableWaves) void moe_tile_table_kernel(const int32_t* __restrict__ expert_ids,
                                                                       const int32_t* __restrict__ num_post_pad,
@@ -1834,6 +1878,7 @@ __global__ __launch_bounds__(64 * kTableWaves) void moe_tile_table_kernel(const 
   const int k_steps = blockIdx.x == 0 ? first.k_steps : second.k_steps;
   const int may_split = blockIdx.x == 0 ? first.may_split : second.may_split;
   constexpr int kTableThreads = 64 * kTableWaves;
+  const int most = may_split == kTwinTiles ? 2 : 4;   // blocks of a tile
   __shared__ int32_t last_start[kTableWaves], heads[2][kTableWaves];
   __shared__ unsigned long long best;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -1861,10 +1906,10 @@ __global__ __launch_bounds__(64 * kTableWaves) void moe_tile_table_kernel(const 
     }
     const unsigned long long upto = starts & (~0ull >> (63 - lane));
     if (upto) run = base + 64 * wave + 63 - __clzll(upto);
-    const bool head = b < blocks && e >= 0 && e < num_experts && ((b - run) & 3) == 0;
+    const bool head = b < blocks && e >= 0 && e < num_experts && ((b - run) & (most - 1)) == 0;
     int n = 1;
     if (head)
-      while (n < 4 && b + n < blocks && expert_ids[b + n] == e) ++n;
+      while (n < most && b + n < blocks && expert_ids[b + n] == e) ++n;
     const int small = table_small != nullptr && n <= 2;
     const unsigned long long mask[2] = {__ballot(head && !small), __ballot(head && small)};
     if (lane < 2) heads[lane][wave] = __popcll(mask[lane]);
@@ -2053,6 +2098,32 @@ int launch_pair_form(const TileParams& p, int max_row_tiles, hipStream_t st) {
   marlin_tile_wide_pair_kernel<T, HAS_ZP, GROUPED, FP4, W8, G32><<<pair_grid(p, max_row_tiles), 256, wide_lds(16), st>>>(p);
   return SONAR_OK;
 }
+template <typename T, bool HAS_ZP, bool GROUPED, bool FP4, bool G32>
+int launch_twin_form(const TileParams& p, hipStream_t st) {
+  static bool attr_set = false;
+  if (!attr_set) {
+    SONAR_HIP(hipFuncSetAttribute((const void*)marlin_tile_twin_kernel<T, HAS_ZP, GROUPED, FP4, G32>,
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, wide_lds(8)));
+    attr_set = true;
+  }
+  marlin_tile_twin_kernel<T, HAS_ZP, GROUPED, FP4, G32><<<tile_grid(p), 256, wide_lds(8), st>>>(p);
+  return SONAR_OK;
+}
+template <typename T, bool GROUPED>
+int launch_twin_type(const TileParams& p, bool fp4, hipStream_t st) {
+  if constexpr (std::is_same<T, __bf16>::value)
+    if (fp4) return launch_twin_form<T, false, GROUPED, true, true>(p, st);
+  if (fp4) return fail(SONAR_E_INVALID, "internal: MXFP4 weights with float16 activations");
+  if (wide_groups_of_32(p))
+    return p.zeros ? launch_twin_form<T, true, GROUPED, false, true>(p, st) : launch_twin_form<T, false, GROUPED, false, true>(p, st);
+  return p.zeros ? launch_twin_form<T, true, GROUPED, false, false>(p, st) : launch_twin_form<T, false, GROUPED, false, false>(p, st);
+}
+template <bool GROUPED>
+int launch_twin(const TileParams& p, int dtype, bool fp4, hipStream_t st) {
+  const int rc = dtype == SONAR_DTYPE_F16 ? launch_twin_type<_Float16, GROUPED>(p, fp4, st) : launch_twin_type<__bf16, GROUPED>(p, fp4, st);
+  return rc ? rc : launch_status("marlin_tile_twin_kernel");
+}
+
 template <typename T, bool GROUPED>
 int launch_pair_type(const TileParams& p, int max_row_tiles, bool fp4, int bits, bool fp8, hipStream_t st) {
   if constexpr (std::is_same<T, __bf16>::value)
@@ -2121,6 +2192,21 @@ bool wide_applies_fp4(const TileParams& p) {
 bool wide_applies8(const TileParams& p, bool fp8) { return fp8 || wide_applies(p); }
 }  // namespace
 
+// The 128-row tiles of marlin_tile_twin_kernel: 4-bit integers and MXFP4 with several groups.
+bool tile_twin_applies(int bits, bool nvfp4, int64_t num_groups, int group_size, int64_t a_row_stride) {
+  // debugging aids: the switch of these tiles, and those that single out an older path
+  static const bool off = [] {
+    for (const char* name : {"SONAR_MARLIN_NO_TWIN_TILES", "SONAR_MARLIN_NO_WIDE_TILE", "SONAR_MARLIN_NO_128_ROW_TILES",
+                             "SONAR_MARLIN_NO_TWO_TILE_SIZES", "SONAR_MARLIN_MAX_K_SPLITS", "SONAR_MARLIN_NO_ASYNC_TILE",
+                             "SONAR_MARLIN_NO_MOE_K_SPLIT"})
+      if (getenv(name) != nullptr) return true;
+    return false;
+  }();
+  if (off || bits != 4 || nvfp4 || num_groups <= 1 || !wide_rows_within_32_bits(a_row_stride)) return false;
+  const int per_group = group_size / kTileK;
+  return group_size == 32 || (group_size % kTileK == 0 && (per_group & (per_group - 1)) == 0);
+}
+
 // The asynchronous tile kernel needs groups of 32 rows or a multiple of 64 and no gather of A.
 bool tile_async_applies(bool has_perm, int64_t num_groups, int group_size) {
   return !has_perm && (num_groups == 1 || group_size % kTileK == 0 || group_size == 32);
@@ -2128,19 +2214,19 @@ bool tile_async_applies(bool has_perm, int64_t num_groups, int group_size) {
 
 namespace {
 // What tile_gemm launches for a call the asynchronous tile kernels take: one tile size (with
-// tile_reduce_kernel behind it when K is split), or both sizes of the wide kernel.
+// tile_reduce_kernel behind it when K is split), both sizes of the wide kernel, or 128-row tiles two at a time.
 struct TileLaunches {
-  bool ok, pair;
+  bool ok, pair, twin;
   TileParams launch;
 };
 
 // `p` arrives with the shape, the pointers and one 256-row launch over the whole of K filled in.
 TileLaunches plan_tile_launches(TileParams p, int64_t size_m, int64_t size_n, int64_t size_k, int64_t num_groups,
                                 int group_size, void* partial, size_t partial_bytes, bool fp4, bool nvfp4, int bits,
-                                bool has_perm) {
+                                bool has_perm, bool float16, bool may_twin = true) {
   TileLaunches out;
   out.ok = true;
-  out.pair = false;
+  out.pair = out.twin = false;
   const int steps_per_group = group_size / kTileK;
   const bool wide128 = bits == 4 && !fp4 && !has_perm &&
                        (num_groups == 1 || (group_size % kTileK == 0 && (steps_per_group & (steps_per_group - 1)) == 0));
@@ -2151,6 +2237,16 @@ TileLaunches plan_tile_launches(TileParams p, int64_t size_m, int64_t size_n, in
   // to hide behind: M = 512, K = 4096, N = 11008: NVFP4 69.9 us against 68.7, MXFP8 91.8 against 82.2)
   const bool rows128_ok = !nvfp4 && !(bits == 8 && num_groups > 1 && group_size == 32);
   GemmPlan plan = tile_plan(size_m, size_n, size_k, rows128_ok && !no_128, rows_97_128);
+  // two 128-row tiles at a time
+  if (may_twin && !has_perm && tile_twin_applies(bits, nvfp4, num_groups, group_size, p.lda) &&
+      twin_pays(size_m, size_n, size_k, float16, fp4, rows128_ok, rows_97_128)) {
+    p.tile_rows = 128;
+    p.tiles_m = (int)((size_m + 127) / 128);
+    p.tile_band = 8;   // the same rows of A per band as four 256-row tiles
+    out.twin = true;
+    out.launch = p;
+    return out;
+  }
   if (plan.tile_rows == 128) {
     TileParams probe = p;
     probe.tile_rows = 128;
@@ -2160,7 +2256,7 @@ TileLaunches plan_tile_launches(TileParams p, int64_t size_m, int64_t size_n, in
         (plan.k_splits == 1 || (partial != nullptr && partial_bytes >= plan_partial_bytes(plan, size_m, size_n)))) {
       p.tile_rows = 128;
       p.tiles_m = (int)((size_m + 127) / 128);
-      p.tile_band = 8;   // the same rows of A per band as four 256-row tiles
+      p.tile_band = 8;
     } else {
       plan = tile_plan(size_m, size_n, size_k, false, rows_97_128);
     }
@@ -2252,7 +2348,7 @@ int tile_gemm(const void* a, int64_t a_row_stride, void* c, const uint32_t* b, c
   if ((nvfp4 || tile_async_applies(pm, num_groups, group_size)) &&
       (!no_async || fp4 || bits == 8)) {   // float4 and 8-bit codes exist here only
     const TileLaunches plan = plan_tile_launches(p, size_m, size_n, size_k, num_groups, group_size, partial,
-                                                 partial_bytes, fp4, nvfp4, bits, pm);
+                                                 partial_bytes, fp4, nvfp4, bits, pm, dtype == SONAR_DTYPE_F16);
     if (!plan.ok)
       return fail(SONAR_E_INVALID, "internal: 128-row tiles exist in the wide tile kernel only");
     // the kernel a launch described by q takes
@@ -2270,6 +2366,7 @@ int tile_gemm(const void* a, int64_t a_row_stride, void* c, const uint32_t* b, c
       return zp ? launch_tile_wide<__bf16, true>(q, st) : launch_tile_wide<__bf16, false>(q, st);
     };
     p = plan.launch;
+    if (plan.twin) return launch_twin<false>(p, dtype, fp4, st);
     if (plan.pair) return launch_pair<false>(p, 0, dtype, fp4, bits, fp8, st);
     rc = launch(p);
     if (rc) return rc;
@@ -2386,11 +2483,29 @@ int moe_tile_gemm(const void* a, void* c, const uint32_t* b, const void* bias, c
   int32_t* table_small = two_sizes ? table + moe_one_table_bytes(sorted_len) / sizeof(int32_t) : nullptr;
   // tiles are cut along K only while they are few (and the second kernel is launched only where they may be): not when
   // the rows nearly fill the chip wherever they go, or, with a long K, fill it twice
-  auto few_tiles = [](const TileParams& q) {
+  auto may_cut = [](const TileParams& q) {
     return (int64_t)(q.rows_total + 255) / 256 * q.tiles_n <= (q.size_k >= 64 * kTileK ? 512 : 192);
   };
-  if (two_sizes) {
-    if (!few_tiles(p)) p.partial = nullptr;
+  // Two 128-row tiles at a time, which hide each other's start and end, instead: always up to 160 rows an expert, whose tiles have 128
+  // rows either way; with more, while the second dequantisation of the weights (integers in bf16 twice the instructions of float16 and
+  // MXFP4) costs less than that; not where K is long and the tiles fill half of the compute units, which K in ranges does.  Us a layer, two
+  // sizes -> here, over 325 random layers of 8 to 64 experts 0.91 times (0.74 to 1.04): 32 experts of 71 rows 2560 x 1152 225 -> 180; 16
+  // MXFP4 of 97, 2688 x 10880 404 -> 361; 16 of 632, 1280 x 2688 270 -> 233; 64 MXFP4 of 500, 2048 x 768 398 -> 342; 32 MXFP4 of 250,
+  // 2880 x 2880 457 -> 429.  Left out: Mixtral-8x7B shapes, bf16, 500 and 1024 rows 1267 -> 1360 and 2417 -> 2529; 16 of 453, bf16, AWQ,
+  // 3968 x 7040 1112 -> 1157; 8 of 200, fp16, 7168 x 7168 505 -> 518; 8 of 116, 2048 x 5888 137 -> 141.
+  auto is_twin = [&](const TileParams& q, bool may_split) {
+    if (!tile_twin_applies(bits, nvfp4, q.num_groups, q.group_size, q.size_k) || sorted_len * q.size_k * 2 >= (1LL << 32)) return false;
+    const int64_t tiles = (q.rows_total / 128 + num_experts / 2) * q.tiles_n;
+    if (may_split && tiles < 128 && q.size_k >= 2048) return false;
+    return q.rows_total <= 160 * num_experts || q.size_k <= (fp4 ? 8192 : dtype == SONAR_DTYPE_F16 ? 6144 : 3072);
+  };
+  if (two_sizes && !may_cut(p)) p.partial = nullptr;
+  const bool twin = two_sizes && is_twin(p, p.partial != nullptr);
+  if (twin) {
+    p.partial = nullptr;
+    p.tile_rows = 128;
+    table_small = nullptr;   // (one table, of tiles of up to two blocks)
+  } else if (two_sizes) {
     if (p.partial != nullptr)
       p.partial_small = reinterpret_cast<float4*>(static_cast<char*>(partial) + moe_partial_bytes_of(kTileM));
   }
@@ -2404,13 +2519,13 @@ int moe_tile_gemm(const void* a, void* c, const uint32_t* b, const void* bias, c
     p.gated_alpha = gated->alpha;
     gated->done = true;
   }
-  TableJob job = {table, table_small, p.tiles_n, (int)(size_k / kTileK), p.partial != nullptr}, next_job = {};
+  TableJob job = {table, table_small, p.tiles_n, (int)(size_k / kTileK), twin ? kTwinTiles : p.partial != nullptr}, next_job = {};
   sonar_moe_tables* ready = layer.ready;
   if (two_sizes && ready != nullptr && ready->built && ready->expert_ids == expert_ids && ready->sorted_len == sorted_len &&
       ready->tiles_n == job.tiles_n && ready->k_steps == job.k_steps && ready->may_split == job.may_split) {
     p.tile_table = table = ready->table;
     ready->built = 0;   // (the routing may change in place before another call)
-    table_small = table + moe_one_table_bytes(sorted_len) / sizeof(int32_t);
+    if (!twin) table_small = table + moe_one_table_bytes(sorted_len) / sizeof(int32_t);
   } else {
     // the layer's next GEMM, if it is one for both tile sizes as well, with the room for partial tiles it would be given
     sonar_moe_tables* next = layer.next;
@@ -2422,7 +2537,8 @@ int moe_tile_gemm(const void* a, void* c, const uint32_t* b, const void* bias, c
       q.tiles_n = (int)((next->size_n + kTileN - 1) / kTileN);
       if (has_two_sizes(q)) {
         next_job = {next->table, next->table + moe_one_table_bytes(sorted_len) / sizeof(int32_t), q.tiles_n, q.size_k / kTileK,
-                    !no_live_split && moe_tile_partial_bytes(q.size_k) > 0 && few_tiles(q)};
+                    !no_live_split && moe_tile_partial_bytes(q.size_k) > 0 && may_cut(q)};
+        if (is_twin(q, next_job.may_split)) next_job.table_small = nullptr, next_job.may_split = kTwinTiles;
         next->expert_ids = expert_ids, next->sorted_len = sorted_len;
         next->tiles_n = next_job.tiles_n, next->k_steps = next_job.k_steps, next->may_split = next_job.may_split;
         next->built = 1;
@@ -2444,6 +2560,7 @@ int moe_tile_gemm(const void* a, void* c, const uint32_t* b, const void* bias, c
     else moe_tile_reduce_kernel<__bf16><<<blocks, 256, 0, st>>>(q);
     return launch_status("moe_tile_reduce_kernel");
   };
+  if (twin) return launch_twin<true>(p, dtype, fp4, st);
   if (two_sizes) {
     p.table_small = table_small;
     if (int rc = launch_pair<true>(p, max_tiles, dtype, fp4, bits, fp8, st)) return rc;
@@ -2517,7 +2634,21 @@ extern "C" double sonar_debug_tile_estimate(int64_t size_m, int64_t size_n, int6
   return tile_estimate(size_m, size_n, size_k, kTileStepInt4, true, plan_rows_97_128(size_m, size_n, size_k, true));
 }
 
-// A dense call (4-bit integer codes, no act-order) with room for every partial tile.
+// A dense call that runs as 128-row tiles two at a time (`format`: 0 integers, 1 MXFP4); no rows: it runs otherwise.
+extern "C" int64_t sonar_debug_twin_schedule(int64_t size_m, int64_t size_n, int64_t size_k, int64_t num_groups, int dtype, int format,
+                                             int32_t* out, int64_t out_rows) {
+  using namespace sonar;
+  if (size_m <= 0 || size_n <= 0 || size_k <= 0 || size_k % kTileK != 0 || num_groups < 1 || size_k % num_groups != 0)
+    return -1;
+  const int group_size = (int)(size_k / num_groups);
+  static float4 never_read;
+  const TileLaunches plan = plan_tile_launches(dense_tile_shape(size_m, size_n, size_k, num_groups, group_size), size_m, size_n, size_k,
+                                               num_groups, group_size, &never_read, ~(size_t)0, format == 1, false, 4, false,
+                                               dtype == SONAR_DTYPE_F16);
+  return plan.twin ? schedule_rows(plan.launch, plan.launch, 0, out, out_rows, 0) : 0;
+}
+
+// A dense call (4-bit integer codes, no act-order) with room for every partial tile, as the other tile kernels run it.
 extern "C" int64_t sonar_debug_tile_schedule(int64_t size_m, int64_t size_n, int64_t size_k, int64_t num_groups,
                                              int32_t* out, int64_t out_rows) {
   using namespace sonar;
@@ -2527,7 +2658,7 @@ extern "C" int64_t sonar_debug_tile_schedule(int64_t size_m, int64_t size_n, int
   static float4 never_read;
   const TileLaunches plan =
       plan_tile_launches(dense_tile_shape(size_m, size_n, size_k, num_groups, group_size), size_m, size_n, size_k,
-                         num_groups, group_size, &never_read, ~(size_t)0, false, false, 4, false);
+                         num_groups, group_size, &never_read, ~(size_t)0, false, false, 4, false, true, false);
   if (!plan.pair) return schedule_rows(plan.launch, plan.launch, 0, out, out_rows, 0);
   return pair_schedule_rows(plan.launch, 0, 0, pair_grid(plan.launch, 0), out, out_rows);
 }

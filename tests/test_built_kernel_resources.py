@@ -14,7 +14,7 @@ LLVM = "/opt/rocm/llvm/bin"
 
 @pytest.mark.parametrize("kernel,at_least", [
     ("marlin_mid_gemm", 140), ("marlin_a8_block", 50), ("marlin_stream_fast_kernel", 80), ("marlin_tile_async_kernel", 10),
-    ("marlin_tile_wide_kernel", 30), ("marlin_tile_wide_pair_kernel", 20)])
+    ("marlin_tile_wide_kernel", 30), ("marlin_tile_wide_pair_kernel", 20), ("marlin_tile_twin_kernel", 18)])
 def test_hand_counted_kernels_do_not_spill(kernel, at_least, tmp_path):
     from sonar_amd import _lib
     _lib.load()

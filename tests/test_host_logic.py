@@ -241,7 +241,8 @@ def test_kernels_with_hand_counted_waits_do_not_spill():
     if not os.path.exists(hipcc):
         pytest.skip("hipcc not available")
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-    watched = {"gemm_tile.hip": ["marlin_tile_async_kernel", "marlin_tile_wide_kernel", "marlin_tile_wide_pair_kernel"],
+    watched = {"gemm_tile.hip": ["marlin_tile_async_kernel", "marlin_tile_wide_kernel", "marlin_tile_wide_pair_kernel",
+                                 "marlin_tile_twin_kernel"],
                "gemm_stream.hip": ["marlin_stream_fast_kernel"]}
     for src, kernels in watched.items():
         out = subprocess.run(
@@ -287,7 +288,7 @@ KERNEL_FORMS = {
     "marlin_dequant_kernel": 7, "marlin_fixup_kernel": 8, "marlin_moe8_kernel": 40, "marlin_moe_a8_kernel": 68,
     "marlin_moe_kernel": 52, "marlin_stream8_kernel": 40, "marlin_stream_fast_kernel": 86,
     "marlin_stream_kernel": 44, "marlin_tile_async_kernel": 13, "marlin_tile_kernel": 6,
-    "marlin_tile_wide_kernel": 38, "marlin_tile_wide_pair_kernel": 26, "marlin_to_gfx950_kernel": 1, "moe_activation_kernel": 12,
+    "marlin_tile_wide_kernel": 38, "marlin_tile_wide_pair_kernel": 26, "marlin_tile_twin_kernel": 18, "marlin_to_gfx950_kernel": 1, "moe_activation_kernel": 12,
     "moe_align_count_kernel": 2, "moe_align_place_kernel": 1, "moe_permute_rows_kernel": 1,
     "moe_sum_kernel": 2, "moe_tile_reduce_kernel": 2, "moe_tile_table_kernel": 2, "per_token_quant_kernel": 6,
     "permute_columns_kernel": 1, "silu_and_mul_kernel": 2, "tile_reduce_kernel": 2, "to_marlin_a8_kernel": 3,
