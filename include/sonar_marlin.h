@@ -457,6 +457,21 @@ int sonar_moe_wna16_marlin_gemm_gated(
     void* gated, int activation, float limit, float alpha, int* gated_written,
     sonar_moe_tables* next, sonar_moe_tables* ready, void* stream);
 
+/* The grouped GEMM of a layer of few slots straight from topk_ids int32[size_m * top_k], the expert of every row of C (those outside
+ * 0 .. num_experts - 1: their rows are not written), without the sorted slots and the launch that makes them; the bits are those of
+ * sonar_moe_wna16_marlin_gemm on what sonar_moe_align_block_size makes of the same ids.  Only where
+ * sonar_moe_routed_gemm_applies(size_m * top_k, ...) is 1 (at most 128 slots and 256 experts, blocks of 8, 16 or 32 slots, 4-bit integers
+ * and MXFP4, sizes that run in the decode kernel); other calls are refused.  gated (may be NULL) to gated_written as for
+ * sonar_moe_wna16_marlin_gemm_gated, the other arguments as for sonar_moe_wna16_marlin_gemm. */
+int sonar_moe_routed_gemm_applies(int64_t slots, int64_t moe_block_size, int64_t num_experts, int64_t b_type_id,
+                                  int64_t size_n, int64_t size_k, int64_t num_groups);
+int sonar_moe_routed_gemm(const void* a, void* c, const uint32_t* b_q_weight, int b_layout, const void* b_bias,
+                          const void* b_scales, const uint32_t* b_zeros, const int32_t* topk_ids,
+                          const float* topk_weights, int64_t moe_block_size, int64_t top_k, int mul_topk_weights,
+                          int64_t num_experts, int dtype, int64_t b_type_id, int64_t size_m, int64_t size_n,
+                          int64_t size_k, int64_t num_groups, void* gated, int activation, float limit, float alpha,
+                          int* gated_written, void* stream);
+
 /* The small kernels around the two grouped GEMMs of a mixture-of-experts layer.
  * They have counterparts in every build of the reference (also on ROCm):
  *   sonar_moe_align_block_size -> _moe_C::moe_align_block_size

@@ -101,6 +101,10 @@ PROTOTYPES = {
         c_size_t, c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int, c_int64, c_int, c_int64,
         c_int64, c_int64, c_int64, c_int64, c_int, c_void_p, c_int, c_float, c_float, c_void_p, c_void_p, c_void_p,
         c_void_p]),
+    "sonar_moe_routed_gemm_applies": (c_int, [c_int64] * 7),
+    "sonar_moe_routed_gemm": (c_int, [
+        c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int, c_int64, c_int,
+        c_int64, c_int64, c_int64, c_int64, c_int64, c_void_p, c_int, c_float, c_float, c_void_p, c_void_p]),
     "sonar_moe_align_block_size": (c_int, [c_void_p, c_int64, c_int64, c_int64, c_void_p, c_int64, c_void_p,
                                            c_int64, c_void_p, c_void_p, c_void_p, c_void_p]),
     "sonar_silu_and_mul": (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_int, c_void_p]),

@@ -40,7 +40,8 @@ int moe_fast_gemm(const void* a, void* c, const uint32_t* b, const void* bias, c
                   const uint32_t* zeros, const int32_t* sorted_ids, int64_t sorted_len, const int32_t* expert_ids,
                   const int32_t* num_post_pad, const float* topk_weights, int64_t moe_block_size, int64_t top_k,
                   int mul_topk, int64_t num_experts, int dtype, int64_t size_m, int64_t size_n, int64_t size_k,
-                  int64_t num_groups, int group_size, int a_by_slot, bool fp4, hipStream_t st);
+                  int64_t num_groups, int group_size, int a_by_slot, bool fp4, const int32_t* topk_ids, GatedOutput* gated, hipStream_t st);
+bool moe_fast_routes(int64_t slots, int64_t moe_block_size, int64_t num_experts);
 
 namespace {
 
@@ -685,7 +686,7 @@ int moe_gemm_any(
   }
   if (size_m == 0 || sorted_len == 0) return SONAR_OK;
   SONAR_REQUIRE(a && c && b_q_weight, "a, c and b_q_weight must not be NULL");
-  SONAR_REQUIRE(sorted_token_ids && expert_ids && num_tokens_past_padded,
+  SONAR_REQUIRE(layer.topk_ids || (sorted_token_ids && expert_ids && num_tokens_past_padded),
                 "sorted_token_ids, expert_ids and num_tokens_past_padded must not be NULL");
   SONAR_REQUIRE(!mul_topk_weights || topk_weights, "topk_weights must be given when mul_topk_weights is set");
   SONAR_REQUIRE(((uintptr_t)a) % 16 == 0 && ((uintptr_t)c) % 8 == 0 && ((uintptr_t)b_q_weight) % 16 == 0,
@@ -733,8 +734,10 @@ int moe_gemm_any(
   const bool tiles = moe_block_size == 64 && !has_perm && !row_groups && !no_tile && size_k % 64 == 0 &&
                      (num_groups == 1 || group_size % 64 == 0 || group_size == 32 || nvfp4) && scratch != nullptr &&
                      scratch_bytes >= moe_tile_table_bytes(sorted_len, num_experts) && ((uintptr_t)scratch) % 4 == 0;
+  if (layer.topk_ids != nullptr && !decode)
+    return fail(SONAR_E_INVALID, "internal: routing in a kernel that takes sorted slots");
   // (Its scales are 16-byte loads, as in the dense call; the other kernels copy them in pieces of 4.)
-  if (!bits8 && !row_groups && !nvfp4 && !has_perm && ((uintptr_t)b_scales) % 16 == 0 &&
+  if (layer.topk_ids == nullptr && !bits8 && !row_groups && !nvfp4 && !has_perm && ((uintptr_t)b_scales) % 16 == 0 &&
       moe_mid_applies(moe_block_size, size_m * top_k, num_experts, a_rows, size_n, size_k, num_groups, group_size, fp4,
                       decode, tiles)) {
     MidMoeParams m = {};
@@ -775,7 +778,7 @@ int moe_gemm_any(
     g_last_grouped_kernel = SONAR_GROUPED_DECODE;
     return moe_fast_gemm(a, c, b_q_weight, b_bias, b_scales, b_zeros, sorted_token_ids, sorted_len, expert_ids,
                          num_tokens_past_padded, topk_weights, moe_block_size, top_k, mul_topk_weights ? 1 : 0,
-                         num_experts, dtype, size_m, size_n, size_k, num_groups, group_size, a_by_slot, fp4, st);
+                         num_experts, dtype, size_m, size_n, size_k, num_groups, group_size, a_by_slot, fp4, layer.topk_ids, layer.gated, st);
   }
   // Full blocks of 64 slots mean many rows per expert: the MFMA-tiled kernel
   if (tiles) {
@@ -882,6 +885,49 @@ extern "C" int sonar_moe_wna16_marlin_gemm_nvfp4(
                       scratch_bytes, sorted_token_ids, sorted_len, expert_ids, num_tokens_past_padded, topk_weights,
                       moe_block_size, top_k, mul_topk_weights, num_experts, dtype, SONAR_TYPE_FLOAT4_E2M1F, size_m,
                       size_n, size_k, num_groups, 1, stream);
+}
+
+// Padded slots of `slots` on num_experts experts at most.
+static int64_t most_sorted(int64_t slots, int64_t moe_block_size, int64_t num_experts) {
+  const int64_t all = slots + num_experts * (moe_block_size - 1);
+  return slots < num_experts ? std::min(slots * moe_block_size, all) : all;
+}
+
+extern "C" int sonar_moe_routed_gemm_applies(int64_t slots, int64_t moe_block_size, int64_t num_experts, int64_t b_type_id,
+                                             int64_t size_n, int64_t size_k, int64_t num_groups) {
+  if (slots <= 0 || num_experts <= 0 || size_n <= 0 || size_n % kStripN != 0 || size_k <= 0 || num_groups <= 0) return 0;
+  if (moe_block_size != 8 && moe_block_size != 16 && moe_block_size != 32) return 0;
+  const bool fp4 = b_type_id == SONAR_TYPE_FLOAT4_E2M1F;
+  if (b_type_id != SONAR_TYPE_UINT4B8 && b_type_id != SONAR_TYPE_UINT4 && !(fp4 && size_k == 32 * num_groups)) return 0;
+  if (size_k % num_groups != 0) return 0;
+  const int group_size = (int)(size_k / num_groups);
+  return moe_fast_routes(slots, moe_block_size, num_experts) &&
+         moe_fast_applies(false, moe_block_size, most_sorted(slots, moe_block_size, num_experts), num_experts, slots, size_n, size_k,
+                          num_groups, group_size) &&
+         !moe_mid_applies(moe_block_size, slots, num_experts, slots, size_n, size_k, num_groups, group_size, fp4, true, false);
+}
+
+extern "C" int sonar_moe_routed_gemm(const void* a, void* c, const uint32_t* b_q_weight, int b_layout, const void* b_bias,
+                                     const void* b_scales, const uint32_t* b_zeros, const int32_t* topk_ids, const float* topk_weights,
+                                     int64_t moe_block_size, int64_t top_k, int mul_topk_weights, int64_t num_experts, int dtype,
+                                     int64_t b_type_id, int64_t size_m, int64_t size_n, int64_t size_k, int64_t num_groups, void* gated,
+                                     int activation, float limit, float alpha, int* gated_written, void* stream) {
+  SONAR_REQUIRE(gated == nullptr || gated_written != nullptr, "gated_written must not be NULL");
+  if (gated_written != nullptr) *gated_written = 0;
+  SONAR_REQUIRE(topk_ids != nullptr, "topk_ids must not be NULL");
+  SONAR_REQUIRE(size_m >= 0 && top_k >= 1 && num_experts >= 1 && size_m <= (1 << 20) && top_k <= (1 << 20), "sizes out of range");
+  if (size_m == 0) return SONAR_OK;
+  SONAR_REQUIRE(sonar_moe_routed_gemm_applies(size_m * top_k, moe_block_size, num_experts, b_type_id, size_n, size_k, num_groups),
+                "sonar_moe_routed_gemm_applies says no to these sizes");
+  GatedOutput out = {gated, activation, limit, alpha, false};
+  MoeLayerCall layer;
+  layer.topk_ids = topk_ids;
+  layer.gated = gated != nullptr ? &out : nullptr;
+  const int rc = moe_gemm_any(a, c, b_q_weight, b_layout, b_bias, b_scales, nullptr, b_zeros, nullptr, nullptr, nullptr, 0, nullptr,
+                      most_sorted(size_m * top_k, moe_block_size, num_experts), nullptr, nullptr, topk_weights, moe_block_size, top_k,
+                              mul_topk_weights, num_experts, dtype, b_type_id, size_m, size_n, size_k, num_groups, 1, stream, layer);
+  if (gated_written != nullptr) *gated_written = out.done ? 1 : 0;
+  return rc;
 }
 
 extern "C" int sonar_moe_wna16_marlin_gemm_gated(

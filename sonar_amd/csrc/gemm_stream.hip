@@ -25,6 +25,7 @@
 #include "dequant.hpp"
 #include "gemm_mid.hpp"
 #include "gemm_plan.hpp"
+#include "moe_activation.hpp"
 #include "wave_reduce.hpp"
 
 namespace sonar {
@@ -101,6 +102,13 @@ struct StreamParams {
   int a_by_slot;               // row of A = slot index (a column-permuted copy made per slot), else row id / top_k
   long expert_b_stride;        // uint4 units between experts in b
   long expert_s_stride, expert_z_stride, expert_bias_stride;  // elements between experts
+  // the expert of every row of C instead of sorted_ids, expert_ids and num_post_pad: every wavefront finds its block's rows itself
+  const int32_t* topk_ids;
+  // the gated activation of C, (rows_total, size_n / 2), in place of C.  `gated_halves`: silu_and_mul, a workgroup has
+  // strip `part` of the gate half (its first wavefronts) and the same strip of the up half; else swigluoai_and_mul of alternating columns
+  uint16_t* gated;
+  int gated_halves;
+  float gated_limit, gated_alpha;
 };
 
 // Unit indices are 32-bit: the host checks total_units * parts < 2^31.
@@ -290,14 +298,10 @@ __device__ __forceinline__ floatx4_t sum_partial_tiles(const StreamParams& p, in
 // weight is rounded to the activation type and the product is formed and
 // rounded in that type (marlin_moe_wna16/marlin_template.h:1883-1909).
 template <typename T>
-__device__ __forceinline__ void finish_block_grouped(const StreamParams& p, int id, int strip, int lane, int j,
-                                                     floatx4_t v) {
-  if (id < 0) return;
-  const int nl = 16 * j + 4 * (lane >> 4);
+__device__ __forceinline__ void round_block_grouped(const StreamParams& p, int id, int strip, int nl, floatx4_t v, uint16_t (&o)[4]) {
   const float r[4] = {v.x, v.y, v.z, v.w};
   float tw = 1.f;
   if (p.mul_topk) tw = Dq<T>::to_float(Dq<T>::from_float(p.topk_weights[id]));
-  uint16_t o[4];
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
     float x = r[t];
@@ -305,10 +309,40 @@ __device__ __forceinline__ void finish_block_grouped(const StreamParams& p, int 
     o[t] = Dq<T>::from_float(x);
     if (p.mul_topk) o[t] = Dq<T>::from_float(Dq<T>::to_float(o[t]) * tw);
   }
+}
+template <typename T>
+__device__ __forceinline__ void finish_block_grouped(const StreamParams& p, int id, int strip, int lane, int j,
+                                                     floatx4_t v) {
+  if (id < 0) return;
+  const int nl = 16 * j + 4 * (lane >> 4);
+  uint16_t o[4];
+  round_block_grouped<T>(p, id, strip, nl, v, o);
   uint2 packed;
   packed.x = (uint32_t)o[0] | ((uint32_t)o[1] << 16);
   packed.y = (uint32_t)o[2] | ((uint32_t)o[3] << 16);
   *reinterpret_cast<uint2*>(p.c + (long)id * p.size_n + strip * kStripN + nl) = packed;
+}
+// The same for a block of the gate and one of the up half, or of alternating columns (`up` is not read): every value is rounded
+// as the GEMM's result would be, and the gated activation formed of it (moe_activation.hpp).
+template <typename T>
+__device__ __forceinline__ void finish_block_gated(const StreamParams& p, int id, int strip, int lane, int j, floatx4_t gate,
+                                                   floatx4_t up) {
+  if (id < 0) return;
+  const int nl = 16 * j + 4 * (lane >> 4);
+  uint16_t g[4], u[4];
+  round_block_grouped<T>(p, id, strip, nl, gate, g);
+  uint16_t* to = p.gated + (long)id * (p.size_n / 2);
+  if (p.gated_halves) {
+    round_block_grouped<T>(p, id, strip + p.parts, nl, up, u);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) g[t] = silu_times<T>(g[t], u[t]);
+    *reinterpret_cast<uint2*>(to + strip * kStripN + nl) =
+        make_uint2((uint32_t)g[0] | ((uint32_t)g[1] << 16), (uint32_t)g[2] | ((uint32_t)g[3] << 16));
+  } else {
+    *reinterpret_cast<uint32_t*>(to + strip * (kStripN / 2) + nl / 2) =
+        (uint32_t)swiglu_oai<T>(g[0], g[1], p.gated_limit, p.gated_alpha) |
+        ((uint32_t)swiglu_oai<T>(g[2], g[3], p.gated_limit, p.gated_alpha) << 16);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -671,6 +705,63 @@ __device__ __forceinline__ int moe_row_id(const StreamParams& p, int block, int 
   return (id < 0 || id >= p.rows_total) ? -1 : id;
 }
 
+// The rows of block `block` of a call that has topk_ids (at most kRoutedSlots slots): the block's expert, or -1 where there is no such
+// block; lane r < 32 gets the row of C that is row r of the block, or -1.  A block is block_size rows of one expert in ascending
+// order, as moe_align_block_size makes them, but blocks are numbered by where their first row comes, so that nothing is added up
+// over the experts: with the ballots of the bits of the experts' numbers a lane knows the rows of its expert, its rank among
+// them, and whether a block begins with it.  A wavefront's own, without barriers; 60 vector instructions (150 with more than 64
+// slots) behind one load, where there were three.  (With a histogram in LDS and a scan over the experts 1 us longer a workgroup: 32
+// MXFP4 experts 1280 x 10112, 18 slots, 75 us a layer with sorted slots, 85 so.)
+constexpr int kRoutedSlots = 128, kRoutedExperts = 256;
+enum SlotsOfFastKernel { kSorted = 1, kRouted = 2 };   // what marlin_stream_fast_kernel's GROUPED takes: sorted slots, or topk_ids
+__device__ __forceinline__ int route_block(const StreamParams& p, int block, volatile int32_t* list, const int lane, int& row) {
+  typedef unsigned long long mask_t;
+  const mask_t below = (1ull << lane) - 1ull;
+  const bool two = p.rows_total > 64;
+  int id[2] = {-1, -1}, rank[2] = {0, 0};
+  if (lane < p.rows_total) id[0] = p.topk_ids[lane];
+  if (two && 64 + lane < p.rows_total) id[1] = p.topk_ids[64 + lane];
+  if (lane < 32) list[lane] = -1;
+#pragma unroll
+  for (int c = 0; c < 2; ++c)
+    if ((unsigned)id[c] >= (unsigned)p.num_experts) id[c] = -1;
+  mask_t there[2], bit[2][8];   // ballots of 64 slots each
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    there[c] = __builtin_amdgcn_ballot_w64(id[c] >= 0);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) bit[c][k] = __builtin_amdgcn_ballot_w64((id[c] >> k) & 1);
+  }
+  auto same = [&](int c, int expert) __attribute__((always_inline)) -> mask_t {   // the slots of ballots c with that expert
+    mask_t m = there[c];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) m &= ~(bit[c][k] ^ (mask_t)(long long)-((expert >> k) & 1));
+    return m;
+  };
+  rank[0] = (int)__popcll(same(0, id[0]) & below);
+  if (two) rank[1] = (int)(__popcll(same(0, id[1])) + __popcll(same(1, id[1]) & below));
+  int expert = -1, first = 0;   // `first`: the rank that the block begins with
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    const bool begins = id[c] >= 0 && (rank[c] & (p.block_size - 1)) == 0;   // (block_size is 8, 16 or 32)
+    const mask_t all = __builtin_amdgcn_ballot_w64(begins);
+    const mask_t here = __builtin_amdgcn_ballot_w64(begins && (int)__popcll(all & below) == block);
+    block -= (int)__popcll(all);
+    if (here != 0) {
+      const int at = (int)__builtin_ctzll(here);
+      expert = __builtin_amdgcn_readlane(id[c], at);
+      first = __builtin_amdgcn_readlane(rank[c], at);
+      break;
+    }
+  }
+  if (expert < 0) return -1;
+#pragma unroll
+  for (int c = 0; c < 2; ++c)
+    if (id[c] == expert && (unsigned)(rank[c] - first) < (unsigned)p.block_size) list[rank[c] - first] = 64 * c + lane;
+  row = list[lane & 31];
+  return expert;
+}
+
 template <int MB>
 struct FastLane {
   uint32_t a_off[2 * MB];  // byte offset of the 16 bytes this lane copies from rows 8h..8h+7 of a 64-column slice of A
@@ -781,7 +872,7 @@ __device__ __forceinline__ floatx4_t quad_transpose(floatx4_t x, int lane) {
 
 // MB blocks of 16 rows per workgroup (1 or 2): the weights of a unit are pulled
 // out of LDS and turned into operands once and multiplied with every block.
-// GROUPED: one workgroup per (block of slots, strip) of a mixture-of-experts
+// GROUPED (kSorted, kRouted): one workgroup per (block of slots, strip) of a mixture-of-experts
 // call; the rows of A are gathered and the rows of C scattered through
 // sorted_ids, everything else is the dense kernel on the expert's matrices.
 // GPU: groups per 128-row unit (2 or 4 for groups of 64 or 32 rows, else 1).  With two blocks of rows and four sets of
@@ -795,7 +886,7 @@ __device__ __forceinline__ floatx4_t quad_transpose(floatx4_t x, int lane) {
 // writes C (the piece is the whole strip) or leaves fp32 partial tiles and draws the
 // strip's ticket.  (A third weight slot per wavefront was measured slower than two on every
 // Llama-3-8B shape: M = 16, down 12.2 against 11.4 us, gate_up 19.1 against 17.4.)
-template <typename T, bool HAS_ZP, int kFastWaves, int MB, bool GROUPED = false, int GPU = 1, bool FP4 = false>
+template <typename T, bool HAS_ZP, int kFastWaves, int MB, int GROUPED = 0, int GPU = 1, bool FP4 = false>
 __global__ __launch_bounds__(kFastWaves * 64, 2) void marlin_stream_fast_kernel(const StreamParams params,
                                                                                 const int unit_group_shift) {
   typedef typename Dq<T>::vec8 vec8;
@@ -825,21 +916,31 @@ __global__ __launch_bounds__(kFastWaves * 64, 2) void marlin_stream_fast_kernel(
   }
   if (part >= p.parts) return;
   const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int routed_row = -1;  // with topk_ids: of row (lane & 31) of the block
   int row_id[MB] = {};  // grouped calls: the row of C that row (quad_lane & 15) of block of rows mb goes to, or -1
   if constexpr (GROUPED) {
     // `slab` names the block of slots and the 32 rows of it; the whole workgroup leaves together
     const int block = slab / p.sub_blocks;
     const int row0 = 32 * (slab - block * p.sub_blocks);
-    if (block * p.block_size >= p.num_post_pad[0]) return;
-    const long expert = p.expert_ids[block];
-    if (expert < 0 || expert >= p.num_experts) return;
+    long expert;
+    if constexpr (GROUPED == kRouted) {
+      expert = route_block(p, block, reinterpret_cast<int32_t*>(smem + wave * kWaveLds), lane, routed_row);
+      if (expert < 0) return;   // (the whole workgroup)
+    } else {
+      if (block * p.block_size >= p.num_post_pad[0]) return;
+      expert = p.expert_ids[block];
+      if (expert < 0 || expert >= p.num_experts) return;
+    }
     p.b += expert * p.expert_b_stride;
     p.scales += expert * p.expert_s_stride;
     if (HAS_ZP) p.zeros += expert * p.expert_z_stride;
     if (p.bias) p.bias += expert * p.expert_bias_stride;
     p.size_m = min(16 * MB, p.block_size - row0);
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) row_id[mb] = moe_row_id(p, block, row0 + 16 * mb + (quad_lane(lane) & 15));
+    for (int mb = 0; mb < MB; ++mb)
+      row_id[mb] = GROUPED == kRouted ? __shfl(routed_row, 16 * mb + (quad_lane(lane) & 15))
+                                         : moe_row_id(p, block, row0 + 16 * mb + (quad_lane(lane) & 15));
     // nothing but padding in these rows (the tail of an expert's last block): every
     // wavefront sees the same ids, so the workgroup leaves as one
     bool any_row = false;
@@ -851,7 +952,6 @@ __global__ __launch_bounds__(kFastWaves * 64, 2) void marlin_stream_fast_kernel(
     p.c += (long)slab * (16 * MB) * p.size_n;
     p.size_m = min(16 * MB, p.size_m - 16 * MB * slab);
   }
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col16 = lane & 15;
   const uint32_t ring_lds = (uint32_t)(uintptr_t)(lds_void_t*)smem + wave * kWaveLds;
   const uint32_t red_lds = (uint32_t)(uintptr_t)(lds_void_t*)smem;
@@ -865,8 +965,13 @@ __global__ __launch_bounds__(kFastWaves * 64, 2) void marlin_stream_fast_kernel(
     first_unit = __umulhi(at, p.piece_recip);
     end_unit = __umulhi(at + p.units_per_strip, p.piece_recip);
   }
-  int unit = first_unit + wave;
-  const int mine = unit < end_unit ? (end_unit - unit + kFastWaves - 1) / kFastWaves : 0;
+  // (gate and up halves: the first half of the wavefronts has a strip of the gate, the other the same strip of the up half)
+  const bool halves = GROUPED != 0 && p.gated != nullptr && p.gated_halves;
+  const int stride = GROUPED != 0 && halves ? kFastWaves / 2 : kFastWaves;   // between a wavefront's units
+  if (halves && wave >= kFastWaves / 2) strip += p.parts;
+  int unit = first_unit + (halves ? wave & (kFastWaves / 2 - 1) : wave);
+  const int mine = unit >= end_unit ? 0 : halves ? (end_unit - unit + kFastWaves / 2 - 1) / (kFastWaves / 2)
+                                                 : (end_unit - unit + kFastWaves - 1) / kFastWaves;
   const bool grouped = p.num_groups > 1;
 
   FastLane<MB> fl;
@@ -877,7 +982,7 @@ __global__ __launch_bounds__(kFastWaves * 64, 2) void marlin_stream_fast_kernel(
       int row = r < p.size_m ? r : p.size_m - 1;  // rows past M are never stored
       if constexpr (GROUPED) {                    // padding slots read row 0 and are never stored
         const int in_block = 32 * (slab % p.sub_blocks) + r;
-        const int id = moe_row_id(p, slab / p.sub_blocks, in_block);
+        const int id = GROUPED == kRouted ? __shfl(routed_row, r) : moe_row_id(p, slab / p.sub_blocks, in_block);
         row = id >= 0 ? (p.a_by_slot ? (slab / p.sub_blocks) * p.block_size + in_block : id / p.top_k) : 0;
       }
       fl.a_off[h] = (uint32_t)((long)row * p.lda * 2 + 16 * ((lane & 7) ^ (lane >> 3)));
@@ -921,7 +1026,7 @@ __global__ __launch_bounds__(kFastWaves * 64, 2) void marlin_stream_fast_kernel(
     copy_weights<HAS_ZP, MB, GPU>(p, fl, strip, unit, ring_lds, lane, unit_group_shift);
     copy_activations<MB>(p, fl, unit, ring_lds + kWaveA);
   }
-  if (mine > 1) copy_weights<HAS_ZP, MB, GPU>(p, fl, strip, unit + kFastWaves, ring_lds + kSlotBytes, lane, unit_group_shift);
+  if (mine > 1) copy_weights<HAS_ZP, MB, GPU>(p, fl, strip, unit + stride, ring_lds + kSlotBytes, lane, unit_group_shift);
 
   floatx4_t acc[MB][4];
 #pragma unroll
@@ -976,7 +1081,7 @@ __global__ __launch_bounds__(kFastWaves * 64, 2) void marlin_stream_fast_kernel(
     for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
       for (int cc = 0; cc < 4; ++cc) asm volatile("" : "+v"(a[mb][cc]));
-    if (left > 1) copy_activations<MB>(p, fl, unit + kFastWaves, ring_lds + kWaveA);
+    if (left > 1) copy_activations<MB>(p, fl, unit + stride, ring_lds + kWaveA);
     constexpr int kChunksPerGroup = 4 / GPU;
     const floatx4_t zero4 = floatx4_t{0.f, 0.f, 0.f, 0.f};
     floatx4_t a_sum[GPU][MB];
@@ -1016,8 +1121,8 @@ __global__ __launch_bounds__(kFastWaves * 64, 2) void marlin_stream_fast_kernel(
       if constexpr (HAS_ZP) asm volatile("" : "+v"(zbits[gi]));
     }
     if (left > 2)
-      copy_weights<HAS_ZP, MB, GPU>(p, fl, strip, unit + 2 * kFastWaves, ring_lds + slot * kSlotBytes, lane, unit_group_shift);
-    unit += kFastWaves;
+      copy_weights<HAS_ZP, MB, GPU>(p, fl, strip, unit + 2 * stride, ring_lds + slot * kSlotBytes, lane, unit_group_shift);
+    unit += stride;
     floatx4_t sum[MB][4];
 #pragma unroll
     for (int gi = 0; gi < GPU; ++gi) {
@@ -1094,7 +1199,7 @@ __global__ __launch_bounds__(kFastWaves * 64, 2) void marlin_stream_fast_kernel(
     }
     __builtin_amdgcn_s_barrier();
     if (wave < kPark) {
-      floatx4_t sum = floatx4_t{0.f, 0.f, 0.f, 0.f};
+      floatx4_t sum = floatx4_t{0.f, 0.f, 0.f, 0.f}, gate = sum;   // `gate`: with halves, the sum of the first half of the wavefronts
       const uint32_t src = red_lds + (wave * 64 + lane) * 16;
 #pragma unroll
       for (int w = 0; w < kFastWaves; w += 4) {
@@ -1108,14 +1213,19 @@ __global__ __launch_bounds__(kFastWaves * 64, 2) void marlin_stream_fast_kernel(
             : "=&v"(t0), "=&v"(t1), "=&v"(t2), "=&v"(t3)
             : "v"(src + w * kPark * 1024), "n"(kPark * 1024), "n"(2 * kPark * 1024), "n"(3 * kPark * 1024)
             : "memory");
+        if (GROUPED != 0 && w > 0 && halves) gate = sum, sum = floatx4_t{0.f, 0.f, 0.f, 0.f};
         sum += t0;
         sum += t1;
+        if (GROUPED != 0 && kFastWaves == 4 && halves) gate = sum, sum = floatx4_t{0.f, 0.f, 0.f, 0.f};
         sum += t2;
         sum += t3;
       }
       const int j = jb + wave, at = quad_lane(lane);
       sum = quad_transpose(sum, lane);
-      if constexpr (GROUPED) {
+      if (GROUPED != 0 && p.gated != nullptr) {
+        gate = halves ? quad_transpose(gate, lane) : sum;
+        finish_block_gated<T>(p, row_id[mb], part, at, j, gate, sum);
+      } else if constexpr (GROUPED) {
         finish_block_grouped<T>(p, row_id[mb], strip, at, j, sum);
       } else if (pieces == 1) {
         store_c_block<T>(p, p.c + (long)(16 * mb) * p.size_n, p.size_m - 16 * mb, strip, at, j, sum);
@@ -1396,7 +1506,7 @@ void launch_stream8_mb(const StreamParams& p, bool fp8, hipStream_t st) {
   else launch_stream8_gidx<T, false, false>(p, st);
 }
 
-template <typename T, bool HAS_ZP, int WAVES, int MB, bool GROUPED, int GPU, bool FP4 = false>
+template <typename T, bool HAS_ZP, int WAVES, int MB, int GROUPED, int GPU, bool FP4 = false>
 int launch_fast_groups(const StreamParams& p, int unit_group_shift, hipStream_t st) {
   static bool attr_set = false;  // raising the dynamic LDS limit is needed once per kernel
   if (!attr_set) {
@@ -1411,7 +1521,7 @@ int launch_fast_groups(const StreamParams& p, int unit_group_shift, hipStream_t 
 }
 
 // unit_group_shift -2 / -4: two / four groups per 128-row unit (groups of 64 / 32 rows)
-template <typename T, bool HAS_ZP, int WAVES, int MB, bool GROUPED>
+template <typename T, bool HAS_ZP, int WAVES, int MB, int GROUPED>
 int launch_fast_waves(const StreamParams& p, int unit_group_shift, hipStream_t st) {
   if (unit_group_shift <= -2) {
     if constexpr (MB == 1 || GROUPED) {
@@ -1425,14 +1535,14 @@ int launch_fast_waves(const StreamParams& p, int unit_group_shift, hipStream_t s
 }
 
 // MXFP4: bf16, four groups of 32 rows per unit; two blocks of 16 rows in grouped calls only
-template <bool GROUPED, int MB = 1>
+template <int GROUPED, int MB = 1>
 int launch_fast_fp4(const StreamParams& p, bool half_workgroups, hipStream_t st) {
   return half_workgroups ? launch_fast_groups<__bf16, false, 4, MB, GROUPED, 4, true>(p, -4, st)
                          : launch_fast_groups<__bf16, false, 8, MB, GROUPED, 4, true>(p, -4, st);
 }
 
 // `row_blocks`: blocks of 16 rows per workgroup (1 or 2).
-template <typename T, bool HAS_ZP, bool GROUPED = false>
+template <typename T, bool HAS_ZP, int GROUPED = 0>
 int launch_fast(const StreamParams& p, int unit_group_shift, bool half_workgroups, int row_blocks, hipStream_t st) {
   if (row_blocks == 2)
     return half_workgroups ? launch_fast_waves<T, HAS_ZP, 4, 2, GROUPED>(p, unit_group_shift, st)
@@ -1598,6 +1708,12 @@ bool moe_fast_applies(bool has_perm, int64_t moe_block_size, int64_t sorted_len,
   return sorted_len <= (shift == -4 ? 900 : 1000);
 }
 
+// Whether a call that moe_fast_applies to can find its rows itself.  (Blocks of at most 32 slots: a workgroup each.)
+bool moe_fast_routes(int64_t slots, int64_t moe_block_size, int64_t num_experts) {
+  static const bool off = getenv("SONAR_MARLIN_NO_MOE_ROUTED") != nullptr;  // debugging aid
+  return !off && slots <= kRoutedSlots && num_experts <= kRoutedExperts && moe_block_size <= 32;
+}
+
 // Called by sonar_moe_wna16_marlin_gemm when moe_fast_applies: one workgroup
 // per (block of slots, strip), nothing reduced through memory.  Arguments have
 // been validated by the caller.
@@ -1605,8 +1721,9 @@ int moe_fast_gemm(const void* a, void* c, const uint32_t* b, const void* bias, c
                   const uint32_t* zeros, const int32_t* sorted_ids, int64_t sorted_len, const int32_t* expert_ids,
                   const int32_t* num_post_pad, const float* topk_weights, int64_t moe_block_size, int64_t top_k,
                   int mul_topk, int64_t num_experts, int dtype, int64_t size_m, int64_t size_n, int64_t size_k,
-                  int64_t num_groups, int group_size, int a_by_slot, bool fp4, hipStream_t st) {
+                  int64_t num_groups, int group_size, int a_by_slot, bool fp4, const int32_t* topk_ids, GatedOutput* gated, hipStream_t st) {
   StreamParams p = {};
+  p.topk_ids = topk_ids;
   p.a_by_slot = a_by_slot;
   p.a = static_cast<const uint16_t*>(a);
   p.lda = size_k;
@@ -1623,7 +1740,21 @@ int moe_fast_gemm(const void* a, void* c, const uint32_t* b, const void* bias, c
   p.chunks_per_strip = (int)(size_k / kChunkK);
   p.unit_chunks = 4;
   p.units_per_strip = p.chunks_per_strip / 4;
-  const int n_strips = (int)(size_n / kStripN);
+  // The gated activation where the rows end: a launch of 3 to 5 us less, and half as many workgroups twice as long.  Not where more
+  // than kRoutedSlots slots make fewer of those than there are compute units.  Us a layer, a launch of its own -> here: 32
+  // experts 1152 x 11136, 704 slots 245 -> 205; 64 MXFP4 of 1024 x 2688, 448 slots 114 -> 97; 16 of 1280 x 2432, 920 slots 81 -> 71; left out: 8 of
+  // 1408 x 896, 186 slots 27.2 -> 29.0; 16 of 2816 x 768, 344 slots 40.1 -> 40.7.
+  const int64_t slots = size_m * top_k, sub_blocks = moe_block_size > 32 ? 2 : 1;
+  const int64_t workgroups = std::max(std::min(num_experts, slots), slots / moe_block_size) * sub_blocks * (size_n / (2 * kStripN));
+  if (gated != nullptr && (topk_ids != nullptr || gated->kind != 0 || workgroups >= cu_count()) && ((uintptr_t)gated->out) % 8 == 0 &&
+      (gated->kind == 0 ? size_n % (2 * kStripN) == 0 : gated->kind == SONAR_ACT_SWIGLUOAI && gated->limit > 0.f)) {
+    p.gated = static_cast<uint16_t*>(gated->out);
+    p.gated_halves = gated->kind == 0;
+    p.gated_limit = gated->limit;
+    p.gated_alpha = gated->alpha;
+    gated->done = true;
+  }
+  const int all_strips = (int)(size_n / kStripN), n_strips = p.gated_halves ? all_strips / 2 : all_strips;   // (halves: pairs of strips)
   p.parts = n_strips;                       // part i is strip i
   p.total_units = n_strips * p.units_per_strip;
   p.sub_blocks = moe_block_size > 32 ? 2 : 1;
@@ -1641,7 +1772,7 @@ int moe_fast_gemm(const void* a, void* c, const uint32_t* b, const void* bias, c
   p.rows_total = (int)(size_m * top_k);
   p.sorted_len = (int)sorted_len;
   p.mul_topk = mul_topk;
-  p.expert_b_stride = (long)n_strips * p.chunks_per_strip * 64;
+  p.expert_b_stride = (long)all_strips * p.chunks_per_strip * 64;
   p.expert_s_stride = (long)num_groups * size_n;
   p.expert_z_stride = (long)num_groups * (size_n / 8);
   p.expert_bias_stride = size_n;
@@ -1662,16 +1793,18 @@ int moe_fast_gemm(const void* a, void* c, const uint32_t* b, const void* bias, c
   // and the caches are all that keeps those reads from memory)
   p.nt_weights = !no_nt && p.sub_blocks == 1 && p.slabs <= 2 * num_experts &&
                  num_experts * size_k * size_n / 2 >= 10 * 1000 * 1000;
-  int rc;
-  if (fp4)   // bf16, groups of 32 rows
-    rc = row_blocks == 2 ? launch_fast_fp4<true, 2>(p, half, st) : launch_fast_fp4<true>(p, half, st);
-  else if (dtype == SONAR_DTYPE_F16)
-    rc = zeros ? launch_fast<_Float16, true, true>(p, unit_group_shift, half, row_blocks, st)
-               : launch_fast<_Float16, false, true>(p, unit_group_shift, half, row_blocks, st);
-  else
-    rc = zeros ? launch_fast<__bf16, true, true>(p, unit_group_shift, half, row_blocks, st)
-               : launch_fast<__bf16, false, true>(p, unit_group_shift, half, row_blocks, st);
-  if (rc) return rc;
+  auto launch = [&](auto slots) -> int {
+    constexpr int kSlots = decltype(slots)::value;
+    if (fp4)   // bf16, groups of 32 rows
+      return row_blocks == 2 ? launch_fast_fp4<kSlots, 2>(p, half, st) : launch_fast_fp4<kSlots>(p, half, st);
+    if (dtype == SONAR_DTYPE_F16)
+      return zeros ? launch_fast<_Float16, true, kSlots>(p, unit_group_shift, half, row_blocks, st)
+                   : launch_fast<_Float16, false, kSlots>(p, unit_group_shift, half, row_blocks, st);
+    return zeros ? launch_fast<__bf16, true, kSlots>(p, unit_group_shift, half, row_blocks, st)
+                 : launch_fast<__bf16, false, kSlots>(p, unit_group_shift, half, row_blocks, st);
+  };
+  if (int rc = topk_ids != nullptr ? launch(std::integral_constant<int, kRouted>()) : launch(std::integral_constant<int, kSorted>()))
+    return rc;
   return launch_status("marlin_stream_fast_kernel (grouped)");
 }
 
@@ -2026,7 +2159,7 @@ int marlin_gemm_any(const void* a, int64_t a_row_stride, void* c, const uint32_t
     g_last_decode_launch[3] = p.nt_weights;
     int rc;
     if (chk.fp4)   // groups of 32 rows: never in blocks of rows (slab_fast is off), so one block of 16 rows
-      rc = launch_fast_fp4<false>(p, half, st);
+      rc = launch_fast_fp4<0>(p, half, st);
     else if (dtype == SONAR_DTYPE_F16)
       rc = chk.has_zp ? launch_fast<_Float16, true>(p, unit_group_shift, half, row_blocks, st)
                       : launch_fast<_Float16, false>(p, unit_group_shift, half, row_blocks, st);

@@ -62,6 +62,7 @@ struct MoeLayerCall {
   GatedOutput* gated = nullptr;
   sonar_moe_tables* next = nullptr;          // build the row tiles of that GEMM in this call's launch
   sonar_moe_tables* ready = nullptr;         // this GEMM's, if an earlier call has built them
+  const int32_t* topk_ids = nullptr;         // the expert of every row of C, in place of the sorted slots
 };
 
 }  // namespace sonar

@@ -1012,6 +1012,7 @@ struct Routing {
   const int32_t* expert_ids;
   const int32_t* past_padded;
   const float* topk_weights;
+  const int32_t* topk_ids = nullptr;   // in place of the sorted slots (sonar_moe_routed_gemm)
 };
 
 // What sonar_moe_wna16_marlin_gemm_gated takes beyond the GEMM: a gated activation that it may write to `out` in place of its
@@ -1120,6 +1121,15 @@ void moe_gemm_16bit(const Tensor& a, void* c, const Tensor& b_q_weight, const Op
   if (size_m == 0) return;
 
   Tensor native = native_weights(b_q_weight, size_k, size_n, experts, bits);
+  if (route.topk_ids != nullptr) {
+    const Tensor scales = fp4 ? mx_scales_as_bf16(b_scales, 0) : b_scales;
+    raise_if_failed(sonar_moe_routed_gemm(
+        a.const_data_ptr(), c, static_cast<const uint32_t*>(native.const_data_ptr()), SONAR_LAYOUT_GFX950, opt_ptr(b_bias_or_none),
+        scales.const_data_ptr(), has_zp ? static_cast<const uint32_t*>(b_zeros_or_none->const_data_ptr()) : nullptr, route.topk_ids,
+        route.topk_weights, moe_block_size, top_k, mul_topk_weights ? 1 : 0, experts, dtype, b_type_id, size_m, size_n, size_k,
+        num_groups, layer->out, layer->activation, layer->limit, layer->alpha, &layer->written, current_stream(a)));
+    return;
+  }
   size_t scratch_bytes =
       sonar_moe_marlin_gemm_scratch_bytes(route.sorted_len, moe_block_size, size_n, size_k);
   // act-order: room for the column-permuted copy of A, one row per slot, behind the table of row tiles
@@ -1340,6 +1350,46 @@ void fused_moe(Tensor& output, const Tensor& hidden, const Tensor& w1, const Ten
   Tensor between = cache2.has_value() ? cache(cache2, rows * n, "intermediate_cache2") : at::empty({rows, n}, hidden.options());
   Tensor wide = cache(cache13, rows * std::max(2 * n, k), "intermediate_cache13");   // gate and up, then the rows of the down GEMM
 
+  const int dtype = dtype_code(hidden);
+  void* stream = current_stream(hidden);
+  auto gate_up_activation = [&]() {
+    raise_if_failed(activation == 0
+                        ? sonar_silu_and_mul(between.mutable_data_ptr(), wide.const_data_ptr(), rows, n, dtype, stream)
+                        : sonar_moe_activation(between.mutable_data_ptr(), wide.const_data_ptr(), rows, n,
+                                               (int)activation, (float)limit, (float)alpha, (float)beta, dtype, stream));
+  };
+  auto down_input = [&]() {
+    return between.dim() == 2 && between.size(0) == rows && between.size(1) == n
+               ? between
+               : between.view({-1}).narrow(0, 0, rows * n).view({rows, n});
+  };
+  // The GEMM may form the activation itself; not where its input would be overwritten meanwhile.
+  auto range = [](const Tensor& t, int64_t values) {
+    const auto at = reinterpret_cast<uintptr_t>(t.const_data_ptr());
+    return std::make_pair(at, at + (uintptr_t)values * 2);
+  };
+  const auto in = range(hidden, m * k), mid = range(between, rows * n);
+  InLayer gate_up, down;
+  if (!(in.first < mid.second && mid.first < in.second)) gate_up.out = between.mutable_data_ptr();
+  gate_up.activation = (int)activation, gate_up.limit = (float)limit, gate_up.alpha = (float)alpha;
+  // Few slots: the GEMMs find their rows in topk_ids themselves, and the launch that sorts them goes (25 -> 19 us for the smallest layers)
+  auto routes = [&](const Tensor& w, const Tensor& scale, const OptTensor& perm, int64_t size_n, int64_t size_k) {
+    return !(perm.has_value() && perm->numel() > 0) && w.dim() == 3 && scale.dim() == 3 &&
+           !(b_type_id == SONAR_TYPE_FLOAT4_E2M1F && !is_mx_scale_type(scale)) &&
+           sonar_moe_routed_gemm_applies(rows, block_size, w.size(0), b_type_id, size_n, size_k, scale.size(1));
+  };
+  if (m > 0 && routes(w1, scale1, perm1, 2 * n, k) && routes(w2, scale2, perm2, k, n)) {
+    Routing route{nullptr, 0, nullptr, nullptr, static_cast<const float*>(topk_weights.const_data_ptr()),
+                  static_cast<const int32_t*>(topk_ids.const_data_ptr())};
+    moe_gemm_16bit(hidden, wide.mutable_data_ptr(), w1, bias1, scale1, std::nullopt, global_scale1, zeros1, g_idx1, perm1,
+                   route, block_size, topk, router_weight_on_input, b_type_id, m, 2 * n, k, is_k_full, false, true, false, &gate_up);
+    if (!gate_up.written) gate_up_activation();
+    moe_gemm_16bit(down_input(), wide.mutable_data_ptr(), w2, bias2, scale2, std::nullopt, global_scale2, zeros2, g_idx2, perm2,
+                   route, block_size, 1, !router_weight_on_input, b_type_id, rows, k, n, is_k_full, false, true, false, &down);
+    raise_if_failed(sonar_moe_sum(output.mutable_data_ptr(), wide.const_data_ptr(), m, topk, k, dtype, stream));
+    return;
+  }
+
   // sorted ids | expert of each block | padded total | scratch of the routing kernel, 16-byte pieces
   int64_t sorted_len = rows + num_experts * (block_size - 1);
   if (rows < num_experts) sorted_len = std::min(rows * block_size, sorted_len);
@@ -1350,39 +1400,21 @@ void fused_moe(Tensor& output, const Tensor& hidden, const Tensor& w1, const Ten
   int32_t* sorted_ids = static_cast<int32_t*>(table.mutable_data_ptr());
   int32_t* expert_ids = sorted_ids + room(sorted_len);
   int32_t* past_padded = expert_ids + room(blocks);
-  void* stream = current_stream(hidden);
   raise_if_failed(sonar_moe_align_block_size(static_cast<const int32_t*>(topk_ids.const_data_ptr()), rows, num_experts,
                                              block_size, sorted_ids, sorted_len, expert_ids, blocks, past_padded,
                                              nullptr, past_padded + 4, stream));
   const Routing route{sorted_ids, sorted_len, expert_ids, past_padded,
                       static_cast<const float*>(topk_weights.const_data_ptr())};
-  const int dtype = dtype_code(hidden);
-  // The GEMM may form the activation itself; not where its input would be overwritten meanwhile.
-  auto range = [](const Tensor& t, int64_t values) {
-    const auto at = reinterpret_cast<uintptr_t>(t.const_data_ptr());
-    return std::make_pair(at, at + (uintptr_t)values * 2);
-  };
-  const auto in = range(hidden, m * k), mid = range(between, rows * n);
   sonar_moe_tables tables = {};
   tables.table = past_padded + 4 + room(num_experts);
   tables.table_bytes = tiles_bytes;
   tables.size_n = k, tables.size_k = n, tables.num_groups = scale2.dim() == 3 ? scale2.size(1) : 0;
-  InLayer gate_up, down;
-  if (!(in.first < mid.second && mid.first < in.second)) gate_up.out = between.mutable_data_ptr();
-  gate_up.activation = (int)activation, gate_up.limit = (float)limit, gate_up.alpha = (float)alpha;
   if (tiles_bytes > 0 && k > 0 && n > 0) gate_up.next = &tables, down.ready = &tables;
   moe_gemm_16bit(hidden, wide.mutable_data_ptr(), w1, bias1, scale1, std::nullopt, global_scale1, zeros1, g_idx1, perm1,
                  route, block_size, topk, router_weight_on_input, b_type_id, m, 2 * n, k, is_k_full, false, true,
                  false, &gate_up);
-  if (!gate_up.written)
-    raise_if_failed(activation == 0
-                        ? sonar_silu_and_mul(between.mutable_data_ptr(), wide.const_data_ptr(), rows, n, dtype, stream)
-                        : sonar_moe_activation(between.mutable_data_ptr(), wide.const_data_ptr(), rows, n,
-                                               (int)activation, (float)limit, (float)alpha, (float)beta, dtype, stream));
-  const Tensor down_in = between.dim() == 2 && between.size(0) == rows && between.size(1) == n
-                             ? between
-                             : between.view({-1}).narrow(0, 0, rows * n).view({rows, n});
-  moe_gemm_16bit(down_in, wide.mutable_data_ptr(), w2, bias2, scale2, std::nullopt, global_scale2, zeros2, g_idx2, perm2,
+  if (!gate_up.written) gate_up_activation();
+  moe_gemm_16bit(down_input(), wide.mutable_data_ptr(), w2, bias2, scale2, std::nullopt, global_scale2, zeros2, g_idx2, perm2,
                  route, block_size, 1, !router_weight_on_input, b_type_id, rows, k, n, is_k_full, false, true, false, &down);
   raise_if_failed(sonar_moe_sum(output.mutable_data_ptr(), wide.const_data_ptr(), m, topk, k, dtype, stream));
 }

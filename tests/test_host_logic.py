@@ -286,7 +286,7 @@ KERNEL_FORMS = {
     "marlin8_gfx950_kernel": 2, "marlin_a8_finish_kernel": 9, "marlin_a8_kernel": 68,
     "marlin_a8_tile_kernel": 48, "marlin_a8_to_gfx950_kernel": 1, "marlin_dequant8_kernel": 4,
     "marlin_dequant_kernel": 7, "marlin_fixup_kernel": 8, "marlin_moe8_kernel": 40, "marlin_moe_a8_kernel": 68,
-    "marlin_moe_kernel": 52, "marlin_stream8_kernel": 40, "marlin_stream_fast_kernel": 86,
+    "marlin_moe_kernel": 52, "marlin_stream8_kernel": 40, "marlin_stream_fast_kernel": 138,
     "marlin_stream_kernel": 44, "marlin_tile_async_kernel": 13, "marlin_tile_kernel": 6,
     "marlin_tile_wide_kernel": 38, "marlin_tile_wide_pair_kernel": 26, "marlin_tile_twin_kernel": 18, "marlin_to_gfx950_kernel": 1, "moe_activation_kernel": 12,
     "moe_align_count_kernel": 2, "moe_align_place_kernel": 1, "moe_permute_rows_kernel": 1,
