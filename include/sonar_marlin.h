@@ -143,6 +143,13 @@ int sonar_load_gptq_linear(const uint32_t* codes, uint32_t* codes_out, const voi
                            const uint32_t* zeros, uint32_t* zeros_out, uint32_t* workspace,
                            int64_t workspace_words, int64_t size_k, int64_t size_n, int64_t groups,
                            int grouped, int zeros_transposed, void* stream);
+/* The groups of an act-order projection's rows, int32[size_k], in ascending order, and the rows in that order, those of one group as
+ * they came (marlin_utils.py: marlin_sort_g_idx); and sonar_load_gptq_linear of such a projection, whose rows are taken in that order. */
+int sonar_sort_g_idx(const int32_t* g_idx, int32_t* sorted, int32_t* order, int64_t size_k, void* stream);
+int sonar_load_gptq_act_order(const uint32_t* codes, uint32_t* codes_out, const void* scales, void* scales_out,
+                              const int32_t* g_idx, int32_t* g_idx_out, int32_t* order, uint32_t* workspace,
+                              int64_t workspace_words, int64_t size_k, int64_t size_n, int64_t groups, int grouped,
+                              void* stream);
 /* Zero points packed along N, eight to a word, in plain or AWQ nibble order -> (rows, N/8) words in the
  * order the GEMM reads (marlin_utils.py:457-559: marlin_zero_points, awq_to_marlin_zero_points);
  * in[row * row_stride + word * word_stride]. */
@@ -153,6 +160,9 @@ int sonar_marlin_pack_zero_points(const uint32_t* in, uint32_t* out, int64_t row
  * transposed to (N/8, G) (_convert_awq_to_standard_format, layers/quantization/auto_awq.py:93-153). */
 int sonar_awq_to_gptq(const uint32_t* in, uint32_t* out, int64_t size_k, int64_t size_n, void* stream);
 int sonar_awq_zeros_to_plain(const uint32_t* in, uint32_t* out, int64_t groups, int64_t size_n, void* stream);
+/* Both, as one launch. */
+int sonar_awq_to_standard(const uint32_t* codes, uint32_t* codes_out, const uint32_t* zeros, uint32_t* zeros_out,
+                          int64_t size_k, int64_t size_n, int64_t groups, void* stream);
 
 /* Marlin (K/16, 2N) int32 <-> gfx950 streaming order, same number of words.
  * K % 32 == 0, N % 64 == 0.  in and out must not overlap. */
@@ -548,6 +558,10 @@ int64_t sonar_debug_moe_pair_schedule(int64_t big, int64_t small, int64_t max_ro
                                       int32_t* out, int64_t out_rows);
 /* What the choice between marlin_mid_gemm and the tile kernels takes the latter's time to be (us; 4-bit integer codes). */
 double sonar_debug_tile_estimate(int64_t size_m, int64_t size_n, int64_t size_k);
+/* The tiles of a dense call that runs as 128-row tiles, two workgroups on a compute unit (format: 0 4-bit integers, 1 MXFP4);
+ * no rows: it runs otherwise. */
+int64_t sonar_debug_twin_schedule(int64_t size_m, int64_t size_n, int64_t size_k, int64_t num_groups, int dtype, int format,
+                                  int32_t* out, int64_t out_rows);
 /* Which of the two that choice falls on (1: marlin_mid_gemm) for a call of more than 64 rows that either could run, integer or
  * fp8 codes, 256 compute units; -1 for arguments out of range. */
 int sonar_debug_mid_beats_tiles(int64_t size_m, int64_t size_n, int64_t size_k, int64_t num_groups, int dtype,

@@ -47,6 +47,9 @@ PROTOTYPES = {
     "sonar_awq_marlin_moe_repack": (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_int64, c_void_p]),
     "sonar_marlin_permute_scales": (c_int, [c_void_p, c_void_p, c_int64, c_int, c_void_p]),
     "sonar_load_gptq_linear": (c_int, [c_void_p] * 7 + [c_int64] * 4 + [c_int, c_int, c_void_p]),
+    "sonar_sort_g_idx": (c_int, [c_void_p] * 3 + [c_int64, c_void_p]),
+    "sonar_load_gptq_act_order": (c_int, [c_void_p] * 8 + [c_int64] * 4 + [c_int, c_void_p]),
+    "sonar_awq_to_standard": (c_int, [c_void_p] * 4 + [c_int64] * 3 + [c_void_p]),
     "sonar_marlin_pack_zero_points": (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_int, c_int,
                                               c_void_p]),
     "sonar_awq_to_gptq": (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_void_p]),

@@ -498,13 +498,14 @@ struct LoadLinear {
   uint32_t zero_blocks;
   uint32_t* workspace;
   int workspace_words;
+  const int32_t* perm;   // act-order: the rows in the order of their groups
 };
-template <bool GROUPS>
+template <bool GROUPS, bool HAS_PERM>
 __global__ __launch_bounds__(256) void load_linear_kernel(const LoadLinear p) {
   __shared__ alignas(16) uint32_t lds[kRepackTiles * kRepackLdsStride];
   uint32_t block = blockIdx.x;
   if (block < p.code_blocks) {
-    gptq_tiles<false>(lds, block, p.codes, nullptr, p.codes_out, p.size_k, p.size_n, p.tiles, 0, p.tiles);
+    gptq_tiles<HAS_PERM>(lds, block, p.codes, p.perm, p.codes_out, p.size_k, p.size_n, p.tiles, 0, p.tiles);
     return;
   }
   block -= p.code_blocks;
@@ -525,10 +526,7 @@ __global__ __launch_bounds__(256) void load_linear_kernel(const LoadLinear p) {
 
 // AutoAWQ codes (K, N/8) -> the GPTQ packing (K/8, N): a thread transposes the 8 x 8 nibbles of eight
 // rows of one word, three rounds of block swaps, and stores the eight columns side by side.
-__global__ __launch_bounds__(256) void awq_codes_to_gptq(const uint32_t* __restrict__ in, uint32_t* __restrict__ out,
-                                                         int words, long total) {
-  const long idx = (long)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= total) return;
+__device__ __forceinline__ void awq_codes_word(const uint32_t* __restrict__ in, uint32_t* __restrict__ out, int words, long idx) {
   const long r = idx / words;
   const int w = (int)(idx - r * words);
   uint32_t x[8];
@@ -560,10 +558,8 @@ __global__ __launch_bounds__(256) void awq_codes_to_gptq(const uint32_t* __restr
 }
 
 // AutoAWQ zero points (G, N/8) -> plain column order, transposed: (N/8, G).
-__global__ __launch_bounds__(256) void awq_zeros_to_plain(const uint32_t* __restrict__ in, uint32_t* __restrict__ out,
-                                                          int groups, int words, long total) {
-  const long idx = (long)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= total) return;
+__device__ __forceinline__ void awq_zeros_word(const uint32_t* __restrict__ in, uint32_t* __restrict__ out, int groups, int words,
+                                               long idx) {
   const long w = idx / groups;
   const uint32_t z = in[(idx - w * groups) * words + w];
   uint32_t packed = 0;
@@ -572,11 +568,104 @@ __global__ __launch_bounds__(256) void awq_zeros_to_plain(const uint32_t* __rest
   out[idx] = packed;
 }
 
+// Codes and zero points of a projection as one launch: bound by the host, it takes two of the 26.6 us off a load of 1024 x 4096.
+struct AwqToPlain {
+  const uint32_t* codes;
+  uint32_t* codes_out;
+  const uint32_t* zeros;
+  uint32_t* zeros_out;
+  int words, groups;         // words of a row (N / 8)
+  long code_words, zero_words;
+  uint32_t code_blocks;
+};
+__global__ __launch_bounds__(256) void awq_to_plain_kernel(const AwqToPlain p) {
+  if (blockIdx.x < p.code_blocks) {
+    const long idx = (long)blockIdx.x * 256 + threadIdx.x;
+    if (idx < p.code_words) awq_codes_word(p.codes, p.codes_out, p.words, idx);
+  } else {
+    const long idx = (long)(blockIdx.x - p.code_blocks) * 256 + threadIdx.x;
+    if (idx < p.zero_words) awq_zeros_word(p.zeros, p.zeros_out, p.groups, p.words, idx);
+  }
+}
+
+// The groups of the rows of an act-order projection in ascending order, and the rows in that order, those of a group as they came
+// (torch.argsort and two gathers of the reference, marlin_utils.py: marlin_sort_g_idx).  The rank of a row is the number of smaller
+// groups and of equal ones before it; a workgroup finds it for 64 rows.  Groups below kSortBins, all that a checkpoint holds, are
+// counted in LDS, over all rows and over those before the workgroup's, and the counts summed up; for any other value the 16
+// wavefronts compare each row with a sixteenth of all rows, which come as scalars, two vector instructions a pair.  Calls
+// in a row: K = 1024 6 us, 14336 8 (compared 22), 32768 16 (compared 73); a library's sort and gathers, launches of their own, 34 to 51.
+constexpr int kSortWaves = 16, kSortBins = 64 * kSortWaves;
+__global__ __launch_bounds__(64 * kSortWaves) void sort_group_indices(const int32_t* __restrict__ g, int32_t* __restrict__ sorted,
+                                                                      int32_t* __restrict__ order, int n) {
+  __shared__ int32_t counts[kSortWaves][64];   // by wavefront and row; or of the rows before the workgroup's, by group
+  __shared__ int32_t all[kSortBins], totals[kSortWaves];
+  int32_t* before = &counts[0][0];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int first = 64 * blockIdx.x, i = first + lane;
+  const int32_t mine = i < n ? g[i] : 0;
+  all[threadIdx.x] = 0;
+  before[threadIdx.x] = 0;
+  __syncthreads();
+  int other = 0;
+#pragma unroll 4
+  for (int j = threadIdx.x; j < n; j += kSortBins) {
+    const int32_t group = g[j];
+    if ((uint32_t)group < (uint32_t)kSortBins) {
+      atomicAdd(&all[group], 1);
+      if (j < first) atomicAdd(&before[group], 1);
+    } else {
+      other = 1;
+    }
+  }
+  int rank = 0;
+  if (!__syncthreads_or(other)) {
+    int sum = all[threadIdx.x];   // up to and with this group
+    const int own = sum;
+#pragma unroll
+    for (int step = 1; step < 64; step *= 2) {
+      const int below = __shfl_up(sum, step);
+      sum += lane >= step ? below : 0;
+    }
+    if (lane == 63) totals[wave] = sum;
+    __syncthreads();
+    for (int w = 0; w < wave; ++w) sum += totals[w];
+    all[threadIdx.x] = sum - own;
+    __syncthreads();
+    if (wave > 0) return;
+    for (int l = 0; l < 64; ++l) rank += l < lane && __builtin_amdgcn_readlane(mine, l) == mine ? 1 : 0;
+    rank += all[mine] + before[mine];
+  } else {
+    const int share = (n + kSortWaves - 1) / kSortWaves, from = wave * share, to = min(n, from + share);
+    int count = 0;
+#pragma unroll 16
+    for (int j = from; j < min(to, first); ++j) count += g[j] <= mine ? 1 : 0;
+    for (int j = max(from, first); j < min(to, first + 64); ++j) count += g[j] < mine || (g[j] == mine && j < i) ? 1 : 0;
+#pragma unroll 16
+    for (int j = max(from, first + 64); j < to; ++j) count += g[j] < mine ? 1 : 0;
+    counts[wave][lane] = count;
+    __syncthreads();
+    if (wave > 0) return;
+#pragma unroll
+    for (int w = 0; w < kSortWaves; ++w) rank += counts[w][lane];
+  }
+  if (i >= n) return;
+  sorted[rank] = mine;
+  order[rank] = i;
+}
+
 int grid_for(long total_words) {
   long blocks = (total_words + 255) / 256;
   if (blocks > 256L * 32) blocks = 256L * 32;
   if (blocks < 1) blocks = 1;
   return (int)blocks;
+}
+
+int launch_awq_to_plain(AwqToPlain p, hipStream_t st) {
+  p.code_blocks = (uint32_t)((p.code_words + 255) / 256);
+  const int64_t blocks = (int64_t)p.code_blocks + (p.zero_words + 255) / 256;
+  SONAR_REQUIRE(blocks < (1LL << 31), "weight too large");
+  awq_to_plain_kernel<<<(int)blocks, 256, 0, st>>>(p);
+  return launch_status("awq_to_plain_kernel");
 }
 
 int check_repack_shape(int64_t size_k, int64_t size_n, int num_bits) {
@@ -821,10 +910,9 @@ extern "C" int sonar_marlin_pack_zero_points(const uint32_t* in, uint32_t* out, 
   return launch_status("pack_zero_points");
 }
 
-extern "C" int sonar_load_gptq_linear(const uint32_t* codes, uint32_t* codes_out, const void* scales, void* scales_out,
-                                      const uint32_t* zeros, uint32_t* zeros_out, uint32_t* workspace,
-                                      int64_t workspace_words, int64_t size_k, int64_t size_n, int64_t groups, int grouped,
-                                      int zeros_transposed, void* stream) {
+static int load_linear(const uint32_t* codes, uint32_t* codes_out, const void* scales, void* scales_out, const uint32_t* zeros,
+                       uint32_t* zeros_out, uint32_t* workspace, int64_t workspace_words, int64_t size_k, int64_t size_n,
+                       int64_t groups, int grouped, int zeros_transposed, const int32_t* perm, void* stream) {
   if (int rc = check_repack_shape(size_k, size_n, 4)) return rc;
   if (int rc = check_experts(1, size_k, size_n)) return rc;
   SONAR_REQUIRE(groups >= 1 && groups * size_n < (1LL << 38), "num_groups = %ld out of range", (long)groups);
@@ -858,9 +946,38 @@ extern "C" int sonar_load_gptq_linear(const uint32_t* codes, uint32_t* codes_out
   p.workspace_words = (int)workspace_words;
   const int64_t blocks = (int64_t)p.code_blocks + p.scale_blocks + p.zero_blocks + (workspace_words > 0);
   SONAR_REQUIRE(blocks < (1LL << 31), "weight too large");
-  auto* kernel = grouped ? load_linear_kernel<true> : load_linear_kernel<false>;
+  p.perm = perm;
+  auto* kernel = perm ? (grouped ? load_linear_kernel<true, true> : load_linear_kernel<false, true>)
+                      : (grouped ? load_linear_kernel<true, false> : load_linear_kernel<false, false>);
   kernel<<<(int)blocks, 256, 0, (hipStream_t)stream>>>(p);
   return launch_status("load_linear_kernel");
+}
+
+extern "C" int sonar_load_gptq_linear(const uint32_t* codes, uint32_t* codes_out, const void* scales, void* scales_out,
+                                      const uint32_t* zeros, uint32_t* zeros_out, uint32_t* workspace,
+                                      int64_t workspace_words, int64_t size_k, int64_t size_n, int64_t groups, int grouped,
+                                      int zeros_transposed, void* stream) {
+  return load_linear(codes, codes_out, scales, scales_out, zeros, zeros_out, workspace, workspace_words, size_k, size_n, groups, grouped,
+                     zeros_transposed, nullptr, stream);
+}
+
+extern "C" int sonar_sort_g_idx(const int32_t* g_idx, int32_t* sorted, int32_t* order, int64_t size_k, void* stream) {
+  SONAR_REQUIRE(size_k >= 0 && size_k <= (1 << 20), "size_k = %ld out of range", (long)size_k);
+  if (size_k == 0) return SONAR_OK;
+  SONAR_REQUIRE(g_idx && sorted && order && g_idx != sorted && g_idx != order && sorted != order,
+                "g_idx and its outputs must be distinct non-NULL buffers");
+  sort_group_indices<<<(int)((size_k + 63) / 64), 64 * kSortWaves, 0, (hipStream_t)stream>>>(g_idx, sorted, order, (int)size_k);
+  return launch_status("sort_group_indices");
+}
+
+extern "C" int sonar_load_gptq_act_order(const uint32_t* codes, uint32_t* codes_out, const void* scales, void* scales_out,
+                                         const int32_t* g_idx, int32_t* g_idx_out, int32_t* order, uint32_t* workspace,
+                                         int64_t workspace_words, int64_t size_k, int64_t size_n, int64_t groups, int grouped,
+                                         void* stream) {
+  if (int rc = check_repack_shape(size_k, size_n, 4)) return rc;
+  if (int rc = sonar_sort_g_idx(g_idx, g_idx_out, order, size_k, stream)) return rc;
+  return load_linear(codes, codes_out, scales, scales_out, nullptr, nullptr, workspace, workspace_words, size_k, size_n, groups, grouped, 0,
+                     order, stream);
 }
 
 extern "C" int sonar_awq_to_gptq(const uint32_t* in, uint32_t* out, int64_t size_k, int64_t size_n, void* stream) {
@@ -870,8 +987,20 @@ extern "C" int sonar_awq_to_gptq(const uint32_t* in, uint32_t* out, int64_t size
   SONAR_REQUIRE(total < (1LL << 38), "weight too large");
   if (total == 0) return SONAR_OK;
   SONAR_REQUIRE(in && out && in != out, "in and out must be distinct non-NULL buffers");
-  awq_codes_to_gptq<<<blocks_of(total), 256, 0, (hipStream_t)stream>>>(in, out, (int)(size_n / 8), total);
-  return launch_status("awq_codes_to_gptq");
+  return launch_awq_to_plain({in, out, nullptr, nullptr, (int)(size_n / 8), 0, total, 0, 0}, (hipStream_t)stream);
+}
+
+extern "C" int sonar_awq_to_standard(const uint32_t* codes, uint32_t* codes_out, const uint32_t* zeros, uint32_t* zeros_out,
+                                     int64_t size_k, int64_t size_n, int64_t groups, void* stream) {
+  SONAR_REQUIRE(size_k >= 0 && size_n > 0 && size_k % 8 == 0 && size_n % 8 == 0 && size_n < (1LL << 30) && size_k < (1LL << 30) &&
+                    groups >= 0 && groups < (1LL << 30), "size_k = %ld and size_n = %ld must be multiples of 8", (long)size_k, (long)size_n);
+  const int64_t code_words = size_k / 8 * (size_n / 8), zero_words = groups * (size_n / 8);
+  SONAR_REQUIRE(code_words < (1LL << 38) && zero_words < (1LL << 38), "weight too large");
+  SONAR_REQUIRE((code_words == 0 || (codes && codes_out && codes != codes_out)) &&
+                    (zero_words == 0 || (zeros && zeros_out && zeros != zeros_out)), "inputs and outputs must be distinct non-NULL buffers");
+  if (code_words + zero_words == 0) return SONAR_OK;
+  return launch_awq_to_plain({codes, codes_out, zeros, zeros_out, (int)(size_n / 8), (int)groups, code_words, zero_words, 0},
+                             (hipStream_t)stream);
 }
 
 extern "C" int sonar_awq_zeros_to_plain(const uint32_t* in, uint32_t* out, int64_t groups, int64_t size_n,
@@ -882,6 +1011,5 @@ extern "C" int sonar_awq_zeros_to_plain(const uint32_t* in, uint32_t* out, int64
   SONAR_REQUIRE(total < (1LL << 38), "too many zero points");
   if (total == 0) return SONAR_OK;
   SONAR_REQUIRE(in && out && in != out, "in and out must be distinct non-NULL buffers");
-  awq_zeros_to_plain<<<blocks_of(total), 256, 0, (hipStream_t)stream>>>(in, out, (int)groups, (int)(size_n / 8), total);
-  return launch_status("awq_zeros_to_plain");
+  return launch_awq_to_plain({nullptr, nullptr, in, out, (int)(size_n / 8), (int)groups, 0, total, 0}, (hipStream_t)stream);
 }

@@ -477,13 +477,49 @@ std::tuple<Tensor, Tensor> awq_to_standard(const Tensor& qweight, const Tensor& 
   c10::hip::HIPGuardMasqueradingAsCUDA guard(qweight.device());
   Tensor codes = at::empty({k / 8, words * 8}, qweight.options());
   Tensor zeros = at::empty({words, groups}, qzeros.options());
-  raise_if_failed(sonar_awq_to_gptq(static_cast<const uint32_t*>(qweight.const_data_ptr()),
-                                    static_cast<uint32_t*>(codes.mutable_data_ptr()), k, words * 8,
-                                    current_stream(qweight)));
-  raise_if_failed(sonar_awq_zeros_to_plain(static_cast<const uint32_t*>(qzeros.const_data_ptr()),
-                                           static_cast<uint32_t*>(zeros.mutable_data_ptr()), groups, words * 8,
-                                           current_stream(qzeros)));
+  raise_if_failed(sonar_awq_to_standard(static_cast<const uint32_t*>(qweight.const_data_ptr()),
+                                        static_cast<uint32_t*>(codes.mutable_data_ptr()),
+                                        static_cast<const uint32_t*>(qzeros.const_data_ptr()),
+                                        static_cast<uint32_t*>(zeros.mutable_data_ptr()), k, words * 8, groups, current_stream(qweight)));
   return {codes, zeros};
+}
+
+// (g_idx in ascending order, the rows in that order)
+std::tuple<Tensor, Tensor> sort_g_idx(const Tensor& g_idx) {
+  TORCH_CHECK(g_idx.is_cuda() && g_idx.is_contiguous() && g_idx.scalar_type() == at::kInt && g_idx.dim() == 1,
+              "g_idx must be a contiguous one-dimensional int32 GPU tensor");
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(g_idx.device());
+  Tensor sorted = at::empty_like(g_idx), order = at::empty_like(g_idx);
+  raise_if_failed(sonar_sort_g_idx(static_cast<const int32_t*>(g_idx.const_data_ptr()), static_cast<int32_t*>(sorted.mutable_data_ptr()),
+                                   static_cast<int32_t*>(order.mutable_data_ptr()), g_idx.numel(), current_stream(g_idx)));
+  return {sorted, order};
+}
+
+// load_gptq_linear of an act-order projection: (codes, scales, sorted g_idx, the rows in that order, workspace).
+std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor> load_gptq_act_order(const Tensor& qweight, const Tensor& scales, const Tensor& g_idx,
+                                                                       bool grouped) {
+  TORCH_CHECK(qweight.is_cuda() && qweight.is_contiguous() && qweight.scalar_type() == at::kInt && qweight.dim() == 2,
+              "qweight must be a contiguous two-dimensional int32 GPU tensor");
+  const int64_t size_k = qweight.size(0) * 8, size_n = qweight.size(1);
+  TORCH_CHECK(scales.is_cuda() && scales.is_contiguous() && scales.element_size() == 2 && scales.dim() == 2 &&
+                  scales.size(1) == size_n && scales.size(0) >= 1 && scales.device() == qweight.device(),
+              "scales must be a contiguous 16-bit (groups, N) tensor on the GPU of qweight");
+  TORCH_CHECK(g_idx.is_cuda() && g_idx.is_contiguous() && g_idx.scalar_type() == at::kInt && g_idx.dim() == 1 &&
+                  g_idx.numel() == size_k && g_idx.device() == qweight.device(),
+              "g_idx must be a contiguous int32 tensor of K values on the GPU of qweight");
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(qweight.device());
+  Tensor codes_out = at::empty({size_k / 16, size_n * 2}, qweight.options());
+  Tensor scales_out = at::empty_like(scales);
+  Tensor sorted = at::empty_like(g_idx), order = at::empty_like(g_idx);
+  Tensor workspace = at::empty({at::cuda::getCurrentDeviceProperties()->multiProcessorCount}, qweight.options());
+  raise_if_failed(sonar_load_gptq_act_order(
+      static_cast<const uint32_t*>(qweight.const_data_ptr()), static_cast<uint32_t*>(codes_out.mutable_data_ptr()),
+      scales.const_data_ptr(), scales_out.mutable_data_ptr(), static_cast<const int32_t*>(g_idx.const_data_ptr()),
+      static_cast<int32_t*>(sorted.mutable_data_ptr()), static_cast<int32_t*>(order.mutable_data_ptr()),
+      static_cast<uint32_t*>(workspace.mutable_data_ptr()), workspace.numel(), size_k, size_n, scales.size(0), grouped ? 1 : 0,
+      current_stream(qweight)));
+  forget_memory_of(codes_out);
+  return {codes_out, scales_out, sorted, order, workspace};
 }
 
 Tensor marlin_to_gfx950(const Tensor& b_q_weight, int64_t size_k, int64_t size_n) {
@@ -1455,6 +1491,8 @@ TORCH_LIBRARY(sonar_amd, m) {
   m.def("permute_scales(Tensor s, bool grouped) -> Tensor");
   m.def("pack_zero_points(Tensor zp, bool awq_order, bool transposed, bool is_a_8bit) -> Tensor");
   m.def("awq_to_standard(Tensor qweight, Tensor qzeros) -> (Tensor, Tensor)");
+  m.def("sort_g_idx(Tensor g_idx) -> (Tensor, Tensor)");
+  m.def("load_gptq_act_order(Tensor qweight, Tensor scales, Tensor g_idx, bool grouped) -> (Tensor, Tensor, Tensor, Tensor, Tensor)");
   m.def("load_gptq_linear(Tensor qweight, Tensor scales, Tensor? zeros, bool grouped, bool transposed) -> "
         "(Tensor, Tensor, Tensor, Tensor)");
   m.def("per_token_quant_fp8(Tensor x) -> (Tensor, Tensor)");
@@ -1478,6 +1516,8 @@ TORCH_LIBRARY_IMPL(sonar_amd, CUDA, m) {
   m.impl("pack_zero_points", &pack_zero_points);
   m.impl("awq_to_standard", &awq_to_standard);
   m.impl("load_gptq_linear", &load_gptq_linear);
+  m.impl("sort_g_idx", &sort_g_idx);
+  m.impl("load_gptq_act_order", &load_gptq_act_order);
   m.impl("per_token_quant_fp8", &per_token_quant_fp8);
 }
 

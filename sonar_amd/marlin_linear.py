@@ -155,11 +155,12 @@ class MarlinLinearKernel:
 
     def _load_in_one_launch(self, layer) -> bool:
         """process_weights_after_loading for tensors already in the layout that the kernels of the general path read: 4-bit
-        codes (K/8, N), 16-bit scales (G, N), zero points packed along N, all contiguous on one GPU, no act-order, no
-        padding.  False: nothing was touched."""
+        codes (K/8, N), 16-bit scales (G, N), zero points packed along N, all contiguous on one GPU, no padding.  Of an
+        act-order projection (no zero points, its groups whole, nothing loaded before) in two: the first sorts the rows.
+        False: nothing was touched."""
         c = self.config
         size_k, size_n = c.partition_weight_shape
-        if (c.has_g_idx or c.weight_type.size_bits != 4 or c.act_type.itemsize != 2 or size_n % 64 or size_k % 128
+        if (c.weight_type.size_bits != 4 or c.act_type.itemsize != 2 or size_n % 64 or size_k % 128
                 or hasattr(self, "workspace")):
             return False
         w_q, w_s = getattr(layer, self.w_q_name), getattr(layer, self.w_s_name)
@@ -176,12 +177,25 @@ class MarlinLinearKernel:
             if (not transposed and zeros.shape != (groups, size_n // 8)) or (
                     zeros.dtype != torch.int32 or zeros.device != w_q.device or not zeros.is_contiguous()):
                 return False
-        codes, scales, zeros, self.workspace = torch.ops.sonar_amd.load_gptq_linear(
-            w_q, w_s, zeros, c.group_size != -1 and c.group_size < size_k, transposed)
-        device = codes.device
-        self.is_k_full = True
-        setattr(layer, self.w_gidx_name, marlin_make_empty_g_idx(device))
-        layer.g_idx_sort_indices = marlin_make_empty_g_idx(device)
+        if c.has_g_idx:
+            g_idx = getattr(layer, self.w_gidx_name)
+            if (c.zero_points or g_idx.dtype != torch.int32 or g_idx.shape != (size_k,) or g_idx.device != w_q.device
+                    or not g_idx.is_contiguous() or size_k > 32768
+                    or isinstance(getattr(layer, "g_idx_sort_indices", None), torch.Tensor)):
+                return False
+            codes, scales, g_idx, order, self.workspace = torch.ops.sonar_amd.load_gptq_act_order(
+                w_q, w_s, g_idx, c.group_size != -1 and c.group_size < size_k)
+            device = codes.device
+            self.is_k_full = marlin_is_k_full(True, size_k != c.full_weight_shape[0])
+            setattr(layer, self.w_gidx_name, g_idx)
+            layer.g_idx_sort_indices = torch.nn.Parameter(order, requires_grad=False)
+        else:
+            codes, scales, zeros, self.workspace = torch.ops.sonar_amd.load_gptq_linear(
+                w_q, w_s, zeros, c.group_size != -1 and c.group_size < size_k, transposed)
+            device = codes.device
+            self.is_k_full = True
+            setattr(layer, self.w_gidx_name, marlin_make_empty_g_idx(device))
+            layer.g_idx_sort_indices = marlin_make_empty_g_idx(device)
         setattr(layer, self.w_zp_name, zeros if c.zero_points else marlin_make_empty_g_idx(device))
         setattr(layer, self.w_q_name, codes)
         setattr(layer, self.w_s_name, scales)

@@ -91,6 +91,16 @@ def _register_fakes() -> None:
                 qweight.new_empty((0 if zeros is None else scales.shape[0], n // 8)),
                 qweight.new_empty((torch.cuda.get_device_properties(qweight.device).multi_processor_count,)))
 
+    @reg("sonar_amd::sort_g_idx")
+    def _(g_idx):
+        return torch.empty_like(g_idx), torch.empty_like(g_idx)
+
+    @reg("sonar_amd::load_gptq_act_order")
+    def _(qweight, scales, g_idx, grouped):
+        k, n = qweight.shape[0] * 8, qweight.shape[1]
+        return (qweight.new_empty((k // 16, n * 2)), torch.empty_like(scales), torch.empty_like(g_idx), torch.empty_like(g_idx),
+                qweight.new_empty((torch.cuda.get_device_properties(qweight.device).multi_processor_count,)))
+
     @reg("sonar_amd::fused_moe")
     def _(output, hidden, w1, w2, bias1, bias2, scale1, scale2, global_scale1, global_scale2, topk_weights, topk_ids,
           g_idx1, g_idx2, perm1, perm2, zeros1, zeros2, cache13, cache2, b_type_id, num_experts, block_size,
