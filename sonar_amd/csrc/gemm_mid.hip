@@ -6,7 +6,9 @@
 // exactly once in the workgroup, a wavefront's accumulators are small (16 MB registers), two wavefronts
 // share a SIMD (one's matrix instructions run beside the other's dequantisation), and the activations,
 // which the two strips share, are staged in LDS at half the bytes per matrix instruction of a one-strip
-// workgroup (at one strip the copies alone would need the whole 64 bytes per clock of a compute unit).
+// workgroup (at one strip the copies alone would need the whole 64 bytes per clock of a compute unit).  Grouped calls of
+// many rounds of workgroups take four strips x two ranges (mid_moe_strips): start, end and the sum of the ranges once for twice the columns,
+// and half the copies (32 experts of 42 rows, K = 1152, N = 15360: 187 -> 132 us).
 //
 // What bounds it: the sum of vector and matrix instructions, which two wavefronts a SIMD overlap in part, and the start and the
 // end.  (Counters at 64 to 333 rows: of the busy cycles vector issue fills 41 to 48 % and the matrix pipes 26 to 38 %; without
@@ -64,8 +66,8 @@ namespace sonar {
 namespace {
 
 constexpr int kMidWaves = 8;
-constexpr int mid_strips(int mb) { return mb == 1 ? 1 : 2; }                 // strips of a workgroup
-constexpr int mid_ranges(int mb) { return kMidWaves / mid_strips(mb); }      // ranges of K
+constexpr int mid_strips(int mb) { return mb == 1 ? 1 : 2; }                 // strips of a workgroup (grouped: or four)
+constexpr int mid_ranges(int strips) { return kMidWaves / strips; }          // ranges of K
 constexpr int kMidStepK = 64;     // rows of K a step takes from each range
 
 // Activation stages in LDS.
@@ -76,10 +78,10 @@ constexpr int mid_stages(int mb, bool deep) { return deep ? 5 : mb > 1 && mb <= 
 // N = 16384 (6) 16.3 -> 15.6, but K = 2048, N = 8192 (4) 9.6 -> 10.2, K = 1024, N = 1024 (2) 5.1 -> 6.1.
 constexpr int kMidDeepSteps = 6;
 constexpr int mid_waves_per_simd(int mb, bool deep) { return mb == 1 && !deep ? 4 : 2; }
-constexpr int mid_stage_bytes(int mb) { return mid_ranges(mb) * mb * 2048; }
+constexpr int mid_stage_bytes(int mb, int strips) { return mid_ranges(strips) * mb * 2048; }
 constexpr int mid_sum_rows(int mb) { return mb < 4 ? mb : 4; }   // row blocks summed at a time at the end
-constexpr int mid_lds(int mb, bool deep) {
-  const int stages = mid_stages(mb, deep) * mid_stage_bytes(mb), sum = kMidWaves * mid_sum_rows(mb) * 4096;
+constexpr int mid_lds(int mb, bool deep, int strips) {
+  const int stages = mid_stages(mb, deep) * mid_stage_bytes(mb, strips), sum = kMidWaves * mid_sum_rows(mb) * 4096;
   return stages > sum ? stages : sum;
 }
 
@@ -98,7 +100,7 @@ struct MidDequant {
   typedef typename std::conditional<k8, typename D8::Col, typename D4::Col>::type Col;
 };
 
-template <typename T, int FMT, int GROUPS, int MB, bool DEEP, bool GROUPED = false>
+template <typename T, int FMT, int GROUPS, int MB, bool DEEP, bool GROUPED = false, int STRIPS = mid_strips(MB)>
 __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(mid_waves_per_simd(MB, DEEP), mid_waves_per_simd(MB, DEEP)))) void marlin_mid_gemm(
     const typename std::conditional<GROUPED, MidMoeParams, MidParams>::type p) {
   MidMoe moe = {};
@@ -127,9 +129,10 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
   constexpr bool kNoScales = GROUPS == kOneGroup || kCodes;   // none among the memory operations of every step
   constexpr int D = mid_stages(MB, DEEP);
   constexpr int W = D - 1;                           // ring of the packed codes and scales in registers
-  constexpr int kStage = mid_stage_bytes(MB);
-  constexpr int kMidStrips = mid_strips(MB), kMidRanges = mid_ranges(MB);
-  constexpr int kCopies = 2 * MB / kMidStrips;       // 8-row copies of activations per wavefront and step
+  constexpr int kStage = mid_stage_bytes(MB, STRIPS);
+  constexpr int kMidStrips = STRIPS, kMidRanges = mid_ranges(STRIPS);
+  // 8-row copies of activations per wavefront and step (three row blocks and four strips: the last wavefront's are copies 5 again)
+  constexpr int kCopies = (2 * MB + kMidStrips - 1) / kMidStrips;
   constexpr int kLoads = Fmt::k8 ? 4 : 2;            // 16-byte loads of packed codes per lane and step
   constexpr int kScaleRows = GROUPS == kChunkGroups ? 2 : 1;
   // memory operations per wavefront and step
@@ -171,7 +174,7 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
   uint32_t a_off[kCopies];
 #pragma unroll
   for (int i = 0; i < kCopies; ++i) {
-    int row = m0 + 8 * (strip_of * kCopies + i) + (lane >> 3);
+    int row = m0 + 8 * min(strip_of * kCopies + i, 2 * MB - 1) + (lane >> 3);
     if constexpr (GROUPED) {   // (padding slots read row 0 and are not stored)
       const int id = row < moe.sorted_len ? moe.sorted_ids[row] : moe.rows_total;
       row = (unsigned)id < (unsigned)moe.rows_total ? (moe.a_by_slot ? row : id / moe.top_k) : 0;
@@ -217,7 +220,7 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
     } else {
       const int i = op - (kOps - kCopies);
       const char* a_src = reinterpret_cast<const char*>(p.a) + (size_t)k * (kMidStepK * 2);
-      copy_to_lds<16>(a_lds + slot * kStage + (strip_of * kCopies + i) * 1024, a_off[i], a_src);
+      copy_to_lds<16>(a_lds + slot * kStage + min(strip_of * kCopies + i, 2 * MB - 1) * 1024, a_off[i], a_src);
     }
   };
   // Scales of the unit of step `k`, behind whose first half they are taken from the registers, and zero points, which fp16
@@ -547,7 +550,7 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
         for (int r = 0; r < 4; ++r) acc[j][i][r] *= Dq<T>::to_float(one_scale[j]);
   }
 
-  // ---- the four ranges meet in LDS, mid_sum_rows(MB) row blocks at a time; a wavefront adds a quarter of
+  // ---- the ranges meet in LDS, mid_sum_rows(MB) row blocks at a time; a wavefront adds its share (a quarter of four ranges) of
   // its strip's accumulator tiles, in the order of the ranges
   constexpr int kSum = mid_sum_rows(MB);
   float4* sums = reinterpret_cast<float4*>(smem);
@@ -574,7 +577,7 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
         }
     __syncthreads();
 #pragma unroll
-    for (int u = 0; u < kSum; ++u) {
+    for (int u = 0; u < (kMidRanges == 2 ? 2 * kSum : kSum); ++u) {
       constexpr int kEach = kSum * 4 / kMidRanges;   // accumulator tiles a wavefront adds
       if (kEach > 0 ? u >= kEach : range >= 4 * kSum) continue;
       const int q = kEach > 0 ? range * kEach + u : range;
@@ -652,15 +655,16 @@ __global__ __launch_bounds__(256) void marlin_mid_sum(const MidParams p) {
   }
 }
 
-template <typename T, int FMT, int GROUPS, int MB, bool DEEP = false, bool GROUPED = false>
+template <typename T, int FMT, int GROUPS, int MB, bool DEEP = false, bool GROUPED = false, int STRIPS = mid_strips(MB)>
 int launch_mid_rows(const typename std::conditional<GROUPED, MidMoeParams, MidParams>::type& p, hipStream_t st) {
   static bool attr_set = false;   // raising the dynamic LDS limit is needed once per form
   if (!attr_set) {
-    SONAR_HIP(hipFuncSetAttribute((const void*)marlin_mid_gemm<T, FMT, GROUPS, MB, DEEP, GROUPED>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, mid_lds(MB, DEEP)));
+    SONAR_HIP(hipFuncSetAttribute((const void*)marlin_mid_gemm<T, FMT, GROUPS, MB, DEEP, GROUPED, STRIPS>,
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, mid_lds(MB, DEEP, STRIPS)));
     attr_set = true;
   }
-  marlin_mid_gemm<T, FMT, GROUPS, MB, DEEP, GROUPED><<<(p.tiles * p.splits + 7) / 8 * 8, kMidWaves * 64, mid_lds(MB, DEEP), st>>>(p);
+  marlin_mid_gemm<T, FMT, GROUPS, MB, DEEP, GROUPED, STRIPS>
+      <<<(p.tiles * p.splits + 7) / 8 * 8, kMidWaves * 64, mid_lds(MB, DEEP, STRIPS), st>>>(p);
   return launch_status("marlin_mid_gemm");
 }
 
@@ -678,7 +682,7 @@ int launch_mid(const MidParams& p, int row_blocks, hipStream_t st) {
   switch (row_blocks) {
     case 1:
       if constexpr (FMT == kMidInt8 || FMT == kMidFp8 || FMT == kMidNvFp4) {
-        if (p.tiles * p.splits <= p.cus && p.split_steps >= kMidDeepSteps * mid_ranges(1)) return launch_mid_rows<T, FMT, GROUPS, 1, true>(p, st);
+        if (p.tiles * p.splits <= p.cus && p.split_steps >= kMidDeepSteps * mid_ranges(mid_strips(1))) return launch_mid_rows<T, FMT, GROUPS, 1, true>(p, st);
         return launch_mid_rows<T, FMT, GROUPS, 1>(p, st);
       }
     case 2: return launch_mid_rows<T, FMT, GROUPS, 2>(p, st);
@@ -721,10 +725,11 @@ int launch_mid_format(const MidParams& p, int format, int row_blocks, hipStream_
 
 template <typename T, int FMT, int GROUPS>
 int launch_mid_moe(const MidMoeParams& p, hipStream_t st) {
+  const bool four = p.strips_each == 4;
   switch (p.moe.block_size) {
-    case 32: return launch_mid_rows<T, FMT, GROUPS, 2, false, true>(p, st);
-    case 48: return launch_mid_rows<T, FMT, GROUPS, 3, false, true>(p, st);
-    case 64: return launch_mid_rows<T, FMT, GROUPS, 4, false, true>(p, st);
+    case 32: return four ? launch_mid_rows<T, FMT, GROUPS, 2, false, true, 4>(p, st) : launch_mid_rows<T, FMT, GROUPS, 2, false, true>(p, st);
+    case 48: return four ? launch_mid_rows<T, FMT, GROUPS, 3, false, true, 4>(p, st) : launch_mid_rows<T, FMT, GROUPS, 3, false, true>(p, st);
+    case 64: return four ? launch_mid_rows<T, FMT, GROUPS, 4, false, true, 4>(p, st) : launch_mid_rows<T, FMT, GROUPS, 4, false, true>(p, st);
     default: return fail(SONAR_E_INVALID, "internal: blocks of %d slots", p.moe.block_size);
   }
 }
@@ -745,7 +750,8 @@ int launch_mid_moe_format(const MidMoeParams& p, int format, hipStream_t st) {
 int mid_moe_gemm(MidMoeParams p, int dtype, int format, int blocks, hipStream_t st) {
   p.splits = 1;
   p.tiles_m = blocks;
-  p.tiles = blocks * ((p.size_n / kStripN + mid_strips(2) - 1) / mid_strips(2));
+  p.strips_each = mid_moe_strips(p.moe.block_size, p.moe.rows_total / p.moe.num_experts, p.moe.num_experts, p.size_n, p.size_k, p.raw_codes, p.cus);
+  p.tiles = blocks * ((p.size_n / kStripN + p.strips_each - 1) / p.strips_each);
   p.split_steps = p.size_k / kMidStepK;
   return dtype == SONAR_DTYPE_F16 ? launch_mid_moe_format<_Float16>(p, format, st) : launch_mid_moe_format<__bf16>(p, format, st);
 }

@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <cmath>
+
 #include "gemm_plan.hpp"
 
 namespace sonar {
@@ -49,6 +51,7 @@ struct MidMoe {
 };
 struct MidMoeParams : MidParams {
   MidMoe moe;
+  int strips_each;   // of a workgroup: filled in by mid_moe_gemm
 };
 
 // Whether the kernel can run a call (no act-order gather; rows of a within 4 GiB; groups of 16, 32 or 64 * 2^i rows or
@@ -140,6 +143,28 @@ inline int mid_splits_16_rows(int64_t size_n, int64_t size_k, int cus) {
     if (us < best) best = us, splits = n;
   }
   return splits;
+}
+
+// Strips of a workgroup in a grouped call, two or four.  A round of workgroups takes as long as six steps beside its loop (start, first
+// bytes, the sum of the ranges), so that twice the columns and half the ranges, whose activations are copied half as often, pay where
+// rounds are many; in whole rounds, with the second blocks of uneven routing counted.  Fitted to both forms of 242 GEMMs of 23 to 57 slots
+// an expert (blocks of 48 and 64): 0.5 % slower than the better of the two, two strips always 16 %; at worst 1.2 times two strips.
+// Us, two -> four strips: 64 of 56, K = 2304, N = 6656, bf16 346 -> 242; 64 of 49, AWQ, 1664 x 8704 291 -> 220; 32 of 42, 1152 x 15360
+// 187 -> 132; 64 of 29, MXFP4, 640 x 2688 51 -> 35; 8 of 49, 1536 x 5888 26.5 -> 21.1; 16 of 52, 1152 x 1536, three quarters of a
+// round 14.9 -> 18.0.
+inline int mid_moe_strips(int64_t block_size, int64_t slots, int64_t num_experts, int64_t size_n, int64_t size_k, bool units, int cus) {
+  if (size_k < 512) return 2;   // (not timed)
+  const int64_t most = block_size * 7 / 8, even = block_size == 64 ? 44 : block_size * 5 / 8;
+  const double second = slots > even ? 0.0009 * (slots - even) * (slots - even) : 0.0;   // second blocks, for each first one
+  const double blocks = (double)num_experts * (slots <= most ? 1.0 + second : slots / most + 1);
+  double cost[2];
+  for (int four = 0; four < 2; ++four) {
+    const int64_t across = (size_n / 64 + (four ? 3 : 1)) / (four ? 4 : 2), ranges = four ? 2 : 4;
+    int64_t steps = (size_k / 64 + ranges - 1) / ranges;
+    if (units) steps = (steps + 1) & ~(int64_t)1;
+    cost[four] = std::ceil(blocks * across / cus - 0.1) * (6 + steps);
+  }
+  return cost[1] < 1.06 * cost[0] ? 4 : 2;
 }
 
 // `row_blocks`: 16-row blocks of a tile, 1 to 6.

@@ -539,20 +539,26 @@ using namespace sonar;
 //   fewer than half a round of workgroups of integer codes, or a quarter of MXFP4, are too few wavefronts here: 8 experts of
 //     51 slots, down 8448 x 1024 92 / 108; of 40, gate and up 1280 x 1024 30.1 / 32.6
 //   blocks of 32: as fast, but for half a round to a round: 16 of 22, down 5632 x 1152 91 / 83; with just half a round only from
-//     21 slots on (8 of 18, gate and up 3584 x 2048 36 / 40), and a full round has a second as soon as an expert has a second
-//     block: 32 of 25, down 8064 x 1024 192 / 200
+//     21 slots on (8 of 18, gate and up 3584 x 2048 36 / 40).  From a round on workgroups of four strips are 5 to 18 % of a layer
+//     faster, unless the decode kernel would end in the gated activation or many slots an expert and a long K make a second round of
+//     second blocks expensive (90 layers of 13 to 28 slots: 64 of 15, down 512 x 3712 88.3 / 71.6; 32 of 17, down 768 x 1664
+//     45.5 / 39.0; 16 of 28, MXFP4, down 6272 x 2432 139 / 128; 32 of 26, down 11776 x 2048 328 / 348; gated: 64 of 18, gate and up
+//     2048 x 7424 201 / 219)
 //   blocks of 48: 1.16 times as fast; 64 of 41, 1024 x 3584 312 / 245; 32 of 41, MXFP4, 1280 x 768 73 / 55
-//   blocks of 64, up to 56 slots an expert: 8 of 53, MXFP4, 4096 x 10752 281 / 217; integer codes are level or behind from one round
-//     to one and a quarter: 16 of 44, AWQ, gate and up 4096 x 2560 84 / 88
+//   blocks of 64, up to 56 slots an expert: 8 of 53, MXFP4, 4096 x 10752 281 / 217; 16 of 50, gate and up
+//     640 x 2560, one and a quarter rounds 53.4 / 44.8 (two strips a workgroup were level or behind there)
 // Against the tile kernels, up to 56 slots: always for one round (32 of 50, AWQ, down 2048 x 384 70 / 61), else as the rounds
 //   of both say, the second blocks of uneven routing counted.  A fit of 131 GEMMs: it loses 0.3 % of a layer on average against
 //   the better of the two; always here 2.6 %, never 5.9 %.  32 of 51, 2560 x 1280 147 / 110; but 64 of 56, AWQ, 3840 x 512
 //   143 / 174, and 32 of 56, down 1152 x 2048 93 / 102 (256 tiles, one round of them).
-// More slots: while it is one round of workgroups (8 of 79, 1536 x 640 62 / 41; 8 of 111, MXFP4, down 4864 x 1536 103 / 96).
+// More slots: while it is one round of workgroups (8 of 79, 1536 x 640 62 / 41; 8 of 111, MXFP4, down 4864 x 1536 103 / 96), of
+//   four strips up to 120 slots (16 of 106, MXFP4, down 5248 x 1280 132 / 109; 16 of 59, down 768 x 2560 56 / 47; 16 of 71, one and an
+//   eighth, 2560 x 2304 67 / 79).
+// Four strips and the 512 rows of K that they are given from (less was not timed) are in mid_moe_strips.
 // The general kernel (MXFP4 with K of no whole units) is never ahead: 16 of 35, 1472 x 704 54 / 37.
 // Blocks of 32 and 48 slots that are nearly full on average were not timed (the rule for block sizes makes none).
 static bool moe_mid_applies(int64_t moe_block_size, int64_t rows_total, int64_t num_experts, int64_t a_rows, int64_t size_n,
-                            int64_t size_k, int64_t num_groups, int group_size, bool fp4, bool decode, bool tiles) {
+                            int64_t size_k, int64_t num_groups, int group_size, bool fp4, bool decode, bool tiles, bool gated) {
   static const bool no_mid = getenv("SONAR_MARLIN_NO_MOE_MID") != nullptr;  // debugging aid
   if (no_mid || moe_block_size < 32 || !mid_applies(a_rows, size_k, size_k, num_groups, group_size)) return false;
   if (!fp4 && (size_k % 128 != 0 || (num_groups > 1 && group_size % 128 != 0))) return false;
@@ -562,11 +568,14 @@ static bool moe_mid_applies(int64_t moe_block_size, int64_t rows_total, int64_t 
   // rounds of workgroups (a pair of strips each) with the blocks there are where the routing is even
   const int64_t pairs = (size_n + 127) / 128;
   const double rounds = (double)(num_experts * (slots <= 56 ? 1 : slots / 56 + 1) * pairs) / cus;
-  if (slots > 56) return rounds <= 1.0;
+  const bool long_k = size_k >= 512;
+  if (slots > 56)
+    return rounds <= 1.0 || (long_k && slots <= 120 && num_experts * (slots / 56 + 1) * ((size_n + 255) / 256) <= cus);
   if (decode) {
-    if (moe_block_size == 32) return rounds >= 0.5 && (rounds > 0.5 || slots > 20) && rounds < 1.0;
+    if (moe_block_size == 32 && rounds >= 1.0) return !gated && long_k && (slots <= 22 || size_k <= 5120);
+    if (moe_block_size == 32) return rounds > 0.5 || (rounds == 0.5 && slots > 20);
     if (fp4) return rounds > 0.25;
-    return rounds >= 0.5 && (moe_block_size == 48 || rounds <= 1.0 || rounds > 1.25);
+    return rounds >= 0.5 && (moe_block_size == 48 || long_k || rounds <= 1.0 || rounds > 1.25);
   }
   if (moe_block_size == 32) return rounds >= 0.5 && rounds <= 1.0;
   if (moe_block_size == 48) return rounds >= 0.25;
@@ -739,7 +748,7 @@ int moe_gemm_any(
   // (Its scales are 16-byte loads, as in the dense call; the other kernels copy them in pieces of 4.)
   if (layer.topk_ids == nullptr && !bits8 && !row_groups && !nvfp4 && !has_perm && ((uintptr_t)b_scales) % 16 == 0 &&
       moe_mid_applies(moe_block_size, size_m * top_k, num_experts, a_rows, size_n, size_k, num_groups, group_size, fp4,
-                      decode, tiles)) {
+                      decode, tiles, layer.gated != nullptr)) {
     MidMoeParams m = {};
     m.a = static_cast<const uint16_t*>(a);
     m.lda = size_k;
@@ -753,6 +762,7 @@ int moe_gemm_any(
     if (!fp4 && num_groups > 1)
       for (int per = group_size / 64; per > 0; per >>= 1) ++m.group_shift;   // (moe_mid_applies: 64 * 2^i rows)
     m.chunks_per_strip = (int)(size_k / kChunkK);
+    m.cus = cu_count();
     m.raw_codes = !fp4;
     m.moe.sorted_ids = sorted_token_ids;
     m.moe.expert_ids = expert_ids;
@@ -904,7 +914,7 @@ extern "C" int sonar_moe_routed_gemm_applies(int64_t slots, int64_t moe_block_si
   return moe_fast_routes(slots, moe_block_size, num_experts) &&
          moe_fast_applies(false, moe_block_size, most_sorted(slots, moe_block_size, num_experts), num_experts, slots, size_n, size_k,
                           num_groups, group_size) &&
-         !moe_mid_applies(moe_block_size, slots, num_experts, slots, size_n, size_k, num_groups, group_size, fp4, true, false);
+         !moe_mid_applies(moe_block_size, slots, num_experts, slots, size_n, size_k, num_groups, group_size, fp4, true, false, true);
 }
 
 extern "C" int sonar_moe_routed_gemm(const void* a, void* c, const uint32_t* b_q_weight, int b_layout, const void* b_bias,

@@ -51,6 +51,27 @@ def test_mxfp4(tokens, k, n):
     _ran(tm.test_full_size_grouped_gemm_agrees_with_dense_rows, tokens, k, n, "mxfp4")
 
 
+# more than a round of workgroups of two strips: four strips a workgroup, the last of which has one, two and three of its own; K of an odd
+# number of units and of fewer steps in the second range; experts with second blocks
+FOUR = [(16, 200, 640, 4160, 32), (16, 296, 640, 2240, 48), (16, 400, 512, 2176, 64), (16, 400, 1152, 3136, 64), (8, 240, 1664, 1984, 64)]
+
+
+@pytest.mark.parametrize("e,m,k,n,slots", FOUR)
+@pytest.mark.parametrize("dtype,zp,group", [("fp16", False, 128), ("fp16", True, -1), ("bf16", True, 128), ("bf16", False, -1)])
+def test_four_strips(e, m, k, n, slots, dtype, zp, group):
+    _ran(tm.test_moe_gemm_within_tolerance, (m, e, 2, k, n, group, dtype, zp, False, zp, slots, not zp))
+
+
+def test_four_strips_act_order():
+    _ran(tm.test_moe_gemm_within_tolerance, (400, 16, 2, 640, 2240, 128, "bf16", False, True, True, 64, True))
+
+
+@pytest.mark.parametrize("tokens,n", [(100, 8256), (150, 5184), (190, 5248)])
+@pytest.mark.parametrize("k", [640, 1152])
+def test_four_strips_mxfp4(tokens, k, n):
+    _ran(tm.test_full_size_grouped_gemm_agrees_with_dense_rows, tokens, k, n, "mxfp4")
+
+
 # the edges of the rule: experts, tokens (top 2), K, N, slots of a block, zero points, and the kernel
 RULE = [(8, 72, 128, 2048, 32, False, "DECODE"), (8, 100, 128, 2048, 32, False, "MID"), (8, 100, 128, 2112, 32, False, "MID"), (8, 100, 128, 4096, 32, True, "DECODE"),
         (8, 120, 128, 1920, 48, True, "DECODE"), (8, 120, 128, 1984, 48, False, "MID"), (8, 120, 128, 8320, 48, False, "MID"),

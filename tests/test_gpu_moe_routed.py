@@ -53,7 +53,7 @@ def test_layer(kind, group, dtype, tokens, k, inter):
                                               activation=activation, w1_zeros=z1, w2_zeros=z2, **kw)
         got, want = layer(), layer(activation_func=fused_moe.apply_moe_activation)
         assert bool(torch.isfinite(want).all())
-        if activation == "silu":
+        if activation == "silu" or block == 32:   # (the layer with sorted slots may have run in the mid-size kernel, which adds in its order)
             # a value between the GEMMs, and one of the result, may be rounded the other way: one unit of their type each
             error = (got.double() - want.double()).norm() / want.double().norm()
             assert error < 2 * 2.0 ** -BITS[dtype], error
