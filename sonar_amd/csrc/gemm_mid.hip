@@ -61,6 +61,7 @@
 #include "common.hpp"
 #include "dequant.hpp"
 #include "gemm_mid.hpp"
+#include "moe_activation.hpp"
 
 namespace sonar {
 namespace {
@@ -150,7 +151,10 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
   // (Grouped: of the blocks that the routing has made, one after the other, so that those of an expert share its chunks.)
   const int strips = p.size_n / kStripN;
   const int tiles_m = GROUPED ? min(p.tiles_m, moe.num_post_pad[0] / moe.block_size) : p.tiles_m;
-  const int tiles = GROUPED ? tiles_m * ((strips + kMidStrips - 1) / kMidStrips) : p.tiles;
+  constexpr int kOfHalf = kMidStrips > 1 ? kMidStrips / 2 : 1;
+  const bool halves = GROUPED && moe.gated != nullptr && moe.gated_halves;
+  const int across = halves ? strips / 2 : strips, each = halves ? kOfHalf : kMidStrips;
+  const int tiles = GROUPED ? tiles_m * ((across + each - 1) / each) : p.tiles;
   const int units = tiles * p.splits, per_xcd = (units + 7) / 8;
   const int unit = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
   if ((int)(blockIdx.x >> 3) >= per_xcd || unit >= units) return;
@@ -160,8 +164,10 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
   const int expert = GROUPED ? moe.expert_ids[tile_m] : 0;
   if (GROUPED && (unsigned)expert >= (unsigned)moe.num_experts) return;
   // (the second strip of an odd last pair is the first again, and not stored)
-  const bool active = tile_n * kMidStrips + strip_of < strips;
-  const int strip = __builtin_amdgcn_readfirstlane(active ? tile_n * kMidStrips + strip_of : strips - 1);
+  // (halves: the first strips are of the gate half, the others the same columns of the up half)
+  const int of_tile = halves ? strip_of % kOfHalf : strip_of;
+  const bool active = tile_n * each + of_tile < across;
+  const int strip = __builtin_amdgcn_readfirstlane((active ? tile_n * each + of_tile : across - 1) + (halves ? strip_of / kOfHalf * across : 0));
 
   const int first = split * p.split_steps;   // of the steps this workgroup takes
   const int steps = min(first + p.split_steps, p.size_k / kMidStepK);
@@ -558,6 +564,42 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
   // Row and first of four columns of a tile that a lane adds.  With kSwap a lane holds rows 4 kb .. + 3 of column col16 and
   // stores them so that four columns of a row lie together; rows change places between the kb, off each other's banks.
   const int tile_row = kSwap ? 4 * kb + ((col16 >> 2) ^ kb) : col16, tile_col = 4 * (kSwap ? lane & 3 : kb);
+  // The gated activation of a column of the gate half and the same of the up half, rounded as the results would be: the wavefronts of a
+  // pair of strips share its tiles.  (Against a launch of 5 to 8 us that reads and writes C: 185 layers 2.5 % less time, 32 experts of
+  // 42 rows, 1152 x 7680 207 -> 202 us, 8 of 52, 2560 x 3968 80.6 -> 77.6.)
+  auto finish_halves = [&](const int round) __attribute__((always_inline)) {
+    const int worker = 2 * range + strip_of / kOfHalf, first_tile = tile_n * kOfHalf + of_tile;
+    if (!active) return;
+    for (int q = worker; q < 4 * kSum; q += 2 * kMidRanges) {
+      const int i = round + (q >> 2), j = q & 3;
+      const int slot = m0 + 16 * i + tile_row;
+      int row = i < MB && slot < moe.sorted_len ? moe.sorted_ids[slot] : moe.rows_total;
+      if ((unsigned)row >= (unsigned)moe.rows_total) continue;   // padding slot
+      const float row_w = moe.mul_topk ? Dq<T>::to_float(Dq<T>::from_float(moe.topk_weights[row])) : 1.f;
+      const int nl = 16 * j + tile_col;
+      uint16_t n[2][4];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        floatx4_t v = floatx4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int g = 0; g < kMidRanges; ++g) {
+          const float4 s = sums[(((kMidStrips * g + h * kOfHalf + of_tile) * kSum + (q >> 2)) * 4 + j) * 64 + lane];
+          v += floatx4_t{s.x, s.y, s.z, s.w};
+        }
+        const uint16_t* bias_row = p.bias ? p.bias + expert * moe.expert_bias_stride + (first_tile + h * across) * kStripN : nullptr;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          n[h][r] = Dq<T>::from_float(v[r] + (bias_row ? Dq<T>::to_float(bias_row[scale_slot(nl + r, false)]) : 0.f));
+          if (moe.mul_topk) n[h][r] = Dq<T>::from_float(Dq<T>::to_float(n[h][r]) * row_w);
+        }
+      }
+      uint16_t o[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[r] = silu_times<T>(n[0][r], n[1][r]);
+      *reinterpret_cast<uint2*>(moe.gated + (size_t)row * (p.size_n / 2) + first_tile * kStripN + nl) =
+          make_uint2((uint32_t)o[0] | ((uint32_t)o[1] << 16), (uint32_t)o[2] | ((uint32_t)o[3] << 16));
+    }
+  };
 #pragma unroll
   for (int round = 0; round < MB; round += kSum) {
     if (round > 0) __syncthreads();
@@ -576,6 +618,12 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
           }
         }
     __syncthreads();
+    if constexpr (GROUPED) {
+      if (halves) {
+        finish_halves(round);
+        continue;
+      }
+    }
 #pragma unroll
     for (int u = 0; u < (kMidRanges == 2 ? 2 * kSum : kSum); ++u) {
       constexpr int kEach = kSum * 4 / kMidRanges;   // accumulator tiles a wavefront adds
@@ -621,6 +669,14 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
       for (int r = 0; r < 4; ++r) {
         n[r] = Dq<T>::from_float(v[r] + bias[r]);
         if (GROUPED && moe.mul_topk) n[r] = Dq<T>::from_float(Dq<T>::to_float(n[r]) * row_w);
+      }
+      if constexpr (GROUPED) {
+        if (moe.gated != nullptr) {
+          *reinterpret_cast<uint32_t*>(moe.gated + (size_t)row * (p.size_n / 2) + (strip * kStripN + nl) / 2) =
+              (uint32_t)swiglu_oai<T>(n[0], n[1], moe.gated_limit, moe.gated_alpha) |
+              ((uint32_t)swiglu_oai<T>(n[2], n[3], moe.gated_limit, moe.gated_alpha) << 16);
+          continue;
+        }
       }
       const uint2 o = make_uint2((uint32_t)n[0] | ((uint32_t)n[1] << 16), (uint32_t)n[2] | ((uint32_t)n[3] << 16));
       *reinterpret_cast<uint2*>(p.c + (size_t)row * p.size_n + strip * kStripN + nl) = o;
@@ -751,7 +807,8 @@ int mid_moe_gemm(MidMoeParams p, int dtype, int format, int blocks, hipStream_t 
   p.splits = 1;
   p.tiles_m = blocks;
   p.strips_each = mid_moe_strips(p.moe.block_size, p.moe.rows_total / p.moe.num_experts, p.moe.num_experts, p.size_n, p.size_k, p.raw_codes, p.cus);
-  p.tiles = blocks * ((p.size_n / kStripN + p.strips_each - 1) / p.strips_each);
+  const int halves = p.moe.gated != nullptr && p.moe.gated_halves ? 2 : 1, across = p.size_n / kStripN / halves, each = p.strips_each / halves;
+  p.tiles = blocks * ((across + each - 1) / each);
   p.split_steps = p.size_k / kMidStepK;
   return dtype == SONAR_DTYPE_F16 ? launch_mid_moe_format<_Float16>(p, format, st) : launch_mid_moe_format<__bf16>(p, format, st);
 }

@@ -48,6 +48,11 @@ struct MidMoe {
   int a_by_slot;               // row of A = slot (a column-permuted copy made per slot), else row id / top_k
   long expert_b_stride;        // uint4 units between experts in b
   long expert_s_stride, expert_z_stride, expert_bias_stride;   // elements between experts
+  // if not null: the gated activation of C, (rows_total, size_n / 2), in place of C.  `gated_halves`: silu_and_mul, a workgroup has
+  // as many strips of the gate half as of the up half; else swigluoai, whose gate and up columns alternate
+  uint16_t* gated;
+  int gated_halves;
+  float gated_limit, gated_alpha;
 };
 struct MidMoeParams : MidParams {
   MidMoe moe;

@@ -72,6 +72,30 @@ def test_four_strips_mxfp4(tokens, k, n):
     _ran(tm.test_full_size_grouped_gemm_agrees_with_dense_rows, tokens, k, n, "mxfp4")
 
 
+# the gated activation where the ranges meet: the bits of the layer whose activation is a launch of its own.  Blocks of 48 and 64 slots, of
+# 32 with less than a round; two and four strips a workgroup, an odd number of strips in a half, experts with second blocks
+@pytest.mark.parametrize("kind,group,dtype", [("uint4b8", 128, torch.float16), ("uint4", 128, torch.bfloat16), ("mxfp4", 32, torch.bfloat16)])
+@pytest.mark.parametrize("e,tokens,k,inter", [(8, 92, 512, 1344), (8, 150, 512, 960), (8, 200, 1152, 832), (16, 296, 640, 1344), (16, 400, 1152, 1600),
+                                              (4, 250, 640, 1088)])
+def test_gated_activation(e, tokens, k, inter, kind, group, dtype):
+    from sonar_amd import fused_moe
+    from sonar_amd.scalar_type import scalar_types
+    from tests.test_gpu_moe_routed import _experts
+    gen = torch.Generator(device=gu.DEV).manual_seed(tokens + k)
+    w1, s1, z1 = _experts(gen, kind, e, k, 2 * inter, group, dtype)
+    w2, s2, z2 = _experts(gen, kind, e, inter, k, min(group, 64), dtype)
+    bias1 = (torch.randn((e, 2 * inter), device=gu.DEV, generator=gen) * 0.1).to(dtype)
+    x = torch.randn((tokens, k), device=gu.DEV, generator=gen).to(dtype) * 0.1
+    weights, ids = torch.topk(torch.softmax(torch.randn((tokens, e), device=gu.DEV, generator=gen), dim=1), 2, dim=1)
+    wtype = {"uint4b8": scalar_types.uint4b8, "uint4": scalar_types.uint4, "mxfp4": scalar_types.float4_e2m1f}[kind]
+    for activation, on_input in (("swigluoai", False), ("silu", False), ("silu", True)):
+        def layer(**kw):
+            return fused_moe.fused_marlin_moe(x, w1, w2, bias1, None, s1, s2, weights.contiguous(), ids.to(torch.int32), wtype.id, on_input,
+                                              activation=activation, w1_zeros=z1, w2_zeros=z2, **kw)
+        got, want = layer(), layer(activation_func=fused_moe.apply_moe_activation)
+        assert bool(torch.isfinite(want).all()) and torch.equal(got, want), activation
+
+
 # the edges of the rule: experts, tokens (top 2), K, N, slots of a block, zero points, and the kernel
 RULE = [(8, 72, 128, 2048, 32, False, "DECODE"), (8, 100, 128, 2048, 32, False, "MID"), (8, 100, 128, 2112, 32, False, "MID"), (8, 100, 128, 4096, 32, True, "DECODE"),
         (8, 120, 128, 1920, 48, True, "DECODE"), (8, 120, 128, 1984, 48, False, "MID"), (8, 120, 128, 8320, 48, False, "MID"),
