@@ -8,7 +8,8 @@
 // which the two strips share, are staged in LDS at half the bytes per matrix instruction of a one-strip
 // workgroup (at one strip the copies alone would need the whole 64 bytes per clock of a compute unit).  Grouped calls of
 // many rounds of workgroups take four strips x two ranges (mid_moe_strips): start, end and the sum of the ranges once for twice the columns,
-// and half the copies (32 experts of 42 rows, K = 1152, N = 15360: 187 -> 132 us).
+// and half the copies (32 experts of 42 rows, K = 1152, N = 15360: 187 -> 132 us); so do 64-row tiles of 4-bit integers in more than a
+// round (M 327, K 1408, N 16704, fp16: 33.6 -> 22.6 with the host; M 110, K 3200, N 24576, bf16: 37.2 -> 31.3).
 //
 // What bounds it: the sum of vector and matrix instructions, which two wavefronts a SIMD overlap in part, and the start and the
 // end.  (Counters at 64 to 333 rows: of the busy cycles vector issue fills 41 to 48 % and the matrix pipes 26 to 38 %; without
@@ -725,11 +726,13 @@ int launch_mid_rows(const typename std::conditional<GROUPED, MidMoeParams, MidPa
 }
 
 template <typename T, int FMT, int GROUPS>
-int launch_mid_raw(const MidParams& p, int row_blocks, hipStream_t st) {
+int launch_mid_raw(const MidParams& p, int row_blocks, int strips, hipStream_t st) {
   switch (row_blocks) {
     case 2: return launch_mid_rows<T, FMT, GROUPS, 2>(p, st);
     case 3: return launch_mid_rows<T, FMT, GROUPS, 3>(p, st);
-    default: return launch_mid_rows<T, FMT, GROUPS, kMidMostRawRows>(p, st);
+    default:
+      if (strips == 4) return launch_mid_rows<T, FMT, GROUPS, kMidMostRawRows, false, false, 4>(p, st);
+      return launch_mid_rows<T, FMT, GROUPS, kMidMostRawRows>(p, st);
   }
 }
 
@@ -750,14 +753,14 @@ int launch_mid(const MidParams& p, int row_blocks, hipStream_t st) {
 }
 
 template <typename T, int FMT>
-int launch_mid_groups(const MidParams& p, int row_blocks, hipStream_t st) {
+int launch_mid_groups(const MidParams& p, int row_blocks, int strips, hipStream_t st) {
   if constexpr (FMT == kMidMxFp4 || FMT == kMidNvFp4) {
     return launch_mid<T, FMT, kChunkGroups>(p, row_blocks, st);
   } else {
     if constexpr (FMT == kMidInt4 || FMT == kMidInt4Zp) {
       if (p.raw_codes)
-        return p.num_groups == 1 ? launch_mid_raw<T, FMT, kOneGroupRaw>(p, row_blocks, st)
-                                 : launch_mid_raw<T, FMT, kUnitGroupsRaw>(p, row_blocks, st);
+        return p.num_groups == 1 ? launch_mid_raw<T, FMT, kOneGroupRaw>(p, row_blocks, strips, st)
+                                 : launch_mid_raw<T, FMT, kUnitGroupsRaw>(p, row_blocks, strips, st);
     }
     if (p.num_groups == 1) return launch_mid<T, FMT, kOneGroup>(p, row_blocks, st);
     if (p.group_shift >= 0) return launch_mid<T, FMT, kStepGroups>(p, row_blocks, st);
@@ -766,15 +769,15 @@ int launch_mid_groups(const MidParams& p, int row_blocks, hipStream_t st) {
 }
 
 template <typename T>
-int launch_mid_format(const MidParams& p, int format, int row_blocks, hipStream_t st) {
+int launch_mid_format(const MidParams& p, int format, int row_blocks, int strips, hipStream_t st) {
   switch (format) {
-    case kMidInt4: return launch_mid_groups<T, kMidInt4>(p, row_blocks, st);
-    case kMidInt4Zp: return launch_mid_groups<T, kMidInt4Zp>(p, row_blocks, st);
-    case kMidInt8: return launch_mid_groups<T, kMidInt8>(p, row_blocks, st);
-    case kMidFp8: return launch_mid_groups<T, kMidFp8>(p, row_blocks, st);
-    case kMidNvFp4: return launch_mid_groups<T, kMidNvFp4>(p, row_blocks, st);
+    case kMidInt4: return launch_mid_groups<T, kMidInt4>(p, row_blocks, strips, st);
+    case kMidInt4Zp: return launch_mid_groups<T, kMidInt4Zp>(p, row_blocks, strips, st);
+    case kMidInt8: return launch_mid_groups<T, kMidInt8>(p, row_blocks, strips, st);
+    case kMidFp8: return launch_mid_groups<T, kMidFp8>(p, row_blocks, strips, st);
+    case kMidNvFp4: return launch_mid_groups<T, kMidNvFp4>(p, row_blocks, strips, st);
     default:   // MXFP4: bf16 only, which the caller has checked
-      if constexpr (std::is_same<T, __bf16>::value) return launch_mid_groups<T, kMidMxFp4>(p, row_blocks, st);
+      if constexpr (std::is_same<T, __bf16>::value) return launch_mid_groups<T, kMidMxFp4>(p, row_blocks, strips, st);
       return fail(SONAR_E_INVALID, "internal: MXFP4 weights with float16 activations");
   }
 }
@@ -819,13 +822,15 @@ int mid_gemm(MidParams p, int dtype, int format, int row_blocks, hipStream_t st)
   if (row_blocks < 2 && (format == kMidInt4 || format == kMidInt4Zp || format == kMidMxFp4)) row_blocks = 2;
   if (p.raw_codes) row_blocks = std::min(row_blocks, kMidMostRawRows);
   p.tiles_m = (p.size_m + 16 * row_blocks - 1) / (16 * row_blocks);
-  p.tiles = p.tiles_m * ((strips + mid_strips(row_blocks) - 1) / mid_strips(row_blocks));
+  const bool by_rounds = p.raw_codes && row_blocks == kMidMostRawRows && p.splits == 1;
+  const int each = by_rounds ? mid_strips_by_rounds(p.tiles_m, 0.0, p.size_n, p.size_k, true, p.cus) : mid_strips(row_blocks);
+  p.tiles = p.tiles_m * ((strips + each - 1) / each);
   const int steps = p.size_k / kMidStepK;
   p.split_steps = (steps + p.splits - 1) / p.splits;
   if (p.raw_codes) p.split_steps = (p.split_steps + 1) & ~1;   // whole units of 128 rows
   p.splits = (steps + p.split_steps - 1) / p.split_steps;
-  const int rc = dtype == SONAR_DTYPE_F16 ? launch_mid_format<_Float16>(p, format, row_blocks, st)
-                                          : launch_mid_format<__bf16>(p, format, row_blocks, st);
+  const int rc = dtype == SONAR_DTYPE_F16 ? launch_mid_format<_Float16>(p, format, row_blocks, each, st)
+                                          : launch_mid_format<__bf16>(p, format, row_blocks, each, st);
   if (rc || p.splits == 1) return rc;
   const int blocks = (int)std::min<int64_t>(((int64_t)p.size_m * p.size_n / 4 + 255) / 256, 2048);
   if (p.splits > kMidMostSplits) return fail(SONAR_E_INVALID, "internal: %d K splits", p.splits);

@@ -68,6 +68,25 @@ inline bool mid_applies(int64_t size_m, int64_t size_k, int64_t lda, int64_t num
   return group_size % 64 == 0 && (per & (per - 1)) == 0;
 }
 
+// Strips of a workgroup, two or four, in a grouped call and in dense 64-row tiles of raw codes with K in one piece.  A round of workgroups takes as long as six steps beside its loop (start, first
+// bytes, the sum of the ranges), so that twice the columns and half the ranges, whose activations are copied half as often, pay where
+// rounds are many; in whole rounds, with the second blocks of uneven routing counted.  Fitted to both forms of 242 GEMMs of 23 to 57 slots
+// an expert (blocks of 48 and 64): 0.5 % slower than the better of the two, two strips always 16 %; at worst 1.2 times two strips.
+// Us, two -> four strips: 64 of 56, K = 2304, N = 6656, bf16 346 -> 242; 64 of 49, AWQ, 1664 x 8704 291 -> 220; 32 of 42, 1152 x 15360
+// 187 -> 132; 64 of 29, MXFP4, 640 x 2688 51 -> 35; 8 of 49, 1536 x 5888 26.5 -> 21.1; 16 of 52, 1152 x 1536, three quarters of a
+// round 14.9 -> 18.0.
+inline int mid_strips_by_rounds(double row_tiles, double slack, int64_t size_n, int64_t size_k, bool units, int cus) {
+  if (size_k < 512) return 2;   // (not timed)
+  double cost[2];
+  for (int four = 0; four < 2; ++four) {
+    const int64_t across = (size_n / 64 + (four ? 3 : 1)) / (four ? 4 : 2), ranges = four ? 2 : 4;
+    int64_t steps = (size_k / 64 + ranges - 1) / ranges;
+    if (units) steps = (steps + 1) & ~(int64_t)1;
+    cost[four] = std::ceil(row_tiles * across / cus - slack) * (6 + steps);
+  }
+  return cost[1] < 1.06 * cost[0] ? 4 : 2;
+}
+
 // Microseconds a call takes in tiles of the best number of row blocks and splits of K, which are returned in
 // `row_blocks` and `splits`.  A fit of measured times (K = 2048 and 4096, N = 2048, 6144 and 20032, 17 to 768 rows, all
 // formats, on weights that a cache holds, mostly within 15 %; from memory two rounds of tiles take 15 to 20 % more): 4 us
@@ -98,6 +117,12 @@ inline double mid_estimate(int64_t size_m, int64_t size_n, int64_t size_k, int64
       if (raw_codes) {   // (one round: slower the more bytes its weights are)
         const double slow = rounds > 1 ? 0.95 : (2 * groups > cus ? 0.86 : 0.8) + 2.5e-9 * size_n * size_k;
         us = 1.4 + rounds * (2.4 + 0.3 * mb + k * (raw[0] + raw[1] * mb) * slow);
+        if (mb == kMidMostRawRows && n == 1 && mid_strips_by_rounds((double)((size_m + 16 * mb - 1) / (16 * mb)), 0.0, size_n, size_k, true, cus) == 4) {
+          const int64_t fours = ((size_m + 16 * mb - 1) / (16 * mb)) * ((size_n + 255) / 256), rounds4 = (fours + cus - 1) / cus;
+          const double k4 = 2 * ((steps / 2 + 1) / 2) * 256 / 4096.0;
+          const double slow4 = rounds4 > 1 ? 0.95 : (2 * fours > cus ? 0.86 : 0.8) + 2.5e-9 * size_n * size_k;
+          us = 1.4 + rounds4 * (2.4 + 0.3 * mb + k4 * (raw[0] + raw[1] * mb) * slow4);
+        }
       }
       if (us < memory) us = memory;
       if (n > 1) us += raw_codes ? 3.0 + 1.6e-6 * n * size_m * size_n : 3.3 + 2e-6 * n * size_m * size_n;
@@ -150,26 +175,10 @@ inline int mid_splits_16_rows(int64_t size_n, int64_t size_k, int cus) {
   return splits;
 }
 
-// Strips of a workgroup in a grouped call, two or four.  A round of workgroups takes as long as six steps beside its loop (start, first
-// bytes, the sum of the ranges), so that twice the columns and half the ranges, whose activations are copied half as often, pay where
-// rounds are many; in whole rounds, with the second blocks of uneven routing counted.  Fitted to both forms of 242 GEMMs of 23 to 57 slots
-// an expert (blocks of 48 and 64): 0.5 % slower than the better of the two, two strips always 16 %; at worst 1.2 times two strips.
-// Us, two -> four strips: 64 of 56, K = 2304, N = 6656, bf16 346 -> 242; 64 of 49, AWQ, 1664 x 8704 291 -> 220; 32 of 42, 1152 x 15360
-// 187 -> 132; 64 of 29, MXFP4, 640 x 2688 51 -> 35; 8 of 49, 1536 x 5888 26.5 -> 21.1; 16 of 52, 1152 x 1536, three quarters of a
-// round 14.9 -> 18.0.
 inline int mid_moe_strips(int64_t block_size, int64_t slots, int64_t num_experts, int64_t size_n, int64_t size_k, bool units, int cus) {
-  if (size_k < 512) return 2;   // (not timed)
   const int64_t most = block_size * 7 / 8, even = block_size == 64 ? 44 : block_size * 5 / 8;
   const double second = slots > even ? 0.0009 * (slots - even) * (slots - even) : 0.0;   // second blocks, for each first one
-  const double blocks = (double)num_experts * (slots <= most ? 1.0 + second : slots / most + 1);
-  double cost[2];
-  for (int four = 0; four < 2; ++four) {
-    const int64_t across = (size_n / 64 + (four ? 3 : 1)) / (four ? 4 : 2), ranges = four ? 2 : 4;
-    int64_t steps = (size_k / 64 + ranges - 1) / ranges;
-    if (units) steps = (steps + 1) & ~(int64_t)1;
-    cost[four] = std::ceil(blocks * across / cus - 0.1) * (6 + steps);
-  }
-  return cost[1] < 1.06 * cost[0] ? 4 : 2;
+  return mid_strips_by_rounds((double)num_experts * (slots <= most ? 1.0 + second : slots / most + 1), 0.1, size_n, size_k, units, cus);
 }
 
 // `row_blocks`: 16-row blocks of a tile, 1 to 6.

@@ -292,7 +292,7 @@ KERNEL_FORMS = {
     "moe_align_count_kernel": 2, "moe_align_place_kernel": 1, "moe_permute_rows_kernel": 1,
     "moe_sum_kernel": 2, "moe_tile_reduce_kernel": 2, "moe_tile_table_kernel": 2, "per_token_quant_kernel": 6,
     "permute_columns_kernel": 1, "silu_and_mul_kernel": 2, "tile_reduce_kernel": 2, "to_marlin_a8_kernel": 3,
-    "marlin_mid_gemm": 241, "marlin_mid_sum": 4, "marlin_a8_block": 59, "load_linear_kernel": 4, "sort_group_indices": 1,
+    "marlin_mid_gemm": 249, "marlin_mid_sum": 4, "marlin_a8_block": 59, "load_linear_kernel": 4, "sort_group_indices": 1,
     "permute_scale_columns": 2,
     "pack_zero_points": 1, "awq_to_plain_kernel": 1,
 }
