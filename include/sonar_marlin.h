@@ -562,6 +562,10 @@ double sonar_debug_tile_estimate(int64_t size_m, int64_t size_n, int64_t size_k)
  * no rows: it runs otherwise. */
 int64_t sonar_debug_twin_schedule(int64_t size_m, int64_t size_n, int64_t size_k, int64_t num_groups, int dtype, int format,
                                   int32_t* out, int64_t out_rows);
+/* Whether a grouped call that the wide tile kernels take runs so (1); rows_total: the rows of C, sorted_len: the slots given, may_split:
+ * whether there is room for K in ranges; -1 for arguments out of range. */
+int sonar_debug_moe_twin(int64_t rows_total, int64_t sorted_len, int64_t num_experts, int64_t size_n, int64_t size_k,
+                         int64_t num_groups, int dtype, int format, int may_split);
 /* Which of the two that choice falls on (1: marlin_mid_gemm) for a call of more than 64 rows that either could run, integer or
  * fp8 codes, 256 compute units; -1 for arguments out of range. */
 int sonar_debug_mid_beats_tiles(int64_t size_m, int64_t size_n, int64_t size_k, int64_t num_groups, int dtype,

@@ -39,6 +39,7 @@ PROTOTYPES = {
     "sonar_debug_moe_tile_schedule": (c_int64, [c_int64, c_int64, c_int64, c_int64, c_int, c_void_p, c_int64]),
     "sonar_debug_moe_pair_schedule": (c_int64, [c_int64, c_int64, c_int64, c_int64, c_int64, c_int, c_void_p, c_void_p, c_int64]),
     "sonar_debug_twin_schedule": (c_int64, [c_int64] * 4 + [c_int, c_int, c_void_p, c_int64]),
+    "sonar_debug_moe_twin": (c_int, [c_int64] * 6 + [c_int] * 3),
     "sonar_debug_tile_estimate": (c_double, [c_int64] * 3),
     "sonar_debug_mid_beats_tiles": (c_int, [c_int64] * 4 + [c_int, c_int64]),
     "sonar_gptq_marlin_repack": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int, c_void_p]),

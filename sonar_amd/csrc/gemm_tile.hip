@@ -2419,6 +2419,24 @@ size_t moe_tile_partial_bytes(int64_t size_k) {
   return moe_partial_bytes_of(kTileM) + moe_partial_bytes_of(128);
 }
 
+// Two 128-row tiles at a time, which hide each other's start and end, instead: always up to 160 rows an expert, whose tiles have 128
+// rows either way; with more, while the second dequantisation of the weights (integers in bf16 twice the instructions of float16 and
+// MXFP4) costs less than that; not where K is long and the tiles fill half of the compute units, which K in ranges does.  Us a layer, two
+// sizes -> here, over 325 random layers of 8 to 64 experts 0.91 times (0.74 to 1.04): 32 experts of 71 rows 2560 x 1152 225 -> 180; 16
+// MXFP4 of 97, 2688 x 10880 404 -> 361; 16 of 632, 1280 x 2688 270 -> 233; 64 MXFP4 of 500, 2048 x 768 398 -> 342; 32 MXFP4 of 250,
+// 2880 x 2880 457 -> 429.  Left out: Mixtral-8x7B shapes, bf16, 500 and 1024 rows 1267 -> 1360 and 2417 -> 2529; 16 of 453, bf16, AWQ,
+// 3968 x 7040 1112 -> 1157; 8 of 200, fp16, 7168 x 7168 505 -> 518; 8 of 116, 2048 x 5888 137 -> 141.
+// (The offsets of A have 32 bits: its rows are slots, at most sorted_len of them, or row ids / top_k, and a list of slots may be shorter
+// than the rows that its ids reach.)
+static bool moe_twin_tiles(const TileParams& q, int64_t sorted_len, int64_t num_experts, int bits, bool fp4, bool nvfp4, bool float16,
+                           bool may_split) {
+  const int64_t a_rows = std::max<int64_t>(sorted_len, q.rows_total);
+  if (!tile_twin_applies(bits, nvfp4, q.num_groups, q.group_size, q.size_k) || a_rows * q.size_k * 2 >= (1LL << 32)) return false;
+  const int64_t tiles = (q.rows_total / 128 + num_experts / 2) * q.tiles_n;
+  if (may_split && tiles < 128 && q.size_k >= 2048) return false;
+  return q.rows_total <= 160 * num_experts || q.size_k <= (fp4 ? 8192 : float16 ? 6144 : 3072);
+}
+
 // Called by sonar_moe_wna16_marlin_gemm for 64-slot blocks without act-order
 // when group_size % 64 == 0 (or one group) and size_k % 64 == 0.
 int moe_tile_gemm(const void* a, void* c, const uint32_t* b, const void* bias, const void* scales,
@@ -2486,18 +2504,8 @@ int moe_tile_gemm(const void* a, void* c, const uint32_t* b, const void* bias, c
   auto may_cut = [](const TileParams& q) {
     return (int64_t)(q.rows_total + 255) / 256 * q.tiles_n <= (q.size_k >= 64 * kTileK ? 512 : 192);
   };
-  // Two 128-row tiles at a time, which hide each other's start and end, instead: always up to 160 rows an expert, whose tiles have 128
-  // rows either way; with more, while the second dequantisation of the weights (integers in bf16 twice the instructions of float16 and
-  // MXFP4) costs less than that; not where K is long and the tiles fill half of the compute units, which K in ranges does.  Us a layer, two
-  // sizes -> here, over 325 random layers of 8 to 64 experts 0.91 times (0.74 to 1.04): 32 experts of 71 rows 2560 x 1152 225 -> 180; 16
-  // MXFP4 of 97, 2688 x 10880 404 -> 361; 16 of 632, 1280 x 2688 270 -> 233; 64 MXFP4 of 500, 2048 x 768 398 -> 342; 32 MXFP4 of 250,
-  // 2880 x 2880 457 -> 429.  Left out: Mixtral-8x7B shapes, bf16, 500 and 1024 rows 1267 -> 1360 and 2417 -> 2529; 16 of 453, bf16, AWQ,
-  // 3968 x 7040 1112 -> 1157; 8 of 200, fp16, 7168 x 7168 505 -> 518; 8 of 116, 2048 x 5888 137 -> 141.
   auto is_twin = [&](const TileParams& q, bool may_split) {
-    if (!tile_twin_applies(bits, nvfp4, q.num_groups, q.group_size, q.size_k) || sorted_len * q.size_k * 2 >= (1LL << 32)) return false;
-    const int64_t tiles = (q.rows_total / 128 + num_experts / 2) * q.tiles_n;
-    if (may_split && tiles < 128 && q.size_k >= 2048) return false;
-    return q.rows_total <= 160 * num_experts || q.size_k <= (fp4 ? 8192 : dtype == SONAR_DTYPE_F16 ? 6144 : 3072);
+    return moe_twin_tiles(q, sorted_len, num_experts, bits, fp4, nvfp4, dtype == SONAR_DTYPE_F16, may_split);
   };
   if (two_sizes && !may_cut(p)) p.partial = nullptr;
   const bool twin = two_sizes && is_twin(p, p.partial != nullptr);
@@ -2646,6 +2654,22 @@ extern "C" int64_t sonar_debug_twin_schedule(int64_t size_m, int64_t size_n, int
                                                num_groups, group_size, &never_read, ~(size_t)0, format == 1, false, 4, false,
                                                dtype == SONAR_DTYPE_F16);
   return plan.twin ? schedule_rows(plan.launch, plan.launch, 0, out, out_rows, 0) : 0;
+}
+
+// Whether a grouped call that the wide tile kernels take runs as 128-row tiles two at a time.
+extern "C" int sonar_debug_moe_twin(int64_t rows_total, int64_t sorted_len, int64_t num_experts, int64_t size_n, int64_t size_k,
+                                    int64_t num_groups, int dtype, int format, int may_split) {
+  using namespace sonar;
+  if (rows_total <= 0 || rows_total >= (1LL << 30) || size_n <= 0 || size_k <= 0 || size_k % kTileK != 0 || num_groups < 1 ||
+      size_k % num_groups != 0)
+    return -1;
+  TileParams q = {};
+  q.rows_total = (int)rows_total;
+  q.size_k = (int)size_k;
+  q.num_groups = (int)num_groups;
+  q.group_size = (int)(size_k / num_groups);
+  q.tiles_n = (int)((size_n + kTileN - 1) / kTileN);
+  return moe_twin_tiles(q, sorted_len, num_experts, 4, format == 1, false, dtype == SONAR_DTYPE_F16, may_split != 0) ? 1 : 0;
 }
 
 // A dense call (4-bit integer codes, no act-order) with room for every partial tile, as the other tile kernels run it.

@@ -35,6 +35,15 @@ def test_which_calls_and_what_their_tiles_cover(m, k, n, groups, dtype, fp4, twi
         _check_cover(rows, {128: set(range(-(-m // 128)))}, -(-n // 256), k // 64)
 
 
+@pytest.mark.parametrize("rows,slots,k,twin", [
+    (1 << 19, (1 << 19) + 64, 2048, True), (1 << 20, (1 << 20) + 64, 2048, False),
+    (1 << 20, 64 * 8, 2048, False),       # few slots given, whose ids reach rows of A behind the first 4 GiB
+    ((1 << 20) - 1, 64 * 8, 2048, True),  # (the last row ends there)
+    (1000, 1 << 20, 2048, False)])        # many slots of few rows: a copy of A by slot
+def test_rows_of_a_lie_within_32_bits(rows, slots, k, twin):
+    assert _lib.load().sonar_debug_moe_twin(rows, slots, 8, 4096, k, k // 64, _lib.DTYPE_F16, 0, 0) == twin
+
+
 def test_accumulators_stay_in_place(tmp_path):
     """The matrix instructions are asm statements, around which the compiler pads no hazard: an accumulator that it moved out of its
     registers around the loop would be read before the last sums have arrived."""
