@@ -1414,7 +1414,10 @@ void fused_moe(Tensor& output, const Tensor& hidden, const Tensor& w1, const Ten
            !(b_type_id == SONAR_TYPE_FLOAT4_E2M1F && !is_mx_scale_type(scale)) &&
            sonar_moe_routed_gemm_applies(rows, block_size, w.size(0), b_type_id, size_n, size_k, scale.size(1));
   };
-  if (m > 0 && routes(w1, scale1, perm1, 2 * n, k) && routes(w2, scale2, perm2, k, n)) {
+  // (They take every expert whose matrices they hold.  Where num_experts is smaller the sorting leaves the others' slots out, and a
+  // number past its range is refused there.)
+  const bool all_experts = w1.dim() == 3 && num_experts >= std::max(w1.size(0), w2.size(0)) && num_experts <= 8192;
+  if (m > 0 && all_experts && routes(w1, scale1, perm1, 2 * n, k) && routes(w2, scale2, perm2, k, n)) {
     Routing route{nullptr, 0, nullptr, nullptr, static_cast<const float*>(topk_weights.const_data_ptr()),
                   static_cast<const int32_t*>(topk_ids.const_data_ptr())};
     moe_gemm_16bit(hidden, wide.mutable_data_ptr(), w1, bias1, scale1, std::nullopt, global_scale1, zeros1, g_idx1, perm1,

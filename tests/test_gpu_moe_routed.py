@@ -106,6 +106,30 @@ def test_routings(block, slots):
         assert torch.equal(got, want)
 
 
+# global_num_experts below the experts held: the slots of the others are left out, as with more slots than this path takes
+@pytest.mark.gpu
+@pytest.mark.parametrize("tokens", [6, 100, 200])
+def test_fewer_experts_than_held(tokens):
+    e, inter, k, dtype = 4, 128, 256, torch.bfloat16
+    gen = torch.Generator(device=DEV).manual_seed(tokens)
+    w1, s1, _ = _experts(gen, "uint4b8", e, k, 2 * inter, 128, dtype)
+    w2, s2, _ = _experts(gen, "uint4b8", e, inter, k, 128, dtype)
+    x = torch.randn((tokens, k), device=DEV, generator=gen).to(dtype) * 0.1
+    ids = (torch.arange(tokens, device=DEV, dtype=torch.int32) % e).view(tokens, 1).contiguous()
+    weights = torch.ones((tokens, 1), device=DEV)
+
+    def layer(experts):   # row i of either GEMM lies at i * k, as 2 * inter == k
+        return fused_moe.fused_marlin_moe(
+            x, w1, w2, None, None, s1, s2, weights, ids, scalar_types.uint4b8.id, global_num_experts=experts,
+            intermediate_cache13=torch.full((tokens * k,), 7.0, dtype=dtype, device=DEV))
+    whole, part = layer(e), layer(e - 1)
+    left_out = ids[:, 0] == e - 1
+    assert bool((part[left_out] == 7.0).all()) and not bool((whole == 7.0).all(dim=1).any())
+    assert bool((part[~left_out] != 7.0).any(dim=1).all())
+    with pytest.raises(RuntimeError, match="out of range"):   # refused with any number of slots
+        layer(8193)
+
+
 @pytest.mark.parametrize("slots,block,experts,code,n,k,groups,want", [
     (128, 8, 256, _lib.TYPE_UINT4B8, 128, 128, 1, 1), (129, 8, 8, _lib.TYPE_UINT4B8, 128, 128, 1, 0),
     (128, 8, 257, _lib.TYPE_UINT4B8, 128, 128, 1, 0), (128, 48, 8, _lib.TYPE_UINT4B8, 128, 128, 1, 0),
