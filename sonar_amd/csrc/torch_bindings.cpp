@@ -477,10 +477,17 @@ std::tuple<Tensor, Tensor> awq_to_standard(const Tensor& qweight, const Tensor& 
   c10::hip::HIPGuardMasqueradingAsCUDA guard(qweight.device());
   Tensor codes = at::empty({k / 8, words * 8}, qweight.options());
   Tensor zeros = at::empty({words, groups}, qzeros.options());
-  raise_if_failed(sonar_awq_to_standard(static_cast<const uint32_t*>(qweight.const_data_ptr()),
-                                        static_cast<uint32_t*>(codes.mutable_data_ptr()),
-                                        static_cast<const uint32_t*>(qzeros.const_data_ptr()),
-                                        static_cast<uint32_t*>(zeros.mutable_data_ptr()), k, words * 8, groups, current_stream(qweight)));
+  const auto* code_words = static_cast<const uint32_t*>(qweight.const_data_ptr());
+  const auto* zero_words = static_cast<const uint32_t*>(qzeros.const_data_ptr());
+  auto* codes_out = static_cast<uint32_t*>(codes.mutable_data_ptr());
+  auto* zeros_out = static_cast<uint32_t*>(zeros.mutable_data_ptr());
+  if (qweight.device() == qzeros.device()) {
+    raise_if_failed(sonar_awq_to_standard(code_words, codes_out, zero_words, zeros_out, k, words * 8, groups, current_stream(qweight)));
+  } else {   // each on the stream of its own GPU
+    raise_if_failed(sonar_awq_to_gptq(code_words, codes_out, k, words * 8, current_stream(qweight)));
+    guard.set_device(qzeros.device());
+    raise_if_failed(sonar_awq_zeros_to_plain(zero_words, zeros_out, groups, words * 8, current_stream(qzeros)));
+  }
   return {codes, zeros};
 }
 

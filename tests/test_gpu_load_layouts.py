@@ -111,3 +111,16 @@ def test_awq_checkpoint_is_loaded_as_on_the_cpu(k, n, group):
     z = mo.awq_to_marlin_zero_points(qz.numpy(), k // group, n)
     assert np.array_equal(gpu.qzeros.cpu().numpy(), z)
     assert torch.equal(gpu.qweight, ops.awq_marlin_repack(qw.to(DEV), k, n, 4))
+
+
+@pytest.mark.skipif(torch.cuda.device_count() < 2, reason="two GPUs")
+def test_awq_tensors_on_two_gpus():
+    """Codes and zero points are converted where they lie: one launch takes both only where they lie together."""
+    from sonar_amd import marlin_linear as ml
+    qw, qz = _words(np.random.default_rng(1), 256, 40), _words(np.random.default_rng(2), 4, 40)
+    cpu = SimpleNamespace(qweight=qw, qzeros=qz)
+    gpu = SimpleNamespace(qweight=qw.to("cuda:0"), qzeros=qz.to("cuda:1"))
+    ml.convert_awq_to_standard_format(cpu)
+    ml.convert_awq_to_standard_format(gpu)
+    assert gpu.qweight.device.index == 0 and gpu.qzeros.device.index == 1
+    assert torch.equal(gpu.qweight.cpu(), cpu.qweight) and torch.equal(gpu.qzeros.cpu(), cpu.qzeros)
