@@ -105,6 +105,9 @@ int sonar_marlin_last_decode_launch(int32_t* out, int n);
 #define SONAR_GROUPED_MID 3       /* marlin_mid_gemm */
 #define SONAR_GROUPED_TILE 4      /* the tile kernels */
 int sonar_marlin_last_grouped_kernel(void);
+/* Strips of 64 columns that a workgroup of marlin_mid_gemm had in the last GEMM, dense or grouped, on the calling thread; 0: another
+ * kernel ran.  For tests. */
+int sonar_marlin_last_mid_strips(void);
 
 /* GPTQ (K/8, N) int32, nibble k%8 of word [k/8][n] = code of W[k][n]
  * -> Marlin (K/16, 2N) int32; with num_bits == 8: (K/4, N) int32, byte k%4

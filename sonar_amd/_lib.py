@@ -35,6 +35,7 @@ PROTOTYPES = {
     "sonar_marlin_version": (c_char_p, []),
     "sonar_marlin_last_decode_launch": (c_int, [c_void_p, c_int]),
     "sonar_marlin_last_grouped_kernel": (c_int, []),
+    "sonar_marlin_last_mid_strips": (c_int, []),
     "sonar_debug_tile_schedule": (c_int64, [c_int64, c_int64, c_int64, c_int64, c_void_p, c_int64]),
     "sonar_debug_moe_tile_schedule": (c_int64, [c_int64, c_int64, c_int64, c_int64, c_int, c_void_p, c_int64]),
     "sonar_debug_moe_pair_schedule": (c_int64, [c_int64, c_int64, c_int64, c_int64, c_int64, c_int, c_void_p, c_void_p, c_int64]),

@@ -806,10 +806,13 @@ int launch_mid_moe_format(const MidMoeParams& p, int format, hipStream_t st) {
 
 }  // namespace
 
+thread_local int g_last_mid_strips = 0;
+
 int mid_moe_gemm(MidMoeParams p, int dtype, int format, int blocks, hipStream_t st) {
   p.splits = 1;
   p.tiles_m = blocks;
   p.strips_each = mid_moe_strips(p.moe.block_size, p.moe.rows_total / p.moe.num_experts, p.moe.num_experts, p.size_n, p.size_k, p.raw_codes, p.cus);
+  g_last_mid_strips = p.strips_each;
   const int halves = p.moe.gated != nullptr && p.moe.gated_halves ? 2 : 1, across = p.size_n / kStripN / halves, each = p.strips_each / halves;
   p.tiles = blocks * ((across + each - 1) / each);
   p.split_steps = p.size_k / kMidStepK;
@@ -825,6 +828,7 @@ int mid_gemm(MidParams p, int dtype, int format, int row_blocks, hipStream_t st)
   const bool by_rounds = p.raw_codes && row_blocks == kMidMostRawRows && p.splits == 1;
   const int each = by_rounds ? mid_strips_by_rounds(p.tiles_m, 0.0, p.size_n, p.size_k, true, p.cus) : mid_strips(row_blocks);
   p.tiles = p.tiles_m * ((strips + each - 1) / each);
+  g_last_mid_strips = each;
   const int steps = p.size_k / kMidStepK;
   p.split_steps = (steps + p.splits - 1) / p.splits;
   if (p.raw_codes) p.split_steps = (p.split_steps + 1) & ~1;   // whole units of 128 rows
@@ -845,3 +849,5 @@ int mid_gemm(MidParams p, int dtype, int format, int row_blocks, hipStream_t st)
 }
 
 }  // namespace sonar
+
+extern "C" int sonar_marlin_last_mid_strips() { return sonar::g_last_mid_strips; }

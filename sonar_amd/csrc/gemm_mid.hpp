@@ -181,6 +181,9 @@ inline int mid_moe_strips(int64_t block_size, int64_t slots, int64_t num_experts
   return mid_strips_by_rounds((double)num_experts * (slots <= most ? 1.0 + second : slots / most + 1), 0.1, size_n, size_k, units, cus);
 }
 
+// Strips of a workgroup in the calling thread's last GEMM; 0: that ran in another kernel.
+extern thread_local int g_last_mid_strips;
+
 // `row_blocks`: 16-row blocks of a tile, 1 to 6.
 int mid_gemm(MidParams p, int dtype, int format, int row_blocks, hipStream_t st);
 

@@ -616,6 +616,7 @@ int moe_gemm_any(
     int64_t size_m, int64_t size_n, int64_t size_k, int64_t num_groups, int is_k_full, void* stream,
     const MoeLayerCall& layer = {}) {
   g_last_grouped_kernel = SONAR_GROUPED_NONE;
+  g_last_mid_strips = 0;
   const bool nvfp4 = global_scale != nullptr;
   SONAR_REQUIRE(b_layout == SONAR_LAYOUT_GFX950, "unknown b_layout = %d", b_layout);
   SONAR_REQUIRE(dtype == SONAR_DTYPE_F16 || dtype == SONAR_DTYPE_BF16, "unsupported `a` scalar_type");

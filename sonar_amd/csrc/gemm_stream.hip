@@ -1902,6 +1902,7 @@ int marlin_gemm_any(const void* a, int64_t a_row_stride, void* c, const uint32_t
                 "scratch of %zu bytes is too small", scratch_bytes);
 
   g_last_decode_launch[0] = 0;
+  g_last_mid_strips = 0;
   hipStream_t st = (hipStream_t)stream;
   // Act-order with room in the scratch buffer for a copy of A: permute the
   // columns of A once and run the plain grouped kernels on the copy.

@@ -1,0 +1,81 @@
+"""The four-strip workgroups of marlin_mid_gemm, each case with the strips that it ran in: grouped calls of every block size whose last
+workgroup has one to four strips of its own, at the fewest rows of K that the form is given and at an odd number of units; the dense
+shapes of test_gpu_mid_four_strips; and the gated activation where the ranges meet, in layers whose gate and up rows are in that
+kernel and are not written."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from sonar_amd import _lib, fused_moe
+from sonar_amd.scalar_type import scalar_types
+from tests import gpu_util as gu
+from tests import test_gpu_mid_four_strips as dense
+from tests import test_gpu_moe as tm
+from tests.test_gpu_moe_routed import _experts
+
+pytestmark = pytest.mark.gpu
+
+
+def _ran_in(strips: int, grouped: bool = True) -> None:
+    lib = _lib.load()
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:   # (rounds of workgroups on 256 compute units)
+        assert not grouped or lib.sonar_marlin_last_grouped_kernel() == _lib.GROUPED_MID
+        assert lib.sonar_marlin_last_mid_strips() == strips
+
+
+@pytest.mark.parametrize("m,slots", [(200, 32), (296, 48), (400, 64)])
+@pytest.mark.parametrize("k,n", [(512, 2240), (512, 2304), (512, 2368), (512, 2432), (1664, 2368)])   # 35 to 38 strips
+@pytest.mark.parametrize("dtype,zp,group", [("fp16", False, 128), ("bf16", True, -1)])
+def test_four_strips(m, slots, k, n, dtype, zp, group):
+    tm.test_moe_gemm_within_tolerance((m, 16, 2, k, n, group, dtype, zp, False, zp, slots, not zp))
+    _ran_in(4)
+
+
+# fewer than a round of two strips a workgroup, and K below 512
+@pytest.mark.parametrize("m,e,k,n,slots", [(400, 16, 512, 2048, 64), (296, 16, 384, 2432, 48)])
+def test_two_strips(m, e, k, n, slots):
+    tm.test_moe_gemm_within_tolerance((m, e, 2, k, n, 128, "bf16", False, False, False, slots, True))
+    _ran_in(2)
+
+
+@pytest.mark.parametrize("dtype", ["fp16", "bf16"])
+@pytest.mark.parametrize("zp", [False, True])
+@pytest.mark.parametrize("m,k,n,group", [(65, 640, 24640, 128), (128, 1408, 24768, -1), (97, 1152, 16576, 128)])
+def test_dense(m, k, n, group, zp, dtype):
+    dense.test_against_the_oracle(m, k, n, group, zp, dtype)
+    _ran_in(4, grouped=False)
+
+
+# blocks of 32, 48 and 64 slots; halves of an odd number of strips
+@pytest.mark.parametrize("kind,group,dtype", [("uint4b8", 128, torch.float16), ("uint4", 128, torch.bfloat16), ("mxfp4", 32, torch.bfloat16)])
+@pytest.mark.parametrize("tokens,k,inter,strips", [(200, 512, 832, 2), (296, 512, 576, 2), (400, 512, 576, 2), (400, 640, 960, 2),
+                                                   (296, 640, 1344, 4), (400, 1152, 1600, 4)])
+def test_gated_activation(tokens, k, inter, strips, kind, group, dtype):
+    e, rows = 16, 2 * tokens
+    gen = torch.Generator(device=gu.DEV).manual_seed(tokens + k)
+    w1, s1, z1 = _experts(gen, kind, e, k, 2 * inter, group, dtype)
+    w2, s2, z2 = _experts(gen, kind, e, inter, k, min(group, 64), dtype)
+    bias1 = (torch.randn((e, 2 * inter), device=gu.DEV, generator=gen) * 0.1).to(dtype)
+    x = torch.randn((tokens, k), device=gu.DEV, generator=gen).to(dtype) * 0.1
+    weights, ids = torch.topk(torch.softmax(torch.randn((tokens, e), device=gu.DEV, generator=gen), dim=1), 2, dim=1)
+    wtype = {"uint4b8": scalar_types.uint4b8, "uint4": scalar_types.uint4, "mxfp4": scalar_types.float4_e2m1f}[kind]
+    assert 2 * inter > k
+    for activation, on_input in (("swigluoai", False), ("silu", False), ("silu", True)):
+        def layer(**kw):
+            return fused_moe.fused_marlin_moe(x, w1, w2, bias1, None, s1, s2, weights.contiguous(), ids.to(torch.int32), wtype.id, on_input,
+                                              activation=activation, w1_zeros=z1, w2_zeros=z2, **kw)
+        between = torch.empty((rows, inter), dtype=dtype, device=gu.DEV)
+
+        def after(name, out, rows_in, **kw):   # behind the GEMM of the gate and up rows
+            _ran_in(strips)
+            fused_moe.apply_moe_activation(name, out, rows_in, **kw)
+            between.copy_(out)
+
+        cache13 = torch.full((rows * 2 * inter,), -7.0, dtype=dtype, device=gu.DEV)
+        cache2 = torch.empty((rows * inter,), dtype=dtype, device=gu.DEV)
+        got = layer(intermediate_cache13=cache13, intermediate_cache2=cache2)
+        assert bool((cache13[rows * k:] == -7.0).all()), activation   # the gate and up rows were not written
+        want = layer(activation_func=after)
+        assert bool(torch.isfinite(want).all())
+        assert torch.equal(cache2.view(rows, inter), between) and torch.equal(got, want), activation
