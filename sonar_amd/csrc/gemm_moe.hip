@@ -42,6 +42,7 @@ int moe_fast_gemm(const void* a, void* c, const uint32_t* b, const void* bias, c
                   int mul_topk, int64_t num_experts, int dtype, int64_t size_m, int64_t size_n, int64_t size_k,
                   int64_t num_groups, int group_size, int a_by_slot, bool fp4, const int32_t* topk_ids, GatedOutput* gated, hipStream_t st);
 bool moe_fast_routes(int64_t slots, int64_t moe_block_size, int64_t num_experts);
+bool moe_fast_gates(const GatedOutput* gated, bool routed, int64_t slots, int64_t moe_block_size, int64_t num_experts, int64_t size_n);
 
 namespace {
 
@@ -557,6 +558,7 @@ using namespace sonar;
 // Four strips and the 512 rows of K that they are given from (less was not timed) are in mid_moe_strips.
 // The general kernel (MXFP4 with K of no whole units) is never ahead: 16 of 35, 1472 x 704 54 / 37.
 // Blocks of 32 and 48 slots that are nearly full on average were not timed (the rule for block sizes makes none).
+// `gated`: the decode kernel would form the layer's gated activation (moe_fast_gates).
 static bool moe_mid_applies(int64_t moe_block_size, int64_t rows_total, int64_t num_experts, int64_t a_rows, int64_t size_n,
                             int64_t size_k, int64_t num_groups, int group_size, bool fp4, bool decode, bool tiles, bool gated) {
   static const bool no_mid = getenv("SONAR_MARLIN_NO_MOE_MID") != nullptr;  // debugging aid
@@ -749,7 +751,7 @@ int moe_gemm_any(
   // (Its scales are 16-byte loads, as in the dense call; the other kernels copy them in pieces of 4.)
   if (layer.topk_ids == nullptr && !bits8 && !row_groups && !nvfp4 && !has_perm && ((uintptr_t)b_scales) % 16 == 0 &&
       moe_mid_applies(moe_block_size, size_m * top_k, num_experts, a_rows, size_n, size_k, num_groups, group_size, fp4,
-                      decode, tiles, layer.gated != nullptr)) {
+                      decode, tiles, moe_fast_gates(layer.gated, false, size_m * top_k, moe_block_size, num_experts, size_n))) {
     MidMoeParams m = {};
     m.a = static_cast<const uint16_t*>(a);
     m.lda = size_k;
@@ -782,8 +784,7 @@ int moe_gemm_any(
     m.moe.expert_bias_stride = size_n;
     // The gated activation where the ranges meet: a launch of 5 to 8 us less
     GatedOutput* gated = layer.gated;
-    if (gated != nullptr && ((uintptr_t)gated->out) % 8 == 0 &&
-        (gated->kind == 0 ? size_n % (2 * kStripN) == 0 : gated->kind == SONAR_ACT_SWIGLUOAI && gated->limit > 0.f)) {
+    if (gated_by_strips(gated, size_n)) {
       m.moe.gated = static_cast<uint16_t*>(gated->out);
       m.moe.gated_halves = gated->kind == 0;
       m.moe.gated_limit = gated->limit;
@@ -922,6 +923,8 @@ extern "C" int sonar_moe_routed_gemm_applies(int64_t slots, int64_t moe_block_si
   if (b_type_id != SONAR_TYPE_UINT4B8 && b_type_id != SONAR_TYPE_UINT4 && !(fp4 && size_k == 32 * num_groups)) return 0;
   if (size_k % num_groups != 0) return 0;
   const int group_size = (int)(size_k / num_groups);
+  // (A layer finds its rows itself in both GEMMs or in none, and saves the launch that sorts them: a round or more of blocks of 32
+  // stays in the decode kernel for that, as if it formed an activation.)
   return moe_fast_routes(slots, moe_block_size, num_experts) &&
          moe_fast_applies(false, moe_block_size, most_sorted(slots, moe_block_size, num_experts), num_experts, slots, size_n, size_k,
                           num_groups, group_size) &&

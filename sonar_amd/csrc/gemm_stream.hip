@@ -1714,6 +1714,17 @@ bool moe_fast_routes(int64_t slots, int64_t moe_block_size, int64_t num_experts)
   return !off && slots <= kRoutedSlots && num_experts <= kRoutedExperts && moe_block_size <= 32;
 }
 
+// Whether such a call forms the gated activation where its rows end: a launch of 3 to 5 us less, and half as many workgroups twice as
+// long.  Not where more than kRoutedSlots slots make fewer of those than there are compute units.  Us a layer, a launch of its own ->
+// here: 32 experts 1152 x 11136, 704 slots 245 -> 205; 64 MXFP4 of 1024 x 2688, 448 slots 114 -> 97; 16 of 1280 x 2432, 920 slots
+// 81 -> 71; left out: 8 of 1408 x 896, 186 slots 27.2 -> 29.0; 16 of 2816 x 768, 344 slots 40.1 -> 40.7.
+bool moe_fast_gates(const GatedOutput* gated, bool routed, int64_t slots, int64_t moe_block_size, int64_t num_experts, int64_t size_n) {
+  if (!gated_by_strips(gated, size_n)) return false;
+  const int64_t sub_blocks = moe_block_size > 32 ? 2 : 1;
+  return routed || gated->kind != 0 ||
+         std::max(std::min(num_experts, slots), slots / moe_block_size) * sub_blocks * (size_n / (2 * kStripN)) >= cu_count();
+}
+
 // Called by sonar_moe_wna16_marlin_gemm when moe_fast_applies: one workgroup
 // per (block of slots, strip), nothing reduced through memory.  Arguments have
 // been validated by the caller.
@@ -1740,14 +1751,7 @@ int moe_fast_gemm(const void* a, void* c, const uint32_t* b, const void* bias, c
   p.chunks_per_strip = (int)(size_k / kChunkK);
   p.unit_chunks = 4;
   p.units_per_strip = p.chunks_per_strip / 4;
-  // The gated activation where the rows end: a launch of 3 to 5 us less, and half as many workgroups twice as long.  Not where more
-  // than kRoutedSlots slots make fewer of those than there are compute units.  Us a layer, a launch of its own -> here: 32
-  // experts 1152 x 11136, 704 slots 245 -> 205; 64 MXFP4 of 1024 x 2688, 448 slots 114 -> 97; 16 of 1280 x 2432, 920 slots 81 -> 71; left out: 8 of
-  // 1408 x 896, 186 slots 27.2 -> 29.0; 16 of 2816 x 768, 344 slots 40.1 -> 40.7.
-  const int64_t slots = size_m * top_k, sub_blocks = moe_block_size > 32 ? 2 : 1;
-  const int64_t workgroups = std::max(std::min(num_experts, slots), slots / moe_block_size) * sub_blocks * (size_n / (2 * kStripN));
-  if (gated != nullptr && (topk_ids != nullptr || gated->kind != 0 || workgroups >= cu_count()) && ((uintptr_t)gated->out) % 8 == 0 &&
-      (gated->kind == 0 ? size_n % (2 * kStripN) == 0 : gated->kind == SONAR_ACT_SWIGLUOAI && gated->limit > 0.f)) {
+  if (moe_fast_gates(gated, topk_ids != nullptr, size_m * top_k, moe_block_size, num_experts, size_n)) {
     p.gated = static_cast<uint16_t*>(gated->out);
     p.gated_halves = gated->kind == 0;
     p.gated_limit = gated->limit;

@@ -56,6 +56,12 @@ struct GatedOutput {
   float limit, alpha;    // of SONAR_ACT_SWIGLUOAI
   bool done;             // set by a call that wrote `out`, which then left c as it was
 };
+// Whether a kernel whose workgroups have whole strips of 64 columns can form it: rows of 8-byte stores, as many strips of the gate half
+// as of the up half.
+inline bool gated_by_strips(const GatedOutput* g, int64_t size_n) {
+  return g != nullptr && ((uintptr_t)g->out) % 8 == 0 &&
+         (g->kind == 0 ? size_n % 128 == 0 : g->kind == SONAR_ACT_SWIGLUOAI && g->limit > 0.f);
+}
 
 // What one grouped GEMM of a layer may do for another one of the same routing, or have had done for it.
 struct MoeLayerCall {

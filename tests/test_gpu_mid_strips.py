@@ -4,9 +4,13 @@ shapes of test_gpu_mid_four_strips; and the gated activation where the ranges me
 kernel and are not written."""
 from __future__ import annotations
 
+import ctypes
+
+import numpy as np
 import pytest
 import torch
 
+from oracle import marlin_oracle as mo
 from sonar_amd import _lib, fused_moe
 from sonar_amd.scalar_type import scalar_types
 from tests import gpu_util as gu
@@ -79,3 +83,36 @@ def test_gated_activation(tokens, k, inter, strips, kind, group, dtype):
         want = layer(activation_func=after)
         assert bool(torch.isfinite(want).all())
         assert torch.equal(cache2.view(rows, inter), between) and torch.equal(got, want), activation
+
+
+# a round or more of blocks of 32 slots: the decode kernel's where it forms the activation, and only there
+@pytest.mark.parametrize("n,activation,limit,written,kernel", [
+    (2304, "SILU", 0.0, 1, "DECODE"), (2304, "SWIGLUOAI", 7.0, 1, "DECODE"), (2368, "SWIGLUOAI", 7.0, 1, "DECODE"),
+    (2304, "GELU", 0.0, 0, "MID"), (2368, "SILU", 0.0, 0, "MID"), (2304, "SWIGLUOAI", 0.0, 0, "MID")])
+def test_an_activation_that_no_kernel_forms_changes_no_route(n, activation, limit, written, kernel):
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("rounds of workgroups on 256 compute units")
+    kinds = {"SILU": 0, "GELU": 2, "SWIGLUOAI": 4}
+    m, e, top_k, k, slots = 200, 16, 2, 512, 32
+    lib = _lib.load()
+    ex = tm.Experts(5, e, k, n, 128, "bf16")
+    sorted_ids, expert_ids, past = mo.moe_align_block_size(tm.route(3, m, e, top_k)[0], slots, e)
+    sid, eid, npp = (gu.dev_i32(np.asarray(x).reshape(-1)) for x in (sorted_ids, expert_ids, past))
+    a = gu.dev_bits16(mo.make_activations(4, m, k, "bf16"), "bf16")
+
+    def call(out, answer):
+        c = torch.full((m * top_k, n), -7.0, dtype=torch.bfloat16, device=gu.DEV)
+        _lib.check(lib.sonar_moe_wna16_marlin_gemm_gated(
+            gu.ptr(a), gu.ptr(c), gu.ptr(ex.native), _lib.LAYOUT_GFX950, None, gu.ptr(ex.scales), None, None, None, None, None, 0,
+            gu.ptr(sid), sid.numel(), gu.ptr(eid), gu.ptr(npp), None, slots, top_k, 0, e, _lib.DTYPE_BF16, ex.b_type, m, n, k, ex.groups, 1,
+            gu.ptr(out), kinds[activation], limit, 1.702, answer, None, None, gu.stream()))
+        torch.cuda.synchronize()
+        return c, lib.sonar_marlin_last_grouped_kernel()
+
+    done = ctypes.c_int(5)
+    plain, ran = call(None, ctypes.byref(done))
+    assert ran == _lib.GROUPED_MID and done.value == 0
+    out = torch.full((m * top_k, n // 2), -7.0, dtype=torch.bfloat16, device=gu.DEV)
+    c, ran = call(out, ctypes.byref(done))
+    assert done.value == written and ran == getattr(_lib, "GROUPED_" + kernel)
+    assert torch.equal(c, torch.full_like(c, -7.0) if written else plain) and bool((out == -7.0).all()) != bool(written)
