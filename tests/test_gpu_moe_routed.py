@@ -5,6 +5,10 @@ range, an expert twice for a token, all slots on one, each number of slots aroun
 from __future__ import annotations
 
 import ctypes
+import hashlib
+import os
+import subprocess
+import sys
 
 import pytest
 import torch
@@ -143,3 +147,46 @@ def test_which_calls(slots, block, experts, code, n, k, groups, want):
         one = ctypes.c_int(5)
         assert lib.sonar_moe_routed_gemm(None, None, None, _lib.LAYOUT_GFX950, None, None, None, 16, None, block, 1, 0, experts,
                                          _lib.DTYPE_BF16, code, slots, n, k, groups, None, 0, 0.0, 0.0, ctypes.byref(one), None) != 0
+
+
+# The same layers with sorted slots (another process, which takes the routing from the decode kernel): where that kernel forms the
+# activation either way, silu_and_mul included, the bits are the same.  Blocks of 8, 16 and 32 slots.
+@pytest.mark.gpu
+def test_same_bits_with_sorted_slots():
+    out = [subprocess.run([sys.executable, "-u", "-m", "tests.test_gpu_moe_routed"], cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
+                          capture_output=True, text=True, env=dict(os.environ, **env), timeout=110)
+           for env in ({}, {"SONAR_MARLIN_NO_MOE_ROUTED": "1"})]
+    assert all(o.returncode == 0 and o.stdout.strip().endswith("done") for o in out), [o.stdout[-500:] + o.stderr[-1500:] for o in out]
+    assert out[0].stdout == out[1].stdout
+
+
+def _digests() -> None:
+    routed = 0 if os.environ.get("SONAR_MARLIN_NO_MOE_ROUTED") else 1
+    e, top_k, k, inter, group = 8, 2, 512, 2048, 32
+    for kind, dtype in (("uint4b8", torch.float16), ("uint4", torch.bfloat16), ("mxfp4", torch.bfloat16)):
+        for tokens, block in ((20, 8), (48, 16), (64, 32)):
+            gen = torch.Generator(device=DEV).manual_seed(tokens)
+            w1, s1, z1 = _experts(gen, kind, e, k, 2 * inter, group, dtype)
+            w2, s2, z2 = _experts(gen, kind, e, inter, k, group, dtype)
+            x = torch.randn((tokens, k), device=DEV, generator=gen).to(dtype) * 0.1
+            weights, ids = torch.topk(torch.softmax(torch.randn((tokens, e), device=DEV, generator=gen), dim=1), top_k, dim=1)
+            wtype = {"uint4b8": scalar_types.uint4b8, "uint4": scalar_types.uint4, "mxfp4": scalar_types.float4_e2m1f}[kind]
+            assert fused_moe.moe_block_size(tokens, top_k, e) == block
+            for n_, k_ in ((2 * inter, k), (k, inter)):
+                assert _lib.load().sonar_moe_routed_gemm_applies(tokens * top_k, block, e, wtype.id, n_, k_, k_ // group) == routed
+            rows = tokens * top_k
+            for activation in ("silu", "swigluoai"):
+                cache13 = torch.full((rows * 2 * inter,), -7.0, dtype=dtype, device=DEV)
+                out = fused_moe.fused_marlin_moe(x, w1, w2, None, None, s1, s2, weights.contiguous(), ids.to(torch.int32), wtype.id,
+                                                 activation=activation, w1_zeros=z1, w2_zeros=z2, intermediate_cache13=cache13)
+                assert bool(torch.isfinite(out).all())
+                # (rounds of workgroups on 256 compute units)
+                if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+                    assert bool((cache13[rows * k:] == -7.0).all())   # no gate and up rows: the kernel formed the activation
+                    assert _lib.load().sonar_marlin_last_grouped_kernel() == _lib.GROUPED_DECODE
+                print(kind, tokens, activation, hashlib.sha256(out.view(torch.uint8).cpu().numpy().tobytes()).hexdigest()[:16], flush=True)
+
+
+if __name__ == "__main__":
+    _digests()
+    print("done", flush=True)
