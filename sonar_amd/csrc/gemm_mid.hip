@@ -135,6 +135,7 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
   constexpr int kMidStrips = STRIPS, kMidRanges = mid_ranges(STRIPS);
   // 8-row copies of activations per wavefront and step (three row blocks and four strips: the last wavefront's are copies 5 again)
   constexpr int kCopies = (2 * MB + kMidStrips - 1) / kMidStrips;
+  constexpr bool kEvenCopies = kCopies * kMidStrips == 2 * MB;
   constexpr int kLoads = Fmt::k8 ? 4 : 2;            // 16-byte loads of packed codes per lane and step
   constexpr int kScaleRows = GROUPS == kChunkGroups ? 2 : 1;
   // memory operations per wavefront and step
@@ -181,7 +182,7 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
   uint32_t a_off[kCopies];
 #pragma unroll
   for (int i = 0; i < kCopies; ++i) {
-    int row = m0 + 8 * min(strip_of * kCopies + i, 2 * MB - 1) + (lane >> 3);
+    int row = m0 + 8 * (kEvenCopies ? strip_of * kCopies + i : min(strip_of * kCopies + i, 2 * MB - 1)) + (lane >> 3);
     if constexpr (GROUPED) {   // (padding slots read row 0 and are not stored)
       const int id = row < moe.sorted_len ? moe.sorted_ids[row] : moe.rows_total;
       row = (unsigned)id < (unsigned)moe.rows_total ? (moe.a_by_slot ? row : id / moe.top_k) : 0;
@@ -227,7 +228,8 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
     } else {
       const int i = op - (kOps - kCopies);
       const char* a_src = reinterpret_cast<const char*>(p.a) + (size_t)k * (kMidStepK * 2);
-      copy_to_lds<16>(a_lds + slot * kStage + min(strip_of * kCopies + i, 2 * MB - 1) * 1024, a_off[i], a_src);
+      const int at = kEvenCopies ? strip_of * kCopies + i : min(strip_of * kCopies + i, 2 * MB - 1);
+      copy_to_lds<16>(a_lds + slot * kStage + at * 1024, a_off[i], a_src);
     }
   };
   // Scales of the unit of step `k`, behind whose first half they are taken from the registers, and zero points, which fp16
