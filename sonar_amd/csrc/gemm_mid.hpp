@@ -68,10 +68,14 @@ inline bool mid_applies(int64_t size_m, int64_t size_k, int64_t lda, int64_t num
   return group_size % 64 == 0 && (per & (per - 1)) == 0;
 }
 
-// Strips of a workgroup, two or four, in a grouped call and in dense 64-row tiles of raw codes with K in one piece.  A round of workgroups takes as long as six steps beside its loop (start, first
-// bytes, the sum of the ranges), so that twice the columns and half the ranges, whose activations are copied half as often, pay where
-// rounds are many; in whole rounds, with the second blocks of uneven routing counted.  Fitted to both forms of 242 GEMMs of 23 to 57 slots
-// an expert (blocks of 48 and 64): 0.5 % slower than the better of the two, two strips always 16 %; at worst 1.2 times two strips.
+// Strips of a workgroup, two or four, in a grouped call and in dense 64-row tiles of raw codes with K in one piece.  A round of
+// workgroups takes as long as six steps beside its loop (start, first bytes, the sum of the ranges), so that twice the columns and half
+// the ranges, whose activations are copied half as often, pay where rounds are many; in whole rounds, less `slack`.
+// Grouped calls (slack 0.1, the second blocks of uneven routing counted by mid_moe_strips) are what this was fitted to: both forms of
+// 242 GEMMs of 23 to 57 slots an expert (blocks of 48 and 64): 0.5 % slower than the better of the two, two strips always 16 %; at
+// worst 1.2 times two strips.
+// Dense calls take it as it stands with slack 0, as their tiles are counted and not estimated.  Timed on 150 random calls against the
+// tree that had two strips only: it changes 10 of them, to 0.67 to 0.93 times the time.
 // Us, two -> four strips: 64 of 56, K = 2304, N = 6656, bf16 346 -> 242; 64 of 49, AWQ, 1664 x 8704 291 -> 220; 32 of 42, 1152 x 15360
 // 187 -> 132; 64 of 29, MXFP4, 640 x 2688 51 -> 35; 8 of 49, 1536 x 5888 26.5 -> 21.1; 16 of 52, 1152 x 1536, three quarters of a
 // round 14.9 -> 18.0.
@@ -95,7 +99,10 @@ inline int mid_strips_by_rounds(double row_tiles, double slack, int64_t size_n, 
 // full chip than of a half empty one; no less than the weights take from memory.  K is split where the tiles leave
 // compute units idle, if the totals fit `room` bytes; the pass that adds them is 3.3 us and its bytes.  `raw_codes` (see
 // MidParams) has a fit of its own (K = 1024 to 14336, N = 2048 to 28672, 17 to 256 rows, weights from memory: 90 % within
-// 6 % below and 13 % above): fewer instructions a chunk for the dequantisation, more a row block for the fold.
+// 6 % below and 13 % above): fewer instructions a chunk for the dequantisation, more a row block for the fold.  Workgroups of four strips
+// (mid_strips_by_rounds) have their own: the fuller their one round, the slower (111 calls of up to 127 rows, K = 512 to 11520, N up to
+// 57344, both types, 5.6 % rms; with two strips' term, which grows with the bytes, 8192 x 57344 was put at twice its time and
+// 49 rows left for the decode kernel: K = 7424, N = 51968, fp16 94 us there, 65 here).
 inline double mid_estimate(int64_t size_m, int64_t size_n, int64_t size_k, int64_t num_groups, int dtype, int format,
                            bool raw_codes, int cus, size_t room, int& row_blocks, int& splits) {
   static const double kDequant[6][2] = {   // float16, bfloat16
@@ -120,7 +127,7 @@ inline double mid_estimate(int64_t size_m, int64_t size_n, int64_t size_k, int64
         if (mb == kMidMostRawRows && n == 1 && mid_strips_by_rounds((double)((size_m + 16 * mb - 1) / (16 * mb)), 0.0, size_n, size_k, true, cus) == 4) {
           const int64_t fours = ((size_m + 16 * mb - 1) / (16 * mb)) * ((size_n + 255) / 256), rounds4 = (fours + cus - 1) / cus;
           const double k4 = 2 * ((steps / 2 + 1) / 2) * 256 / 4096.0;
-          const double slow4 = rounds4 > 1 ? 0.95 : (2 * fours > cus ? 0.86 : 0.8) + 2.5e-9 * size_n * size_k;
+          const double slow4 = rounds4 > 1 ? 1.0 : 0.63 + 0.58 * fours / cus;
           us = 1.4 + rounds4 * (2.4 + 0.3 * mb + k4 * (raw[0] + raw[1] * mb) * slow4);
         }
       }

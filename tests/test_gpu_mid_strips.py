@@ -11,7 +11,7 @@ import pytest
 import torch
 
 from oracle import marlin_oracle as mo
-from sonar_amd import _lib, fused_moe
+from sonar_amd import _lib, fused_moe, marlin_utils as mu, ops
 from sonar_amd.scalar_type import scalar_types
 from tests import gpu_util as gu
 from tests import test_gpu_mid_four_strips as dense
@@ -116,3 +116,25 @@ def test_an_activation_that_no_kernel_forms_changes_no_route(n, activation, limi
     c, ran = call(out, ctypes.byref(done))
     assert done.value == written and ran == getattr(_lib, "GROUPED_" + kernel)
     assert torch.equal(c, torch.full_like(c, -7.0) if written else plain) and bool((out == -7.0).all()) != bool(written)
+
+
+# up to 64 rows of a matrix of more than 256 pairs of strips: one round of four strips, the longer the fuller it is and not the more bytes the
+# matrix has; the widest of these were left to kernels that take 1.1 to 1.4 times as long.  Against the decode kernel, 16 rows at a time.
+@pytest.mark.parametrize("m,k,n,dtype", [(49, 7424, 51968, torch.float16), (62, 2944, 46592, torch.bfloat16), (64, 8192, 57344, torch.bfloat16)])
+def test_wide_matrices(m, k, n, dtype):
+    gen = torch.Generator(device=gu.DEV).manual_seed(m)
+    q = torch.randint(-2 ** 31, 2 ** 31 - 1, (k // 16, 2 * n), dtype=torch.int32, device=gu.DEV, generator=gen)
+    s = (torch.rand((k // 128, n), device=gu.DEV, generator=gen) * 9e-3 + 1e-3).to(dtype)
+    a = torch.randn((m, k), device=gu.DEV, generator=gen).to(dtype)
+    empty = torch.empty(0, dtype=torch.int32, device=gu.DEV)
+    workspace = mu.marlin_make_workspace_new(torch.device(gu.DEV))
+
+    def gemm(rows):
+        return ops.marlin_gemm(rows, None, q, None, s, None, None, empty, empty, empty, workspace, scalar_types.uint4b8, rows.shape[0], n, k,
+                               True, False, True, False)
+    got = gemm(a)
+    _ran_in(4, grouped=False)
+    want = torch.cat([gemm(a[i:i + 16]) for i in range(0, m, 16)])
+    assert _lib.load().sonar_marlin_last_mid_strips() == 0
+    scale = float(want.float().abs().max())
+    assert bool(torch.isfinite(want).all()) and float((got.float() - want.float()).abs().max()) <= 1e-2 * scale
