@@ -36,6 +36,15 @@ def test_four_strips(m, slots, k, n, dtype, zp, group):
     _ran_in(4)
 
 
+# ... and the types and groups that those leave out
+@pytest.mark.parametrize("m,slots", [(200, 32), (296, 48), (400, 64)])
+@pytest.mark.parametrize("dtype,zp,group", [("fp16", False, -1), ("fp16", True, 128), ("fp16", True, -1), ("bf16", False, 128), ("bf16", False, -1),
+                                            ("bf16", True, 128)])
+def test_four_strips_in_every_form(m, slots, dtype, zp, group):
+    tm.test_moe_gemm_within_tolerance((m, 16, 2, 640, 2368, group, dtype, zp, False, zp, slots, not zp))
+    _ran_in(4)
+
+
 # fewer than a round of two strips a workgroup, and K below 512
 @pytest.mark.parametrize("m,e,k,n,slots", [(400, 16, 512, 2048, 64), (296, 16, 384, 2432, 48)])
 def test_two_strips(m, e, k, n, slots):

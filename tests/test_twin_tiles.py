@@ -95,6 +95,21 @@ def test_the_other_tile_kernels_on_these_sizes(dtype):
     _child("grouped", dtype, SONAR_MARLIN_NO_TWIN_TILES="1")
 
 
+# 256-row tiles of groups of 32 rows: 252 tiles, a launch of that size alone, in front of which these tiles stand for most calls
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["fp16", "bf16"])
+def test_256_row_tiles_of_small_groups(dtype):
+    _child("small_groups", dtype, SONAR_MARLIN_NO_MID="1", SONAR_MARLIN_NO_TWIN_TILES="1")
+
+
+def _small_groups(dtype: str) -> None:
+    from tests import gpu_util as gu
+    from tests import test_gpu_parity as tp
+    for k, zp in ((192, False), (128, True)):
+        tp.test_wide_tile_kernel_forms_within_tolerance(gu, dtype, 2049, k, 7168, 32, zp, zp)
+        print(k, zp, "ok", flush=True)
+
+
 def _grouped(dtype: str) -> None:
     from tests import test_gpu_moe as tm
     for g, zp in ((64, False), (64, True), (32, False), (32, True), (-1, False)):
@@ -169,5 +184,5 @@ def _layers() -> None:
 
 
 if __name__ == "__main__":
-    {"oracle": _oracle, "grouped": _grouped, "dense": _dense, "layers": _layers}[sys.argv[1]](*sys.argv[2:])
+    {"oracle": _oracle, "grouped": _grouped, "dense": _dense, "layers": _layers, "small_groups": _small_groups}[sys.argv[1]](*sys.argv[2:])
     print("done", flush=True)
