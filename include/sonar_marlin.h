@@ -441,8 +441,9 @@ int sonar_moe_wna16_marlin_gemm_nvfp4(
 /* A grouped GEMM whose result goes through a gated activation (the first of a mixture-of-experts layer's two; marlin_moe.py:134-180
  * of the reference, two calls there).  Where the kernel of the call can form the activation itself, gated
  * dtype[size_m * top_k][size_n / 2] is written, c is left as it was and *gated_written is 1; the bits are those of the GEMM and the
- * activation after one another.  Otherwise *gated_written is 0 and c holds the GEMM's result.  `activation` 0 is sonar_silu_and_mul,
- * else a SONAR_ACT_* kind with its limit and alpha (formed here: 0 and SONAR_ACT_SWIGLUOAI).  gated must not overlap the inputs.
+ * activation after one another, but for silu_and_mul in the decode kernel, where half of a workgroup's wavefronts have the gate and half the
+ * up columns, so that the fp32 sums over K are added in another order.  Otherwise *gated_written is 0 and c holds the GEMM's result.
+ * `activation` 0 is sonar_silu_and_mul, else a SONAR_ACT_* kind with its limit and alpha (formed here: 0 and SONAR_ACT_SWIGLUOAI).  gated must not overlap the inputs.
  * global_scale != NULL: NVFP4.  The other arguments as for sonar_moe_wna16_marlin_gemm.
  * next (may be NULL): sizes of the layer's next GEMM over the same routing, experts of the same type, and `table` of table_bytes
  * (sonar_moe_marlin_gemm_scratch_bytes(sorted_len, moe_block_size, size_n, 64)) of device memory, where this call may lay down what
@@ -472,7 +473,8 @@ int sonar_moe_wna16_marlin_gemm_gated(
 
 /* The grouped GEMM of a layer of few slots straight from topk_ids int32[size_m * top_k], the expert of every row of C (those outside
  * 0 .. num_experts - 1: their rows are not written), without the sorted slots and the launch that makes them; the bits are those of
- * sonar_moe_wna16_marlin_gemm on what sonar_moe_align_block_size makes of the same ids.  Only where
+ * sonar_moe_wna16_marlin_gemm (with gated: of sonar_moe_wna16_marlin_gemm_gated in the decode kernel) on what sonar_moe_align_block_size
+ * makes of the same ids.  Only where
  * sonar_moe_routed_gemm_applies(size_m * top_k, ...) is 1 (at most 128 slots and 256 experts, blocks of 8, 16 or 32 slots, 4-bit integers
  * and MXFP4, sizes that run in the decode kernel); other calls are refused.  gated (may be NULL) to gated_written as for
  * sonar_moe_wna16_marlin_gemm_gated, the other arguments as for sonar_moe_wna16_marlin_gemm. */

@@ -1712,7 +1712,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 // operands of A instead of eight, one set of column constants (a column block's are replaced behind its last use), 32-bit
 // offsets of A, a scale row read from one address (several groups only), and no partial tiles: K is never cut here.  The price is
 // that every weight is dequantised once for 128 rows: per matrix instruction 1.7 other vector instructions in float16, 1.2 for
-// MXFP4, 2.3 for integers in bfloat16.  Us, before -> now (bits equal): twin_pays and is_twin have the figures.
+// MXFP4, 2.3 for integers in bfloat16.  Us, before -> now (bits equal): twin_pays and moe_twin_tiles have the figures.
 template <typename T, bool HAS_ZP, bool GROUPED, bool FP4, bool G32>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void marlin_tile_twin_kernel(const TileParams p) {
   int tile, tile_m, tile_n, split;
