@@ -228,8 +228,9 @@ __global__ __launch_bounds__(kMidWaves * 64) __attribute__((amdgpu_waves_per_eu(
     } else {
       const int i = op - (kOps - kCopies);
       const char* a_src = reinterpret_cast<const char*>(p.a) + (size_t)k * (kMidStepK * 2);
-      const int at = kEvenCopies ? strip_of * kCopies + i : min(strip_of * kCopies + i, 2 * MB - 1);
-      copy_to_lds<16>(a_lds + slot * kStage + at * 1024, a_off[i], a_src);
+      // (not one call with a chosen index: that costs every copy an instruction more)
+      if constexpr (kEvenCopies) copy_to_lds<16>(a_lds + slot * kStage + (strip_of * kCopies + i) * 1024, a_off[i], a_src);
+      else copy_to_lds<16>(a_lds + slot * kStage + min(strip_of * kCopies + i, 2 * MB - 1) * 1024, a_off[i], a_src);
     }
   };
   // Scales of the unit of step `k`, behind whose first half they are taken from the registers, and zero points, which fp16
